@@ -258,6 +258,147 @@ __global__ __launch_bounds__(256) void quant_rows_generic_lane(
         dst[c * q_sc] = (uint8_t)e4m3fn_encode(fetch<T, SILU>(src + c * a_sc) * s);
 }
 
+// ---- rows that are columns in memory (a_sr == 1: an [E, K, N] weight quantised per output column, q as
+// [E, N, K] bytes).  Two launches: the amax of every row over the whole chip, then the transposing
+// quantisation, tile by tile.  Bound by HBM: the operand is read twice (the second time mostly from the
+// last-level cache where it fits) and its bytes written once.  A lane per row, the form this replaces,
+// kept rows / 64 waves in flight, each with a serial walk over its columns and one-byte stores a row apart:
+// 8 x 1024 x 4096 took 751 us (N = 4096) and 3147 us (N = 1024); the two launches take 15 + 19 us on both (67 MB
+// read at 4.5 TB/s; 67 MB read, half of it written, at 5.3 TB/s).
+
+constexpr int kColTileN = 64;       // rows of the result per block: 128 bytes of a memory row
+constexpr int kColTileK = 128;      // columns per block of the second launch: a whole line of result bytes
+constexpr int kColMaxSplit = 64;
+
+// Blocks of the first launch along the columns: enough to fill the chip (4 per CU), at least 64 columns each.
+inline int col_splits(int64_t batch, int64_t rows, int64_t cols) {
+    const int64_t strips = batch * ((rows + kColTileN - 1) / kColTileN);
+    int64_t s = (1024 + strips - 1) / strips;
+    const int64_t most = (cols + 63) / 64;
+    s = s < most ? s : most;
+    return (int)(s < 1 ? 1 : (s > kColMaxSplit ? kColMaxSplit : s));
+}
+
+// |value| bits of a bf16 pair, each in the position that compares as an integer (NaN above inf)
+__device__ __forceinline__ void amax_bits(uint32_t pair, uint32_t& lo, uint32_t& hi) {
+    lo = max(lo, (pair << 16) & 0x7fffffffu);
+    hi = max(hi, pair & 0x7fff0000u);
+}
+
+// block (strip, split, batch): 8 lanes x 16 bytes across the strip, 32 rows of memory at a time, four loads
+// in flight per lane; part[split][batch * rows] receives the strip's |max| bits over the split's columns.
+__global__ __launch_bounds__(256) void quant_cols_amax(const uint16_t* __restrict__ a, int64_t rows, int64_t cols,
+                                                       int64_t a_sb, int64_t a_sc, uint32_t* __restrict__ part,
+                                                       int64_t total_rows, int64_t cols_per_split) {
+    __shared__ uint32_t s_max[4][kColTileN];
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    const int64_t n = (int64_t)blockIdx.x * kColTileN + (lane & 7) * 8;
+    const int64_t k_lo = blockIdx.y * cols_per_split;
+    const int64_t k_hi = k_lo + cols_per_split < cols ? k_lo + cols_per_split : cols;
+    uint32_t m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (n < rows) {             // (rows are whole 8-element chunks on this path)
+        const uint16_t* src = a + blockIdx.z * a_sb + n;
+        int64_t k = k_lo + threadIdx.x / 8;
+        for (; k + 96 < k_hi; k += 128) {
+            u32x4 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const u32x4*>(src + (k + 32 * i) * a_sc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) amax_bits(v[i][j], m[2 * j], m[2 * j + 1]);
+        }
+        for (; k < k_hi; k += 32) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(src + k * a_sc);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) amax_bits(v[j], m[2 * j], m[2 * j + 1]);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+#pragma unroll
+        for (int o = 8; o < kWave; o <<= 1) m[j] = max(m[j], (uint32_t)__shfl_xor((int)m[j], o, kWave));
+        if (lane < 8) s_max[wave][lane * 8 + j] = m[j];
+    }
+    __syncthreads();
+    if (threadIdx.x < kColTileN) {
+        const int64_t r = (int64_t)blockIdx.x * kColTileN + threadIdx.x;
+        if (r < rows)
+            part[blockIdx.y * total_rows + blockIdx.z * rows + r] =
+                max(max(s_max[0][threadIdx.x], s_max[1][threadIdx.x]), max(s_max[2][threadIdx.x], s_max[3][threadIdx.x]));
+    }
+}
+
+// block (row tile, column tile, batch): 64 rows x 128 columns.  A lane loads 8 rows of four consecutive columns;
+// the conversion instruction packs two values of its choice, so the four columns of a row leave it as one dword
+// of consecutive bytes and the transposition costs no instruction of its own.  LDS rows are 33 dwords apart: the
+// 64 dwords a wave stores at a time fall into 64 banks.
+__global__ __launch_bounds__(256) void quant_cols_store(const uint16_t* __restrict__ a, int64_t rows, int64_t cols,
+                                                        int64_t a_sb, int64_t a_sc, const uint32_t* __restrict__ part,
+                                                        int splits, int64_t total_rows, uint8_t* __restrict__ q,
+                                                        int64_t q_sb, int64_t q_sr, float* __restrict__ scale,
+                                                        int store_reciprocal, int wide) {
+    __shared__ uint32_t tile[kColTileN * 33];
+    __shared__ float s_scale[kColTileN];
+    __shared__ int s_special;
+    const int tid = threadIdx.x;
+    const int64_t n0 = (int64_t)blockIdx.x * kColTileN, k0 = (int64_t)blockIdx.y * kColTileK;
+    const int ng = tid & 7, kq = tid >> 3;
+    const int64_t n = n0 + 8 * ng, k = k0 + 4 * kq;
+    // the tile's loads first: they are in flight while the scales are worked out
+    u32x4 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        v[i] = n < rows && k + i < cols ? *reinterpret_cast<const u32x4*>(a + blockIdx.z * a_sb + (k + i) * a_sc + n)
+                                        : u32x4{0, 0, 0, 0};
+    if (tid == 0) s_special = 0;
+    __syncthreads();
+    if (tid < kColTileN) {
+        const int64_t r = n0 + tid;
+        uint32_t bits = 0;
+        if (r < rows)
+            for (int i = 0; i < splits; ++i) bits = max(bits, part[i * total_rows + blockIdx.z * rows + r]);
+        const float s = scale_from_amax<true>(__uint_as_float(bits));
+        s_scale[tid] = s;
+        if (bits >= 0x7f800000u) s_special = 1;
+        if (r < rows && blockIdx.y == 0) scale[blockIdx.z * rows + r] = store_reciprocal ? 1.0f / s : s;
+    }
+    __syncthreads();
+    const bool special = s_special != 0;        // a row with NaN or inf: the software encoder, as in encode8
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float s = s_scale[8 * ng + j];
+        float f[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            f[i] = ((j & 1) ? __uint_as_float(v[i][j / 2] & 0xffff0000u) : bf16_bits_to_f32(v[i][j / 2] & 0xffffu)) * s;
+        uint32_t w;
+        if (!special) {
+            int t = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
+            w = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], t, true);
+        } else {
+            w = e4m3fn_encode(f[0]) | (e4m3fn_encode(f[1]) << 8) | (e4m3fn_encode(f[2]) << 16) | (e4m3fn_encode(f[3]) << 24);
+        }
+        tile[(8 * ng + j) * 33 + kq] = w;
+    }
+    __syncthreads();
+    // rows out: 8 lanes cover the 128 bytes of one
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = (tid >> 3) + 32 * i, c = 4 * (tid & 7);
+        if (n0 + r >= rows) continue;
+        uint8_t* dst = q + blockIdx.z * q_sb + (n0 + r) * q_sr + k0 + 4 * c;
+        const uint32_t* t = tile + r * 33 + c;
+        if (wide && k0 + 4 * c + 16 <= cols) {
+            *reinterpret_cast<u32x4*>(dst) = u32x4{t[0], t[1], t[2], t[3]};
+        } else {
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+                if (k0 + 4 * (c + d) < cols) *reinterpret_cast<uint32_t*>(dst + 4 * d) = t[d];     // (cols % 4 == 0)
+        }
+    }
+}
+
 // rows that are whole pairs of chunks, stored 16 bytes at a time
 inline bool wide_stores(int64_t cols, const uint8_t* q, int64_t q_sb, int64_t q_sr) {
     return cols % 16 == 0 && (reinterpret_cast<uintptr_t>(q) & 15u) == 0 && q_sb % 16 == 0 && q_sr % 16 == 0;
@@ -365,4 +506,44 @@ extern "C" int fmoe_quant_rows_e4m3(const void* a, int a_dtype, int64_t batch, i
         launch_generic<float>(apply_silu != 0, lane_per_row, a, total, rows, cols, a_sb, a_sr, a_sc, q,
                               q_sb, q_sr, q_sc, scale, store_reciprocal, stream);
     return check_launch("fmoe_quant_rows_e4m3");
+}
+
+// What the two-launch form takes: bf16, memory rows of whole aligned 16-byte chunks, result rows of whole dwords.
+static bool takes_cols(int a_dtype, int64_t batch, int64_t rows, int64_t cols, int64_t a_sb, int64_t a_sr, int64_t a_sc,
+                       int apply_silu) {
+    return a_dtype == FMOE_BF16 && !apply_silu && a_sr == 1 && a_sc >= rows && rows % 8 == 0 && cols % 4 == 0 &&
+           a_sc % 8 == 0 && (batch == 1 || a_sb % 8 == 0) && batch >= 1 && batch <= 65535 && rows >= 8 &&
+           (cols + kColTileK - 1) / kColTileK <= 65535;
+}
+
+extern "C" size_t fmoe_quant_rows_workspace_bytes(int a_dtype, int64_t batch, int64_t rows, int64_t cols, int64_t a_sb,
+                                                  int64_t a_sr, int64_t a_sc, int apply_silu) {
+    if (!takes_cols(a_dtype, batch, rows, cols, a_sb, a_sr, a_sc, apply_silu)) return 0;
+    return (size_t)col_splits(batch, rows, cols) * (size_t)(batch * rows) * sizeof(uint32_t);
+}
+
+extern "C" int fmoe_quant_rows_e4m3_ws(const void* a, int a_dtype, int64_t batch, int64_t rows, int64_t cols,
+                                       int64_t a_sb, int64_t a_sr, int64_t a_sc, int apply_silu, uint8_t* q,
+                                       int64_t q_sb, int64_t q_sr, int64_t q_sc, float* scale, int store_reciprocal,
+                                       void* workspace, size_t workspace_bytes, fmoe_stream_t stream_) {
+    const size_t need = fmoe_quant_rows_workspace_bytes(a_dtype, batch, rows, cols, a_sb, a_sr, a_sc, apply_silu);
+    const bool cols_form = need > 0 && workspace_bytes >= need && workspace && a && q && scale && aligned16(a) &&
+                           q_sc == 1 && q_sr % 4 == 0 && q_sb % 4 == 0 && q_sr >= cols &&
+                           (reinterpret_cast<uintptr_t>(q) & 3u) == 0;
+    if (!cols_form)
+        return fmoe_quant_rows_e4m3(a, a_dtype, batch, rows, cols, a_sb, a_sr, a_sc, apply_silu, q, q_sb, q_sr, q_sc,
+                                    scale, store_reciprocal, stream_);
+    hipStream_t stream = (hipStream_t)stream_;
+    const int splits = col_splits(batch, rows, cols);
+    const int64_t per_split = (cols + splits - 1) / splits;
+    const int64_t strips = (rows + kColTileN - 1) / kColTileN;
+    FMOE_REQUIRE(strips < ((int64_t)1 << 31), "fmoe_quant_rows_e4m3_ws: too many rows");
+    uint32_t* part = (uint32_t*)workspace;
+    quant_cols_amax<<<dim3((unsigned)strips, (unsigned)splits, (unsigned)batch), 256, 0, stream>>>(
+        (const uint16_t*)a, rows, cols, a_sb, a_sc, part, batch * rows, per_split);
+    const int wide = (reinterpret_cast<uintptr_t>(q) & 15u) == 0 && q_sr % 16 == 0 && q_sb % 16 == 0;
+    quant_cols_store<<<dim3((unsigned)strips, (unsigned)((cols + kColTileK - 1) / kColTileK), (unsigned)batch), 256, 0,
+                       stream>>>((const uint16_t*)a, rows, cols, a_sb, a_sc, part, splits, batch * rows, q, q_sb, q_sr,
+                                 scale, store_reciprocal, wide);
+    return check_launch("fmoe_quant_rows_e4m3_ws");
 }

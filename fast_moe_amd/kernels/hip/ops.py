@@ -180,10 +180,14 @@ def quant_rows_fp8(a: torch.Tensor, apply_silu: bool = False, reciprocal_scale: 
         q3 = torch.empty(a3.shape, dtype=torch.uint8, device=dev)
     scale = torch.empty((B, Rr), dtype=torch.float32, device=dev)
     lib = _lib.load()
-    rc = lib.fmoe_quant_rows_e4m3(
-        a3.data_ptr(), _DTYPE_CODE[a.dtype], B, Rr, C, a3.stride(0), a3.stride(1), a3.stride(2),
-        int(apply_silu), q3.data_ptr(), q3.stride(0), q3.stride(1), q3.stride(2), scale.data_ptr(),
-        int(reciprocal_scale), _stream(a))
+    args = (a3.data_ptr(), _DTYPE_CODE[a.dtype], B, Rr, C, *a3.stride(), int(apply_silu), q3.data_ptr(), *q3.stride(),
+            scale.data_ptr(), int(reciprocal_scale))
+    if a3.stride(1) == 1 and a3.stride(2) != 1:         # rows are columns in memory
+        ws_bytes = lib.fmoe_quant_rows_workspace_bytes(*args[1:8], args[8])
+        ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
+        rc = lib.fmoe_quant_rows_e4m3_ws(*args, _ptr(ws), ws_bytes, _stream(a))
+    else:
+        rc = lib.fmoe_quant_rows_e4m3(*args, _stream(a))
     _lib.check(rc, "fmoe_quant_rows_e4m3")
     q = q3.view(FP8_DTYPE)
     if a.ndim == 1:

@@ -156,6 +156,20 @@ int fmoe_quant_rows_e4m3(const void* a, int a_dtype, int64_t batch, int64_t rows
                          int64_t q_stride_c, float* scale, int store_reciprocal,
                          fmoe_stream_t stream);
 
+/*
+ * The same with a scratch buffer of the caller (fmoe_quant_rows_workspace_bytes bytes; 0: none is needed), which
+ * lets matrices whose rows are columns in memory (a_stride_r == 1: an [E, K, N] weight quantised per output
+ * column) be read and written in whole lines by the whole chip.  Same bytes and scales.
+ */
+size_t fmoe_quant_rows_workspace_bytes(int a_dtype, int64_t batch, int64_t rows, int64_t cols,
+                                       int64_t a_stride_b, int64_t a_stride_r, int64_t a_stride_c,
+                                       int apply_silu);
+int fmoe_quant_rows_e4m3_ws(const void* a, int a_dtype, int64_t batch, int64_t rows, int64_t cols,
+                            int64_t a_stride_b, int64_t a_stride_r, int64_t a_stride_c,
+                            int apply_silu, uint8_t* q, int64_t q_stride_b, int64_t q_stride_r,
+                            int64_t q_stride_c, float* scale, int store_reciprocal,
+                            void* workspace, size_t workspace_bytes, fmoe_stream_t stream);
+
 /* -------------------------------------------------------------- grouped GEMM */
 
 /*

@@ -222,3 +222,21 @@ def test_fp8_operators_requantise_every_call_and_take_a_kept_pair():
         assert torch.equal(moe_fp8.cached_quantize_expert_weights(w)[1], pair2[1] * 0.5)
     with pytest.raises(ValueError):
         moe_fp8.index_select_jagged_bmm(0, off, idx, x, w, None, fp8=True, fp8_weight=(pair[0][:4], pair[1]))
+
+
+@pytest.mark.parametrize("E,K,N", [(1, 4, 8), (3, 60, 72), (2, 128, 64), (2, 132, 136), (1, 1000, 8), (5, 1028, 264),
+                                   (1, 8200, 128), (2, 126, 64)])
+def test_rows_that_are_columns_in_memory(E, K, N):
+    """[E, K, N]-contiguous weights quantised per output column: tiles of 64 rows x 128 columns, their
+    remainders on both sides, whole and partial 16-byte results (K = 126 takes the lane-per-row form).  Bit for bit."""
+    from fast_moe_amd.kernels import moe_fp8
+    g = torch.Generator().manual_seed(K + N)
+    w = (torch.randn(E, K, N, generator=g) * torch.exp(torch.randn(E, 1, N, generator=g) * 4)).to(torch.bfloat16)
+    w[0, 0, 1], w[-1, K - 1, N - 1] = float("inf"), float("nan")
+    w[0, :, 0] = 0
+    q_ref, s_ref = o_fp8.rowwise_quant_fp8(w.permute(0, 2, 1).contiguous().float().numpy(), "bf16")
+    q, s = moe_fp8.quantize_expert_weights(w.cuda())
+    assert np.array_equal(s.cpu().numpy(), s_ref)
+    got = q.permute(0, 2, 1).view(torch.uint8).cpu().numpy()
+    nan = (q_ref & 0x7F) == 0x7F          # (the sign of a NaN code is not defined by the arithmetic)
+    assert np.array_equal((got & 0x7F) == 0x7F, nan) and np.array_equal(got[~nan], q_ref[~nan])
