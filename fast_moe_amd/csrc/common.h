@@ -67,20 +67,35 @@ __device__ __forceinline__ void round_bf16_pair(float& a, float& b) {
 
 __device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + expf(-x)); }
 
-// round(silu(x)) to bf16 for a bf16-valued x, equal on every one of the 65536 inputs to what
+// round(silu(x)) to bf16 for two bf16-valued x, equal on every one of the 65536 inputs to what
 // x / (1 + exp(-x)) gives when it is evaluated in fp32 with correctly rounded steps and then rounded
-// to bf16 (F.silu on a bf16 tensor).  The fp32 evaluation here may be a few units in the last
-// place off, which only matters when the result lies next to the midpoint of two bf16 values: those
-// (about one input in 4000) are evaluated again in double.  exp(-x) overflows fp32 from x = -88.8
-// down and the quotient is -0 there, as in the fp32 formula; such results never take the second path.
-__device__ __forceinline__ float silu_round_bf16(float x) {
-    float y = x / (1.0f + expf(-x));
-    const uint32_t low = __float_as_uint(y) & 0xffffu;
-    if (low - 0x7ff0u <= 0x20u) {
-        const double xd = (double)x;
-        y = (float)(xd / (1.0 + exp(-xd)));
+// to bf16 (F.silu on a bf16 tensor).  v_exp_f32 and v_rcp_f32 give that rounding on every input with two
+// corrections: at x = 5.9375 the fp32 quotient comes out on the midpoint of two bf16 values, one unit in the last
+// place above the exact one, which the addend one unit above 1 takes back (it moves no other input's rounding);
+// and at -87.5, -88 and -88.5 the reciprocal lies below the normal range and is flushed: x * exp(x), scaled through
+// the exponent, rounds right there.  Further down exp(-x) overflows and the quotient is -0, as in the fp32 formula.
+// (Library expf, a division and a double-precision second look bound the passes that call this by VALU work and by the
+// size of their unrolled code: 33 M hidden elements took the SiLU quantiser 54 us, 24 M silu_mul 32 us.)
+__device__ __forceinline__ void silu_round_bf16_pair(float& a, float& b) {
+    constexpr float kLog2e = 1.44269504088896341f, kOnePlus = 1.00000012f;
+    float ya = a * __builtin_amdgcn_rcpf(kOnePlus + __builtin_amdgcn_exp2f(a * -kLog2e));
+    float yb = b * __builtin_amdgcn_rcpf(kOnePlus + __builtin_amdgcn_exp2f(b * -kLog2e));
+    if (fminf(a, b) < -87.0f) {
+        auto low = [](float x, float y) {
+            const float scaled = x * __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2e, 32.0f));
+            return x < -87.0f && x > -88.7f ? scaled * 0x1p-32f : y;
+        };
+        ya = low(a, ya);
+        yb = low(b, yb);
     }
-    return round_bf16(y);
+    round_bf16_pair(ya, yb);
+    a = ya;
+    b = yb;
+}
+__device__ __forceinline__ float silu_round_bf16(float x) {
+    float other = 0.0f;
+    silu_round_bf16_pair(x, other);
+    return x;
 }
 
 // SiLU from the hardware exp / reciprocal (about 2 ulp in fp32): for values that

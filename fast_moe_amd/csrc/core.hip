@@ -35,14 +35,10 @@ __global__ __launch_bounds__(256) void silu_mul_bf16_kernel(const uint16_t* __re
         u32x4 vo;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            uint32_t r = 0;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const float x = bf16_bits_to_f32((va[j] >> (16 * h)) & 0xffffu);
-                const float y = bf16_bits_to_f32((vb[j] >> (16 * h)) & 0xffffu);
-                r |= f32_to_bf16_bits(GATED ? silu_round_bf16(x) * y : silu_round_bf16(x)) << (16 * h);
-            }
-            vo[j] = r;
+            float x0 = bf16_bits_to_f32(va[j] & 0xffffu), x1 = __uint_as_float(va[j] & 0xffff0000u);
+            silu_round_bf16_pair(x0, x1);
+            vo[j] = GATED ? cvt_pk_bf16(x0 * bf16_bits_to_f32(vb[j] & 0xffffu), x1 * __uint_as_float(vb[j] & 0xffff0000u))
+                          : cvt_pk_bf16(x0, x1);
         }
         *reinterpret_cast<u32x4*>(out + i0) = vo;
     } else {

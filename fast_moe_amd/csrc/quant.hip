@@ -117,8 +117,7 @@ __global__ __launch_bounds__(256) void quant_rows_bf16_wave(
             float lo = bf16_bits_to_f32(v[i][j] & 0xffffu);
             float hi = __uint_as_float(v[i][j] & 0xffff0000u);
             if (SILU) {
-                lo = silu_round_bf16(lo);
-                hi = silu_round_bf16(hi);
+                silu_round_bf16_pair(lo, hi);
                 v[i][j] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
             }
             m = amax_update(m, lo, nan);
@@ -167,8 +166,8 @@ __global__ __launch_bounds__(256) void quant_rows_bf16_block(
         if (SILU) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float lo = silu_round_bf16(bf16_bits_to_f32(v[j] & 0xffffu));
-                const float hi = silu_round_bf16(__uint_as_float(v[j] & 0xffff0000u));
+                float lo = bf16_bits_to_f32(v[j] & 0xffffu), hi = __uint_as_float(v[j] & 0xffff0000u);
+                silu_round_bf16_pair(lo, hi);
                 v[j] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
             }
         }
