@@ -165,15 +165,16 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
     const int64_t span32 = ((int64_t)1 << 32) - 4096;
     const bool near = d->a_rows * d->a_stride_row * esize + (int64_t)d->k * esize < span32 &&
                       (int64_t)d->n * d->b_stride_n * esize + (int64_t)d->k * esize < span32;
-    const bool ring = fast && big && !f32 && !d->a_silu && (d->k % slice) == 0 && d->k / slice >= 3 &&
+    const bool tail = !f32 && !d->k_window && !two && ring_tail_takes(esize, d->k, d->num_experts, d->total_rows);
+    const bool ring = fast && big && !f32 && !d->a_silu && (tail || ((d->k % slice) == 0 && d->k / slice >= 3)) &&
                       p.vec_store && d->num_experts <= 1024 && d->total_rows < ((int64_t)1 << 31) * 128 && near;
     // N-contiguous bf16 weights (B[e][k][n], n fastest) are read in place by the paired ring
     const bool ring_tr = !fp8 && !f32 && big && !d->a_silu && !d->k_window && d->b_stride_n == 1 &&
                          d->b_stride_k != 1 && (d->b_stride_k % chunk) == 0 && (d->b_stride_e % chunk) == 0 &&
                          (d->a_stride_row % chunk) == 0 && (d->a_stride_e % chunk) == 0 && aligned16(d->a) &&
-                         aligned16(d->b) && (!(swiglu || two) || aligned16(d->b2)) && (d->k % (2 * slice)) == 0 &&
-                         (ktot % (2 * slice)) == 0 && (!two || aligned16(d->a2)) &&
-                         ktot / slice >= 4 && p.vec_store && d->num_experts <= TileRing5W::kMaxExperts &&
+                         aligned16(d->b) && (!(swiglu || two) || aligned16(d->b2)) && (!two || aligned16(d->a2)) &&
+                         (tail || ((d->k % (2 * slice)) == 0 && (ktot % (2 * slice)) == 0 && ktot / slice >= 4)) &&
+                         p.vec_store && d->num_experts <= TileRing5W::kMaxExperts &&
                          d->total_rows < ((int64_t)1 << 31) && lds_per_block() >= TileRing5::LDS_BYTES &&
                          d->a_rows * d->a_stride_row * esize + (int64_t)ktot * esize < span32 &&
                          ((int64_t)ktot * d->b_stride_k + d->n) * esize < span32;

@@ -89,7 +89,8 @@ int launch_stream(GemmParams p, hipStream_t stream) {
     return go(grouped_gemm_stream_kernel<DT, EPI, false>, done);
 }
 
-template <typename TL, bool FP8, int EPI, bool WTR = false, bool KWIN = false, bool XTR = false, bool MSC = false>
+template <typename TL, bool FP8, int EPI, bool WTR = false, bool KWIN = false, bool XTR = false, bool MSC = false,
+          bool KTAIL = false>
 int launch_ring_cfg(GemmParams p, hipStream_t stream) {
     constexpr int bn_out = EPI == FMOE_EPI_SWIGLU ? TL::BN / 2 : TL::BN;
     p.n_tiles = (p.N + bn_out - 1) / bn_out;
@@ -107,7 +108,7 @@ int launch_ring_cfg(GemmParams p, hipStream_t stream) {
         // second tile of most experts is a short one: the shortened loop stays on whatever K is.
         p.short_tile_rows = (p.K / (FP8 ? 64 : 32) <= 64 || p.total_rows / p.E <= 2 * TL::BM) ? TL::BM / 2 : 0;
     }
-    auto kern = grouped_gemm_ring_kernel<TL, FP8, EPI, WTR, KWIN, XTR, MSC>;
+    auto kern = grouped_gemm_ring_kernel<TL, FP8, EPI, WTR, KWIN, XTR, MSC, KTAIL>;
     static bool attr_done = false;
     if (int rc = reserve_lds(kern, TL::LDS_BYTES, attr_done)) return rc;
     // persistent: one block per CU (the LDS footprint admits no second one), a multiple of
@@ -116,6 +117,20 @@ int launch_ring_cfg(GemmParams p, hipStream_t stream) {
     if (grid < kNumXcd) grid = kNumXcd;
     kern<<<(unsigned)grid, TL::NT, TL::LDS_BYTES, stream>>>(p);
     return check_launch("fmoe_grouped_gemm");
+}
+
+// Ring kernels for K that is no whole number of K-slice pairs (gemm_bf16_tail.hip, gemm_fp8_tail.hip).
+int run_ring_tail_bf16(const GemmParams& p, int epilogue, hipStream_t stream);
+int run_ring_tail_fp8(const GemmParams& p, int epilogue, hipStream_t stream);
+
+// What they take beyond the ring's own conditions: at least one pair of slices and a 16-byte chunk.  (An odd slice count
+// goes there as well; the 4-slot ring is left with more than 256 experts.)  On 9189 rows, 12 experts, 1000 <-> 2600
+// columns: weights with n contiguous 85 us per GEMM where the element-load kernel took 1368 and 1620; weights with k
+// contiguous 94 us against 99 on the register-staged kernel.
+inline bool ring_tail_takes(int esize, int64_t k, int num_experts, int64_t total_rows) {
+    const int pair = 128 / esize, chunk = 16 / esize;
+    return k > pair && k % pair != 0 && k % chunk == 0 && num_experts <= TileRing5W::kMaxExperts &&
+           total_rows < ((int64_t)1 << 31) && lds_per_block() >= TileRing5W::LDS_BYTES;
 }
 
 // The 5-slot ring needs every byte of a 160 KB LDS, an even number of K-slices per tile,
@@ -135,6 +150,8 @@ int launch_ring(const GemmParams& p, hipStream_t stream) {
         }
         return fail(FMOE_ERR_UNSUPPORTED, "fmoe_grouped_gemm: row-indexed operands need bf16 and no epilogue");
     }
+    if (!p.k_window && ring_tail_takes(FP8 ? 1 : 2, p.K, p.E, p.total_rows))
+        return FP8 ? run_ring_tail_fp8(p, EPI, stream) : run_ring_tail_bf16(p, EPI, stream);
     if (p.b_sn == 1 && p.b_sk != 1) {      // N-contiguous weights in place (the caller checked pair_ok's terms)
         if constexpr (!FP8) {
             if (p.E <= TileRing5::kMaxExperts) return launch_ring_cfg<TileRing5, FP8, EPI, true>(p, stream);

@@ -82,12 +82,20 @@ __device__ __forceinline__ int uniform_lane(int v, int src_lane) {
 // would give).  The scales of the next tile are fetched inside the epilogue of the current one
 // (row indices before it, the scales behind its first row block, packed at its end), so that no
 // tile waits for an index -> scale chain and the epilogue multiplies nothing.
-template <typename TL, bool FP8, int EPI, bool WTR = false, bool KWIN = false, bool XTR = false, bool MSC = false>
+//
+// KTAIL (paired ring, no window): K is any whole number of 16-byte chunks above one pair of K-slices.  The last
+// pair of a tile is fetched from the last 2 * BK columns of the operands, wherever the pair before it ended: the
+// columns both hold are masked out of the last pair's fragments, on both sides (a product of a real infinity with a
+// masked zero would be NaN).  No address beyond a row's end, no per-lane predicate in the DMA stream: the tail costs a
+// scalar select per pair and the masks of one double step per tile.
+template <typename TL, bool FP8, int EPI, bool WTR = false, bool KWIN = false, bool XTR = false, bool MSC = false,
+          bool KTAIL = false>
 __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmParams p) {
     static_assert(!MSC || (FP8 && TL::PAIR && !KWIN && !WTR && !XTR), "MFMA-applied scales: e4m3 on the paired ring");
     static_assert(!WTR || (TL::PAIR && !FP8 && TL::BN == 256 && TL::NW == 8),
                   "in-place N-contiguous weights: bf16, paired ring, 256-column tiles of 8 waves");
     static_assert(!KWIN || TL::PAIR, "contraction windows: paired ring");
+    static_assert(!KTAIL || (TL::PAIR && !KWIN && !XTR), "K tails: paired ring without windows");
     static_assert(XTR ? (WTR && KWIN && TL::BM == 256 && EPI == FMOE_EPI_NONE) : !(KWIN && WTR),
                   "row-indexed operands come together, with a window, and without an epilogue");
     constexpr int BM = TL::BM, BN = TL::BN, NW = TL::NW, STAGES = TL::STAGES;
@@ -266,7 +274,9 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         return (round * kNumXcd + pos) * group_span + (j - round * group_span);
     };
 
-    const int KT = p.K / BK;
+    const int KT = KTAIL ? (p.K + 2 * BK - 1) / (2 * BK) * 2 : p.K / BK;
+    // KTAIL: columns at the start of the last pair that the pair before it has multiplied already
+    const int tail_dup = KTAIL ? KT * BK - p.K : 0;
     struct TileInfo { int expert; int nt; int64_t row0; int rows_valid; int64_t k_begin; int kt; int m0; int klen; };
     auto locate = [&](int64_t logical) -> TileInfo {
         const int64_t group = div_span(logical);
@@ -460,10 +470,12 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     // A second product a2 * b2 continued in the same accumulators: the K-slices from split_kt on
     // come from a2 and b2, addressed with the strides of a and b.  (A pair of slices never
     // straddles the split: k_split is a whole number of pairs.)
-    constexpr bool SPLIT = WTR && PAIR && !FP8 && !SWIGLU && !KWIN && !XTR;
+    constexpr bool SPLIT = WTR && PAIR && !FP8 && !SWIGLU && !KWIN && !XTR && !KTAIL;
     const int split_kt = SPLIT && p.a2 ? p.k_split / BK : 0x7fffffff;
     const int64_t split_x = SPLIT && p.a2 ? (p.a2 - p.a) - (int64_t)split_kt * xstep : 0;
     const int64_t split_w = SPLIT && p.a2 ? (p.b2 - p.b) - (int64_t)split_kt * wstep : 0;
+    const int64_t tail_x = KTAIL ? (int64_t)(p.K - 2 * BK) * ESIZE : 0;
+    const int64_t tail_w = KTAIL ? (WTR ? (int64_t)(p.K - 2 * BK) * p.b_sk * ESIZE : tail_x) : 0;
     // one K-slice into slot sa; in pair mode also the following slice into slot sb, the two
     // 64-byte halves of every row's 128 bytes requested by adjacent instructions
     auto issue = [&](int kt, int sa, int sb) {
@@ -474,6 +486,10 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         if constexpr (SPLIT) {
             koff += kt >= split_kt ? split_x : 0;
             wkoff += kt >= split_kt ? split_w : 0;
+        }
+        if constexpr (KTAIL) {
+            koff = kt == KT - 2 ? tail_x : koff;
+            wkoff = kt == KT - 2 ? tail_w : wkoff;
         }
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
@@ -757,6 +773,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             // k lies at or beyond the end of the tile's window (XTR, the tile's last slices)
             auto load_block = [&](bf16x8 (&wf)[FN], bf16x8 (&xf)[FM], int slot_i, int sub, int item, auto mask_c, auto act_c) {
                 constexpr bool MASK = XTR && decltype(mask_c)::value;
+                constexpr bool MASK_TAIL = KTAIL && decltype(mask_c)::value;
                 constexpr int ACT = decltype(act_c)::value;     // row blocks that are multiplied
                 const uint8_t* sx = smem + slot_i * TL::STAGE_BYTES;
                 const uint8_t* sw = sx + BM * 64;
@@ -770,6 +787,17 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 for (int fm = 0; fm < ACT; ++fm) {
                     if constexpr (XTR) xf[fm] = read_tr(sx + xtr_off[fm] + sub * 4096);
                     else xf[fm] = *reinterpret_cast<const bf16x8*>(sx + lds_off64(xfrag_row[fm], chunk));
+                }
+                if constexpr (MASK_TAIL) {      // (a fragment is one 16-byte chunk: masked whole or not at all)
+                    const int at = (item - (KT - 2)) * BK + 16 * sub + 8 * khalf;
+                    const uint32_t m1 = at >= 0 && at < tail_dup ? 0u : 0xffffffffu;
+                    const u32x4 m = {m1, m1, m1, m1};
+#pragma unroll
+                    for (int fn = 0; fn < FN; ++fn)
+                        wf[fn] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, wf[fn]) & m);
+#pragma unroll
+                    for (int fm = 0; fm < ACT; ++fm)
+                        xf[fm] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, xf[fm]) & m);
                 }
                 if constexpr (MASK) {
                     // register i of a fragment holds k = first + 2i, first + 2i + 1
@@ -863,6 +891,10 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                     part_koff += ikt >= split_kt ? split_x : 0;
                     part_wkoff += ikt >= split_kt ? split_w : 0;
                 }
+                if constexpr (KTAIL) {
+                    part_koff = ikt == KT - 2 ? tail_x : part_koff;
+                    part_wkoff = ikt == KT - 2 ? tail_w : part_wkoff;
+                }
                 ikt += 2;
                 load_block(wfb, xfb, s1, 1, kitem + 1, mask_c, act_c);
                 if constexpr (HALF == 0) __builtin_amdgcn_sched_barrier(0);
@@ -939,6 +971,19 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
 #pragma unroll
                 for (int fm = 0; fm < HM; ++fm) xh[fm] = load_frag(sx, xfrag_row[HM + fm]);
             };
+            // KTAIL: the fragment of the item in the first (HALF_ITEM 0) or second slot of the last pair, masked
+            // where the pair before it reached (a lane's 32 bytes are two 16-byte chunks)
+            auto tail_mask = [&](i32x8& f, auto half_item_c) {
+                if constexpr (KTAIL) {
+                    const int at = decltype(half_item_c)::value * BK + 32 * khalf;
+                    const int lo = at < tail_dup ? 0 : -1, hi = at + 16 < tail_dup ? 0 : -1;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        f[i] &= lo;
+                        f[4 + i] &= hi;
+                    }
+                }
+            };
             // skip_c: the block's row blocks hold no valid row (sparse tile); only its share of the
             // DMA issue is left
             auto mma_block = [&](const i32x8 (&wf)[FN], const i32x8 (&xh)[HM], auto fm0_c, auto dma_c, auto skip_c) {
@@ -995,6 +1040,15 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 const int s1 = cslot + 1 == STAGES ? 0 : cslot + 1;
                 const int s2 = s1 + 1 == STAGES ? 0 : s1 + 1;
                 if (!SP) load_x1(qx1, cslot);
+                if constexpr (KTAIL && LAST) {
+#pragma unroll
+                    for (int fn = 0; fn < FN; ++fn) tail_mask(qwa[fn], std::integral_constant<int, 0>{});
+#pragma unroll
+                    for (int fm = 0; fm < HM; ++fm) {
+                        tail_mask(qx0[fm], std::integral_constant<int, 0>{});
+                        if (!SP) tail_mask(qx1[fm], std::integral_constant<int, 0>{});
+                    }
+                }
                 __builtin_amdgcn_sched_barrier(0);
                 mma_block(qwa, qx0, std::integral_constant<int, 0>{}, std::false_type{}, full);
                 __builtin_amdgcn_sched_barrier(0);
@@ -1009,8 +1063,21 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 islot = islot + 1 == STAGES ? 0 : islot + 1;
                 part_koff = (int64_t)ikt * xstep;
                 part_wkoff = WTR ? (int64_t)ikt * wstep : part_koff;
+                if constexpr (KTAIL) {
+                    part_koff = ikt == KT - 2 ? tail_x : part_koff;
+                    part_wkoff = ikt == KT - 2 ? tail_w : part_wkoff;
+                }
                 ikt += 2;
                 if (!SP) load_x1(qx1, s1);
+                if constexpr (KTAIL && LAST) {
+#pragma unroll
+                    for (int fn = 0; fn < FN; ++fn) tail_mask(qwb[fn], std::integral_constant<int, 1>{});
+#pragma unroll
+                    for (int fm = 0; fm < HM; ++fm) {
+                        tail_mask(qx0[fm], std::integral_constant<int, 1>{});
+                        if (!SP) tail_mask(qx1[fm], std::integral_constant<int, 1>{});
+                    }
+                }
                 __builtin_amdgcn_sched_barrier(0);
                 mma_block(qwb, qx0, std::integral_constant<int, 0>{}, std::integral_constant<bool, HALF == 0>{}, full);
                 __builtin_amdgcn_sched_barrier(0);

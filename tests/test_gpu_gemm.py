@@ -1009,3 +1009,53 @@ def test_scales_applied_by_the_mfma_equal_scales_divided_out_in_the_epilogue(E, 
     assert torch.isfinite(plain.float()).all()
     assert torch.equal(folded.view(torch.int16), plain.view(torch.int16))
     assert torch.equal(again.view(torch.int16), folded.view(torch.int16))
+
+
+@pytest.mark.parametrize("E,rows,K,N,layout,epi", [
+    (3, 700, 72, 264, "nk", 0), (3, 700, 120, 136, "kn", 0),        # one pair of K-slices and the shortest / longest rest
+    (2, 1000, 1000, 520, "nk", 2), (2, 1000, 1000, 520, "kn", 2),
+    (5, 600, 2600, 256, "kn", 0), (4, 500, 96, 128, "nk", 1),       # 96: an odd number of whole slices
+    (200, 20000, 136, 72, "nk", 1), (2, 513, 200, 320, "kn", 3),
+    (3, 700, 144, 264, "fp8", 0), (2, 1000, 1040, 136, "fp8", 2), (4, 600, 240, 512, "fp8", 1),
+])
+def test_ring_kernel_contraction_tails(E, rows, K, N, layout, epi):
+    """K that is no whole number of K-slice pairs: the last pair overlaps the one before it and is
+    masked.  The operands are the left columns of wider tensors whose other columns are NaN.  Against
+    float64 on the GPU; 2 roundings to bf16 (SwiGLU: of either factor and the product)."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    g = torch.Generator().manual_seed(K + N)
+    off = torch.tensor([0] + sorted(torch.randint(0, rows, (E - 1,), generator=g).tolist()) + [rows]).cuda()
+    def wide(*shape):
+        t = torch.full((*shape[:-1], shape[-1] + 16), float("nan"), dtype=BF16, device="cuda")
+        t[..., :shape[-1]] = (torch.randn(*shape, generator=g) * shape[-1] ** -0.5).to(BF16).cuda()
+        return t[..., :shape[-1]]
+    x = wide(rows, K)
+    ws = [wide(E, K, N) * 2 if layout == "kn" else wide(E, N, K).permute(0, 2, 1) for _ in range(2)]
+    kw = dict(total_rows=rows, b2=ws[1] if epi == _lib.EPI_SWIGLU else None, epilogue=epi)
+    gate = (torch.randn(rows, N, generator=g)).to(BF16).cuda()
+    if epi == _lib.EPI_GATED:
+        kw["gate"] = gate
+    args = (x, ws[0])
+    if layout == "fp8":
+        qx, sx = ops.quant_rows_fp8(x)
+        qw = [ops.quant_rows_fp8(w.permute(0, 2, 1)) for w in ws]
+        kw.update(a_scale=sx, b_scale=qw[0][1], scales_pow2=True)
+        if epi == _lib.EPI_SWIGLU:
+            kw.update(b2=qw[1][0].permute(0, 2, 1), b2_scale=qw[1][1])
+        args = (qx, qw[0][0].permute(0, 2, 1))
+        x = qx.float() / sx[:, None]
+        ws = [(q.float() / s[..., None]).permute(0, 2, 1) for q, s in qw]
+    assert ops.grouped_gemm(off, *args, plan_only=True, **kw) == _lib.PLAN_RING
+    out = ops.grouped_gemm(off, *args, **kw)
+    kw.pop("scales_pow2", None)
+    assert layout != "fp8" or torch.equal(ops.grouped_gemm(off, *args, **kw), out)      # scales divided out instead
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        a = x[lo:hi].double() @ ws[0][e].double()
+        if epi in (_lib.EPI_SILU, _lib.EPI_SWIGLU):
+            a = torch.nn.functional.silu(a)
+        if epi == _lib.EPI_SWIGLU:
+            a = a * (x[lo:hi].double() @ ws[1][e].double())
+        if epi == _lib.EPI_GATED:
+            a = a * torch.nn.functional.silu(gate[lo:hi].double())
+        assert_bf16_close(out[lo:hi], a.float(), rtol=1.6e-2, atol=4e-3, what=f"expert {e}")
