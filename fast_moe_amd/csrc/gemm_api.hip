@@ -156,6 +156,11 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
                       (!swiglu || aligned16(d->b2)) && (d->a_stride_row % chunk) == 0 &&
                       (d->a_stride_e % chunk) == 0 && (d->b_stride_n % chunk) == 0 &&
                       (d->b_stride_e % chunk) == 0;
+    // fp32 weights whose n is contiguous (every fp32 input gradient): chunks along n
+    const bool fast_n = f32 && !d->k_window && d->b_stride_n == 1 && d->b_stride_k != 1 && d->n >= 4 &&
+                        (d->k % chunk) == 0 && (d->n % chunk) == 0 && aligned16(d->a) && aligned16(d->b) &&
+                        (!swiglu || aligned16(d->b2)) && (d->a_stride_row % chunk) == 0 &&
+                        (d->a_stride_e % chunk) == 0 && (d->b_stride_k % chunk) == 0 && (d->b_stride_e % chunk) == 0;
     // rows per expert decide the tile height: tall tiles for prefill-like loads,
     // short ones when the experts see a handful of rows (weight-streaming regime)
     const bool big = d->total_rows / d->num_experts >= 96;
@@ -208,7 +213,7 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
         sel = kSelRing;
         return FMOE_OK;
     }
-    sel = ring_tr ? kSelRing : !fast ? kSelGeneric : take_ring ? kSelRing : big ? kSelStagedBig : kSelStagedSmall;
+    sel = ring_tr ? kSelRing : !fast && !fast_n ? kSelGeneric : take_ring ? kSelRing : big ? kSelStagedBig : kSelStagedSmall;
     return FMOE_OK;
 }
 

@@ -19,7 +19,7 @@
 //       weight stream does not stop at tile boundaries.
 //   grouped_gemm_kernel        register-staged, double-buffered LDS; serves everything the
 //       other two do not: arbitrary B strides and K / N tails (element loads), SiLU applied
-//       to A on load, fp32 operands.
+//       to A on load, fp32 operands (on tiles of their own, gemm_f32.hip).
 //
 // e4m3 row-wise scales that are exact powers of two (GemmParams::scale_pow2) are handed to
 // v_mfma_scale_f32_32x32x64_f8f6f4 as E8M0 codes of their reciprocals instead of being divided

@@ -37,11 +37,11 @@ int reserve_lds(Kern kern, int bytes, bool& done) {
     return FMOE_OK;
 }
 
-template <typename TL, int DT, int EPI, bool FAST, bool A_SILU>
+template <typename TL, int DT, int EPI, int LOADS, bool A_SILU>
 int launch_gemm(GemmParams p, hipStream_t stream) {
     constexpr int bn_out = EPI == FMOE_EPI_SWIGLU ? TL::BN / 2 : TL::BN;
     p.n_tiles = (p.N + bn_out - 1) / bn_out;
-    auto kern = grouped_gemm_kernel<TL, DT, EPI, FAST, A_SILU>;
+    auto kern = grouped_gemm_kernel<TL, DT, EPI, LOADS, A_SILU>;
     static bool attr_done = false;
     if (int rc = reserve_lds(kern, TL::LDS_BYTES, attr_done)) return rc;
     const int64_t max_m_tiles = p.total_rows / TL::BM + p.E;
@@ -166,7 +166,7 @@ int launch_ring(const GemmParams& p, hipStream_t stream) {
             if (pair_ok && window_ok && p.E <= TileRing5W::kMaxExperts)
                 return launch_ring_cfg<TileRing5W, FP8, EPI, false, true>(p, stream);
         }
-        return launch_gemm<TileBig, FP8 ? kDtE4m3 : kDtBf16, EPI, true, false>(p, stream);
+        return launch_gemm<TileBig, FP8 ? kDtE4m3 : kDtBf16, EPI, kLoadChunks, false>(p, stream);
     }
     if constexpr (FP8) {                   // power-of-two scales: applied by the MFMAs (row numbers fit 31 bits: pair_ok)
         if (p.scale_pow2 && pair_ok && p.E <= TileRing5::kMaxExperts)
@@ -184,17 +184,18 @@ int launch_ring(const GemmParams& p, hipStream_t stream) {
 
 template <int DT, int EPI, bool A_SILU>
 int dispatch_tile(const GemmParams& p, int sel, hipStream_t stream) {
+    static_assert(DT != kDtF32, "fp32 operands choose among tiles of their own (gemm_f32.hip)");
     switch (sel) {
         case kSelRing:
-            if constexpr (!A_SILU && DT != kDtF32) return launch_ring<DT == kDtE4m3, EPI>(p, stream);
-            else return launch_gemm<TileBig, DT, EPI, true, A_SILU>(p, stream);
-        case kSelStagedBig: return launch_gemm<TileBig, DT, EPI, true, A_SILU>(p, stream);
+            if constexpr (!A_SILU) return launch_ring<DT == kDtE4m3, EPI>(p, stream);
+            else return launch_gemm<TileBig, DT, EPI, kLoadChunks, A_SILU>(p, stream);
+        case kSelStagedBig: return launch_gemm<TileBig, DT, EPI, kLoadChunks, A_SILU>(p, stream);
         case kSelStagedSmall:
-            if constexpr (!A_SILU && DT != kDtF32 && EPI != FMOE_EPI_GATED) {
+            if constexpr (!A_SILU && EPI != FMOE_EPI_GATED) {
                 if (stream_kernel_takes(p)) return launch_stream<DT, EPI>(p, stream);
             }
-            return launch_gemm<TileSmall, DT, EPI, true, A_SILU>(p, stream);
-        default: return launch_gemm<TileSmall, DT, EPI, false, A_SILU>(p, stream);
+            return launch_gemm<TileSmall, DT, EPI, kLoadChunks, A_SILU>(p, stream);
+        default: return launch_gemm<TileSmall, DT, EPI, kLoadElements, A_SILU>(p, stream);
     }
 }
 

@@ -14,7 +14,7 @@ struct TileCfg {
     static constexpr int FM = TM / 32, FN = TN / 32;
     static constexpr int STAGE_BYTES = (BM + BN) * 128;
     static constexpr int LDS_BYTES = 2 * STAGE_BYTES;
-    static_assert(TM % 32 == 0 && TN % 64 == 0, "wave tile must hold whole 32x32 fragments, FN even");
+    static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile must hold whole 32x32 fragments");
     static_assert((BM * 8) % NT == 0 && (BN * 8) % NT == 0, "loader passes must be whole");
 };
 
@@ -22,13 +22,22 @@ __device__ __forceinline__ int lds_off(int row, int chunk) {     // 128-byte row
     return row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4);
 }
 
+enum { kLoadElements = 0, kLoadChunks = 1, kLoadChunksN = 2 };
+
 // DT: operand type, kDtBf16 / kDtE4m3 (bf16 output) or kDtF32 (fp32 operands, bias and output,
 // v_mfma_f32_32x32x2_f32: full fp32 products, no tf32).
-template <typename TL, int DT, int EPI, bool FAST, bool A_SILU>
+// LOADS: kLoadChunks 16-byte loads along k of both operands; kLoadChunksN (fp32) the same for A, and
+// 16-byte loads along n of weights whose n is contiguous, spread over four LDS rows as they are
+// parked (the fp32 MFMAs leave the LDS port idle nine tenths of the time); kLoadElements element
+// loads through any strides.
+template <typename TL, int DT, int EPI, int LOADS, bool A_SILU>
 __global__ __launch_bounds__(TL::NT) void grouped_gemm_kernel(const GemmParams p) {
     constexpr int BM = TL::BM, BN = TL::BN, NT = TL::NT;
     constexpr int FM = TL::FM, FN = TL::FN, TM = TL::TM, TN = TL::TN;
     constexpr bool FP8 = DT == kDtE4m3, F32 = DT == kDtF32;
+    constexpr bool FAST = LOADS != kLoadElements, NCONT = LOADS == kLoadChunksN;
+    static_assert(!NCONT || F32, "n-contiguous weights of 16-bit operands go to the ring kernel");
+    static_assert(EPI != FMOE_EPI_SWIGLU || FN % 2 == 0, "gate and up fragments come in pairs");
     constexpr int ESIZE = FP8 ? 1 : (F32 ? 4 : 2);
     constexpr int CHUNK_ELEMS = 16 / ESIZE;         // elements per 16-byte chunk
     constexpr int BK = 128 / ESIZE;                 // elements per K-slice
@@ -164,6 +173,17 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_kernel(const GemmParams p
 #pragma unroll
     for (int i = 0; i < WP; ++i) {
         int row, chunk;
+        if constexpr (NCONT) {      // unit q: columns 4 * (q % (BN/4)) .. + 3 of k = q / (BN/4)
+            const int q = tid + i * NT;
+            row = 4 * (q % (BN / 4));
+            const uint8_t* base;
+            int n = w_row_of(row, base);
+            n = n + 4 <= p.N ? n : p.N - 4;
+            wchunk[i] = q / (BN / 4);
+            wptr[i] = base + ((int64_t)expert * p.b_se + n + (k_begin + wchunk[i]) * p.b_sk) * ESIZE;
+            woff[i] = BM * 128 + (wchunk[i] & 3) * 4;
+            continue;
+        }
         if (FAST) { chunk = tid & 7; row = (tid >> 3) + i * (NT / 8); }
         else { const int q = tid + i * NT; row = q % BN; chunk = q / BN; }
         const uint8_t* base;
@@ -200,6 +220,11 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_kernel(const GemmParams p
         }
 #pragma unroll
         for (int i = 0; i < WP; ++i) {
+            if constexpr (NCONT) {
+                const uint8_t* src = wptr[i] + (int64_t)kt * BK * p.b_sk * ESIZE;
+                wr[i] = whole || kt * BK + wchunk[i] < Kdim ? *reinterpret_cast<const u32x4*>(src) : u32x4{0, 0, 0, 0};
+                continue;
+            }
             const int k = kt * BK + wchunk[i] * CHUNK_ELEMS;
             if (FAST) {
                 if (whole) wr[i] = *reinterpret_cast<const u32x4*>(wptr[i] + (int64_t)k * ESIZE);
@@ -227,7 +252,16 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_kernel(const GemmParams p
 #pragma unroll
         for (int i = 0; i < XP; ++i) *reinterpret_cast<u32x4*>(s + xoff[i]) = xr[i];
 #pragma unroll
-        for (int i = 0; i < WP; ++i) *reinterpret_cast<u32x4*>(s + woff[i]) = wr[i];
+        for (int i = 0; i < WP; ++i) {
+            if constexpr (NCONT) {
+                const int row = 4 * ((tid + i * NT) % (BN / 4));
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    *reinterpret_cast<uint32_t*>(s + woff[i] + lds_off(row + j, wchunk[i] >> 2)) = wr[i][j];
+            } else {
+                *reinterpret_cast<u32x4*>(s + woff[i]) = wr[i];
+            }
+        }
     };
 
     // ------------------------------------------------------------- main loop

@@ -1059,3 +1059,38 @@ def test_ring_kernel_contraction_tails(E, rows, K, N, layout, epi):
         if epi == _lib.EPI_GATED:
             a = a * torch.nn.functional.silu(gate[lo:hi].double())
         assert_bf16_close(out[lo:hi], a.float(), rtol=1.6e-2, atol=4e-3, what=f"expert {e}")
+
+
+@pytest.mark.parametrize("E,rows,K,N,layout,epi", [
+    (3, 190, 36, 68, "kn", 0), (3, 190, 36, 60, "nk", 0),       # below / above one 64-column tile, a rest of one chunk
+    (1, 64, 32, 64, "kn", 1), (1, 65, 4, 4, "kn", 0),           # whole tiles; one row more, the least K and N
+    (5, 700, 1000, 132, "kn", 2), (5, 700, 1000, 132, "nk", 2), # gate and up halves of a 128-column tile
+    (2, 2600, 100, 3500, "nk", 1), (2, 2600, 100, 3500, "kn", 1),   # enough tiles for the wide form (nk)
+    (70, 900, 68, 256, "kn", 0),                                # more experts than lanes, some empty
+])
+def test_fp32_kernel_tiles_and_weight_layouts(E, rows, K, N, layout, epi):
+    """fp32 tiles of 64 rows, weights with k or n contiguous.  The operands are the left columns of
+    wider tensors whose other columns are NaN.  Against float64; the bound of a K-term fp32 sum,
+    (K + 2) * 2^-24 * sum |a||b|, through SiLU (|slope| <= 1.1) and the product."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    g = torch.Generator().manual_seed(K + N + rows)
+    off = torch.tensor([0] + sorted(torch.randint(0, rows, (E - 1,), generator=g).tolist()) + [rows]).cuda()
+    def wide(*shape):
+        t = torch.full((*shape[:-1], shape[-1] + 4), float("nan"), device="cuda")
+        t[..., :shape[-1]] = torch.randn(*shape, generator=g).cuda()
+        return t[..., :shape[-1]]
+    x = wide(rows, K)
+    ws = [wide(E, K, N) if layout == "kn" else wide(E, N, K).permute(0, 2, 1) for _ in range(2)]
+    kw = dict(total_rows=rows, b2=ws[1] if epi == _lib.EPI_SWIGLU else None, epilogue=epi)
+    assert ops.grouped_gemm(off, x, ws[0], plan_only=True, **kw) != _lib.PLAN_ELEMENT
+    out = ops.grouped_gemm(off, x, ws[0], **kw)
+    unit = (K + 2) * 2.0 ** -24
+    for e in range(E):
+        a = x[int(off[e]):int(off[e + 1])].double()
+        want, err = a @ ws[0][e].double(), unit * (a.abs() @ ws[0][e].double().abs())
+        if epi != _lib.EPI_NONE:
+            want, err = torch.nn.functional.silu(want), 1.1 * err + 2.0 ** -21 * want.abs()
+        if epi == _lib.EPI_SWIGLU:
+            up, up_err = a @ ws[1][e].double(), unit * (a.abs() @ ws[1][e].double().abs())
+            want, err = want * up, err * up.abs() + (want.abs() + err) * up_err + 2.0 ** -23 * (want * up).abs()
+        assert bool(((out[int(off[e]):int(off[e + 1])].double() - want).abs() <= err).all()), f"expert {e}"
