@@ -18,7 +18,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libfastmoe_hip.so")
 OBJ_DIR = os.path.join(CSRC, "build")
 
-SOURCES = ["gemm_bf16.hip", "gemm_fp8.hip", "gemm_bf16_tail.hip", "gemm_fp8_tail.hip", "gemm_f32.hip", "gemm_api.hip",
+SOURCES = ["gemm_bf16.hip", "gemm_fp8.hip", "gemm_bf16_tail.hip", "gemm_fp8_tail.hip", "gemm_bf16_short.hip", "gemm_fp8_short.hip",
+           "gemm_f32.hip", "gemm_api.hip",
            "core.hip", "routing.hip", "quant.hip", "combine.hip", "backward.hip"]
 
 HIPCC_FLAGS = [

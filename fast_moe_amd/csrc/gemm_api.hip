@@ -183,6 +183,16 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
                          d->total_rows < ((int64_t)1 << 31) && lds_per_block() >= TileRing5::LDS_BYTES &&
                          d->a_rows * d->a_stride_row * esize + (int64_t)ktot * esize < span32 &&
                          ((int64_t)ktot * d->b_stride_k + d->n) * esize < span32;
+    // experts with few rows: the ring on 64-row tiles, weights with k or n contiguous
+    const bool near_tr = d->a_rows * d->a_stride_row * esize + (int64_t)ktot * esize < span32 &&
+                         ((int64_t)ktot * d->b_stride_k + d->n) * esize < span32;
+    const bool short_ok = !big && !f32 && !d->a_silu && !d->k_window && !two && !row_indexed && p.vec_store &&
+                          ring_short_takes(esize, d->k, d->num_experts, d->total_rows);
+    const bool short_tr = short_ok && !fp8 && d->b_stride_n == 1 && d->b_stride_k != 1 && (d->b_stride_k % chunk) == 0 &&
+                          (d->b_stride_e % chunk) == 0 && (d->a_stride_row % chunk) == 0 &&
+                          (d->a_stride_e % chunk) == 0 && aligned16(d->a) && aligned16(d->b) &&
+                          (!swiglu || aligned16(d->b2)) && near_tr;
+    p.ring_short = short_tr || (short_ok && fast && near);
     // the second product exists in that kernel only; a caller that is turned away runs two
     // GEMMs and adds
     if (two)
@@ -213,7 +223,7 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
         sel = kSelRing;
         return FMOE_OK;
     }
-    sel = ring_tr ? kSelRing : !fast && !fast_n ? kSelGeneric : take_ring ? kSelRing : big ? kSelStagedBig : kSelStagedSmall;
+    sel = ring_tr ? kSelRing : !fast && !fast_n && !p.ring_short ? kSelGeneric : take_ring ? kSelRing : big ? kSelStagedBig : kSelStagedSmall;
     return FMOE_OK;
 }
 

@@ -1,0 +1,28 @@
+// bf16 ring kernels on 64-row tiles: experts with a handful of rows.
+#include "gemm_kernel.h"
+
+namespace fmoe {
+
+template <int EPI, bool KTAIL>
+static int launch(const GemmParams& p, hipStream_t stream) {
+    if (p.b_sn == 1 && p.b_sk != 1)
+        return launch_ring_cfg<TileRingS, false, EPI, true, false, false, false, KTAIL>(p, stream);
+    return launch_ring_cfg<TileRingS, false, EPI, false, false, false, false, KTAIL>(p, stream);
+}
+
+template <int EPI>
+static int launch(const GemmParams& p, hipStream_t stream) {
+    return p.K % 64 ? launch<EPI, true>(p, stream) : launch<EPI, false>(p, stream);
+}
+
+int run_ring_short_bf16(const GemmParams& p, int epilogue, hipStream_t stream) {
+    switch (epilogue) {
+        case FMOE_EPI_NONE: return launch<FMOE_EPI_NONE>(p, stream);
+        case FMOE_EPI_SILU: return launch<FMOE_EPI_SILU>(p, stream);
+        case FMOE_EPI_SWIGLU: return launch<FMOE_EPI_SWIGLU>(p, stream);
+        case FMOE_EPI_GATED: return launch<FMOE_EPI_GATED>(p, stream);
+    }
+    return fail(FMOE_ERR_ARGUMENT, "fmoe_grouped_gemm: unknown epilogue %d", epilogue);
+}
+
+}  // namespace fmoe

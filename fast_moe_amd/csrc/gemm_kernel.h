@@ -11,7 +11,9 @@
 //       the current tile's epilogue stores drain.  With few experts the ring takes all of
 //       LDS (5 slots), slices are fetched in pairs as full 128-byte lines and the K loop is
 //       a software pipeline of 8-MFMA blocks (see RingCfg); otherwise 4 slots, one slice at
-//       a time, schedule tables in LDS.
+//       a time, schedule tables in LDS.  With few rows per expert the same kernel runs 64 x 256
+//       tiles of 4 wavefronts on seven slots of 20 KB (TileRingS): weights with n contiguous, and
+//       weights with k contiguous where ring_short_pays says so.
 //   grouped_gemm_stream_kernel experts with a handful of rows (the weights are streamed once
 //       and that stream is the cost).  Persistent 64 x 256 tiles, 4 wavefronts, two blocks per
 //       CU; a K-slice travels global -> registers -> LDS while the previous one is multiplied,

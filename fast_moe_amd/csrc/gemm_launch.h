@@ -22,6 +22,7 @@ typedef TileRing5 TileRing5F;
 #endif
 typedef RingCfg<256, 256, 2, 4, 2> TileRing5M;  // 5-slot ring, paired slices, E <= 128 (the plain forward calls)
 typedef RingCfg<256, 256, 2, 4, 4> TileRing5W;  // 5-slot ring, paired slices, E <= 256
+typedef RingCfg<64, 256, 1, 4, 4, 3> TileRingS; // 4 waves, wave tile 64 x 64, 7 slots of 20 KB, E <= 256
 
 enum GemmKernelSel { kSelRing = 0, kSelStagedBig = 1, kSelStagedSmall = 2, kSelGeneric = 3 };
 
@@ -61,7 +62,7 @@ int lds_per_block();   // largest LDS allocation of one block on the current dev
 
 // the streaming kernel takes what the 64-row register-staged kernel takes with 16-byte loads, when
 // the output can be stored 16 bytes at a time and no contraction window is set
-inline bool stream_kernel_takes(const GemmParams& p) { return p.vec_store && !p.k_window; }
+inline bool stream_kernel_takes(const GemmParams& p) { return p.vec_store && !p.k_window && p.b_sk == 1; }
 
 template <int DT, int EPI>
 int launch_stream(GemmParams p, hipStream_t stream) {
@@ -115,6 +116,10 @@ int launch_ring_cfg(GemmParams p, hipStream_t stream) {
     // the XCD count so that every XCD owns the same number of blocks
     int grid = compute_units() / kNumXcd * kNumXcd;
     if (grid < kNumXcd) grid = kNumXcd;
+    if (TL::BM < 256) {     // few rows: often fewer tiles than CUs
+        const int64_t need = ((p.total_rows / TL::BM + p.E) * p.n_tiles + kNumXcd - 1) / kNumXcd * kNumXcd;
+        if (need < grid) grid = (int)need;
+    }
     kern<<<(unsigned)grid, TL::NT, TL::LDS_BYTES, stream>>>(p);
     return check_launch("fmoe_grouped_gemm");
 }
@@ -131,6 +136,35 @@ inline bool ring_tail_takes(int esize, int64_t k, int num_experts, int64_t total
     const int pair = 128 / esize, chunk = 16 / esize;
     return k > pair && k % pair != 0 && k % chunk == 0 && num_experts <= TileRing5W::kMaxExperts &&
            total_rows < ((int64_t)1 << 31) && lds_per_block() >= TileRing5W::LDS_BYTES;
+}
+
+// The ring on 64-row tiles (gemm_bf16_short.hip, gemm_fp8_short.hip): experts with a handful of rows.
+int run_ring_short_bf16(const GemmParams& p, int epilogue, hipStream_t stream);
+int run_ring_short_fp8(const GemmParams& p, int epilogue, hipStream_t stream);
+
+inline bool ring_short_takes(int esize, int64_t k, int num_experts, int64_t total_rows) {
+    const int pair = 128 / esize, chunk = 16 / esize;
+    return k > (TileRingS::AHEAD - 1) * pair && k % chunk == 0 && num_experts <= TileRingS::kMaxExperts &&
+           total_rows < ((int64_t)1 << 31) && lds_per_block() >= TileRingS::LDS_BYTES;
+}
+
+// Where both take a call (weights with k contiguous).  Both read large launches at 5.9 - 6.0 TB/s (a read loop without
+// anything else gets 6.3 on this access pattern); they differ where a launch is a round or two of tiles, and in the cost of
+// a tile boundary.  us per GEMM, streaming kernel / ring:
+//   * up to one tile per CU the ring keeps 120 KB per CU in flight where a lone streaming block has 40:
+//     138 rows, 32 experts, 1728 -> 2 x 576 SwiGLU  30.2 / 22.5 (e4m3 19.5 / 16.6); 162 rows, 21 experts, 3648 -> 576  49.9 / 30.1
+//   * above that the streaming kernel's two blocks per CU leave fewer CUs without a tile in the last round:
+//     1000 rows, 63 experts, 1792 -> 2 x 640  52.4 / 61.4 (e4m3 28.1 / 32.7)
+//   * with many rounds that is gone; the ring is ahead where a weight row is 4 KB or longer (3000 rows, 64 experts,
+//     2048 -> 2 x 1408  143.7 / 136.9; 8000 rows, 128 experts, 4096 -> 2 x 1536  689 / 673, e4m3 378 / 362), behind where
+//     tiles are shorter (4096 rows, 128 experts, 1536 -> 4096  298.6 / 304.5; e4m3 158 / 163).
+template <int DT, int EPI>
+bool ring_short_pays(const GemmParams& p) {
+    constexpr int bn_out = EPI == FMOE_EPI_SWIGLU ? TileRingS::BN / 2 : TileRingS::BN;
+    const int64_t experts = p.E < p.total_rows ? p.E : p.total_rows;       // that can hold a row
+    const int64_t tiles = (p.total_rows / TileRingS::BM + experts) * ((p.N + bn_out - 1) / bn_out);
+    const int64_t cus = compute_units();
+    return tiles <= cus || (tiles > 3 * cus && (int64_t)p.K * (DT == kDtE4m3 ? 1 : 2) >= 4096);
 }
 
 // The 5-slot ring needs every byte of a 160 KB LDS, an even number of K-slices per tile,
@@ -191,6 +225,10 @@ int dispatch_tile(const GemmParams& p, int sel, hipStream_t stream) {
             else return launch_gemm<TileBig, DT, EPI, kLoadChunks, A_SILU>(p, stream);
         case kSelStagedBig: return launch_gemm<TileBig, DT, EPI, kLoadChunks, A_SILU>(p, stream);
         case kSelStagedSmall:
+            if constexpr (!A_SILU) {
+                if (p.ring_short && (EPI == FMOE_EPI_GATED || !stream_kernel_takes(p) || ring_short_pays<DT, EPI>(p)))
+                    return DT == kDtE4m3 ? run_ring_short_fp8(p, EPI, stream) : run_ring_short_bf16(p, EPI, stream);
+            }
             if constexpr (!A_SILU && EPI != FMOE_EPI_GATED) {
                 if (stream_kernel_takes(p)) return launch_stream<DT, EPI>(p, stream);
             }

@@ -7,15 +7,17 @@ namespace fmoe {
 
 // --------------------------------------------------------------------- ring kernel
 // NREG_ == 0: 4 slots, one K-slice issued per step, schedule tables in LDS (E <= 1024).
-// NREG_  > 0: 5 slots (all 160 KB of LDS), K-slices issued in pairs so that the two
+// NREG_  > 0: 2 * AHEAD_ + 1 slots (5 of 32 KB: all of LDS), K-slices issued in pairs so that the two
 //             instructions touching the halves of a 128-byte line are adjacent and reach L2
 //             as one full-line request; the schedule tables live in 3 * NREG_ registers of
 //             every wave (E <= 64 * NREG_, total_rows < 2^31, K-slices per tile even).
-template <int BM_, int BN_, int WGM_, int WGN_, int NREG_>
+// AHEAD_: pairs of K-slices in flight ahead of the one being multiplied (2 * AHEAD_ + 1 slots).
+template <int BM_, int BN_, int WGM_, int WGN_, int NREG_, int AHEAD_ = 2>
 struct RingCfg {
     static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NREG = NREG_;
     static constexpr bool PAIR = NREG_ > 0;
-    static constexpr int STAGES = PAIR ? 5 : 4;
+    static constexpr int AHEAD = AHEAD_;
+    static constexpr int STAGES = PAIR ? 2 * AHEAD + 1 : 4;
     static constexpr int NW = WGM * WGN;
     static constexpr int NT = kWave * NW;
     static constexpr int TM = BM / WGM, TN = BN / WGN;
@@ -92,8 +94,7 @@ template <typename TL, bool FP8, int EPI, bool WTR = false, bool KWIN = false, b
           bool KTAIL = false>
 __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmParams p) {
     static_assert(!MSC || (FP8 && TL::PAIR && !KWIN && !WTR && !XTR), "MFMA-applied scales: e4m3 on the paired ring");
-    static_assert(!WTR || (TL::PAIR && !FP8 && TL::BN == 256 && TL::NW == 8),
-                  "in-place N-contiguous weights: bf16, paired ring, 256-column tiles of 8 waves");
+    static_assert(!WTR || (TL::PAIR && !FP8 && TL::BN == 256), "in-place N-contiguous weights: bf16, paired ring, 256-column tiles");
     static_assert(!KWIN || TL::PAIR, "contraction windows: paired ring");
     static_assert(!KTAIL || (TL::PAIR && !KWIN && !XTR), "K tails: paired ring without windows");
     static_assert(XTR ? (WTR && KWIN && TL::BM == 256 && EPI == FMOE_EPI_NONE) : !(KWIN && WTR),
@@ -241,7 +242,8 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     const int xcd = blockIdx.x % kNumXcd, slot = blockIdx.x / kNumXcd;
     const int64_t group_span = (int64_t)kGroupM * p.n_tiles;
     constexpr bool windowed = KWIN;
-    constexpr bool deal_groups = PAIR;
+    // (BM = 64: a launch is a stream of weights with little to share and often has no 8 groups)
+    constexpr bool deal_groups = PAIR && BM >= 256;
     int64_t xcd_begin, xcd_count;
     if (deal_groups) {
         const int64_t n_groups = (total_m + kGroupM - 1) / kGroupM;
@@ -447,12 +449,14 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         for (int i = 0; i < WI; ++i) {
             const bool up = SWIGLU && i * NW * 16 >= BN / 2;
             if constexpr (WTR) {
-                // instruction i of this wave: rows 4*wave + lane/16 of column block i, LDS position lane%16
+                // instruction i of this wave is the slot's transfer q = i * NW + wave: k rows 4*(q%8) + lane/16
+                // of column block q/8, LDS position lane%16
                 int l = lane;
                 asm volatile("" : "+v"(l));
-                const int kr = 4 * wave + (l >> 4);
+                const int q = i * NW + wave;
+                const int kr = 4 * (q & 7) + (l >> 4);
                 const int c = (l & 15) ^ (4 * (l >> 4));
-                int n = n0 + (SWIGLU ? 0 : i * (BN / 2)) + 8 * c;
+                int n = n0 + (SWIGLU ? 0 : (q >> 3) * (BN / 2)) + 8 * c;
                 n = n + 8 <= p.N ? n : p.N - 8;
                 wbase[i] = (up ? p.b2 : p.b) + ((int64_t)expert * p.b_se + k_begin * p.b_sk) * ESIZE;
                 woff[i] = (uint32_t)(((int64_t)kr * p.b_sk + n) * ESIZE);
@@ -578,7 +582,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             uint32_t x = 0, w = 0x7f7f7f7fu;
 #pragma unroll
             for (int fm = 0; fm < FM; ++fm) x |= e8m0_of_reciprocal(sc_xraw[fm]) << (8 * fm);
-            static_assert(FM == 4 && FN <= 4, "one byte per row block / weight fragment");
+            static_assert(FM <= 4 && FN <= 4, "one byte per row block / weight fragment");
 #pragma unroll
             for (int fn = 0; fn < FN; ++fn) w = (w & ~(0xffu << (8 * fn))) | (e8m0_of_reciprocal(sc_wraw[fn]) << (8 * fn));
             sc_x = x;
@@ -589,7 +593,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     if (slot >= xcd_count) return;
     const int my_tiles = (int)((xcd_count - slot + nslots - 1) / nslots);
     // 4-slot ring: every item of the block; paired ring: issue_next only starts the first tile
-    const int total_items = PAIR ? 4 : my_tiles * KT;
+    const int total_items = PAIR ? 2 * TL::AHEAD : my_tiles * KT;
 
     // The block's work is one flat stream of K-slices ("items"): KT per tile, tile after
     // tile.  Item i lives in ring slot i % STAGES.  The issue side runs ahead of the compute
@@ -673,8 +677,8 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     prefetch_next();
     rows_to_offsets(ridx_next, xoff_next);
     if (PAIR) {
-        issue_next();                       // items 0..3
-        issue_next();
+#pragma unroll
+        for (int j = 0; j < TL::AHEAD; ++j) issue_next();     // items 0 .. 2 * AHEAD - 1
     } else {
         for (int j = 0; j < STAGES - 1; ++j) issue_next();
     }
@@ -881,7 +885,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 interleave();
                 __builtin_amdgcn_sched_barrier(0);
                 barrier();                  // B
-                part_a = lds_base + islot * TL::STAGE_BYTES;    // pair (c+4, c+5)
+                part_a = lds_base + islot * TL::STAGE_BYTES;    // pair (c + 2 * AHEAD, + 1)
                 islot = islot + 1 == STAGES ? 0 : islot + 1;
                 part_b = lds_base + islot * TL::STAGE_BYTES;
                 islot = islot + 1 == STAGES ? 0 : islot + 1;
@@ -901,10 +905,11 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 mma_block(wfa, xfa, std::integral_constant<bool, HALF == 0>{}, act_c);
                 if constexpr (HALF != 0) interleave();
                 __builtin_amdgcn_sched_barrier(0);
-                // pair (c+2, c+3) is older than the 2L instructions the first half just issued
+                // pair (c+2, c+3) is older than the other pairs in flight, 2L instructions each, the one the
+                // first half just issued among them
                 if (!skip_wait) {
-                    if (HALF == 0) wait_vmcnt<2 * L>();
-                    else wait_vmcnt<0>();
+                    if (HALF == 0) wait_vmcnt<2 * L * (TL::AHEAD - 1)>();
+                    else wait_vmcnt<2 * L * (TL::AHEAD - 2)>();
                 }
                 barrier();                  // A'
                 if (!LAST) load_block(wfa, xfa, s2, 0, kitem + 2, mask_c, act_c);
@@ -915,12 +920,12 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 cslot = s2;
                 kitem += 2;
             };
-            // the issue side runs 4 items ahead: it enters the next tile 4 items before the end;
+            // the issue side runs 2 * AHEAD items ahead: it enters the next tile that many items before the end;
             // the last two double steps hold the end of an XTR tile's window and mask it
             auto tile_steps = [&](auto half_c, auto act_c) __attribute__((always_inline)) {
                 const int tile_kt = KWIN ? cur.kt : KT;
                 bool landed = tile_i > 0;       // the first step's pair landed before the previous epilogue's stores
-                for (int kt = 0; kt < tile_kt - 4; kt += 2) {
+                for (int kt = 0; kt < tile_kt - 2 * TL::AHEAD; kt += 2) {
                     double_step(half_c, std::false_type{}, std::false_type{}, act_c, landed);
                     landed = false;
 #ifdef FMOE_TRACE
@@ -930,12 +935,17 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 FMOE_TRACE_STAMP(10);
                 enter_next();
                 ikt = 0;
+#pragma unroll
+                for (int j = 2; j < TL::AHEAD; ++j) {
+                    double_step(half_c, std::false_type{}, std::false_type{}, act_c, landed);
+                    landed = false;
+                }
                 double_step(half_c, std::false_type{}, std::true_type{}, act_c, landed);
                 FMOE_TRACE_STAMP(11);
                 double_step(half_c, std::true_type{}, std::true_type{}, act_c, false);
             };
             if (tile_i == 0) {              // pair 0 has landed everywhere
-                wait_vmcnt<2 * L>();
+                wait_vmcnt<2 * L * (TL::AHEAD - 1)>();
                 barrier();
             }
             load_block(wfa, xfa, cslot, 0, 0, std::true_type{}, std::integral_constant<int, FM>{});
@@ -1003,11 +1013,12 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                     if constexpr (MSC) {
                         // (the byte selectors are immediates of the instruction: after unrolling fn and
                         // fm are constants and one of the four forms is left)
-                        static_assert(FN == 2 && HM == 2, "selector forms below");
+                        static_assert(FN == 2 && HM <= 2, "selector forms below");
+                        constexpr int M1 = HM - 1;
                         if (fn == 0 && fm == 0) mfma_e4m3_scaled<0, FM0>(wf[0], xh[0], acc[0][FM0], sc_w, sc_x);
-                        else if (fn == 0) mfma_e4m3_scaled<0, FM0 + 1>(wf[0], xh[1], acc[0][FM0 + 1], sc_w, sc_x);
+                        else if (fn == 0) mfma_e4m3_scaled<0, FM0 + M1>(wf[0], xh[M1], acc[0][FM0 + M1], sc_w, sc_x);
                         else if (fm == 0) mfma_e4m3_scaled<1, FM0>(wf[1], xh[0], acc[1][FM0], sc_w, sc_x);
-                        else mfma_e4m3_scaled<1, FM0 + 1>(wf[1], xh[1], acc[1][FM0 + 1], sc_w, sc_x);
+                        else mfma_e4m3_scaled<1, FM0 + M1>(wf[1], xh[M1], acc[1][FM0 + M1], sc_w, sc_x);
                     } else {
                         acc[fn][FM0 + fm] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
                             wf[fn], xh[fm], acc[fn][FM0 + fm], 0, 0, 0, 0, 0, 0);
@@ -1057,7 +1068,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 mma_block(qwa, qx1, std::integral_constant<int, HM>{}, std::false_type{}, sparse_c);
                 __builtin_amdgcn_sched_barrier(0);
                 barrier();                  // B
-                part_a = lds_base + islot * TL::STAGE_BYTES;    // pair (c+4, c+5)
+                part_a = lds_base + islot * TL::STAGE_BYTES;    // pair (c + 2 * AHEAD, + 1)
                 islot = islot + 1 == STAGES ? 0 : islot + 1;
                 part_b = lds_base + islot * TL::STAGE_BYTES;
                 islot = islot + 1 == STAGES ? 0 : islot + 1;
@@ -1082,8 +1093,8 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 mma_block(qwb, qx0, std::integral_constant<int, 0>{}, std::integral_constant<bool, HALF == 0>{}, full);
                 __builtin_amdgcn_sched_barrier(0);
                 if (!skip_wait) {
-                    if (HALF == 0) wait_vmcnt<2 * L>();
-                    else wait_vmcnt<0>();
+                    if (HALF == 0) wait_vmcnt<2 * L * (TL::AHEAD - 1)>();
+                    else wait_vmcnt<2 * L * (TL::AHEAD - 2)>();
                 }
                 barrier();                  // A'
                 if (!LAST) load_w_x0(qwa, qx0, s2);
@@ -1099,7 +1110,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 // the epilogue's end: left pending, such a wait lands inside this loop, where it
                 // drains the LDS-DMA stream, which the compiler cannot see, on every iteration)
                 bool landed = tile_i > 0;
-                for (int kt = 0; kt < tile_kt - 4; kt += 2) {
+                for (int kt = 0; kt < tile_kt - 2 * TL::AHEAD; kt += 2) {
                     double_step(half_c, std::false_type{}, sparse_c, landed);
                     landed = false;
 #ifdef FMOE_TRACE
@@ -1109,12 +1120,17 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 FMOE_TRACE_STAMP(10);
                 enter_next();
                 ikt = 0;
+#pragma unroll
+                for (int j = 2; j < TL::AHEAD; ++j) {
+                    double_step(half_c, std::false_type{}, sparse_c, landed);
+                    landed = false;
+                }
                 double_step(half_c, std::false_type{}, sparse_c, landed);
                 FMOE_TRACE_STAMP(11);
                 double_step(half_c, std::true_type{}, sparse_c, false);
             };
             if (tile_i == 0) {              // pair 0 has landed everywhere
-                wait_vmcnt<2 * L>();
+                wait_vmcnt<2 * L * (TL::AHEAD - 1)>();
                 barrier();
             }
             load_w_x0(qwa, qx0, cslot);

@@ -1094,3 +1094,54 @@ def test_fp32_kernel_tiles_and_weight_layouts(E, rows, K, N, layout, epi):
             up, up_err = a @ ws[1][e].double(), unit * (a.abs() @ ws[1][e].double().abs())
             want, err = want * up, err * up.abs() + (want.abs() + err) * up_err + 2.0 ** -23 * (want * up).abs()
         assert bool(((out[int(off[e]):int(off[e + 1])].double() - want).abs() <= err).all()), f"expert {e}"
+
+
+@pytest.mark.parametrize("E,rows,K,N,layout,epi", [
+    (3, 130, 136, 264, "nk", 0), (3, 130, 192, 136, "kn", 0),       # the least K: three pairs of K-slices, the last in part / whole
+    (1, 64, 256, 256, "kn", 1), (1, 65, 256, 256, "nk", 1),         # one whole tile; one row more
+    (2, 3, 1000, 520, "nk", 2), (2, 3, 1000, 520, "kn", 2),
+    (200, 900, 328, 72, "kn", 0), (130, 5000, 264, 1032, "kn", 2),  # more experts than lanes; more tiles than CUs
+    (2, 150, 200, 320, "kn", 3), (40, 2000, 640, 2048, "kn", 3),
+    (3, 130, 272, 264, "fp8", 0), (3, 70, 384, 136, "fp8", 2), (8, 760, 4096, 10400, "fp8", 0),
+])
+def test_ring_kernel_on_short_tiles(E, rows, K, N, layout, epi):
+    """The ring on 64-row tiles (few rows per expert).  The operands are the left columns of wider
+    tensors whose other columns are NaN.  Against float64 on the GPU; roundings as in
+    test_ring_kernel_contraction_tails."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    off = torch.tensor([0] + sorted(torch.randint(0, rows, (E - 1,), generator=g, device="cuda").tolist()) + [rows]).cuda()
+    def wide(*shape):
+        t = torch.full((*shape[:-1], shape[-1] + 16), float("nan"), dtype=BF16, device="cuda")
+        t[..., :shape[-1]] = (torch.randn(*shape, generator=g, device="cuda") * shape[-1] ** -0.5).to(BF16)
+        return t[..., :shape[-1]]
+    x = wide(rows, K)
+    ws = [wide(E, K, N) if layout == "kn" else wide(E, N, K).permute(0, 2, 1) for _ in range(2)]
+    kw = dict(total_rows=rows, b2=ws[1] if epi == _lib.EPI_SWIGLU else None, epilogue=epi)
+    gate = torch.randn(rows, N, generator=g, device="cuda").to(BF16)
+    if epi == _lib.EPI_GATED:
+        kw["gate"] = gate
+    args = (x, ws[0])
+    if layout == "fp8":
+        qx, sx = ops.quant_rows_fp8(x)
+        qw = [ops.quant_rows_fp8(w.permute(0, 2, 1)) for w in ws]
+        kw.update(a_scale=sx, b_scale=qw[0][1], scales_pow2=True)
+        if epi == _lib.EPI_SWIGLU:
+            kw.update(b2=qw[1][0].permute(0, 2, 1), b2_scale=qw[1][1])
+        args = (qx, qw[0][0].permute(0, 2, 1))
+        x = qx.float() / sx[:, None]
+        ws = [(q.float() / s[..., None]).permute(0, 2, 1) for q, s in qw]
+    assert ops.grouped_gemm(off, *args, plan_only=True, **kw) == _lib.PLAN_STAGED_SHORT
+    out = ops.grouped_gemm(off, *args, **kw)
+    kw.pop("scales_pow2", None)
+    assert layout != "fp8" or torch.equal(ops.grouped_gemm(off, *args, **kw), out)      # scales divided out instead
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        a = x[lo:hi].double() @ ws[0][e].double()
+        if epi in (_lib.EPI_SILU, _lib.EPI_SWIGLU):
+            a = torch.nn.functional.silu(a)
+        if epi == _lib.EPI_SWIGLU:
+            a = a * (x[lo:hi].double() @ ws[1][e].double())
+        if epi == _lib.EPI_GATED:
+            a = a * torch.nn.functional.silu(gate[lo:hi].double())
+        assert_bf16_close(out[lo:hi], a.float(), rtol=1.6e-2, atol=4e-3, what=f"expert {e}")
