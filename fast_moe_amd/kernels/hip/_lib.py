@@ -24,7 +24,8 @@ EXPORTED_SYMBOLS = (
     "fmoe_quant_rows_workspace_bytes", "fmoe_quant_rows_e4m3_ws", "fmoe_grouped_gemm", "fmoe_grouped_gemm_plan",
     "fmoe_combine",
     "fmoe_silu_mul", "fmoe_transpose_last2", "fmoe_jagged_transpose", "fmoe_segment_colsum",
-    "fmoe_swiglu_bwd", "fmoe_combine_bwd", "fmoe_gather_rows", "fmoe_route_topk_static", "fmoe_hbm_probe",
+    "fmoe_swiglu_bwd", "fmoe_combine_bwd", "fmoe_gather_rows", "fmoe_invert_index",
+    "fmoe_gate_l1_bwd", "fmoe_route_topk_static", "fmoe_hbm_probe",
 )
 ROUTE_STATIC_MAX_POSITIONS, ROUTE_STATIC_MAX_EXPERTS = 1 << 20, 512
 
@@ -116,6 +117,10 @@ def load() -> ctypes.CDLL:
     lib.fmoe_combine_bwd.argtypes = [c_void_p, c_void_p, c_int, c_int64, c_int, c_int64, c_int64, c_void_p,
                                      c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
                                      c_void_p]
+    lib.fmoe_invert_index.restype = c_int
+    lib.fmoe_invert_index.argtypes = [c_void_p, c_int64, c_int, c_void_p, c_void_p]
+    lib.fmoe_gate_l1_bwd.restype = c_int
+    lib.fmoe_gate_l1_bwd.argtypes = [c_void_p, c_int, c_int64, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]
     lib.fmoe_hbm_probe.restype = c_int
     lib.fmoe_hbm_probe.argtypes = [c_void_p, c_int64, c_int, c_int, c_void_p]
     _lib = lib

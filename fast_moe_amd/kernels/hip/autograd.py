@@ -47,16 +47,6 @@ def _pad_layout(offsets: torch.Tensor, total_rows: int) -> Tuple[torch.Tensor, i
     return pad_offsets, bound
 
 
-def _reverse_from_index(index: torch.Tensor) -> torch.Tensor:
-    """index [T, K] (sorted position -> flat token*K+slot) -> [T, K] sorted positions of each
-    token's rows, ascending (the order a sequential index_add meets them in)."""
-    T, K = index.shape
-    flat = index.reshape(-1)
-    inv = torch.empty_like(flat)
-    inv[flat] = torch.arange(flat.numel(), device=flat.device, dtype=flat.dtype)
-    return inv.view(T, K).sort(dim=1).values
-
-
 class _WgradOperand:
     """The input rows of the routed rows as the weight-gradient GEMM wants them, shared by the
     weight gradients of every weight that multiplied the same input (SwiGLU's gate and up
@@ -167,7 +157,7 @@ class IndexSelectJaggedBmm(torch.autograd.Function):
         need = ctx.needs_input_grad
         d_jagged = d_w = d_b = d_wp = d_bp = None
         if need[2]:
-            d_jagged = _input_grad(drows, weights, offsets, _reverse_from_index(index)).view_as(jagged)
+            d_jagged = _input_grad(drows, weights, offsets, ops.invert_index(index)).view_as(jagged)
         operand = None
         if need[3] or (swiglu and need[5]):
             operand = _WgradOperand(jagged, offsets, R, row_index=index.reshape(-1), index_div=K)
@@ -229,7 +219,7 @@ class IndexSelectJaggedBmmFp8(torch.autograd.Function):
                 w_rows = ops.to_k_contiguous(weight.permute(0, 2, 1)).permute(0, 2, 1)
             qw, sw = ops.quant_rows_fp8(w_rows)                         # [E, Kin, N], [E, Kin]
             d_rows = ops.grouped_gemm(offsets, qd, qw.permute(0, 2, 1), total_rows=R, scales_pow2=True, a_scale=sd, b_scale=sw)
-            d_jagged = ops.combine(d_rows, _reverse_from_index(index)).view_as(jagged)
+            d_jagged = ops.combine(d_rows, ops.invert_index(index)).view_as(jagged)
         if need[3]:
             pad_offsets, bound = _pad_layout(offsets, R)
             a_t = ops.jagged_transpose(jagged, offsets, pad_offsets, bound, index.reshape(-1), K)   # [Kin, bound]
@@ -272,7 +262,7 @@ class IndexSelectJaggedGatingBmm(torch.autograd.Function):
         R, K = index.numel(), index.shape[-1]
         d_a, d_b = ops.swiglu_bwd(pre_a, pre_b, dout.contiguous())
         need = ctx.needs_input_grad
-        reverse = _reverse_from_index(index) if need[2] or need[3] else None
+        reverse = ops.invert_index(index) if need[2] or need[3] else None
         grads = []
         for pos, (src, w, bias, d) in enumerate(((jagged_a, weight_a, bias_a, d_a), (jagged_b, weight_b, bias_b, d_b))):
             d_src = d_w = d_bias = None
@@ -320,7 +310,7 @@ class IndexSelectJaggedBmm3D(torch.autograd.Function):
             # Gather form instead: slot j of cell (l, e) names the j-th routed row of token l if
             # that row went to expert e, else nothing; the merge kernel adds a cell's rows in
             # ascending order in fp32 and writes zeros where there are none.
-            rows_of_token = _reverse_from_index(index)                                  # [L, K] ascending
+            rows_of_token = ops.invert_index(index)                                  # [L, K] ascending
             experts_of = expert[rows_of_token]                                          # [L, K]
             here = experts_of[:, None, :] == torch.arange(E, device=index.device)[None, :, None]
             slots = torch.where(here, rows_of_token[:, None, :], rows_of_token.new_full((), -1))
@@ -414,6 +404,42 @@ class SiluJaggedBmmCombine(torch.autograd.Function):
         if need_g:
             d_g = d_gate.view(gating_scores.shape).to(gating_scores.dtype)
         return None, d_jagged, d_w, d_b, None, None, d_g, None, None, None, None
+
+
+class TopkGates(torch.autograd.Function):
+    """Routing with differentiable gate values: (scores [T, E], k, routing dict to fill) -> the K
+    L1-normalised gate values of every token (modules/fast_moe_module.py:93-105).  The selection
+    itself has no gradient."""
+
+    MAX_K = 64      # slots are lanes of one wave in the backward kernel
+
+    @staticmethod
+    def forward(ctx, scores, k, routing):
+        routing.update(ops.route_topk(scores, k, renorm=True))
+        ctx.save_for_backward(scores, routing["topk_idx"])
+        return routing["gates"]
+
+    @staticmethod
+    def backward(ctx, d_gates):
+        scores, topk_idx = ctx.saved_tensors
+        if torch.is_grad_enabled():     # create_graph=True: the formula in differentiable torch ops
+            picked = scores.gather(1, topk_idx)
+            total = picked.sum(dim=1, keepdim=True)
+            c = total.clamp_min(1e-12)
+            d_total = (-d_gates * ((picked / c) / c)).sum(dim=1, keepdim=True)
+            d_picked = d_gates / c + torch.where(total >= 1e-12, d_total, torch.zeros_like(d_total))
+            return torch.zeros_like(scores).scatter_add(1, topk_idx, d_picked), None, None
+        return ops.gate_l1_bwd(scores, topk_idx, d_gates), None, None
+
+
+def topk_gates(scores: torch.Tensor, k: int):
+    """-> (routing dict, gates [T, k] with a gradient to ``scores``)."""
+    if k > TopkGates.MAX_K:
+        r = ops.route_topk(scores.detach(), k, renorm=True)
+        picked = scores.gather(1, r["topk_idx"])
+        return r, picked / picked.sum(dim=1, keepdim=True).clamp_min(1e-12)
+    r = {}
+    return r, TopkGates.apply(scores, k, r)
 
 
 def needs_grad(*tensors: Optional[torch.Tensor]) -> bool:

@@ -263,7 +263,7 @@ def jagged_weight_grad(dout: torch.Tensor, a_rows: torch.Tensor, offsets: torch.
         return None
     dev = dout.device
     offsets = _i64("offsets", offsets)
-    seg = torch.arange(E + 1, device=dev, dtype=torch.int64) * N
+    seg = torch.arange(0, E * N + 1, N, device=dev, dtype=torch.int64)
     if halves:
         out = torch.empty((E * (N // 2), Kin), dtype=torch.bfloat16, device=dev)
         out2 = torch.empty_like(out)
@@ -672,3 +672,31 @@ def combine_bwd(dy: torch.Tensor, value: Optional[torch.Tensor], token_index: to
         _ptr(d_gates), _stream(dy))
     _lib.check(rc, "fmoe_combine_bwd")
     return d_value, d_gates
+
+
+def invert_index(index: torch.Tensor) -> torch.Tensor:
+    """index [T, K] (sorted position -> flat token*K + slot) -> [T, K] sorted positions of each
+    token's rows, ascending (the order a sequential index_add meets them in), see fmoe_invert_index."""
+    _need_cuda("invert_index", index)
+    index = _i64("index", index)
+    T, K = index.shape
+    reverse = torch.empty_like(index)
+    rc = _lib.load().fmoe_invert_index(index.data_ptr(), T, K, reverse.data_ptr(), _stream(index))
+    _lib.check(rc, "fmoe_invert_index")
+    return reverse
+
+
+def gate_l1_bwd(scores: torch.Tensor, topk_idx: torch.Tensor, d_gates: torch.Tensor) -> torch.Tensor:
+    """Gradient of the L1-normalised top-k gates with respect to the scores [T, E], see fmoe_gate_l1_bwd."""
+    dev = _need_cuda("gate_l1_bwd", scores, topk_idx, d_gates)
+    if scores.dtype not in _DTYPE_CODE or d_gates.dtype != scores.dtype:
+        raise ValueError("gate_l1_bwd: scores and d_gates must be fp32 or bf16, of one dtype")
+    T, E = scores.shape
+    if tuple(d_gates.shape) != tuple(topk_idx.shape) or topk_idx.shape[0] != T:
+        raise ValueError("gate_l1_bwd: d_gates and topk_idx must be [T, K]")
+    scores, topk_idx, d_gates = scores.contiguous(), _i64("topk_idx", topk_idx), d_gates.contiguous()
+    d_scores = torch.empty((T, E), dtype=scores.dtype, device=dev)
+    rc = _lib.load().fmoe_gate_l1_bwd(scores.data_ptr(), _DTYPE_CODE[scores.dtype], T, E, topk_idx.shape[1],
+                                      topk_idx.data_ptr(), d_gates.data_ptr(), d_scores.data_ptr(), _stream(scores))
+    _lib.check(rc, "fmoe_gate_l1_bwd")
+    return d_scores

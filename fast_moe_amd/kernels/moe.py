@@ -231,6 +231,6 @@ def fused_jagged_bmm_swiglu_combine(
     assert index.ndim == 2 and index.shape[1] == k, f"{index.shape=}, {k=}"
     hidden = index_select_jagged_bmm_swiglu(0, offsets, index, jagged, weight, bias, weight_p, bias_p, kernel)
     token_index = torch.div(index.reshape(-1), k, rounding_mode="floor")
-    reverse_index = _ag._reverse_from_index(index)
+    reverse_index = ops.invert_index(index)
     return silu_jagged_bmm_combine(0, offsets, hidden, weight_out, bias_out, token_index, reverse_index,
                                    gates, gates_index, has_silu=False, kernel=kernel)

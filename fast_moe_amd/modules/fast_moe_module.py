@@ -83,17 +83,15 @@ class FastMoELayer(nn.Module):
     def _forward_with_grad(self, x: torch.Tensor, k: int) -> torch.Tensor:
         """The two-operator form of fast_moe_module.py:146-186 on the differentiable HIP operators
         (same values as ``forward``: the fused SiLU epilogue rounds where this form rounds).  The
-        routing integers come from the library; the K gate values are re-derived from the gate
-        probabilities with torch ops so that the gate network receives its gradient
-        (fast_moe_module.py:93-105: mask, then L1 normalisation)."""
+        routing integers and the K gate values come from the library; the gate values' backward gives the
+        gate network its gradient (fast_moe_module.py:93-105: mask, then L1 normalisation)."""
         from ..kernels import moe
+        from ..kernels.hip.autograd import topk_gates
         if x.dtype not in (torch.bfloat16, torch.float32):
             raise NotImplementedError(f"FastMoELayer: the HIP kernels take bf16 or fp32 activations, got {x.dtype}")
         original_shape = x.shape
         scores = self.gate(x).reshape(-1, self.num_experts)
-        r = ops.route_topk(scores.detach(), k, renorm=True)
-        picked = scores.gather(1, r["topk_idx"])
-        gates = picked / picked.sum(dim=1, keepdim=True).clamp_min(1e-12)
+        r, gates = topk_gates(scores, k)
         x_flat = x.reshape(-1, self.input_dim)
         T = x_flat.shape[0]
         hidden = moe.index_select_jagged_bmm(

@@ -405,6 +405,24 @@ int fmoe_segment_colsum(const void* src, int dtype, int64_t total_rows, int64_t 
                         fmoe_stream_t stream);
 
 /*
+ * index [T*K]: expert-sorted position -> flat token*K + slot, a permutation.  reverse [T, K]: the
+ * positions of every token's rows, ascending (the order in which a sequential index_add meets
+ * them): what the gather-form sum of a token's input-gradient rows reads (fmoe_combine; the
+ * reference adds them atomically, kernels/triton/triton_moe.py:606-804).  A slot that no position
+ * names gets -1.
+ */
+int fmoe_invert_index(const int64_t* index, int64_t T, int K, int64_t* reverse, fmoe_stream_t stream);
+
+/*
+ * Gradient of the L1-normalised top-k gate values (modules/fast_moe_module.py:93-105) with respect
+ * to the gate probabilities: gates[t, j] = s_j / max(sum_i s_i, 1e-12) with s_j =
+ * scores[t, topk_idx[t, j]].  scores, d_gates [T, K] and d_scores [T, E] share one type, FMOE_F32
+ * or FMOE_BF16; contiguous.  d_scores is written whole (0 for experts not picked).  K <= 64.
+ */
+int fmoe_gate_l1_bwd(const void* scores, int dtype, int64_t T, int num_experts, int K,
+                     const int64_t* topk_idx, const void* d_gates, void* d_scores, fmoe_stream_t stream);
+
+/*
  * Element-wise backward of h = silu(g) * u (the SwiGLU epilogue; kernels/triton/triton_moe.py:62-141):
  *   du = dh * silu(g),   dg = (dh * u) * sigmoid(g) * (1 + g * (1 - sigmoid(g)))
  * rounded where torch autograd rounds (silu(g), dh * u and both results in `dtype`).

@@ -666,3 +666,47 @@ def test_segment_colsum(lens, cols, dtype):
         wide[:, cols:] = src
         again = ops.segment_colsum(wide.cuda()[:, cols:], offsets.cuda())
         assert torch.equal(again, out)
+
+
+@pytest.mark.parametrize("T,K", [(1, 1), (5, 8), (257, 3), (4097, 8), (300, 9), (33, 70)])
+def test_invert_index(T, K):
+    from fast_moe_amd.kernels.hip import ops
+    g = torch.Generator().manual_seed(T * 100 + K)
+    index = torch.randperm(T * K, generator=g)
+    want = torch.argsort(index).view(T, K).sort(dim=1).values
+    assert torch.equal(ops.invert_index(dev(index.view(T, K))).cpu(), want)
+    if T * K > 3:       # entries that no position names are "no row", whatever the buffer held before
+        broken = index.clone()
+        lost = [int(broken[0]), int(broken[2])]
+        broken[0], broken[2] = -1, T * K + 5
+        want = torch.argsort(index)
+        want[lost] = -1
+        assert torch.equal(ops.invert_index(dev(broken.view(T, K))).cpu(), want.view(T, K).sort(dim=1).values)
+
+
+@pytest.mark.parametrize("T,E,K", [(1, 4, 2), (7, 8, 8), (1021, 12, 3), (130, 65, 1), (257, 128, 8), (65, 200, 64)])
+@pytest.mark.parametrize("dtype", [BF16, torch.float32])
+def test_topk_gates_backward(T, E, K, dtype):
+    """The gate values and their gradient against the chain of torch ops they stand for: bf16 rounds where the chain
+    rounds (a sum over K in another order may move one rounding: 2^-8 of the terms summed), fp32 to 2^-21 of them."""
+    from fast_moe_amd.kernels.hip.autograd import topk_gates
+    scores = torch.softmax(randn((T, E), E + K).float() * 2, dim=1).to(dtype)
+    dg = (randn((T, K), K) * 0.1).to(dtype)
+    s = leaf(scores, device="cuda")
+    r, gates = topk_gates(s, K)
+    gates.backward(dev(dg))
+    ref = leaf(scores)
+    picked = ref.gather(1, r["topk_idx"].cpu())
+    want = picked / picked.sum(dim=1, keepdim=True).clamp_min(1e-12)
+    want.backward(dg)
+    eps = 2.0 ** -8 if dtype == BF16 else K * 2.0 ** -22
+    torch.testing.assert_close(gates.detach().cpu().float(), want.detach().float(), rtol=eps, atol=0)
+    total = picked.detach().float().sum(dim=1, keepdim=True)
+    bound = eps * 4 * (dg.float().abs().max(dim=1, keepdim=True).values / total)
+    assert ((s.grad.cpu().float() - ref.grad.float()).abs() <= bound).all()
+    # under create_graph the same gradient comes from torch ops and can be differentiated again
+    s2 = leaf(scores, device="cuda")
+    _, gates2 = topk_gates(s2, K)
+    grad, = torch.autograd.grad(gates2, s2, dev(dg), create_graph=True)
+    assert grad.requires_grad
+    assert ((grad.detach().cpu().float() - s.grad.cpu().float()).abs() <= bound).all()
