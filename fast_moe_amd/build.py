@@ -16,6 +16,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libfastmoe_hip.so")
+HOST_PATH = os.path.join(HERE, "_host.so")     # the native side of the Python wrappers (csrc/host_calls.cpp)
 OBJ_DIR = os.path.join(CSRC, "build")
 
 SOURCES = ["gemm_bf16.hip", "gemm_fp8.hip", "gemm_bf16_tail.hip", "gemm_fp8_tail.hip", "gemm_bf16_short.hip", "gemm_fp8_short.hip",
@@ -46,12 +47,33 @@ def _compile(src: str, extra, obj_dir: str = OBJ_DIR) -> str:
     return obj
 
 
+def _build_host() -> str:
+    """The extension module that issues the forward operators' calls: plain C++ against torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           *(f"-isystem{p}" for p in cpp_extension.include_paths()), "-isystem" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "host_calls.cpp"), "-o", HOST_PATH, "-L" + torch_lib,
+           "-ltorch_cpu", "-ltorch", "-lc10", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for host_calls.cpp:\n{res.stdout}\n{res.stderr}")
+    return HOST_PATH
+
+
 def build(extra_flags=(), jobs: int = 8, verbose: bool = True, out: str = LIB_PATH) -> str:
     # (a library under another name keeps its objects apart from the product's)
     obj_dir = OBJ_DIR if os.path.abspath(out) == LIB_PATH else os.path.join(OBJ_DIR, os.path.splitext(os.path.basename(out))[0])
     os.makedirs(obj_dir, exist_ok=True)
     with ThreadPoolExecutor(max_workers=max(1, min(jobs, len(SOURCES)))) as pool:
+        # (a library under another name goes with the product's extension module, which takes its entry points by address)
+        host = pool.submit(_build_host) if obj_dir == OBJ_DIR else None
         objs = list(pool.map(lambda s: _compile(s, list(extra_flags), obj_dir), SOURCES))
+    if host is not None:
+        host.result()
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out, *objs]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

@@ -127,6 +127,25 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_host = None
+
+
+def host():
+    """The extension module whose functions take a forward operator's call whole or return None (csrc/host_calls.cpp)."""
+    global _host
+    if _host is None:
+        lib = load()
+        try:
+            from ... import _host as mod
+        except ImportError as e:
+            raise RuntimeError(f"fast_moe_amd/_host.so is missing or does not load ({e}): build it with "
+                               f"`python -m fast_moe_amd.build`") from e
+        mod.init(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in (
+            "fmoe_route_workspace_bytes", "fmoe_route_topk", "fmoe_grouped_gemm", "fmoe_combine", "fmoe_quant_rows_e4m3")))
+        _host = mod
+    return _host
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = load().fmoe_last_error().decode("utf-8", "replace")

@@ -18,7 +18,9 @@ FP8_DTYPE = torch.float8_e4m3fn
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Handle of the current stream of t's device (0 for a tensor that is on none: every call refuses it)."""
+    device = t.get_device()
+    return torch._C._cuda_getCurrentRawStream(device) if device >= 0 else 0
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -61,6 +63,9 @@ def _rows_contiguous(t: torch.Tensor) -> torch.Tensor:
 GATE_RAW, GATE_L1, GATE_SOFTMAX_ALL, GATE_SOFTMAX_TOPK = 0, 1, 2, 3
 
 
+_ROUTE_NAMES = ("topk_idx", "gates", "lengths", "offsets", "gate_index", "token_index", "reverse_index")
+
+
 def route_topk(scores: torch.Tensor, k: int, renorm=True, static_scratch: bool = False,
                out: Optional[Dict[str, torch.Tensor]] = None) -> Dict[str, torch.Tensor]:
     """scores [T, E] (fp32 / bf16 gate probabilities, or router logits for the softmax modes)
@@ -68,6 +73,10 @@ def route_topk(scores: torch.Tensor, k: int, renorm=True, static_scratch: bool =
     ``static_scratch``: fmoe_route_topk_static, whose scratch is built into the library (no
     workspace allocation; T*k <= 2^20, E <= 512).  ``out``: a dict of a previous call with the
     same shapes, written in place (with static_scratch the call then allocates nothing)."""
+    if out is None and not static_scratch:
+        parts = _lib.host().route_topk(scores, k, int(renorm), _stream(scores))
+        if parts is not None:
+            return dict(zip(_ROUTE_NAMES, parts))
     dev = _need_cuda("route_topk", scores)
     if scores.ndim != 2:
         raise ValueError("route_topk: scores must be [T, E]")
@@ -159,6 +168,11 @@ def quant_rows_fp8(a: torch.Tensor, apply_silu: bool = False, reciprocal_scale: 
 
     Returns ``(q, scale)``: q is float8_e4m3fn, contiguous in a's logical shape (or laid out
     with a's own strides when ``out_like_input``), scale is fp32 with a's leading shape."""
+    if not out_like_input and a.ndim == 2:
+        pair = _lib.host().quant_rows(a, int(apply_silu), int(reciprocal_scale), _stream(a))
+        if pair is not None:
+            pair[1]._fmoe_pow2 = pair[1]._version       # (see scales_are_pow2)
+            return pair
     dev = _need_cuda("quant_rows_fp8", a)
     if a.dtype not in _DTYPE_CODE:
         raise ValueError(f"quant_rows_fp8: input must be fp32 or bf16, got {a.dtype}")
@@ -307,6 +321,12 @@ def grouped_gemm(offsets: torch.Tensor, a: torch.Tensor, b: torch.Tensor, *, tot
     _lib.PLAN_* code of the kernel this call would run (fmoe_grouped_gemm_plan).  ``scales_pow2``
     (e4m3): a promise that every scale is an exact power of two, as ``quant_rows_fp8`` writes them;
     the ring kernel then folds them into its MFMAs (fmoe_gemm_desc.scale_pow2)."""
+    if not (a_silu or a_expert_stride or plan_only) and k_window is None and out is None and aux is None and gate is None:
+        res = _lib.host().grouped_gemm(
+            offsets, a, b, total_rows, row_index if row_index is None or row_index.ndim == 1 else row_index.reshape(-1),
+            index_div, bias, b2, bias2, epilogue, a_scale, b_scale, b2_scale, int(bool(scales_pow2)), _stream(a))
+        if res is not None:
+            return res
     dev = _need_cuda("grouped_gemm", offsets, a, b, row_index, bias, b2, bias2, a_scale, b_scale, b2_scale)
     fp8 = a.dtype == FP8_DTYPE
     if not fp8 and a.dtype not in (torch.bfloat16, torch.float32):
@@ -487,6 +507,9 @@ def gemm_plan(d: GemmDesc) -> int:
 def combine(value: torch.Tensor, reverse_index: torch.Tensor, gates: Optional[torch.Tensor] = None,
             gates_index: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Weighted merge, see fmoe_combine.  value [T*K, D]; reverse_index [T, K]."""
+    res = _lib.host().combine(value, reverse_index, gates, gates_index, _stream(value))
+    if res is not None:
+        return res
     dev = _need_cuda("combine", value, reverse_index, gates, gates_index)
     if value.dtype not in _DTYPE_CODE:
         raise NotImplementedError(f"combine: value must be fp32 or bf16, got {value.dtype}")

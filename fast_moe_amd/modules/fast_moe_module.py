@@ -17,7 +17,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd.profiler import record_function
 
-from ..kernels.hip import ops
+from ..kernels.hip import _lib, ops
 from ..kernels.hip._lib import EPI_NONE, EPI_SILU
 from ..kernels.utils import KernelType, require_hip_kernel
 from ..utils.utils import _create_fused_mlp_weights
@@ -111,7 +111,17 @@ class FastMoELayer(nn.Module):
             raise NotImplementedError(f"FastMoELayer: the HIP kernels take bf16 or fp32 activations, got {x.dtype}")
         original_shape = x.shape
         k = num_experts_per_tok
-        r = self.route(x, k)
+        if getattr(self.route, "__func__", None) is FastMoELayer.route and x.ndim == 3:
+            # the same steps as below, issued by one native call
+            scores = self.gate(x).reshape(-1, self.num_experts)
+            y = _lib.host().mlp_forward(
+                scores, x.reshape(-1, self.input_dim), self._experts_hidden_w.permute(0, 2, 1), self._experts_hidden_bias,
+                self._experts_w.permute(0, 2, 1), self._experts_bias, k, ops.GATE_L1, EPI_SILU, ops._stream(x))
+            if y is not None:
+                return y.view(original_shape[0], original_shape[1], self.output_dim)
+            r = ops.route_topk(scores, k, renorm=True)
+        else:
+            r = self.route(x, k)
         with record_function("## expert_forward##"):
             x_flat = x.reshape(-1, self.input_dim)
             # GEMM1 with SiLU in the epilogue: the hidden is rounded to bf16 before and after the

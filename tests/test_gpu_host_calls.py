@@ -1,0 +1,107 @@
+"""The native host calls (csrc/host_calls.cpp) against the Python code that takes what they decline: the same
+kernels on the same operands, so the same bits, for calls they take and for calls they leave."""
+import pytest
+import torch
+
+from helpers import BF16, dev, make_routing, randn
+
+pytestmark = pytest.mark.gpu
+
+
+class Declines:
+    """A host module that takes nothing."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+def both(fn):
+    from fast_moe_amd.kernels.hip import _lib
+    taken = fn()
+    real = _lib.host()
+    _lib._host = Declines()
+    try:
+        return taken, fn()
+    finally:
+        _lib._host = real
+
+
+def same(a, b):
+    if isinstance(a, dict):
+        a, b = list(a.values()), [b[n] for n in a]
+    for x, y in zip(*((v if isinstance(v, (list, tuple)) else [v]) for v in (a, b))):
+        assert x.dtype == y.dtype and x.shape == y.shape and x.stride() == y.stride()
+        assert torch.equal(x.view(torch.uint8) if x.element_size() == 1 else x, y.view(torch.uint8) if y.element_size() == 1 else y)
+
+
+@pytest.mark.parametrize("T,E,K", [(1, 4, 1), (65, 8, 2), (300, 130, 8)])
+@pytest.mark.parametrize("form", ["plain", "strided", "subclass", "fp32"])
+def test_operators(T, E, K, form):
+    from fast_moe_amd.kernels.hip import ops
+    from fast_moe_amd.kernels.hip._lib import EPI_SWIGLU
+    dtype = torch.float32 if form == "fp32" else BF16
+    make = {"plain": lambda t: t, "fp32": lambda t: t, "subclass": lambda t: t.as_subclass(Sub),
+            "strided": lambda t: torch.cat([t, t], dim=-1)[..., :t.shape[-1]]}[form]
+    D, H = 64, 96
+    scores = make(dev(torch.softmax(randn((T, E), 1).float(), 1)))
+    x = make(dev(randn((T, D), 2).to(dtype)))
+    w, wp = (make(dev(randn((E, H, D), s, scale=D ** -0.5).to(dtype))).permute(0, 2, 1) for s in (3, 4))
+    bias = make(dev(randn((E, H), 5).to(dtype)))
+    same(*both(lambda: ops.route_topk(scores, K)))
+    r = ops.route_topk(scores, K)
+    off, idx = r["offsets"], r["gate_index"]
+    for kw in (dict(), dict(bias=bias), dict(bias=bias, bias2=bias, b2=wp, epilogue=EPI_SWIGLU)):
+        same(*both(lambda: ops.grouped_gemm(off, x, w, total_rows=T * K, row_index=idx.view(-1, K), index_div=K, **kw)))
+    value = ops.grouped_gemm(off, x, w, total_rows=T * K, row_index=idx, index_div=K)
+    for gates in (None, r["gates"], r["gates"].to(BF16), r["gates"].reshape(-1)):
+        same(*both(lambda: ops.combine(value, r["reverse_index"], gates, idx)))
+    for silu in (False, True):
+        same(*both(lambda: ops.quant_rows_fp8(x, apply_silu=silu)))
+        q, s = ops.quant_rows_fp8(x, apply_silu=silu)
+        assert ops.scales_are_pow2(s)
+
+
+@pytest.mark.parametrize("dtype", [BF16, torch.float32])
+@pytest.mark.parametrize("B,S", [(1, 1), (2, 33), (3, 0)])
+def test_layer_forward(B, S, dtype):
+    from fast_moe_amd import FastMoELayer
+    torch.manual_seed(0)
+    layer = FastMoELayer(64, 96, 64, 8, dtype=dtype).to(dtype).cuda()
+    x = dev(randn((B, S, 64), 1).to(dtype))
+    with torch.no_grad():
+        same(*both(lambda: layer(x, 2)))
+
+    class Rerouted(FastMoELayer):       # a route() of its own is asked
+        def route(self, x, k):
+            self.asked = True
+            return super().route(x, k)
+
+    if S:
+        other = Rerouted(64, 96, 64, 8, dtype=dtype).to(dtype).cuda()
+        other.load_state_dict(layer.state_dict())
+        with torch.no_grad():
+            same(other(x, 2), layer(x, 2))
+        assert other.asked
+
+
+def test_refusals_are_the_python_codes():
+    from fast_moe_amd.kernels.hip import ops
+    r = make_routing(16, 4, 2, seed=1)
+    x, w = dev(randn((16, 64), 1)), dev(randn((4, 32, 64), 2)).permute(0, 2, 1)
+    off = dev(r["offsets"])
+    with pytest.raises(ValueError, match="share a dtype"):
+        ops.grouped_gemm(off, x, w.float(), total_rows=32)
+    with pytest.raises(ValueError, match="bias must be"):
+        ops.grouped_gemm(off, x, w, total_rows=32, bias=dev(randn((4, 31), 3)))
+    with pytest.raises(ValueError, match="total_rows entries"):
+        ops.grouped_gemm(off, x, w, total_rows=32, row_index=dev(r["index"]).view(-1)[:31])
+    with pytest.raises(ValueError, match="different devices|live on the GPU"):
+        ops.grouped_gemm(off, x, w.cpu(), total_rows=32)
+    with pytest.raises(ValueError, match="int64"):
+        ops.combine(x, dev(r["index"]).int())
+    with pytest.raises((RuntimeError, ValueError)):
+        ops.route_topk(dev(torch.rand(16, 4)), 5)
