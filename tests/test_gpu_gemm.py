@@ -1145,3 +1145,31 @@ def test_ring_kernel_on_short_tiles(E, rows, K, N, layout, epi):
         if epi == _lib.EPI_GATED:
             a = a * torch.nn.functional.silu(gate[lo:hi].double())
         assert_bf16_close(out[lo:hi], a.float(), rtol=1.6e-2, atol=4e-3, what=f"expert {e}")
+
+
+@pytest.mark.parametrize("row_tiles", [1, 7, 28, 31, 32, 33, 59, 60, 61, 97])
+@pytest.mark.parametrize("N", [256, 776])
+def test_ring_kernel_deals_every_tile_once(row_tiles, N):
+    """Row-tile counts around the scheduler's lines (groups of 4 row tiles, rounds of 8 groups, seven groups and more of a
+    last round kept whole): every output tile is written, and once.  Short last tiles included.  fp32 sums of 128 bf16
+    products differ from another order's by less than 2^-16 of sum |a||b|, the result's rounding adds 2^-8 of it."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    K, E = 128, 3
+    cut = [row_tiles // 3, row_tiles // 2]
+    lens = [256 * cut[0], 256 * (cut[1] - cut[0]), 256 * (row_tiles - cut[1]) - 200]
+    offsets = torch.tensor([0, *torch.tensor(lens).cumsum(0)])
+    R = int(offsets[-1])
+    a, w = dev(randn((R, K), row_tiles)), dev(randn((E, N, K), N, scale=K ** -0.5))
+    b = w.permute(0, 2, 1)
+    off = dev(offsets)
+    total = max(R, 96 * E)      # (fewer rows per expert would take another kernel)
+    if total > R:
+        a = torch.cat([a, a.new_zeros(total - R, K)])
+    assert ops.grouped_gemm(off, a, b, total_rows=total, plan_only=True) == _lib.PLAN_RING
+    out = torch.full((total, N), float("nan"), dtype=BF16, device="cuda")
+    ops.grouped_gemm(off, a, b, total_rows=total, out=out)
+    for e in range(E):
+        rows = slice(int(offsets[e]), int(offsets[e + 1]))
+        ref = a[rows].float() @ w[e].float().t()
+        mag = a[rows].float().abs() @ w[e].float().abs().t()
+        assert ((out[rows].float() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * 2.0 ** -16).all()
