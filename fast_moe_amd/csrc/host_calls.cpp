@@ -6,12 +6,15 @@
 // output and descriptor field.
 //
 // Every function here takes a call whole or returns None and has done nothing that matters: whatever it does not recognise
-// (other dtypes, layouts, tensor subclasses, wrong shapes, an error status) is left to the Python code in ops.py, which
-// handles it or raises.  Nothing is kept from one call for the next.  The C entry points are handed over as addresses once
-// (init), so that this module works with whichever build of the library ctypes has loaded.
+// (other dtypes, layouts, tensor subclasses, wrong shapes, a call the library refuses) is left to the Python code in ops.py,
+// which handles it or raises.  What fails once work is being issued (no memory, a launch error) raises here: issued again it
+// would run twice, and a launch error that the first attempt has read is gone for the second.  Nothing is kept from one call
+// for the next.  The C entry points are handed over as addresses once (init), so that this module works with whichever build
+// of the library ctypes has loaded.
 #include <Python.h>
 #include <ATen/ATen.h>
 #include <ATen/record_function.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
@@ -25,8 +28,11 @@ decltype(&fmoe_route_topk) c_route_topk;
 decltype(&fmoe_grouped_gemm) c_grouped_gemm;
 decltype(&fmoe_combine) c_combine;
 decltype(&fmoe_quant_rows_e4m3) c_quant_rows;
+decltype(&fmoe_last_error) last_error;
 
 constexpr int64_t kSlackRows = 128;      // ops.SLACK_ROWS
+
+constexpr int kDeclined = -1;           // beside the C status codes: left to the Python code
 
 struct NoGil {
     PyThreadState* state = PyEval_SaveThread();
@@ -74,12 +80,17 @@ struct Routing {
     at::Tensor topk_idx, gates, lengths, offsets, gate_index, token_index, reverse_index;
 };
 
-bool route(const at::Tensor& scores, int64_t k, int64_t mode, void* stream, Routing& r) {
+bool route_ok(const at::Tensor& scores, int64_t k, const void** data) {
     if (scores.dim() != 2 || !scores.is_contiguous()) return false;
     const int code = dtype_code(scores.scalar_type());
     if (code != FMOE_F32 && code != FMOE_BF16) return false;
+    const int64_t E = scores.size(1);
+    *data = scores.data_ptr();
+    return k >= 1 && k <= E && E <= INT32_MAX;
+}
+
+int route(const at::Tensor& scores, const void* data, int64_t k, int64_t mode, void* stream, Routing& r) {
     const int64_t T = scores.size(0), E = scores.size(1);
-    if (k < 1 || k > E || E > INT32_MAX) return false;
     r.topk_idx = empty({T, k}, at::kLong, scores);
     r.gates = empty({T, k}, scores.scalar_type(), scores);
     r.lengths = empty({E}, at::kLong, scores);
@@ -89,10 +100,10 @@ bool route(const at::Tensor& scores, int64_t k, int64_t mode, void* stream, Rout
     r.reverse_index = empty({T, k}, at::kLong, scores);
     const size_t ws_bytes = route_workspace_bytes(T, (int)E, (int)k);
     const at::Tensor ws = empty({(int64_t)(ws_bytes ? ws_bytes : 1)}, at::kByte, scores);
-    return c_route_topk(scores.data_ptr(), code, T, (int)E, (int)k, (int)mode, r.topk_idx.data_ptr<int64_t>(),
+    return c_route_topk(data, dtype_code(scores.scalar_type()), T, (int)E, (int)k, (int)mode, r.topk_idx.data_ptr<int64_t>(),
                         r.gates.data_ptr(), r.lengths.data_ptr<int64_t>(), r.offsets.data_ptr<int64_t>(),
                         r.gate_index.data_ptr<int64_t>(), r.token_index.data_ptr<int64_t>(),
-                        r.reverse_index.data_ptr<int64_t>(), ws.data_ptr(), ws_bytes, stream) == FMOE_OK;
+                        r.reverse_index.data_ptr<int64_t>(), ws.data_ptr(), ws_bytes, stream);
 }
 
 struct GemmArgs {
@@ -100,7 +111,8 @@ struct GemmArgs {
     int64_t total_rows = 0, index_div = 1, epilogue = FMOE_EPI_NONE, pow2 = 0;
 };
 
-bool gemm(const GemmArgs& g, void* stream, at::Tensor& out) {
+// Checks the operands and fills everything of the descriptor but the output.
+bool gemm_ok(const GemmArgs& g, fmoe_gemm_desc& d) {
     const at::Tensor &a = g.a, &b = g.b;
     const int code = dtype_code(a.scalar_type());
     if (code < 0 || b.scalar_type() != a.scalar_type() || a.dim() != 2 || b.dim() != 3) return false;
@@ -131,8 +143,7 @@ bool gemm(const GemmArgs& g, void* stream, at::Tensor& out) {
     } else if (g.a_scale.defined() || g.b_scale.defined() || g.b2_scale.defined()) {
         return false;
     }
-    out = empty({g.total_rows + kSlackRows, N}, out_dtype, a).narrow(0, 0, g.total_rows);
-    fmoe_gemm_desc d = {};
+    d = {};
     d.num_experts = (int32_t)E;
     d.n = (int32_t)N;
     d.k = (int32_t)K;
@@ -160,71 +171,106 @@ bool gemm(const GemmArgs& g, void* stream, at::Tensor& out) {
     d.bias_stride_e = g.bias.defined() ? g.bias.stride(0) : g.bias2.defined() ? g.bias2.stride(0) : 0;
     d.epilogue = (int32_t)g.epilogue;
     d.out_dtype = dtype_code(out_dtype);
-    d.out = out.data_ptr();
-    d.out_stride_row = out.stride(0);
-    return c_grouped_gemm(&d, stream) == FMOE_OK;
+    return true;
 }
 
-bool combine(const at::Tensor& value, const at::Tensor& reverse, const at::Tensor& gates, const at::Tensor& gates_index,
-             void* stream, at::Tensor& out) {
-    const int code = dtype_code(value.scalar_type());
-    if ((code != FMOE_F32 && code != FMOE_BF16) || value.dim() != 2 || value.stride(1) != 1 || reverse.dim() != 2)
+int gemm(fmoe_gemm_desc& d, const at::Tensor& like, void* stream, at::Tensor& out) {
+    out = empty({d.total_rows + kSlackRows, d.n}, d.out_dtype == FMOE_F32 ? at::kFloat : at::kBFloat16, like)
+              .narrow(0, 0, d.total_rows);
+    d.out = out.data_ptr();
+    d.out_stride_row = out.stride(0);
+    return c_grouped_gemm(&d, stream);
+}
+
+struct Combine {
+    at::Tensor value, reverse, gates, gates_index;
+    const void *value_data, *gates_data = nullptr;
+    const int64_t *reverse_data, *index_data = nullptr;
+    at::ScalarType out_dtype;
+    int code, g_code = FMOE_F32;
+    int64_t T, K, D, cols = 1, sr = 1, sc = 1;
+};
+
+bool combine_ok(Combine& c) {
+    c.code = dtype_code(c.value.scalar_type());
+    if ((c.code != FMOE_F32 && c.code != FMOE_BF16) || c.value.dim() != 2 || c.value.stride(1) != 1 || c.reverse.dim() != 2)
         return false;
-    if (!same_device(value, reverse) || !same_device(value, gates) || !same_device(value, gates_index)) return false;
-    const int64_t T = reverse.size(0), K = reverse.size(1), D = value.size(1);
-    if (!i64_list(reverse, T * K) || value.size(0) != T * K || K < 1 || K > INT32_MAX) return false;
-    at::ScalarType out_dtype = value.scalar_type();
-    int g_code = FMOE_F32;
-    int64_t cols = 1, sr = 1, sc = 1;
-    if (gates.defined()) {
-        g_code = dtype_code(gates.scalar_type());
-        if ((g_code != FMOE_F32 && g_code != FMOE_BF16) || gates.dim() != 2 || gates.numel() != T * K) return false;
-        if (g_code == FMOE_F32) out_dtype = at::kFloat;
-        cols = gates.size(1);
-        sr = gates.stride(0);
-        sc = gates.stride(1);
-        if (gates_index.defined() && !i64_list(gates_index, T * K)) return false;
+    if (!same_device(c.value, c.reverse) || !same_device(c.value, c.gates) || !same_device(c.value, c.gates_index)) return false;
+    c.T = c.reverse.size(0);
+    c.K = c.reverse.size(1);
+    c.D = c.value.size(1);
+    if (!i64_list(c.reverse, c.T * c.K) || c.value.size(0) != c.T * c.K || c.K < 1 || c.K > INT32_MAX) return false;
+    c.out_dtype = c.value.scalar_type();
+    if (c.gates.defined()) {
+        c.g_code = dtype_code(c.gates.scalar_type());
+        if ((c.g_code != FMOE_F32 && c.g_code != FMOE_BF16) || c.gates.dim() != 2 || c.gates.numel() != c.T * c.K) return false;
+        if (c.g_code == FMOE_F32) c.out_dtype = at::kFloat;
+        c.cols = c.gates.size(1);
+        c.sr = c.gates.stride(0);
+        c.sc = c.gates.stride(1);
+        c.gates_data = c.gates.data_ptr();
+        if (c.gates_index.defined()) {
+            if (!i64_list(c.gates_index, c.T * c.K)) return false;
+            c.index_data = c.gates_index.data_ptr<int64_t>();
+        }
     }
-    const bool indexed = gates.defined() && gates_index.defined();
-    out = empty({T, D}, out_dtype, value);
-    return c_combine(value.data_ptr(), code, T, (int)K, D, value.stride(0), reverse.data_ptr<int64_t>(),
-                     gates.defined() ? gates.data_ptr() : nullptr, g_code, cols, sr, sc,
-                     indexed ? gates_index.data_ptr<int64_t>() : nullptr, out.data_ptr(), dtype_code(out_dtype),
-                     stream) == FMOE_OK;
+    c.value_data = c.value.data_ptr();
+    c.reverse_data = c.reverse.data_ptr<int64_t>();
+    return true;
+}
+
+int combine(const Combine& c, void* stream, at::Tensor& out) {
+    out = empty({c.T, c.D}, c.out_dtype, c.value);
+    return c_combine(c.value_data, c.code, c.T, (int)c.K, c.D, c.value.stride(0), c.reverse_data, c.gates_data, c.g_code, c.cols,
+                     c.sr, c.sc, c.index_data, out.data_ptr(), dtype_code(c.out_dtype), stream);
 }
 
 PyObject* none() { Py_RETURN_NONE; }
 PyObject* wrap(const at::Tensor& t) { return THPVariable_Wrap(t); }
 
-// A C++ exception (a tensor that hides its storage, out of memory) also leaves the call to the Python code, which raises it
-// as torch raises it there.
-template <typename F>
-bool guarded(F&& f) {
+// check() looks at the operands (what throws there, a tensor that hides its storage say, is left to the Python code, which
+// raises it as torch does), issue() allocates and launches (what throws there is the call's).  -> kDeclined or a C status.
+template <typename Check, typename Issue>
+int run(Check&& check, Issue&& issue) {
     NoGil nogil;
     try {
-        return f();
+        if (!check()) return kDeclined;
     } catch (const std::exception&) {
-        return false;
+        return kDeclined;
     }
+    return issue();
+}
+
+// The library's other refusals come before its first launch: the Python code raises them, in its own words where it has any.
+bool raised(int status, const char* what) {
+    if (status != FMOE_ERR_LAUNCH) return false;
+    PyErr_Format(PyExc_RuntimeError, "%s failed (status %d): %s", what, status, last_error());
+    return true;
 }
 
 // (scores, k, mode, stream) -> (topk_idx, gates, lengths, offsets, gate_index, token_index, reverse_index)
 PyObject* py_route_topk(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     int64_t k, mode, stream;
     const at::Tensor scores = n == 4 ? gpu_tensor(args[0]) : at::Tensor();
     if (!scores.defined() || !as_int(args[1], &k) || !as_int(args[2], &mode) || !as_int(args[3], &stream)) return none();
     Routing r;
-    if (!guarded([&] { return route(scores, k, mode, (void*)stream, r); })) return none();
+    const void* data;
+    const int status = run([&] { return route_ok(scores, k, &data); }, [&] { return route(scores, data, k, mode, (void*)stream, r); });
+    if (raised(status, "fmoe_route_topk")) return nullptr;
+    if (status != FMOE_OK) return none();
     PyObject* out = PyTuple_New(7);
     if (!out) return nullptr;
     const at::Tensor* parts[7] = {&r.topk_idx, &r.gates, &r.lengths, &r.offsets, &r.gate_index, &r.token_index,
                                   &r.reverse_index};
     for (int i = 0; i < 7; ++i) PyTuple_SET_ITEM(out, i, wrap(*parts[i]));
     return out;
+    END_HANDLE_TH_ERRORS
 }
 
 // (offsets, a, b, total_rows, row_index, index_div, bias, b2, bias2, epilogue, a_scale, b_scale, b2_scale, pow2, stream)
 PyObject* py_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 15) return none();
     GemmArgs g;
     int64_t stream;
@@ -238,44 +284,64 @@ PyObject* py_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         !as_int(args[14], &stream))
         return none();
     at::Tensor out;
-    return guarded([&] { return gemm(g, (void*)stream, out); }) ? wrap(out) : none();
+    fmoe_gemm_desc d;
+    const int status = run([&] { return gemm_ok(g, d); }, [&] { return gemm(d, g.a, (void*)stream, out); });
+    if (raised(status, "fmoe_grouped_gemm")) return nullptr;
+    return status == FMOE_OK ? wrap(out) : none();
+    END_HANDLE_TH_ERRORS
 }
 
 // (value, reverse_index, gates, gates_index, stream)
 PyObject* py_combine(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 5) return none();
-    const at::Tensor value = gpu_tensor(args[0]), reverse = gpu_tensor(args[1]);
-    at::Tensor gates, gates_index;
+    Combine c;
+    c.value = gpu_tensor(args[0]);
+    c.reverse = gpu_tensor(args[1]);
     int64_t stream;
-    if (!value.defined() || !reverse.defined() || !optional_tensor(args[2], &gates) || !optional_tensor(args[3], &gates_index) ||
-        !as_int(args[4], &stream))
+    if (!c.value.defined() || !c.reverse.defined() || !optional_tensor(args[2], &c.gates) ||
+        !optional_tensor(args[3], &c.gates_index) || !as_int(args[4], &stream))
         return none();
     at::Tensor out;
-    return guarded([&] { return combine(value, reverse, gates, gates_index, (void*)stream, out); }) ? wrap(out) : none();
+    const int status = run([&] { return combine_ok(c); }, [&] { return combine(c, (void*)stream, out); });
+    if (raised(status, "fmoe_combine")) return nullptr;
+    return status == FMOE_OK ? wrap(out) : none();
+    END_HANDLE_TH_ERRORS
 }
 
 // (a, apply_silu, reciprocal, stream) -> (q, scale): a 2-D input with contiguous rows
 PyObject* py_quant_rows(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     const at::Tensor a = n == 4 ? gpu_tensor(args[0]) : at::Tensor();
     int64_t silu, reciprocal, stream;
     if (!a.defined() || !as_int(args[1], &silu) || !as_int(args[2], &reciprocal) || !as_int(args[3], &stream)) return none();
     at::Tensor q, scale;
-    const bool ok = guarded([&] {
-        const int code = dtype_code(a.scalar_type());
-        if ((code != FMOE_F32 && code != FMOE_BF16) || a.dim() != 2 || a.size(1) < 1 || a.stride(1) != 1) return false;
-        const int64_t rows = a.size(0), cols = a.size(1);
-        q = empty({rows, cols}, at::kFloat8_e4m3fn, a);
-        scale = empty({rows}, at::kFloat, a);
-        return c_quant_rows(a.data_ptr(), code, 1, rows, cols, rows * a.stride(0), a.stride(0), 1, (int)silu,
-                            (uint8_t*)q.data_ptr(), rows * cols, cols, 1, scale.data_ptr<float>(), (int)reciprocal,
-                            (void*)stream) == FMOE_OK;
-    });
-    return ok ? Py_BuildValue("(NN)", wrap(q), wrap(scale)) : none();
+    const void* data;
+    int code;
+    const int status = run(
+        [&] {
+            code = dtype_code(a.scalar_type());
+            if ((code != FMOE_F32 && code != FMOE_BF16) || a.dim() != 2 || a.size(1) < 1 || a.stride(1) != 1) return false;
+            data = a.data_ptr();
+            return true;
+        },
+        [&] {
+            const int64_t rows = a.size(0), cols = a.size(1);
+            q = empty({rows, cols}, at::kFloat8_e4m3fn, a);
+            scale = empty({rows}, at::kFloat, a);
+            return c_quant_rows(data, code, 1, rows, cols, rows * a.stride(0), a.stride(0), 1, (int)silu,
+                                (uint8_t*)q.data_ptr(), rows * cols, cols, 1, scale.data_ptr<float>(), (int)reciprocal,
+                                (void*)stream);
+        });
+    if (raised(status, "fmoe_quant_rows_e4m3")) return nullptr;
+    return status == FMOE_OK ? Py_BuildValue("(NN)", wrap(q), wrap(scale)) : none();
+    END_HANDLE_TH_ERRORS
 }
 
 // (scores [T, E], x [T, D], w1 [E, D, H], bias1, w2 [E, H, O], bias2, k, mode, epilogue1, stream) -> [T, O]:
 // routing, the gather GEMM with its activation, the second GEMM, the merge
 PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 10) return none();
     const at::Tensor scores = gpu_tensor(args[0]), x = gpu_tensor(args[1]), w1 = gpu_tensor(args[2]);
     const at::Tensor b1 = gpu_tensor(args[3]), w2 = gpu_tensor(args[4]), b2 = gpu_tensor(args[5]);
@@ -285,43 +351,60 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!as_int(args[6], &k) || !as_int(args[7], &mode) || !as_int(args[8], &epilogue) || !as_int(args[9], &stream))
         return none();
     at::Tensor y;
-    const bool ok = guarded([&] {
-        if (x.dim() != 2 || scores.dim() != 2 || scores.size(0) != x.size(0) || w1.dim() != 3 ||
-            w1.size(0) != scores.size(1) || scores.device() != x.device())
-            return false;
-        Routing r;
-        if (!route(scores, k, mode, (void*)stream, r)) return false;
-        RECORD_USER_SCOPE("## expert_forward##");
-        at::Tensor hidden, rows;
-        GemmArgs g;
-        g.offsets = r.offsets;
-        g.a = x;
-        g.b = w1;
-        g.row_index = r.gate_index;
-        g.bias = b1;
-        g.total_rows = x.size(0) * k;
-        g.index_div = k;
-        g.epilogue = epilogue;
-        if (!gemm(g, (void*)stream, hidden)) return false;
-        GemmArgs down;
-        down.offsets = r.offsets;
-        down.a = hidden;
-        down.b = w2;
-        down.bias = b2;
-        down.total_rows = hidden.size(0);
-        return gemm(down, (void*)stream, rows) && combine(rows, r.reverse_index, r.gates, r.gate_index, (void*)stream, y);
-    });
-    return ok ? wrap(y) : none();
+    const void* data;
+    const char* what = "fmoe_route_topk";
+    const int status = run(
+        [&] {
+            return x.dim() == 2 && scores.dim() == 2 && scores.size(0) == x.size(0) && w1.dim() == 3 &&
+                   w1.size(0) == scores.size(1) && scores.device() == x.device() && route_ok(scores, k, &data);
+        },
+        [&] {
+            Routing r;
+            if (const int rc = route(scores, data, k, mode, (void*)stream, r)) return rc;
+            RECORD_USER_SCOPE("## expert_forward##");
+            what = "fmoe_grouped_gemm";
+            at::Tensor hidden, rows;
+            fmoe_gemm_desc d;
+            GemmArgs g;
+            g.offsets = r.offsets;
+            g.a = x;
+            g.b = w1;
+            g.row_index = r.gate_index;
+            g.bias = b1;
+            g.total_rows = x.size(0) * k;
+            g.index_div = k;
+            g.epilogue = epilogue;
+            if (!gemm_ok(g, d)) return kDeclined;
+            if (const int rc = gemm(d, x, (void*)stream, hidden)) return rc;
+            GemmArgs down;
+            down.offsets = r.offsets;
+            down.a = hidden;
+            down.b = w2;
+            down.bias = b2;
+            down.total_rows = hidden.size(0);
+            if (!gemm_ok(down, d)) return kDeclined;
+            if (const int rc = gemm(d, x, (void*)stream, rows)) return rc;
+            what = "fmoe_combine";
+            Combine c;
+            c.value = rows;
+            c.reverse = r.reverse_index;
+            c.gates = r.gates;
+            c.gates_index = r.gate_index;
+            return combine_ok(c) ? combine(c, (void*)stream, y) : kDeclined;
+        });
+    if (raised(status, what)) return nullptr;
+    return status == FMOE_OK ? wrap(y) : none();
+    END_HANDLE_TH_ERRORS
 }
 
 // init(addresses of the C entry points, in the order of the pointers above)
 PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    int64_t v[5];
-    if (n != 5) {
-        PyErr_SetString(PyExc_TypeError, "init: five addresses expected");
+    int64_t v[6];
+    if (n != 6) {
+        PyErr_SetString(PyExc_TypeError, "init: six addresses expected");
         return nullptr;
     }
-    for (int i = 0; i < 5; ++i)
+    for (int i = 0; i < 6; ++i)
         if (!as_int(args[i], &v[i])) {
             PyErr_SetString(PyExc_TypeError, "init: addresses are integers");
             return nullptr;
@@ -331,6 +414,7 @@ PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
     c_grouped_gemm = (decltype(c_grouped_gemm))v[2];
     c_combine = (decltype(c_combine))v[3];
     c_quant_rows = (decltype(c_quant_rows))v[4];
+    last_error = (decltype(last_error))v[5];
     return none();
 }
 

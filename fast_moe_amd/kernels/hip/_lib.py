@@ -127,6 +127,9 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+# what csrc/host_calls.cpp calls, in the order its init() takes the addresses
+HOST_ENTRY_POINTS = ("fmoe_route_workspace_bytes", "fmoe_route_topk", "fmoe_grouped_gemm", "fmoe_combine",
+                     "fmoe_quant_rows_e4m3", "fmoe_last_error")
 _host = None
 
 
@@ -140,8 +143,7 @@ def host():
         except ImportError as e:
             raise RuntimeError(f"fast_moe_amd/_host.so is missing or does not load ({e}): build it with "
                                f"`python -m fast_moe_amd.build`") from e
-        mod.init(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in (
-            "fmoe_route_workspace_bytes", "fmoe_route_topk", "fmoe_grouped_gemm", "fmoe_combine", "fmoe_quant_rows_e4m3")))
+        mod.init(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in HOST_ENTRY_POINTS))
         _host = mod
     return _host
 

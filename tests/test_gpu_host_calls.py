@@ -1,5 +1,8 @@
 """The native host calls (csrc/host_calls.cpp) against the Python code that takes what they decline: the same
 kernels on the same operands, so the same bits, for calls they take and for calls they leave."""
+import contextlib
+import ctypes
+
 import pytest
 import torch
 
@@ -105,3 +108,43 @@ def test_refusals_are_the_python_codes():
         ops.combine(x, dev(r["index"]).int())
     with pytest.raises((RuntimeError, ValueError)):
         ops.route_topk(dev(torch.rand(16, 4)), 5)
+
+
+@contextlib.contextmanager
+def entry_point(name, fn):
+    """The host module calls ``fn`` (a ctypes callback) in the place of one C entry point."""
+    from fast_moe_amd.kernels.hip import _lib
+    lib, host = _lib.load(), _lib.host()
+    real = [ctypes.cast(lib[n], ctypes.c_void_p).value for n in _lib.HOST_ENTRY_POINTS]
+    swapped = list(real)
+    swapped[_lib.HOST_ENTRY_POINTS.index(name)] = ctypes.cast(fn, ctypes.c_void_p).value
+    host.init(*swapped)
+    try:
+        yield
+    finally:
+        host.init(*real)
+
+
+@pytest.mark.parametrize("name", ["fmoe_route_topk", "fmoe_grouped_gemm", "fmoe_combine", "fmoe_quant_rows_e4m3"])
+def test_a_launch_error_is_raised_and_nothing_is_issued_again(name, monkeypatch):
+    """A launch error (forced on the host: the entry point returns the status and launches nothing) raises what the Python
+    code raises for it; the operator is not tried a second time."""
+    from fast_moe_amd import FastMoELayer
+    from fast_moe_amd.kernels.hip import _lib, ops
+    r = ops.route_topk(dev(torch.rand(16, 4)), 2)
+    x, w = dev(randn((16, 64), 1)), dev(randn((4, 32, 64), 2)).permute(0, 2, 1)
+    value = dev(randn((32, 64), 3))
+    layer = FastMoELayer(64, 96, 64, 4, dtype=BF16).to(BF16).cuda()
+    calls = {"fmoe_route_topk": lambda: ops.route_topk(dev(torch.rand(16, 4)), 2),
+             "fmoe_grouped_gemm": lambda: ops.grouped_gemm(r["offsets"], value, w, total_rows=32),
+             "fmoe_combine": lambda: ops.combine(value, r["reverse_index"], r["gates"], r["gate_index"]),
+             "fmoe_quant_rows_e4m3": lambda: ops.quant_rows_fp8(x)}
+    issued = []
+    fails = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: issued.append(name) or 4)     # FMOE_ERR_LAUNCH
+    monkeypatch.setattr(_lib.load(), name, lambda *a: pytest.fail("issued again by the Python code"))
+    with torch.no_grad():
+        for fn in [calls[name]] + ([] if name == "fmoe_quant_rows_e4m3" else [lambda: layer(x.view(1, 16, 64), 2)]):
+            issued.clear()
+            with entry_point(name, fails), pytest.raises(RuntimeError, match=f"{name} failed .status 4"):
+                fn()
+            assert issued == [name]
