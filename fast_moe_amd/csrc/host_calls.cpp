@@ -77,7 +77,7 @@ bool same_device(const at::Tensor& a, const at::Tensor& b) { return !b.defined()
 bool i64_list(const at::Tensor& t, int64_t n) { return t.scalar_type() == at::kLong && t.is_contiguous() && t.numel() == n; }
 
 struct Routing {
-    at::Tensor topk_idx, gates, lengths, offsets, gate_index, token_index, reverse_index;
+    at::Tensor topk_idx, gates, lengths, offsets, gate_index, token_index, reverse_index, workspace;
 };
 
 bool route_ok(const at::Tensor& scores, int64_t k, const void** data) {
@@ -89,7 +89,7 @@ bool route_ok(const at::Tensor& scores, int64_t k, const void** data) {
     return k >= 1 && k <= E && E <= INT32_MAX;
 }
 
-int route(const at::Tensor& scores, const void* data, int64_t k, int64_t mode, void* stream, Routing& r) {
+void allocate(const at::Tensor& scores, int64_t k, Routing& r) {
     const int64_t T = scores.size(0), E = scores.size(1);
     r.topk_idx = empty({T, k}, at::kLong, scores);
     r.gates = empty({T, k}, scores.scalar_type(), scores);
@@ -99,11 +99,14 @@ int route(const at::Tensor& scores, const void* data, int64_t k, int64_t mode, v
     r.token_index = empty({T * k}, at::kLong, scores);
     r.reverse_index = empty({T, k}, at::kLong, scores);
     const size_t ws_bytes = route_workspace_bytes(T, (int)E, (int)k);
-    const at::Tensor ws = empty({(int64_t)(ws_bytes ? ws_bytes : 1)}, at::kByte, scores);
-    return c_route_topk(data, dtype_code(scores.scalar_type()), T, (int)E, (int)k, (int)mode, r.topk_idx.data_ptr<int64_t>(),
-                        r.gates.data_ptr(), r.lengths.data_ptr<int64_t>(), r.offsets.data_ptr<int64_t>(),
-                        r.gate_index.data_ptr<int64_t>(), r.token_index.data_ptr<int64_t>(),
-                        r.reverse_index.data_ptr<int64_t>(), ws.data_ptr(), ws_bytes, stream);
+    r.workspace = empty({(int64_t)(ws_bytes ? ws_bytes : 1)}, at::kByte, scores);
+}
+
+int route(const at::Tensor& scores, const void* data, int64_t k, int64_t mode, void* stream, const Routing& r) {
+    return c_route_topk(data, dtype_code(scores.scalar_type()), scores.size(0), (int)scores.size(1), (int)k, (int)mode,
+                        r.topk_idx.data_ptr<int64_t>(), r.gates.data_ptr(), r.lengths.data_ptr<int64_t>(),
+                        r.offsets.data_ptr<int64_t>(), r.gate_index.data_ptr<int64_t>(), r.token_index.data_ptr<int64_t>(),
+                        r.reverse_index.data_ptr<int64_t>(), r.workspace.data_ptr(), r.workspace.numel(), stream);
 }
 
 struct GemmArgs {
@@ -174,12 +177,12 @@ bool gemm_ok(const GemmArgs& g, fmoe_gemm_desc& d) {
     return true;
 }
 
-int gemm(fmoe_gemm_desc& d, const at::Tensor& like, void* stream, at::Tensor& out) {
-    out = empty({d.total_rows + kSlackRows, d.n}, d.out_dtype == FMOE_F32 ? at::kFloat : at::kBFloat16, like)
-              .narrow(0, 0, d.total_rows);
+at::Tensor allocate(fmoe_gemm_desc& d, const at::Tensor& like) {
+    const at::Tensor out = empty({d.total_rows + kSlackRows, d.n}, d.out_dtype == FMOE_F32 ? at::kFloat : at::kBFloat16, like)
+                               .narrow(0, 0, d.total_rows);
     d.out = out.data_ptr();
     d.out_stride_row = out.stride(0);
-    return c_grouped_gemm(&d, stream);
+    return out;
 }
 
 struct Combine {
@@ -219,8 +222,9 @@ bool combine_ok(Combine& c) {
     return true;
 }
 
-int combine(const Combine& c, void* stream, at::Tensor& out) {
-    out = empty({c.T, c.D}, c.out_dtype, c.value);
+at::Tensor allocate(const Combine& c) { return empty({c.T, c.D}, c.out_dtype, c.value); }
+
+int combine(const Combine& c, const at::Tensor& out, void* stream) {
     return c_combine(c.value_data, c.code, c.T, (int)c.K, c.D, c.value.stride(0), c.reverse_data, c.gates_data, c.g_code, c.cols,
                      c.sr, c.sc, c.index_data, out.data_ptr(), dtype_code(c.out_dtype), stream);
 }
@@ -256,7 +260,11 @@ PyObject* py_route_topk(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!scores.defined() || !as_int(args[1], &k) || !as_int(args[2], &mode) || !as_int(args[3], &stream)) return none();
     Routing r;
     const void* data;
-    const int status = run([&] { return route_ok(scores, k, &data); }, [&] { return route(scores, data, k, mode, (void*)stream, r); });
+    const int status = run([&] { return route_ok(scores, k, &data); },
+                           [&] {
+                               allocate(scores, k, r);
+                               return route(scores, data, k, mode, (void*)stream, r);
+                           });
     if (raised(status, "fmoe_route_topk")) return nullptr;
     if (status != FMOE_OK) return none();
     PyObject* out = PyTuple_New(7);
@@ -285,7 +293,11 @@ PyObject* py_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         return none();
     at::Tensor out;
     fmoe_gemm_desc d;
-    const int status = run([&] { return gemm_ok(g, d); }, [&] { return gemm(d, g.a, (void*)stream, out); });
+    const int status = run([&] { return gemm_ok(g, d); },
+                           [&] {
+                               out = allocate(d, g.a);
+                               return c_grouped_gemm(&d, (void*)stream);
+                           });
     if (raised(status, "fmoe_grouped_gemm")) return nullptr;
     return status == FMOE_OK ? wrap(out) : none();
     END_HANDLE_TH_ERRORS
@@ -303,7 +315,11 @@ PyObject* py_combine(PyObject*, PyObject* const* args, Py_ssize_t n) {
         !optional_tensor(args[3], &c.gates_index) || !as_int(args[4], &stream))
         return none();
     at::Tensor out;
-    const int status = run([&] { return combine_ok(c); }, [&] { return combine(c, (void*)stream, out); });
+    const int status = run([&] { return combine_ok(c); },
+                           [&] {
+                               out = allocate(c);
+                               return combine(c, out, (void*)stream);
+                           });
     if (raised(status, "fmoe_combine")) return nullptr;
     return status == FMOE_OK ? wrap(out) : none();
     END_HANDLE_TH_ERRORS
@@ -350,21 +366,20 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (!t->defined()) return none();
     if (!as_int(args[6], &k) || !as_int(args[7], &mode) || !as_int(args[8], &epilogue) || !as_int(args[9], &stream))
         return none();
-    at::Tensor y;
+    at::Tensor hidden, rows, y;
     const void* data;
+    Routing r;
+    fmoe_gemm_desc up, down;
+    Combine merge;
     const char* what = "fmoe_route_topk";
+    // All operands of the four launches, intermediates included, exist and are checked before the first launch: a call that
+    // is declined has routed nothing.
     const int status = run(
         [&] {
-            return x.dim() == 2 && scores.dim() == 2 && scores.size(0) == x.size(0) && w1.dim() == 3 &&
-                   w1.size(0) == scores.size(1) && scores.device() == x.device() && route_ok(scores, k, &data);
-        },
-        [&] {
-            Routing r;
-            if (const int rc = route(scores, data, k, mode, (void*)stream, r)) return rc;
-            RECORD_USER_SCOPE("## expert_forward##");
-            what = "fmoe_grouped_gemm";
-            at::Tensor hidden, rows;
-            fmoe_gemm_desc d;
+            if (x.dim() != 2 || scores.dim() != 2 || scores.size(0) != x.size(0) || w1.dim() != 3 ||
+                w1.size(0) != scores.size(1) || scores.device() != x.device() || !route_ok(scores, k, &data))
+                return false;
+            allocate(scores, k, r);
             GemmArgs g;
             g.offsets = r.offsets;
             g.a = x;
@@ -374,23 +389,32 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
             g.total_rows = x.size(0) * k;
             g.index_div = k;
             g.epilogue = epilogue;
-            if (!gemm_ok(g, d)) return kDeclined;
-            if (const int rc = gemm(d, x, (void*)stream, hidden)) return rc;
-            GemmArgs down;
-            down.offsets = r.offsets;
-            down.a = hidden;
-            down.b = w2;
-            down.bias = b2;
-            down.total_rows = hidden.size(0);
-            if (!gemm_ok(down, d)) return kDeclined;
-            if (const int rc = gemm(d, x, (void*)stream, rows)) return rc;
+            if (!gemm_ok(g, up)) return false;
+            hidden = allocate(up, x);
+            g = GemmArgs();
+            g.offsets = r.offsets;
+            g.a = hidden;
+            g.b = w2;
+            g.bias = b2;
+            g.total_rows = hidden.size(0);
+            if (!gemm_ok(g, down)) return false;
+            rows = allocate(down, x);
+            merge.value = rows;
+            merge.reverse = r.reverse_index;
+            merge.gates = r.gates;
+            merge.gates_index = r.gate_index;
+            if (!combine_ok(merge)) return false;
+            y = allocate(merge);
+            return true;
+        },
+        [&] {
+            if (const int rc = route(scores, data, k, mode, (void*)stream, r)) return rc;
+            RECORD_USER_SCOPE("## expert_forward##");
+            what = "fmoe_grouped_gemm";
+            if (const int rc = c_grouped_gemm(&up, (void*)stream)) return rc;
+            if (const int rc = c_grouped_gemm(&down, (void*)stream)) return rc;
             what = "fmoe_combine";
-            Combine c;
-            c.value = rows;
-            c.reverse = r.reverse_index;
-            c.gates = r.gates;
-            c.gates_index = r.gate_index;
-            return combine_ok(c) ? combine(c, (void*)stream, y) : kDeclined;
+            return combine(merge, y, (void*)stream);
         });
     if (raised(status, what)) return nullptr;
     return status == FMOE_OK ? wrap(y) : none();

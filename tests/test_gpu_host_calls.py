@@ -141,6 +141,7 @@ def test_a_launch_error_is_raised_and_nothing_is_issued_again(name, monkeypatch)
              "fmoe_quant_rows_e4m3": lambda: ops.quant_rows_fp8(x)}
     issued = []
     fails = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: issued.append(name) or 4)     # FMOE_ERR_LAUNCH
+    _lib.host()
     monkeypatch.setattr(_lib.load(), name, lambda *a: pytest.fail("issued again by the Python code"))
     with torch.no_grad():
         for fn in [calls[name]] + ([] if name == "fmoe_quant_rows_e4m3" else [lambda: layer(x.view(1, 16, 64), 2)]):
@@ -148,3 +149,36 @@ def test_a_launch_error_is_raised_and_nothing_is_issued_again(name, monkeypatch)
             with entry_point(name, fails), pytest.raises(RuntimeError, match=f"{name} failed .status 4"):
                 fn()
             assert issued == [name]
+
+
+@pytest.mark.parametrize("case", ["experts of another dtype", "no tokens", "a bias of other strides", "plain"])
+def test_the_layer_routes_once(case, monkeypatch):
+    """A layer call has issued its routing once, whether the host module takes the call whole or declines it (the first case
+    is a default-constructed layer: bf16 experts under an fp32 gate and fp32 tokens)."""
+    from fast_moe_amd import FastMoELayer
+    from fast_moe_amd.kernels.hip import _lib
+    layer = FastMoELayer(64, 96, 64, 4, dtype=BF16).cuda()
+    if case != "experts of another dtype":
+        layer = layer.to(BF16)
+    if case == "a bias of other strides":       # (only the second GEMM's operands tell)
+        layer._experts_bias.data = torch.zeros(64, 4, dtype=BF16, device="cuda").t()
+    x = dev(randn((1, 0 if case == "no tokens" else 16, 64), 1).to(layer.gate.gate.weight.dtype))
+    lib = _lib.load()
+    _lib.host()         # (takes the entry points' addresses: before one is replaced below)
+    routed = []
+    proto = ctypes.CFUNCTYPE(ctypes.c_int, *lib.fmoe_route_topk.argtypes)
+    real = proto(ctypes.cast(lib["fmoe_route_topk"], ctypes.c_void_p).value)
+
+    def native(*a):
+        routed.append("native")
+        return real(*a)
+
+    def python(*a, fn=lib.fmoe_route_topk):
+        routed.append("python")
+        return fn(*a)
+
+    calls = proto(native)
+    monkeypatch.setattr(lib, "fmoe_route_topk", python)
+    with torch.no_grad(), entry_point("fmoe_route_topk", calls):
+        y = layer(x, 2)
+    assert len(routed) == 1 and y.shape == x.shape
