@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from ctypes import POINTER, c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_uint8, c_void_p
 
 _PKG_DIR = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
@@ -133,17 +134,28 @@ HOST_ENTRY_POINTS = ("fmoe_route_workspace_bytes", "fmoe_route_topk", "fmoe_grou
 _host = None
 
 
+class _Declines:
+    """In the place of the extension module where that does not load: every call is left to the Python code in ops.py."""
+
+    route_topk = grouped_gemm = combine = quant_rows = mlp_forward = staticmethod(lambda *args: None)
+
+
 def host():
-    """The extension module whose functions take a forward operator's call whole or return None (csrc/host_calls.cpp)."""
+    """The extension module whose functions take a forward operator's call whole or return None (csrc/host_calls.cpp).  It
+    saves host time only: without it (not built, or built for another torch) the same kernels are launched from Python."""
     global _host
     if _host is None:
         lib = load()
         try:
             from ... import _host as mod
+            import torch
+            if mod.torch_version != torch.__version__.split("+")[0]:
+                raise ImportError(f"built for torch {mod.torch_version}, this is {torch.__version__}")
+            mod.init(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in HOST_ENTRY_POINTS))
         except ImportError as e:
-            raise RuntimeError(f"fast_moe_amd/_host.so is missing or does not load ({e}): build it with "
-                               f"`python -m fast_moe_amd.build`") from e
-        mod.init(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in HOST_ENTRY_POINTS))
+            warnings.warn(f"fast_moe_amd/_host.so is not used ({e}); calls are issued from Python, which takes longer on the "
+                          f"host. Build it with `python -m fast_moe_amd.build`", RuntimeWarning, stacklevel=3)
+            mod = _Declines()
         _host = mod
     return _host
 

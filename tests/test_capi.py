@@ -312,3 +312,33 @@ def test_combine_helper_opens_the_reference_profiler_range():
     import inspect
     from fast_moe.utils import utils as u
     assert '"## combine ##"' in inspect.getsource(u._combine)
+
+
+@pytest.mark.parametrize("how", ["missing", "another torch"])
+def test_without_the_host_module_calls_are_left_to_python(lib, how, monkeypatch):
+    """The library depends on no torch: an extension module that does not load (none built, or one for another torch) costs
+    a warning and host time, not the package."""
+    import sys
+    import types
+
+    import fast_moe_amd
+    from fast_moe_amd.kernels.hip import _lib
+    monkeypatch.setattr(_lib, "_host", None)
+    other = types.ModuleType("fast_moe_amd._host")
+    other.torch_version = "1.0"
+    monkeypatch.setitem(sys.modules, "fast_moe_amd._host", None if how == "missing" else other)
+    monkeypatch.setattr(fast_moe_amd, "_host", other, raising=False)
+    if how == "missing":
+        monkeypatch.delattr(fast_moe_amd, "_host")
+    with pytest.warns(RuntimeWarning, match="_host.so is not used"):
+        host = _lib.host()
+    assert host is _lib.host()      # once
+    for name in ("route_topk", "grouped_gemm", "combine", "quant_rows", "mlp_forward"):
+        assert getattr(host, name)(1, 2, 3) is None
+
+
+def test_the_built_host_module_loads(lib):
+    from fast_moe_amd import build
+    from fast_moe_amd.kernels.hip import _lib
+    if os.path.exists(build.HOST_PATH):
+        assert _lib.host().torch_version
