@@ -111,8 +111,8 @@ class FastMoELayer(nn.Module):
             raise NotImplementedError(f"FastMoELayer: the HIP kernels take bf16 or fp32 activations, got {x.dtype}")
         original_shape = x.shape
         k = num_experts_per_tok
-        if getattr(self.route, "__func__", None) is FastMoELayer.route and x.ndim == 3:
-            # the same steps as below, issued by one native call
+        if getattr(self.route, "__func__", None) is _ROUTE and x.ndim == 3:
+            # the same steps as below, issued by one native call (a route() of a subclass's or a caller's own is asked)
             scores = self.gate(x).reshape(-1, self.num_experts)
             y = _lib.host().mlp_forward(
                 scores, x.reshape(-1, self.input_dim), self._experts_hidden_w.permute(0, 2, 1), self._experts_hidden_bias,
@@ -135,3 +135,6 @@ class FastMoELayer(nn.Module):
                 total_rows=hidden.shape[0], bias=self._experts_bias.to(x.dtype), epilogue=EPI_NONE)
             y = ops.combine(out_rows, r["reverse_index"], r["gates"], r["gate_index"])
         return y.view(original_shape[0], original_shape[1], self.output_dim)
+
+
+_ROUTE = FastMoELayer.route     # what the native call stands for

@@ -91,6 +91,27 @@ def test_layer_forward(B, S, dtype):
         assert other.asked
 
 
+@pytest.mark.parametrize("where", ["class", "object"])
+def test_a_replaced_route_is_asked(where, monkeypatch):
+    from fast_moe_amd import FastMoELayer
+    layer = FastMoELayer(64, 96, 64, 8, dtype=BF16).to(BF16).cuda()
+    x = dev(randn((1, 33, 64), 1))
+    asked, real = [], FastMoELayer.route
+
+    def route(self, x, k):
+        asked.append(k)
+        return real(self, x, k)
+
+    with torch.no_grad():
+        want = layer(x, 2)
+        if where == "class":
+            monkeypatch.setattr(FastMoELayer, "route", route)
+        else:
+            layer.route = route.__get__(layer)
+        same(layer(x, 2), want)
+    assert asked == [2]
+
+
 def test_refusals_are_the_python_codes():
     from fast_moe_amd.kernels.hip import ops
     r = make_routing(16, 4, 2, seed=1)
