@@ -240,3 +240,19 @@ def test_rows_that_are_columns_in_memory(E, K, N):
     got = q.permute(0, 2, 1).view(torch.uint8).cpu().numpy()
     nan = (q_ref & 0x7F) == 0x7F          # (the sign of a NaN code is not defined by the arithmetic)
     assert np.array_equal((got & 0x7F) == 0x7F, nan) and np.array_equal(got[~nan], q_ref[~nan])
+
+
+def test_the_column_form_allocates_scratch_only_where_it_runs():
+    """The two-launch form writes rows of consecutive bytes: a result laid out like its [E, K, N] input is left to the other
+    kernel, without a scratch buffer."""
+    from fast_moe_amd.kernels import moe_fp8
+    w = torch.randn(2, 128, 64, device="cuda").to(torch.bfloat16)
+
+    def allocations(fn):
+        fn()
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        fn()
+        return torch.cuda.memory_stats()["allocation.all.allocated"] - before
+
+    assert allocations(lambda: moe_fp8.bmm_weight_rowwise_quant_fp8(w)) == 2        # bytes and scales
+    assert allocations(lambda: moe_fp8.quantize_expert_weights(w)) == 3
