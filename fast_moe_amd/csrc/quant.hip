@@ -507,12 +507,22 @@ extern "C" int fmoe_quant_rows_e4m3(const void* a, int a_dtype, int64_t batch, i
     return check_launch("fmoe_quant_rows_e4m3");
 }
 
+// Where the two launches are faster than the one of the other form.  A caller that allocates the scratch through torch pays
+// 3 us of host time for the second launch and the scratch, and a serial walk over a few columns is short: us per call,
+// lane per row / two launches, 40 columns: 15.0 / 18.4 (64 rows), 17.1 / 18.2 (32768); 48 columns 17.9 / 18.4 and 21.0 / 18.4.
+// With many rows the crossing moves down: 2^16 rows x 24 columns 15.2 / 18.4, 2^19 x 16 15.4 / 24.4, 2^19 x 24 30.9 / 26.1.
+// Under 16 rows the other form is a wave per row, good for more columns: 8 rows x 512 columns 15.3 / 18.9, 8 x 65536 248 / 19.
+static bool cols_pays(int64_t total_rows, int64_t rows, int64_t cols) {
+    if (rows < 16) return cols > 4096;
+    return cols > 40 || (cols > 16 && total_rows > ((int64_t)1 << 17));
+}
+
 // What the two-launch form takes: bf16, memory rows of whole aligned 16-byte chunks, result rows of whole dwords.
 static bool takes_cols(int a_dtype, int64_t batch, int64_t rows, int64_t cols, int64_t a_sb, int64_t a_sr, int64_t a_sc,
                        int apply_silu) {
     return a_dtype == FMOE_BF16 && !apply_silu && a_sr == 1 && a_sc >= rows && rows % 8 == 0 && cols % 4 == 0 &&
            a_sc % 8 == 0 && (batch == 1 || a_sb % 8 == 0) && batch >= 1 && batch <= 65535 && rows >= 8 &&
-           (cols + kColTileK - 1) / kColTileK <= 65535;
+           (cols + kColTileK - 1) / kColTileK <= 65535 && cols_pays(batch * rows, rows, cols);
 }
 
 extern "C" size_t fmoe_quant_rows_workspace_bytes(int a_dtype, int64_t batch, int64_t rows, int64_t cols, int64_t a_sb,

@@ -196,10 +196,12 @@ def quant_rows_fp8(a: torch.Tensor, apply_silu: bool = False, reciprocal_scale: 
     lib = _lib.load()
     args = (a3.data_ptr(), _DTYPE_CODE[a.dtype], B, Rr, C, *a3.stride(), int(apply_silu), q3.data_ptr(), *q3.stride(),
             scale.data_ptr(), int(reciprocal_scale))
+    ws_bytes = 0
     if a3.stride(1) == 1 and a3.stride(2) != 1 and not out_like_input:      # rows are columns in memory, but not of q
         ws_bytes = lib.fmoe_quant_rows_workspace_bytes(*args[1:8], args[8])
+    if ws_bytes:
         ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
-        rc = lib.fmoe_quant_rows_e4m3_ws(*args, _ptr(ws), ws_bytes, _stream(a))
+        rc = lib.fmoe_quant_rows_e4m3_ws(*args, ws.data_ptr(), ws_bytes, _stream(a))
     else:
         rc = lib.fmoe_quant_rows_e4m3(*args, _stream(a))
     _lib.check(rc, "fmoe_quant_rows_e4m3")
