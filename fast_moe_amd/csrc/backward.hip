@@ -434,6 +434,31 @@ __global__ __launch_bounds__(256) void invert_sort_kernel(const int64_t* __restr
     }
 }
 
+// K between the two: a block ranks the entries of as many whole tokens as make about kRankEntries, every entry counting the
+// smaller ones of its token in LDS.  An insertion in place, which this stands for, is K^2 dependent steps of one lane
+// through memory.  us per call, in place / ranked / index_put and a segmented sort on the torch side:
+//   4096 tokens, K = 16  39 / 9 / 34      K = 32  136 / 10 / 34     K = 64  494 / 15 / 70
+//  32768 tokens, K = 16  50 / 16 / 40     K = 32  167 / 35 / 58     K = 64  598 / 76 / 393
+constexpr int kRankEntries = 1024, kRankMax = 4096;
+__global__ __launch_bounds__(256) void invert_rank_kernel(const int64_t* __restrict__ index, int64_t T, int K, int tokens,
+                                                          int64_t* __restrict__ reverse) {
+    __shared__ int s_pos[kRankMax];
+    const int64_t t0 = (int64_t)blockIdx.x * tokens, first = t0 * K;
+    const int n = (int)(T - t0 < tokens ? T - t0 : tokens) * K;
+    for (int e = threadIdx.x; e < n; e += 256)      // (positions fit 32 bits: the launcher checks)
+        s_pos[e] = (int)checked_position(index, T * K, reverse[first + e], first + e);
+    __syncthreads();
+    for (int e = threadIdx.x; e < n; e += 256) {
+        const int base = e / K * K, x = s_pos[e];
+        int rank = 0;
+        for (int j = 0; j < K; ++j) {               // (equal ones, "no row", keep their order)
+            const int y = s_pos[base + j];
+            rank += y < x || (y == x && base + j < e);
+        }
+        reverse[first + base + rank] = x;
+    }
+}
+
 // Gradient of gates[t, j] = s_j / max(sum_i s_i, 1e-12), s_j = scores[t, idx[t, j]], with respect to the scores: one wave
 // per token, lane j holds slot j (K <= 64), the row of E gradients is written whole.  Every step is rounded to the scores'
 // type where torch's chain of gather, sum, clamp_min and div rounds its intermediate tensors, so the result is that
@@ -633,8 +658,13 @@ extern "C" int fmoe_invert_index(const int64_t* index, int64_t T, int K, int64_t
     invert_scatter_kernel<<<(unsigned)((R + 255) / 256), 256, 0, s>>>(index, R, reverse);
     if (int rc = check_launch("fmoe_invert_index")) return rc;
     const unsigned blocks = (unsigned)((T + 255) / 256);
-    if (K <= 8) invert_sort_kernel<8><<<blocks, 256, 0, s>>>(index, T, K, reverse);
-    else invert_sort_kernel<0><<<blocks, 256, 0, s>>>(index, T, K, reverse);
+    if (K <= 8) {
+        invert_sort_kernel<8><<<blocks, 256, 0, s>>>(index, T, K, reverse);
+    } else if (K <= kRankMax && R < ((int64_t)1 << 31)) {
+        const int tokens = K < kRankEntries ? kRankEntries / K : 1;
+        invert_rank_kernel<<<(unsigned)((T + tokens - 1) / tokens), 256, 0, s>>>(index, T, K, tokens, reverse);
+    } else
+        invert_sort_kernel<0><<<blocks, 256, 0, s>>>(index, T, K, reverse);
     return check_launch("fmoe_invert_index");
 }
 

@@ -668,7 +668,8 @@ def test_segment_colsum(lens, cols, dtype):
         assert torch.equal(again, out)
 
 
-@pytest.mark.parametrize("T,K", [(1, 1), (5, 8), (257, 3), (4097, 8), (300, 9), (33, 70)])
+@pytest.mark.parametrize("T,K", [(1, 1), (5, 8), (257, 3), (4097, 8), (300, 9), (33, 70), (1000, 33), (65, 64),
+                                 (5, 1000), (3, 4096), (2, 4100)])
 def test_invert_index(T, K):
     from fast_moe_amd.kernels.hip import ops
     g = torch.Generator().manual_seed(T * 100 + K)
