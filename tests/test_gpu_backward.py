@@ -685,7 +685,8 @@ def test_invert_index(T, K):
         assert torch.equal(ops.invert_index(dev(broken.view(T, K))).cpu(), want.view(T, K).sort(dim=1).values)
 
 
-@pytest.mark.parametrize("T,E,K", [(1, 4, 2), (7, 8, 8), (1021, 12, 3), (130, 65, 1), (257, 128, 8), (65, 200, 64)])
+@pytest.mark.parametrize("T,E,K", [(1, 4, 2), (7, 8, 8), (1021, 12, 3), (130, 65, 1), (257, 128, 8), (65, 200, 64),
+                                   (30, 512, 64)])
 @pytest.mark.parametrize("dtype", [BF16, torch.float32])
 def test_topk_gates_backward(T, E, K, dtype):
     """The gate values and their gradient against the chain of torch ops they stand for: bf16 rounds where the chain
@@ -711,3 +712,19 @@ def test_topk_gates_backward(T, E, K, dtype):
     grad, = torch.autograd.grad(gates2, s2, dev(dg), create_graph=True)
     assert grad.requires_grad
     assert ((grad.detach().cpu().float() - s.grad.cpu().float()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("T,E,K", [(5, 511, 3), (9, 513, 8), (6, 1100, 64), (4, 1024, 1)])
+@pytest.mark.parametrize("dtype", [BF16, torch.float32])
+def test_gate_gradient_rows_of_many_experts(T, E, K, dtype):
+    """Rows of gradients in chunks of 512 experts, more than routing takes: picks on either side of a chunk's edge, each
+    gradient where its expert is and zeros elsewhere.  A call on the picked columns alone gives the same values."""
+    from fast_moe_amd.kernels.hip import ops
+    g = torch.Generator().manual_seed(E + K)
+    idx = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(T)])
+    edge = [e for e in (0, 511, 512, E - 1) if e < E][:K]
+    idx[0] = torch.tensor(edge + [e for e in range(1, 400)][:K - len(edge)])
+    scores, dg = torch.rand(T, E, generator=g).to(dtype), torch.randn(T, K, generator=g).to(dtype)
+    got = ops.gate_l1_bwd(dev(scores), dev(idx), dev(dg)).cpu()
+    small = ops.gate_l1_bwd(dev(scores.gather(1, idx)), dev(torch.arange(K).expand(T, K).contiguous()), dev(dg)).cpu()
+    assert torch.equal(got, torch.zeros_like(scores).scatter_(1, idx, small))
