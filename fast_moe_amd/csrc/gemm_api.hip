@@ -192,7 +192,7 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
                           (d->b_stride_e % chunk) == 0 && (d->a_stride_row % chunk) == 0 &&
                           (d->a_stride_e % chunk) == 0 && aligned16(d->a) && aligned16(d->b) &&
                           (!swiglu || aligned16(d->b2)) && near_tr;
-    p.ring_short = short_tr || (short_ok && fast && near);
+    p.ring_short = short_tr || (short_ok && fast && near && ring_short_pays(p, esize, d->epilogue));
     // the second product exists in that kernel only; a caller that is turned away runs two
     // GEMMs and adds
     if (two)

@@ -148,23 +148,28 @@ inline bool ring_short_takes(int esize, int64_t k, int num_experts, int64_t tota
            total_rows < ((int64_t)1 << 31) && lds_per_block() >= TileRingS::LDS_BYTES;
 }
 
-// Where both take a call (weights with k contiguous).  Both read large launches at 5.9 - 6.0 TB/s (a read loop without
-// anything else gets 6.3 on this access pattern); they differ where a launch is a round or two of tiles, and in the cost of
-// a tile boundary.  us per GEMM, streaming kernel / ring:
-//   * up to one tile per CU the ring keeps 120 KB per CU in flight where a lone streaming block has 40:
-//     138 rows, 32 experts, 1728 -> 2 x 576 SwiGLU  30.2 / 22.5 (e4m3 19.5 / 16.6); 162 rows, 21 experts, 3648 -> 576  49.9 / 30.1
-//   * above that the streaming kernel's two blocks per CU leave fewer CUs without a tile in the last round:
-//     1000 rows, 63 experts, 1792 -> 2 x 640  52.4 / 61.4 (e4m3 28.1 / 32.7)
-//   * with many rounds that is gone; the ring is ahead where a weight row is 4 KB or longer (3000 rows, 64 experts,
-//     2048 -> 2 x 1408  143.7 / 136.9; 8000 rows, 128 experts, 4096 -> 2 x 1536  689 / 673, e4m3 378 / 362), behind where
-//     tiles are shorter (4096 rows, 128 experts, 1536 -> 4096  298.6 / 304.5; e4m3 158 / 163).
-template <int DT, int EPI>
-bool ring_short_pays(const GemmParams& p) {
-    constexpr int bn_out = EPI == FMOE_EPI_SWIGLU ? TileRingS::BN / 2 : TileRingS::BN;
+// Where it is taken although another kernel takes the call as well (weights with k contiguous; with n contiguous the other is
+// the element-load kernel and the ring always the faster one).  Only the row count is known here, not how the experts share
+// it, so the rule goes by bounds that hold for every load.  us per GEMM, the streaming kernel / the ring (GATED: the
+// register-staged kernel / the ring):
+//   * no more tiles than CUs, however the rows fall: the ring keeps 120 KB per CU in flight where a lone streaming block has 40.
+//     138 rows, 32 experts, 1728 -> 2 x 576 SwiGLU  30.2 / 22.5 (e4m3 19.5 / 16.6); 162 rows, 21 experts, 3648 -> 576
+//     49.9 / 30.1 (GATED 63.8 / 31.0)
+//   * beyond that one block per CU pays for a part-filled second round, where two blocks per CU hold it in the first:
+//     512 rows, 128 experts, 4096 -> 1536: nine tenths of the rows in one expert 108 / 135, uniform 307 / 291; 9000 rows, 100
+//     experts, 4096 -> 2 x 512 230 / 238; Zipf 243 / 258; 1000 rows, 63 experts, 1792 -> 2 x 640 52.4 / 61.4.  With twelve
+//     rounds it depends on the load still (8000 rows, 128 experts, 4096 -> 2 x 1536: uniform 659 / 647, Zipf 725 / 735).
+//   * GATED: 64 rows, 8 experts, 4096 -> 11008 142 / 154; 64 rows, 128 experts, 4096 -> 1536 125 / 148; 4096 rows, 128 experts,
+//     4096 -> 1536 uniform 341 / 323, Zipf 309 / 317.  With more than two rounds of tiles even if one expert had all rows, and
+//     whole pairs of K-slices, the ring is ahead by 3 to 11 % for every load: 8000 rows, 128 experts, 4096 -> 1536 uniform
+//     402 / 367, Zipf 413 / 384, one hot expert 389 / 370 (5000 rows, 60 experts, 1000 -> 2600, K in part: 132 / 147).
+inline bool ring_short_pays(const GemmParams& p, int esize, int epilogue) {
+    const int bn_out = epilogue == FMOE_EPI_SWIGLU ? TileRingS::BN / 2 : TileRingS::BN;
+    const int64_t cus = compute_units(), n_tiles = (p.N + bn_out - 1) / bn_out;
     const int64_t experts = p.E < p.total_rows ? p.E : p.total_rows;       // that can hold a row
-    const int64_t tiles = (p.total_rows / TileRingS::BM + experts) * ((p.N + bn_out - 1) / bn_out);
-    const int64_t cus = compute_units();
-    return tiles <= cus || (tiles > 3 * cus && (int64_t)p.K * (DT == kDtE4m3 ? 1 : 2) >= 4096);
+    if ((p.total_rows / TileRingS::BM + experts) * n_tiles <= cus) return true;
+    return epilogue == FMOE_EPI_GATED && p.K % (128 / esize) == 0 &&
+           (p.total_rows + TileRingS::BM - 1) / TileRingS::BM * n_tiles > 2 * cus;
 }
 
 // The 5-slot ring needs every byte of a 160 KB LDS, an even number of K-slices per tile,
@@ -226,7 +231,7 @@ int dispatch_tile(const GemmParams& p, int sel, hipStream_t stream) {
         case kSelStagedBig: return launch_gemm<TileBig, DT, EPI, kLoadChunks, A_SILU>(p, stream);
         case kSelStagedSmall:
             if constexpr (!A_SILU) {
-                if (p.ring_short && (EPI == FMOE_EPI_GATED || !stream_kernel_takes(p) || ring_short_pays<DT, EPI>(p)))
+                if (p.ring_short)
                     return DT == kDtE4m3 ? run_ring_short_fp8(p, EPI, stream) : run_ring_short_bf16(p, EPI, stream);
             }
             if constexpr (!A_SILU && EPI != FMOE_EPI_GATED) {

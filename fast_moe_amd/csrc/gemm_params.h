@@ -39,7 +39,7 @@ struct GemmParams {
     uint16_t* out;
     int64_t out_stride;
     int n_tiles;
-    int ring_short;                     // the ring on 64-row tiles takes the call
+    int ring_short;                     // the ring on 64-row tiles runs the call
     int vec_store;                      // 16-byte stores of 8 bf16 are legal
     int scale_vec;                      // e4m3: 16-byte loads of 4 weight scales are legal
     int scale_pow2;                     // e4m3: the caller promises that every scale is an exact power of two

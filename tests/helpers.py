@@ -76,3 +76,15 @@ def special_scores(T=64, E=16, seed=3):
     s[7, 2] = float("nan")
     s[7, 11] = float("inf")
     return s
+
+
+def kernels_run(fn):
+    """Names (with their template arguments) of the GPU kernels that ``fn`` launches, in order, from a trace of the call."""
+    import warnings
+    torch.cuda.synchronize()
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+            fn()
+            torch.cuda.synchronize()
+    return [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]

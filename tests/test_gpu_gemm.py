@@ -8,7 +8,7 @@ import torch
 
 from oracle import moe as o_moe
 from oracle import moe_fp8 as o_fp8
-from tests.helpers import BF16, assert_bf16_close, dev, make_routing, randn, skewed_topk, uniform
+from tests.helpers import BF16, assert_bf16_close, dev, kernels_run, make_routing, randn, skewed_topk, uniform
 from oracle import routing as o_routing
 
 pytestmark = pytest.mark.gpu
@@ -1102,7 +1102,8 @@ def test_fp32_kernel_tiles_and_weight_layouts(E, rows, K, N, layout, epi):
     (2, 3, 1000, 520, "nk", 2), (2, 3, 1000, 520, "kn", 2),
     (200, 900, 328, 72, "kn", 0), (130, 5000, 264, 1032, "kn", 2),  # more experts than lanes; more tiles than CUs
     (2, 150, 200, 320, "kn", 3), (40, 2000, 640, 2048, "kn", 3),
-    (3, 130, 272, 264, "fp8", 0), (3, 70, 384, 136, "fp8", 2), (8, 760, 4096, 10400, "fp8", 0),
+    (3, 280, 640, 32768, "nk", 3),                                  # more tiles than CUs with k contiguous
+    (3, 130, 272, 264, "fp8", 0), (3, 70, 384, 136, "fp8", 2), (8, 760, 4096, 2816, "fp8", 0),
 ])
 def test_ring_kernel_on_short_tiles(E, rows, K, N, layout, epi):
     """The ring on 64-row tiles (few rows per expert).  The operands are the left columns of wider
@@ -1133,6 +1134,8 @@ def test_ring_kernel_on_short_tiles(E, rows, K, N, layout, epi):
         ws = [(q.float() / s[..., None]).permute(0, 2, 1) for q, s in qw]
     assert ops.grouped_gemm(off, *args, plan_only=True, **kw) == _lib.PLAN_STAGED_SHORT
     out = ops.grouped_gemm(off, *args, **kw)
+    ran, = kernels_run(lambda: ops.grouped_gemm(off, *args, **kw))
+    assert "ring_kernel" in ran and "RingCfg<64," in ran, ran
     kw.pop("scales_pow2", None)
     assert layout != "fp8" or torch.equal(ops.grouped_gemm(off, *args, **kw), out)      # scales divided out instead
     for e in range(E):
@@ -1145,6 +1148,43 @@ def test_ring_kernel_on_short_tiles(E, rows, K, N, layout, epi):
         if epi == _lib.EPI_GATED:
             a = a * torch.nn.functional.silu(gate[lo:hi].double())
         assert_bf16_close(out[lo:hi], a.float(), rtol=1.6e-2, atol=4e-3, what=f"expert {e}")
+
+
+@pytest.mark.parametrize("E,rows,K,N,layout,epi,kernel", [
+    (8, 760, 4096, 3328, "nk", 0, "ring"), (8, 760, 4096, 3584, "nk", 0, "stream"),     # 247 / 266 tiles if the rows fall badly
+    (8, 760, 4096, 3328, "fp8", 0, "ring"), (8, 760, 4096, 3584, "fp8", 0, "stream"),
+    (128, 512, 4096, 1536, "nk", 2, "stream"), (128, 512, 4096, 1536, "fp8", 0, "stream"),
+    (128, 8000, 4096, 1536, "nk", 2, "stream"),                                         # many rounds of tiles
+    (200, 3, 1024, 8192, "nk", 0, "ring"),                                              # no more experts than rows can have one
+    (64, 64, 1024, 2048, "nk", 3, "staged"), (64, 5000, 1024, 1408, "nk", 3, "staged"),
+    (64, 5900, 1024, 1408, "nk", 3, "ring"), (64, 5900, 1000, 1408, "nk", 3, "staged"), # GATED: more than two rounds for certain
+    (128, 512, 4096, 1536, "kn", 2, "ring"),
+])
+def test_kernel_choice_for_few_rows(E, rows, K, N, layout, epi, kernel):
+    """Which kernel runs a call with few rows per expert, on either side of the rule's lines; the same for an even load and for
+    one expert with nine tenths of the rows (the host does not know the load)."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    x = torch.zeros(rows, K, dtype=BF16, device="cuda")
+    w = torch.zeros((E, K, N) if layout == "kn" else (E, N, K), dtype=BF16, device="cuda")
+    kw = dict(total_rows=rows, epilogue=epi)
+    args = (x, w if layout == "kn" else w.permute(0, 2, 1))
+    if layout == "fp8":
+        args = tuple(t.to(torch.float8_e4m3fn) for t in (x, w))
+        args = (args[0], args[1].permute(0, 2, 1))
+        kw.update(a_scale=torch.ones(rows, device="cuda"), b_scale=torch.ones(E, N, device="cuda"))
+    if epi == _lib.EPI_SWIGLU:
+        kw["b2"] = args[1]
+        if layout == "fp8":
+            kw["b2_scale"] = kw["b_scale"]
+    if epi == _lib.EPI_GATED:
+        kw["gate"] = torch.zeros(rows, N, dtype=BF16, device="cuda")
+    even = torch.arange(E + 1) * rows // E
+    hot = torch.cat([torch.zeros(1, dtype=torch.int64), (torch.arange(E) * (rows // 10) // max(E - 1, 1)) + rows - rows // 10])
+    want = {"ring": "grouped_gemm_ring_kernel<fmoe::RingCfg<64,", "stream": "grouped_gemm_stream_kernel<",
+            "staged": "grouped_gemm_kernel<fmoe::TileCfg<64, 256,"}[kernel]
+    for off in (even.cuda(), hot.cuda()):
+        ran, = kernels_run(lambda: ops.grouped_gemm(off, *args, **kw))
+        assert want in ran, ran
 
 
 @pytest.mark.parametrize("row_tiles", [1, 7, 28, 31, 32, 33, 59, 60, 61, 97])
