@@ -128,14 +128,27 @@ int launch_ring_cfg(GemmParams p, hipStream_t stream) {
 int run_ring_tail_bf16(const GemmParams& p, int epilogue, hipStream_t stream);
 int run_ring_tail_fp8(const GemmParams& p, int epilogue, hipStream_t stream);
 
-// What they take beyond the ring's own conditions: at least one pair of slices and a 16-byte chunk.  (An odd slice count
-// goes there as well; the 4-slot ring is left with more than 256 experts.)  On 9189 rows, 12 experts, 1000 <-> 2600
+// What they take beyond the ring's own conditions: at least one pair of slices and a 16-byte chunk.  On 9189 rows, 12 experts, 1000 <-> 2600
 // columns: weights with n contiguous 85 us per GEMM where the element-load kernel took 1368 and 1620; weights with k
 // contiguous 94 us against 99 on the register-staged kernel.
 inline bool ring_tail_takes(int esize, int64_t k, int num_experts, int64_t total_rows) {
     const int pair = 128 / esize, chunk = 16 / esize;
     return k > pair && k % pair != 0 && k % chunk == 0 && num_experts <= TileRing5W::kMaxExperts &&
            total_rows < ((int64_t)1 << 31) && lds_per_block() >= TileRing5W::LDS_BYTES;
+}
+
+// An odd number of whole slices is the 4-slot ring's as well, where it costs no half-empty pair but every slice comes as half
+// lines.  us per GEMM, 4-slot ring / tail kernel, K in slices:
+//   8192 rows, 8 experts, 1024 columns (one round of tiles)  bf16 3: 10.5 / 12.1   9: 14.5 / 15.1   17: 20.3 / 19.4
+//                                                           e4m3 3: 11.7 / 12.9   9: 15.9 / 16.4   17: 21.1 / 20.8
+//   16384 rows, 64 experts, 1408 columns (several)           bf16 3: 22.8 / 24.7   5: 26.9 / 27.4    7: 31.7 / 31.1
+// Scales divided out in the epilogue (no powers of two) leave the e4m3 tail kernel short of registers:
+//   one round  17: 21.3 / 21.6   21: 23.8 / 23.6        several  9: 39.7 / 39.8   17: 57.4 / 54.3
+inline bool ring_tail_pays(const GemmParams& p, int esize, int epilogue) {
+    const int slice = 64 / esize, bn_out = epilogue == FMOE_EPI_SWIGLU ? 128 : 256;
+    if (p.K % slice || p.b_sk != 1) return true;
+    const bool rounds = p.total_rows / 256 * ((p.N + bn_out - 1) / bn_out) > compute_units();   // however the rows fall
+    return p.K / slice >= (esize == 1 && !p.scale_pow2 ? (rounds ? 17 : 21) : (rounds ? 7 : 17));
 }
 
 // The ring on 64-row tiles (gemm_bf16_short.hip, gemm_fp8_short.hip): experts with a handful of rows.
@@ -189,7 +202,7 @@ int launch_ring(const GemmParams& p, hipStream_t stream) {
         }
         return fail(FMOE_ERR_UNSUPPORTED, "fmoe_grouped_gemm: row-indexed operands need bf16 and no epilogue");
     }
-    if (!p.k_window && ring_tail_takes(FP8 ? 1 : 2, p.K, p.E, p.total_rows))
+    if (!p.k_window && ring_tail_takes(FP8 ? 1 : 2, p.K, p.E, p.total_rows) && ring_tail_pays(p, FP8 ? 1 : 2, EPI))
         return FP8 ? run_ring_tail_fp8(p, EPI, stream) : run_ring_tail_bf16(p, EPI, stream);
     if (p.b_sn == 1 && p.b_sk != 1) {      // N-contiguous weights in place (the caller checked pair_ok's terms)
         if constexpr (!FP8) {

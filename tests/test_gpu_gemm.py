@@ -13,6 +13,8 @@ from oracle import routing as o_routing
 
 pytestmark = pytest.mark.gpu
 
+KTAIL = ", true>(fmoe::GemmParams)"      # the ring kernel's last template argument, in a trace
+
 # kernels/tests/moe_test.py:35-84: default assert_close for bf16 is rtol 1.6e-2, atol 1e-5
 REF_RTOL, REF_ATOL = 1.6e-2, 1e-5
 
@@ -1014,9 +1016,10 @@ def test_scales_applied_by_the_mfma_equal_scales_divided_out_in_the_epilogue(E, 
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
     (3, 700, 72, 264, "nk", 0), (3, 700, 120, 136, "kn", 0),        # one pair of K-slices and the shortest / longest rest
     (2, 1000, 1000, 520, "nk", 2), (2, 1000, 1000, 520, "kn", 2),
-    (5, 600, 2600, 256, "kn", 0), (4, 500, 96, 128, "nk", 1),       # 96: an odd number of whole slices
+    (5, 600, 2600, 256, "kn", 0), (4, 500, 544, 128, "nk", 1),      # 544: an odd number of whole slices
     (200, 20000, 136, 72, "nk", 1), (2, 513, 200, 320, "kn", 3),
     (3, 700, 144, 264, "fp8", 0), (2, 1000, 1040, 136, "fp8", 2), (4, 600, 240, 512, "fp8", 1),
+    (3, 700, 1344, 136, "fp8", 0),
 ])
 def test_ring_kernel_contraction_tails(E, rows, K, N, layout, epi):
     """K that is no whole number of K-slice pairs: the last pair overlaps the one before it and is
@@ -1047,6 +1050,8 @@ def test_ring_kernel_contraction_tails(E, rows, K, N, layout, epi):
         ws = [(q.float() / s[..., None]).permute(0, 2, 1) for q, s in qw]
     assert ops.grouped_gemm(off, *args, plan_only=True, **kw) == _lib.PLAN_RING
     out = ops.grouped_gemm(off, *args, **kw)
+    ran, = kernels_run(lambda: ops.grouped_gemm(off, *args, **kw))
+    assert KTAIL in ran, ran
     kw.pop("scales_pow2", None)
     assert layout != "fp8" or torch.equal(ops.grouped_gemm(off, *args, **kw), out)      # scales divided out instead
     for e in range(E):
@@ -1059,6 +1064,32 @@ def test_ring_kernel_contraction_tails(E, rows, K, N, layout, epi):
         if epi == _lib.EPI_GATED:
             a = a * torch.nn.functional.silu(gate[lo:hi].double())
         assert_bf16_close(out[lo:hi], a.float(), rtol=1.6e-2, atol=4e-3, what=f"expert {e}")
+
+
+@pytest.mark.parametrize("E,rows,K,N,dtype,tail", [
+    (3, 700, 96, 264, "bf16", False), (3, 700, 480, 264, "bf16", False), (3, 700, 544, 264, "bf16", True),
+    (8, 8192, 160, 2304, "bf16", False), (8, 8192, 224, 2304, "bf16", True),      # more than a round of tiles for certain
+    (3, 700, 960, 264, "pow2", False), (3, 700, 1088, 264, "pow2", True), (8, 8192, 448, 2304, "pow2", True),
+    (3, 700, 1216, 264, "fp8", False), (3, 700, 1344, 264, "fp8", True),
+    (8, 8192, 960, 2304, "fp8", False), (8, 8192, 1088, 2304, "fp8", True), (300, 30000, 544, 264, "bf16", False),
+])
+def test_odd_numbers_of_whole_slices(E, rows, K, N, dtype, tail):
+    """The 4-slot ring and the kernel for contraction tails both take them: which one runs on either side of the rule's lines,
+    and the same sums from both (fp32 sums of exact products of small integers: bit for bit)."""
+    from fast_moe_amd.kernels.hip import ops
+    g = torch.Generator(device="cuda").manual_seed(K)
+    off = (torch.arange(E + 1) * rows // E).cuda()
+    x, w = (torch.randint(-2, 3, s, generator=g, device="cuda").to(BF16) for s in ((rows, K), (E, N, K)))
+    args, kw = (x, w.permute(0, 2, 1)), dict(total_rows=rows)
+    if dtype != "bf16":
+        args = (x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn).permute(0, 2, 1))
+        kw.update(a_scale=torch.ones(rows, device="cuda"), b_scale=torch.ones(E, N, device="cuda"), scales_pow2=dtype == "pow2")
+    out = ops.grouped_gemm(off, *args, **kw)
+    ran, = kernels_run(lambda: ops.grouped_gemm(off, *args, **kw))
+    assert "ring_kernel" in ran and (KTAIL in ran) == tail and ("RingCfg<256, 256, 2, 4, 0, 2>" in ran) != tail, ran
+    for e in range(0, E, 7):
+        lo, hi = int(off[e]), int(off[e + 1])
+        assert torch.equal(out[lo:hi], (x[lo:hi].float() @ w[e].float().t()).to(BF16))
 
 
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
