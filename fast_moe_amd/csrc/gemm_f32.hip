@@ -19,15 +19,35 @@ typedef TileCfg<64, 128, 2, 2> TileF32Wide;     // 4 waves, wave tile 32 x 64
 typedef TileCfg<64, 64, 2, 2> TileF32;          // 4 waves, wave tile 32 x 32
 
 // From four wide tiles per CU on, the remainder of the last round is a small share and the 25 % fewer operand bytes of the
-// wide tile count for more (1172 against 1235 us above); below, the finer tile fills the chip better (390 against 421).
+// wide tile count for more (1172 against 1235 us above); below, the finer tile fills the chip better (390 against 421).  With
+// SiLU on load, which every column of tiles repeats, from one per CU on: 375 rows, 16 experts, 860 -> 3320 columns 91 / 107 us,
+// 300 rows, 8 experts, 1024 -> 1024 80 / 61.
 // With n-contiguous weights, whose parking costs four LDS writes a chunk, the small tile was faster at every size (four to
 // seven blocks per CU instead of three): 398 / 350, 527 / 413, 1425 / 1299 us for the first, second and fourth line.
-// SwiGLU needs gate and up fragments in one wave: always wide.
+// SwiGLU needs gate and up fragments in one wave: wide, or 64 x 256 where that is one round of tiles (two blocks per CU) and
+// wide more than one (three): 2000 rows, 200 experts, 256 -> 2 x 256 51.0 / 45.2 us.
+//
+// Whole rounds of 256 x 256 tiles, one block per CU, are faster still: a quarter of the operand reads and of the SiLU.  us,
+// 256 x 256 / 64 x 128: 4096 rows, 1 expert, 4096 -> 4096 (one round) 1037 / 1123, SiLU on load 1241 / 1479; 8192 rows, 2048 -> 4096
+// 1053 / 1123; but with 1056 tiles (65536 rows, 8 experts, 512 -> 1024: a fifth round of 32) 750 / 614.  The bound on the row
+// tiles holds however the experts share the rows; 6 % (15 % with SiLU on load) is what an unfilled remainder may cost.
 template <int EPI, int LOADS, bool A_SILU>
 int pick_tile(const GemmParams& p, hipStream_t stream) {
+    constexpr int out_cols = EPI == FMOE_EPI_SWIGLU ? 2 : 1;    // tile columns per output column
+    const int64_t cus = compute_units();
+    auto tiles = [&](int bm, int bn) { return (p.total_rows / bm + p.E) * ((p.N + bn / out_cols - 1) / (bn / out_cols)); };
+    if constexpr (LOADS == kLoadChunks) {
+        const int64_t most = (p.total_rows + 255 * (int64_t)p.E) / 256 * ((p.N + 256 / out_cols - 1) / (256 / out_cols));
+        const double rounds = (double)((most + cus - 1) / cus * cus) * (256 * 256 / out_cols);
+        if (rounds <= (A_SILU ? 1.15 : 1.06) * (double)p.total_rows * p.N)
+            return launch_gemm<TileBig, kDtF32, EPI, LOADS, A_SILU>(p, stream);
+        if constexpr (EPI == FMOE_EPI_SWIGLU) {
+            if (tiles(TileF32Wide::BM, TileF32Wide::BN) > 3 * cus && tiles(TileSmall::BM, TileSmall::BN) <= 2 * cus)
+                return launch_gemm<TileSmall, kDtF32, EPI, LOADS, A_SILU>(p, stream);
+        }
+    }
     if constexpr (EPI != FMOE_EPI_SWIGLU) {
-        const int64_t wide = (p.total_rows / TileF32Wide::BM + p.E) * ((p.N + TileF32Wide::BN - 1) / TileF32Wide::BN);
-        if (LOADS == kLoadChunksN || wide < 4 * (int64_t)compute_units())
+        if (LOADS == kLoadChunksN || tiles(TileF32Wide::BM, TileF32Wide::BN) < (A_SILU ? 1 : 4) * cus)
             return launch_gemm<TileF32, kDtF32, EPI, LOADS, A_SILU>(p, stream);
     }
     if constexpr (EPI == FMOE_EPI_SWIGLU || LOADS != kLoadChunksN)

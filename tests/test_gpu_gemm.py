@@ -1098,11 +1098,14 @@ def test_odd_numbers_of_whole_slices(E, rows, K, N, dtype, tail):
     (5, 700, 1000, 132, "kn", 2), (5, 700, 1000, 132, "nk", 2), # gate and up halves of a 128-column tile
     (2, 2600, 100, 3500, "nk", 1), (2, 2600, 100, 3500, "kn", 1),   # enough tiles for the wide form (nk)
     (70, 900, 68, 256, "kn", 0),                                # more experts than lanes, some empty
+    (1, 4096, 100, 4096, "nk", 1), (1, 4000, 36, 4096, "nk", 2),    # whole rounds of 256 x 256 tiles
+    (1, 4096, 40, 4092, "nk", "silu"), (200, 2000, 256, 256, "nk", 2), (200, 2000, 40, 256, "nk", "silu"),
+    (3, 190, 36, 60, "nk", "silu"), (3, 190, 36, 68, "kn", "silu"),
 ])
 def test_fp32_kernel_tiles_and_weight_layouts(E, rows, K, N, layout, epi):
-    """fp32 tiles of 64 rows, weights with k or n contiguous.  The operands are the left columns of
-    wider tensors whose other columns are NaN.  Against float64; the bound of a K-term fp32 sum,
-    (K + 2) * 2^-24 * sum |a||b|, through SiLU (|slope| <= 1.1) and the product."""
+    """fp32 tiles, weights with k or n contiguous, SiLU in the epilogue or ("silu") on load.  The operands are the left
+    columns of wider tensors whose other columns are NaN.  Against float64; the bound of a K-term fp32 sum,
+    (K + 2) * 2^-24 * sum |a||b|, through SiLU (|slope| <= 1.1, its value on load to 2^-21) and the product."""
     from fast_moe_amd.kernels.hip import _lib, ops
     g = torch.Generator().manual_seed(K + N + rows)
     off = torch.tensor([0] + sorted(torch.randint(0, rows, (E - 1,), generator=g).tolist()) + [rows]).cuda()
@@ -1112,12 +1115,14 @@ def test_fp32_kernel_tiles_and_weight_layouts(E, rows, K, N, layout, epi):
         return t[..., :shape[-1]]
     x = wide(rows, K)
     ws = [wide(E, K, N) if layout == "kn" else wide(E, N, K).permute(0, 2, 1) for _ in range(2)]
-    kw = dict(total_rows=rows, b2=ws[1] if epi == _lib.EPI_SWIGLU else None, epilogue=epi)
+    a_silu, epi = epi == "silu", 0 if epi == "silu" else epi
+    kw = dict(total_rows=rows, b2=ws[1] if epi == _lib.EPI_SWIGLU else None, epilogue=epi, a_silu=a_silu)
     assert ops.grouped_gemm(off, x, ws[0], plan_only=True, **kw) != _lib.PLAN_ELEMENT
     out = ops.grouped_gemm(off, x, ws[0], **kw)
-    unit = (K + 2) * 2.0 ** -24
+    unit = (K + 2) * 2.0 ** -24 + (2.0 ** -21 if a_silu else 0)
     for e in range(E):
         a = x[int(off[e]):int(off[e + 1])].double()
+        a = torch.nn.functional.silu(a) if a_silu else a
         want, err = a @ ws[0][e].double(), unit * (a.abs() @ ws[0][e].double().abs())
         if epi != _lib.EPI_NONE:
             want, err = torch.nn.functional.silu(want), 1.1 * err + 2.0 ** -21 * want.abs()
@@ -1125,6 +1130,23 @@ def test_fp32_kernel_tiles_and_weight_layouts(E, rows, K, N, layout, epi):
             up, up_err = a @ ws[1][e].double(), unit * (a.abs() @ ws[1][e].double().abs())
             want, err = want * up, err * up.abs() + (want.abs() + err) * up_err + 2.0 ** -23 * (want * up).abs()
         assert bool(((out[int(off[e]):int(off[e + 1])].double() - want).abs() <= err).all()), f"expert {e}"
+
+
+@pytest.mark.parametrize("E,rows,N,epi,tile", [
+    (1, 4096, 4096, 0, "256, 256"), (1, 4097, 4096, 0, "64, 128"), (1, 3868, 4096, 0, "256, 256"), (1, 3860, 4096, 0, "64, 128"),
+    (2, 4096, 4096, 0, "64, 128"), (1, 4096, 4096, 2, "256, 256"), (1, 4097, 4096, 2, "64, 128"),
+    (1, 3580, 4096, "silu", "256, 256"), (1, 3560, 4096, "silu", "64, 128"),
+    (1, 4000, 512, "silu", "64, 64"), (1, 4096, 512, "silu", "64, 128"), (1, 4096, 512, 0, "64, 64"),
+    (200, 2000, 256, 2, "64, 256"), (200, 2000, 384, 2, "64, 128"), (8, 2000, 256, 2, "64, 128"),
+])
+def test_fp32_tile_choice(E, rows, N, epi, tile):
+    """The tile on either side of the lines of the fp32 rule, from a trace."""
+    from fast_moe_amd.kernels.hip import ops
+    x, w = torch.zeros(rows, 32, device="cuda"), torch.zeros(E, N, 32, device="cuda").permute(0, 2, 1)
+    off = (torch.arange(E + 1) * rows // E).cuda()
+    a_silu, epi = epi == "silu", 0 if epi == "silu" else epi
+    ran, = kernels_run(lambda: ops.grouped_gemm(off, x, w, total_rows=rows, epilogue=epi, b2=w if epi else None, a_silu=a_silu))
+    assert f"grouped_gemm_kernel<fmoe::TileCfg<{tile}," in ran, ran
 
 
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
