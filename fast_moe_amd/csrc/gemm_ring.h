@@ -1,6 +1,7 @@
 // LDS-ring grouped GEMM kernel: the fast path (persistent, 256 x 256 tiles, LDS-DMA, software-pipelined MFMA loop).
 #pragma once
 
+#include "gemm_deal.h"
 #include "gemm_epilogue.h"
 
 namespace fmoe {
@@ -230,44 +231,20 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         total_m = s_tab[p.E];
         r_end[0] = 0;
     }
-    // The tiles of an XCD, numbered 0 .. xcd_count-1.  Paired ring: whole groups (kGroupM row
-    // tiles x all column tiles: what shares operands in an XCD's L2) are dealt to the XCDs back
-    // and forth (0..7, 7..0, ...).  A tile's cost follows its expert (the contraction window of
-    // a weight gradient; a last row tile with few rows runs the shortened main loop), and a
-    // contiguous range per XCD hands one of them all the long experts and another all the short
-    // ones; a plain round robin still favours the low XCDs when the experts come sorted by
-    // load.  What is left after the last whole round of groups goes out as an equal run of tiles per XCD: dealt
-    // as whole groups, a launch of few groups keeps one XCD's blocks at work for a round or two while others are
-    // done (us per GEMM, whole groups / runs: 9189 rows, 12 experts, 1024 -> 2560 columns 76.9 / 58.3 and
-    // 2560 -> 1024 66.4 / 56.9; 16384 rows, 8 experts, 1024 -> 4096 176.6 / 151.5).  4-slot ring: one contiguous range of the tile order per XCD.
+    // Paired ring: groups of tiles dealt to the XCDs (gemm_deal.h).  A contiguous range per XCD instead hands one of them all
+    // the long experts and another all the short ones where tiles differ in cost (experts of a weight gradient; a last row
+    // tile with few rows runs the shortened main loop), and a plain round robin still favours the low XCDs when the
+    // experts come sorted by load.  4-slot ring, and 64-row tiles (a launch is a stream of weights with little to share and
+    // often has no 8 groups): one contiguous range of the tile order per XCD.
     using tile_t = std::conditional_t<PAIR, int, int64_t>;     // (the paired ring's launcher checks that they fit)
-    const tile_t total_tiles = (tile_t)total_m * p.n_tiles;
     const int nslots = gridDim.x / kNumXcd;
     const int xcd = blockIdx.x % kNumXcd, slot = blockIdx.x / kNumXcd;
     const tile_t group_span = (tile_t)kGroupM * p.n_tiles;
     constexpr bool windowed = KWIN;
-    // (BM = 64: a launch is a stream of weights with little to share and often has no 8 groups)
     constexpr bool deal_groups = PAIR && BM >= 256;
-    tile_t xcd_count;
-    tile_t dealt = 0;           // tiles of this XCD that come in whole groups
-    tile_t run_base;            // number of the run's first tile, less dealt
-    if (deal_groups) {
-        // whole rounds of 8 groups (in odd rounds XCD x takes position 7 - x), then an equal run of what is left;
-        // seven groups and more are as good as a round and stay groups
-        const int rounds = total_m / (kGroupM * kNumXcd);
-        const tile_t whole = rounds * group_span, rest = total_tiles - whole * kNumXcd;
-        const bool runs = rest < (kNumXcd - 1) * group_span;
-        const tile_t run = runs ? (rest + kNumXcd - 1) / kNumXcd : group_span;
-        const int pos = runs || !(rounds & 1) ? xcd : kNumXcd - 1 - xcd;
-        const tile_t left = rest - pos * run;
-        xcd_count = whole + (left < 0 ? 0 : left < run ? left : run);
-        dealt = runs ? whole : xcd_count;
-        run_base = whole * (kNumXcd - 1) + pos * run;
-    } else {
-        const tile_t per_xcd = (total_tiles + kNumXcd - 1) / kNumXcd;
-        run_base = xcd * per_xcd;
-        xcd_count = total_tiles - run_base < per_xcd ? total_tiles - run_base : per_xcd;
-    }
+    using Deal = TileDeal<tile_t, kNumXcd, kGroupM>;
+    const Deal deal = deal_groups ? Deal(total_m, p.n_tiles, xcd, nslots) : Deal::contiguous(total_m, p.n_tiles, xcd);
+    const tile_t xcd_count = deal.count;
     // tile numbers of the paired ring fit 31 bits (the launcher checks): divisions by the group
     // span are one scalar multiply by a constant the host prepared, no division sequence whose
     // per-lane pieces the compiler would keep (or spill) across the tile loop
@@ -276,10 +253,8 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         else return v / group_span;
     };
     auto to_logical = [&](tile_t j) -> tile_t {
-        if (!deal_groups || j >= dealt) return run_base + j;
-        const tile_t round = div_span(j);
-        const int pos = (round & 1) ? kNumXcd - 1 - xcd : xcd;
-        return (round * kNumXcd + pos) * group_span + (j - round * group_span);
+        if constexpr (deal_groups) return deal.tile(j, div_span(j));
+        else return deal.run_base + j;
     };
 
     const int KT = KTAIL ? (p.K + 2 * BK - 1) / (2 * BK) * 2 : p.K / BK;

@@ -1242,10 +1242,11 @@ def test_kernel_choice_for_few_rows(E, rows, K, N, layout, epi, kernel):
 
 @pytest.mark.parametrize("row_tiles", [1, 7, 28, 31, 32, 33, 59, 60, 61, 97])
 @pytest.mark.parametrize("N", [256, 776])
-def test_ring_kernel_deals_every_tile_once(row_tiles, N):
+def test_ring_kernel_writes_every_tile(row_tiles, N):
     """Row-tile counts around the scheduler's lines (groups of 4 row tiles, rounds of 8 groups, seven groups and more of a
-    last round kept whole): every output tile is written, and once.  Short last tiles included.  fp32 sums of 128 bf16
-    products differ from another order's by less than 2^-16 of sum |a||b|, the result's rounding adds 2^-8 of it."""
+    last round kept whole): every output tile is written (that none is dealt twice, test_tile_deal.py shows).  Short last
+    tiles included.  fp32 sums of 128 bf16 products differ from another order's by less than 2^-16 of sum |a||b|, the
+    result's rounding adds 2^-8 of it."""
     from fast_moe_amd.kernels.hip import _lib, ops
     K, E = 128, 3
     cut = [row_tiles // 3, row_tiles // 2]
