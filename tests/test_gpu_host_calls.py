@@ -18,17 +18,35 @@ class Declines:
         return lambda *a: None
 
 
+class Recorder:
+    """The host module, noting of every call whether it took it."""
+
+    def __init__(self, real):
+        self.real, self.took = real, []
+
+    def __getattr__(self, name):
+        def call(*a):
+            res = getattr(self.real, name)(*a)
+            self.took.append(res is not None)
+            return res
+        return call
+
+
 class Sub(torch.Tensor):
     pass
 
 
-def both(fn):
+def both(fn, taken):
+    """fn's result by way of the host module, which takes (all of) the call or declines it as ``taken`` says (None: some of
+    it), and by the Python code alone."""
     from fast_moe_amd.kernels.hip import _lib
-    taken = fn()
     real = _lib.host()
-    _lib._host = Declines()
+    recorder = _lib._host = Recorder(real)
     try:
-        return taken, fn()
+        native = fn()
+        assert taken is None or (recorder.took and (all if taken else any)(recorder.took) == taken), recorder.took
+        _lib._host = Declines()
+        return native, fn()
     finally:
         _lib._host = real
 
@@ -54,16 +72,19 @@ def test_operators(T, E, K, form):
     x = make(dev(randn((T, D), 2).to(dtype)))
     w, wp = (make(dev(randn((E, H, D), s, scale=D ** -0.5).to(dtype))).permute(0, 2, 1) for s in (3, 4))
     bias = make(dev(randn((E, H), 5).to(dtype)))
-    same(*both(lambda: ops.route_topk(scores, K)))
+    taken = form != "subclass"
+    same(*both(lambda: ops.route_topk(scores, K), taken and scores.is_contiguous()))
     r = ops.route_topk(scores, K)
     off, idx = r["offsets"], r["gate_index"]
     for kw in (dict(), dict(bias=bias), dict(bias=bias, bias2=bias, b2=wp, epilogue=EPI_SWIGLU)):
-        same(*both(lambda: ops.grouped_gemm(off, x, w, total_rows=T * K, row_index=idx.view(-1, K), index_div=K, **kw)))
-    value = ops.grouped_gemm(off, x, w, total_rows=T * K, row_index=idx, index_div=K)
+        same(*both(lambda: ops.grouped_gemm(off, x, w, total_rows=T * K, row_index=idx.view(-1, K), index_div=K, **kw), taken))
+    n_contiguous = w.contiguous()
+    same(*both(lambda: ops.grouped_gemm(off, x, n_contiguous, total_rows=T * K, row_index=idx, index_div=K), False))
+    value = make(ops.grouped_gemm(off, x, w, total_rows=T * K, row_index=idx, index_div=K))
     for gates in (None, r["gates"], r["gates"].to(BF16), r["gates"].reshape(-1)):
-        same(*both(lambda: ops.combine(value, r["reverse_index"], gates, idx)))
+        same(*both(lambda: ops.combine(value, r["reverse_index"], gates, idx), taken and (gates is None or gates.ndim == 2)))
     for silu in (False, True):
-        same(*both(lambda: ops.quant_rows_fp8(x, apply_silu=silu)))
+        same(*both(lambda: ops.quant_rows_fp8(x, apply_silu=silu), taken))
         q, s = ops.quant_rows_fp8(x, apply_silu=silu)
         assert ops.scales_are_pow2(s)
 
@@ -76,7 +97,7 @@ def test_layer_forward(B, S, dtype):
     layer = FastMoELayer(64, 96, 64, 8, dtype=dtype).to(dtype).cuda()
     x = dev(randn((B, S, 64), 1).to(dtype))
     with torch.no_grad():
-        same(*both(lambda: layer(x, 2)))
+        same(*both(lambda: layer(x, 2), True if S else None))
 
     class Rerouted(FastMoELayer):       # a route() of its own is asked
         def route(self, x, k):
