@@ -459,9 +459,9 @@ __global__ __launch_bounds__(256) void invert_rank_kernel(const int64_t* __restr
     }
 }
 
-// Gradient of gates[t, j] = s_j / max(sum_i s_i, 1e-12), s_j = scores[t, idx[t, j]], with respect to the scores: one wave
+// Gradient of gates[t, j] = s_j / max(sum_i |s_i|, 1e-12), s_j = scores[t, idx[t, j]], with respect to the scores: one wave
 // per token, lane j holds slot j (K <= 64), the row of E gradients is written whole.  Every step is rounded to the scores'
-// type where torch's chain of gather, sum, clamp_min and div rounds its intermediate tensors, so the result is that
+// type where torch's chain of gather, norm, clamp_min and div rounds its intermediate tensors, so the result is that
 // chain's (the sums over K run in slot order).  Bound by nothing but its launch: it stands for about fifteen element-wise
 // launches forward and backward (3063 tokens, 12 experts: 4 us for about 75).
 constexpr int kGateChunk = 512;
@@ -484,7 +484,7 @@ __global__ __launch_bounds__(256) void gate_l1_bwd_kernel(const T* __restrict__ 
         }
     }
     float sum = 0.0f;
-    for (int j = 0; j < K; ++j) sum += __shfl(s, j, kWave);
+    for (int j = 0; j < K; ++j) sum += fabsf(__shfl(s, j, kWave));
     sum = Val<T>::round(sum);
     const float floor_ = Val<T>::round(1e-12f);
     const float c = sum < floor_ ? floor_ : sum;
@@ -492,7 +492,8 @@ __global__ __launch_bounds__(256) void gate_l1_bwd_kernel(const T* __restrict__ 
     float d_sum = 0.0f;
     for (int j = 0; j < K; ++j) d_sum += __shfl(part, j, kWave);
     d_sum = sum >= floor_ ? Val<T>::round(d_sum) : 0.0f;
-    const float d = Val<T>::round(Val<T>::round(g / c) + d_sum);
+    const float sign = s > 0.0f ? 1.0f : s < 0.0f ? -1.0f : 0.0f;
+    const float d = Val<T>::round(Val<T>::round(g / c) + d_sum * sign);
     // the row of gradients by way of LDS, a chunk at a time: zeros, the K values over them, out.  (One wave's LDS accesses
     // execute in order; the fence keeps the compiler from answering the loads from a lane's own stores.)  Every lane asking
     // every slot whether it is its expert, 2 K shuffles per 64 experts, took longer than torch's scatter: 8192 tokens, 512

@@ -411,8 +411,6 @@ class TopkGates(torch.autograd.Function):
     L1-normalised gate values of every token (modules/fast_moe_module.py:93-105).  The selection
     itself has no gradient."""
 
-    MAX_K = 64      # slots are lanes of one wave in the backward kernel
-
     @staticmethod
     def forward(ctx, scores, k, routing):
         routing.update(ops.route_topk(scores, k, renorm=True))
@@ -424,20 +422,16 @@ class TopkGates(torch.autograd.Function):
         scores, topk_idx = ctx.saved_tensors
         if torch.is_grad_enabled():     # create_graph=True: the formula in differentiable torch ops
             picked = scores.gather(1, topk_idx)
-            total = picked.sum(dim=1, keepdim=True)
+            total = picked.abs().sum(dim=1, keepdim=True)
             c = total.clamp_min(1e-12)
             d_total = (-d_gates * ((picked / c) / c)).sum(dim=1, keepdim=True)
-            d_picked = d_gates / c + torch.where(total >= 1e-12, d_total, torch.zeros_like(d_total))
+            d_picked = d_gates / c + torch.where(total >= 1e-12, d_total, torch.zeros_like(d_total)) * picked.sign()
             return torch.zeros_like(scores).scatter_add(1, topk_idx, d_picked), None, None
         return ops.gate_l1_bwd(scores, topk_idx, d_gates), None, None
 
 
 def topk_gates(scores: torch.Tensor, k: int):
     """-> (routing dict, gates [T, k] with a gradient to ``scores``)."""
-    if k > TopkGates.MAX_K:
-        r = ops.route_topk(scores.detach(), k, renorm=True)
-        picked = scores.gather(1, r["topk_idx"])
-        return r, picked / picked.sum(dim=1, keepdim=True).clamp_min(1e-12)
     r = {}
     return r, TopkGates.apply(scores, k, r)
 

@@ -415,7 +415,7 @@ int fmoe_invert_index(const int64_t* index, int64_t T, int K, int64_t* reverse, 
 
 /*
  * Gradient of the L1-normalised top-k gate values (modules/fast_moe_module.py:93-105) with respect
- * to the gate probabilities: gates[t, j] = s_j / max(sum_i s_i, 1e-12) with s_j =
+ * to the gate probabilities: gates[t, j] = s_j / max(sum_i |s_i|, 1e-12) with s_j =
  * scores[t, topk_idx[t, j]].  scores, d_gates [T, K] and d_scores [T, E] share one type, FMOE_F32
  * or FMOE_BF16; contiguous.  d_scores is written whole (0 for experts not picked).  K <= 64.
  */

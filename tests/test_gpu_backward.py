@@ -714,6 +714,34 @@ def test_topk_gates_backward(T, E, K, dtype):
     assert ((grad.detach().cpu().float() - s.grad.cpu().float()).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("E,K", [(6, 3), (70, 8)])
+@pytest.mark.parametrize("dtype", [BF16, torch.float32])
+def test_topk_gates_of_any_sign(E, K, dtype):
+    """Scores that are no probabilities (a gate network of the caller's own): the gates are divided by sum |s|, as F.normalize
+    does it, and the gradient is the gradient of that, also where every pick is negative, zero or sums to nothing.  Against
+    float64 autograd; each of the few roundings is 2^-9 (bf16) / 2^-24 of terms bounded by max |dg| / sum |s|."""
+    from fast_moe_amd.kernels.hip.autograd import topk_gates
+    T = 40
+    scores = randn((T, E), 3).to(dtype)
+    scores[0] = -scores[0].abs() - 1            # all negative
+    scores[1], scores[1, 2] = 0, 0.5            # one score, the other picks 0
+    scores[2] = 0                               # nothing: divided by 1e-12
+    dg = randn((T, K), 4).to(dtype)
+    s = leaf(scores, device="cuda")
+    r, gates = topk_gates(s, K)
+    ref = leaf(scores.double())
+    picked = ref.gather(1, r["topk_idx"].cpu())
+    want = torch.nn.functional.normalize(picked, p=1, dim=1)
+    eps = (K + 8) * (2.0 ** -9 if dtype == BF16 else 2.0 ** -24)
+    assert ((gates.detach().cpu().double() - want.detach()).abs() <= eps).all()
+    want.backward(dg.double())
+    total = picked.detach().abs().sum(dim=1, keepdim=True).clamp_min(1e-12)
+    bound = eps * 2 * dg.double().abs().max(dim=1, keepdim=True).values / total
+    for create_graph in (False, True):
+        grad, = torch.autograd.grad(gates, s, dev(dg), create_graph=create_graph, retain_graph=True)
+        assert ((grad.detach().cpu().double() - ref.grad).abs() <= bound).all(), create_graph
+
+
 @pytest.mark.parametrize("T,E,K", [(5, 511, 3), (9, 513, 8), (6, 1100, 64), (4, 1024, 1)])
 @pytest.mark.parametrize("dtype", [BF16, torch.float32])
 def test_gate_gradient_rows_of_many_experts(T, E, K, dtype):
