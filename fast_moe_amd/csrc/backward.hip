@@ -462,7 +462,8 @@ __global__ __launch_bounds__(256) void invert_rank_kernel(const int64_t* __restr
 // Gradient of gates[t, j] = s_j / max(sum_i |s_i|, 1e-12), s_j = scores[t, idx[t, j]], with respect to the scores: one wave
 // per token, lane j holds slot j (K <= 64), the row of E gradients is written whole.  Every step is rounded to the scores'
 // type where torch's chain of gather, norm, clamp_min and div rounds its intermediate tensors, so the result is that
-// chain's (the sums over K run in slot order).  Bound by nothing but its launch: it stands for about fifteen element-wise
+// chain's; the sums over K run in slot order, in double for fp32 scores (in fp32 the slot order's error was a quarter above
+// that of torch's tree).  Bound by nothing but its launch: it stands for about fifteen element-wise
 // launches forward and backward (3063 tokens, 12 experts: 4 us for about 75).
 constexpr int kGateChunk = 512;
 template <typename T>
@@ -483,15 +484,16 @@ __global__ __launch_bounds__(256) void gate_l1_bwd_kernel(const T* __restrict__ 
             s = Val<T>::load(scores + t * E + id);
         }
     }
-    float sum = 0.0f;
-    for (int j = 0; j < K; ++j) sum += fabsf(__shfl(s, j, kWave));
-    sum = Val<T>::round(sum);
+    using Acc = std::conditional_t<sizeof(T) == 4, double, float>;
+    Acc total = 0;
+    for (int j = 0; j < K; ++j) total += fabsf(__shfl(s, j, kWave));
+    const float sum = Val<T>::round((float)total);
     const float floor_ = Val<T>::round(1e-12f);
     const float c = sum < floor_ ? floor_ : sum;
     const float part = Val<T>::round(-g * Val<T>::round(Val<T>::round(s / c) / c));
-    float d_sum = 0.0f;
-    for (int j = 0; j < K; ++j) d_sum += __shfl(part, j, kWave);
-    d_sum = sum >= floor_ ? Val<T>::round(d_sum) : 0.0f;
+    Acc d_total = 0;
+    for (int j = 0; j < K; ++j) d_total += __shfl(part, j, kWave);
+    const float d_sum = sum >= floor_ ? Val<T>::round((float)d_total) : 0.0f;
     const float sign = s > 0.0f ? 1.0f : s < 0.0f ? -1.0f : 0.0f;
     const float d = Val<T>::round(Val<T>::round(g / c) + d_sum * sign);
     // the row of gradients by way of LDS, a chunk at a time: zeros, the K values over them, out.  (One wave's LDS accesses

@@ -415,6 +415,10 @@ class TopkGates(torch.autograd.Function):
     def forward(ctx, scores, k, routing):
         routing.update(ops.route_topk(scores, k, renorm=True))
         ctx.save_for_backward(scores, routing["topk_idx"])
+        if scores.dtype == torch.float32:
+            # the library adds the K scores in slot order, in fp32; torch's tree is a third nearer to the exact gates
+            picked = scores.gather(1, routing["topk_idx"])
+            routing["gates"] = picked / picked.abs().sum(dim=1, keepdim=True).clamp_min(1e-12)
         return routing["gates"]
 
     @staticmethod

@@ -742,6 +742,27 @@ def test_topk_gates_of_any_sign(E, K, dtype):
         assert ((grad.detach().cpu().double() - ref.grad).abs() <= bound).all(), create_graph
 
 
+@pytest.mark.parametrize("T,E,K", [(8192, 64, 8), (4096, 128, 6), (2048, 16, 2)])
+def test_fp32_gates_are_as_near_to_exact_as_the_torch_chain(T, E, K):
+    """Gates and their gradient in fp32 lie no further from float64 than torch's gather, sum, clamp_min and div."""
+    from fast_moe_amd.kernels.hip.autograd import topk_gates
+    scores, dg = torch.softmax(randn((T, E), 1).float() * 2, 1).cuda(), randn((T, K), 2).float().cuda()
+    s = leaf(scores)
+    r, gates = topk_gates(s, K)
+    gates.backward(dg)
+
+    def chain(x):
+        x = leaf(x)
+        picked = x.gather(1, r["topk_idx"])
+        g = picked / picked.sum(dim=1, keepdim=True).clamp_min(1e-12)
+        g.backward(dg.to(g.dtype))
+        return g.detach(), x.grad
+
+    (g64, d64), (g32, d32) = chain(scores.double()), chain(scores)
+    assert torch.equal(gates.detach(), g32)
+    assert (s.grad - d64).norm() <= (d32 - d64).norm() * 1.02
+
+
 @pytest.mark.parametrize("T,E,K", [(5, 511, 3), (9, 513, 8), (6, 1100, 64), (4, 1024, 1)])
 @pytest.mark.parametrize("dtype", [BF16, torch.float32])
 def test_gate_gradient_rows_of_many_experts(T, E, K, dtype):
