@@ -19,9 +19,12 @@ namespace fmoe {
 //     rows, 12 experts, 2624 -> 1024 62.7 / 53.7; 4476 rows, 3136 -> 2048 74 / 67);
 //   * its last round is three quarters full or more, and more than one group is left (20294 rows, 4 experts, 1792 -> 2560
 //     178 / 169; with three quarters of a group left, 16384 rows, 8 experts, 4096 -> 2 x 1024, Zipf 265 / 274).
+// Tiles of unequal cost (contraction windows, the longest first) go out in runs only where there is no whole round: after one,
+// the left-over groups are the cheapest and belong to the XCDs that had the shorter windows (weight gradients of 9189 rows, 12
+// experts, 1000 x 2600, Zipf 138 / 148; 2600 x 1000 75.7 / 77.2; one expert, 4096 x 4096, no whole round 462 / 232).
 // Otherwise they only give every XCD a last round of its own: 6138 rows, 12 experts, 3648 -> 4096 (16 tiles left, 80 on one XCD
 // or 66 on each, 32 slots) 209 / 234; 24576 rows, 64 experts, 2048 -> 1408 195 / 202.  Seven groups and more are as good as a round.
-template <typename tile_t, int XCDS, int GROUP_M>
+template <typename tile_t, int XCDS, int GROUP_M, bool EQUAL_COST = true>
 struct TileDeal {
     tile_t span;        // tiles of a group
     tile_t count;       // tiles of this XCD
@@ -37,7 +40,7 @@ struct TileDeal {
         const tile_t even = (rest + XCDS - 1) / XCDS;
         const tile_t busiest = whole + (rest < span ? rest : span);
         const tile_t last_round = busiest > 0 ? (busiest - 1) % slots + 1 : 0;
-        const bool runs = rest < (XCDS - 1) * span &&
+        const bool runs = rest < (XCDS - 1) * span && (EQUAL_COST || rounds == 0) &&
                           (busiest <= slots || busiest - (whole + even) >= last_round || (4 * last_round >= 3 * slots && rest > span));
         const tile_t run = runs ? even : span;
         const int pos = runs || !(rounds & 1) ? xcd : XCDS - 1 - xcd;

@@ -242,7 +242,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     const tile_t group_span = (tile_t)kGroupM * p.n_tiles;
     constexpr bool windowed = KWIN;
     constexpr bool deal_groups = PAIR && BM >= 256;
-    using Deal = TileDeal<tile_t, kNumXcd, kGroupM>;
+    using Deal = TileDeal<tile_t, kNumXcd, kGroupM, !KWIN>;
     const Deal deal = deal_groups ? Deal(total_m, p.n_tiles, xcd, nslots) : Deal::contiguous(total_m, p.n_tiles, xcd);
     const tile_t xcd_count = deal.count;
     // tile numbers of the paired ring fit 31 bits (the launcher checks): divisions by the group
