@@ -413,12 +413,12 @@ class TopkGates(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, scores, k, routing):
-        routing.update(ops.route_topk(scores, k, renorm=True))
+        fp32 = scores.dtype == torch.float32
+        routing.update(ops.route_topk(scores, k, renorm=not fp32))
         ctx.save_for_backward(scores, routing["topk_idx"])
-        if scores.dtype == torch.float32:
-            # the library adds the K scores in slot order, in fp32; torch's tree is a third nearer to the exact gates
-            picked = scores.gather(1, routing["topk_idx"])
-            routing["gates"] = picked / picked.abs().sum(dim=1, keepdim=True).clamp_min(1e-12)
+        if fp32:    # the library adds the K scores in slot order, in fp32; torch's tree is a third nearer to the exact gates
+            picked = routing["gates"]
+            routing["gates"] = picked / torch.linalg.vector_norm(picked, 1, dim=1, keepdim=True).clamp_min_(1e-12)
         return routing["gates"]
 
     @staticmethod
