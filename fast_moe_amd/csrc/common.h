@@ -20,6 +20,7 @@ int check_launch(const char* what);
         if (!(cond)) return ::fmoe::fail(FMOE_ERR_ARGUMENT, __VA_ARGS__); \
     } while (0)
 
+__host__ __device__ static inline bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
 __host__ __device__ static inline bool aligned16(const void* p) {
     return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }

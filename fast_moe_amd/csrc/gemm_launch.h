@@ -128,11 +128,12 @@ int launch_ring_cfg(GemmParams p, hipStream_t stream) {
 int run_ring_tail_bf16(const GemmParams& p, int epilogue, hipStream_t stream);
 int run_ring_tail_fp8(const GemmParams& p, int epilogue, hipStream_t stream);
 
-// What they take beyond the ring's own conditions: at least one pair of slices and a 16-byte chunk.  On 9189 rows, 12 experts, 1000 <-> 2600
-// columns: weights with n contiguous 85 us per GEMM where the element-load kernel took 1368 and 1620; weights with k
-// contiguous 94 us against 99 on the register-staged kernel.
+// What they take beyond the ring's own conditions: at least one pair of slices and a 16-byte chunk (8 bytes of e4m3).  On 9189 rows,
+// 12 experts, 1000 <-> 2600 columns: weights with n contiguous 85 us per GEMM where the element-load kernel took 1368 and 1620;
+// weights with k contiguous 94 us against 99 on the register-staged kernel.
+constexpr int kRingTailChunk = 8;       // elements: 16 bytes of bf16, 8 of e4m3
 inline bool ring_tail_takes(int esize, int64_t k, int num_experts, int64_t total_rows) {
-    const int pair = 128 / esize, chunk = 16 / esize;
+    const int pair = 128 / esize, chunk = kRingTailChunk;
     return k > pair && k % pair != 0 && k % chunk == 0 && num_experts <= TileRing5W::kMaxExperts &&
            total_rows < ((int64_t)1 << 31) && lds_per_block() >= TileRing5W::LDS_BYTES;
 }
@@ -156,7 +157,7 @@ int run_ring_short_bf16(const GemmParams& p, int epilogue, hipStream_t stream);
 int run_ring_short_fp8(const GemmParams& p, int epilogue, hipStream_t stream);
 
 inline bool ring_short_takes(int esize, int64_t k, int num_experts, int64_t total_rows) {
-    const int pair = 128 / esize, chunk = 16 / esize;
+    const int pair = 128 / esize, chunk = kRingTailChunk;
     return k > (TileRingS::AHEAD - 1) * pair && k % chunk == 0 && num_experts <= TileRingS::kMaxExperts &&
            total_rows < ((int64_t)1 << 31) && lds_per_block() >= TileRingS::LDS_BYTES;
 }

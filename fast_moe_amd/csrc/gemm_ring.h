@@ -86,7 +86,7 @@ __device__ __forceinline__ int uniform_lane(int v, int src_lane) {
 // (row indices before it, the scales behind its first row block, packed at its end), so that no
 // tile waits for an index -> scale chain and the epilogue multiplies nothing.
 //
-// KTAIL (paired ring, no window): K is any whole number of 16-byte chunks above one pair of K-slices.  The last
+// KTAIL (paired ring, no window): K is any whole number of 8 elements above one pair of K-slices.  The last
 // pair of a tile is fetched from the last 2 * BK columns of the operands, wherever the pair before it ended: the
 // columns both hold are masked out of the last pair's fragments, on both sides (a product of a real infinity with a
 // masked zero would be NaN).  No address beyond a row's end, no per-lane predicate in the DMA stream: the tail costs a
@@ -963,15 +963,15 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 for (int fm = 0; fm < HM; ++fm) xh[fm] = load_frag(sx, xfrag_row[HM + fm]);
             };
             // KTAIL: the fragment of the item in the first (HALF_ITEM 0) or second slot of the last pair, masked
-            // where the pair before it reached (a lane's 32 bytes are two 16-byte chunks)
+            // where the pair before it reached (in groups of 8 bytes of a lane's 32)
             auto tail_mask = [&](i32x8& f, auto half_item_c) {
                 if constexpr (KTAIL) {
                     const int at = decltype(half_item_c)::value * BK + 32 * khalf;
-                    const int lo = at < tail_dup ? 0 : -1, hi = at + 16 < tail_dup ? 0 : -1;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        f[i] &= lo;
-                        f[4 + i] &= hi;
+                        const int keep = at + 8 * i < tail_dup ? 0 : -1;
+                        f[2 * i] &= keep;
+                        f[2 * i + 1] &= keep;
                     }
                 }
             };

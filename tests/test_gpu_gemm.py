@@ -1203,6 +1203,39 @@ def test_ring_kernel_on_short_tiles(E, rows, K, N, layout, epi):
         assert_bf16_close(out[lo:hi], a.float(), rtol=1.6e-2, atol=4e-3, what=f"expert {e}")
 
 
+@pytest.mark.parametrize("short,E,rows,K,N,epi", [
+    (False, 3, 700, 136, 264, 0), (False, 3, 700, 248, 136, 1),     # one pair of K-slices and the shortest / longest rest
+    (False, 2, 1000, 1000, 520, 2), (False, 70, 9000, 520, 1032, 0),
+    (True, 3, 130, 264, 264, 0), (True, 2, 3, 1000, 520, 2),        # the least K; more than a pair of a rest
+    (True, 111, 333, 2888, 3072, 0), (True, 130, 900, 376, 72, 1),
+])
+def test_e4m3_rows_of_an_odd_number_of_8_byte_groups(short, E, rows, K, N, epi):
+    """K % 16 == 8: every other row starts off a 16-byte boundary."""
+    (test_ring_kernel_on_short_tiles if short else test_ring_kernel_contraction_tails)(E, rows, K, N, "fp8", epi)
+
+
+@pytest.mark.parametrize("rows,K,lead", [(700, 256, 8), (700, 320, 8), (700, 200, 24), (60, 512, 8), (60, 392, 40)])
+def test_e4m3_operands_off_a_16_byte_boundary(rows, K, lead):
+    """Columns ``lead`` .. ``lead + K`` of wider e4m3 tensors, NaN codes around them: the ring reads them in place.  Small
+    integers with scale 1: exact sums, rounded once."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    g = torch.Generator().manual_seed(K)
+    E, N = 3, 264
+    def wide(*shape):
+        t = torch.full((*shape[:-1], shape[-1] + 64), float("nan"))
+        t[..., lead:lead + shape[-1]] = torch.randint(-2, 3, shape, generator=g).float()
+        return t.cuda().to(torch.float8_e4m3fn)[..., lead:lead + shape[-1]]
+    x, w = wide(rows, K), wide(E, N, K)
+    off = torch.tensor([0, rows // 3, rows // 3, rows]).cuda()
+    kw = dict(total_rows=rows, a_scale=torch.ones(rows, device="cuda"), b_scale=torch.ones(E, N, device="cuda"))
+    assert ops.grouped_gemm(off, x, w.permute(0, 2, 1), plan_only=True, **kw) != _lib.PLAN_ELEMENT
+    for pow2 in (False, True):
+        out = ops.grouped_gemm(off, x, w.permute(0, 2, 1), scales_pow2=pow2, **kw)
+        for e in range(E):
+            lo, hi = int(off[e]), int(off[e + 1])
+            assert torch.equal(out[lo:hi], (x[lo:hi].float() @ w[e].float().t()).to(BF16))
+
+
 @pytest.mark.parametrize("E,rows,K,N,layout,epi,kernel", [
     (8, 760, 4096, 3328, "nk", 0, "ring"), (8, 760, 4096, 3584, "nk", 0, "stream"),     # 247 / 266 tiles if the rows fall badly
     (8, 760, 4096, 3328, "fp8", 0, "ring"), (8, 760, 4096, 3584, "fp8", 0, "stream"),
