@@ -1,12 +1,15 @@
-// fp32 instantiations of the jagged GEMM (v_mfma_f32_32x32x2_f32: fp32 operands, bias and
-// output).  Serves the fp32 cases of the reference's operator tests and fp32 FastMoELayer.
+// fp32 instantiations of the jagged GEMM (fp32 operands, bias and output).  Serves the fp32 cases of the reference's operator tests
+// and fp32 FastMoELayer: on the bf16 matrix cores with every value in three parts (gemm_f32x3.h), and, where K is short or the
+// strides allow no 16-byte loads, with v_mfma_f32_32x32x2_f32 on the register-staged kernel.
+#include "gemm_f32x3.h"
 #include "gemm_kernel.h"
 
 namespace fmoe {
 
 namespace {
 
-// An fp32 MFMA runs 64 cycles on operands of two LDS reads, so LDS and L2 bandwidth leave room for small tiles, and small
+// The tiles of v_mfma_f32_32x32x2_f32 (their figures are from before longer K went to the other kernel).
+// It runs 64 cycles on operands of two LDS reads, so LDS and L2 bandwidth leave room for small tiles, and small
 // tiles are what fills the chip: a launch is bound by the last round of tiles over 256 CUs (4096 rows, 8 experts,
 // 4096 -> 1024 columns: 80 tiles of 256 x 256).  Several blocks share a CU and hide each other's barriers and epilogues.
 // us per GEMM, tiles of 256 x 256 / 128 x 128 / 64 x 128 / 64 x 64:
@@ -54,9 +57,47 @@ int pick_tile(const GemmParams& p, hipStream_t stream) {
         return launch_gemm<TileF32Wide, kDtF32, EPI, LOADS, A_SILU>(p, stream);
 }
 
+template <typename TL, int EPI, bool NCONT, bool A_SILU>
+int launch_f32x3(GemmParams p, hipStream_t stream) {
+    constexpr int bn_out = EPI == FMOE_EPI_SWIGLU ? TL::BN / 2 : TL::BN;
+    p.n_tiles = (p.N + bn_out - 1) / bn_out;
+    auto kern = grouped_gemm_f32x3_kernel<TL, EPI, NCONT, A_SILU>;
+    static bool attr_done = false;
+    return launch_tiles<TL>(kern, p, attr_done, stream);
+}
+
+// From three slices on; up to two (K = 64) there is hardly a loop to be faster in: 4096 rows, 8 experts, 64 -> 512 columns 10.2 us on
+// v_mfma_f32_32x32x2_f32, 10.9 here (K = 72, SwiGLU: 16.5 / 13.4).
+//
+// us per GEMM, v_mfma_f32_32x32x2_f32 on its best tile / three parts on 64 x 64 / 64 x 128 / 128 x 128:
+//   4096 rows,  8 experts, 1024 -> 4096 columns  355 / 247 / 209 / 198        16384 rows  1156 /  -  / 835 / 743
+//   4096 rows,  8 experts, 4096 -> 1024          343 / 242 / 211 / 237        6000 rows, 10 experts, 1024 -> 1024  139 / 107 / 102 / 88
+//   1000 rows, 32 experts,  512 -> 1024           28 /  23 /  25 /  36        2048 rows, 64 experts,  256 -> 1024   28 /  23 /  21 / 29
+//     64 rows,  8 experts, 1024 -> 2048           33 /  32 /  41 /  61        512 rows, 8 experts, 128 -> 256     10.8 / 9.6 / 11.9 / 18
+//   SwiGLU (not on 64 x 64): 4096 rows, 8 experts, 1024 -> 4096  623 / 412 / 364; 600 rows, 16 experts, 512 -> 2048  79 / 43 / 48
+// 16384 rows are 185 TFLOP/s, 1110 of bf16 products: what the chip's power allows.
+//   * 128 x 128 reads the least from LDS for a product: where the rows fill five such tiles for every four CUs.
+//   * 64 x 64: up to four per CU however the rows fall (two with SiLU on load, which every column of tiles repeats: 600 rows, 16
+//     experts, 512 -> 2048  45 / 41).
+template <int EPI, bool NCONT, bool A_SILU>
+int pick_f32x3(const GemmParams& p, hipStream_t stream) {
+    constexpr bool swiglu = EPI == FMOE_EPI_SWIGLU;     // its gate and up fragments share a wave
+    typedef TileF32x3<128, 128, 2, 2> Large;            // wave tile 64 x 64
+    typedef TileF32x3<64, 128, swiglu ? 2 : 1, swiglu ? 2 : 4> Mid;
+    typedef TileF32x3<64, 64, 2, 2> Small;
+    const int64_t cus = compute_units();
+    auto columns = [&](int bn) { return (p.N * (swiglu ? 2 : 1) + bn - 1) / bn; };
+    if (p.total_rows / 128 * columns(128) * 4 >= 5 * cus) return launch_f32x3<Large, EPI, NCONT, A_SILU>(p, stream);
+    if constexpr (!swiglu) {
+        if ((p.total_rows / 64 + p.E) * columns(64) <= (A_SILU ? 2 : 4) * cus) return launch_f32x3<Small, EPI, NCONT, A_SILU>(p, stream);
+    }
+    return launch_f32x3<Mid, EPI, NCONT, A_SILU>(p, stream);
+}
+
 template <int EPI, bool A_SILU>
 int dispatch(const GemmParams& p, int sel, hipStream_t stream) {
     if (sel == kSelGeneric) return launch_gemm<TileSmall, kDtF32, EPI, kLoadElements, A_SILU>(p, stream);
+    if (p.K > 2 * 32) return p.b_sk != 1 ? pick_f32x3<EPI, true, A_SILU>(p, stream) : pick_f32x3<EPI, false, A_SILU>(p, stream);
     if (p.b_sk != 1) return pick_tile<EPI, kLoadChunksN, A_SILU>(p, stream);
     return pick_tile<EPI, kLoadChunks, A_SILU>(p, stream);
 }

@@ -1,0 +1,283 @@
+// fp32 grouped GEMM on the bf16 matrix cores: every operand value is cut into three bf16 values on its way into LDS.
+#pragma once
+
+#include "gemm_staged.h"
+
+namespace fmoe {
+
+// x = h + m + l with h, m, l the bf16 roundings of x and of what the ones before it leave: 8 + 8 + 8 bits and the signs of the
+// remainders cover the 24 of an fp32 value, so the sum is exact.  A product of two such values is taken as the six partial
+// products hh, hm, mh, hl, mm, lh; what is left out is below 2^-25 of it.  All six go into one fp32 accumulator.
+//
+// Both operands are multiplied by 2^24 first (and the sums by 2^-48 last), so that l of the smallest normal fp32 value is still a
+// normal bf16 value.  That, and the rounding of h, overflows for |x| near 2^104 and sums near 2^80; an infinity or a NaN in an
+// operand makes a NaN of the partial products as well.  A wave that finds a sum that is not finite computes its part of the tile
+// again with v_mfma_f32_32x32x2_f32, straight from global memory: what comes out for such operands is what that instruction gives.
+constexpr float kF32x3Scale = 16777216.0f, kF32x3Unscale = 0x1p-48f;
+
+template <int BM_, int BN_, int WGM_, int WGN_>
+struct TileF32x3 {
+    static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_;
+    static constexpr int NT = kWave * WGM * WGN;
+    static constexpr int TM = BM / WGM, TN = BN / WGN;
+    static constexpr int FM = TM / 32, FN = TN / 32;
+    static constexpr int BK = 32;                           // k per slice: 64-byte rows in each of the three planes
+    static constexpr int A_PLANE = BM * 64, B_PLANE = BN * 64;
+    static constexpr int LDS_BYTES = 3 * (A_PLANE + B_PLANE);
+    static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile must hold whole 32x32 fragments");
+    static_assert((BM * 4) % NT == 0 && (BN * 4) % NT == 0, "loader passes must be whole");
+};
+
+// Written out with packed operations on two values: 11 VALU instructions, which a block does once per operand value and slice.
+__device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = cvt_pk_bf16(a, b);
+    a -= __uint_as_float(h << 16);
+    b -= __uint_as_float(h & 0xffff0000u);
+    m = cvt_pk_bf16(a, b);
+    a -= __uint_as_float(m << 16);
+    b -= __uint_as_float(m & 0xffff0000u);
+    l = cvt_pk_bf16(a, b);
+}
+
+// Register-staged: the next slice is loaded while one is multiplied, then cut into parts and parked in the one LDS buffer (48 KB
+// for 128 x 128, so that three blocks share a CU and multiply in each other's barriers).  A second buffer, or two slices in
+// registers, cost blocks and were slower (16384 rows, 8 experts, 1024 -> 4096: 785 us with two slices, 764 with one).
+//
+// The error against 64 bits is that of the fp32 sums, 12 roundings per 32 k where v_mfma_f32_32x32x2_f32 has 16: 2-norm over
+// standard normal operands 2.5e-7 / 2.87e-7 at K = 256, 4.95e-7 / 5.73e-7 at 1024, 1.01e-6 / 1.15e-6 at 4096.
+//
+// NCONT: weights whose n is contiguous.  They are parked as they come, [32 k][128 n] per plane, and read with ds_read_b64_tr_b16.
+template <typename TL, int EPI, bool NCONT, bool A_SILU>
+__global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const GemmParams p) {
+    constexpr int BM = TL::BM, BN = TL::BN, NT = TL::NT, BK = TL::BK;
+    constexpr int FM = TL::FM, FN = TL::FN, TM = TL::TM, TN = TL::TN;
+    constexpr bool SWIGLU = EPI == FMOE_EPI_SWIGLU;
+    constexpr int BN_OUT = SWIGLU ? BN / 2 : BN;
+    constexpr int XP = BM * 4 / NT, WP = BN * 4 / NT;       // units of 8 values a thread brings in per slice
+    static_assert(EPI != FMOE_EPI_SWIGLU || FN % 2 == 0, "gate and up fragments come in pairs");
+    constexpr int NB = BN < 128 ? BN : 128;                 // NCONT: columns of a block of weights in LDS
+    static_assert(!NCONT || BN == 64 || BN % 128 == 0, "n-contiguous weights are parked in blocks of 64 or 128 columns");
+
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave % TL::WGM, wn = wave / TL::WGM;
+    const int khalf = lane >> 5;
+
+    BlockTile tile;
+    if (!tile.locate(p, BM)) return;
+    const int expert = __builtin_amdgcn_readfirstlane(tile.expert), nt = __builtin_amdgcn_readfirstlane(tile.nt);
+    const int rows_valid = __builtin_amdgcn_readfirstlane(tile.rows_valid);
+    const int64_t row0 = tile.row0;
+    const int n0 = nt * BN_OUT;
+
+    int Kdim = p.K;
+    int64_t k_begin = 0;
+    if (p.k_window) {
+        k_begin = p.k_window[expert];
+        const int64_t span = p.k_window[expert + 1] - k_begin;
+        Kdim = (int)(span < 0 ? 0 : (span < p.K ? span : p.K));
+    }
+
+    const float* a_base = reinterpret_cast<const float*>(p.a) + (int64_t)expert * p.a_stride_e + k_begin;
+    auto a_row = [&](int tile_row) -> const float* {
+        return a_base + source_row(p, row0 + (tile_row < rows_valid ? tile_row : 0)) * p.a_stride_row;
+    };
+    // the matrix and the output column behind column c of the tile
+    auto w_matrix = [&](int c) -> const float* {
+        return reinterpret_cast<const float*>(SWIGLU && c >= BN / 2 ? p.b2 : p.b) + (int64_t)expert * p.b_se;
+    };
+    auto w_col = [&](int c) -> int { return n0 + (SWIGLU && c >= BN / 2 ? c - BN / 2 : c); };
+
+    // ------------------------------------------------------------------- loaders
+    const float* xptr[XP];
+    const float* wptr[WP];
+    int w_second[WP];           // NCONT: elements from the unit's first 16-byte chunk to its second
+#pragma unroll
+    for (int i = 0; i < XP; ++i) xptr[i] = a_row((tid + i * NT) >> 2) + (tid & 3) * 8;
+#pragma unroll
+    for (int i = 0; i < WP; ++i) {
+        const int q = tid + i * NT;
+        if constexpr (NCONT) {
+            const int c = (q % (BN / 8)) * 8, k = q / (BN / 8);
+            const int n = w_col(c), first = n + 4 <= p.N ? n : p.N - 4, second = n + 8 <= p.N ? n + 4 : p.N - 4;
+            wptr[i] = w_matrix(c) + (k_begin + k) * p.b_sk + first;
+            w_second[i] = second - first;
+        } else {
+            const int c = q >> 2, n = w_col(c);
+            wptr[i] = w_matrix(c) + (int64_t)(n < p.N ? n : p.N - 1) * p.b_sn + k_begin + (q & 3) * 8;
+            w_second[i] = 4;
+        }
+    }
+    // NCONT: 16-byte chunk c of row k lies at position c ^ tr_swizzle(k): the four rows of a transposing read and the two groups
+    // of 16 lanes served together fall into eight different groups of 32 bytes of the 64 banks
+    auto tr_swizzle = [](int k) -> int { return NB == 64 ? 2 * (k & 2) : 4 * (k & 3); };
+    u32x4 xr[XP][2], wr[WP][2];
+    auto load_global = [&](int kt) {
+        const bool whole = (kt + 1) * BK <= Kdim;           // uniform: no per-lane predicate inside K
+        const int k0 = kt * BK;
+        auto chunk = [&](const float* src, int k) { return whole || k < Kdim ? *reinterpret_cast<const u32x4*>(src) : u32x4{0, 0, 0, 0}; };
+#pragma unroll
+        for (int i = 0; i < XP; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) xr[i][j] = chunk(xptr[i] + k0 + 4 * j, k0 + (tid & 3) * 8 + 4 * j);
+#pragma unroll
+        for (int i = 0; i < WP; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                if constexpr (NCONT) wr[i][j] = chunk(wptr[i] + (int64_t)k0 * p.b_sk + (j ? w_second[i] : 0), k0 + (tid + i * NT) / (BN / 8));
+                else wr[i][j] = chunk(wptr[i] + k0 + 4 * j, k0 + (tid & 3) * 8 + 4 * j);
+            }
+    };
+    auto park = [&](const u32x4 (&v)[2], uint8_t* dst, int plane) {
+        u32x4 h, m, l;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t ph, pm, pl;
+            split3(__uint_as_float(v[j >> 1][2 * (j & 1)]) * kF32x3Scale, __uint_as_float(v[j >> 1][2 * (j & 1) + 1]) * kF32x3Scale, ph, pm, pl);
+            h[j] = ph;
+            m[j] = pm;
+            l[j] = pl;
+        }
+        *reinterpret_cast<u32x4*>(dst) = h;
+        *reinterpret_cast<u32x4*>(dst + plane) = m;
+        *reinterpret_cast<u32x4*>(dst + 2 * plane) = l;
+    };
+    uint8_t* const sw = smem + 3 * TL::A_PLANE;
+    auto store_lds = [&]() {
+#pragma unroll
+        for (int i = 0; i < XP; ++i) {
+            if constexpr (A_SILU) {
+                xr[i][0] = silu_f32x4(xr[i][0]);
+                xr[i][1] = silu_f32x4(xr[i][1]);
+            }
+            const int q = tid + i * NT;
+            park(xr[i], smem + lds_off64(q >> 2, q & 3), TL::A_PLANE);
+        }
+#pragma unroll
+        for (int i = 0; i < WP; ++i) {
+            const int q = tid + i * NT;
+            if constexpr (NCONT) {
+                const int c8 = q % (BN / 8), k = q / (BN / 8);
+                park(wr[i], sw + c8 / (NB / 8) * (64 * NB) + k * (2 * NB) + (((c8 % (NB / 8)) ^ tr_swizzle(k)) << 4), TL::B_PLANE);
+            } else {
+                park(wr[i], sw + lds_off64(q >> 2, q & 3), TL::B_PLANE);
+            }
+        }
+    };
+
+    // ----------------------------------------------------------------- main loop
+    f32x16 acc[FN][FM];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+
+    // first tile column of weight fragment fn
+    auto frag_col = [&](int fn) -> int {
+        return SWIGLU ? (fn < FN / 2 ? 0 : BN / 2) + wn * (TN / 2) + (fn % (FN / 2)) * 32 : wn * TN + fn * 32;
+    };
+    auto read_w = [&](int fn, int plane, int sub) -> bf16x8 {
+        const uint8_t* s = sw + plane * TL::B_PLANE;
+        if constexpr (NCONT) {
+            const int l16 = lane & 15, row = 8 * khalf + (l16 >> 2);
+            const int col = frag_col(fn) % NB + 16 * ((lane >> 4) & 1) + 4 * (l16 & 3);
+            return read_tr8<8 * NB>(s + frag_col(fn) / NB * (64 * NB) + row * (2 * NB) + (((col >> 3) ^ tr_swizzle(row)) << 4) + (col & 7) * 2 +
+                                    sub * (32 * NB));
+        } else {
+            return *reinterpret_cast<const bf16x8*>(s + lds_off64(frag_col(fn) + (lane & 31), 2 * sub + khalf));
+        }
+    };
+    auto read_x = [&](int fm, int plane, int sub) -> bf16x8 {
+        return *reinterpret_cast<const bf16x8*>(smem + plane * TL::A_PLANE + lds_off64(wm * TM + fm * 32 + (lane & 31), 2 * sub + khalf));
+    };
+    auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+    const int KT = (Kdim + BK - 1) / BK;
+    load_global(0);
+    for (int kt = 0; kt < KT; ++kt) {
+        if (kt) barrier();              // every wave has read the slice before
+        store_lds();
+        if (kt + 1 < KT) load_global(kt + 1);
+        barrier();
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+            bf16x8 wf[3][FN], xf[3][FM];
+#pragma unroll
+            for (int pl = 0; pl < 3; ++pl) {
+#pragma unroll
+                for (int fn = 0; fn < FN; ++fn) wf[pl][fn] = read_w(fn, pl, sub);
+#pragma unroll
+                for (int fm = 0; fm < FM; ++fm) xf[pl][fm] = read_x(fm, pl, sub);
+            }
+            constexpr int W[6] = {0, 1, 0, 1, 2, 0}, X[6] = {0, 0, 1, 1, 0, 2};
+#pragma unroll
+            for (int t = 0; t < 6; ++t)
+#pragma unroll
+                for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+                    for (int fm = 0; fm < FM; ++fm)
+                        acc[fn][fm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[W[t]][fn], xf[X[t]][fm], acc[fn][fm], 0, 0, 0);
+        }
+    }
+
+    float probe = 0.0f;                 // NaN as soon as one sum is not finite
+#pragma unroll
+    for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                probe = __builtin_fmaf(acc[fn][fm][v], 0.0f, probe);
+                acc[fn][fm][v] *= kF32x3Unscale;
+            }
+    if (__builtin_expect(__any(probe != 0.0f), 0)) {
+        // (k in groups of 8, the wave halves on 4 each, as the register-staged kernel steps)
+        const float* xrow[FM];
+        const float* wrow[FN];
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm) xrow[fm] = a_row(wm * TM + fm * 32 + (lane & 31));
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn) {
+            const int c = frag_col(fn) + (lane & 31), n = w_col(c);
+            wrow[fn] = w_matrix(c) + (int64_t)(n < p.N ? n : p.N - 1) * p.b_sn + k_begin * p.b_sk;
+#pragma unroll
+            for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[fn][fm][v] = 0.0f;
+        }
+        for (int k0 = 0; k0 < Kdim; k0 += 8) {
+            const int k = k0 + 4 * khalf;
+            const bool in = k < Kdim;
+            u32x4 xv[FM], wv[FN];
+#pragma unroll
+            for (int fm = 0; fm < FM; ++fm) {
+                xv[fm] = in ? *reinterpret_cast<const u32x4*>(xrow[fm] + k) : u32x4{0, 0, 0, 0};
+                if constexpr (A_SILU) xv[fm] = silu_f32x4(xv[fm]);
+            }
+#pragma unroll
+            for (int fn = 0; fn < FN; ++fn) {
+                if constexpr (NCONT) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) wv[fn][j] = in ? __float_as_uint(wrow[fn][(int64_t)(k + j) * p.b_sk]) : 0u;
+                } else {
+                    wv[fn] = in ? *reinterpret_cast<const u32x4*>(wrow[fn] + k) : u32x4{0, 0, 0, 0};
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+                    for (int fm = 0; fm < FM; ++fm)
+                        acc[fn][fm] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(wv[fn][j]), __uint_as_float(xv[fm][j]),
+                                                                            acc[fn][fm], 0, 0, 0);
+        }
+    }
+    gemm_epilogue_f32<FM, FN, TM, TN, EPI>(p, acc, expert, n0, row0, rows_valid, wm, wn, lane);
+}
+
+}  // namespace fmoe

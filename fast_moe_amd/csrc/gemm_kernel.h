@@ -21,7 +21,9 @@
 //       weight stream does not stop at tile boundaries.
 //   grouped_gemm_kernel        register-staged, double-buffered LDS; serves everything the
 //       other two do not: arbitrary B strides and K / N tails (element loads), SiLU applied
-//       to A on load, fp32 operands (on tiles of their own, gemm_f32.hip).
+//       to A on load, fp32 operands of few k (on tiles of their own, gemm_f32.hip).
+//   grouped_gemm_f32x3_kernel  fp32 operands otherwise: register-staged too, every value cut into three
+//       bf16 parts on its way into LDS (gemm_f32x3.h).
 //
 // e4m3 row-wise scales that are exact powers of two (GemmParams::scale_pow2) are handed to
 // v_mfma_scale_f32_32x32x64_f8f6f4 as E8M0 codes of their reciprocals instead of being divided
@@ -47,7 +49,7 @@
 //     XCD one contiguous range of the tile order.
 //
 // Files: gemm_params.h (launch parameters, helpers), gemm_epilogue.h, gemm_ring.h, gemm_stream.h,
-// gemm_staged.h (the kernels), gemm_launch.h (kernel choice and launches).
+// gemm_staged.h, gemm_f32x3.h (the kernels), gemm_launch.h (kernel choice and launches).
 #pragma once
 
 #include "gemm_launch.h"

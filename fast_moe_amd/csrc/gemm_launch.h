@@ -38,12 +38,9 @@ int reserve_lds(Kern kern, int bytes, bool& done) {
     return FMOE_OK;
 }
 
-template <typename TL, int DT, int EPI, int LOADS, bool A_SILU>
-int launch_gemm(GemmParams p, hipStream_t stream) {
-    constexpr int bn_out = EPI == FMOE_EPI_SWIGLU ? TL::BN / 2 : TL::BN;
-    p.n_tiles = (p.N + bn_out - 1) / bn_out;
-    auto kern = grouped_gemm_kernel<TL, DT, EPI, LOADS, A_SILU>;
-    static bool attr_done = false;
+// one block per tile of TL, the grid an upper bound of their number
+template <typename TL, typename Kern>
+int launch_tiles(Kern kern, const GemmParams& p, bool& attr_done, hipStream_t stream) {
     if (int rc = reserve_lds(kern, TL::LDS_BYTES, attr_done)) return rc;
     const int64_t max_m_tiles = p.total_rows / TL::BM + p.E;
     const int64_t max_tiles = max_m_tiles * p.n_tiles;
@@ -55,6 +52,15 @@ int launch_gemm(GemmParams p, hipStream_t stream) {
     if (grid >= ((int64_t)1 << 31)) return fail(FMOE_ERR_UNSUPPORTED, "fmoe_grouped_gemm: grid too large");
     kern<<<(unsigned)grid, TL::NT, TL::LDS_BYTES, stream>>>(p);
     return check_launch("fmoe_grouped_gemm");
+}
+
+template <typename TL, int DT, int EPI, int LOADS, bool A_SILU>
+int launch_gemm(GemmParams p, hipStream_t stream) {
+    constexpr int bn_out = EPI == FMOE_EPI_SWIGLU ? TL::BN / 2 : TL::BN;
+    p.n_tiles = (p.N + bn_out - 1) / bn_out;
+    auto kern = grouped_gemm_kernel<TL, DT, EPI, LOADS, A_SILU>;
+    static bool attr_done = false;
+    return launch_tiles<TL>(kern, p, attr_done, stream);
 }
 
 int compute_units();   // CUs of the current device (gemm_api.hip)

@@ -153,6 +153,24 @@ __device__ __forceinline__ u32x4 silu_f32x4(u32x4 v) {
     return v;
 }
 
+// LDS byte offset of a 16-byte chunk of a 64-byte row: the ds_read_b128 of an MFMA fragment is conflict free
+__device__ __forceinline__ int lds_off64(int row, int chunk) {
+    return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4);
+}
+
+// two transposing LDS reads: this lane's 8 k values of one column of 16 rows (one MFMA's depth), a pointing at the lane's place
+// in the first of the two groups of 4 rows of its wave half, which lie STEP bytes apart
+template <int STEP>
+__device__ __forceinline__ bf16x8 read_tr8(const uint8_t* a) {
+    typedef __attribute__((ext_vector_type(4))) short s16x4;
+    typedef __attribute__((ext_vector_type(8))) short s16x8;
+    typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)a);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a + STEP));
+    const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(bf16x8, both);
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {   // s_waitcnt vmcnt(N) only
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));

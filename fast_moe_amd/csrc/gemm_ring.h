@@ -34,10 +34,6 @@ struct RingCfg {
     static_assert(TM % 32 == 0 && TN % 64 == 0, "wave tile must hold whole 32x32 fragments, FN even");
 };
 
-__device__ __forceinline__ int lds_off64(int row, int chunk) {   // 64-byte rows
-    return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4);
-}
-
 // One 16-byte-per-lane global -> LDS transfer from base + voff: a wave-uniform base in
 // SGPRs plus a 32-bit per-lane offset, so that stepping along K costs scalar adds only (VALU
 // instructions queue behind the MFMAs of the SIMD's other wave).  No immediate offset: the
@@ -743,17 +739,6 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             // something to fetch (past the end of the block's stream it re-reads the last
             // tile's rows into slots nobody looks at), and everything that depends on the
             // wave's half is a template parameter.
-            // two transposing reads: this lane's 8 k values of one column, 16 rows of 256 bytes
-            // (one MFMA's depth) starting at byte offset off of a slot part
-            auto read_tr = [&](const uint8_t* a) -> bf16x8 {
-                typedef __attribute__((ext_vector_type(4))) short s16x4;
-                typedef __attribute__((ext_vector_type(8))) short s16x8;
-                typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
-                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)a);
-                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a + 1024));
-                const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                return __builtin_bit_cast(bf16x8, both);
-            };
             // item: the slice's number inside the tile; mask_c: zero the weight-side values whose
             // k lies at or beyond the end of the tile's window (XTR, the tile's last slices)
             auto load_block = [&](bf16x8 (&wf)[FN], bf16x8 (&xf)[FM], int slot_i, int sub, int item, auto mask_c, auto act_c) {
@@ -765,12 +750,12 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 const int chunk = 2 * sub + khalf;
 #pragma unroll
                 for (int fn = 0; fn < FN; ++fn) {
-                    if constexpr (WTR) wf[fn] = read_tr(sw + wtr_off[fn] + sub * 4096);
+                    if constexpr (WTR) wf[fn] = read_tr8<1024>(sw + wtr_off[fn] + sub * 4096);
                     else wf[fn] = *reinterpret_cast<const bf16x8*>(sw + lds_off64(wfrag_row[fn], chunk));
                 }
 #pragma unroll
                 for (int fm = 0; fm < ACT; ++fm) {
-                    if constexpr (XTR) xf[fm] = read_tr(sx + xtr_off[fm] + sub * 4096);
+                    if constexpr (XTR) xf[fm] = read_tr8<1024>(sx + xtr_off[fm] + sub * 4096);
                     else xf[fm] = *reinterpret_cast<const bf16x8*>(sx + lds_off64(xfrag_row[fm], chunk));
                 }
                 if constexpr (MASK_TAIL) {      // (a fragment is one 16-byte chunk: masked whole or not at all)

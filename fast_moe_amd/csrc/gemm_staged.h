@@ -24,6 +24,87 @@ __device__ __forceinline__ int lds_off(int row, int chunk) {     // 128-byte row
 
 enum { kLoadElements = 0, kLoadChunks = 1, kLoadChunksN = 2 };
 
+// The tile of a block: one block per tile, tiles located from offsets[] by every wave for itself.
+struct BlockTile {
+    int expert, nt, rows_valid;
+    int64_t row0;
+
+    // false: the launch has no tile for this block (the grid is an upper bound)
+    __device__ __forceinline__ bool locate(const GemmParams& p, int BM) {
+        const int lane = threadIdx.x & 63;
+        const int64_t R = p.total_rows;
+        int64_t total_m = 0;
+        for (int e0 = 0; e0 < p.E; e0 += kWave) {
+            const int e = e0 + lane;
+            int64_t len = 0;
+            if (e < p.E) {
+                const int64_t lo = clamp_i64(p.offsets[e], 0, R), hi = clamp_i64(p.offsets[e + 1], 0, R);
+                len = hi > lo ? hi - lo : 0;
+            }
+            const long long inc = wave_inclusive_scan((long long)((len + BM - 1) / BM));
+            total_m += wave_bcast(inc, kWave - 1);
+        }
+        const int64_t total_tiles = total_m * p.n_tiles;
+        const int64_t per_xcd = (total_tiles + kNumXcd - 1) / kNumXcd;
+        const int64_t slot = blockIdx.x / kNumXcd;
+        const int64_t group_span = (int64_t)kGroupM * p.n_tiles;
+        int64_t group;
+        int within;
+        if (p.k_window) {
+            // the cost of a tile follows its expert's contraction length, so contiguous tile ranges
+            // per XCD would leave one XCD with the long experts: deal the groups out round-robin
+            group = slot / group_span * kNumXcd + blockIdx.x % kNumXcd;
+            within = (int)(slot % group_span);
+        } else {
+            if (slot >= per_xcd) return false;
+            const int64_t logical = (int64_t)(blockIdx.x % kNumXcd) * per_xcd + slot;
+            if (logical >= total_tiles) return false;
+            group = logical / group_span;
+            within = (int)(logical - group * group_span);
+        }
+        const int64_t first_m = group * kGroupM;
+        if (first_m >= total_m) return false;
+        const int gsize = (int)(total_m - first_m < kGroupM ? total_m - first_m : kGroupM);
+        if (within >= gsize * p.n_tiles) return false;
+        const int64_t mt = first_m + within % gsize;
+        nt = within / gsize;
+
+        expert = 0;
+        row0 = 0;
+        rows_valid = 0;
+        {
+            int64_t before = 0;
+            for (int e0 = 0; e0 < p.E; e0 += kWave) {
+                const int e = e0 + lane;
+                int64_t lo = 0, len = 0;
+                if (e < p.E) {
+                    lo = clamp_i64(p.offsets[e], 0, R);
+                    const int64_t hi = clamp_i64(p.offsets[e + 1], 0, R);
+                    len = hi > lo ? hi - lo : 0;
+                }
+                const long long tiles = (len + BM - 1) / BM;
+                const long long inc = wave_inclusive_scan(tiles);
+                const long long excl = before + inc - tiles;
+                const bool mine = mt >= excl && mt < excl + tiles;
+                const unsigned long long hit = __ballot(mine);
+                if (hit) {
+                    const int src = __ffsll((long long)hit) - 1;
+                    const int64_t f_lo = wave_bcast(lo, src);
+                    const int64_t f_len = wave_bcast(len, src);
+                    const int64_t f_excl = wave_bcast((int64_t)excl, src);
+                    expert = e0 + src;
+                    row0 = f_lo + (mt - f_excl) * BM;
+                    const int64_t left = f_lo + f_len - row0;
+                    rows_valid = (int)(left < BM ? left : BM);
+                    break;
+                }
+                before += wave_bcast(inc, kWave - 1);
+            }
+        }
+        return rows_valid > 0;      // (true for consistent offsets)
+    }
+};
+
 // DT: operand type, kDtBf16 / kDtE4m3 (bf16 output) or kDtF32 (fp32 operands, bias and output,
 // v_mfma_f32_32x32x2_f32: full fp32 products, no tf32).
 // LOADS: kLoadChunks 16-byte loads along k of both operands; kLoadChunksN (fp32) the same for A, and
@@ -52,77 +133,10 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_kernel(const GemmParams p
     const int wave = tid >> 6;
     const int wm = wave % TL::WGM, wn = wave / TL::WGM;
 
-    // ------------------------------------------------------------ scheduling
-    const int64_t R = p.total_rows;
-    int64_t total_m = 0;
-    for (int e0 = 0; e0 < p.E; e0 += kWave) {
-        const int e = e0 + lane;
-        int64_t len = 0;
-        if (e < p.E) {
-            const int64_t lo = clamp_i64(p.offsets[e], 0, R), hi = clamp_i64(p.offsets[e + 1], 0, R);
-            len = hi > lo ? hi - lo : 0;
-        }
-        const long long inc = wave_inclusive_scan((long long)((len + BM - 1) / BM));
-        total_m += wave_bcast(inc, kWave - 1);
-    }
-    const int64_t total_tiles = total_m * p.n_tiles;
-    const int64_t per_xcd = (total_tiles + kNumXcd - 1) / kNumXcd;
-    const int64_t slot = blockIdx.x / kNumXcd;
-    const int64_t group_span = (int64_t)kGroupM * p.n_tiles;
-    int64_t group;
-    int within;
-    if (p.k_window) {
-        // the cost of a tile follows its expert's contraction length, so contiguous tile ranges
-        // per XCD would leave one XCD with the long experts: deal the groups out round-robin
-        group = slot / group_span * kNumXcd + blockIdx.x % kNumXcd;
-        within = (int)(slot % group_span);
-    } else {
-        if (slot >= per_xcd) return;
-        const int64_t logical = (int64_t)(blockIdx.x % kNumXcd) * per_xcd + slot;
-        if (logical >= total_tiles) return;
-        group = logical / group_span;
-        within = (int)(logical - group * group_span);
-    }
-    const int64_t first_m = group * kGroupM;
-    if (first_m >= total_m) return;
-    const int gsize = (int)(total_m - first_m < kGroupM ? total_m - first_m : kGroupM);
-    if (within >= gsize * p.n_tiles) return;
-    const int64_t mt = first_m + within % gsize;
-    const int nt = within / gsize;
-
-    int expert = 0;
-    int64_t row0 = 0;
-    int rows_valid = 0;
-    {
-        int64_t before = 0;
-        for (int e0 = 0; e0 < p.E; e0 += kWave) {
-            const int e = e0 + lane;
-            int64_t lo = 0, len = 0;
-            if (e < p.E) {
-                lo = clamp_i64(p.offsets[e], 0, R);
-                const int64_t hi = clamp_i64(p.offsets[e + 1], 0, R);
-                len = hi > lo ? hi - lo : 0;
-            }
-            const long long tiles = (len + BM - 1) / BM;
-            const long long inc = wave_inclusive_scan(tiles);
-            const long long excl = before + inc - tiles;
-            const bool mine = mt >= excl && mt < excl + tiles;
-            const unsigned long long hit = __ballot(mine);
-            if (hit) {
-                const int src = __ffsll((long long)hit) - 1;
-                const int64_t f_lo = wave_bcast(lo, src);
-                const int64_t f_len = wave_bcast(len, src);
-                const int64_t f_excl = wave_bcast((int64_t)excl, src);
-                expert = e0 + src;
-                row0 = f_lo + (mt - f_excl) * BM;
-                const int64_t left = f_lo + f_len - row0;
-                rows_valid = (int)(left < BM ? left : BM);
-                break;
-            }
-            before += wave_bcast(inc, kWave - 1);
-        }
-    }
-    if (rows_valid <= 0) return;   // unreachable for consistent offsets
+    BlockTile tile;
+    if (!tile.locate(p, BM)) return;
+    const int expert = tile.expert, nt = tile.nt, rows_valid = tile.rows_valid;
+    const int64_t row0 = tile.row0;
 
     // per-expert contraction window (weight gradients): both operands start k_begin elements in
     int Kdim = p.K;

@@ -1149,6 +1149,75 @@ def test_fp32_tile_choice(E, rows, N, epi, tile):
     assert f"grouped_gemm_kernel<fmoe::TileCfg<{tile}," in ran, ran
 
 
+@pytest.mark.parametrize("E,rows,K,N,layout,epi,tile", [
+    (3, 190, 68, 68, "kn", 0, "64, 64"), (3, 190, 96, 60, "nk", 0, "64, 64"),          # the least K, a rest of one chunk / whole slices
+    (1, 65, 132, 4, "kn", 1, "64, 64"), (2, 600, 100, 8192, "nk", 0, "64, 128"),       # the least N; more than four small tiles per CU
+    (2, 600, 100, 8192, "kn", 1, "64, 128"), (3, 700, 72, 4100, "nk", "silu", "64, 128"),
+    (5, 700, 100, 132, "kn", 2, "64, 128"), (5, 700, 100, 132, "nk", 2, "64, 128"),    # gate and up halves of a tile
+    (3, 4800, 100, 1156, "nk", 0, "128, 128"), (3, 4800, 100, 1156, "kn", 0, "128, 128"),
+    (3, 4800, 132, 1156, "nk", "silu", "128, 128"), (2, 4500, 68, 580, "kn", 2, "128, 128"), (70, 4800, 96, 1156, "nk", 2, "128, 128"),
+])
+@pytest.mark.parametrize("case", ["normal", "small", "large", "special"])
+def test_fp32_on_bf16_matrix_cores(E, rows, K, N, layout, epi, tile, case):
+    """fp32 values in three bf16 parts, on every tile.  small, large: rows and columns scaled by powers of two, operands
+    down to the smallest normal values, up to sums where the parts overflow.  special: an infinity, a NaN and values beyond 2^104 in single
+    rows and columns, whose results are those of the plain fp32 sum; the other results do not see them.  Against float64; the
+    bound of a K-term fp32 sum and the partial products left out (2^-25 each), (K + 3) * 2^-24 * sum |a||b|; as in
+    test_fp32_kernel_tiles_and_weight_layouts through SiLU and the product."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    g = torch.Generator(device="cuda").manual_seed(K + N + rows)
+    randn_ = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    off = torch.tensor([0] + sorted(torch.randint(0, rows, (E - 1,), generator=torch.Generator().manual_seed(N)).tolist()) + [rows]).cuda()
+    a_silu, epi = epi == "silu", 0 if epi == "silu" else epi
+    x, ws = randn_(rows, K), [randn_(E, K, N) for _ in range(2)]
+    odd_rows = torch.zeros(rows, dtype=torch.bool, device="cuda")
+    odd_cols = torch.zeros(N, dtype=torch.bool, device="cuda")
+    if case in ("small", "large"):
+        a_silu, epi = False, _lib.EPI_NONE      # (SiLU and the product have ranges of their own)
+        lo, hi, w_hi = (-112, -40, 40) if case == "small" else (-90, 70, 26)
+        x = torch.where(x.abs() < 2.0 ** -14, torch.ones_like(x), x)        # (no denormal value)
+        x *= torch.exp2(torch.randint(lo, hi, (rows, 1), generator=g, device="cuda").float())
+        ws = [w * torch.exp2(torch.randint(0, w_hi, (1, 1, N), generator=g, device="cuda").float()) for w in ws]
+    if case == "special":
+        x[5, K - 1], x[rows - 1, 0], x[rows // 2, 3] = float("inf"), float("nan"), 3e38
+        odd_rows[[5, rows - 1, rows // 2]] = True
+        for w in ws:
+            w[:, 1, N - 1], w[:, 2, 1] = float("inf"), 2.0 ** 110
+        odd_cols[[1, N - 1]] = True
+    if layout == "nk":
+        ws = [w.permute(0, 2, 1).contiguous().permute(0, 2, 1) for w in ws]
+    kw = dict(total_rows=rows, b2=ws[1] if epi == _lib.EPI_SWIGLU else None, epilogue=epi, a_silu=a_silu)
+    out = ops.grouped_gemm(off, x, ws[0], **kw)
+    ran, = kernels_run(lambda: ops.grouped_gemm(off, x, ws[0], **kw))
+    assert f"grouped_gemm_f32x3_kernel<fmoe::TileF32x3<{tile if case in ('normal', 'special') else ''}" in ran, ran
+    unit = (K + 3) * 2.0 ** -24 + (2.0 ** -21 if a_silu else 0)
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        a = torch.nn.functional.silu(x[lo:hi].double()) if a_silu else x[lo:hi].double()
+        want, err = a @ ws[0][e].double(), unit * (a.abs() @ ws[0][e].double().abs()) + 2.0 ** -149
+        if epi != _lib.EPI_NONE:
+            want, err = torch.nn.functional.silu(want), 1.1 * err + 2.0 ** -21 * want.abs()
+        if epi == _lib.EPI_SWIGLU:
+            up, up_err = a @ ws[1][e].double(), unit * (a.abs() @ ws[1][e].double().abs())
+            want, err = want * up, err * up.abs() + (want.abs() + err) * up_err + 2.0 ** -23 * (want * up).abs()
+        got, plain = out[lo:hi].double(), ~odd_rows[lo:hi, None] & ~odd_cols[None]
+        assert bool(((got - want).abs() <= err)[plain].all()), f"expert {e}"
+        if case == "special" and epi == _lib.EPI_NONE and not a_silu:
+            plain_fp32 = x[lo:hi].cpu() @ ws[0][e].cpu()
+            far = want.abs().cpu() > 1e39                       # beyond fp32 for certain, whatever the order
+            near = want.abs().cpu() < 1e38
+            assert torch.equal(got.cpu().isnan(), plain_fp32.isnan()) and bool(got.cpu()[far].isinf().all())
+            assert bool(((got - want).abs() <= err).cpu()[near].all())
+
+
+@pytest.mark.parametrize("K,new", [(64, False), (68, True)])
+def test_fp32_kernel_for_short_k(K, new):
+    from fast_moe_amd.kernels.hip import ops
+    x, w, off = torch.zeros(64, K, device="cuda"), torch.zeros(1, 64, K, device="cuda").permute(0, 2, 1), torch.tensor([0, 64]).cuda()
+    ran, = kernels_run(lambda: ops.grouped_gemm(off, x, w, total_rows=64))
+    assert ("f32x3" in ran) == new, ran
+
+
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
     (3, 130, 136, 264, "nk", 0), (3, 130, 192, 136, "kn", 0),       # the least K: three pairs of K-slices, the last in part / whole
     (1, 64, 256, 256, "kn", 1), (1, 65, 256, 256, "nk", 1),         # one whole tile; one row more
