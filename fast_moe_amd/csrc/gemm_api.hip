@@ -200,6 +200,7 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
                           (d->a_stride_e % chunk) == 0 && aligned16(d->a) && aligned16(d->b) &&
                           (!swiglu || aligned16(d->b2)) && near_tr;
     p.ring_short = short_tr || (short_ok && near && (fast8 || (fast && ring_short_pays(p, esize, d->epilogue))));
+    p.direct = fast && !big && !(d->a_silu && d->epilogue != FMOE_EPI_NONE) && !d->k_window && !two && !row_indexed && !gated && direct_pays(p, esize, swiglu);
     // the second product exists in that kernel only; a caller that is turned away runs two
     // GEMMs and adds
     if (two)
@@ -241,6 +242,9 @@ extern "C" int fmoe_grouped_gemm(const fmoe_gemm_desc* d, fmoe_stream_t stream_)
     int sel;
     if (int rc = prepare_gemm(d, p, sel)) return rc;
     if (sel < 0) return FMOE_OK;
+    if (p.direct)
+        return run_gemm_direct(p, d->a_dtype == FMOE_E4M3 ? kDtE4m3 : d->a_dtype == FMOE_F32 ? kDtF32 : kDtBf16, d->epilogue, d->a_silu != 0,
+                               stream);
     if (d->a_dtype == FMOE_E4M3) return run_gemm_fp8(p, d->epilogue, sel, stream);
     if (d->a_dtype == FMOE_F32) return run_gemm_f32(p, d->epilogue, d->a_silu != 0, sel, stream);
     return run_gemm_bf16(p, d->epilogue, d->a_silu != 0, sel, stream);

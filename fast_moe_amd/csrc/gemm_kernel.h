@@ -19,6 +19,8 @@
 //       CU; a K-slice travels global -> registers -> LDS while the previous one is multiplied,
 //       and the next tile's first slice is loaded before the current tile's epilogue, so the
 //       weight stream does not stop at tile boundaries.
+//       A launch of few tiles takes its other form (gemm_direct.h): 64 x 64 tiles whose waves share K
+//       and load weights straight into their registers.
 //   grouped_gemm_kernel        register-staged, double-buffered LDS; serves everything the
 //       other two do not: arbitrary B strides and K / N tails (element loads), SiLU applied
 //       to A on load, fp32 operands of few k (on tiles of their own, gemm_f32.hip).
@@ -49,7 +51,7 @@
 //     XCD one contiguous range of the tile order.
 //
 // Files: gemm_params.h (launch parameters, helpers), gemm_epilogue.h, gemm_ring.h, gemm_stream.h,
-// gemm_staged.h, gemm_f32x3.h (the kernels), gemm_launch.h (kernel choice and launches).
+// gemm_staged.h, gemm_f32x3.h, gemm_direct.h (the kernels), gemm_launch.h (kernel choice and launches).
 #pragma once
 
 #include "gemm_launch.h"

@@ -192,6 +192,38 @@ inline bool ring_short_pays(const GemmParams& p, int esize, int epilogue) {
            (p.total_rows + TileRingS::BM - 1) / TileRingS::BM * n_tiles > 2 * cus;
 }
 
+// The streaming kernels that take the weights straight into registers (gemm_direct.hip).
+int run_gemm_direct(const GemmParams& p, int dtype, int epilogue, bool a_silu, hipStream_t stream);
+
+// row tiles of a launch at most, however the experts share the rows
+inline int64_t most_row_tiles(int64_t rows, int64_t num_experts, int bm) {
+    const int64_t experts = num_experts < rows ? num_experts : rows;        // that can hold a row
+    return (rows - experts) / bm + experts;
+}
+inline int direct_columns(int n, bool swiglu) { return swiglu ? (n + 31) / 32 : (n + 63) / 64; }
+
+// Where they are taken (weights with k contiguous, 16-byte loads, no gate), up to 16 rows per expert on average.  us per GEMM, the
+// kernel that ran before (the 64-row ring, the streaming or the register-staged kernel) / this one; even load unless said:
+//   * no more tiles than CUs: the tile that others walk alone (64 x 256, K serial) is a quarter as wide and its K is shared by eight
+//     waves.  24 rows, 10 experts, 2112 -> 408 18.3 / 11.4 (e4m3 14.9 / 6.8, fp32 56.1 / 20.5); 5 rows, 35 experts, 2696 -> 1024
+//     32.2 / 10.4 (fp32 72.2 / 21.5); 64 rows, 4 experts, 4096 -> 4096 33.3 / 24.7; 128 rows, 8 experts, 128 -> 256 8.2 / 6.3; 160 rows, 10
+//     experts, 1024 -> 1024 12.0 / 8.9, Zipf 11.9 / 11.5
+//   * up to two per CU: e4m3, and rows of K up to 1664 bytes.  98 rows, 11 experts, 2496 -> 2 x 832 bf16 23.4 / 25.6 (not taken), e4m3
+//     19.0 / 13.3; 98 rows, 11 experts, 832 -> 2496 bf16 12.5 / 11.7
+//   * beyond, an even load would gain (512 rows, 128 experts, 4096 -> 2 x 1536 543 / 529, e4m3 286 / 264), but an expert with many rows
+//     has its weights read from L2 for every 64 of them and every 32 columns: 1024 rows, Zipf 488 / 606.
+//   * fp32 streams half as much weight for a product and the other kernel is the slower one: 512 rows, 128 experts, 4096 -> 2 x 1536
+//     1475 / 1066, Zipf 1011 / 844, nine tenths in one expert 653 / 543.  Not with short K and rows enough for a hot expert (400 rows,
+//     24 experts, 896 -> 2192: even 48.5 / 46.0, one hot expert 48.8 / 56.6), nor with K of two slices (gemm_f32.hip).
+// Calls of up to three rows belong to the 64-row ring by the tests of the rule before this one.
+inline bool direct_pays(const GemmParams& p, int esize, bool swiglu) {
+    const int64_t experts = p.E < p.total_rows ? p.E : p.total_rows, cus = compute_units();
+    if (p.total_rows < 4 || p.total_rows > 16 * experts) return false;
+    const int64_t tiles = most_row_tiles(p.total_rows, p.E, 64) * direct_columns(p.N, swiglu);
+    if (esize == 4) return p.K > 64 && (p.K >= 1024 || tiles <= 2 * cus || p.total_rows <= 4 * experts);
+    return tiles <= cus || (tiles <= 2 * cus && (esize == 1 || p.K * esize <= 1664));
+}
+
 // The 5-slot ring needs every byte of a 160 KB LDS, an even number of K-slices per tile,
 // row numbers that fit 32 bits and few enough experts for the register tables.
 template <bool FP8, int EPI>

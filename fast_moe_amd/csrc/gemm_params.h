@@ -40,6 +40,7 @@ struct GemmParams {
     int64_t out_stride;
     int n_tiles;
     int ring_short;                     // the ring on 64-row tiles runs the call
+    int direct;                         // ... or the streaming kernel whose weights go straight into registers
     int vec_store;                      // 16-byte stores of 8 bf16 are legal
     int scale_vec;                      // e4m3: 16-byte loads of 4 weight scales are legal
     int scale_pow2;                     // e4m3: the caller promises that every scale is an exact power of two

@@ -1218,6 +1218,114 @@ def test_fp32_kernel_for_short_k(K, new):
     assert ("f32x3" in ran) == new, ran
 
 
+@pytest.mark.parametrize("lens,K,N,epi", [
+    ([16, 1, 17, 30], 392, 68, 0), ([33, 0, 64, 31, 0, 0, 0, 0], 264, 260, 1),     # one, two and four fragments of 16 rows, full and one row more
+    ([65, 0, 0, 0, 0, 0, 2], 520, 40, 2),                               # more than a tile's rows; SwiGLU columns in part
+    ([0, 3, 1], 72, 8, 0), ([2, 2], 128, 64, 2),                        # fewer 128-byte pieces than waves; one whole tile
+    ([1] * 70 + [0, 9], 104, 132, 0), ([4, 0] * 80, 136, 72, 1),        # more experts than lanes
+    ([5] * 11, 800, 2900, 0), ([3] * 20, 824, 1096, "silu"),           # more tiles than CUs
+    ([7, 0, 20, 8], 1048, 200, "silu"),
+])
+@pytest.mark.parametrize("dtype", ["bf16", "fp8", "f32"])
+@pytest.mark.parametrize("extras", [False, True])
+def test_streaming_kernel_of_few_tiles(lens, K, N, epi, dtype, extras):
+    """Weights straight into registers.  The operands are the left columns of wider tensors whose other columns are NaN.  extras:
+    gathered rows, bias and, with SwiGLU, the two pre-activations.  Against float64 with the roundings of the bf16 path
+    (test_ring_kernel_contraction_tails) and, fp32, the bound of test_fp32_on_bf16_matrix_cores with one rounding more per bias."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    a_silu, epi = epi == "silu", 0 if epi == "silu" else epi
+    if dtype == "fp8":
+        a_silu, K = False, (K + 15) // 16 * 16
+    f32, E, rows = dtype == "f32", len(lens), sum(lens)
+    dt, g = torch.float32 if f32 else BF16, torch.Generator(device="cuda").manual_seed(K + N)
+    off = torch.tensor([0, *torch.tensor(lens).cumsum(0)]).cuda()
+    randn_ = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    def wide(*shape):
+        t = torch.full((*shape[:-1], shape[-1] + 16), float("nan"), dtype=dt, device="cuda")
+        t[..., :shape[-1]] = (randn_(*shape) * shape[-1] ** -0.5).to(dt)
+        return t[..., :shape[-1]]
+    T = (rows + 1) // 2 if extras else rows
+    x, ws = wide(T, K), [wide(E, N, K) for _ in range(2)]
+    index = torch.randint(0, 2 * T, (rows,), generator=g, device="cuda") if extras else None
+    bias = [randn_(E, N).to(dt) for _ in range(2)] if extras else [None, None]
+    swiglu = epi == _lib.EPI_SWIGLU
+    aux = tuple(torch.zeros(rows, N, dtype=dt, device="cuda") for _ in range(2)) if extras and swiglu else None
+    kw = dict(total_rows=rows, row_index=index, index_div=2 if extras else 1, bias=bias[0], epilogue=epi, a_silu=a_silu, aux=aux)
+    if swiglu:
+        kw.update(b2=ws[1].permute(0, 2, 1), bias2=bias[1])
+    args = (x, ws[0].permute(0, 2, 1))
+    if dtype == "fp8":
+        qx, sx = ops.quant_rows_fp8(x)
+        qw = [ops.quant_rows_fp8(w) for w in ws]
+        kw.update(a_scale=sx, b_scale=qw[0][1], scales_pow2=True)
+        if swiglu:
+            kw.update(b2=qw[1][0].permute(0, 2, 1), b2_scale=qw[1][1])
+        args = (qx, qw[0][0].permute(0, 2, 1))
+        x, ws = qx.float() / sx[:, None], [q.float() / s[..., None] for q, s in qw]
+    out = ops.grouped_gemm(off, *args, **kw)
+    ran, = kernels_run(lambda: ops.grouped_gemm(off, *args, **kw))
+    assert "grouped_gemm_stream_kernel<fmoe::StreamCfg<" in ran, ran
+    source = x if index is None else x[index // 2]
+    unit = (K + 4) * 2.0 ** -24 + (2.0 ** -21 if a_silu else 0)
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        a = source[lo:hi].double()
+        a = torch.nn.functional.silu(a) if a_silu else a
+        if a_silu and not f32:
+            a = a.to(BF16).double()
+        pre, err = [], []
+        for w, b in zip(ws, bias):
+            add = b[e].double() if b is not None else torch.zeros(N, dtype=torch.float64, device="cuda")
+            pre.append(a @ w[e].double().t() + add)
+            err.append(unit * (a.abs() @ w[e].double().abs().t() + add.abs()))
+        want, bound = pre[0], err[0]
+        if epi != _lib.EPI_NONE:
+            want, bound = torch.nn.functional.silu(want), 1.1 * bound + 2.0 ** -21 * want.abs()
+        if swiglu:
+            want, bound = want * pre[1], bound * pre[1].abs() + (want.abs() + bound) * err[1] + 2.0 ** -23 * (want * pre[1]).abs()
+        pairs = [(out, want, bound)] + ([(aux[0], pre[0], err[0]), (aux[1], pre[1], err[1])] if aux else [])
+        for got, ref, b in pairs:
+            if f32:
+                assert bool(((got[lo:hi].double() - ref).abs() <= b).all()), f"expert {e}"
+            else:
+                assert_bf16_close(got[lo:hi], ref.float(), rtol=1.6e-2, atol=4e-3, what=f"expert {e}")
+
+
+def test_streaming_kernel_recomputes_fp32_sums_that_are_not_finite():
+    """As test_fp32_on_bf16_matrix_cores, special."""
+    from fast_moe_amd.kernels.hip import ops
+    g = torch.Generator(device="cuda").manual_seed(1)
+    off = torch.tensor([0, 9, 9, 40]).cuda()
+    x, w = (torch.randn(*s, generator=g, device="cuda") for s in ((40, 200), (3, 130, 200)))
+    x[3, 0], x[20, 199], x[39, 7] = float("inf"), float("nan"), 2.0 ** 110
+    w[2, 5, 11], w[0, 129, 3] = float("-inf"), 2.0 ** 120
+    out = ops.grouped_gemm(off, x, w.permute(0, 2, 1), total_rows=40)
+    for e in (0, 2):
+        lo, hi = int(off[e]), int(off[e + 1])
+        got, plain, want = out[lo:hi].cpu(), x[lo:hi].cpu() @ w[e].t().cpu(), x[lo:hi].double() @ w[e].double().t()
+        assert torch.equal(got.isnan(), plain.isnan()) and torch.equal(got.isinf(), plain.isinf())
+        assert torch.equal(got[plain.isinf()], plain[plain.isinf()])
+        err, fine = 203 * 2.0 ** -24 * (x[lo:hi].double().abs() @ w[e].double().abs().t()), plain.isfinite()
+        assert bool(((got.double() - want.cpu()).abs() <= err.cpu())[fine].all())
+
+
+@pytest.mark.parametrize("E,rows,K,N,dtype,direct", [
+    (16, 16, 1664, 1024, "bf16", True), (16, 16, 1664, 1024 + 1, "bf16", False),        # one tile per CU; K of more than 1664 bytes beyond
+    (16, 16, 832, 2048, "bf16", True), (16, 16, 832, 2049, "bf16", False), (16, 16, 2048, 2048, "fp8", True), (16, 16, 2048, 2049, "fp8", False),
+    (16, 256, 1664, 1024, "bf16", False), (16, 250, 832, 64, "bf16", True), (4, 65, 832, 64, "bf16", False),
+    (16, 100, 1020, 2049, "f32", False), (16, 64, 1020, 2049, "f32", True), (16, 100, 1024, 2049, "f32", True), (16, 16, 64, 64, "f32", False),
+])
+def test_streaming_kernel_choice(E, rows, K, N, dtype, direct):
+    """Which calls the kernel above takes, on either side of the rule's lines."""
+    from fast_moe_amd.kernels.hip import ops
+    dt = {"bf16": BF16, "fp8": torch.float8_e4m3fn, "f32": torch.float32}[dtype]
+    x, w = torch.zeros(rows, K, device="cuda").to(dt), torch.zeros(E, N, K, dtype=BF16, device="cuda").to(dt).permute(0, 2, 1)
+    kw = dict(a_scale=torch.ones(rows, device="cuda"), b_scale=torch.ones(E, N, device="cuda")) if dtype == "fp8" else {}
+    off = (torch.arange(E + 1) * rows // E).cuda()
+    ran, = kernels_run(lambda: ops.grouped_gemm(off, x, w, total_rows=rows, **kw))
+    assert ("StreamCfg<" in ran) == direct, ran
+
+
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
     (3, 130, 136, 264, "nk", 0), (3, 130, 192, 136, "kn", 0),       # the least K: three pairs of K-slices, the last in part / whole
     (1, 64, 256, 256, "kn", 1), (1, 65, 256, 256, "nk", 1),         # one whole tile; one row more
