@@ -4,7 +4,7 @@
 // function of the selected ids (a stable counting sort), so they are
 // reproducible bit for bit.
 //
-// Two launches on one stream, no host synchronisation.  The tokens are cut into up to 256
+// Two launches on one stream (one for a batch of few tokens, route_block_kernel), no host synchronisation.  The tokens are cut into up to 256
 // chunks (one block each: 16 waves up to 256 experts, 4 beyond; a wave owns a contiguous
 // share of its chunk):
 //   1. topk_hist_kernel (or compact_hist_kernel for caller-supplied ids): a token's scores sit
@@ -131,30 +131,16 @@ __device__ __forceinline__ void wave_lds_fence() {
 // One token per LPT lanes (8 or 16: a token's lanes sit in one DPP row), VPL scores per lane
 // (expert id = v*LPT + sub).  K rounds of "largest remaining key, lowest expert id among equal
 // keys", each two group maxima on the DPP network; the round is the slot (descending score,
-// ties -> lower expert id).
-template <typename T, int LPT, int VPL, int WPB>
-__global__ __launch_bounds__(WPB * kWave) void topk_hist_kernel(const T* __restrict__ scores, int64_t num_tokens,
-                                                        int E, int K, int renorm, int64_t tokens_per_wave,
-                                                        int64_t* __restrict__ topk_idx,
-                                                        T* __restrict__ gates,
-                                                        uint16_t* __restrict__ compact,
-                                                        int32_t* __restrict__ sub_hist,
-                                                        int32_t* __restrict__ tot_hist) {
+// ties -> lower expert id).  A wave takes tokens [w_begin, w_end), TPW of them per pass; compact (global memory or
+// LDS) receives the expert ids of its positions, s_hist (this wave's, E entries, zeroed) their counts, s_sel is its scratch.
+template <typename T, int LPT, int VPL>
+__device__ __forceinline__ void select_experts(const T* __restrict__ scores, int64_t w_begin, int64_t w_end, int64_t tokens_per_wave,
+                                               int E, int K, int renorm, int64_t* __restrict__ topk_idx, T* __restrict__ gates,
+                                               uint16_t* compact, float (&s_sel)[kWave / LPT][64], int32_t* s_hist) {
     constexpr int TPW = kWave / LPT;          // tokens per wave and pass
-    constexpr int NT = WPB * kWave;
-    __shared__ float s_sel[WPB][TPW][64];     // selected scores by slot (K <= 64)
-    extern __shared__ int32_t s_hist[];       // [WPB][E] experts chosen by this wave's tokens
     const int lane = lane_id();
-    const int wave = threadIdx.x / kWave;
     const int sub = lane % LPT;
     const int grp = lane / LPT;
-    for (int i = threadIdx.x; i < WPB * E; i += NT) s_hist[i] = 0;
-    __syncthreads();
-    // this wave's tokens: a contiguous range, TPW of them per pass; every wave of the grid makes
-    // the same number of passes (the block-wide barriers below sit inside the loop)
-    const int64_t w_begin = ((int64_t)blockIdx.x * WPB + wave) * tokens_per_wave;
-    int64_t w_end = w_begin + tokens_per_wave;
-    if (w_end > num_tokens) w_end = num_tokens;
     const int64_t passes = (tokens_per_wave + TPW - 1) / TPW;
     const float ninf = -__builtin_inff();
     // the scores of the next pass are fetched while this one is ranked (as long as registers allow)
@@ -231,7 +217,7 @@ __global__ __launch_bounds__(WPB * kWave) void topk_hist_kernel(const T* __restr
 #pragma unroll
         for (int v = 0; v < VPL; ++v) {
             const int e = v * LPT + sub;
-            if (live && e < E && rank[v] < K) s_sel[wave][grp][rank[v]] = my[v];
+            if (live && e < E && rank[v] < K) s_sel[grp][rank[v]] = my[v];
         }
         // gates of modes 2 and 3: softmax of the normalised logits over all experts (2) or over
         // the K selected ones (3)
@@ -239,7 +225,7 @@ __global__ __launch_bounds__(WPB * kWave) void topk_hist_kernel(const T* __restr
         wave_lds_fence();
         if (renorm == 2) {
             // the largest normalised logit is slot 0; exp(n_i - n_max) summed over all experts
-            const float nmax0 = live ? s_sel[wave][grp][0] : 0.0f;
+            const float nmax0 = live ? s_sel[grp][0] : 0.0f;
 #pragma unroll
             for (int v = 0; v < VPL; ++v) {
                 const int e = v * LPT + sub;
@@ -252,16 +238,16 @@ __global__ __launch_bounds__(WPB * kWave) void topk_hist_kernel(const T* __restr
             float denom = 1.0f;
             if (renorm == 1) {
                 float s = 0.0f;
-                for (int j = 0; j < K; ++j) s = s + fabsf(s_sel[wave][grp][j]);   // slot order
+                for (int j = 0; j < K; ++j) s = s + fabsf(s_sel[grp][j]);   // slot order
                 // (clamp_min keeps a NaN norm, fmaxf would drop it)
                 denom = s != s ? s : fmaxf(round_to<T>(s), round_to<T>(1e-12f));
             }
             float nmax = 0.0f;
             if (renorm >= 2) {
-                nmax = s_sel[wave][grp][0];
+                nmax = s_sel[grp][0];
                 if (renorm == 3) {
                     soft_sum = 0.0f;
-                    for (int j = 0; j < K; ++j) soft_sum += expf(s_sel[wave][grp][j] - nmax);
+                    for (int j = 0; j < K; ++j) soft_sum += expf(s_sel[grp][j] - nmax);
                 }
             }
 #pragma unroll
@@ -271,7 +257,7 @@ __global__ __launch_bounds__(WPB * kWave) void topk_hist_kernel(const T* __restr
                     const int64_t p = t * K + rank[v];
                     topk_idx[p] = e;
                     compact[p] = (uint16_t)e;
-                    atomicAdd(&s_hist[wave * E + e], 1);      // integer counts in LDS: exact
+                    atomicAdd(&s_hist[e], 1);      // integer counts in LDS: exact
                     float g = my[v];
                     if (renorm == 1) g = round_to<T>(my[v] / denom);
                     else if (renorm >= 2) g = round_to<T>(expf(my[v] - nmax) / soft_sum);
@@ -281,6 +267,28 @@ __global__ __launch_bounds__(WPB * kWave) void topk_hist_kernel(const T* __restr
         }
         wave_lds_fence();       // s_sel is rewritten by the next pass
     }
+}
+
+template <typename T, int LPT, int VPL, int WPB>
+__global__ __launch_bounds__(WPB * kWave) void topk_hist_kernel(const T* __restrict__ scores, int64_t num_tokens,
+                                                        int E, int K, int renorm, int64_t tokens_per_wave,
+                                                        int64_t* __restrict__ topk_idx,
+                                                        T* __restrict__ gates,
+                                                        uint16_t* __restrict__ compact,
+                                                        int32_t* __restrict__ sub_hist,
+                                                        int32_t* __restrict__ tot_hist) {
+    constexpr int NT = WPB * kWave;
+    __shared__ float s_sel[WPB][kWave / LPT][64];     // selected scores by slot (K <= 64)
+    extern __shared__ int32_t s_hist[];       // [WPB][E] experts chosen by this wave's tokens
+    const int wave = threadIdx.x / kWave;
+    for (int i = threadIdx.x; i < WPB * E; i += NT) s_hist[i] = 0;
+    __syncthreads();
+    // this wave's tokens: a contiguous range
+    const int64_t w_begin = ((int64_t)blockIdx.x * WPB + wave) * tokens_per_wave;
+    int64_t w_end = w_begin + tokens_per_wave;
+    if (w_end > num_tokens) w_end = num_tokens;
+    select_experts<T, LPT, VPL>(scores, w_begin, w_end, tokens_per_wave, E, K, renorm, topk_idx, gates, compact, s_sel[wave],
+                                s_hist + wave * E);
     __syncthreads();
     for (int i = threadIdx.x; i < WPB * E; i += NT) sub_hist[(int64_t)blockIdx.x * WPB * E + i] = s_hist[i];
     for (int e = threadIdx.x; e < E; e += NT) {
@@ -333,11 +341,58 @@ __global__ __launch_bounds__(1024) void compact_hist_kernel(const int64_t* __res
     }
 }
 
+// Places the positions of a wave's tokens [t_begin, t_end): next[e] (LDS, this wave's) is the next free slot of expert e.  Each pass
+// takes TPI = 64/K whole tokens, lane i <-> position begin + pass*TPI*K + i, so the K slots of a token sit in one pass.
+__device__ __forceinline__ void place_positions(const uint16_t* compact, int64_t t_begin, int64_t t_end,
+                                                int64_t tokens_per_wave, int K, int ebits, int32_t* next,
+                                                int64_t* __restrict__ gate_index, int64_t* __restrict__ token_index,
+                                                int64_t* __restrict__ reverse_index) {
+    const int lane = lane_id();
+    const int tpi = kWave / K;
+    const int64_t passes = (tokens_per_wave + tpi - 1) / tpi;
+    const int tok_in_iter = lane / K;
+    const int slot = lane - tok_in_iter * K;
+    const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    for (int64_t pass = 0; pass < passes; ++pass) {
+        const int64_t t = t_begin + pass * tpi + tok_in_iter;
+        const bool live = tok_in_iter < tpi && t < t_end;
+        const int64_t p = t * K + slot;
+        const uint32_t e = live ? compact[p] : (uint32_t)kBadExpert;
+        const bool counted = live && e != kBadExpert;
+        // lanes holding the same expert id
+        uint64_t same = __ballot(counted);
+        for (int b = 0; b < ebits; ++b) {
+            const uint64_t bal = __ballot((e >> b) & 1u);
+            same &= ((e >> b) & 1u) ? bal : ~bal;
+        }
+        const int before = __popcll(same & lt_mask);
+        const int count = __popcll(same);
+        int32_t base = 0;
+        if (counted) base = next[e];
+        wave_lds_fence();
+        if (counted && before == 0) next[e] = base + count;
+        wave_lds_fence();
+        const int64_t dst = (int64_t)base + before;
+        // rank of this slot among the token's K slots, ordered by (expert, slot)
+        int rank = 0;
+        for (int j = 0; j < K; ++j) {
+            const uint32_t oe = __shfl(e, tok_in_iter * K + j, kWave);
+            rank += (oe < e || (oe == e && j < slot)) ? 1 : 0;
+        }
+        if (counted) {
+            gate_index[dst] = p;
+            token_index[dst] = t;
+            reverse_index[t * K + rank] = dst;
+        } else if (live) {
+            reverse_index[t * K + rank] = 0;    // a dropped position (out-of-range id): sorts last in its token
+        }
+    }
+}
+
 // Block = chunk, 4 or 16 waves.  Phase 1: per expert, the rows of all chunks (lengths) and of the chunks
 // before this one.  Phase 2: wave scan over the experts = offsets.  Phase 3: every wave starts
 // from offsets + rows of earlier chunks + rows of the earlier waves of its chunk and places its
-// positions.  Each pass takes TPI = 64/K whole tokens, lane i <-> position begin + pass*TPI*K + i,
-// so the K slots of a token sit in one pass.  s_next[e] is the next free slot of expert e.
+// positions.
 __global__ __launch_bounds__(1024) void scan_scatter_kernel(const uint16_t* __restrict__ compact,
                                                            int64_t num_tokens, int64_t tokens_per_wave,
                                                            int E, int K, int ebits, int num_chunks,
@@ -438,49 +493,61 @@ __global__ __launch_bounds__(1024) void scan_scatter_kernel(const uint16_t* __re
         if (e < E) s_next[wave * E + e] = at[i];
     }
     __syncthreads();
-    int32_t* next = s_next + wave * E;
-    const int tpi = kWave / K;
     const int64_t t_begin = ((int64_t)c * WPB + wave) * tokens_per_wave;
     int64_t t_end = t_begin + tokens_per_wave;
     if (t_end > num_tokens) t_end = num_tokens;
-    const int64_t passes = (tokens_per_wave + tpi - 1) / tpi;     // the same for every wave (barriers below)
-    const int tok_in_iter = lane / K;
-    const int slot = lane - tok_in_iter * K;
-    const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    for (int64_t pass = 0; pass < passes; ++pass) {
-        const int64_t t = t_begin + pass * tpi + tok_in_iter;
-        const bool live = tok_in_iter < tpi && t < t_end;
-        const int64_t p = t * K + slot;
-        const uint32_t e = live ? compact[p] : (uint32_t)kBadExpert;
-        const bool counted = live && e != kBadExpert;
-        // lanes holding the same expert id
-        uint64_t same = __ballot(counted);
-        for (int b = 0; b < ebits; ++b) {
-            const uint64_t bal = __ballot((e >> b) & 1u);
-            same &= ((e >> b) & 1u) ? bal : ~bal;
+    place_positions(compact, t_begin, t_end, tokens_per_wave, K, ebits, s_next + wave * E, gate_index, token_index, reverse_index);
+}
+
+// Both launches in one block of 16 waves for a batch of few tokens (route_one_block): the counts and the expert ids stay in LDS, and
+// one barrier on either side of the prefix sums takes the place of the second launch.
+template <typename T, int LPT, int VPL>
+__global__ __launch_bounds__(kMaxRouteWaves* kWave) void route_block_kernel(const T* __restrict__ scores, int num_tokens, int E, int K,
+                                                                    int ebits, int renorm, int tokens_per_wave,
+                                                                    int64_t* __restrict__ topk_idx, T* __restrict__ gates,
+                                                                    int64_t* __restrict__ lengths, int64_t* __restrict__ offsets,
+                                                                    int64_t* __restrict__ gate_index,
+                                                                    int64_t* __restrict__ token_index,
+                                                                    int64_t* __restrict__ reverse_index) {
+    constexpr int WPB = kMaxRouteWaves, NT = WPB * kWave;
+    __shared__ float s_sel[WPB][kWave / LPT][64];
+    extern __shared__ int32_t s_hist[];       // [WPB][E] counts per wave, then every wave's next free slots
+    uint16_t* s_ids = reinterpret_cast<uint16_t*>(s_hist + WPB * E);     // [T * K]
+    const int lane = lane_id();
+    const int wave = threadIdx.x / kWave;
+    for (int i = threadIdx.x; i < WPB * E; i += NT) s_hist[i] = 0;
+    __syncthreads();
+    const int t_begin = wave * tokens_per_wave;
+    const int t_end = t_begin + tokens_per_wave < num_tokens ? t_begin + tokens_per_wave : num_tokens;
+    select_experts<T, LPT, VPL>(scores, t_begin, t_end, tokens_per_wave, E, K, renorm, topk_idx, gates, s_ids, s_sel[wave],
+                                s_hist + wave * E);
+    __syncthreads();
+    if (wave == 0) {
+        int run = 0;
+        for (int e0 = 0; e0 < E; e0 += kWave) {
+            const int e = e0 + lane;
+            int count[WPB], len = 0;
+#pragma unroll
+            for (int w = 0; w < WPB; ++w) count[w] = e < E ? s_hist[w * E + e] : 0;
+#pragma unroll
+            for (int w = 0; w < WPB; ++w) len += count[w];
+            const int inc = wave_inclusive_scan(len);
+            if (e < E) {
+                int at = run + inc - len;
+                lengths[e] = len;
+                offsets[e] = at;
+#pragma unroll
+                for (int w = 0; w < WPB; ++w) {
+                    s_hist[w * E + e] = at;
+                    at += count[w];
+                }
+            }
+            run += wave_bcast(inc, kWave - 1);
         }
-        const int before = __popcll(same & lt_mask);
-        const int count = __popcll(same);
-        int32_t base = 0;
-        if (counted) base = next[e];
-        wave_lds_fence();
-        if (counted && before == 0) next[e] = base + count;
-        wave_lds_fence();
-        const int64_t dst = (int64_t)base + before;
-        // rank of this slot among the token's K slots, ordered by (expert, slot)
-        int rank = 0;
-        for (int j = 0; j < K; ++j) {
-            const uint32_t oe = __shfl(e, tok_in_iter * K + j, kWave);
-            rank += (oe < e || (oe == e && j < slot)) ? 1 : 0;
-        }
-        if (counted) {
-            gate_index[dst] = p;
-            token_index[dst] = t;
-            reverse_index[t * K + rank] = dst;
-        } else if (live) {
-            reverse_index[t * K + rank] = 0;    // a dropped position (out-of-range id): sorts last in its token
-        }
+        if (lane == 0) offsets[E] = run;
     }
+    __syncthreads();
+    place_positions(s_ids, t_begin, t_end, tokens_per_wave, K, ebits, s_hist + wave * E, gate_index, token_index, reverse_index);
 }
 
 int ceil_log2(int v) {
@@ -511,6 +578,41 @@ void launch_topk(const void* scores, int64_t T_, int E, int K, int renorm, int64
         topk_hist_kernel<T, LPT, VPL, 4><<<plan.num_chunks, 4 * kWave, lds, stream>>>(
             (const T*)scores, T_, E, K, renorm, plan.tokens_per_wave, topk_idx, (T*)gates, ws.compact, ws.sub_hist,
             ws.tot_hist);
+}
+
+// One block takes the batch where its 16 waves rank all tokens in one pass (two: up to 64 experts and 8 slots), so that the second
+// launch is what it saves.  us, two launches / one block: 64 tokens, 8 experts, top-2 8.9 / 5.0; 256, top-8 11.0 / 9.5; 64 tokens, 32
+// experts, top-2 9.4 / 5.5; 128, 64 experts, top-8 12.7 / 12.5; 64, 128 experts, top-8 16.7 / 12.1; 64, 256 experts 27.5 / 22.8.  One pass
+// more: 384 tokens, 8 experts, top-8 10.9 / 12.4; 192, 64 experts, top-8 13.0 / 17.4; 100, 128 experts, top-8 16.9 / 18.1.  Beyond
+// 16 slots a wave of the block places its four tokens one after the other.
+inline bool route_one_block(int64_t T, int E, int K) {
+    const int64_t pass = kMaxRouteWaves * (E <= 8 ? 8 : 4);
+    return E <= 256 && K <= 16 && T <= (E <= 64 && K <= 8 ? 2 * pass : pass);
+}
+
+struct RouteOut {
+    int64_t *topk_idx, *lengths, *offsets, *gate_index, *token_index, *reverse_index;
+};
+
+template <typename T, int LPT, int VPL>
+void launch_one_block(const void* scores, int64_t T_, int E, int K, int renorm, void* gates, const RouteOut& out, hipStream_t stream) {
+    const size_t lds = (size_t)kMaxRouteWaves * E * sizeof(int32_t) + (size_t)T_ * K * sizeof(uint16_t);
+    route_block_kernel<T, LPT, VPL><<<1, kMaxRouteWaves * kWave, lds, stream>>>(
+        (const T*)scores, (int)T_, E, K, ceil_log2(E), renorm, (int)((T_ + kMaxRouteWaves - 1) / kMaxRouteWaves), out.topk_idx,
+        (T*)gates, out.lengths, out.offsets, out.gate_index, out.token_index, out.reverse_index);
+}
+
+template <typename T>
+int dispatch_one_block(const void* scores, int64_t T_, int E, int K, int renorm, void* gates, const RouteOut& out, hipStream_t stream) {
+#define FMOE_ROUTE(LPT, VPL) launch_one_block<T, LPT, VPL>(scores, T_, E, K, renorm, gates, out, stream)
+    if (E <= 8) FMOE_ROUTE(8, 1);
+    else if (E <= 16) FMOE_ROUTE(16, 1);
+    else if (E <= 32) FMOE_ROUTE(16, 2);
+    else if (E <= 64) FMOE_ROUTE(16, 4);
+    else if (E <= 128) FMOE_ROUTE(16, 8);
+    else FMOE_ROUTE(16, 16);
+#undef FMOE_ROUTE
+    return check_launch("routing");
 }
 
 template <typename T>
@@ -576,6 +678,11 @@ static int route_topk_impl(const char* who, const void* scores, int score_dtype,
     }
     FMOE_REQUIRE(scores && topk_idx && gates && gate_index && token_index && reverse_index,
                  "%s: NULL tensor pointer", who);
+    if (route_one_block(T, E, K)) {
+        const RouteOut out = {topk_idx, lengths, offsets, gate_index, token_index, reverse_index};
+        return score_dtype == FMOE_F32 ? dispatch_one_block<float>(scores, T, E, K, renorm, gates, out, stream)
+                                       : dispatch_one_block<uint16_t>(scores, T, E, K, renorm, gates, out, stream);
+    }
     const RoutePlan plan = make_plan(T, E, K);
     const RouteScratch ws = carve(workspace, plan);
     int rc = score_dtype == FMOE_F32

@@ -39,6 +39,23 @@ def test_route_topk_matches_oracle(dtype, T, E, K):
     check_route(softmax_scores(T, E, T * 7 + E + K, dtype), K)
 
 
+@pytest.mark.parametrize("mode", [True, 2, 3])
+@pytest.mark.parametrize("E,K", [(8, 8), (9, 8), (9, 9), (64, 3), (65, 8), (256, 16), (257, 16), (256, 17)])
+def test_route_topk_one_block_and_beyond(E, K, mode):
+    """Batches around the largest that one block takes (64, 128 and 256 tokens, by E and K): every token is routed on its own, so a
+    batch's first T tokens get the ids and gates they get in a batch of 1000 (two launches), and the permutation follows from them."""
+    from fast_moe_amd.kernels.hip import ops
+    scores = softmax_scores(1000, E, E + K, torch.float32).cuda()
+    whole = ops.route_topk(scores, K, renorm=mode)
+    for T in (1, 15, 63, 64, 65, 127, 128, 129, 255, 256, 257):
+        got = ops.route_topk(scores[:T].contiguous(), K, renorm=mode)
+        for key in ("topk_idx", "gates"):
+            assert torch.equal(got[key], whole[key][:T]), (key, T)
+        ref = ops.route_from_topk(got["topk_idx"], E)
+        for key in ("lengths", "offsets", "gate_index", "token_index", "reverse_index"):
+            assert torch.equal(got[key].view(-1), ref[key].view(-1)), (key, T)
+
+
 def test_route_topk_ties_and_no_renorm():
     # bf16 softmax over many experts: plenty of exactly equal scores
     scores = softmax_scores(512, 64, 3, torch.bfloat16, temp=0.3)
