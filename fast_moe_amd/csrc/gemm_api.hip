@@ -163,7 +163,7 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
                         (d->a_stride_e % chunk) == 0 && (d->b_stride_k % chunk) == 0 && (d->b_stride_e % chunk) == 0;
     // rows per expert decide the tile height: tall tiles for prefill-like loads,
     // short ones when the experts see a handful of rows (weight-streaming regime)
-    const bool big = d->total_rows / d->num_experts >= 96;
+    const bool big = d->total_rows / d->num_experts >= kTallRows;
     // the ring kernel moves whole 64-byte K-slices by LDS-DMA and stores 16-byte groups
     const int slice = 64 / esize;
     // ... and addresses rows as a 64-bit base per expert plus a 32-bit byte offset
@@ -200,7 +200,8 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
                           (d->a_stride_e % chunk) == 0 && aligned16(d->a) && aligned16(d->b) &&
                           (!swiglu || aligned16(d->b2)) && near_tr;
     p.ring_short = short_tr || (short_ok && near && (fast8 || (fast && ring_short_pays(p, esize, d->epilogue))));
-    p.direct = fast && !big && !(d->a_silu && d->epilogue != FMOE_EPI_NONE) && !d->k_window && !two && !row_indexed && !gated && direct_pays(p, esize, swiglu);
+    p.direct = fast && !(d->a_silu && d->epilogue != FMOE_EPI_NONE) && !d->k_window && !two && !row_indexed && !gated &&
+               direct_pays(p, esize, swiglu);
     // the second product exists in that kernel only; a caller that is turned away runs two
     // GEMMs and adds
     if (two)

@@ -192,6 +192,9 @@ inline bool ring_short_pays(const GemmParams& p, int esize, int epilogue) {
            (p.total_rows + TileRingS::BM - 1) / TileRingS::BM * n_tiles > 2 * cus;
 }
 
+// rows per expert, on average, from which the tall tiles (256 rows) are the rule
+constexpr int kTallRows = 96;
+
 // The streaming kernels that take the weights straight into registers (gemm_direct.hip).
 int run_gemm_direct(const GemmParams& p, int dtype, int epilogue, bool a_silu, hipStream_t stream);
 
@@ -202,26 +205,40 @@ inline int64_t most_row_tiles(int64_t rows, int64_t num_experts, int bm) {
 }
 inline int direct_columns(int n, bool swiglu) { return swiglu ? (n + 31) / 32 : (n + 63) / 64; }
 
-// Where they are taken (weights with k contiguous, 16-byte loads, no gate), up to 16 rows per expert on average.  us per GEMM, the
-// kernel that ran before (the 64-row ring, the streaming or the register-staged kernel) / this one; even load unless said:
-//   * no more tiles than CUs: the tile that others walk alone (64 x 256, K serial) is a quarter as wide and its K is shared by eight
-//     waves.  24 rows, 10 experts, 2112 -> 408 18.3 / 11.4 (e4m3 14.9 / 6.8, fp32 56.1 / 20.5); 5 rows, 35 experts, 2696 -> 1024
-//     32.2 / 10.4 (fp32 72.2 / 21.5); 64 rows, 4 experts, 4096 -> 4096 33.3 / 24.7; 128 rows, 8 experts, 128 -> 256 8.2 / 6.3; 160 rows, 10
-//     experts, 1024 -> 1024 12.0 / 8.9, Zipf 11.9 / 11.5
-//   * up to two per CU: e4m3, and rows of K up to 1664 bytes.  98 rows, 11 experts, 2496 -> 2 x 832 bf16 23.4 / 25.6 (not taken), e4m3
-//     19.0 / 13.3; 98 rows, 11 experts, 832 -> 2496 bf16 12.5 / 11.7
+// Where they are taken (weights with k contiguous, 16-byte loads, no gate).  us per GEMM, the kernel that ran before (the 64-row or the tall
+// ring, the streaming or the register-staged kernel) / this one; even load unless said:
+//   * no more tiles than CUs, whatever the rows (beyond 16 per expert on average from rows of K of 513 bytes on, from 96 per expert on of 2
+//     KB: the chain that is shared out is short below, 3 us are left to gain: 2000 rows, 4 experts, 128 -> 256 8.7 / 5.6): the tile that others walk alone (64 x 256 or 256 x 256, K serial) is a quarter as wide or
+//     less and its K is shared by eight waves.  24 rows, 10 experts, 2112 -> 408 18.3 / 11.4 (e4m3 14.9 / 6.8, fp32 56.1 / 20.5); 5 rows, 35
+//     experts, 2696 -> 1024 32.2 / 10.4 (fp32 72.2 / 21.5); 64 rows, 4 experts, 4096 -> 4096 33.3 / 24.7; 160 rows, 10
+//     experts, 1024 -> 1024 12.0 / 8.9, Zipf 11.9 / 11.5; 207 rows, 4 experts, 1088 -> 1152 13.2 / 11.7; 256 rows, 4 experts, 4096 -> 1024 32.1 /
+//     32.2, one hot expert 31.3 / 32.0; 3000 rows, 4 experts, 1024 -> 320 22.7 / 11.6 (e4m3 16.1 /
+//     8.6), 4096 -> 320 69.3 / 33.5; 766 rows, 6 experts, 3904 -> 640 65.3 / 31.4; fp32 320 rows, 8 experts, 1024 -> 512 30.6 / 15.8
+//   * up to two per CU: e4m3, and rows of K up to 1664 bytes, with up to 16 rows per expert on average.  98 rows, 11 experts, 2496 -> 2 x
+//     832 bf16 23.4 / 25.6 (not taken), e4m3 19.0 / 13.3; 98 rows, 11 experts, 832 -> 2496 bf16 12.5 / 11.7.  With more rows the 64-row
+//     ring is ahead (500 rows, 8 experts, 2048 -> 2 x 1024 bf16 21.0 / 32.5, e4m3 14.8 / 20.3) until the tall ring's are the tiles, which
+//     then are a sixteenth as many: 1000 rows, 8 experts, 2048 -> 2 x 512 39.6 / 33.0 (e4m3 26.0 / 20.0); 1000 rows, 4 experts, 1024 -> 1024
+//     22.5 / 12.2; 2000 rows, 8 experts, 4096 -> 512 69.4 / 60.5.  Three: 2000 rows, 8 experts, 4096 -> 1024 70.2 / 88.8.
 //   * beyond, an even load would gain (512 rows, 128 experts, 4096 -> 2 x 1536 543 / 529, e4m3 286 / 264), but an expert with many rows
 //     has its weights read from L2 for every 64 of them and every 32 columns: 1024 rows, Zipf 488 / 606.
 //   * fp32 streams half as much weight for a product and the other kernel is the slower one: 512 rows, 128 experts, 4096 -> 2 x 1536
 //     1475 / 1066, Zipf 1011 / 844, nine tenths in one expert 653 / 543.  Not with short K and rows enough for a hot expert (400 rows,
-//     24 experts, 896 -> 2192: even 48.5 / 46.0, one hot expert 48.8 / 56.6), nor with K of two slices (gemm_f32.hip).
+//     24 experts, 896 -> 2192: even 48.5 / 46.0, one hot expert 48.8 / 56.6), nor with K of two slices (gemm_f32.hip).  With more than 16
+//     rows per expert the other kernel's tiles hold more of them: K from 1024 on and one tile per CU only (2048 rows, 8 experts, 256 ->
+//     256 10.7 / 13.3; 4000 rows, 8 experts, 4096 -> 512, four per CU, 162 / 218).
 // Calls of up to three rows belong to the 64-row ring by the tests of the rule before this one.
 inline bool direct_pays(const GemmParams& p, int esize, bool swiglu) {
     const int64_t experts = p.E < p.total_rows ? p.E : p.total_rows, cus = compute_units();
-    if (p.total_rows < 4 || p.total_rows > 16 * experts) return false;
+    if (p.total_rows < 4) return false;
     const int64_t tiles = most_row_tiles(p.total_rows, p.E, 64) * direct_columns(p.N, swiglu);
-    if (esize == 4) return p.K > 64 && (p.K >= 1024 || tiles <= 2 * cus || p.total_rows <= 4 * experts);
-    return tiles <= cus || (tiles <= 2 * cus && (esize == 1 || p.K * esize <= 1664));
+    const bool few = p.total_rows <= 16 * experts, tall = p.total_rows / p.E >= kTallRows;
+    if (esize == 4) {
+        if (!few) return p.K >= 1024 && tiles <= cus;
+        return p.K > 64 && (p.K >= 1024 || tiles <= 2 * cus || p.total_rows <= 4 * experts);
+    }
+    const int row = p.K * esize;
+    if (few) return tiles <= cus || (tiles <= 2 * cus && (esize == 1 || row <= 1664));
+    return tall ? row >= 2048 && tiles <= 2 * cus : row > 512 && tiles <= cus;
 }
 
 // The 5-slot ring needs every byte of a 160 KB LDS, an even number of K-slices per tile,

@@ -1225,6 +1225,7 @@ def test_fp32_kernel_for_short_k(K, new):
     ([1] * 70 + [0, 9], 104, 132, 0), ([4, 0] * 80, 136, 72, 1),        # more experts than lanes
     ([5] * 11, 800, 2900, 0), ([3] * 20, 824, 1096, "silu"),           # more tiles than CUs
     ([7, 0, 20, 8], 1048, 200, "silu"),
+    ([65, 0, 129, 255, 1], 2056, 72, 0), ([300, 40, 0, 320], 2064, 296, 2),     # rows enough for taller tiles, but few of them
 ])
 @pytest.mark.parametrize("dtype", ["bf16", "fp8", "f32"])
 @pytest.mark.parametrize("extras", [False, True])
@@ -1312,7 +1313,10 @@ def test_streaming_kernel_recomputes_fp32_sums_that_are_not_finite():
 @pytest.mark.parametrize("E,rows,K,N,dtype,direct", [
     (16, 16, 1664, 1024, "bf16", True), (16, 16, 1664, 1024 + 1, "bf16", False),        # one tile per CU; K of more than 1664 bytes beyond
     (16, 16, 832, 2048, "bf16", True), (16, 16, 832, 2049, "bf16", False), (16, 16, 2048, 2048, "fp8", True), (16, 16, 2048, 2049, "fp8", False),
-    (16, 256, 1664, 1024, "bf16", False), (16, 250, 832, 64, "bf16", True), (4, 65, 832, 64, "bf16", False),
+    (16, 256, 1664, 1024, "bf16", False), (16, 250, 832, 64, "bf16", True), (4, 65, 832, 64, "bf16", True),
+    (4, 80, 256, 64, "bf16", False), (4, 80, 264, 64, "bf16", True), (4, 4096, 1024, 240, "bf16", True), (4, 4096, 1016, 240, "bf16", False),
+    (4, 800, 1024, 2048, "bf16", True), (4, 800, 1024, 2056, "bf16", False), (4, 800, 2048, 2048, "fp8", True), (4, 800, 2048, 2064, "fp8", False),
+    (4, 380, 1024, 2048, "bf16", False), (4, 300, 1024, 512, "f32", True), (4, 300, 1020, 512, "f32", False),
     (16, 100, 1020, 2049, "f32", False), (16, 64, 1020, 2049, "f32", True), (16, 100, 1024, 2049, "f32", True), (16, 16, 64, 64, "f32", False),
 ])
 def test_streaming_kernel_choice(E, rows, K, N, dtype, direct):
