@@ -26,6 +26,7 @@
 //       to A on load, fp32 operands of few k (on tiles of their own, gemm_f32.hip).
 //   grouped_gemm_f32x3_kernel  fp32 operands otherwise: register-staged too, every value cut into three
 //       bf16 parts on its way into LDS (gemm_f32x3.h).
+//   grouped_wgrad_kernel       weight gradients of experts with few rows (gemm_wgrad.h).
 //
 // e4m3 row-wise scales that are exact powers of two (GemmParams::scale_pow2) are handed to
 // v_mfma_scale_f32_32x32x64_f8f6f4 as E8M0 codes of their reciprocals instead of being divided
@@ -51,7 +52,7 @@
 //     XCD one contiguous range of the tile order.
 //
 // Files: gemm_params.h (launch parameters, helpers), gemm_epilogue.h, gemm_ring.h, gemm_stream.h,
-// gemm_staged.h, gemm_f32x3.h, gemm_direct.h (the kernels), gemm_launch.h (kernel choice and launches).
+// gemm_staged.h, gemm_f32x3.h, gemm_direct.h, gemm_wgrad.h (the kernels), gemm_launch.h (kernel choice and launches).
 #pragma once
 
 #include "gemm_launch.h"

@@ -428,6 +428,36 @@ def test_weight_gradient_from_rows_in_place(lens):
     assert torch.equal(out2, out)
 
 
+@pytest.mark.parametrize("lens,N,Kin,halves,few", [
+    ([0, 1, 31, 32, 33, 63, 64, 65, 16, 0], 128, 128, False, True),
+    ([3] * 43, 8, 8, False, True), ([5, 200, 0, 11], 136, 648, False, True),        # a row tile and a column tile in part
+    ([130, 0, 2], 64, 120, True, True), ([50, 78, 99], 192, 264, True, True),        # both halves in one tile of 128 rows
+    ([300] * 9 + [1, 0, 4], 264, 392, False, True), ([70, 0, 64, 126] * 40, 520, 1032, False, False),
+    ([64] * 70, 1544, 1400, False, True), ([65] * 70, 1544, 1400, False, False),      # strips of column tiles, the last in part
+    ([900, 0, 513, 130, 1, 300, 64, 77], 1032, 1544, False, False), ([900, 0, 513, 130, 1, 300, 64, 77], 1088, 1544, True, False),
+])
+def test_weight_gradient_of_few_rows(lens, N, Kin, halves, few):
+    """The kernel for short contractions and small matrices, and its neighbours on the ring: against fp64, with the roundings of an fp32 sum
+    over the longest expert's rows (2^-24 each) and of the bf16 result (8 significant bits: 2^-8 at most); rows behind the last expert are NaN."""
+    from fast_moe_amd.kernels.hip import ops
+    from helpers import kernels_run
+    E, R = len(lens), sum(lens)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    offsets = torch.tensor([0, *torch.tensor(lens).cumsum(0)]).cuda()
+    x, d = (ops.empty_rows(R, n, BF16, "cuda") for n in (Kin, N))
+    for t in (x, d):
+        t.copy_(torch.randn(t.shape, generator=g, device="cuda"))
+        torch.as_strided(t, (ops.SLACK_ROWS, t.shape[1]), (t.shape[1], 1), R * t.shape[1]).fill_(float("nan"))
+    out = ops.jagged_weight_grad(d, x, offsets, halves=halves)
+    ran = kernels_run(lambda: ops.jagged_weight_grad(d, x, offsets, halves=halves))[-1]
+    assert ("grouped_wgrad_kernel" in ran) == few, ran
+    out = torch.cat(out, dim=1) if halves else out
+    for e in range(E):
+        a, b = d[offsets[e]:offsets[e + 1]].double(), x[offsets[e]:offsets[e + 1]].double()
+        want, bound = a.t() @ b, 2.0 ** -24 * max(1, max(lens)) * (a.abs().t() @ b.abs())
+        assert bool(((out[e].double() - want).abs() <= bound + 2.0 ** -8 * (want.abs() + bound)).all()), e
+
+
 @pytest.mark.parametrize("lens,K1,K2,N", [
     ([300, 0, 1000, 128, 77, 515], 256, 256, 256),
     ([4096, 640], 384, 384, 520),
