@@ -262,12 +262,15 @@ __global__ __launch_bounds__(256) void quant_rows_generic_lane(
 // quantisation, tile by tile.  Bound by HBM: the operand is read twice (the second time mostly from the
 // last-level cache where it fits) and its bytes written once.  A lane per row, the form this replaces,
 // kept rows / 64 waves in flight, each with a serial walk over its columns and one-byte stores a row apart:
-// 8 x 1024 x 4096 took 751 us (N = 4096) and 3147 us (N = 1024); the two launches take 15 + 19 us on both (67 MB
-// read at 4.5 TB/s; 67 MB read, half of it written, at 5.3 TB/s).
+// 8 x 1024 x 4096 took 751 us (N = 4096) and 3147 us (N = 1024).
+// Columns that fit a block's registers (kColOneMost) take one launch that reads them once.  us, two launches / one: 8 x 1024 x
+// 4096 30.3 / 21.7 (100 MB, 15.7 at copy speed), 8 x 4096 x 1024 32.9 / 23.9; 64 x 2048 x 1408 173 / 120, 64 x 1408 x 2048 191 / 120; 128 x
+// 4096 x 1536 804 / 568, 128 x 1536 x 4096 785 / 450; 100 x 200 x 1024 27.7 / 17.9; 4 x 512 x 512 7.0 / 6.1; 4 x 4096 x 64 19.9 / 11.6.
 
 constexpr int kColTileN = 64;       // rows of the result per block: 128 bytes of a memory row
 constexpr int kColTileK = 128;      // columns per block of the second launch: a whole line of result bytes
 constexpr int kColMaxSplit = 64;
+constexpr int64_t kColOneMost = 4096;
 
 // Blocks of the first launch along the columns: enough to fill the chip (4 per CU), at least 64 columns each.
 inline int col_splits(int64_t batch, int64_t rows, int64_t cols) {
@@ -394,6 +397,108 @@ __global__ __launch_bounds__(256) void quant_cols_store(const uint16_t* __restri
 #pragma unroll
             for (int d = 0; d < 4; ++d)
                 if (k0 + 4 * (c + d) < cols) *reinterpret_cast<uint32_t*>(dst + 4 * d) = t[d];     // (cols % 4 == 0)
+        }
+    }
+}
+
+// Both launches in one for columns that fit a block's registers: block (strip of STRIP rows, batch) holds PASSES x 4 x NT / (STRIP / 8)
+// columns, 16 bytes of four consecutive columns per lane and pass; the amax meets in LDS, and every pass leaves through the
+// transposing tile.  Two blocks and more to a CU where the registers allow, so that one loads under the other's stores; narrow strips
+// for that (8 x 3000 x 3000: 32 rows, one block of 1024 threads 92 us, 512 threads of 96 registers 67), and neighbours on one XCD, which
+// share the 128-byte lines then (64-row strips dealt round-robin 8 x 4096 x 1024 32, 128 x 4096 x 1536 760; now 24 and 568).
+template <int STRIP, int NT, int PASSES>
+__global__ __launch_bounds__(NT, 4) void quant_cols_one(const uint16_t* __restrict__ a, int64_t rows, int64_t cols, int64_t a_sb,
+                                                     int64_t a_sc, uint8_t* __restrict__ q, int64_t q_sb, int64_t q_sr,
+                                                     float* __restrict__ scale, int store_reciprocal, int wide, int strips) {
+    constexpr int LPR = STRIP / 8, QUADS = NT / LPR, PASS = 4 * QUADS;      // lanes across the strip, groups of 4 columns in a pass
+    // (lanes of a wave store rows 8 * ng + j, dwords q .. of the tile: 8 * DW * ng + q has to name 64 banks)
+    constexpr int DW = QUADS + 64 / LPR / 8;
+    static_assert((8 * (DW % 64)) % 64 == 64 / LPR, "tile rows");
+    constexpr int NW = NT / kWave;
+    __shared__ uint32_t tile[STRIP * DW];
+    __shared__ uint32_t s_max[NW][STRIP];
+    __shared__ float s_scale[STRIP];
+    __shared__ int s_special;
+    const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+    const int ng = tid % LPR, quad = tid / LPR;
+    // neighbouring strips share lines: a run of them to every XCD
+    const int strip = gridDim.x > 8 ? (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8) : (int)blockIdx.x;
+    if (strip >= strips) return;
+    const int64_t n0 = (int64_t)strip * STRIP, n = n0 + 8 * ng;
+    const uint16_t* const src = a + blockIdx.y * a_sb + n;
+    u32x4 v[PASSES][4];
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+        const int64_t k = p * PASS + 4 * quad;              // (columns come in fours)
+        const bool in = n < rows && k < cols;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[p][i] = in ? *reinterpret_cast<const u32x4*>(src + (k + i) * a_sc) : u32x4{0, 0, 0, 0};
+    }
+    if (tid == 0) s_special = 0;
+    uint32_t m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) amax_bits(v[p][i][j], m[2 * j], m[2 * j + 1]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+#pragma unroll
+        for (int o = LPR; o < kWave; o <<= 1) m[j] = max(m[j], (uint32_t)__shfl_xor((int)m[j], o, kWave));
+        if (lane < LPR) s_max[wave][lane * 8 + j] = m[j];
+    }
+    __syncthreads();
+    if (tid < STRIP) {
+        uint32_t bits = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) bits = max(bits, s_max[w][tid]);
+        const float s = scale_from_amax<true>(__uint_as_float(bits));
+        s_scale[tid] = s;
+        if (bits >= 0x7f800000u) s_special = 1;
+        if (n0 + tid < rows) scale[blockIdx.y * rows + n0 + tid] = store_reciprocal ? 1.0f / s : s;
+    }
+    __syncthreads();
+    const bool special = s_special != 0;
+    float sc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sc[j] = s_scale[8 * ng + j];
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+        if (p * PASS >= cols) break;
+        if (p) __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            float f[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                f[i] = ((j & 1) ? __uint_as_float(v[p][i][j / 2] & 0xffff0000u) : bf16_bits_to_f32(v[p][i][j / 2] & 0xffffu)) * sc[j];
+            uint32_t w;
+            if (!special) {
+                int t = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
+                w = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], t, true);
+            } else {
+                w = e4m3fn_encode(f[0]) | (e4m3fn_encode(f[1]) << 8) | (e4m3fn_encode(f[2]) << 16) | (e4m3fn_encode(f[3]) << 24);
+            }
+            tile[(8 * ng + j) * DW + quad] = w;
+        }
+        __syncthreads();
+        // rows out: QUADS / 4 lanes cover a pass's bytes of one, 16 each
+        constexpr int LANES = QUADS / 4;
+#pragma unroll
+        for (int i = 0; i < STRIP * LANES / NT; ++i) {
+            const int r = tid / LANES + i * (NT / LANES), c = 4 * (tid % LANES);
+            const int64_t k = p * PASS + 4 * c;
+            if (n0 + r >= rows) continue;
+            uint8_t* dst = q + blockIdx.y * q_sb + (n0 + r) * q_sr + k;
+            const uint32_t* t = tile + r * DW + c;
+            if (wide && k + 16 <= cols) {
+                *reinterpret_cast<u32x4*>(dst) = u32x4{t[0], t[1], t[2], t[3]};
+            } else {
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    if (k + 4 * d < cols) *reinterpret_cast<uint32_t*>(dst + 4 * d) = t[d];
+            }
         }
     }
 }
@@ -543,6 +648,23 @@ extern "C" int fmoe_quant_rows_e4m3_ws(const void* a, int a_dtype, int64_t batch
         return fmoe_quant_rows_e4m3(a, a_dtype, batch, rows, cols, a_sb, a_sr, a_sc, apply_silu, q, q_sb, q_sr, q_sc,
                                     scale, store_reciprocal, stream_);
     hipStream_t stream = (hipStream_t)stream_;
+    const int wide = (reinterpret_cast<uintptr_t>(q) & 15u) == 0 && q_sr % 16 == 0 && q_sb % 16 == 0;
+    if (cols <= kColOneMost) {
+        auto one = [&](auto kern, int strip, int threads) {
+            const int strips = (int)((rows + strip - 1) / strip);
+            kern<<<dim3((unsigned)(strips > 8 ? (strips + 7) / 8 * 8 : strips), (unsigned)batch), threads, 0, stream>>>(
+                (const uint16_t*)a, rows, cols, a_sb, a_sc, q, q_sb, q_sr, scale, store_reciprocal, wide, strips);
+            return check_launch("fmoe_quant_rows_e4m3_ws");
+        };
+        FMOE_REQUIRE((rows + 7) / 8 < ((int64_t)1 << 31) - 8, "fmoe_quant_rows_e4m3_ws: too many rows");
+        if (cols <= 256) return one(quant_cols_one<32, 256, 1>, 32, 256);
+        if (cols <= 512) return one(quant_cols_one<32, 256, 2>, 32, 256);
+        if (cols <= 1024) return one(quant_cols_one<64, 512, 4>, 64, 512);
+        if (cols <= 1536) return one(quant_cols_one<32, 512, 3>, 32, 512);
+        if (cols <= 2048) return one(quant_cols_one<32, 512, 4>, 32, 512);
+        if (cols <= 3072) return one(quant_cols_one<32, 512, 6>, 32, 512);
+        return one(quant_cols_one<32, 1024, 4>, 32, 1024);
+    }
     const int splits = col_splits(batch, rows, cols);
     const int64_t per_split = (cols + splits - 1) / splits;
     const int64_t strips = (rows + kColTileN - 1) / kColTileN;
@@ -550,7 +672,6 @@ extern "C" int fmoe_quant_rows_e4m3_ws(const void* a, int a_dtype, int64_t batch
     uint32_t* part = (uint32_t*)workspace;
     quant_cols_amax<<<dim3((unsigned)strips, (unsigned)splits, (unsigned)batch), 256, 0, stream>>>(
         (const uint16_t*)a, rows, cols, a_sb, a_sc, part, batch * rows, per_split);
-    const int wide = (reinterpret_cast<uintptr_t>(q) & 15u) == 0 && q_sr % 16 == 0 && q_sb % 16 == 0;
     quant_cols_store<<<dim3((unsigned)strips, (unsigned)((cols + kColTileK - 1) / kColTileK), (unsigned)batch), 256, 0,
                        stream>>>((const uint16_t*)a, rows, cols, a_sb, a_sc, part, splits, batch * rows, q, q_sb, q_sr,
                                  scale, store_reciprocal, wide);

@@ -242,6 +242,23 @@ def test_rows_that_are_columns_in_memory(E, K, N):
     assert np.array_equal((got & 0x7F) == 0x7F, nan) and np.array_equal(got[~nan], q_ref[~nan])
 
 
+@pytest.mark.parametrize("K", [44, 252, 256, 260, 512, 516, 1024, 1028, 1536, 1540, 2048, 2052, 3072, 3076, 4096])
+@pytest.mark.parametrize("E,N", [(1, 16), (2, 24), (1, 72), (3, 296), (2, 544)])
+def test_columns_that_fit_a_block(E, K, N):
+    """One launch for up to 4096 columns: every size of block and its remainders (strips of 32 and 64 rows, more and fewer than eight of
+    them), bit for bit what the row kernel gives for the transposed copy; matrices of a wider tensor; rows with inf, NaN and zeros."""
+    from fast_moe_amd.kernels import moe_fp8
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    w = torch.full((E, K + 3, N + 8), float("nan"), dtype=torch.bfloat16, device="cuda")[:, :K, :N]
+    w.copy_(torch.randn(E, K, N, generator=g, device="cuda") * torch.exp(torch.randn(E, 1, N, generator=g, device="cuda") * 4))
+    w[0, 0, 1], w[-1, K - 1, N - 1] = float("inf"), float("nan")
+    w[0, :, 0] = 0
+    q, s = moe_fp8.quantize_expert_weights(w)
+    q_ref, s_ref = moe_fp8.rowwise_quant_fp8(w.permute(0, 2, 1).contiguous())
+    assert torch.equal(s.view(torch.int32), s_ref.view(torch.int32))
+    assert torch.equal(q.permute(0, 2, 1).view(torch.uint8), q_ref.view(torch.uint8))
+
+
 def test_the_column_form_allocates_scratch_only_where_it_runs():
     """The two-launch form writes rows of consecutive bytes: a result laid out like its [E, K, N] input is left to the other
     kernel, without a scratch buffer."""
