@@ -39,8 +39,6 @@ __device__ __forceinline__ int wave_scan_dpp(int v) {
 struct BlockTile32 {
     int expert, nt, row0, rows_valid;
 
-    // DEAL: whole groups of row tiles to the XCDs in turn (BlockTile with a contraction window), else one range of tiles per XCD
-    template <bool DEAL = false>
     __device__ __forceinline__ bool locate(const GemmParams& p, int BM) {
         const int lane = threadIdx.x & 63, R = (int)p.total_rows;
         auto rows_of = [&](int e, int& lo) -> int {
@@ -56,21 +54,10 @@ struct BlockTile32 {
             inc = wave_scan_dpp((len + BM - 1) / BM);
             total_m += __builtin_amdgcn_readlane(inc, 63);
         }
-        const int slot = blockIdx.x / kNumXcd, span = kGroupM * p.n_tiles;
-        int group, within;
-        if constexpr (DEAL) {
-            const int round = slot / span;
-            group = round * kNumXcd + blockIdx.x % kNumXcd;
-            within = slot - round * span;
-            const int rest = total_m - group * kGroupM;
-            if (within >= (rest < kGroupM ? rest : kGroupM) * p.n_tiles) return false;
-        } else {
-            const int total = total_m * p.n_tiles, per_xcd = (total + kNumXcd - 1) / kNumXcd;
-            const int logical = blockIdx.x % kNumXcd * per_xcd + slot;
-            if (slot >= per_xcd || logical >= total) return false;
-            group = logical / span;
-            within = logical - group * span;
-        }
+        const int total = total_m * p.n_tiles, per_xcd = (total + kNumXcd - 1) / kNumXcd;
+        const int slot = blockIdx.x / kNumXcd, logical = blockIdx.x % kNumXcd * per_xcd + slot;
+        if (slot >= per_xcd || logical >= total) return false;
+        const int span = kGroupM * p.n_tiles, group = logical / span, within = logical - group * span;
         const int gsize = total_m - group * kGroupM < kGroupM ? total_m - group * kGroupM : kGroupM;
         const int mt = group * kGroupM + within % gsize;
         nt = within / gsize;

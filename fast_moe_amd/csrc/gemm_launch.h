@@ -241,21 +241,6 @@ inline bool direct_pays(const GemmParams& p, int esize, bool swiglu) {
     return tall ? row >= 2048 && tiles <= 2 * cus : row > 512 && tiles <= cus;
 }
 
-// Weight gradients of experts with few rows (gemm_wgrad.hip).
-int run_wgrad_short(GemmParams p, hipStream_t stream);
-
-// Where that kernel is taken: a short contraction, whose cost is the stores, and matrices that leave the 256 x 256 tiles less than half
-// the CUs (up to 1024 rows per expert).  us, the ring / it:
-//   330 rows, 77 experts, 704 x 1896, Zipf 97 / 40; 490 rows, 52 experts, 1648 x 368 34 / 16.5; 469 rows, 10 experts, 2720 x 3136 56.5 / 35;
-//   128 experts, 1536 x 4096 (1.6 GB, 252 at copy speed): 8 rows each 421 / 279, 32 500 / 334 (Zipf 473 / 385, one hot expert 740 / 543), 64
-//   511 / 465, 96 491 / 542; 64 experts, 2816 x 2048, 96 each 217 / 249; 16 experts, 2048 x 2048, 128 each 40.7 / 37.3, 192 45.1 / 47.1
-//   8 experts, 512 x 256, 1024 rows each 25.7 / 19.2, one hot expert 124 / 115; 1024 x 512, 512 each 18.8 / 13.5; 4096 x 1024, 256 each (two
-//   rounds of the ring) 30.0 / 33.7
-inline bool wgrad_short_pays(const GemmParams& p) {
-    const int64_t ring_tiles = most_row_tiles(p.total_rows, p.E, 256) * ((p.N + 255) / 256);
-    return p.K <= 64 * (int64_t)p.E || (p.K <= 1024 * (int64_t)p.E && 2 * ring_tiles <= compute_units());
-}
-
 // The 5-slot ring needs every byte of a 160 KB LDS, an even number of K-slices per tile,
 // row numbers that fit 32 bits and few enough experts for the register tables.
 template <bool FP8, int EPI>
@@ -268,7 +253,6 @@ int launch_ring(const GemmParams& p, hipStream_t stream) {
     const bool window_ok = !p.k_window || (p.k_window_multiple >= pair_elems && p.k_window_multiple % pair_elems == 0);
     if (p.a_sk != 1) {                     // both operands row-indexed (the caller checked the rest)
         if constexpr (!FP8 && EPI == FMOE_EPI_NONE) {
-            if (wgrad_short_pays(p)) return run_wgrad_short(p, stream);
             if (p.E <= TileRing5::kMaxExperts) return launch_ring_cfg<TileRing5, FP8, EPI, true, true, true>(p, stream);
             return launch_ring_cfg<TileRing5W, FP8, EPI, true, true, true>(p, stream);
         }

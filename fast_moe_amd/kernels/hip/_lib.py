@@ -26,7 +26,7 @@ EXPORTED_SYMBOLS = (
     "fmoe_combine",
     "fmoe_silu_mul", "fmoe_transpose_last2", "fmoe_jagged_transpose", "fmoe_segment_colsum",
     "fmoe_swiglu_bwd", "fmoe_combine_bwd", "fmoe_gather_rows", "fmoe_invert_index",
-    "fmoe_gate_l1_bwd", "fmoe_route_topk_static", "fmoe_hbm_probe",
+    "fmoe_gate_l1_bwd", "fmoe_weight_grad_pays", "fmoe_weight_grad", "fmoe_route_topk_static", "fmoe_hbm_probe",
 )
 ROUTE_STATIC_MAX_POSITIONS, ROUTE_STATIC_MAX_EXPERTS = 1 << 20, 512
 
@@ -94,6 +94,10 @@ def load() -> ctypes.CDLL:
     lib.fmoe_grouped_gemm.argtypes = [POINTER(GemmDesc), c_void_p]
     lib.fmoe_grouped_gemm_plan.restype = c_int
     lib.fmoe_grouped_gemm_plan.argtypes = [POINTER(GemmDesc), POINTER(c_int)]
+    lib.fmoe_weight_grad_pays.restype = c_int
+    lib.fmoe_weight_grad_pays.argtypes = [c_int, c_int, c_int, c_int, c_int64]
+    lib.fmoe_weight_grad.restype = c_int
+    lib.fmoe_weight_grad.argtypes = [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int64, c_int64, c_int64] + [c_void_p] * 4
     lib.fmoe_combine.restype = c_int
     lib.fmoe_combine.argtypes = [c_void_p, c_int, c_int64, c_int, c_int64, c_int64, c_void_p, c_void_p,
                                  c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_int, c_void_p]

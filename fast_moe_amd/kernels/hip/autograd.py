@@ -9,10 +9,10 @@ backward), built from the library's kernels:
   place; the two branches of a SwiGLU layer summed in one GEMM, fmoe_gemm_desc.a2), then the
   deterministic gather-form sum of the K routed rows of every token (fmoe_combine);
 * weight gradient = grouped GEMM over the rows of each expert as its contraction window
-  (fmoe_grouped_gemm + k_window), on the row-major tensors themselves (a_stride_k; the token
-  rows first put in expert order by fmoe_gather_rows; both matrices of a SwiGLU layer from one
-  launch, out2), or, for operands that do not qualify, on copies that fmoe_jagged_transpose
-  laid out K-contiguous and zero padded;
+  (fmoe_grouped_gemm + k_window; fmoe_weight_grad for few rows), on the row-major tensors
+  themselves (the token rows first put in expert order by fmoe_gather_rows; both matrices of a
+  SwiGLU layer from one launch, out2), or, for operands that do not qualify, on copies that
+  fmoe_jagged_transpose laid out K-contiguous and zero padded; in the weight's own memory order;
 * bias gradient   = fmoe_segment_colsum; activation and merge backward = fmoe_swiglu_bwd,
   fmoe_combine_bwd;
 * the e4m3 operators: backward in bf16 for silu_jagged_bmm_combine_fp8, on re-quantised e4m3
@@ -83,24 +83,33 @@ class _WgradOperand:
             return None
         return ops.jagged_weight_grad(both, self.rows, self.offsets, halves=True)
 
-    def weight_grad(self, dout: torch.Tensor) -> torch.Tensor:
-        """dW[e, n, k] = sum over the rows r of expert e of dout[r, n] * a(r)[k] -> [E, N, K_in]."""
-        if self.rows is not None:
-            dw = ops.jagged_weight_grad(dout, self.rows, self.offsets)
+    def weight_grad(self, dout: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+        """dW[e, k, n] = sum over the rows r of expert e of a(r)[k] * dout[r, n] -> [E, K_in, N], in the memory order of
+        ``weight``: autograd turns a gradient of another order around with an element-wise copy (8 x the time of the GEMM
+        for 49 experts, 1472 x 832)."""
+        by_k = weight.stride(2) == 1 and weight.stride(1) != 1          # [E, K_in, N] storage: the input's columns are the rows
+        E, N = self.offsets.numel() - 1, dout.shape[1]
+        a_src, total_rows, row_index, index_div, apply_silu = self.args
+        rows = self.rows
+        if rows is None and a_src.dtype == torch.float32 and a_src.ndim == 2 and a_src.shape[1] % 4 == 0 and dout.shape[1] % 4 == 0 \
+                and ops.weight_grad_pays(a_src.dtype, E, N, a_src.shape[1], total_rows):
+            rows = a_src if row_index is None else ops.gather_rows(a_src, row_index, index_div)
+            rows = self.rows = ops.silu_mul(rows, None) if apply_silu else rows
+        if rows is not None:
+            dw = ops.jagged_weight_grad(rows, dout, self.offsets) if by_k else ops.jagged_weight_grad(dout, rows, self.offsets)
             if dw is not None:
-                return dw
+                return dw if by_k else dw.permute(0, 2, 1)
         self._transposed()
-        N = dout.shape[1]
-        Kin = self.a_t.shape[0]
-        E = self.offsets.numel() - 1
         dout_t = ops.jagged_transpose(dout, self.offsets, self.pad_offsets, self.bound)        # [N, bound]
+        left, right = (self.a_t, dout_t) if by_k else (dout_t, self.a_t)
+        M, C = left.shape[0], right.shape[0]
         dev = dout.device
-        seg = torch.arange(E + 1, device=dev, dtype=torch.int64) * N
-        rows = torch.arange(E * N, device=dev, dtype=torch.int64) % N
-        b = self.a_t.t().unsqueeze(0).expand(E, self.bound, Kin)                               # B[e, k, n'] = a_t[n', k]
-        dw = ops.grouped_gemm(seg, dout_t, b, total_rows=E * N, row_index=rows, index_div=1, epilogue=EPI_NONE,
-                              k_window=self.pad_offsets, k_window_multiple=_WINDOW_MULTIPLE)
-        return dw.view(E, N, Kin)
+        seg = torch.arange(E + 1, device=dev, dtype=torch.int64) * M
+        rows = torch.arange(E * M, device=dev, dtype=torch.int64) % M
+        b = right.t().unsqueeze(0).expand(E, self.bound, C)                                    # B[e, r, c] = right[c, r]
+        dw = ops.grouped_gemm(seg, left, b, total_rows=E * M, row_index=rows, index_div=1, epilogue=EPI_NONE,
+                              k_window=self.pad_offsets, k_window_multiple=_WINDOW_MULTIPLE).view(E, M, C)
+        return dw if by_k else dw.permute(0, 2, 1)
 
 
 def _input_grad(drow_list, weights, offsets, reverse_index) -> torch.Tensor:
@@ -163,7 +172,7 @@ class IndexSelectJaggedBmm(torch.autograd.Function):
             operand = _WgradOperand(jagged, offsets, R, row_index=index.reshape(-1), index_div=K)
         H = drows[0].shape[1]
         pair = None
-        if both is not None and need[3] and need[5]:
+        if both is not None and need[3] and need[5] and not (weight.stride(2) == 1 and weight.stride(1) != 1):
             # one GEMM for both weight gradients (2H = 2816 rows per expert fill whole 256-row tiles
             # where H = 1408 leaves every sixth one half empty), each into its own tensor
             pair = operand.weight_grad_pair(both)
@@ -171,9 +180,9 @@ class IndexSelectJaggedBmm(torch.autograd.Function):
             d_w, d_wp = pair[0].permute(0, 2, 1), pair[1].permute(0, 2, 1)
         else:
             if need[3]:
-                d_w = operand.weight_grad(drows[0]).permute(0, 2, 1)
+                d_w = operand.weight_grad(drows[0], weight)
             if swiglu and need[5]:
-                d_wp = operand.weight_grad(drows[1]).permute(0, 2, 1)
+                d_wp = operand.weight_grad(drows[1], weight_p)
         if both is not None and bias is not None and bias_p is not None and need[4] and need[6]:
             d_sum = ops.segment_colsum(both, offsets)
             d_b, d_bp = d_sum[:, :H], d_sum[:, H:]
@@ -270,7 +279,7 @@ class IndexSelectJaggedGatingBmm(torch.autograd.Function):
                 d_src = _input_grad([d], [w], offsets, reverse).view_as(src)
             if need[4 + pos]:
                 operand = _WgradOperand(src, offsets, R, row_index=index.reshape(-1), index_div=K)
-                d_w = operand.weight_grad(d).permute(0, 2, 1)
+                d_w = operand.weight_grad(d, w)
             if bias is not None and need[6 + pos]:
                 d_bias = ops.segment_colsum(d, offsets)
             grads.append((d_src, d_w, d_bias))
@@ -317,7 +326,7 @@ class IndexSelectJaggedBmm3D(torch.autograd.Function):
             d_jagged = ops.combine(d_rows, slots.view(L * E, K)).view(L, E, Kin).to(jagged.dtype)
         if need[3]:
             src = jagged.contiguous().view(L * E, Kin)
-            d_w = _WgradOperand(src, offsets, R, row_index=cell, index_div=1).weight_grad(dout).permute(0, 2, 1)
+            d_w = _WgradOperand(src, offsets, R, row_index=cell, index_div=1).weight_grad(dout, weight)
         if bias is not None and need[4]:
             d_b = ops.segment_colsum(dout, offsets)
         return None, None, d_jagged, d_w, d_b
@@ -398,7 +407,7 @@ class SiluJaggedBmmCombine(torch.autograd.Function):
                 operand = _WgradOperand(silu_rows, offsets, jagged.shape[0])
             else:
                 operand = _WgradOperand(jagged, offsets, jagged.shape[0], apply_silu=ctx.has_silu)
-            d_w = operand.weight_grad(d_bmm).permute(0, 2, 1)
+            d_w = operand.weight_grad(d_bmm, weight)
         if bias is not None and need[3]:
             d_b = ops.segment_colsum(d_bmm, offsets)
         if need_g:

@@ -259,23 +259,42 @@ def slack_rows(t: torch.Tensor) -> int:
     return max(0, (have - t.shape[1]) // t.stride(0) + 1 - t.shape[0]) if t.stride(0) > 0 else 0
 
 
+def weight_grad_pays(dtype: torch.dtype, num_experts: int, m: int, n: int, rows: int) -> bool:
+    """Whether fmoe_weight_grad is the faster form of such a weight gradient."""
+    return bool(_lib.load().fmoe_weight_grad_pays(_DTYPE_CODE[dtype], num_experts, m, n, rows))
+
+
 def jagged_weight_grad(dout: torch.Tensor, a_rows: torch.Tensor, offsets: torch.Tensor, halves: bool = False):
     """dW[e, n, k] = sum over the rows r of expert e of dout[r, n] * a_rows[r, k] -> [E, N, K_in],
-    both operands read in place (fmoe_grouped_gemm with a_stride_k).  Returns None when the
-    operands do not qualify (dtype, alignment, no slack behind them): the caller then takes the
-    route over transposed copies.  ``halves``: dout holds the row gradients of two matrices side
-    by side; the result is two tensors [E, N/2, K_in] (fmoe_gemm_desc.out2)."""
-    if dout.dtype != torch.bfloat16 or a_rows.dtype != torch.bfloat16 or dout.shape[0] != a_rows.shape[0]:
+    both operands read in place: fmoe_weight_grad where that pays (few rows, fp32), else fmoe_grouped_gemm
+    with a_stride_k (bf16).  Returns None when the operands do not qualify (dtype, alignment, no slack behind
+    them): the caller then takes the route over transposed copies.  ``halves``: dout holds the row gradients of
+    two matrices side by side; the result is two tensors [E, N/2, K_in] (fmoe_gemm_desc.out2)."""
+    if dout.dtype not in _DTYPE_CODE or a_rows.dtype != dout.dtype or dout.shape[0] != a_rows.shape[0]:
         return None
     R, N = dout.shape
     Kin = a_rows.shape[1]
     E = offsets.numel() - 1
-    ok = (dout.stride(1) == 1 and a_rows.stride(1) == 1 and N % 8 == 0 and Kin % 8 == 0 and E <= 256
-          and dout.stride(0) % 8 == 0 and a_rows.stride(0) % 8 == 0 and dout.data_ptr() % 16 == 0
-          and a_rows.data_ptr() % 16 == 0 and R >= 128 and E * N < (1 << 31)
-          and slack_rows(dout) >= SLACK_ROWS and slack_rows(a_rows) >= SLACK_ROWS
-          and (not halves or N % 64 == 0))
-    if not ok:
+    bf16 = dout.dtype == torch.bfloat16
+    chunk = 8 if bf16 else 4
+    if not (dout.stride(1) == 1 and a_rows.stride(1) == 1 and N % chunk == 0 and Kin % chunk == 0 and R >= 1
+            and dout.stride(0) % chunk == 0 and a_rows.stride(0) % chunk == 0 and dout.stride(0) >= N
+            and a_rows.stride(0) >= Kin and dout.data_ptr() % 16 == 0 and a_rows.data_ptr() % 16 == 0
+            and E * N < (1 << 31) and (not halves or N % 64 == 0)):
+        return None
+    if bf16 and not (slack_rows(dout) >= SLACK_ROWS and slack_rows(a_rows) >= SLACK_ROWS):
+        return None
+    lib, code = _lib.load(), _DTYPE_CODE[dout.dtype]
+    if (bf16 and R < 128) or lib.fmoe_weight_grad_pays(code, E, N, Kin, R):
+        offsets = _i64("offsets", offsets)
+        outs = [torch.empty((E, N // 2 if halves else N, Kin), dtype=dout.dtype, device=dout.device)
+                for _ in range(2 if halves else 1)]
+        rc = lib.fmoe_weight_grad(dout.data_ptr(), a_rows.data_ptr(), code, E, N, Kin, R, dout.stride(0), a_rows.stride(0),
+                                  offsets.data_ptr(), outs[0].data_ptr(), outs[1].data_ptr() if halves else None,
+                                  _stream(dout))
+        _lib.check(rc, "fmoe_weight_grad")
+        return tuple(outs) if halves else outs[0]
+    if not bf16 or R < 128 or E > 256:
         return None
     dev = dout.device
     offsets = _i64("offsets", offsets)

@@ -405,6 +405,18 @@ int fmoe_segment_colsum(const void* src, int dtype, int64_t total_rows, int64_t 
                         fmoe_stream_t stream);
 
 /*
+ * Weight gradient of experts with few rows: out[e, i, j] = sum over the rows r of expert e (offsets[e] .. offsets[e+1]) of
+ * a[r, i] * b[r, j], a [rows, m] and b [rows, n] row-major of one type (FMOE_BF16 or FMOE_F32), out [E, m, n] contiguous.  With
+ * out2 the rows i >= m/2 of every expert go to out2 and both are [E, m/2, n] (m a multiple of 64).  m, n and the row strides whole
+ * 16-byte chunks, 16-byte aligned pointers.  Nothing is read behind the last row.  What fmoe_grouped_gemm with a_stride_k and a
+ * k_window computes (kernels/triton/triton_moe.py:606-804); fmoe_weight_grad_pays: non-zero where this is the faster form.
+ */
+int fmoe_weight_grad_pays(int dtype, int num_experts, int m, int n, int64_t rows);
+int fmoe_weight_grad(const void* a, const void* b, int dtype, int num_experts, int m, int n, int64_t rows,
+                     int64_t a_stride_row, int64_t b_stride_row, const int64_t* offsets, void* out, void* out2,
+                     fmoe_stream_t stream);
+
+/*
  * index [T*K]: expert-sorted position -> flat token*K + slot, a permutation.  reverse [T, K]: the
  * positions of every token's rows, ascending (the order in which a sequential index_add meets
  * them): what the gather-form sum of a token's input-gradient rows reads (fmoe_combine; the
