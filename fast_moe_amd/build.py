@@ -21,7 +21,7 @@ OBJ_DIR = os.path.join(CSRC, "build")
 
 SOURCES = ["gemm_bf16.hip", "gemm_fp8.hip", "gemm_bf16_tail.hip", "gemm_fp8_tail.hip", "gemm_bf16_short.hip", "gemm_fp8_short.hip",
            "gemm_f32.hip", "gemm_direct.hip", "gemm_wgrad.hip", "gemm_api.hip",
-           "core.hip", "routing.hip", "quant.hip", "combine.hip", "backward.hip"]
+           "gate.hip", "core.hip", "routing.hip", "quant.hip", "combine.hip", "backward.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

@@ -29,6 +29,7 @@ decltype(&fmoe_route_topk) c_route_topk;
 decltype(&fmoe_grouped_gemm) c_grouped_gemm;
 decltype(&fmoe_combine) c_combine;
 decltype(&fmoe_quant_rows_e4m3) c_quant_rows;
+decltype(&fmoe_gate_softmax) c_gate_softmax;
 decltype(&fmoe_last_error) last_error;
 
 constexpr int64_t kSlackRows = 128;      // ops.SLACK_ROWS
@@ -110,25 +111,30 @@ int route(const at::Tensor& scores, const void* data, int64_t k, int64_t mode, v
                         r.reverse_index.data_ptr<int64_t>(), r.workspace.data_ptr(), r.workspace.numel(), stream);
 }
 
+// Intermediates of a call that is issued whole have no tensors of their own (one allocation holds them all): offsets and row_index are
+// pointers then, and a stands for contiguous rows at a_data.
 struct GemmArgs {
     at::Tensor offsets, a, b, row_index, bias, b2, bias2, a_scale, b_scale, b2_scale;
     int64_t total_rows = 0, index_div = 1, epilogue = FMOE_EPI_NONE, pow2 = 0;
+    const int64_t *offsets_data = nullptr, *row_index_data = nullptr;
+    const void* a_data = nullptr;
+    int64_t a_rows = 0;
 };
 
 // Checks the operands and fills everything of the descriptor but the output.
 bool gemm_ok(const GemmArgs& g, fmoe_gemm_desc& d) {
     const at::Tensor &a = g.a, &b = g.b;
-    const int code = dtype_code(a.scalar_type());
-    if (code < 0 || b.scalar_type() != a.scalar_type() || a.dim() != 2 || b.dim() != 3) return false;
+    const int code = dtype_code(b.scalar_type());
+    if (code < 0 || b.dim() != 3 || (!g.a_data && (a.scalar_type() != b.scalar_type() || a.dim() != 2))) return false;
     const bool fp8 = code == FMOE_E4M3;
     const at::ScalarType out_dtype = code == FMOE_F32 ? at::kFloat : at::kBFloat16;
     const int64_t E = b.size(0), K = b.size(1), N = b.size(2);
-    if (a.size(1) != K || a.stride(1) != 1 || g.total_rows < 1 || g.index_div < 1 || E > INT32_MAX || K > INT32_MAX ||
+    if ((!g.a_data && (a.size(1) != K || a.stride(1) != 1)) || g.total_rows < 1 || g.index_div < 1 || E > INT32_MAX || K > INT32_MAX ||
         N > INT32_MAX || g.index_div > INT32_MAX)
         return false;
-    for (const at::Tensor* t : {&g.offsets, &g.b, &g.row_index, &g.bias, &g.b2, &g.bias2, &g.a_scale, &g.b_scale, &g.b2_scale})
-        if (!same_device(a, *t)) return false;
-    if (!i64_list(g.offsets, E + 1) || (g.row_index.defined() && !i64_list(g.row_index, g.total_rows))) return false;
+    for (const at::Tensor* t : {&g.offsets, &g.a, &g.row_index, &g.bias, &g.b2, &g.bias2, &g.a_scale, &g.b_scale, &g.b2_scale})
+        if (!same_device(b, *t)) return false;
+    if ((!g.offsets_data && !i64_list(g.offsets, E + 1)) || (g.row_index.defined() && !i64_list(g.row_index, g.total_rows))) return false;
     if (g.b2.defined() &&
         (g.b2.scalar_type() != b.scalar_type() || g.b2.sizes() != b.sizes() || g.b2.strides() != b.strides()))
         return false;
@@ -153,14 +159,14 @@ bool gemm_ok(const GemmArgs& g, fmoe_gemm_desc& d) {
     d.k = (int32_t)K;
     d.index_div = (int32_t)g.index_div;
     d.total_rows = g.total_rows;
-    d.a_rows = a.size(0);
+    d.a_rows = g.a_data ? g.a_rows : a.size(0);
     auto data = [](const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
     auto floats = [](const at::Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; };
-    d.offsets = g.offsets.data_ptr<int64_t>();
-    d.row_index = g.row_index.defined() ? g.row_index.data_ptr<int64_t>() : nullptr;
-    d.a = a.data_ptr();
+    d.offsets = g.offsets_data ? g.offsets_data : g.offsets.data_ptr<int64_t>();
+    d.row_index = g.row_index.defined() ? g.row_index.data_ptr<int64_t>() : g.row_index_data;
+    d.a = g.a_data ? g.a_data : a.data_ptr();
     d.a_dtype = code;
-    d.a_stride_row = a.stride(0);
+    d.a_stride_row = g.a_data ? K : a.stride(0);
     d.a_scale = floats(g.a_scale);
     d.b = b.data_ptr();
     d.b2 = data(g.b2);
@@ -192,7 +198,7 @@ struct Combine {
     const int64_t *reverse_data, *index_data = nullptr;
     at::ScalarType out_dtype;
     int code, g_code = FMOE_F32;
-    int64_t T, K, D, cols = 1, sr = 1, sc = 1;
+    int64_t T, K, D, value_stride, cols = 1, sr = 1, sc = 1;
 };
 
 bool combine_ok(Combine& c) {
@@ -219,14 +225,15 @@ bool combine_ok(Combine& c) {
         }
     }
     c.value_data = c.value.data_ptr();
+    c.value_stride = c.value.stride(0);
     c.reverse_data = c.reverse.data_ptr<int64_t>();
     return true;
 }
 
-at::Tensor allocate(const Combine& c) { return empty({c.T, c.D}, c.out_dtype, c.value); }
+at::Tensor allocate(const Combine& c, const at::Tensor& like) { return empty({c.T, c.D}, c.out_dtype, like); }
 
 int combine(const Combine& c, const at::Tensor& out, void* stream) {
-    return c_combine(c.value_data, c.code, c.T, (int)c.K, c.D, c.value.stride(0), c.reverse_data, c.gates_data, c.g_code, c.cols,
+    return c_combine(c.value_data, c.code, c.T, (int)c.K, c.D, c.value_stride, c.reverse_data, c.gates_data, c.g_code, c.cols,
                      c.sr, c.sc, c.index_data, out.data_ptr(), dtype_code(c.out_dtype), stream);
 }
 
@@ -318,7 +325,7 @@ PyObject* py_combine(PyObject*, PyObject* const* args, Py_ssize_t n) {
     at::Tensor out;
     const int status = run([&] { return combine_ok(c); },
                            [&] {
-                               out = allocate(c);
+                               out = allocate(c, c.value);
                                return combine(c, out, (void*)stream);
                            });
     if (raised(status, "fmoe_combine")) return nullptr;
@@ -355,6 +362,38 @@ PyObject* py_quant_rows(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// (x [T, D], weight [E, D], bias [E] or None, stream) -> softmax(x weight^T + bias) [T, E]
+PyObject* py_gate_softmax(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 4) return none();
+    const at::Tensor x = gpu_tensor(args[0]), w = gpu_tensor(args[1]);
+    at::Tensor bias, scores;
+    int64_t stream;
+    if (!x.defined() || !w.defined() || !optional_tensor(args[2], &bias) || !as_int(args[3], &stream)) return none();
+    const void *x_data, *w_data, *b_data = nullptr;
+    const int status = run(
+        [&] {
+            const int code = dtype_code(x.scalar_type());
+            if ((code != FMOE_F32 && code != FMOE_BF16) || w.scalar_type() != x.scalar_type() || x.dim() != 2 || w.dim() != 2 ||
+                x.size(1) != w.size(1) || x.stride(1) != 1 || !w.is_contiguous() || !same_device(x, w) || !same_device(x, bias) ||
+                w.size(0) > INT32_MAX || w.size(1) > INT32_MAX)
+                return false;
+            if (bias.defined() && (bias.scalar_type() != x.scalar_type() || !bias.is_contiguous() || bias.numel() != w.size(0))) return false;
+            x_data = x.data_ptr();
+            w_data = w.data_ptr();
+            if (bias.defined()) b_data = bias.data_ptr();
+            return true;
+        },
+        [&] {
+            scores = empty({x.size(0), w.size(0)}, x.scalar_type(), x);
+            return c_gate_softmax(x_data, dtype_code(x.scalar_type()), x.size(0), (int)x.size(1), x.stride(0), w_data, b_data, (int)w.size(0),
+                                  scores.data_ptr(), (void*)stream);
+        });
+    if (raised(status, "fmoe_gate_softmax")) return nullptr;
+    return status == FMOE_OK ? wrap(scores) : none();
+    END_HANDLE_TH_ERRORS
+}
+
 // (scores [T, E], x [T, D], w1 [E, D, H], bias1, w2 [E, H, O], bias2, k, mode, epilogue1, stream) -> [T, O]:
 // routing, the gather GEMM with its activation, the second GEMM, the merge
 PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -367,49 +406,85 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (!t->defined()) return none();
     if (!as_int(args[6], &k) || !as_int(args[7], &mode) || !as_int(args[8], &epilogue) || !as_int(args[9], &stream))
         return none();
-    at::Tensor hidden, rows, y;
+    at::Tensor scratch, y;
     const void* data;
-    Routing r;
+    char* base = nullptr;
+    size_t at_ws = 0, ws_bytes = 0;
+    int64_t *topk_idx = nullptr, *lengths = nullptr, *offsets = nullptr, *gate_index = nullptr, *token_index = nullptr, *reverse = nullptr;
+    void* gates = nullptr;
     fmoe_gemm_desc up, down;
     Combine merge;
     const char* what = "fmoe_route_topk";
     // All operands of the four launches, intermediates included, exist and are checked before the first launch: a call that
-    // is declined has routed nothing.
+    // is declined has routed nothing.  One allocation holds the intermediates (twelve were 10 of the 30 us that the call took).
     const int status = run(
         [&] {
-            if (x.dim() != 2 || scores.dim() != 2 || scores.size(0) != x.size(0) || w1.dim() != 3 ||
-                w1.size(0) != scores.size(1) || scores.device() != x.device() || !route_ok(scores, k, &data))
+            if (x.dim() != 2 || scores.dim() != 2 || scores.size(0) != x.size(0) || w1.dim() != 3 || w2.dim() != 3 ||
+                w1.size(0) != scores.size(1) || w2.size(0) != scores.size(1) || w2.size(1) != w1.size(2) ||
+                w2.scalar_type() != w1.scalar_type() || scores.device() != x.device() || w1.device() != x.device() ||
+                w2.device() != x.device() || !route_ok(scores, k, &data))
                 return false;
-            allocate(scores, k, r);
+            const int64_t T = x.size(0), E = scores.size(1), H = w1.size(2), O = w2.size(2), R = T * k;
+            const int64_t row_size = w1.scalar_type() == at::kFloat ? 4 : 2;
+            size_t bytes = 0;
+            auto take = [&](int64_t n, int64_t size) {
+                const size_t at = bytes;
+                bytes += ((size_t)(n * size) + 255) & ~(size_t)255;
+                return at;
+            };
+            ws_bytes = route_workspace_bytes(T, (int)E, (int)k);
+            const size_t at_topk = take(R, 8), at_lengths = take(E, 8), at_offsets = take(E + 1, 8), at_gate = take(R, 8);
+            const size_t at_token = take(R, 8), at_reverse = take(R, 8), at_gates = take(R, (int64_t)scores.element_size());
+            at_ws = take((int64_t)ws_bytes, 1);
+            const size_t at_hidden = take((R + kSlackRows) * H, row_size), at_rows = take((R + kSlackRows) * O, row_size);
+            scratch = empty({(int64_t)bytes}, at::kByte, x);
+            base = (char*)scratch.data_ptr();
+            topk_idx = (int64_t*)(base + at_topk);
+            lengths = (int64_t*)(base + at_lengths);
+            offsets = (int64_t*)(base + at_offsets);
+            gate_index = (int64_t*)(base + at_gate);
+            token_index = (int64_t*)(base + at_token);
+            reverse = (int64_t*)(base + at_reverse);
+            gates = base + at_gates;
             GemmArgs g;
-            g.offsets = r.offsets;
+            g.offsets_data = offsets;
             g.a = x;
             g.b = w1;
-            g.row_index = r.gate_index;
+            g.row_index_data = gate_index;
             g.bias = b1;
-            g.total_rows = x.size(0) * k;
+            g.total_rows = R;
             g.index_div = k;
             g.epilogue = epilogue;
             if (!gemm_ok(g, up)) return false;
-            hidden = allocate(up, x);
+            up.out = base + at_hidden;
+            up.out_stride_row = H;
             g = GemmArgs();
-            g.offsets = r.offsets;
-            g.a = hidden;
+            g.offsets_data = offsets;
+            g.a_data = up.out;
+            g.a_rows = R;
             g.b = w2;
             g.bias = b2;
-            g.total_rows = hidden.size(0);
+            g.total_rows = R;
             if (!gemm_ok(g, down)) return false;
-            rows = allocate(down, x);
-            merge.value = rows;
-            merge.reverse = r.reverse_index;
-            merge.gates = r.gates;
-            merge.gates_index = r.gate_index;
-            if (!combine_ok(merge)) return false;
-            y = allocate(merge);
+            down.out = base + at_rows;
+            down.out_stride_row = O;
+            merge.code = down.out_dtype;
+            merge.g_code = dtype_code(scores.scalar_type());
+            merge.out_dtype = merge.code == FMOE_F32 || merge.g_code == FMOE_F32 ? at::kFloat : at::kBFloat16;
+            merge.T = T;
+            merge.K = merge.cols = merge.sr = k;
+            merge.D = merge.value_stride = O;
+            merge.value_data = down.out;
+            merge.reverse_data = reverse;
+            merge.gates_data = gates;
+            merge.index_data = gate_index;
+            y = allocate(merge, x);
             return true;
         },
         [&] {
-            if (const int rc = route(scores, data, k, mode, (void*)stream, r)) return rc;
+            if (const int rc = c_route_topk(data, dtype_code(scores.scalar_type()), merge.T, (int)scores.size(1), (int)k, (int)mode, topk_idx,
+                                            gates, lengths, offsets, gate_index, token_index, reverse, base + at_ws, ws_bytes, (void*)stream))
+                return rc;
             RECORD_USER_SCOPE("## expert_forward##");
             what = "fmoe_grouped_gemm";
             if (const int rc = c_grouped_gemm(&up, (void*)stream)) return rc;
@@ -424,12 +499,12 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // init(addresses of the C entry points, in the order of the pointers above)
 PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    int64_t v[6];
-    if (n != 6) {
-        PyErr_SetString(PyExc_TypeError, "init: six addresses expected");
+    int64_t v[7];
+    if (n != 7) {
+        PyErr_SetString(PyExc_TypeError, "init: seven addresses expected");
         return nullptr;
     }
-    for (int i = 0; i < 6; ++i)
+    for (int i = 0; i < 7; ++i)
         if (!as_int(args[i], &v[i])) {
             PyErr_SetString(PyExc_TypeError, "init: addresses are integers");
             return nullptr;
@@ -439,7 +514,8 @@ PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
     c_grouped_gemm = (decltype(c_grouped_gemm))v[2];
     c_combine = (decltype(c_combine))v[3];
     c_quant_rows = (decltype(c_quant_rows))v[4];
-    last_error = (decltype(last_error))v[5];
+    c_gate_softmax = (decltype(c_gate_softmax))v[5];
+    last_error = (decltype(last_error))v[6];
     return none();
 }
 
@@ -450,6 +526,7 @@ PyMethodDef methods[] = {
     FASTCALL("grouped_gemm", py_grouped_gemm),
     FASTCALL("combine", py_combine),
     FASTCALL("quant_rows", py_quant_rows),
+    FASTCALL("gate_softmax", py_gate_softmax),
     FASTCALL("mlp_forward", py_mlp_forward),
     {nullptr, nullptr, 0, nullptr},
 };

@@ -26,7 +26,7 @@ EXPORTED_SYMBOLS = (
     "fmoe_combine",
     "fmoe_silu_mul", "fmoe_transpose_last2", "fmoe_jagged_transpose", "fmoe_segment_colsum",
     "fmoe_swiglu_bwd", "fmoe_combine_bwd", "fmoe_gather_rows", "fmoe_invert_index",
-    "fmoe_gate_l1_bwd", "fmoe_weight_grad_pays", "fmoe_weight_grad", "fmoe_route_topk_static", "fmoe_hbm_probe",
+    "fmoe_gate_l1_bwd", "fmoe_gate_softmax_pays", "fmoe_gate_softmax", "fmoe_weight_grad_pays", "fmoe_weight_grad", "fmoe_route_topk_static", "fmoe_hbm_probe",
 )
 ROUTE_STATIC_MAX_POSITIONS, ROUTE_STATIC_MAX_EXPERTS = 1 << 20, 512
 
@@ -94,6 +94,10 @@ def load() -> ctypes.CDLL:
     lib.fmoe_grouped_gemm.argtypes = [POINTER(GemmDesc), c_void_p]
     lib.fmoe_grouped_gemm_plan.restype = c_int
     lib.fmoe_grouped_gemm_plan.argtypes = [POINTER(GemmDesc), POINTER(c_int)]
+    lib.fmoe_gate_softmax_pays.restype = c_int
+    lib.fmoe_gate_softmax_pays.argtypes = [c_int, c_int64, c_int, c_int]
+    lib.fmoe_gate_softmax.restype = c_int
+    lib.fmoe_gate_softmax.argtypes = [c_void_p, c_int, c_int64, c_int, c_int64, c_void_p, c_void_p, c_int, c_void_p, c_void_p]
     lib.fmoe_weight_grad_pays.restype = c_int
     lib.fmoe_weight_grad_pays.argtypes = [c_int, c_int, c_int, c_int, c_int64]
     lib.fmoe_weight_grad.restype = c_int
@@ -134,14 +138,14 @@ def load() -> ctypes.CDLL:
 
 # what csrc/host_calls.cpp calls, in the order its init() takes the addresses
 HOST_ENTRY_POINTS = ("fmoe_route_workspace_bytes", "fmoe_route_topk", "fmoe_grouped_gemm", "fmoe_combine",
-                     "fmoe_quant_rows_e4m3", "fmoe_last_error")
+                     "fmoe_quant_rows_e4m3", "fmoe_gate_softmax", "fmoe_last_error")
 _host = None
 
 
 class _Declines:
     """In the place of the extension module where that does not load: every call is left to the Python code in ops.py."""
 
-    route_topk = grouped_gemm = combine = quant_rows = mlp_forward = staticmethod(lambda *args: None)
+    route_topk = grouped_gemm = combine = quant_rows = gate_softmax = mlp_forward = staticmethod(lambda *args: None)
 
 
 def host():

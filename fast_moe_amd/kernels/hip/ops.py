@@ -127,6 +127,30 @@ def route_topk(scores: torch.Tensor, k: int, renorm=True, static_scratch: bool =
     return out
 
 
+def gate_softmax(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """``softmax(F.linear(x, weight, bias), dim=1)`` of a small batch [T, D] in one launch (fmoe_gate_softmax), or None where
+    that is not the faster form or does not take the operands."""
+    T, D = x.shape
+    if weight.dtype != x.dtype or x.dtype not in _DTYPE_CODE or not x.is_cuda:
+        return None
+    lib, code = _lib.load(), _DTYPE_CODE[x.dtype]
+    if not lib.fmoe_gate_softmax_pays(code, T, D, weight.shape[0]) or x.data_ptr() % 16 or weight.data_ptr() % 16:
+        return None
+    chunk = 4 if code == 0 else 8
+    if (x.stride(1) != 1 or x.stride(0) < D or x.stride(0) % chunk or weight.shape[1] != D or not weight.is_contiguous()
+            or (bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous()))):
+        return None
+    scores = _lib.host().gate_softmax(x, weight, bias, _stream(x))
+    if scores is not None:
+        return scores
+    _need_cuda("gate_softmax", x, weight, bias)
+    scores = torch.empty((T, weight.shape[0]), dtype=x.dtype, device=x.device)
+    rc = lib.fmoe_gate_softmax(x.data_ptr(), code, T, D, x.stride(0), weight.data_ptr(), _ptr(bias), weight.shape[0],
+                               scores.data_ptr(), _stream(x))
+    _lib.check(rc, "fmoe_gate_softmax")
+    return scores
+
+
 def route_from_topk(topk_idx: torch.Tensor, num_experts: int) -> Dict[str, torch.Tensor]:
     """topk_idx [T, K] int64 expert ids -> routing tensors, see fmoe_route_from_topk.  Ids outside
     [0, num_experts) are dropped and counted in ``bad_count`` (a device tensor: reading it

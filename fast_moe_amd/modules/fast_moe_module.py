@@ -3,7 +3,7 @@ on the MI355X HIP back-end.
 
 Constructor arguments, parameter names / shapes / dtypes (so state_dicts
 interchange) and ``forward(x, num_experts_per_tok)`` are the reference's.  The
-gate (Linear + softmax) stays a torch call; everything after it -- top-k, gate
+gate (Linear + softmax) is one launch for a small batch without gradients and a torch call otherwise; everything after it -- top-k, gate
 renormalisation, routing tensors, both expert GEMMs, SiLU and the weighted
 merge -- runs in libfastmoe_hip.so with no host synchronisation (the reference
 syncs once for ``max_seq_len``, fast_moe_module.py:135).
@@ -16,6 +16,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd.profiler import record_function
+from torch.nn.modules import module as _nn_module
 
 from ..kernels.hip import _lib, ops
 from ..kernels.hip._lib import EPI_NONE, EPI_SILU
@@ -62,8 +63,7 @@ class FastMoELayer(nn.Module):
 
     def route(self, x: torch.Tensor, num_experts_per_tok: int) -> Dict[str, torch.Tensor]:
         """fast_moe_module.py:93-144 in one library call on the gate probabilities."""
-        scores = self.gate(x).reshape(-1, self.num_experts)
-        return ops.route_topk(scores, num_experts_per_tok, renorm=True)
+        return ops.route_topk(self._scores(x), num_experts_per_tok, renorm=True)
 
     def quantized_expert_weights(self, refresh: bool = False) -> Dict[str, torch.Tensor]:
         """Row-quantised e4m3 copies of both expert weight tensors in the layout the fp8 operators
@@ -103,6 +103,20 @@ class FastMoELayer(nn.Module):
             has_silu=True)
         return y.view(original_shape[0], original_shape[1], self.output_dim)
 
+    def _scores(self, x: torch.Tensor) -> torch.Tensor:
+        """The gate's probabilities [tokens, E]: from one launch where the batch is small, nothing needs a gradient and the gate is the
+        class's own; a caller's module, hooks and autocast are asked through the modules."""
+        gate = self.gate
+        if x.numel() <= _SMALL_BATCH * self.input_dim and type(gate) is GatingNetwork and type(gate.gate) is nn.Linear \
+                and type(x) is torch.Tensor and GatingNetwork.forward is _GATE_FORWARD and not _watched(gate) \
+                and not _watched(gate.gate) and not torch.is_autocast_enabled():
+            weight, bias = gate.gate.weight, gate.gate.bias
+            if not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)):
+                scores = ops.gate_softmax(x.reshape(-1, self.input_dim), weight, bias)
+                if scores is not None:
+                    return scores
+        return gate(x).reshape(-1, self.num_experts)
+
     def forward(self, x: torch.Tensor, num_experts_per_tok: int) -> torch.Tensor:
         require_hip_kernel(self.kernel, "FastMoELayer.forward")
         if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters())):
@@ -113,7 +127,7 @@ class FastMoELayer(nn.Module):
         k = num_experts_per_tok
         if getattr(self.route, "__func__", None) is _ROUTE and x.ndim == 3:
             # the same steps as below, issued by one native call (a route() of a subclass's or a caller's own is asked)
-            scores = self.gate(x).reshape(-1, self.num_experts)
+            scores = self._scores(x)
             y = _lib.host().mlp_forward(
                 scores, x.reshape(-1, self.input_dim), self._experts_hidden_w.permute(0, 2, 1), self._experts_hidden_bias,
                 self._experts_w.permute(0, 2, 1), self._experts_bias, k, ops.GATE_L1, EPI_SILU, ops._stream(x))
@@ -138,3 +152,11 @@ class FastMoELayer(nn.Module):
 
 
 _ROUTE = FastMoELayer.route     # what the native call stands for
+_GATE_FORWARD = GatingNetwork.forward
+_SMALL_BATCH = 128              # (the library's own rule, fmoe_gate_softmax_pays, without a call for the others)
+
+
+def _watched(module: nn.Module) -> bool:
+    """Whether a call of the module does more than its class's forward."""
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or "forward" in module.__dict__ or _nn_module._has_any_global_hook())

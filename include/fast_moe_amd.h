@@ -132,6 +132,16 @@ int fmoe_route_from_topk(const int64_t* topk_idx, int64_t T, int E, int K,
                          int64_t* token_index, int64_t* reverse_index, int64_t* bad_count,
                          void* workspace, size_t workspace_bytes, fmoe_stream_t stream);
 
+/*
+ * The gate of a small batch (modules/fast_moe_module.py:21-27): scores [T, E] = softmax(x weight^T + bias), x [T, D] rows at
+ * x_stride_row, weight [E, D] and bias [E] (or NULL) contiguous, all of one type (FMOE_BF16 or FMOE_F32): fp32 sums, logits rounded
+ * to that type before the softmax.  D in whole 16-byte chunks, x and weight 16-byte aligned, E <= 96.  fmoe_gate_softmax_pays:
+ * non-zero where one launch is faster than a library GEMM and a softmax (few tokens).
+ */
+int fmoe_gate_softmax_pays(int dtype, int64_t T, int D, int E);
+int fmoe_gate_softmax(const void* x, int dtype, int64_t T, int D, int64_t x_stride_row, const void* weight, const void* bias,
+                      int E, void* scores, fmoe_stream_t stream);
+
 /* ---------------------------------------------------------- FP8 quantisation */
 
 /*

@@ -257,3 +257,71 @@ def test_forward_replays_from_a_hip_graph(fp8):
             assert torch.equal(y, ref), f"replay {i}"
             assert torch.equal(forward(), ref)      # eager work between the replays
             torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,D,E", [(1, 8, 1), (3, 24, 4), (16, 128, 8), (17, 136, 16), (64, 2048, 17), (40, 1000, 32), (128, 264, 33), (100, 512, 64),
+                                   (33, 72, 65), (9, 4096, 96)])
+def test_gate_of_a_small_batch(T, D, E, dtype):
+    """One launch for Linear + softmax: logits within the rounding of an fp32 sum (2^-24 for every product) of float64's, the softmax of the
+    rounded logits as torch gives it; rows of a wider tensor; up to E = 96."""
+    from fast_moe_amd.kernels.hip import ops
+    g = torch.Generator(device="cuda").manual_seed(T + D + E)
+    x = torch.full((T, D + 8), float("nan"), dtype=dtype, device="cuda")[:, :D]
+    x.copy_(torch.randn(T, D, generator=g, device="cuda"))
+    w = (torch.randn(E, D, generator=g, device="cuda") * D ** -0.5).to(dtype)
+    for bias in (torch.randn(E, generator=g, device="cuda").to(dtype), None):
+        got = ops.gate_softmax(x, w, bias)
+        exact = x.double() @ w.double().t() + (0 if bias is None else bias.double())
+        err = (D + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + (0 if bias is None else bias.double().abs()))
+        if dtype == torch.bfloat16:
+            err = err + 2.0 ** -8 * (exact.abs() + err)         # the logit's own rounding
+        want = torch.softmax(exact, dim=1)
+        # d softmax <= softmax * (own error + the largest of the row); its own few roundings, and bf16's
+        step = want * torch.expm1(err + err.amax(dim=1, keepdim=True)) + 64 * 2.0 ** -24
+        if dtype == torch.bfloat16:
+            step = step + 2.0 ** -8 * want
+        assert got.dtype == dtype and got.shape == (T, E)
+        assert bool(((got.double() - want).abs() <= step).all())
+    assert ops.gate_softmax(torch.zeros(129, D, dtype=dtype, device="cuda"), w, None) is None
+    assert ops.gate_softmax(x, torch.zeros(97, D, dtype=dtype, device="cuda"), None) is None
+
+
+def test_gate_modules_that_are_watched_are_called(monkeypatch):
+    """Hooks, autocast, gradients, a subclass or an instance's own forward: the gate module is asked, not the launch that stands for it."""
+    import torch.nn as nn
+    from fast_moe_amd import FastMoELayer
+    from fast_moe_amd.kernels.hip import ops
+    from fast_moe_amd.modules import fast_moe_module as m
+    layer = FastMoELayer(64, 96, 64, 4).to(torch.bfloat16).cuda()
+    x = torch.randn(2, 8, 64, device="cuda").to(torch.bfloat16)
+    calls, fused, real = [], [], ops.gate_softmax
+    monkeypatch.setattr(ops, "gate_softmax", lambda *a: fused.append(1) or real(*a))
+
+    class Gate(m.GatingNetwork):
+        pass
+
+    with torch.no_grad():
+        layer(x, 2)
+        assert len(fused) == 1
+        for hooked in (layer.gate, layer.gate.gate):
+            handle = hooked.register_forward_hook(lambda *a: calls.append(1))
+            layer(x, 2)
+            handle.remove()
+        handle = nn.modules.module.register_module_forward_hook(lambda *a: None)
+        layer(x, 2)
+        handle.remove()
+        layer.gate.gate.forward = lambda t, real=layer.gate.gate.forward: calls.append(1) or real(t)
+        layer(x, 2)
+        del layer.gate.gate.forward
+        with torch.autocast("cuda", torch.bfloat16):
+            layer(x, 2)
+        layer.gate.__class__ = Gate
+        layer(x, 2)
+    layer.gate.__class__ = m.GatingNetwork
+    layer(x, 2)
+    layer.route(x, 2)
+    assert len(calls) == 3 and len(fused) == 1
+    layer.requires_grad_(False)
+    layer(x, 2)
+    assert len(fused) == 2
