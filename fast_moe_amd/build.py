@@ -20,7 +20,7 @@ HOST_PATH = os.path.join(HERE, "_host.so")     # the native side of the Python w
 OBJ_DIR = os.path.join(CSRC, "build")
 
 SOURCES = ["gemm_bf16.hip", "gemm_fp8.hip", "gemm_bf16_tail.hip", "gemm_fp8_tail.hip", "gemm_bf16_short.hip", "gemm_fp8_short.hip",
-           "gemm_f32.hip", "gemm_direct.hip", "gemm_wgrad.hip", "gemm_api.hip",
+           "gemm_bf16_split.hip", "gemm_fp8_split.hip", "gemm_f32.hip", "gemm_direct.hip", "gemm_wgrad.hip", "gemm_api.hip",
            "gate.hip", "core.hip", "routing.hip", "quant.hip", "combine.hip", "backward.hip"]
 
 HIPCC_FLAGS = [

@@ -99,6 +99,7 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
         p.out_half = d->total_rows / (2 * (int64_t)d->num_experts);
     }
     p.a2 = (const uint8_t*)d->a2;
+    p.split_ws = nullptr;
     p.k_split = d->k;
     p.index_div = d->index_div;
     p.index_shift = -1;
@@ -237,12 +238,35 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
     return FMOE_OK;
 }
 
-extern "C" int fmoe_grouped_gemm(const fmoe_gemm_desc* d, fmoe_stream_t stream_) {
+// Whether a prepared call is one the ring cuts along K (both operands as the paired tall ring takes them: whole pairs of slices or
+// the tail kernels' conditions).
+static bool split_takes(const fmoe_gemm_desc* d, const GemmParams& p, int sel) {
+    const bool fp8 = d->a_dtype == FMOE_E4M3;
+    const int esize = fp8 ? 1 : 2, pair = 128 / esize;
+    return sel == kSelRing && !p.direct && d->a_dtype != FMOE_F32 && d->epilogue != FMOE_EPI_GATED && !d->k_window && !d->a2 && d->a_stride_k <= 1 && !d->a_silu &&
+           p.E <= (fp8 ? TileRing5::kMaxExperts : TileRing5W::kMaxExperts) && p.total_rows < ((int64_t)1 << 31) &&
+           lds_per_block() >= TileRing5::LDS_BYTES &&
+           (p.K % pair == 0 ? p.K >= 4 * pair : !fp8 && ring_tail_takes(esize, p.K, p.E, p.total_rows)) && split_pays(p, esize, d->epilogue);
+}
+
+extern "C" size_t fmoe_grouped_gemm_workspace_bytes(const fmoe_gemm_desc* d) {
+    GemmParams p;
+    int sel;
+    if (prepare_gemm(d, p, sel) || sel < 0 || !split_takes(d, p, sel)) return 0;
+    return kSplitHeaderBytes + (size_t)(compute_units() / kNumXcd * kNumXcd) * kSplitPieceBytes;
+}
+
+extern "C" int fmoe_grouped_gemm_ws(const fmoe_gemm_desc* d, void* workspace, size_t workspace_bytes, fmoe_stream_t stream_) {
     hipStream_t stream = (hipStream_t)stream_;
     GemmParams p;
     int sel;
     if (int rc = prepare_gemm(d, p, sel)) return rc;
     if (sel < 0) return FMOE_OK;
+    if (workspace && aligned16(workspace) && split_takes(d, p, sel) &&
+        workspace_bytes >= kSplitHeaderBytes + (size_t)(compute_units() / kNumXcd * kNumXcd) * kSplitPieceBytes) {
+        p.split_ws = (SplitWorkspace*)workspace;
+        return d->a_dtype == FMOE_E4M3 ? run_ring_split_fp8(p, d->epilogue, stream) : run_ring_split_bf16(p, d->epilogue, stream);
+    }
     if (p.direct)
         return run_gemm_direct(p, d->a_dtype == FMOE_E4M3 ? kDtE4m3 : d->a_dtype == FMOE_F32 ? kDtF32 : kDtBf16, d->epilogue, d->a_silu != 0,
                                stream);
@@ -250,6 +274,8 @@ extern "C" int fmoe_grouped_gemm(const fmoe_gemm_desc* d, fmoe_stream_t stream_)
     if (d->a_dtype == FMOE_F32) return run_gemm_f32(p, d->epilogue, d->a_silu != 0, sel, stream);
     return run_gemm_bf16(p, d->epilogue, d->a_silu != 0, sel, stream);
 }
+
+extern "C" int fmoe_grouped_gemm(const fmoe_gemm_desc* d, fmoe_stream_t stream_) { return fmoe_grouped_gemm_ws(d, nullptr, 0, stream_); }
 
 extern "C" int fmoe_grouped_gemm_plan(const fmoe_gemm_desc* d, int* plan) {
     FMOE_REQUIRE(plan != nullptr, "fmoe_grouped_gemm_plan: plan is NULL");

@@ -127,8 +127,13 @@ int launch_ring_cfg(GemmParams p, hipStream_t stream) {
         if (need < grid) grid = (int)need;
     }
     kern<<<(unsigned)grid, TL::NT, TL::LDS_BYTES, stream>>>(p);
+    if constexpr (TL::KSPLIT) split_reduce_kernel<FP8, EPI, MSC><<<8 * kSplitMost, 256, 0, stream>>>(p);
     return check_launch("fmoe_grouped_gemm");
 }
+
+// Ring kernels that cut the tiles of a part-filled last round along K (gemm_bf16_split.hip, gemm_fp8_split.hip).
+int run_ring_split_bf16(const GemmParams& p, int epilogue, hipStream_t stream);
+int run_ring_split_fp8(const GemmParams& p, int epilogue, hipStream_t stream);
 
 // Ring kernels for K that is no whole number of K-slice pairs (gemm_bf16_tail.hip, gemm_fp8_tail.hip).
 int run_ring_tail_bf16(const GemmParams& p, int epilogue, hipStream_t stream);
@@ -239,6 +244,22 @@ inline bool direct_pays(const GemmParams& p, int esize, bool swiglu) {
     const int row = p.K * esize;
     if (few) return tiles <= cus || (tiles <= 2 * cus && (esize == 1 || row <= 1664));
     return tall ? row >= 2048 && tiles <= 2 * cus : row > 512 && tiles <= cus;
+}
+
+// Where the tall ring cuts its last round of tiles along K, for a caller that brings the workspace: K long enough and the round, however the
+// experts share the rows, empty enough that the model of split_pieces gains 8 us at its fullest.  Only the row count is known here: the least
+// and the most tiles it allows have to lie in the same round.  us, whole tiles / cut: 16384 rows, 8 experts, 4096 -> 1024 (256 tiles and up
+// to 28) 171 / 135; 2000 rows, 8 experts, 4096 -> 1024 70.4 / 39.6; 4000, 4096 -> 512 70.4 / 38.3; 8000 70.6 / 49.9; 6540 rows, 5 experts, 3584
+// -> 2 x 1216, Zipf 160 / 122; 33000 rows, 16 experts, 4096 -> 1024 290 / 260.  Launches that may have fewer tiles than XCDs stay whole.
+inline bool split_pays(const GemmParams& p, int esize, int epilogue) {
+    const int bn = epilogue == FMOE_EPI_SWIGLU ? 128 : 256, pairs = (p.K * esize + 127) / 128;
+    const int64_t blocks = compute_units() / kNumXcd * kNumXcd, n_tiles = (p.N + bn - 1) / bn;
+    const int64_t least = (p.total_rows + 255) / 256 * n_tiles, most = most_row_tiles(p.total_rows, p.E, 256) * n_tiles;
+    if (blocks < kNumXcd || blocks > kSplitMost || pairs < 4 || most < kNumXcd || most >= ((int64_t)1 << 30)) return false;
+    const int64_t rounds = least / blocks, rest = most - rounds * blocks;
+    if (rest >= blocks || rest < 1) return false;
+    int cost;
+    return split_pieces((int)rest, pairs, (int)blocks, &cost) > 1 && 10 * pairs - cost >= 80;
 }
 
 // The 5-slot ring needs every byte of a 160 KB LDS, an even number of K-slices per tile,

@@ -11,6 +11,8 @@ namespace fmoe {
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 
+struct SplitWorkspace;
+
 struct GemmParams {
     const int64_t* offsets;
     const int64_t* row_index;
@@ -57,6 +59,7 @@ struct GemmParams {
     int64_t out_half;
     const uint8_t* a2;                  // second product a2 * b2 summed into the same output, or null
     int k_split;                        // ... whose contraction covers k in [k_split, K)
+    SplitWorkspace* split_ws;           // ring with tiles cut along K: where their sums meet, or null
 #ifdef FMOE_TRACE
     uint64_t* trace;                    // debug builds: per-tile time stamps of the ring kernel
 #endif

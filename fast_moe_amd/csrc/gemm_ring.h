@@ -3,6 +3,7 @@
 
 #include "gemm_deal.h"
 #include "gemm_epilogue.h"
+#include "gemm_split.h"
 
 namespace fmoe {
 
@@ -17,6 +18,7 @@ template <int BM_, int BN_, int WGM_, int WGN_, int NREG_, int AHEAD_ = 2>
 struct RingCfg {
     static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NREG = NREG_;
     static constexpr bool PAIR = NREG_ > 0;
+    static constexpr bool KSPLIT = false;
     static constexpr int AHEAD = AHEAD_;
     static constexpr int STAGES = PAIR ? 2 * AHEAD + 1 : 4;
     static constexpr int NW = WGM * WGN;
@@ -32,6 +34,12 @@ struct RingCfg {
     static constexpr int XI = BM / 16 / NW, WI = BN / 16 / NW;   // LDS-DMA instructions per lane per slice
     static_assert(BM % (16 * NW) == 0 && BN % (16 * NW) == 0, "DMA passes must be whole");
     static_assert(TM % 32 == 0 && TN % 64 == 0, "wave tile must hold whole 32x32 fragments, FN even");
+};
+
+// the 256 x 256 tiles with the last round's cut along K
+template <int NREG_>
+struct RingSplitCfg : RingCfg<256, 256, 2, 4, NREG_> {
+    static constexpr bool KSPLIT = true;
 };
 
 // One 16-byte-per-lane global -> LDS transfer from base + voff: a wave-uniform base in
@@ -87,9 +95,15 @@ __device__ __forceinline__ int uniform_lane(int v, int src_lane) {
 // columns both hold are masked out of the last pair's fragments, on both sides (a product of a real infinity with a
 // masked zero would be NaN).  No address beyond a row's end, no per-lane predicate in the DMA stream: the tail costs a
 // scalar select per pair and the masks of one double step per tile.
+//
+// TL::KSPLIT (tall tiles, no window): the tiles left after whole rounds of one per block are cut along K among the blocks (SplitDeal,
+// gemm_split.h).  A piece is the last thing a block computes; its sums go to the workspace as they lie in the accumulators, and
+// split_reduce_kernel adds the pieces of a tile and runs the epilogue.
 template <typename TL, bool FP8, int EPI, bool WTR = false, bool KWIN = false, bool XTR = false, bool MSC = false,
           bool KTAIL = false>
 __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmParams p) {
+    constexpr bool KSPLIT = TL::KSPLIT;
+    static_assert(!KSPLIT || (TL::PAIR && TL::BM == 256 && TL::BN == 256 && TL::NW == 8 && !KWIN && !XTR), "split tiles: tall paired ring");
     static_assert(!MSC || (FP8 && TL::PAIR && !KWIN && !WTR && !XTR), "MFMA-applied scales: e4m3 on the paired ring");
     static_assert(!WTR || (TL::PAIR && !FP8 && TL::BN == 256), "in-place N-contiguous weights: bf16, paired ring, 256-column tiles");
     static_assert(!KWIN || TL::PAIR, "contraction windows: paired ring");
@@ -240,7 +254,15 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     constexpr bool deal_groups = PAIR && BM >= 256;
     using Deal = TileDeal<tile_t, kNumXcd, kGroupM, !KWIN>;
     const Deal deal = deal_groups ? Deal(total_m, p.n_tiles, xcd, nslots) : Deal::contiguous(total_m, p.n_tiles, xcd);
-    const tile_t xcd_count = deal.count;
+    const int KT = KTAIL ? (p.K + 2 * BK - 1) / (2 * BK) * 2 : p.K / BK;
+    const SplitDeal split = KSPLIT ? SplitDeal(total_m * p.n_tiles, nslots, xcd, KT / 2) : SplitDeal();
+    if constexpr (KSPLIT) {
+        if (blockIdx.x == 0 && tid == 0) {      // what split_reduce_kernel has to do
+            p.split_ws->tiles = split.pieces > 1 ? split.rest : 0;
+            p.split_ws->pieces = split.pieces;
+        }
+    }
+    const tile_t xcd_count = KSPLIT ? split.count : deal.count;
     // tile numbers of the paired ring fit 31 bits (the launcher checks): divisions by the group
     // span are one scalar multiply by a constant the host prepared, no division sequence whose
     // per-lane pieces the compiler would keep (or spill) across the tile loop
@@ -253,11 +275,15 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         else return deal.run_base + j;
     };
 
-    const int KT = KTAIL ? (p.K + 2 * BK - 1) / (2 * BK) * 2 : p.K / BK;
     // KTAIL: columns at the start of the last pair that the pair before it has multiplied already
     const int tail_dup = KTAIL ? KT * BK - p.K : 0;
-    struct TileInfo { int expert; int nt; int64_t row0; int rows_valid; int64_t k_begin; int kt; int m0; int klen; };
-    auto locate = [&](tile_t logical) -> TileInfo {
+    struct TileInfo { int expert; int nt; int64_t row0; int rows_valid; int64_t k_begin; int kt; int m0; int klen; int k0; int piece; };
+    // j: number of the tile (KSPLIT: or piece) among the XCD's
+    auto locate = [&](tile_t j) -> TileInfo {
+        int piece = -1, part = 0;
+        tile_t logical;
+        if constexpr (KSPLIT) logical = split.tile(j, piece, part);
+        else logical = to_logical(j);
         const tile_t group = div_span(logical);
         const int first_m = (int)(group * kGroupM);
         const int gsize = total_m - first_m < kGroupM ? total_m - first_m : kGroupM;
@@ -319,6 +345,11 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         t.k_begin = 0;
         t.kt = KT;
         t.klen = 0;
+        t.k0 = 0;
+        t.piece = piece;
+        if constexpr (KSPLIT) {
+            if (piece >= 0) split.slices(part, KT / 2, t.k0, t.kt);
+        }
         if constexpr (!PAIR) t.m0 = 0;
         if constexpr (XTR) {
             // any row range; whole pairs of K-slices, at least two pairs
@@ -576,10 +607,10 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     // tile.  Item i lives in ring slot i % STAGES.  The issue side runs ahead of the compute
     // side and crosses tile boundaries on its own; it only needs the row pointers of the
     // tile it is in, the compute side only the TileInfo for the epilogue.
-    TileInfo cur = locate(to_logical(slot));   // tile being computed
+    TileInfo cur = locate(slot);   // tile being computed
     TileInfo nxt = cur;                     // tile after it (located one tile ahead)
     tile_t ilogical = slot;                 // its number among the XCD's tiles
-    int ikt = 0;                            // next K-slice to issue inside the issue tile
+    int ikt = KSPLIT ? cur.k0 : 0;          // next K-slice to issue inside the issue tile
     int issued = 0;                         // items issued so far
     int islot = 0;                          // issued % STAGES
     // The row indices of a tile are fetched two tiles ahead, before the epilogue of the tile in
@@ -647,7 +678,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     auto prefetch_next = [&]() {            // once per tile, early: locate the next tile and
         ilogical += nslots;                 // start fetching its source-row indices
         if (ilogical < xcd_count) {
-            nxt = locate(to_logical(ilogical));
+            nxt = locate(ilogical);
             fetch_rows(nxt, ridx_next);
         }
     };
@@ -820,7 +851,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             };
             // sched_barrier(0) pins the order "reads of the next block, then the MFMAs of this
             // one"; left alone the scheduler sinks the reads to just before their first use.
-            int kitem = 0;                  // number, inside the tile, of the item in slot cslot
+            int kitem = KSPLIT ? cur.k0 : 0;        // number, inside the tile, of the item in slot cslot
             // skip_wait (wave-uniform): the pair this step would wait for is known to have landed.  That
             // holds for the first step of every tile but the block's first: the pair was issued before
             // the previous epilogue, whose stores are all issued whatever their lanes' predicates
@@ -889,7 +920,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             // the issue side runs 2 * AHEAD items ahead: it enters the next tile that many items before the end;
             // the last two double steps hold the end of an XTR tile's window and mask it
             auto tile_steps = [&](auto half_c, auto act_c) __attribute__((always_inline)) {
-                const int tile_kt = KWIN ? cur.kt : KT;
+                const int tile_kt = KWIN || KSPLIT ? cur.kt : KT;
                 bool landed = tile_i > 0;       // the first step's pair landed before the previous epilogue's stores
                 for (int kt = 0; kt < tile_kt - 2 * TL::AHEAD; kt += 2) {
                     double_step(half_c, std::false_type{}, std::false_type{}, act_c, landed);
@@ -900,7 +931,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 }
                 FMOE_TRACE_STAMP(10);
                 enter_next();
-                ikt = 0;
+                ikt = KSPLIT ? nxt.k0 : 0;
 #pragma unroll
                 for (int j = 2; j < TL::AHEAD; ++j) {
                     double_step(half_c, std::false_type{}, std::false_type{}, act_c, landed);
@@ -914,7 +945,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 wait_vmcnt<2 * L * (TL::AHEAD - 1)>();
                 barrier();
             }
-            load_block(wfa, xfa, cslot, 0, 0, std::true_type{}, std::integral_constant<int, FM>{});
+            load_block(wfa, xfa, cslot, 0, KSPLIT ? cur.k0 : 0, std::true_type{}, std::integral_constant<int, FM>{});
             const bool sparse = SPARSE && cur.rows_valid <= p.short_tile_rows;
             if (wave < NW / 2) {
                 if (sparse) tile_steps(std::integral_constant<int, 0>{}, std::integral_constant<int, SPARSE ? ACT_SPARSE : FM>{});
@@ -952,9 +983,10 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             auto tail_mask = [&](i32x8& f, auto half_item_c) {
                 if constexpr (KTAIL) {
                     const int at = decltype(half_item_c)::value * BK + 32 * khalf;
+                    const int dup = KSPLIT && cur.k0 + cur.kt != KT ? 0 : tail_dup;      // (a piece that is not the last one)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const int keep = at + 8 * i < tail_dup ? 0 : -1;
+                        const int keep = at + 8 * i < dup ? 0 : -1;
                         f[2 * i] &= keep;
                         f[2 * i + 1] &= keep;
                     }
@@ -1070,7 +1102,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 cslot = s2;
             };
             auto tile_steps = [&](auto half_c, auto sparse_c) __attribute__((always_inline)) {
-                const int tile_kt = KWIN ? cur.kt : KT;
+                const int tile_kt = KWIN || KSPLIT ? cur.kt : KT;
                 // (whatever the compiler still counts as pending from the tile's set-up or the last
                 // epilogue, spill reloads and the row-index loads, is settled by the counted wait at
                 // the epilogue's end: left pending, such a wait lands inside this loop, where it
@@ -1085,7 +1117,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 }
                 FMOE_TRACE_STAMP(10);
                 enter_next();
-                ikt = 0;
+                ikt = KSPLIT ? nxt.k0 : 0;
 #pragma unroll
                 for (int j = 2; j < TL::AHEAD; ++j) {
                     double_step(half_c, std::false_type{}, sparse_c, landed);
@@ -1130,6 +1162,24 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         }
         if constexpr (MSC) mfma_results_guard();    // the last MFMAs' results are read by VALU code from here on
         FMOE_TRACE_STAMP(1);
+        if constexpr (KSPLIT) {
+            if (cur.piece >= 0) {       // the block's last
+                SplitTile* const info = p.split_ws->tile + cur.piece % split.rest;
+                if (cur.k0 == 0 && tid == 0) *info = SplitTile{__builtin_amdgcn_readfirstlane(cur.expert), cur.nt, (int)cur.row0, cur.rows_valid};
+                f32x4* const out = split_sums(p.split_ws, cur.piece, wave) + lane;
+#pragma unroll
+                for (int fm = 0; fm < FM; ++fm) {
+                    if ((ROW_IL ? (fm * 2 + wm) * 32 : wm * TM + fm * 32) >= cur.rows_valid) continue;
+#pragma unroll
+                    for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g)
+                            out[((fm * FN + fn) * 4 + g) * kWave] = f32x4{acc[fn][fm][4 * g], acc[fn][fm][4 * g + 1], acc[fn][fm][4 * g + 2],
+                                                                          acc[fn][fm][4 * g + 3]};
+                }
+                break;
+            }
+        }
         const TileInfo done = cur;
         cur = nxt;          // valid when another tile follows
         prefetch_next();    // nxt: the tile after that one; its row indices arrive during the epilogue

@@ -27,6 +27,8 @@ namespace {
 decltype(&fmoe_route_workspace_bytes) route_workspace_bytes;
 decltype(&fmoe_route_topk) c_route_topk;
 decltype(&fmoe_grouped_gemm) c_grouped_gemm;
+decltype(&fmoe_grouped_gemm_workspace_bytes) gemm_workspace_bytes;
+decltype(&fmoe_grouped_gemm_ws) c_grouped_gemm_ws;
 decltype(&fmoe_combine) c_combine;
 decltype(&fmoe_quant_rows_e4m3) c_quant_rows;
 decltype(&fmoe_gate_softmax) c_gate_softmax;
@@ -192,6 +194,14 @@ at::Tensor allocate(fmoe_gemm_desc& d, const at::Tensor& like) {
     return out;
 }
 
+// (the workspace may be handed out again as soon as the call is issued: what takes it runs behind the call on the stream)
+int gemm(const fmoe_gemm_desc& d, const at::Tensor& like, void* stream) {
+    const size_t bytes = gemm_workspace_bytes(&d);
+    if (!bytes) return c_grouped_gemm(&d, stream);
+    const at::Tensor workspace = empty({(int64_t)bytes}, at::kByte, like);
+    return c_grouped_gemm_ws(&d, workspace.data_ptr(), bytes, stream);
+}
+
 struct Combine {
     at::Tensor value, reverse, gates, gates_index;
     const void *value_data, *gates_data = nullptr;
@@ -304,7 +314,7 @@ PyObject* py_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int status = run([&] { return gemm_ok(g, d); },
                            [&] {
                                out = allocate(d, g.a);
-                               return c_grouped_gemm(&d, (void*)stream);
+                               return gemm(d, g.a, (void*)stream);
                            });
     if (raised(status, "fmoe_grouped_gemm")) return nullptr;
     return status == FMOE_OK ? wrap(out) : none();
@@ -487,8 +497,8 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 return rc;
             RECORD_USER_SCOPE("## expert_forward##");
             what = "fmoe_grouped_gemm";
-            if (const int rc = c_grouped_gemm(&up, (void*)stream)) return rc;
-            if (const int rc = c_grouped_gemm(&down, (void*)stream)) return rc;
+            if (const int rc = gemm(up, x, (void*)stream)) return rc;
+            if (const int rc = gemm(down, x, (void*)stream)) return rc;
             what = "fmoe_combine";
             return combine(merge, y, (void*)stream);
         });
@@ -499,12 +509,12 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // init(addresses of the C entry points, in the order of the pointers above)
 PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    int64_t v[7];
-    if (n != 7) {
-        PyErr_SetString(PyExc_TypeError, "init: seven addresses expected");
+    int64_t v[9];
+    if (n != 9) {
+        PyErr_SetString(PyExc_TypeError, "init: nine addresses expected");
         return nullptr;
     }
-    for (int i = 0; i < 7; ++i)
+    for (int i = 0; i < 9; ++i)
         if (!as_int(args[i], &v[i])) {
             PyErr_SetString(PyExc_TypeError, "init: addresses are integers");
             return nullptr;
@@ -515,7 +525,9 @@ PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
     c_combine = (decltype(c_combine))v[3];
     c_quant_rows = (decltype(c_quant_rows))v[4];
     c_gate_softmax = (decltype(c_gate_softmax))v[5];
-    last_error = (decltype(last_error))v[6];
+    gemm_workspace_bytes = (decltype(gemm_workspace_bytes))v[6];
+    c_grouped_gemm_ws = (decltype(c_grouped_gemm_ws))v[7];
+    last_error = (decltype(last_error))v[8];
     return none();
 }
 

@@ -23,6 +23,7 @@ EXPORTED_SYMBOLS = (
     "fmoe_version", "fmoe_last_error", "fmoe_route_workspace_bytes", "fmoe_route_topk",
     "fmoe_route_from_topk", "fmoe_quant_rows_e4m3",
     "fmoe_quant_rows_workspace_bytes", "fmoe_quant_rows_e4m3_ws", "fmoe_grouped_gemm", "fmoe_grouped_gemm_plan",
+    "fmoe_grouped_gemm_workspace_bytes", "fmoe_grouped_gemm_ws",
     "fmoe_combine",
     "fmoe_silu_mul", "fmoe_transpose_last2", "fmoe_jagged_transpose", "fmoe_segment_colsum",
     "fmoe_swiglu_bwd", "fmoe_combine_bwd", "fmoe_gather_rows", "fmoe_invert_index",
@@ -92,6 +93,10 @@ def load() -> ctypes.CDLL:
     lib.fmoe_quant_rows_e4m3_ws.argtypes = (lib.fmoe_quant_rows_e4m3.argtypes[:-1] + [c_void_p, c_size_t, c_void_p])
     lib.fmoe_grouped_gemm.restype = c_int
     lib.fmoe_grouped_gemm.argtypes = [POINTER(GemmDesc), c_void_p]
+    lib.fmoe_grouped_gemm_workspace_bytes.restype = c_size_t
+    lib.fmoe_grouped_gemm_workspace_bytes.argtypes = [POINTER(GemmDesc)]
+    lib.fmoe_grouped_gemm_ws.restype = c_int
+    lib.fmoe_grouped_gemm_ws.argtypes = [POINTER(GemmDesc), c_void_p, c_size_t, c_void_p]
     lib.fmoe_grouped_gemm_plan.restype = c_int
     lib.fmoe_grouped_gemm_plan.argtypes = [POINTER(GemmDesc), POINTER(c_int)]
     lib.fmoe_gate_softmax_pays.restype = c_int
@@ -138,7 +143,7 @@ def load() -> ctypes.CDLL:
 
 # what csrc/host_calls.cpp calls, in the order its init() takes the addresses
 HOST_ENTRY_POINTS = ("fmoe_route_workspace_bytes", "fmoe_route_topk", "fmoe_grouped_gemm", "fmoe_combine",
-                     "fmoe_quant_rows_e4m3", "fmoe_gate_softmax", "fmoe_last_error")
+                     "fmoe_quant_rows_e4m3", "fmoe_gate_softmax", "fmoe_grouped_gemm_workspace_bytes", "fmoe_grouped_gemm_ws", "fmoe_last_error")
 _host = None
 
 

@@ -501,7 +501,12 @@ def grouped_gemm(offsets: torch.Tensor, a: torch.Tensor, b: torch.Tensor, *, tot
             d.a_silu = 1
     if plan_only:
         return gemm_plan(d)
-    rc = lib.fmoe_grouped_gemm(ctypes.byref(d), _stream(a))
+    ws_bytes = lib.fmoe_grouped_gemm_workspace_bytes(ctypes.byref(d))
+    if ws_bytes:
+        ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=a.device)
+        rc = lib.fmoe_grouped_gemm_ws(ctypes.byref(d), ws.data_ptr(), ws_bytes, _stream(a))
+    else:
+        rc = lib.fmoe_grouped_gemm(ctypes.byref(d), _stream(a))
     _lib.check(rc, "fmoe_grouped_gemm")
     return out
 

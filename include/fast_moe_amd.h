@@ -318,6 +318,14 @@ enum fmoe_gemm_plan {
 };
 int fmoe_grouped_gemm_plan(const fmoe_gemm_desc* desc, int* plan);
 
+/*
+ * fmoe_grouped_gemm with a scratch buffer of the caller (16-byte aligned, fmoe_grouped_gemm_workspace_bytes bytes; 0: none is used): the
+ * tiles that would leave most CUs idle in a last round are cut along K, their fp32 sums meet in the buffer and are added in
+ * the order of K.  The results differ from fmoe_grouped_gemm's by the grouping of those sums.
+ */
+size_t fmoe_grouped_gemm_workspace_bytes(const fmoe_gemm_desc* desc);
+int fmoe_grouped_gemm_ws(const fmoe_gemm_desc* desc, void* workspace, size_t workspace_bytes, fmoe_stream_t stream);
+
 /* ------------------------------------------------------------------ combine */
 
 /*

@@ -1481,3 +1481,70 @@ def test_ring_kernel_writes_every_tile(row_tiles, N):
         ref = a[rows].float() @ w[e].float().t()
         mag = a[rows].float().abs() @ w[e].float().abs().t()
         assert ((out[rows].float() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * 2.0 ** -16).all()
+
+
+@pytest.mark.parametrize("lens,K,N,layout,epi", [
+    ([2048] * 7 + [2049], 4096, 1024, "nk", 0),              # a whole round and four tiles of a row
+    ([520, 0, 500, 600, 400, 33], 4096, 904, "nk", 1), ([520, 0, 500, 600, 400, 33], 4096 + 72, 904, "nk", 0),     # a tail of K
+    ([30] * 4 + [650, 250], 4096, 1096, "nk", 2), ([300, 200, 400, 100], 4096, 712, "kn", 2), ([300, 200, 400, 100], 2600, 1224, "kn", 0),
+    ([130] * 70, 6208, 192, "nk", 0),                         # more than 64 experts
+])
+@pytest.mark.parametrize("dtype", ["bf16", "fp8", "pow2"])
+@pytest.mark.parametrize("extras", [False, True])
+def test_ring_kernel_cuts_its_last_round_along_k(lens, K, N, layout, epi, dtype, extras):
+    """Against the call without a workspace, which walks every tile's K alone: the same but for the grouping of fp32 sums (2 x K x 2^-24 of
+    the sum of |products|) and the roundings to bf16 behind them, which the bound of assert_bf16_close holds; the same bits twice.  extras: gathered
+    rows, bias and, with SwiGLU, the two pre-activations."""
+    import ctypes
+
+    from fast_moe_amd.kernels.hip import _lib, ops
+    if dtype != "bf16" and (layout == "kn" or len(lens) > 64):
+        pytest.skip("e4m3: weights with k contiguous, up to 64 experts")
+    if dtype != "bf16":
+        K = (2 * K + 127) // 128 * 128
+    E, rows = len(lens), sum(lens)
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    off = torch.tensor([0, *torch.tensor(lens).cumsum(0)]).cuda()
+    T = (rows + 1) // 2 if extras else rows
+    x = (torch.randn(T, K, generator=g, device="cuda") * 0.5).to(BF16)
+    ws = [(torch.randn(*((E, K, N) if layout == "kn" else (E, N, K)), generator=g, device="cuda") * K ** -0.5).to(BF16) for _ in range(2)]
+    views = [w if layout == "kn" else w.permute(0, 2, 1) for w in ws]
+    index = torch.randint(0, 2 * T, (rows,), generator=g, device="cuda") if extras else None
+    bias = [torch.randn(E, N, generator=g, device="cuda").to(BF16) for _ in range(2)] if extras else [None, None]
+    swiglu = epi == _lib.EPI_SWIGLU
+    aux = tuple(torch.zeros(rows, N, dtype=BF16, device="cuda") for _ in range(2)) if extras and swiglu and dtype == "bf16" else None
+    kw = dict(total_rows=rows, row_index=index, index_div=2 if extras else 1, bias=bias[0], epilogue=epi, aux=aux)
+    if swiglu:
+        kw.update(b2=views[1], bias2=bias[1])
+    args = (x, views[0])
+    if dtype != "bf16":
+        qx, sx = ops.quant_rows_fp8(x)
+        qw = [ops.quant_rows_fp8(w) for w in ws]
+        kw.update(a_scale=sx, b_scale=qw[0][1], scales_pow2=dtype == "pow2")
+        if swiglu:
+            kw.update(b2=qw[1][0].permute(0, 2, 1), b2_scale=qw[1][1])
+        args = (qx, qw[0][0].permute(0, 2, 1))
+    ran = kernels_run(lambda: ops.grouped_gemm(off, *args, **kw))
+    out = ops.grouped_gemm(off, *args, **kw)
+    parts = [t.clone() for t in (out, *(aux or ()))]
+    again = ops.grouped_gemm(off, *args, **kw)
+    assert torch.equal(out, again)
+    assert [n.split("<")[0].split("::")[-1] for n in ran] == ["grouped_gemm_ring_kernel", "split_reduce_kernel"], ran
+
+    # the same call through Python alone, with no workspace
+    lib, host = _lib.load(), _lib.host()
+    class NoWorkspace:
+        def __getattr__(self, name):
+            return (lambda d: 0) if name == "fmoe_grouped_gemm_workspace_bytes" else getattr(lib, name)
+    class Declines:
+        def __getattr__(self, name):
+            return lambda *a: None
+    try:
+        _lib._lib, _lib._host = NoWorkspace(), Declines()
+        for t in aux or ():
+            t.zero_()
+        ref = ops.grouped_gemm(off, *args, **kw)
+    finally:
+        _lib._lib, _lib._host = lib, host
+    for got, want in zip(parts, (ref, *(aux or ()))):
+        assert_bf16_close(got, want.float(), rtol=1.6e-2, atol=4e-3, what="split")
