@@ -1,4 +1,4 @@
-// The host side of the forward operators as one native call each: argument checks, output allocation, stride marshalling and
+// The host side of the operators, forward and backward, as one native call each: argument checks, output allocation, stride marshalling and
 // the launch, for the calls a forward pass makes.
 //
 // What it is for: a pass over a few tokens is bound by the host (64 tokens, 8 experts, 128 -> 256 -> 128: seven launches that
@@ -32,6 +32,16 @@ decltype(&fmoe_grouped_gemm_ws) c_grouped_gemm_ws;
 decltype(&fmoe_combine) c_combine;
 decltype(&fmoe_quant_rows_e4m3) c_quant_rows;
 decltype(&fmoe_gate_softmax) c_gate_softmax;
+decltype(&fmoe_grouped_gemm_plan) c_gemm_plan;
+decltype(&fmoe_combine_bwd) c_combine_bwd;
+decltype(&fmoe_segment_colsum) c_segment_colsum;
+decltype(&fmoe_swiglu_bwd) c_swiglu_bwd;
+decltype(&fmoe_silu_mul) c_silu_mul;
+decltype(&fmoe_gather_rows) c_gather_rows;
+decltype(&fmoe_invert_index) c_invert_index;
+decltype(&fmoe_gate_l1_bwd) c_gate_l1_bwd;
+decltype(&fmoe_weight_grad) c_weight_grad;
+decltype(&fmoe_weight_grad_pays) weight_grad_pays;
 decltype(&fmoe_last_error) last_error;
 
 constexpr int64_t kSlackRows = 128;      // ops.SLACK_ROWS
@@ -121,6 +131,7 @@ struct GemmArgs {
     const int64_t *offsets_data = nullptr, *row_index_data = nullptr;
     const void* a_data = nullptr;
     int64_t a_rows = 0;
+    bool n_contiguous = false;      // weights with n contiguous are taken
 };
 
 // Checks the operands and fills everything of the descriptor but the output.
@@ -140,7 +151,6 @@ bool gemm_ok(const GemmArgs& g, fmoe_gemm_desc& d) {
     if (g.b2.defined() &&
         (g.b2.scalar_type() != b.scalar_type() || g.b2.sizes() != b.sizes() || g.b2.strides() != b.strides()))
         return false;
-    if (b.stride(2) == 1 && b.stride(1) != 1) return false;     // ops.grouped_gemm asks for the plan of these first
     for (const at::Tensor* t : {&g.bias, &g.bias2})
         if (t->defined() &&
             (t->scalar_type() != out_dtype || t->dim() != 2 || t->size(0) != E || t->size(1) != N || t->stride(1) != 1))
@@ -183,6 +193,14 @@ bool gemm_ok(const GemmArgs& g, fmoe_gemm_desc& d) {
     d.bias_stride_e = g.bias.defined() ? g.bias.stride(0) : g.bias2.defined() ? g.bias2.stride(0) : 0;
     d.epilogue = (int32_t)g.epilogue;
     d.out_dtype = dtype_code(out_dtype);
+    // ... unless only the element-load kernel would read them in place: ops.grouped_gemm copies them first
+    if (b.stride(2) == 1 && b.stride(1) != 1 && !g.n_contiguous) return false;
+    if (b.stride(2) == 1 && b.stride(1) != 1 && K % 16 == 0 && N % 8 == 0 && g.total_rows * N >= (1 << 22)) {
+        d.out = (void*)(uintptr_t)256;      // (where the allocator would put it, as far as alignment goes)
+        d.out_stride_row = N;
+        int plan;
+        if (c_gemm_plan(&d, &plan) != FMOE_OK || plan == FMOE_PLAN_ELEMENT) return false;
+    }
     return true;
 }
 
@@ -295,10 +313,12 @@ PyObject* py_route_topk(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // (offsets, a, b, total_rows, row_index, index_div, bias, b2, bias2, epilogue, a_scale, b_scale, b2_scale, pow2, stream)
+template <bool N_CONTIGUOUS>
 PyObject* py_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (n != 15) return none();
     GemmArgs g;
+    g.n_contiguous = N_CONTIGUOUS;
     int64_t stream;
     g.offsets = gpu_tensor(args[0]);
     g.a = gpu_tensor(args[1]);
@@ -507,27 +527,252 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// ---- the backward pass's operators, as ops.py issues them
+at::Tensor empty_rows(int64_t rows, int64_t cols, at::ScalarType dtype, const at::Tensor& like) {
+    return empty({rows + kSlackRows, cols}, dtype, like).narrow(0, 0, rows);
+}
+bool float_matrix(const at::Tensor& t) {
+    return (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16) && t.dim() == 2 && t.size(1) > 0 && t.stride(1) == 1;
+}
+// rows of t's pitch that its storage holds behind its last (ops.slack_rows)
+int64_t slack_rows(const at::Tensor& t) {
+    if (t.stride(0) < t.size(1) || t.stride(0) < 1) return 0;
+    const int64_t have = (int64_t)(t.storage().nbytes() / t.element_size()) - t.storage_offset();
+    const int64_t rows = (have - t.size(1)) / t.stride(0) + 1 - t.size(0);
+    return rows > 0 ? rows : 0;
+}
+PyObject* wrap_or_none(const at::Tensor& t) { return t.defined() ? wrap(t) : none(); }
+
+// (dy [T, D], value [T*K, D] or None, token_index, K, gates or None, gates_index or None, need_gate_grad, stream) -> (d_value, d_gates)
+PyObject* py_combine_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 8) return none();
+    const at::Tensor dy = gpu_tensor(args[0]), index = gpu_tensor(args[2]);
+    at::Tensor value, gates, gates_index, d_value, d_gates;
+    int64_t K, need, stream;
+    if (!dy.defined() || !index.defined() || !optional_tensor(args[1], &value) || !as_int(args[3], &K) || !optional_tensor(args[4], &gates) ||
+        !optional_tensor(args[5], &gates_index) || !as_int(args[6], &need) || !as_int(args[7], &stream))
+        return none();
+    const int status = run(
+        [&] {
+            if (!float_matrix(dy) || !dy.is_contiguous() || K < 1 || K > INT32_MAX) return false;
+            const int64_t R = dy.size(0) * K;
+            if (R < 1 || !same_device(dy, index) || !same_device(dy, value) || !same_device(dy, gates) || !same_device(dy, gates_index) ||
+                !i64_list(index, R))
+                return false;
+            if (gates.defined() && (dtype_code(gates.scalar_type()) < 0 || gates.scalar_type() == at::kFloat8_e4m3fn || gates.dim() != 2 ||
+                                    gates.numel() != R || (gates_index.defined() && !i64_list(gates_index, R))))
+                return false;
+            return !need || (value.defined() && float_matrix(value) && value.scalar_type() == dy.scalar_type() && value.size(0) == R &&
+                             value.size(1) == dy.size(1));
+        },
+        [&] {
+            const int64_t T = dy.size(0), D = dy.size(1);
+            if (need) d_gates = at::zeros({T * K}, at::TensorOptions(dy.device()).dtype(at::kFloat));
+            d_value = empty_rows(T * K, D, dy.scalar_type(), dy);
+            const bool g = gates.defined();
+            return c_combine_bwd(dy.data_ptr(), need ? value.data_ptr() : nullptr, dtype_code(dy.scalar_type()), T, (int)K, D,
+                                 need ? value.stride(0) : D, index.data_ptr<int64_t>(), g ? gates.data_ptr() : nullptr,
+                                 g ? dtype_code(gates.scalar_type()) : FMOE_F32, g ? gates.size(1) : 1, g ? gates.stride(0) : 1,
+                                 g ? gates.stride(1) : 1, g && gates_index.defined() ? gates_index.data_ptr<int64_t>() : nullptr,
+                                 d_value.data_ptr(), need ? d_gates.data_ptr<float>() : nullptr, (void*)stream);
+        });
+    if (raised(status, "fmoe_combine_bwd")) return nullptr;
+    return status == FMOE_OK ? Py_BuildValue("(NN)", wrap(d_value), wrap_or_none(d_gates)) : none();
+    END_HANDLE_TH_ERRORS
+}
+
+// (src [R, C], offsets, stream) -> [E, C]
+PyObject* py_segment_colsum(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 3) return none();
+    const at::Tensor src = gpu_tensor(args[0]), offsets = gpu_tensor(args[1]);
+    at::Tensor out;
+    int64_t stream;
+    if (!src.defined() || !offsets.defined() || !as_int(args[2], &stream)) return none();
+    const int status = run([&] { return float_matrix(src) && same_device(src, offsets) && offsets.numel() >= 2 && i64_list(offsets, offsets.numel()); },
+                           [&] {
+                               const int64_t E = offsets.numel() - 1;
+                               out = empty({E, src.size(1)}, src.scalar_type(), src);
+                               return c_segment_colsum(src.data_ptr(), dtype_code(src.scalar_type()), src.size(0), src.size(1), src.stride(0),
+                                                       offsets.data_ptr<int64_t>(), (int)E, out.data_ptr(), (void*)stream);
+                           });
+    if (raised(status, "fmoe_segment_colsum")) return nullptr;
+    return status == FMOE_OK ? wrap(out) : none();
+    END_HANDLE_TH_ERRORS
+}
+
+// (g [R, C], u or None, dh, joint, stream) -> (dg, du)
+PyObject* py_swiglu_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 5) return none();
+    const at::Tensor g = gpu_tensor(args[0]), dh = gpu_tensor(args[2]);
+    at::Tensor u, dg, du;
+    int64_t joint, stream;
+    if (!g.defined() || !dh.defined() || !optional_tensor(args[1], &u) || !as_int(args[3], &joint) || !as_int(args[4], &stream)) return none();
+    const int status = run(
+        [&] {
+            for (const at::Tensor* t : {&g, &dh, (const at::Tensor*)&u})
+                if (t->defined() && (!float_matrix(*t) || !t->is_contiguous() || t->scalar_type() != g.scalar_type() || t->sizes() != g.sizes() ||
+                                     !same_device(g, *t)))
+                    return false;
+            return g.numel() > 0;
+        },
+        [&] {
+            const int64_t rows = g.size(0), cols = g.size(1);
+            int64_t pitch = 0;
+            if (joint && u.defined() && g.scalar_type() == at::kBFloat16 && cols % 8 == 0) {
+                const at::Tensor both = empty_rows(rows, 2 * cols, g.scalar_type(), g);
+                dg = both.narrow(1, 0, cols);
+                du = both.narrow(1, cols, cols);
+                pitch = 2 * cols;
+            } else {
+                dg = empty_rows(rows, cols, g.scalar_type(), g);
+                if (u.defined()) du = empty_rows(rows, cols, g.scalar_type(), g);
+            }
+            return c_swiglu_bwd(g.data_ptr(), u.defined() ? u.data_ptr() : nullptr, dh.data_ptr(), dg.data_ptr(),
+                                du.defined() ? du.data_ptr() : nullptr, dtype_code(g.scalar_type()), g.numel(), cols, pitch, (void*)stream);
+        });
+    if (raised(status, "fmoe_swiglu_bwd")) return nullptr;
+    return status == FMOE_OK ? Py_BuildValue("(NN)", wrap(dg), wrap_or_none(du)) : none();
+    END_HANDLE_TH_ERRORS
+}
+
+// (a [R, C], with_slack, stream) -> silu(a)
+PyObject* py_silu(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 3) return none();
+    const at::Tensor a = gpu_tensor(args[0]);
+    at::Tensor out;
+    int64_t slack, stream;
+    if (!a.defined() || !as_int(args[1], &slack) || !as_int(args[2], &stream)) return none();
+    const int status = run([&] { return float_matrix(a) && a.is_contiguous() && a.numel() > 0; },
+                           [&] {
+                               out = slack ? empty_rows(a.size(0), a.size(1), a.scalar_type(), a) : empty(a.sizes(), a.scalar_type(), a);
+                               return c_silu_mul(a.data_ptr(), nullptr, out.data_ptr(), dtype_code(a.scalar_type()), a.numel(), (void*)stream);
+                           });
+    if (raised(status, "fmoe_silu_mul")) return nullptr;
+    return status == FMOE_OK ? wrap(out) : none();
+    END_HANDLE_TH_ERRORS
+}
+
+// (src [T, C], index, index_div, stream) -> src[index / index_div] with slack rows
+PyObject* py_gather_rows(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 4) return none();
+    const at::Tensor src = gpu_tensor(args[0]), index = gpu_tensor(args[1]);
+    at::Tensor out;
+    int64_t div, stream;
+    if (!src.defined() || !index.defined() || !as_int(args[2], &div) || !as_int(args[3], &stream)) return none();
+    const int status = run([&] { return float_matrix(src) && same_device(src, index) && div >= 1 && div <= INT32_MAX && i64_list(index, index.numel()); },
+                           [&] {
+                               const int64_t es = src.element_size(), rows = index.numel();
+                               out = empty_rows(rows, src.size(1), src.scalar_type(), src);
+                               return c_gather_rows(src.data_ptr(), src.size(0), src.size(1) * es, src.stride(0) * es, index.data_ptr<int64_t>(),
+                                                    (int)div, rows, out.data_ptr(), out.stride(0) * es, (void*)stream);
+                           });
+    if (raised(status, "fmoe_gather_rows")) return nullptr;
+    return status == FMOE_OK ? wrap(out) : none();
+    END_HANDLE_TH_ERRORS
+}
+
+// (index [T, K], stream) -> reverse [T, K]
+PyObject* py_invert_index(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 2) return none();
+    const at::Tensor index = gpu_tensor(args[0]);
+    at::Tensor out;
+    int64_t stream;
+    if (!index.defined() || !as_int(args[1], &stream)) return none();
+    const int status = run([&] { return index.dim() == 2 && i64_list(index, index.numel()) && index.size(1) <= INT32_MAX; },
+                           [&] {
+                               out = empty(index.sizes(), at::kLong, index);
+                               return c_invert_index(index.data_ptr<int64_t>(), index.size(0), (int)index.size(1), out.data_ptr<int64_t>(), (void*)stream);
+                           });
+    if (raised(status, "fmoe_invert_index")) return nullptr;
+    return status == FMOE_OK ? wrap(out) : none();
+    END_HANDLE_TH_ERRORS
+}
+
+// (scores [T, E], topk_idx [T, K], d_gates [T, K], stream) -> d_scores
+PyObject* py_gate_l1_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 4) return none();
+    const at::Tensor scores = gpu_tensor(args[0]), topk = gpu_tensor(args[1]), d_gates = gpu_tensor(args[2]);
+    at::Tensor out;
+    int64_t stream;
+    if (!scores.defined() || !topk.defined() || !d_gates.defined() || !as_int(args[3], &stream)) return none();
+    const int status = run(
+        [&] {
+            return float_matrix(scores) && scores.is_contiguous() && d_gates.scalar_type() == scores.scalar_type() && d_gates.is_contiguous() &&
+                   topk.dim() == 2 && i64_list(topk, topk.numel()) && d_gates.sizes() == topk.sizes() && topk.size(0) == scores.size(0) &&
+                   same_device(scores, topk) && same_device(scores, d_gates) && scores.size(1) <= INT32_MAX && topk.size(1) <= INT32_MAX;
+        },
+        [&] {
+            out = empty(scores.sizes(), scores.scalar_type(), scores);
+            return c_gate_l1_bwd(scores.data_ptr(), dtype_code(scores.scalar_type()), scores.size(0), (int)scores.size(1), (int)topk.size(1),
+                                 topk.data_ptr<int64_t>(), d_gates.data_ptr(), out.data_ptr(), (void*)stream);
+        });
+    if (raised(status, "fmoe_gate_l1_bwd")) return nullptr;
+    return status == FMOE_OK ? wrap(out) : none();
+    END_HANDLE_TH_ERRORS
+}
+
+// (dout [R, N], rows [R, K_in], offsets, halves, stream) -> [E, N, K_in], or two [E, N/2, K_in]: the calls fmoe_weight_grad takes
+// (ops.jagged_weight_grad; its other route is left to it)
+PyObject* py_weight_grad(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 5) return none();
+    const at::Tensor a = gpu_tensor(args[0]), b = gpu_tensor(args[1]), offsets = gpu_tensor(args[2]);
+    at::Tensor out, out2;
+    int64_t halves, stream;
+    if (!a.defined() || !b.defined() || !offsets.defined() || !as_int(args[3], &halves) || !as_int(args[4], &stream)) return none();
+    const int status = run(
+        [&] {
+            if (!float_matrix(a) || !float_matrix(b) || a.scalar_type() != b.scalar_type() || a.size(0) != b.size(0) || !same_device(a, b) ||
+                !same_device(a, offsets) || offsets.numel() < 2 || !i64_list(offsets, offsets.numel()))
+                return false;
+            const bool bf16 = a.scalar_type() == at::kBFloat16;
+            const int64_t R = a.size(0), N = a.size(1), Kin = b.size(1), E = offsets.numel() - 1, chunk = bf16 ? 8 : 4;
+            if (R < 1 || N % chunk || Kin % chunk || a.stride(0) % chunk || b.stride(0) % chunk || a.stride(0) < N || b.stride(0) < Kin ||
+                (uintptr_t)a.data_ptr() % 16 || (uintptr_t)b.data_ptr() % 16 || E > INT32_MAX || Kin > INT32_MAX || E * N > INT32_MAX ||
+                (halves && N % 64))
+                return false;
+            if (bf16 && (slack_rows(a) < kSlackRows || slack_rows(b) < kSlackRows)) return false;
+            return (bf16 && R < 128) || weight_grad_pays(dtype_code(a.scalar_type()), (int)E, (int)N, (int)Kin, R) != 0;
+        },
+        [&] {
+            const int64_t E = offsets.numel() - 1, N = a.size(1), Kin = b.size(1);
+            out = empty({E, halves ? N / 2 : N, Kin}, a.scalar_type(), a);
+            if (halves) out2 = empty({E, N / 2, Kin}, a.scalar_type(), a);
+            return c_weight_grad(a.data_ptr(), b.data_ptr(), dtype_code(a.scalar_type()), (int)E, (int)N, (int)Kin, a.size(0), a.stride(0),
+                                 b.stride(0), offsets.data_ptr<int64_t>(), out.data_ptr(), halves ? out2.data_ptr() : nullptr, (void*)stream);
+        });
+    if (raised(status, "fmoe_weight_grad")) return nullptr;
+    if (status != FMOE_OK) return none();
+    return halves ? Py_BuildValue("(NN)", wrap(out), wrap(out2)) : wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
 // init(addresses of the C entry points, in the order of the pointers above)
 PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    int64_t v[9];
-    if (n != 9) {
-        PyErr_SetString(PyExc_TypeError, "init: nine addresses expected");
+    void** const entry[] = {(void**)&route_workspace_bytes, (void**)&c_route_topk, (void**)&c_grouped_gemm, (void**)&c_combine,
+                            (void**)&c_quant_rows, (void**)&c_gate_softmax, (void**)&gemm_workspace_bytes, (void**)&c_grouped_gemm_ws,
+                            (void**)&c_gemm_plan, (void**)&c_combine_bwd, (void**)&c_segment_colsum, (void**)&c_swiglu_bwd,
+                            (void**)&c_silu_mul, (void**)&c_gather_rows, (void**)&c_invert_index, (void**)&c_gate_l1_bwd,
+                            (void**)&c_weight_grad, (void**)&weight_grad_pays, (void**)&last_error};
+    constexpr Py_ssize_t count = sizeof(entry) / sizeof(entry[0]);
+    if (n != count) {
+        PyErr_Format(PyExc_TypeError, "init: %d addresses expected", (int)count);
         return nullptr;
     }
-    for (int i = 0; i < 9; ++i)
+    int64_t v[count];
+    for (int i = 0; i < count; ++i)
         if (!as_int(args[i], &v[i])) {
             PyErr_SetString(PyExc_TypeError, "init: addresses are integers");
             return nullptr;
         }
-    route_workspace_bytes = (decltype(route_workspace_bytes))v[0];
-    c_route_topk = (decltype(c_route_topk))v[1];
-    c_grouped_gemm = (decltype(c_grouped_gemm))v[2];
-    c_combine = (decltype(c_combine))v[3];
-    c_quant_rows = (decltype(c_quant_rows))v[4];
-    c_gate_softmax = (decltype(c_gate_softmax))v[5];
-    gemm_workspace_bytes = (decltype(gemm_workspace_bytes))v[6];
-    c_grouped_gemm_ws = (decltype(c_grouped_gemm_ws))v[7];
-    last_error = (decltype(last_error))v[8];
+    for (int i = 0; i < count; ++i) *entry[i] = (void*)v[i];
     return none();
 }
 
@@ -535,9 +780,18 @@ PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyMethodDef methods[] = {
     FASTCALL("init", py_init),
     FASTCALL("route_topk", py_route_topk),
-    FASTCALL("grouped_gemm", py_grouped_gemm),
+    FASTCALL("grouped_gemm", py_grouped_gemm<false>),
+    FASTCALL("grouped_gemm_n", py_grouped_gemm<true>),
     FASTCALL("combine", py_combine),
     FASTCALL("quant_rows", py_quant_rows),
+    FASTCALL("combine_bwd", py_combine_bwd),
+    FASTCALL("segment_colsum", py_segment_colsum),
+    FASTCALL("swiglu_bwd", py_swiglu_bwd),
+    FASTCALL("silu", py_silu),
+    FASTCALL("gather_rows", py_gather_rows),
+    FASTCALL("invert_index", py_invert_index),
+    FASTCALL("gate_l1_bwd", py_gate_l1_bwd),
+    FASTCALL("weight_grad", py_weight_grad),
     FASTCALL("gate_softmax", py_gate_softmax),
     FASTCALL("mlp_forward", py_mlp_forward),
     {nullptr, nullptr, 0, nullptr},

@@ -143,14 +143,18 @@ def load() -> ctypes.CDLL:
 
 # what csrc/host_calls.cpp calls, in the order its init() takes the addresses
 HOST_ENTRY_POINTS = ("fmoe_route_workspace_bytes", "fmoe_route_topk", "fmoe_grouped_gemm", "fmoe_combine",
-                     "fmoe_quant_rows_e4m3", "fmoe_gate_softmax", "fmoe_grouped_gemm_workspace_bytes", "fmoe_grouped_gemm_ws", "fmoe_last_error")
+                     "fmoe_quant_rows_e4m3", "fmoe_gate_softmax", "fmoe_grouped_gemm_workspace_bytes", "fmoe_grouped_gemm_ws",
+                     "fmoe_grouped_gemm_plan", "fmoe_combine_bwd", "fmoe_segment_colsum", "fmoe_swiglu_bwd", "fmoe_silu_mul",
+                     "fmoe_gather_rows", "fmoe_invert_index", "fmoe_gate_l1_bwd", "fmoe_weight_grad", "fmoe_weight_grad_pays",
+                     "fmoe_last_error")
 _host = None
 
 
 class _Declines:
     """In the place of the extension module where that does not load: every call is left to the Python code in ops.py."""
 
-    route_topk = grouped_gemm = combine = quant_rows = gate_softmax = mlp_forward = staticmethod(lambda *args: None)
+    def __getattr__(self, name):
+        return lambda *args: None
 
 
 def host():

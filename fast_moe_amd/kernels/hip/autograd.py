@@ -122,11 +122,11 @@ def _input_grad(drow_list, weights, offsets, reverse_index) -> torch.Tensor:
         value = ops.grouped_gemm_sum2(offsets, drow_list[0], w0, drow_list[1], w1, total_rows=R)
         if value is not None:
             return ops.combine(value, reverse_index)
+    if n == 1:
+        return ops.combine(ops.input_grad_gemm(offsets, drow_list[0], weights[0].permute(0, 2, 1)), reverse_index)
     value = torch.empty((n * R, Kin), dtype=drow_list[0].dtype, device=drow_list[0].device)
     for i, (d, w) in enumerate(zip(drow_list, weights)):
         ops.grouped_gemm(offsets, d, w.permute(0, 2, 1), total_rows=R, out=value[i * R:(i + 1) * R])
-    if n == 1:
-        return ops.combine(value, reverse_index)
     rev = torch.cat([reverse_index + i * R for i in range(n)], dim=1)
     return ops.combine(value, rev)
 
@@ -400,7 +400,7 @@ class SiluJaggedBmmCombine(torch.autograd.Function):
                                         need_gate_grad=need_g)
         d_jagged = d_w = d_b = d_g = None
         if need[1]:
-            d_h = ops.grouped_gemm(offsets, d_bmm, weight.permute(0, 2, 1), total_rows=d_bmm.shape[0])
+            d_h = ops.input_grad_gemm(offsets, d_bmm, weight.permute(0, 2, 1))
             d_jagged = ops.swiglu_bwd(jagged, None, d_h)[0] if ctx.has_silu else d_h
         if need[2]:
             if silu_rows is not None:

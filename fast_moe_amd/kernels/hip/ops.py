@@ -294,6 +294,9 @@ def jagged_weight_grad(dout: torch.Tensor, a_rows: torch.Tensor, offsets: torch.
     with a_stride_k (bf16).  Returns None when the operands do not qualify (dtype, alignment, no slack behind
     them): the caller then takes the route over transposed copies.  ``halves``: dout holds the row gradients of
     two matrices side by side; the result is two tensors [E, N/2, K_in] (fmoe_gemm_desc.out2)."""
+    dw = _lib.host().weight_grad(dout, a_rows, offsets, int(halves), _stream(dout))
+    if dw is not None:
+        return dw
     if dout.dtype not in _DTYPE_CODE or a_rows.dtype != dout.dtype or dout.shape[0] != a_rows.shape[0]:
         return None
     R, N = dout.shape
@@ -511,6 +514,13 @@ def grouped_gemm(offsets: torch.Tensor, a: torch.Tensor, b: torch.Tensor, *, tot
     return out
 
 
+def input_grad_gemm(offsets: torch.Tensor, d: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """``grouped_gemm`` of row gradients with the transposed weights [E, N, K_in] of a forward call: n contiguous for the
+    layers' storage, which the native call takes here."""
+    res = _lib.host().grouped_gemm_n(offsets, d, weight, d.shape[0], None, 1, None, None, None, EPI_NONE, None, None, None, 0, _stream(d))
+    return grouped_gemm(offsets, d, weight, total_rows=d.shape[0]) if res is None else res
+
+
 def grouped_gemm_sum2(offsets: torch.Tensor, a: torch.Tensor, b: torch.Tensor, a2: torch.Tensor,
                       b2: torch.Tensor, *, total_rows: int,
                       out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
@@ -598,6 +608,9 @@ def combine(value: torch.Tensor, reverse_index: torch.Tensor, gates: Optional[to
 def gather_rows(src: torch.Tensor, index: torch.Tensor, index_div: int = 1) -> torch.Tensor:
     """``src[index // index_div]`` for a 2-D src with contiguous rows of whole 16-byte chunks
     (fmoe_gather_rows); the result has slack rows behind it."""
+    out = _lib.host().gather_rows(src, index, index_div, _stream(src))
+    if out is not None:
+        return out
     dev = _need_cuda("gather_rows", src, index)
     if src.ndim != 2:
         raise ValueError("gather_rows: src must be 2-D")
@@ -615,6 +628,10 @@ def gather_rows(src: torch.Tensor, index: torch.Tensor, index_div: int = 1) -> t
 def silu_mul(a: torch.Tensor, b: Optional[torch.Tensor], with_slack: bool = False) -> torch.Tensor:
     """``silu(a) * b`` element-wise (bf16 or fp32, same shape); ``silu(a)`` when b is None.
     ``with_slack`` (2-D a): the result has SLACK_ROWS readable rows behind it."""
+    if b is None:
+        out = _lib.host().silu(a, int(with_slack), _stream(a))
+        if out is not None:
+            return out
     _need_cuda("silu_mul", a, b)
     if a.dtype not in _DTYPE_CODE or (b is not None and (b.dtype != a.dtype or a.shape != b.shape)):
         raise ValueError("silu_mul: two bf16 (or two fp32) tensors of one shape expected")
@@ -653,6 +670,9 @@ def jagged_transpose(src: torch.Tensor, offsets: torch.Tensor, pad_offsets: torc
 
 def segment_colsum(src: torch.Tensor, offsets: torch.Tensor) -> torch.Tensor:
     """Per-expert column sums [E, C] of jagged rows [R, C], see fmoe_segment_colsum."""
+    out = _lib.host().segment_colsum(src, offsets, _stream(src))
+    if out is not None:
+        return out
     dev = _need_cuda("segment_colsum", src, offsets)
     if src.ndim != 2 or src.dtype not in _DTYPE_CODE:
         raise ValueError("segment_colsum: src must be a 2-D bf16 or fp32 tensor")
@@ -671,6 +691,9 @@ def swiglu_bwd(g: torch.Tensor, u: Optional[torch.Tensor], dh: torch.Tensor, joi
     ``joint`` (gated form, 2-D bf16, columns a multiple of 8): dg and du are the two halves of one
     [rows, 2 * cols] buffer, ``torch.cat([dg, du], 1)`` without the copy, so that the GEMMs that
     consume both can take them as one operand (``dg._base`` is that buffer's storage)."""
+    pair = _lib.host().swiglu_bwd(g, u, dh, int(joint), _stream(g))
+    if pair is not None:
+        return pair
     _need_cuda("swiglu_bwd", g, u, dh)
     if g.dtype not in _DTYPE_CODE or dh.dtype != g.dtype or dh.shape != g.shape or (
             u is not None and (u.dtype != g.dtype or u.shape != g.shape)):
@@ -710,6 +733,9 @@ def combine_bwd(dy: torch.Tensor, value: Optional[torch.Tensor], token_index: to
                 gates: Optional[torch.Tensor] = None, gates_index: Optional[torch.Tensor] = None,
                 need_gate_grad: bool = False):
     """Backward of ``combine``: (d_value [T*K, D], d_gates fp32 [T*K] in the gates' flat layout or None)."""
+    pair = _lib.host().combine_bwd(dy, value, token_index, K, gates, gates_index, int(need_gate_grad), _stream(dy))
+    if pair is not None:
+        return pair
     dev = _need_cuda("combine_bwd", dy, value, token_index, gates, gates_index)
     if dy.ndim != 2 or dy.dtype not in _DTYPE_CODE:
         raise ValueError("combine_bwd: dy must be a 2-D bf16 or fp32 tensor")
@@ -750,6 +776,9 @@ def combine_bwd(dy: torch.Tensor, value: Optional[torch.Tensor], token_index: to
 def invert_index(index: torch.Tensor) -> torch.Tensor:
     """index [T, K] (sorted position -> flat token*K + slot) -> [T, K] sorted positions of each
     token's rows, ascending (the order a sequential index_add meets them in), see fmoe_invert_index."""
+    reverse = _lib.host().invert_index(index, _stream(index))
+    if reverse is not None:
+        return reverse
     _need_cuda("invert_index", index)
     index = _i64("index", index)
     T, K = index.shape
@@ -761,6 +790,9 @@ def invert_index(index: torch.Tensor) -> torch.Tensor:
 
 def gate_l1_bwd(scores: torch.Tensor, topk_idx: torch.Tensor, d_gates: torch.Tensor) -> torch.Tensor:
     """Gradient of the L1-normalised top-k gates with respect to the scores [T, E], see fmoe_gate_l1_bwd."""
+    d_scores = _lib.host().gate_l1_bwd(scores, topk_idx, d_gates, _stream(scores))
+    if d_scores is not None:
+        return d_scores
     dev = _need_cuda("gate_l1_bwd", scores, topk_idx, d_gates)
     if scores.dtype not in _DTYPE_CODE or d_gates.dtype != scores.dtype:
         raise ValueError("gate_l1_bwd: scores and d_gates must be fp32 or bf16, of one dtype")

@@ -112,6 +112,40 @@ def test_layer_forward(B, S, dtype):
         assert other.asked
 
 
+@pytest.mark.parametrize("T,E,K", [(2, 4, 1), (40, 8, 2), (300, 130, 8)])
+@pytest.mark.parametrize("form", ["plain", "strided", "subclass", "fp32"])
+def test_backward_operators(T, E, K, form):
+    from fast_moe_amd.kernels.hip import ops
+    dtype = torch.float32 if form == "fp32" else BF16
+    make = {"plain": lambda t: t, "fp32": lambda t: t, "subclass": lambda t: t.as_subclass(Sub),
+            "strided": lambda t: torch.cat([t, t], dim=-1)[..., :t.shape[-1]]}[form]
+    D, H, R = 64, 96, T * K
+    r = {k: v.cuda() for k, v in make_routing(T, E, K, seed=T).items()}
+    rows = lambda n, seed: dev(randn((R, n), seed).to(dtype))
+    dy, value, g, u, dh = dev(randn((T, D), 1).to(dtype)), rows(D, 2), rows(H, 3), rows(H, 4), rows(H, 5)
+    gates, index = dev(torch.rand(T, K).to(dtype)), r["gate_index"]
+    plain = form in ("plain", "fp32")
+    for need in (False, True):
+        same(*both(lambda: [t for t in ops.combine_bwd(make(dy), value, index, K, gates, index, need_gate_grad=need) if t is not None], plain))
+    same(*both(lambda: [t for t in ops.combine_bwd(make(dy), None, index, K) if t is not None], plain))
+    same(*both(lambda: ops.segment_colsum(make(value), r["offsets"]), plain or form == "strided"))
+    for joint in (False, True):
+        same(*both(lambda: ops.swiglu_bwd(make(g), u, dh, joint=joint), plain))
+    same(*both(lambda: ops.swiglu_bwd(make(g), None, dh)[:1], plain))
+    for slack in (False, True):
+        same(*both(lambda: ops.silu_mul(make(g), None, with_slack=slack), plain))
+    same(*both(lambda: ops.gather_rows(make(dy), index, K), plain or form == "strided"))
+    same(*both(lambda: ops.invert_index(index.view(T, K)), True))
+    scores = dev(torch.rand(T, E).to(dtype))
+    same(*both(lambda: ops.gate_l1_bwd(make(scores), r["topk_idx"], gates), plain))
+    for halves in (False, True):
+        a, b = ops.empty_rows(R, 128, dtype, "cuda").normal_(), ops.empty_rows(R, D, dtype, "cuda").normal_()
+        same(*both(lambda: ops.jagged_weight_grad(a, b, r["offsets"], halves=halves), True))
+    # weights with n contiguous, read in place
+    w = dev(randn((E, H, D), 6).to(dtype))
+    same(*both(lambda: ops.input_grad_gemm(r["offsets"], make(g), w), form != "subclass"))
+
+
 @pytest.mark.parametrize("where", ["class", "object"])
 def test_a_replaced_route_is_asked(where, monkeypatch):
     from fast_moe_amd import FastMoELayer
