@@ -439,7 +439,7 @@ def test_weight_gradient_from_rows_in_place(lens):
     ([1], 8, 16, False, True), ([0, 2, 0, 15, 17], 2560, 136, False, True), ([1, 2] * 150, 72, 40, False, True),
 ])
 def test_weight_gradient_of_few_rows(lens, N, Kin, halves, few, dtype):
-    """The kernel for short contractions and small matrices, and its neighbours on the ring (fp32: left to the transposed copies): against
+    """The kernel for short contractions and small matrices, and its neighbours on the ring (fp32: up to 1.2e10 products): against
     fp64, with the roundings of an fp32 sum over the longest expert's rows (2^-24 each) and of the bf16 result (8 significant bits: 2^-8 at
     most); rows behind the last expert are NaN."""
     from fast_moe_amd.kernels.hip import ops
@@ -452,11 +452,8 @@ def test_weight_gradient_of_few_rows(lens, N, Kin, halves, few, dtype):
         t.copy_(torch.randn(t.shape, generator=g, device="cuda"))
         torch.as_strided(t, (ops.SLACK_ROWS, t.shape[1]), (t.shape[1], 1), R * t.shape[1]).fill_(float("nan"))
     out = ops.jagged_weight_grad(d, x, offsets, halves=halves)
-    if dtype == torch.float32 and R > 64 * E:
-        assert out is None
-        return
     ran = kernels_run(lambda: ops.jagged_weight_grad(d, x, offsets, halves=halves))[-1]
-    assert ("grouped_wgrad_kernel" in ran) == few, ran
+    assert ("grouped_wgrad_kernel" in ran) == (few or dtype == torch.float32), ran
     out = torch.cat(out, dim=1) if halves else out
     for e in range(E):
         a, b = d[offsets[e]:offsets[e + 1]].double(), x[offsets[e]:offsets[e + 1]].double()
@@ -465,8 +462,16 @@ def test_weight_gradient_of_few_rows(lens, N, Kin, halves, few, dtype):
         assert bool(((out[e].double() - want).abs() <= bound + rounded).all()), e
 
 
+def test_large_fp32_weight_gradients_take_the_transposed_copies():
+    from fast_moe_amd.kernels.hip import ops
+    assert ops.weight_grad_pays(torch.float32, 8, 1000, 1000, 12000) and not ops.weight_grad_pays(torch.float32, 8, 1000, 1000, 12001)
+    offsets = torch.tensor([0, 9000, 12004]).cuda()
+    d, x = torch.zeros(12004, 1000, device="cuda"), torch.zeros(12004, 1000, device="cuda")
+    assert ops.jagged_weight_grad(d, x, offsets) is None
+
+
 @pytest.mark.parametrize("T,dtype", [(5, BF16), (300, BF16), (4000, BF16), (40, torch.float32), (2000, torch.float32)])
-@pytest.mark.parametrize("N,Kin,silu", [(264, 392, False), (520, 1032, True), (76, 36, False)])
+@pytest.mark.parametrize("N,Kin,silu", [(264, 392, False), (1504, 2024, True), (520, 1032, True), (76, 36, False)])
 def test_weight_gradients_in_the_weights_own_order(T, dtype, N, Kin, silu):
     """[E, D_in, D_out]-contiguous weights get gradients of that layout, with the values that weights in the other order get: the sums run
     over the same rows, regrouped at most (2^-24 for every row, and the rounding to bf16)."""
