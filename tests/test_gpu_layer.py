@@ -325,3 +325,26 @@ def test_gate_modules_that_are_watched_are_called(monkeypatch):
     layer.requires_grad_(False)
     layer(x, 2)
     assert len(fused) == 2
+
+
+@pytest.mark.parametrize("T,D,H", [(64, 128, 256), (4096, 256, 4096)])
+def test_short_and_split_passes_replay_from_a_graph(T, D, H):
+    """A small batch (gate and routing in one launch each) and one whose second GEMM is cut along K (its workspace comes from the graph's
+    pool): replays between eager passes on other inputs give the eager result every time."""
+    from fast_moe_amd import FastMoELayer
+    from tests.helpers import kernels_run
+    layer = FastMoELayer(D, H, D, 4, dtype=BF16).to(BF16).cuda()
+    xs = [torch.randn(1, T, D, device="cuda").to(BF16) for _ in range(3)]
+    with torch.no_grad():
+        ran = kernels_run(lambda: layer(xs[0], 2))
+        assert any("gate_softmax" in n if T == 64 else "split_reduce" in n for n in ran), ran
+        want = [layer(x, 2) for x in xs]
+        held = xs[0].clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = layer(held, 2)
+        for i in (1, 2, 0, 1):
+            held.copy_(xs[i])
+            graph.replay()
+            assert torch.equal(y, want[i])
+            assert torch.equal(layer(xs[(i + 1) % 3], 2), want[(i + 1) % 3])
