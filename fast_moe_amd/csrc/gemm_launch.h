@@ -224,11 +224,14 @@ inline int direct_columns(int n, bool swiglu) { return swiglu ? (n + 31) / 32 : 
 //     ring is ahead (500 rows, 8 experts, 2048 -> 2 x 1024 bf16 21.0 / 32.5, e4m3 14.8 / 20.3) until the tall ring's are the tiles, which
 //     then are a sixteenth as many: 1000 rows, 8 experts, 2048 -> 2 x 512 39.6 / 33.0 (e4m3 26.0 / 20.0); 1000 rows, 4 experts, 1024 -> 1024
 //     22.5 / 12.2; 2000 rows, 8 experts, 4096 -> 512 69.4 / 60.5.  Three: 2000 rows, 8 experts, 4096 -> 1024 70.2 / 88.8.
-//   * up to two rows per expert on average, where a hot expert has few as well: up to six tiles per CU, seven with K in part (no whole number
-//     of 128 bytes, which the other kernels mask or pad), not e4m3 with whole K.  Even load / nine tenths of the rows in one expert: 60 rows,
-//     32 experts, 2048 -> 2048 61.2 / 51.7, 19.4 / 18.9; 2440 -> 2048 64.3 / 59.6, 35.1 / 19.4; e4m3 2448 -> 2048 39.0 / 32.3, 21.8 / 13.0; 80 rows, 40
-//     experts, 1000 -> 2 x 1024 45.6 / 32.8, 21.7 / 10.7; 180 rows, 96 experts, 3248 -> 1024 e4m3 77.7 / 61.7, 32.5 / 22.4.  Beyond: 128 rows,
-//     64 experts, 1024 -> 2048 (eight tiles per CU) 41.2 / 41.0, 17.9 / 19.1; e4m3 23.2 / 25.0, 12.2 / 13.6; 256 rows, 64 experts 48.0 / 48.5, 24.5 / 33.1.
+//   * few rows per expert on average, where a hot expert has few as well, bf16 and up to six tiles per CU: two.  Even load / nine tenths of the
+//     rows in one expert: 60 rows, 32 experts, 2048 -> 2048 61.2 / 51.7, 19.4 / 18.9; 64 rows, 2048 -> 3072 88.0 / 71.9, 40.6 / 34.1.  Eight: 128
+//     rows, 64 experts, 1024 -> 2048 41.2 / 41.0, 17.9 / 19.1; e4m3 23.2 / 25.0, 12.2 / 13.6.  Four rows: 256 rows 48.0 / 48.5, 24.5 / 33.1.
+//   * K in part (no whole number of 128 bytes), which the other kernels mask or pad: four rows per expert and 13 tiles per CU; 160 rows, 40
+//     experts, 2440 -> 2 x 1024 107 / 83, 68.6 / 34.5; 256 rows, 64 experts, 2440 -> 2048 125 / 126, 73.8 / 66.2, -> 3072 199 / 187, 102 / 87; e4m3
+//     2448 -> 3072 113 / 97, 54 / 48; 400 rows, 100 experts (20 tiles) 176 / 148, 63 / 74.  Eight rows and seven tiles, rows of K of 2000 bytes:
+//     768 rows, 96 experts, 1000 -> 768 45.8 / 34.9, 32.3 / 24.2; e4m3 2448 56.6 / 43.8, 40.6 / 33.5 (1008 20.9 / 16.9, 16.6 / 17.6).  Sixteen:
+//     620 rows, 40 experts, 3240 -> 2 x 1024 141 / 119, 132 / 139.
 //   * beyond, an even load would gain (512 rows, 128 experts, 4096 -> 2 x 1536 543 / 529, e4m3 286 / 264), but an expert with many rows
 //     has its weights read from L2 for every 64 of them and every 32 columns: 1024 rows, Zipf 488 / 606.
 //   * fp32 streams half as much weight for a product and the other kernel is the slower one: 512 rows, 128 experts, 4096 -> 2 x 1536
@@ -247,7 +250,10 @@ inline bool direct_pays(const GemmParams& p, int esize, bool swiglu) {
         return p.K > 64 && (p.K >= 1024 || tiles <= 2 * cus || p.total_rows <= 4 * experts);
     }
     const int row = p.K * esize;
-    if (few && p.total_rows <= 2 * (int64_t)p.E && (row % 128 ? tiles <= 7 * cus : esize == 2 && tiles <= 6 * cus)) return true;
+    const int64_t rows = p.total_rows, E = p.E;
+    if (few && (row % 128 ? (rows <= 4 * E && tiles <= 13 * cus) || (rows <= 8 * E && row >= 2000 && tiles <= 7 * cus)
+                          : rows <= 2 * E && esize == 2 && tiles <= 6 * cus))
+        return true;
     if (few) return tiles <= cus || (tiles <= 2 * cus && (esize == 1 || row <= 1664));
     return tall ? row >= 2048 && tiles <= 2 * cus : row > 512 && tiles <= cus;
 }

@@ -1313,8 +1313,10 @@ def test_streaming_kernel_recomputes_fp32_sums_that_are_not_finite():
 @pytest.mark.parametrize("E,rows,K,N,dtype,direct", [
     (16, 16, 1664, 1024, "bf16", True), (16, 40, 1664, 1024 + 1, "bf16", False),        # one tile per CU; K of more than 1664 bytes beyond
     (16, 16, 832, 2048, "bf16", True), (16, 40, 832, 2049, "bf16", False), (16, 16, 2048, 2048, "fp8", True), (16, 16, 2048, 2049, "fp8", False),
-    (24, 48, 1024, 4096, "bf16", True), (24, 48, 1024, 4100, "bf16", False), (24, 48, 1032, 4672, "bf16", True), (24, 49, 1032, 4096, "bf16", False),
-    (24, 48, 1024, 4096, "fp8", False), (24, 48, 1040, 4672, "fp8", True), (24, 48, 1040, 4800, "fp8", False),
+    (24, 48, 1024, 4096, "bf16", True), (24, 48, 1024, 4100, "bf16", False), (24, 49, 1024, 4096, "bf16", False), (24, 48, 1024, 4096, "fp8", False),
+    (24, 96, 1032, 8512, "bf16", True), (24, 96, 1032, 8584, "bf16", False), (24, 96, 1040, 8512, "fp8", True),         # K in part
+    (24, 97, 1032, 4544, "bf16", True), (24, 97, 1032, 4616, "bf16", False), (24, 97, 1040, 4096, "fp8", False), (24, 97, 2064, 4096, "fp8", True),
+    (24, 193, 1032, 4096, "bf16", False),
     (16, 256, 1664, 1024, "bf16", False), (16, 250, 832, 64, "bf16", True), (4, 65, 832, 64, "bf16", True),
     (4, 80, 256, 64, "bf16", False), (4, 80, 264, 64, "bf16", True), (4, 4096, 1024, 240, "bf16", True), (4, 4096, 1016, 240, "bf16", False),
     (4, 800, 1024, 2048, "bf16", True), (4, 800, 1024, 2056, "bf16", False), (4, 800, 2048, 2048, "fp8", True), (4, 800, 2048, 2064, "fp8", False),
