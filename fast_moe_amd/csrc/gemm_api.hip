@@ -250,6 +250,9 @@ static bool split_takes(const fmoe_gemm_desc* d, const GemmParams& p, int sel) {
 }
 
 extern "C" size_t fmoe_grouped_gemm_workspace_bytes(const fmoe_gemm_desc* d) {
+    // asked before every call: those that are no tall ring's, and K of up to 15 pairs of slices, which split_pays never takes, end here
+    if (!d || d->a_dtype == FMOE_F32 || d->total_rows < kTallRows * (int64_t)d->num_experts || d->k <= (d->a_dtype == FMOE_E4M3 ? 1920 : 960))
+        return 0;
     GemmParams p;
     int sel;
     if (prepare_gemm(d, p, sel) || sel < 0 || !split_takes(d, p, sel)) return 0;
