@@ -137,8 +137,9 @@ def gate_softmax(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     if not lib.fmoe_gate_softmax_pays(code, T, D, weight.shape[0]) or x.data_ptr() % 16 or weight.data_ptr() % 16:
         return None
     chunk = 4 if code == 0 else 8
-    if (x.stride(1) != 1 or x.stride(0) < D or x.stride(0) % chunk or weight.shape[1] != D or not weight.is_contiguous()
-            or (bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous()))):
+    if (x.stride(1) != 1 or x.stride(0) < D or x.stride(0) % chunk or weight.ndim != 2 or weight.shape[1] != D
+            or not weight.is_contiguous()
+            or (bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous() or bias.numel() != weight.shape[0]))):
         return None
     scores = _lib.host().gate_softmax(x, weight, bias, _stream(x))
     if scores is not None:

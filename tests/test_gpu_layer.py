@@ -287,6 +287,17 @@ def test_gate_of_a_small_batch(T, D, E, dtype):
     assert ops.gate_softmax(x, torch.zeros(97, D, dtype=dtype, device="cuda"), None) is None
 
 
+@pytest.mark.parametrize("entries", [1, 7, 9])
+def test_gate_of_a_small_batch_declines_a_bias_of_another_length(entries):
+    """The kernel reads one entry per expert; the native call and the Python code behind it both turn such a bias away."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    x, w = torch.randn(5, 64, device="cuda"), torch.randn(8, 64, device="cuda")
+    bias = torch.zeros(entries, device="cuda")
+    assert _lib.host().gate_softmax(x, w, bias, ops._stream(x)) is None
+    assert ops.gate_softmax(x, w, bias) is None
+    assert ops.gate_softmax(x, w, torch.zeros(8, device="cuda")) is not None
+
+
 def test_gate_modules_that_are_watched_are_called(monkeypatch):
     """Hooks, autocast, gradients, a subclass or an instance's own forward: the gate module is asked, not the launch that stands for it."""
     import torch.nn as nn
