@@ -134,7 +134,9 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, const BlockTile
     for (int s = 0; s < SETS; ++s)
         if (wave + s * NW < pieces) load_x(wave + s * NW, xs[s]);
 
-    f32x4 acc[4][FM];
+    // fp32: the sums of the largest partial products, and of the others (gemm_f32x3.h)
+    constexpr int SUMS = F32 ? 2 : 1;
+    f32x4 acc[4 * SUMS][FM];
     auto multiply = [&](auto exact_c, const u32x4 (&w)[4][2], u32x4 (&x)[FM][2]) {
         constexpr bool EXACT = decltype(exact_c)::value;        // fp32 operands on fp32 MFMAs
         if constexpr (A_SILU) {
@@ -171,16 +173,18 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, const BlockTile
             bf16x8 xp[FM][3];
 #pragma unroll
             for (int fm = 0; fm < FM; ++fm) parts(x[fm], xp[fm]);
-            constexpr int W[6] = {0, 1, 0, 1, 2, 0}, X[6] = {0, 0, 1, 1, 0, 2};
+            FMOE_F32X3_TERMS;
 #pragma unroll
             for (int f = 0; f < 4; ++f) {
                 bf16x8 wp[3];
                 parts(w[f], wp);
 #pragma unroll
-                for (int t = 0; t < 6; ++t)
+                for (int t = 0; t < 8; ++t)
 #pragma unroll
-                    for (int fm = 0; fm < FM; ++fm)
-                        acc[f][fm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[W[t]], xp[fm][X[t]], acc[f][fm], 0, 0, 0);
+                    for (int fm = 0; fm < FM; ++fm) {
+                        f32x4& sum = acc[t ? 4 + f : f][fm];
+                        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[W[t]], xp[fm][X[t]], sum, 0, 0, 0);
+                    }
             }
         } else if constexpr (FP8) {
             auto join = [&](const u32x4 (&v)[2]) -> i32x8 {
@@ -205,7 +209,7 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, const BlockTile
     // the first SETS pieces of the wave are in its registers already
     auto contract = [&](auto exact_c) {
 #pragma unroll
-        for (int f = 0; f < 4; ++f)
+        for (int f = 0; f < 4 * SUMS; ++f)
 #pragma unroll
             for (int fm = 0; fm < FM; ++fm) acc[f][fm] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         for (int c = wave; c < pieces; c += SETS * NW) {
@@ -226,13 +230,17 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, const BlockTile
     // slot (l % 16) ^ c4 of its 16, so that neither writing by rows nor reading by columns has bank conflicts.
     f32x4* const red = reinterpret_cast<f32x4*>(smem);
     const int64_t bias_row = (int64_t)expert * p.bias_se;
-    constexpr int STEP = FM < 2 ? FM : 2;               // fragments whose sums LDS holds at a time
+    constexpr int STEP = FM < 2 || F32 ? 1 : 2;         // fragments whose sums LDS holds at a time
+    constexpr int PER_WAVE = STEP * SUMS * 256;
     auto finish = [&](int fm0, float scale) -> bool {
         bool finite = true;
 #pragma unroll
         for (int i = 0; i < STEP; ++i)
 #pragma unroll
-            for (int f = 0; f < 4; ++f) red[((wave * STEP + i) * 16 + 4 * f + quarter) * 16 + (r16 ^ (4 * f + quarter))] = acc[f][fm0 + i];
+            for (int f = 0; f < 4 * SUMS; ++f) {
+                const int c4 = 4 * (f & 3) + quarter;
+                red[wave * PER_WAVE + ((i * SUMS + (f >> 2)) * 16 + c4) * 16 + (r16 ^ c4)] = acc[f][fm0 + i];
+            }
         __syncthreads();
         constexpr int GROUPS = SWIGLU ? 8 : 16;         // of 4 output columns
         for (int q = tid; q < 16 * STEP * GROUPS; q += NT) {
@@ -241,17 +249,23 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, const BlockTile
             f32x4 sum[2];
 #pragma unroll
             for (int h = 0; h < (SWIGLU ? 2 : 1); ++h) {
-                const int c = c4 + 8 * h, at = (((row >> 4) - fm0) * 16 + c) * 16 + ((row & 15) ^ c);
-                sum[h] = red[at];
+                const int c = c4 + 8 * h, at = (((row >> 4) - fm0) * SUMS * 16 + c) * 16 + ((row & 15) ^ c);
+                f32x4 total[SUMS];
 #pragma unroll
-                for (int i = 1; i < NW; ++i) {
-                    const f32x4 part = red[i * (STEP * 256) + at];
+                for (int s = 0; s < SUMS; ++s) {
+                    total[s] = red[s * 256 + at];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) sum[h][j] += part[j];
+                    for (int i = 1; i < NW; ++i) {
+                        const f32x4 part = red[i * PER_WAVE + s * 256 + at];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) total[s][j] += part[j];
+                    }
                 }
+                sum[h] = total[0];
                 if constexpr (F32) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
+                        sum[h][j] += total[1][j];
                         finite &= __builtin_fabsf(sum[h][j]) < __builtin_inff();
                         sum[h][j] *= scale;
                     }

@@ -66,19 +66,18 @@ int launch_f32x3(GemmParams p, hipStream_t stream) {
     return launch_tiles<TL>(kern, p, attr_done, stream);
 }
 
-// From three slices on; up to two (K = 64) there is hardly a loop to be faster in: 4096 rows, 8 experts, 64 -> 512 columns 10.2 us on
-// v_mfma_f32_32x32x2_f32, 10.9 here (K = 72, SwiGLU: 16.5 / 13.4).
+// From three slices on; up to two (K = 64) there is hardly a loop to be faster in (4096 rows, 8 experts, 512 columns, K = 72: 10.2 us on
+// v_mfma_f32_32x32x2_f32, 9.6 here; SwiGLU, K = 68: 15.2 / 13.7).
 //
 // us per GEMM, v_mfma_f32_32x32x2_f32 on its best tile / three parts on 64 x 64 / 64 x 128 / 128 x 128:
-//   4096 rows,  8 experts, 1024 -> 4096 columns  355 / 247 / 209 / 198        16384 rows  1156 /  -  / 835 / 743
-//   4096 rows,  8 experts, 4096 -> 1024          343 / 242 / 211 / 237        6000 rows, 10 experts, 1024 -> 1024  139 / 107 / 102 / 88
-//   1000 rows, 32 experts,  512 -> 1024           28 /  23 /  25 /  36        2048 rows, 64 experts,  256 -> 1024   28 /  23 /  21 / 29
-//     64 rows,  8 experts, 1024 -> 2048           33 /  32 /  41 /  61        512 rows, 8 experts, 128 -> 256     10.8 / 9.6 / 11.9 / 18
-//   SwiGLU (not on 64 x 64): 4096 rows, 8 experts, 1024 -> 4096  623 / 412 / 364; 600 rows, 16 experts, 512 -> 2048  79 / 43 / 48
-// 16384 rows are 185 TFLOP/s, 1110 of bf16 products: what the chip's power allows.
+//   4096 rows,  8 experts, 1024 -> 4096 columns  291 / 274 / 252 / 225        16384 rows  1130 / 1051 / 960 / 865
+//   4096 rows,  8 experts, 4096 -> 1024          305 / 272 / 238 / 256        6000 rows, 10 experts, 1024 -> 1024  138 / 116 / 127 / 97
+//   1000 rows, 32 experts,  512 -> 1024           26 /  24 /  27 /  38        2048 rows, 64 experts,  256 -> 1024   26 /  24 /  21 / 30
+//   1600 rows, 32 experts,  512 -> 512             - /  19 /  26 /  39        512 rows, 8 experts, 128 -> 256      8.3 / 8.3 / 10.6 / 15.4
+//   SwiGLU (not on 64 x 64): 4096 rows, 8 experts, 1024 -> 4096  577 / 507 / 446; 600 rows, 16 experts, 512 -> 2048  47 / 38 / 57
+// 16384 rows are 159 TFLOP/s, 1270 of bf16 products: what the chip's power allows.
 //   * 128 x 128 reads the least from LDS for a product: where the rows fill five such tiles for every four CUs.
-//   * 64 x 64: up to four per CU however the rows fall (two with SiLU on load, which every column of tiles repeats: 600 rows, 16
-//     experts, 512 -> 2048  45 / 41).
+//   * 64 x 64: up to four per CU however the rows fall (two with SiLU on load, which every column of tiles repeats).
 template <int EPI, bool NCONT, bool A_SILU>
 int pick_f32x3(const GemmParams& p, hipStream_t stream) {
     constexpr bool swiglu = EPI == FMOE_EPI_SWIGLU;     // its gate and up fragments share a wave

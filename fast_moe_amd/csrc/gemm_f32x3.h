@@ -6,14 +6,20 @@
 namespace fmoe {
 
 // x = h + m + l with h, m, l the bf16 roundings of x and of what the ones before it leave: 8 + 8 + 8 bits and the signs of the
-// remainders cover the 24 of an fp32 value, so the sum is exact.  A product of two such values is taken as the six partial
-// products hh, hm, mh, hl, mm, lh; what is left out is below 2^-25 of it.  All six go into one fp32 accumulator.
+// remainders cover the 24 of an fp32 value, so the sum is exact.  A product of two such values is taken as eight of its nine partial
+// products; ll, which is left out, is at most 2^-34 of it (|l| <= 2^-17 of the power of two below |x|), a thousandth of what rounding the
+// product to fp32 costs.  hh, exact in fp32, has an accumulator of its own; the other seven, 2^-7 of it, share a second one, and the two
+// are added once, behind the contraction.  So a product is not rounded before it meets the sum, as in a fused multiply-add: with six
+// products in one accumulator a row of a single product had twice the error of one.
 //
 // Both operands are multiplied by 2^24 first (and the sums by 2^-48 last), so that l of the smallest normal fp32 value is still a
 // normal bf16 value.  That, and the rounding of h, overflows for |x| near 2^104 and sums near 2^80; an infinity or a NaN in an
 // operand makes a NaN of the partial products as well.  A wave that finds a sum that is not finite computes its part of the tile
 // again with v_mfma_f32_32x32x2_f32, straight from global memory: what comes out for such operands is what that instruction gives.
 constexpr float kF32x3Scale = 16777216.0f, kF32x3Unscale = 0x1p-48f;
+
+// The partial products: the weight's and the activation's part of each (0: h, 1: m, 2: l).  The first has an accumulator of its own.
+#define FMOE_F32X3_TERMS constexpr int W[8] = {0, 1, 0, 1, 2, 0, 2, 1}, X[8] = {0, 0, 1, 1, 0, 2, 1, 2}
 
 template <int BM_, int BN_, int WGM_, int WGN_>
 struct TileF32x3 {
@@ -40,11 +46,12 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
 }
 
 // Register-staged: the next slice is loaded while one is multiplied, then cut into parts and parked in the one LDS buffer (48 KB
-// for 128 x 128, so that three blocks share a CU and multiply in each other's barriers).  A second buffer, or two slices in
-// registers, cost blocks and were slower (16384 rows, 8 experts, 1024 -> 4096: 785 us with two slices, 764 with one).
+// for 128 x 128; its two accumulators leave registers for two blocks to a CU, which multiply in each other's barriers).
 //
-// The error against 64 bits is that of the fp32 sums, 12 roundings per 32 k where v_mfma_f32_32x32x2_f32 has 16: 2-norm over
-// standard normal operands 2.5e-7 / 2.87e-7 at K = 256, 4.95e-7 / 5.73e-7 at 1024, 1.01e-6 / 1.15e-6 at 4096.
+// The error against 64 bits: 2 roundings of the large sum per 32 k where v_mfma_f32_32x32x2_f32 has 16.  Here / that instruction, 2-norm
+// over standard normal operands: 8.9e-8 / 2.87e-7 at K = 256, 1.86e-7 / 5.73e-7 at 1024, 3.96e-7 / 1.15e-6 at 4096.  Rows of 1, 2, 4, 16 and 64
+// non-zero values of 1024: 2.53e-8 / 2.53e-8, 2.56e-8 / 3.09e-8, 2.63e-8 / 3.98e-8, 3.37e-8 / 7.39e-8, 5.6e-8 / 1.45e-7; largest, of sum |a||b|:
+// 5.99e-8 / 5.96e-8, 1.40e-7 / 1.14e-7, 1.72e-7 / 1.84e-7, 1.8e-7 / 3.2e-7, 1.7e-7 / 3.8e-7.
 //
 // NCONT: weights whose n is contiguous.  They are parked as they come, [32 k][128 n] per plane, and read with ds_read_b64_tr_b16.
 template <typename TL, int EPI, bool NCONT, bool A_SILU>
@@ -168,13 +175,13 @@ __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const Gem
     };
 
     // ----------------------------------------------------------------- main loop
-    f32x16 acc[FN][FM];
+    f32x16 acc[FN][FM], low[FN][FM];
 #pragma unroll
     for (int i = 0; i < FN; ++i)
 #pragma unroll
         for (int j = 0; j < FM; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = low[i][j][v] = 0.0f;
 
     // first tile column of weight fragment fn
     auto frag_col = [&](int fn) -> int {
@@ -213,14 +220,16 @@ __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const Gem
 #pragma unroll
                 for (int fm = 0; fm < FM; ++fm) xf[pl][fm] = read_x(fm, pl, sub);
             }
-            constexpr int W[6] = {0, 1, 0, 1, 2, 0}, X[6] = {0, 0, 1, 1, 0, 2};
+            FMOE_F32X3_TERMS;
 #pragma unroll
-            for (int t = 0; t < 6; ++t)
+            for (int t = 0; t < 8; ++t)
 #pragma unroll
                 for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-                    for (int fm = 0; fm < FM; ++fm)
-                        acc[fn][fm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[W[t]][fn], xf[X[t]][fm], acc[fn][fm], 0, 0, 0);
+                    for (int fm = 0; fm < FM; ++fm) {
+                        f32x16& sum = t ? low[fn][fm] : acc[fn][fm];
+                        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[W[t]][fn], xf[X[t]][fm], sum, 0, 0, 0);
+                    }
         }
     }
 
@@ -231,6 +240,7 @@ __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const Gem
         for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
+                acc[fn][fm][v] += low[fn][fm][v];
                 probe = __builtin_fmaf(acc[fn][fm][v], 0.0f, probe);
                 acc[fn][fm][v] *= kF32x3Unscale;
             }

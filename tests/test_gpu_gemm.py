@@ -1162,7 +1162,7 @@ def test_fp32_on_bf16_matrix_cores(E, rows, K, N, layout, epi, tile, case):
     """fp32 values in three bf16 parts, on every tile.  small, large: rows and columns scaled by powers of two, operands
     down to the smallest normal values, up to sums where the parts overflow.  special: an infinity, a NaN and values beyond 2^104 in single
     rows and columns, whose results are those of the plain fp32 sum; the other results do not see them.  Against float64; the
-    bound of a K-term fp32 sum and the partial products left out (2^-25 each), (K + 3) * 2^-24 * sum |a||b|; as in
+    bound of a K-term fp32 sum, the sum of the small partial products and those left out (2^-34 each) in (K + 3) * 2^-24 * sum |a||b|; as in
     test_fp32_kernel_tiles_and_weight_layouts through SiLU and the product."""
     from fast_moe_amd.kernels.hip import _lib, ops
     g = torch.Generator(device="cuda").manual_seed(K + N + rows)
@@ -1208,6 +1208,38 @@ def test_fp32_on_bf16_matrix_cores(E, rows, K, N, layout, epi, tile, case):
             near = want.abs().cpu() < 1e38
             assert torch.equal(got.cpu().isnan(), plain_fp32.isnan()) and bool(got.cpu()[far].isinf().all())
             assert bool(((got - want).abs() <= err).cpu()[near].all())
+
+
+@pytest.mark.parametrize("E,rows,K,N,layout", [(3, 700, 256, 1156, "nk"), (3, 700, 256, 1156, "kn"), (3, 190, 200, 60, "nk"), (3, 4800, 256, 1156, "kn"),
+                                               (4, 40, 1024, 264, "nk"), (8, 200, 1024, 132, "nk")])
+@pytest.mark.parametrize("nonzero", [1, 2, 5, 16])
+def test_fp32_rows_of_few_nonzero_products(E, rows, K, N, layout, nonzero):
+    """Results of few products have no more error than fused multiply-adds in fp32 leave, one rounding of the running sum for each: in the
+    2-norm (the roundings' signs are random: 2 %), and in every value the bound of the sum of the large partial products, which are exact
+    (n - 1 additions, the last place each as an MFMA may cut it: 2^-23), of adding the small ones (2^-24) and of their sum (2^-7 of the
+    products, seven additions each: 2^-27)."""
+    from fast_moe_amd.kernels.hip import ops
+    g = torch.Generator(device="cuda").manual_seed(K + N + nonzero)
+    x = torch.randn(rows, K, generator=g, device="cuda")
+    x = x * (torch.rand(rows, K, generator=g, device="cuda").argsort(dim=1) < nonzero)
+    w = torch.randn(E, K, N, generator=g, device="cuda")
+    if layout == "nk":
+        w = w.permute(0, 2, 1).contiguous().permute(0, 2, 1)
+    off = (torch.arange(E + 1) * rows // E).cuda()
+    out = ops.grouped_gemm(off, x, w, total_rows=rows).double()
+    ours = fused = 0.0
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        a, b = x[lo:hi], w[e]
+        want, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+        bound = (2 * nonzero - 1) * 2.0 ** -24 + nonzero * 2.0 ** -27
+        assert bool(((out[lo:hi] - want).abs() <= bound * size).all()), f"expert {e}"
+        where, chain = a.ne(0).float().topk(nonzero, dim=1).indices, torch.zeros_like(want)
+        for i in range(nonzero):
+            chain = (chain + a.gather(1, where[:, i:i + 1]).double() * b[where[:, i]].double()).float().double()
+        ours += float((out[lo:hi] - want).square().sum())
+        fused += float((chain - want).square().sum())
+    assert ours <= 1.02 ** 2 * fused, (ours / fused) ** 0.5
 
 
 @pytest.mark.parametrize("K,new", [(64, False), (68, True)])
