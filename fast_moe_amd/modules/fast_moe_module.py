@@ -105,11 +105,11 @@ class FastMoELayer(nn.Module):
 
     def _scores(self, x: torch.Tensor) -> torch.Tensor:
         """The gate's probabilities [tokens, E]: from one launch where the batch is small, nothing needs a gradient and the gate is the
-        class's own; a caller's module, hooks and autocast are asked through the modules."""
+        class's own; a caller's module, hooks and autocast are asked through the modules, and so are other shapes, which they refuse."""
         gate = self.gate
-        if x.numel() <= _SMALL_BATCH * self.input_dim and type(gate) is GatingNetwork and type(gate.gate) is nn.Linear \
-                and type(x) is torch.Tensor and GatingNetwork.forward is _GATE_FORWARD and not _watched(gate) \
-                and not _watched(gate.gate) and not torch.is_autocast_enabled():
+        if type(x) is torch.Tensor and x.ndim == 3 and x.shape[2] == self.input_dim and x.numel() <= _SMALL_BATCH * self.input_dim \
+                and type(gate) is GatingNetwork and type(gate.gate) is nn.Linear and GatingNetwork.forward is _GATE_FORWARD \
+                and not _watched(gate) and not _watched(gate.gate) and not torch.is_autocast_enabled():
             weight, bias = gate.gate.weight, gate.gate.bias
             if not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)):
                 scores = ops.gate_softmax(x.reshape(-1, self.input_dim), weight, bias)

@@ -298,6 +298,28 @@ def test_gate_of_a_small_batch_declines_a_bias_of_another_length(entries):
     assert ops.gate_softmax(x, w, torch.zeros(8, device="cuda")) is not None
 
 
+@pytest.mark.parametrize("shape", [(1, 4, 128), (2, 4, 32), (8, 64), (512,), (2, 2, 2, 64)])
+def test_small_batches_of_another_shape_go_through_the_gate_module(shape):
+    """What Linear and the softmax over the third dimension refuse is refused whatever the batch, before anything is routed, and what they
+    make of four dimensions is routed."""
+    from fast_moe_amd import FastMoELayer
+    from fast_moe_amd.kernels.hip import ops
+    layer = FastMoELayer(64, 96, 64, 4).to(BF16).cuda()
+    x = torch.randn(shape, device="cuda").to(BF16)
+    with torch.no_grad():
+        if len(shape) == 4:
+            want = ops.route_topk(layer.gate(x).reshape(-1, 4), 2)
+            got = layer.route(x, 2)
+            assert all(torch.equal(got[n], want[n]) for n in want)
+            return
+        with pytest.raises((RuntimeError, IndexError)) as asked:
+            layer.gate(x)
+        for call in (layer.route, layer):
+            with pytest.raises(asked.type, match="shapes cannot be multiplied|Dimension out of range") as refused:
+                call(x, 2)
+            assert str(refused.value) == str(asked.value)
+
+
 def test_gate_modules_that_are_watched_are_called(monkeypatch):
     """Hooks, autocast, gradients, a subclass or an instance's own forward: the gate module is asked, not the launch that stands for it."""
     import torch.nn as nn
