@@ -65,7 +65,7 @@ class _WgradOperand:
                 self.rows = a_src
             elif row_index is None:             # SiLU rounded as the forward GEMM rounds it on load
                 self.rows = ops.silu_mul(a_src, None, with_slack=True)
-            elif not apply_silu:
+            elif not apply_silu and ops.gather_takes(a_src):
                 self.rows = ops.gather_rows(a_src, row_index, index_div)
 
     def _transposed(self):
@@ -92,7 +92,7 @@ class _WgradOperand:
         a_src, total_rows, row_index, index_div, apply_silu = self.args
         rows = self.rows
         if rows is None and a_src.dtype == torch.float32 and a_src.ndim == 2 and a_src.shape[1] % 4 == 0 and dout.shape[1] % 4 == 0 \
-                and ops.weight_grad_pays(a_src.dtype, E, N, a_src.shape[1], total_rows):
+                and (row_index is None or ops.gather_takes(a_src)) and ops.weight_grad_pays(a_src.dtype, E, N, a_src.shape[1], total_rows):
             rows = a_src if row_index is None else ops.gather_rows(a_src, row_index, index_div)
             rows = self.rows = ops.silu_mul(rows, None) if apply_silu else rows
         if rows is not None:

@@ -606,6 +606,14 @@ def combine(value: torch.Tensor, reverse_index: torch.Tensor, gates: Optional[to
     return out
 
 
+def gather_takes(src: torch.Tensor) -> bool:
+    """Whether gather_rows takes the rows of a 2-D src: whole 16-byte chunks at 16-byte boundaries (rows that are not contiguous are copied
+    by it first, to such boundaries)."""
+    es = src.element_size()
+    return src.shape[1] * es % 16 == 0 and (src.stride(1) != 1 or (
+        src.data_ptr() % 16 == 0 and src.stride(0) * es % 16 == 0 and src.stride(0) >= src.shape[1]))
+
+
 def gather_rows(src: torch.Tensor, index: torch.Tensor, index_div: int = 1) -> torch.Tensor:
     """``src[index // index_div]`` for a 2-D src with contiguous rows of whole 16-byte chunks
     (fmoe_gather_rows); the result has slack rows behind it."""

@@ -462,6 +462,41 @@ def test_weight_gradient_of_few_rows(lens, N, Kin, halves, few, dtype):
         assert bool(((out[e].double() - want).abs() <= bound + rounded).all()), e
 
 
+@pytest.mark.parametrize("dtype", [BF16, torch.float32])
+@pytest.mark.parametrize("where", ["column", "pitch", "base"])
+def test_gradients_of_rows_off_a_16_byte_boundary(dtype, where):
+    """The input rows start off a 16-byte boundary (a column of a wider tensor, an odd pitch, an odd first element): the weight gradient takes
+    the route over transposed copies, which reads any row.  Input and bias gradients do not see the input rows: same bits.  fp32 sums
+    over the longest expert's rows, 2^-24 each, and the rounding to bf16."""
+    from fast_moe_amd.kernels import moe
+    T, E, K, D, H = 60, 5, 2, 128, 96
+    r = {k: v.cuda() for k, v in make_routing(T, E, K, seed=3).items()}
+    off, index = r["offsets"], r["gate_index"].view(T, K)
+    values = dev(randn((T, D), 1)).to(dtype)
+    if where == "column":
+        x = torch.zeros(T, D + 8, dtype=dtype, device="cuda")[:, 1:D + 1]
+    elif where == "pitch":
+        x = torch.zeros(T, D + 1, dtype=dtype, device="cuda")[:, :D]
+    else:
+        x = torch.zeros(T * D + 1, dtype=dtype, device="cuda")[1:].view(T, D)
+    x.copy_(values)
+    w, b, dy = dev(randn((E, D, H), 2)).to(dtype), dev(randn((E, H), 4)).to(dtype), dev(randn((T * K, H), 5)).to(dtype)
+    grads = []
+    for rows in (x, values):
+        leaves = [t.detach().requires_grad_(True) for t in (rows, w, b)]
+        assert leaves[0].data_ptr() == rows.data_ptr() and leaves[0].stride() == rows.stride()
+        moe.index_select_jagged_bmm(0, off, index, *leaves).backward(dy)
+        grads.append([t.grad for t in leaves])
+    assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][2], grads[1][2])
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        a, d = values[r["gate_index"][lo:hi] // K].double(), dy[lo:hi].double()
+        want, bound = a.t() @ d, (hi - lo + 1) * 2.0 ** -24 * (a.abs().t() @ d.abs())
+        rounded = 2.0 ** -8 * (want.abs() + bound) if dtype == BF16 else 0
+        for got in grads:
+            assert bool(((got[1][e].double() - want).abs() <= bound + rounded).all()), e
+
+
 def test_large_fp32_weight_gradients_take_the_transposed_copies():
     from fast_moe_amd.kernels.hip import ops
     assert ops.weight_grad_pays(torch.float32, 8, 1000, 1000, 12000) and not ops.weight_grad_pays(torch.float32, 8, 1000, 1000, 12001)
