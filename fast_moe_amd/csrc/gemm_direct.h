@@ -16,7 +16,7 @@ namespace fmoe {
 // launch; with all CUs busy the 64-byte pieces a CU can ask for, about 30 KB/us (32 x 32 MFMAs, whose loads touch 32 rows, half as
 // fast: 512 rows, 128 experts, 4096 -> 2 x 1536 586 us, now 525 to 529).
 template <int DT, int NW_>
-struct StreamCfg {
+struct DirectCfg {
     static constexpr int NW = NW_, SETS = NW == 4 ? 2 : 1;      // pieces of weights a wave has on their way
     static constexpr int FM = DT == kDtF32 ? 2 : 4, BM = 16 * FM;
     static constexpr int NT = kWave * NW;
@@ -85,7 +85,7 @@ struct BlockTile32 {
 };
 
 template <typename CF, int DT, int EPI, bool A_SILU, int FM, int SETS>
-__device__ __forceinline__ void stream_tile(const GemmParams& p, const BlockTile32& tile) {
+__device__ __forceinline__ void direct_tile(const GemmParams& p, const BlockTile32& tile) {
     constexpr int NW = CF::NW, NT = CF::NT;
     constexpr bool FP8 = DT == kDtE4m3, F32 = DT == kDtF32, SWIGLU = EPI == FMOE_EPI_SWIGLU;
     constexpr int ESIZE = FP8 ? 1 : F32 ? 4 : 2;
@@ -345,12 +345,12 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, const BlockTile
 }
 
 template <typename CF, int DT, int EPI, bool A_SILU>
-__global__ __launch_bounds__(CF::NT, 2) void grouped_gemm_stream_kernel(const GemmParams p) {
+__global__ __launch_bounds__(CF::NT, 2) void grouped_gemm_direct_kernel(const GemmParams p) {
     BlockTile32 tile;
     if (!tile.locate(p, CF::BM)) return;
-    if (tile.rows_valid <= 16) return stream_tile<CF, DT, EPI, A_SILU, 1, CF::SETS>(p, tile);
-    if (tile.rows_valid <= 32) return stream_tile<CF, DT, EPI, A_SILU, 2, CF::SETS>(p, tile);
-    if constexpr (CF::FM == 4) stream_tile<CF, DT, EPI, A_SILU, 4, 1>(p, tile);
+    if (tile.rows_valid <= 16) return direct_tile<CF, DT, EPI, A_SILU, 1, CF::SETS>(p, tile);
+    if (tile.rows_valid <= 32) return direct_tile<CF, DT, EPI, A_SILU, 2, CF::SETS>(p, tile);
+    if constexpr (CF::FM == 4) direct_tile<CF, DT, EPI, A_SILU, 4, 1>(p, tile);
 }
 
 }  // namespace fmoe

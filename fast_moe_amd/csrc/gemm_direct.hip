@@ -9,8 +9,8 @@ namespace fmoe {
 // 512 rows, 128 experts, 1536 -> 4096 fp32 630 / 571).
 template <int DT, int EPI, bool A_SILU, int NW>
 static int launch(GemmParams p, hipStream_t stream) {
-    typedef StreamCfg<DT, NW> CF;
-    auto kern = grouped_gemm_stream_kernel<CF, DT, EPI, A_SILU>;
+    typedef DirectCfg<DT, NW> CF;
+    auto kern = grouped_gemm_direct_kernel<CF, DT, EPI, A_SILU>;
     static bool attr_done = false;
     if (int rc = reserve_lds(kern, CF::LDS_BYTES, attr_done)) return rc;
     const int64_t tiles = most_row_tiles(p.total_rows, p.E, CF::BM) * p.n_tiles;

@@ -2,7 +2,7 @@
 // bf16 or OCP-e4m3 operands, fp32 MFMA accumulation, fused bias / SiLU / SwiGLU
 // epilogue.  Shared by gemm_bf16.hip and gemm_fp8.hip.
 //
-// Three kernels share the scheduler and the epilogue:
+// The kernels (gemm_launch.h and gemm_api.hip say which runs what):
 //
 //   grouped_gemm_ring_kernel   the fast path.  Persistent (one block per CU), 256 x 256 tiles,
 //       8 wavefronts.  Operand K-slices of 64 bytes per row travel global -> LDS with
@@ -19,10 +19,10 @@
 //       CU; a K-slice travels global -> registers -> LDS while the previous one is multiplied,
 //       and the next tile's first slice is loaded before the current tile's epilogue, so the
 //       weight stream does not stop at tile boundaries.
-//       A launch of few tiles takes its other form (gemm_direct.h): 64 x 64 tiles whose waves share K
-//       and load weights straight into their registers.
+//   grouped_gemm_direct_kernel launches of few tiles, or of a row or two per expert: 64 x 64 tiles
+//       whose waves share K and load weights straight into their registers (gemm_direct.h).
 //   grouped_gemm_kernel        register-staged, double-buffered LDS; serves everything the
-//       other two do not: arbitrary B strides and K / N tails (element loads), SiLU applied
+//       others do not: arbitrary B strides and K / N tails (element loads), SiLU applied
 //       to A on load, fp32 operands of few k (on tiles of their own, gemm_f32.hip).
 //   grouped_gemm_f32x3_kernel  fp32 operands otherwise: register-staged too, every value cut into three
 //       bf16 parts on its way into LDS (gemm_f32x3.h).

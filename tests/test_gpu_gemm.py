@@ -1297,7 +1297,7 @@ def test_streaming_kernel_of_few_tiles(lens, K, N, epi, dtype, extras):
         x, ws = qx.float() / sx[:, None], [q.float() / s[..., None] for q, s in qw]
     out = ops.grouped_gemm(off, *args, **kw)
     ran, = kernels_run(lambda: ops.grouped_gemm(off, *args, **kw))
-    assert "grouped_gemm_stream_kernel<fmoe::StreamCfg<" in ran, ran
+    assert "grouped_gemm_direct_kernel<" in ran, ran
     source = x if index is None else x[index // 2]
     unit = (K + 4) * 2.0 ** -24 + (2.0 ** -21 if a_silu else 0)
     for e in range(E):
@@ -1363,7 +1363,7 @@ def test_streaming_kernel_choice(E, rows, K, N, dtype, direct):
     kw = dict(a_scale=torch.ones(rows, device="cuda"), b_scale=torch.ones(E, N, device="cuda")) if dtype == "fp8" else {}
     off = (torch.arange(E + 1) * rows // E).cuda()
     ran, = kernels_run(lambda: ops.grouped_gemm(off, x, w, total_rows=rows, **kw))
-    assert ("StreamCfg<" in ran) == direct, ran
+    assert ("grouped_gemm_direct_kernel<" in ran) == direct, ran
 
 
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
