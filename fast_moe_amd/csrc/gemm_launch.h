@@ -210,39 +210,36 @@ inline int64_t most_row_tiles(int64_t rows, int64_t num_experts, int bm) {
 }
 inline int direct_columns(int n, bool swiglu) { return swiglu ? (n + 31) / 32 : (n + 63) / 64; }
 
-// Where they are taken (weights with k contiguous, 16-byte loads, no gate).  us per GEMM, the kernel that ran before (the 64-row or the tall
-// ring, the streaming or the register-staged kernel) / this one; even load unless said:
+// Where they are taken (weights with k contiguous, 16-byte loads, no gate).  The host knows the row count and not how the experts share it, so
+// the rule goes by the most tiles it allows.  us per GEMM on weights that are in no cache, the kernel that runs otherwise (the 64-row or the tall
+// ring, the streaming or a register-staged kernel) / this one; even load, "hot" with nine tenths of the rows in one expert:
 //   * no more tiles than CUs, whatever the rows (beyond 16 per expert on average from rows of K of 513 bytes on, from 96 per expert on of 2
-//     KB: the chain that is shared out is short below, 3 us are left to gain: 2000 rows, 4 experts, 128 -> 256 8.7 / 5.6): the tile that others walk alone (64 x 256 or 256 x 256, K serial) is a quarter as wide or
-//     less and its K is shared by eight waves.  24 rows, 10 experts, 2112 -> 408 18.3 / 11.4 (e4m3 14.9 / 6.8, fp32 56.1 / 20.5); 5 rows, 35
-//     experts, 2696 -> 1024 32.2 / 10.4 (fp32 72.2 / 21.5); 64 rows, 4 experts, 4096 -> 4096 33.3 / 24.7; 160 rows, 10
-//     experts, 1024 -> 1024 12.0 / 8.9, Zipf 11.9 / 11.5; 207 rows, 4 experts, 1088 -> 1152 13.2 / 11.7; 256 rows, 4 experts, 4096 -> 1024 32.1 /
-//     32.2, one hot expert 31.3 / 32.0; 3000 rows, 4 experts, 1024 -> 320 22.7 / 11.6 (e4m3 16.1 /
-//     8.6), 4096 -> 320 69.3 / 33.5; 766 rows, 6 experts, 3904 -> 640 65.3 / 31.4; fp32 320 rows, 8 experts, 1024 -> 512 30.6 / 15.8
+//     KB): the tile that others walk alone (64 x 256 or 256 x 256, K serial) is a quarter as wide or less and its K is shared by eight
+//     waves.  1 row, 8 experts, 1024 -> 4096 12.2 / 7.6 (e4m3 10.0 / 5.8, fp32 30.3 / 12.7); 3 rows, 64 experts, 2048 -> 2 x 1408 26.5 / 12.9
+//     (14.2 / 8.7, 93 / 25); 24 rows, 10 experts, 2112 -> 408 27.9 / 12.6 (15.9 / 6.5, 70 / 22); 64 rows, 4 experts, 4096 -> 4096 54.2 / 30.4, hot
+//     55.3 / 36.4; 160 rows, 10 experts, 1024 -> 1024 16.9 / 9.7, hot 16.6 / 12.3; 207 rows, 4 experts, 1088 -> 1152 13.4 / 11.8; 256 rows, 4
+//     experts, 4096 -> 1024 46.8 / 33.1; 3000 rows, 4 experts, 1024 -> 320 23.1 / 12.2 (e4m3 16.9 / 9.3)
 //   * up to two per CU: e4m3, and rows of K up to 1664 bytes, with up to 16 rows per expert on average.  98 rows, 11 experts, 2496 -> 2 x
-//     832 bf16 23.4 / 25.6 (not taken), e4m3 19.0 / 13.3; 98 rows, 11 experts, 832 -> 2496 bf16 12.5 / 11.7.  With more rows the 64-row
-//     ring is ahead (500 rows, 8 experts, 2048 -> 2 x 1024 bf16 21.0 / 32.5, e4m3 14.8 / 20.3) until the tall ring's are the tiles, which
-//     then are a sixteenth as many: 1000 rows, 8 experts, 2048 -> 2 x 512 39.6 / 33.0 (e4m3 26.0 / 20.0); 1000 rows, 4 experts, 1024 -> 1024
-//     22.5 / 12.2; 2000 rows, 8 experts, 4096 -> 512 69.4 / 60.5.  Three: 2000 rows, 8 experts, 4096 -> 1024 70.2 / 88.8.
-//   * few rows per expert on average, where a hot expert has few as well, bf16 and up to six tiles per CU: two.  Even load / nine tenths of the
-//     rows in one expert: 60 rows, 32 experts, 2048 -> 2048 61.2 / 51.7, 19.4 / 18.9; 64 rows, 2048 -> 3072 88.0 / 71.9, 40.6 / 34.1.  Eight: 128
-//     rows, 64 experts, 1024 -> 2048 41.2 / 41.0, 17.9 / 19.1; e4m3 23.2 / 25.0, 12.2 / 13.6.  Four rows: 256 rows 48.0 / 48.5, 24.5 / 33.1.
+//     832 e4m3 27.8 / 17.5, hot 26.9 / 14.5; 832 -> 2496 bf16 17.0 / 12.9, hot 15.8 / 16.6.  With more rows the 64-row ring is ahead where one
+//     expert is hot (500 rows, 8 experts, 2048 -> 2 x 1024 bf16 32.6 / 22.7, hot 30.1 / 33.8; e4m3 19.0 / 16.0, 18.1 / 21.4) until the tall ring's
+//     are the tiles, which then are a sixteenth as many: 1000 rows, 8 experts, 2048 -> 2 x 512 39.2 / 20.8, hot 44.9 / 33.4 (e4m3 26.1 / 14.7, 28.7 /
+//     20.9); 1000 rows, 4 experts, 1024 -> 1024 23.0 / 13.0, hot 23.1 / 19.4.
+//   * few rows per expert on average, where a hot expert has few as well, bf16 and up to six tiles per CU: two.  60 rows, 32 experts, 2048 -> 2048
+//     65 / 71, hot 28.5 / 20.3; 64 rows, 2048 -> 3072 98 / 78, hot 40.0 / 32.7; 2 rows, 128 experts, 4096 -> 2 x 1536 47.0 / 21.2.  Eight: 128 rows, 64
+//     experts, 1024 -> 2048 50.7 / 49.4, hot 23.1 / 19.9; e4m3 30.2 / 35.6.  Four rows: 256 rows 50.7 / 49.9, hot 24.8 / 31.3.
 //   * K in part (no whole number of 128 bytes), which the other kernels mask or pad: four rows per expert and 13 tiles per CU; 160 rows, 40
-//     experts, 2440 -> 2 x 1024 107 / 83, 68.6 / 34.5; 256 rows, 64 experts, 2440 -> 2048 125 / 126, 73.8 / 66.2, -> 3072 199 / 187, 102 / 87; e4m3
-//     2448 -> 3072 113 / 97, 54 / 48; 400 rows, 100 experts (20 tiles) 176 / 148, 63 / 74.  Eight rows and seven tiles, rows of K of 2000 bytes:
-//     768 rows, 96 experts, 1000 -> 768 45.8 / 34.9, 32.3 / 24.2; e4m3 2448 56.6 / 43.8, 40.6 / 33.5 (1008 20.9 / 16.9, 16.6 / 17.6).  Sixteen:
-//     620 rows, 40 experts, 3240 -> 2 x 1024 141 / 119, 132 / 139.
-//   * beyond, an even load would gain (512 rows, 128 experts, 4096 -> 2 x 1536 543 / 529, e4m3 286 / 264), but an expert with many rows
-//     has its weights read from L2 for every 64 of them and every 32 columns: 1024 rows, Zipf 488 / 606.
-//   * fp32 streams half as much weight for a product and the other kernel is the slower one: 512 rows, 128 experts, 4096 -> 2 x 1536
-//     1475 / 1066, Zipf 1011 / 844, nine tenths in one expert 653 / 543.  Not with short K and rows enough for a hot expert (400 rows,
-//     24 experts, 896 -> 2192: even 48.5 / 46.0, one hot expert 48.8 / 56.6), nor with K of two slices (gemm_f32.hip).  With more than 16
-//     rows per expert the other kernel's tiles hold more of them: K from 1024 on and one tile per CU only (2048 rows, 8 experts, 256 ->
-//     256 10.7 / 13.3; 4000 rows, 8 experts, 4096 -> 512, four per CU, 162 / 218).
-// Calls of up to three rows belong to the 64-row ring by the tests of the rule before this one.
+//     experts, 2440 -> 2 x 1024 105 / 79, hot 67 / 39; 256 rows, 64 experts, 2440 -> 2048 126 / 126, hot 71 / 61, -> 3072 200 / 189, hot 101 / 88; e4m3
+//     2448 -> 3072 113 / 101, hot 52 / 44.  Eight rows and seven tiles, rows of K of 2000 bytes: 768 rows, 96 experts, 1000 -> 768 46.5 / 35.8, hot
+//     33.5 / 24.6; e4m3 2448 59 / 45, hot 40 / 31.  Sixteen, not taken: 620 rows, 40 experts, 3240 -> 2 x 1024 139 / 115, hot 127 / 116.
+//   * beyond, an even load would gain (512 rows, 128 experts, 4096 -> 2 x 1536 526 / 513, e4m3 278 / 274), but an expert with many rows
+//     has its weights read from L2 for every 64 of them and every 32 columns: hot 238 / 288, e4m3 124 / 156.
+//   * fp32 streams half as much weight for a product and the other kernel is the slower one: up to 16 rows per expert whatever the tiles, from
+//     K = 1024 on, up to two per CU or up to four rows (512 rows, 128 experts, 4096 -> 2 x 1536 1384 / 1075, hot 571 / 530; 512 rows, 64 experts, 512
+//     -> 2048, not taken, level where one expert is hot), but not K of two slices (gemm_f32.hip).  With more rows the other kernel's tiles
+//     hold more of them: K from 1024 on and one tile per CU (320 rows, 8 experts, 1024 -> 512 40.0 / 17.6).  256 rows per expert and more below
+//     that K: 1000 rows, 8 experts, 256 -> 512 hot 12.6 / 16.5; more tiles: 4000 rows, 8 experts, 4096 -> 512, four per CU, 143 / 180.
 inline bool direct_pays(const GemmParams& p, int esize, bool swiglu) {
     const int64_t experts = p.E < p.total_rows ? p.E : p.total_rows, cus = compute_units();
-    if (p.total_rows < 4) return false;
     const int64_t tiles = most_row_tiles(p.total_rows, p.E, 64) * direct_columns(p.N, swiglu);
     const bool few = p.total_rows <= 16 * experts, tall = p.total_rows / p.E >= kTallRows;
     if (esize == 4) {

@@ -1253,6 +1253,7 @@ def test_fp32_kernel_for_short_k(K, new):
 @pytest.mark.parametrize("lens,K,N,epi", [
     ([16, 1, 17, 30], 392, 68, 0), ([33, 0, 64, 31, 0, 0, 0, 0], 264, 260, 1),     # one, two and four fragments of 16 rows, full and one row more
     ([65, 0, 0, 0, 0, 0, 2], 520, 40, 2),                               # more than a tile's rows; SwiGLU columns in part
+    ([0, 1], 136, 72, 0), ([0, 1, 0, 1], 1032, 200, 2), ([2, 0, 1], 520, 64, 1), # one, two and three rows
     ([0, 3, 1], 72, 8, 0), ([2, 2], 128, 64, 2),                        # fewer 128-byte pieces than waves; one whole tile
     ([1] * 70 + [0, 9], 104, 132, 0), ([4, 0] * 80, 136, 72, 1),        # more experts than lanes
     ([5] * 11, 800, 2900, 0), ([3] * 20, 824, 1096, "silu"),           # more tiles than CUs
@@ -1354,6 +1355,7 @@ def test_streaming_kernel_recomputes_fp32_sums_that_are_not_finite():
     (4, 800, 1024, 2048, "bf16", True), (4, 800, 1024, 2056, "bf16", False), (4, 800, 2048, 2048, "fp8", True), (4, 800, 2048, 2064, "fp8", False),
     (4, 380, 1024, 2048, "bf16", False), (4, 300, 1024, 512, "f32", True), (4, 300, 1020, 512, "f32", False),
     (16, 100, 1020, 2049, "f32", False), (16, 64, 1020, 2049, "f32", True), (16, 100, 1024, 2049, "f32", True), (16, 16, 64, 64, "f32", False),
+    (8, 1, 4096, 1024, "bf16", True), (8, 2, 4096, 1024, "fp8", True), (8, 3, 4096, 1024, "f32", True), (1, 1, 128, 256, "bf16", True),
 ])
 def test_streaming_kernel_choice(E, rows, K, N, dtype, direct):
     """Which calls the kernel above takes, on either side of the rule's lines."""
@@ -1369,7 +1371,7 @@ def test_streaming_kernel_choice(E, rows, K, N, dtype, direct):
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
     (3, 130, 136, 264, "nk", 0), (3, 130, 192, 136, "kn", 0),       # the least K: three pairs of K-slices, the last in part / whole
     (1, 64, 256, 256, "kn", 1), (1, 65, 256, 256, "nk", 1),         # one whole tile; one row more
-    (2, 3, 1000, 520, "nk", 2), (2, 3, 1000, 520, "kn", 2),
+    (3, 130, 1000, 4104, "nk", 2), (2, 3, 1000, 520, "nk", 3), (2, 3, 1000, 520, "kn", 2),
     (200, 900, 328, 72, "kn", 0), (130, 5000, 264, 1032, "kn", 2),  # more experts than lanes; more tiles than CUs
     (2, 150, 200, 320, "kn", 3), (40, 2000, 640, 2048, "kn", 3),
     (3, 280, 640, 32768, "nk", 3),                                  # more tiles than CUs with k contiguous
@@ -1458,7 +1460,8 @@ def test_e4m3_operands_off_a_16_byte_boundary(rows, K, lead):
     (8, 760, 4096, 3328, "fp8", 0, "ring"), (8, 760, 4096, 3584, "fp8", 0, "stream"),
     (128, 512, 4096, 1536, "nk", 2, "stream"), (128, 512, 4096, 1536, "fp8", 0, "stream"),
     (128, 8000, 4096, 1536, "nk", 2, "stream"),                                         # many rounds of tiles
-    (200, 3, 1024, 8192, "nk", 0, "ring"),                                              # no more experts than rows can have one
+    (20, 3, 1024, 16384, "fp8", 0, "ring"),                                             # no more experts than rows can have one
+    (200, 3, 1024, 8192, "nk", 0, "direct"), (64, 1, 2048, 1408, "nk", 2, "direct"), (64, 2, 2048, 1408, "fp8", 2, "direct"),
     (64, 64, 1024, 2048, "nk", 3, "staged"), (64, 5000, 1024, 1408, "nk", 3, "staged"),
     (64, 5900, 1024, 1408, "nk", 3, "ring"), (64, 5900, 1000, 1408, "nk", 3, "staged"), # GATED: more than two rounds for certain
     (128, 512, 4096, 1536, "kn", 2, "ring"),
@@ -1484,7 +1487,7 @@ def test_kernel_choice_for_few_rows(E, rows, K, N, layout, epi, kernel):
     even = torch.arange(E + 1) * rows // E
     hot = torch.cat([torch.zeros(1, dtype=torch.int64), (torch.arange(E) * (rows // 10) // max(E - 1, 1)) + rows - rows // 10])
     want = {"ring": "grouped_gemm_ring_kernel<fmoe::RingCfg<64,", "stream": "grouped_gemm_stream_kernel<",
-            "staged": "grouped_gemm_kernel<fmoe::TileCfg<64, 256,"}[kernel]
+            "staged": "grouped_gemm_kernel<fmoe::TileCfg<64, 256,", "direct": "grouped_gemm_direct_kernel<"}[kernel]
     for off in (even.cuda(), hot.cuda()):
         ran, = kernels_run(lambda: ops.grouped_gemm(off, *args, **kw))
         assert want in ran, ran
