@@ -243,7 +243,7 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
 static bool split_takes(const fmoe_gemm_desc* d, const GemmParams& p, int sel) {
     const bool fp8 = d->a_dtype == FMOE_E4M3;
     const int esize = fp8 ? 1 : 2, pair = 128 / esize;
-    return sel == kSelRing && !p.direct && d->a_dtype != FMOE_F32 && d->epilogue != FMOE_EPI_GATED && !d->k_window && !d->a2 && d->a_stride_k <= 1 && !d->a_silu &&
+    return sel == kSelRing && (!p.direct || split_before_direct(p, esize, d->epilogue)) && d->a_dtype != FMOE_F32 && d->epilogue != FMOE_EPI_GATED && !d->k_window && !d->a2 && d->a_stride_k <= 1 && !d->a_silu &&
            p.E <= (fp8 ? TileRing5::kMaxExperts : TileRing5W::kMaxExperts) && p.total_rows < ((int64_t)1 << 31) &&
            lds_per_block() >= TileRing5::LDS_BYTES &&
            (p.K % pair == 0 ? p.K >= 4 * pair : !fp8 && ring_tail_takes(esize, p.K, p.E, p.total_rows)) && split_pays(p, esize, d->epilogue);

@@ -271,6 +271,16 @@ inline bool split_pays(const GemmParams& p, int esize, int epilogue) {
     return split_pieces((int)rest, pairs, (int)blocks, &cost) > 1 && 10 * pairs - cost >= 80;
 }
 
+// ... and where it does so with a call that the few-tiles kernel takes as well (96 rows per expert and more): bf16, beyond one of that kernel's
+// 64 x 64 tiles per CU, and for K of more than 3584.  us, few-tiles kernel / cut; of 130 such calls the mean and the extremes of the ratio, even
+// load / hot: more tiles than CUs 1.31 (0.68 to 1.84) / 1.47 (0.95 to 1.82), 2000 rows, 8 experts, 4096 -> 512 34.2 / 33.3, hot 60.4 / 33.1; up to
+// one per CU, K of 3904 and 4096 1.08 (0.86 to 1.36) / 1.05 (0.86 to 1.19), 766 rows, 6 experts, 3904 -> 640 32.3 / 26.6; of 1536 to 3072 0.87 (0.65 to
+// 1.12) / 0.84 (0.66 to 0.99).  e4m3, 30 calls, 0.75 (0.65 to 0.97).
+inline bool split_before_direct(const GemmParams& p, int esize, int epilogue) {
+    return esize == 2 &&
+           (p.K > 3584 || most_row_tiles(p.total_rows, p.E, 64) * direct_columns(p.N, epilogue == FMOE_EPI_SWIGLU) > compute_units());
+}
+
 // The 5-slot ring needs every byte of a 160 KB LDS, an even number of K-slices per tile,
 // row numbers that fit 32 bits and few enough experts for the register tables.
 template <bool FP8, int EPI>

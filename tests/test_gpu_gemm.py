@@ -1368,6 +1368,22 @@ def test_streaming_kernel_choice(E, rows, K, N, dtype, direct):
     assert ("grouped_gemm_direct_kernel<" in ran) == direct, ran
 
 
+@pytest.mark.parametrize("E,rows,K,N,dtype,cut", [
+    (6, 766, 3592, 640, "bf16", True), (6, 766, 3584, 640, "bf16", False), (6, 766, 3968, 640, "fp8", False),       # one tile per CU: by K
+    (8, 2000, 3072, 448, "bf16", True), (8, 2000, 3072, 384, "bf16", False), (8, 2000, 4096, 512, "bf16", True),    # 273 and 234 tiles
+])
+def test_cut_along_k_or_few_tiles_kernel(E, rows, K, N, dtype, cut):
+    """Which of the two runs a call that both take, on either side of the rule's lines."""
+    from fast_moe_amd.kernels.hip import ops
+    dt = {"bf16": BF16, "fp8": torch.float8_e4m3fn}[dtype]
+    x, w = torch.zeros(rows, K, device="cuda").to(dt), torch.zeros(E, N, K, dtype=BF16, device="cuda").to(dt).permute(0, 2, 1)
+    kw = dict(a_scale=torch.ones(rows, device="cuda"), b_scale=torch.ones(E, N, device="cuda")) if dtype == "fp8" else {}
+    off = (torch.arange(E + 1) * rows // E).cuda()
+    ran = kernels_run(lambda: ops.grouped_gemm(off, x, w, total_rows=rows, **kw))
+    names = [n.split("<")[0].split("::")[-1] for n in ran]
+    assert names == (["grouped_gemm_ring_kernel", "split_reduce_kernel"] if cut else ["grouped_gemm_direct_kernel"]), ran
+
+
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
     (3, 130, 136, 264, "nk", 0), (3, 130, 192, 136, "kn", 0),       # the least K: three pairs of K-slices, the last in part / whole
     (1, 64, 256, 256, "kn", 1), (1, 65, 256, 256, "nk", 1),         # one whole tile; one row more
