@@ -550,6 +550,44 @@ void launch_generic(bool silu, bool lane_per_row, const void* a_, int64_t total,
 #undef FMOE_ARGS
 }
 
+// Where the one launch is faster than the form of a lane (under 16 rows: a wave) per row, whose time is a serial walk over the columns.  us, lane
+// per row / one launch: 64 rows, 12 columns 5.3 / 4.5, 16 6.5 / 4.3, 44 16.4 / 4.5; 32768 rows, 12 6.1 / 5.6, 16 7.6 / 5.4; 2^17 rows, 16 8.4 / 12.0,
+// 24 12.0 / 12.5, 32 16.5 / 12.3; 2^19 rows, 24 31 / 40, 32 54 / 39.  Wave per row: 8 rows, 1024 columns 6.2 / 7.3, 2048 9.9 / 7.9.
+inline bool cols_one_pays(int64_t total_rows, int64_t rows, int64_t cols) {
+    if (rows < 16) return cols > 1024;
+    return cols >= (total_rows <= (1 << 15) ? 16 : 32);
+}
+
+// What the forms for rows that are columns in memory take: bf16, memory rows of whole aligned 16-byte chunks, result rows of whole dwords.
+inline bool takes_cols(int a_dtype, int64_t batch, int64_t rows, int64_t cols, int64_t a_sb, int64_t a_sr, int64_t a_sc, int apply_silu) {
+    return a_dtype == FMOE_BF16 && !apply_silu && a_sr == 1 && a_sc >= rows && rows % 8 == 0 && cols % 4 == 0 &&
+           a_sc % 8 == 0 && (batch == 1 || a_sb % 8 == 0) && batch >= 1 && batch <= 65535 && rows >= 8 && rows < (1 << 27) &&
+           (cols + kColTileK - 1) / kColTileK <= 65535 && (cols > kColOneMost || cols_one_pays(batch * rows, rows, cols));
+}
+inline bool cols_result(const void* a, const uint8_t* q, int64_t cols, int64_t q_sb, int64_t q_sr, int64_t q_sc) {
+    return aligned16(a) && q_sc == 1 && q_sr % 4 == 0 && q_sb % 4 == 0 && q_sr >= cols && (reinterpret_cast<uintptr_t>(q) & 3u) == 0;
+}
+inline int wide_cols(const uint8_t* q, int64_t q_sb, int64_t q_sr) {
+    return (reinterpret_cast<uintptr_t>(q) & 15u) == 0 && q_sr % 16 == 0 && q_sb % 16 == 0;
+}
+
+int launch_cols_one(const uint16_t* a, int64_t batch, int64_t rows, int64_t cols, int64_t a_sb, int64_t a_sc, uint8_t* q, int64_t q_sb,
+                    int64_t q_sr, float* scale, int recip, hipStream_t stream) {
+    auto one = [&](auto kern, int strip, int threads) {
+        const int strips = (int)((rows + strip - 1) / strip);
+        kern<<<dim3((unsigned)(strips > 8 ? (strips + 7) / 8 * 8 : strips), (unsigned)batch), threads, 0, stream>>>(
+            a, rows, cols, a_sb, a_sc, q, q_sb, q_sr, scale, recip, wide_cols(q, q_sb, q_sr), strips);
+        return check_launch("fmoe_quant_rows_e4m3");
+    };
+    if (cols <= 256) return one(quant_cols_one<32, 256, 1>, 32, 256);
+    if (cols <= 512) return one(quant_cols_one<32, 256, 2>, 32, 256);
+    if (cols <= 1024) return one(quant_cols_one<64, 512, 4>, 64, 512);
+    if (cols <= 1536) return one(quant_cols_one<32, 512, 3>, 32, 512);
+    if (cols <= 2048) return one(quant_cols_one<32, 512, 4>, 32, 512);
+    if (cols <= 3072) return one(quant_cols_one<32, 512, 6>, 32, 512);
+    return one(quant_cols_one<32, 1024, 4>, 32, 1024);
+}
+
 }  // namespace
 }  // namespace fmoe
 
@@ -602,6 +640,8 @@ extern "C" int fmoe_quant_rows_e4m3(const void* a, int a_dtype, int64_t batch, i
                                                                               q, q_sb, q_sr, scale, store_reciprocal);
         return check_launch("fmoe_quant_rows_e4m3");
     }
+    if (cols <= kColOneMost && takes_cols(a_dtype, batch, rows, cols, a_sb, a_sr, a_sc, apply_silu) && cols_result(a, q, cols, q_sb, q_sr, q_sc))
+        return launch_cols_one((const uint16_t*)a, batch, rows, cols, a_sb, a_sc, q, q_sb, q_sr, scale, store_reciprocal, stream);
     const bool lane_per_row = a_sc != 1 && a_sr == 1 && rows >= 16;
     if (a_dtype == FMOE_BF16)
         launch_generic<uint16_t>(apply_silu != 0, lane_per_row, a, total, rows, cols, a_sb, a_sr, a_sc, q,
@@ -612,27 +652,9 @@ extern "C" int fmoe_quant_rows_e4m3(const void* a, int a_dtype, int64_t batch, i
     return check_launch("fmoe_quant_rows_e4m3");
 }
 
-// Where the two launches are faster than the one of the other form.  A caller that allocates the scratch through torch pays
-// 3 us of host time for the second launch and the scratch, and a serial walk over a few columns is short: us per call,
-// lane per row / two launches, 40 columns: 15.0 / 18.4 (64 rows), 17.1 / 18.2 (32768); 48 columns 17.9 / 18.4 and 21.0 / 18.4.
-// With many rows the crossing moves down: 2^16 rows x 24 columns 15.2 / 18.4, 2^19 x 16 15.4 / 24.4, 2^19 x 24 30.9 / 26.1.
-// Under 16 rows the other form is a wave per row, good for more columns: 8 rows x 512 columns 15.3 / 18.9, 8 x 65536 248 / 19.
-static bool cols_pays(int64_t total_rows, int64_t rows, int64_t cols) {
-    if (rows < 16) return cols > 4096;
-    return cols > 40 || (cols > 16 && total_rows > ((int64_t)1 << 17));
-}
-
-// What the two-launch form takes: bf16, memory rows of whole aligned 16-byte chunks, result rows of whole dwords.
-static bool takes_cols(int a_dtype, int64_t batch, int64_t rows, int64_t cols, int64_t a_sb, int64_t a_sr, int64_t a_sc,
-                       int apply_silu) {
-    return a_dtype == FMOE_BF16 && !apply_silu && a_sr == 1 && a_sc >= rows && rows % 8 == 0 && cols % 4 == 0 &&
-           a_sc % 8 == 0 && (batch == 1 || a_sb % 8 == 0) && batch >= 1 && batch <= 65535 && rows >= 8 &&
-           (cols + kColTileK - 1) / kColTileK <= 65535 && cols_pays(batch * rows, rows, cols);
-}
-
 extern "C" size_t fmoe_quant_rows_workspace_bytes(int a_dtype, int64_t batch, int64_t rows, int64_t cols, int64_t a_sb,
                                                   int64_t a_sr, int64_t a_sc, int apply_silu) {
-    if (!takes_cols(a_dtype, batch, rows, cols, a_sb, a_sr, a_sc, apply_silu)) return 0;
+    if (cols <= kColOneMost || !takes_cols(a_dtype, batch, rows, cols, a_sb, a_sr, a_sc, apply_silu)) return 0;
     return (size_t)col_splits(batch, rows, cols) * (size_t)(batch * rows) * sizeof(uint32_t);
 }
 
@@ -641,39 +663,18 @@ extern "C" int fmoe_quant_rows_e4m3_ws(const void* a, int a_dtype, int64_t batch
                                        int64_t q_sb, int64_t q_sr, int64_t q_sc, float* scale, int store_reciprocal,
                                        void* workspace, size_t workspace_bytes, fmoe_stream_t stream_) {
     const size_t need = fmoe_quant_rows_workspace_bytes(a_dtype, batch, rows, cols, a_sb, a_sr, a_sc, apply_silu);
-    const bool cols_form = need > 0 && workspace_bytes >= need && workspace && a && q && scale && aligned16(a) &&
-                           q_sc == 1 && q_sr % 4 == 0 && q_sb % 4 == 0 && q_sr >= cols &&
-                           (reinterpret_cast<uintptr_t>(q) & 3u) == 0;
-    if (!cols_form)
+    if (need == 0 || workspace_bytes < need || !workspace || !a || !q || !scale || !cols_result(a, q, cols, q_sb, q_sr, q_sc))
         return fmoe_quant_rows_e4m3(a, a_dtype, batch, rows, cols, a_sb, a_sr, a_sc, apply_silu, q, q_sb, q_sr, q_sc,
                                     scale, store_reciprocal, stream_);
     hipStream_t stream = (hipStream_t)stream_;
-    const int wide = (reinterpret_cast<uintptr_t>(q) & 15u) == 0 && q_sr % 16 == 0 && q_sb % 16 == 0;
-    if (cols <= kColOneMost) {
-        auto one = [&](auto kern, int strip, int threads) {
-            const int strips = (int)((rows + strip - 1) / strip);
-            kern<<<dim3((unsigned)(strips > 8 ? (strips + 7) / 8 * 8 : strips), (unsigned)batch), threads, 0, stream>>>(
-                (const uint16_t*)a, rows, cols, a_sb, a_sc, q, q_sb, q_sr, scale, store_reciprocal, wide, strips);
-            return check_launch("fmoe_quant_rows_e4m3_ws");
-        };
-        FMOE_REQUIRE((rows + 7) / 8 < ((int64_t)1 << 31) - 8, "fmoe_quant_rows_e4m3_ws: too many rows");
-        if (cols <= 256) return one(quant_cols_one<32, 256, 1>, 32, 256);
-        if (cols <= 512) return one(quant_cols_one<32, 256, 2>, 32, 256);
-        if (cols <= 1024) return one(quant_cols_one<64, 512, 4>, 64, 512);
-        if (cols <= 1536) return one(quant_cols_one<32, 512, 3>, 32, 512);
-        if (cols <= 2048) return one(quant_cols_one<32, 512, 4>, 32, 512);
-        if (cols <= 3072) return one(quant_cols_one<32, 512, 6>, 32, 512);
-        return one(quant_cols_one<32, 1024, 4>, 32, 1024);
-    }
     const int splits = col_splits(batch, rows, cols);
     const int64_t per_split = (cols + splits - 1) / splits;
     const int64_t strips = (rows + kColTileN - 1) / kColTileN;
-    FMOE_REQUIRE(strips < ((int64_t)1 << 31), "fmoe_quant_rows_e4m3_ws: too many rows");
     uint32_t* part = (uint32_t*)workspace;
     quant_cols_amax<<<dim3((unsigned)strips, (unsigned)splits, (unsigned)batch), 256, 0, stream>>>(
         (const uint16_t*)a, rows, cols, a_sb, a_sc, part, batch * rows, per_split);
     quant_cols_store<<<dim3((unsigned)strips, (unsigned)((cols + kColTileK - 1) / kColTileK), (unsigned)batch), 256, 0,
                        stream>>>((const uint16_t*)a, rows, cols, a_sb, a_sc, part, splits, batch * rows, q, q_sb, q_sr,
-                                 scale, store_reciprocal, wide);
+                                 scale, store_reciprocal, wide_cols(q, q_sb, q_sr));
     return check_launch("fmoe_quant_rows_e4m3_ws");
 }

@@ -167,9 +167,10 @@ int fmoe_quant_rows_e4m3(const void* a, int a_dtype, int64_t batch, int64_t rows
                          fmoe_stream_t stream);
 
 /*
- * The same with a scratch buffer of the caller (fmoe_quant_rows_workspace_bytes bytes; 0: none is needed), which
+ * The same with a scratch buffer of the caller (fmoe_quant_rows_workspace_bytes bytes; 0: none is used), which
  * lets matrices whose rows are columns in memory (a_stride_r == 1: an [E, K, N] weight quantised per output
- * column) be read and written in whole lines by the whole chip.  Same bytes and scales.
+ * column) with more than 4096 columns be read and written in whole lines by the whole chip; up to 4096 both
+ * functions do so without one.  Same bytes and scales.
  */
 size_t fmoe_quant_rows_workspace_bytes(int a_dtype, int64_t batch, int64_t rows, int64_t cols,
                                        int64_t a_stride_b, int64_t a_stride_r, int64_t a_stride_c,

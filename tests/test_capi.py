@@ -345,11 +345,11 @@ def test_the_built_host_module_loads(lib):
 
 
 @pytest.mark.parametrize("E,K,N,two_launches", [
-    (1, 8, 8, False), (1, 4096, 8, False), (1, 4100, 8, True), (1, 40, 16, False), (1, 44, 16, True), (128, 16, 4096, False),
-    (128, 20, 1024, False), (128, 20, 1032, True), (1, 44, 12, False), (1, 46, 16, False),
+    (1, 4096, 8, False), (1, 4100, 8, True), (1, 4096, 64, False), (2, 4100, 64, True), (128, 44, 1024, False),
+    (1, 4104, 12, False), (1, 4102, 16, False),
 ])
 def test_column_quantiser_scratch_rule(lib, E, K, N, two_launches):
-    """[E, K, N] weights per output column: the form with scratch on either side of the lines where it pays (few columns, few
-    rows) and of what it can read (rows in eights, columns in fours)."""
+    """[E, K, N] weights per output column: scratch is asked for from the columns on that one block's registers do not hold, where the form of
+    two launches can read the operand (rows in eights, columns in fours)."""
     need = lib.fmoe_quant_rows_workspace_bytes(1, E, N, K, K * N, 1, N, 0)       # (1: FMOE_BF16)
     assert (need > 0) == two_launches

@@ -242,7 +242,33 @@ def test_rows_that_are_columns_in_memory(E, K, N):
     assert np.array_equal((got & 0x7F) == 0x7F, nan) and np.array_equal(got[~nan], q_ref[~nan])
 
 
-@pytest.mark.parametrize("K", [44, 252, 256, 260, 512, 516, 1024, 1028, 1536, 1540, 2048, 2052, 3072, 3076, 4096])
+@pytest.mark.parametrize("E,K,N,kernel", [
+    (1, 16, 64, "quant_cols_one"), (1, 12, 64, "quant_rows_generic_lane"), (8, 16, 4096, "quant_cols_one"), (8, 16, 4104, "quant_rows_generic_lane"),
+    (9, 32, 4096, "quant_cols_one"), (1, 1028, 8, "quant_cols_one"), (1, 1024, 8, "quant_rows_generic_wave"), (1, 4096, 16, "quant_cols_one"),
+    (2, 256, 20, "quant_rows_generic_lane"), (2, 254, 32, "quant_rows_generic_lane"), (1, 4100, 16, "quant_cols_store"),
+])
+def test_column_quantiser_choice(E, K, N, kernel):
+    """[E, K, N] weights per output column: which form runs, on either side of the lines where each pays and of what they read; up to 4096
+    columns the entry without scratch runs the same one.  Bit for bit what the row kernel gives for the transposed copy."""
+    from fast_moe_amd.kernels import moe_fp8
+    from fast_moe_amd.kernels.hip import _lib
+    from tests.helpers import kernels_run
+    w = torch.randn(E, K, N, generator=torch.Generator(device="cuda").manual_seed(K + N), device="cuda").to(torch.bfloat16)
+    ran = kernels_run(lambda: moe_fp8.quantize_expert_weights(w))
+    assert f"::{kernel}<" in ran[-1] or f"::{kernel}(" in ran[-1], ran
+    q, s = moe_fp8.quantize_expert_weights(w)
+    q_ref, s_ref = moe_fp8.rowwise_quant_fp8(w.permute(0, 2, 1).contiguous())
+    assert torch.equal(q.permute(0, 2, 1).view(torch.uint8), q_ref.view(torch.uint8)) and torch.equal(s, s_ref)
+    if K <= 4096:
+        bare, scale = torch.zeros(E, N, K, dtype=torch.uint8, device="cuda"), torch.zeros(E, N, device="cuda")
+        def call():
+            assert _lib.load().fmoe_quant_rows_e4m3(w.data_ptr(), 1, E, N, K, K * N, 1, N, 0, bare.data_ptr(), N * K, K, 1, scale.data_ptr(), 0,
+                                                    torch.cuda.current_stream().cuda_stream) == 0
+        assert kernels_run(call)[-1] == ran[-1]
+        assert torch.equal(bare, q_ref.view(torch.uint8)) and torch.equal(scale, s_ref)
+
+
+@pytest.mark.parametrize("K", [32, 44, 252, 256, 260, 512, 516, 1024, 1028, 1536, 1540, 2048, 2052, 3072, 3076, 4096])
 @pytest.mark.parametrize("E,N", [(1, 16), (2, 24), (1, 72), (3, 296), (2, 544)])
 def test_columns_that_fit_a_block(E, K, N):
     """One launch for up to 4096 columns: every size of block and its remainders (strips of 32 and 64 rows, more and fewer than eight of
@@ -263,7 +289,7 @@ def test_the_column_form_allocates_scratch_only_where_it_runs():
     """The two-launch form writes rows of consecutive bytes: a result laid out like its [E, K, N] input is left to the other
     kernel, without a scratch buffer."""
     from fast_moe_amd.kernels import moe_fp8
-    w = torch.randn(2, 128, 64, device="cuda").to(torch.bfloat16)
+    w = torch.randn(2, 4100, 64, device="cuda").to(torch.bfloat16)
 
     def allocations(fn):
         fn()
@@ -273,3 +299,5 @@ def test_the_column_form_allocates_scratch_only_where_it_runs():
 
     assert allocations(lambda: moe_fp8.bmm_weight_rowwise_quant_fp8(w)) == 2        # bytes and scales
     assert allocations(lambda: moe_fp8.quantize_expert_weights(w)) == 3
+    w = w[:, :128].contiguous()         # columns that fit a block's registers: one launch
+    assert allocations(lambda: moe_fp8.quantize_expert_weights(w)) == 2
