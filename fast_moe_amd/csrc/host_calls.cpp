@@ -534,13 +534,6 @@ at::Tensor empty_rows(int64_t rows, int64_t cols, at::ScalarType dtype, const at
 bool float_matrix(const at::Tensor& t) {
     return (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16) && t.dim() == 2 && t.size(1) > 0 && t.stride(1) == 1;
 }
-// rows of t's pitch that its storage holds behind its last (ops.slack_rows)
-int64_t slack_rows(const at::Tensor& t) {
-    if (t.stride(0) < t.size(1) || t.stride(0) < 1) return 0;
-    const int64_t have = (int64_t)(t.storage().nbytes() / t.element_size()) - t.storage_offset();
-    const int64_t rows = (have - t.size(1)) / t.stride(0) + 1 - t.size(0);
-    return rows > 0 ? rows : 0;
-}
 PyObject* wrap_or_none(const at::Tensor& t) { return t.defined() ? wrap(t) : none(); }
 
 // (dy [T, D], value [T*K, D] or None, token_index, K, gates or None, gates_index or None, need_gate_grad, stream) -> (d_value, d_gates)
@@ -738,7 +731,6 @@ PyObject* py_weight_grad(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 (uintptr_t)a.data_ptr() % 16 || (uintptr_t)b.data_ptr() % 16 || E > INT32_MAX || Kin > INT32_MAX || E * N > INT32_MAX ||
                 (halves && N % 64))
                 return false;
-            if (bf16 && (slack_rows(a) < kSlackRows || slack_rows(b) < kSlackRows)) return false;
             return (bf16 && R < 128) || weight_grad_pays(dtype_code(a.scalar_type()), (int)E, (int)N, (int)Kin, R) != 0;
         },
         [&] {

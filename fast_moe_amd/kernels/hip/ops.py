@@ -292,8 +292,8 @@ def weight_grad_pays(dtype: torch.dtype, num_experts: int, m: int, n: int, rows:
 def jagged_weight_grad(dout: torch.Tensor, a_rows: torch.Tensor, offsets: torch.Tensor, halves: bool = False):
     """dW[e, n, k] = sum over the rows r of expert e of dout[r, n] * a_rows[r, k] -> [E, N, K_in],
     both operands read in place: fmoe_weight_grad where that pays (few rows, fp32), else fmoe_grouped_gemm
-    with a_stride_k (bf16).  Returns None when the operands do not qualify (dtype, alignment, no slack behind
-    them): the caller then takes the route over transposed copies.  ``halves``: dout holds the row gradients of
+    with a_stride_k (bf16, slack behind both).  Returns None when the operands do not qualify (dtype, alignment,
+    no slack): the caller then takes the route over transposed copies.  ``halves``: dout holds the row gradients of
     two matrices side by side; the result is two tensors [E, N/2, K_in] (fmoe_gemm_desc.out2)."""
     dw = _lib.host().weight_grad(dout, a_rows, offsets, int(halves), _stream(dout))
     if dw is not None:
@@ -310,8 +310,6 @@ def jagged_weight_grad(dout: torch.Tensor, a_rows: torch.Tensor, offsets: torch.
             and a_rows.stride(0) >= Kin and dout.data_ptr() % 16 == 0 and a_rows.data_ptr() % 16 == 0
             and E * N < (1 << 31) and (not halves or N % 64 == 0)):
         return None
-    if bf16 and not (slack_rows(dout) >= SLACK_ROWS and slack_rows(a_rows) >= SLACK_ROWS):
-        return None
     lib, code = _lib.load(), _DTYPE_CODE[dout.dtype]
     if (bf16 and R < 128) or lib.fmoe_weight_grad_pays(code, E, N, Kin, R):
         offsets = _i64("offsets", offsets)
@@ -322,7 +320,7 @@ def jagged_weight_grad(dout: torch.Tensor, a_rows: torch.Tensor, offsets: torch.
                                   _stream(dout))
         _lib.check(rc, "fmoe_weight_grad")
         return tuple(outs) if halves else outs[0]
-    if not bf16 or R < 128 or E > 256:
+    if not bf16 or R < 128 or E > 256 or slack_rows(dout) < SLACK_ROWS or slack_rows(a_rows) < SLACK_ROWS:
         return None
     dev = dout.device
     offsets = _i64("offsets", offsets)

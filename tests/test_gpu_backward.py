@@ -398,7 +398,8 @@ def test_weight_gradient_from_rows_in_place(lens):
     """fmoe_grouped_gemm with a_stride_k: dW[e] = dout_e^T x_e read straight from the row-major tensors
     (arbitrary row ranges, masked window ends, slack behind the last row), against per-expert matmuls."""
     from fast_moe_amd.kernels.hip import ops
-    E, N, Kin = len(lens), 264, 392                             # N, Kin tails inside the 256-wide tiles
+    from helpers import kernels_run
+    E, N, Kin = len(lens), 1032, 1160                           # N, Kin tails inside the 256-wide tiles (of which smaller matrices have too few)
     g = torch.Generator().manual_seed(11)
     lens = torch.tensor(lens)
     offsets = torch.zeros(E + 1, dtype=torch.int64)
@@ -412,6 +413,7 @@ def test_weight_gradient_from_rows_in_place(lens):
     assert ops.slack_rows(xg) >= ops.SLACK_ROWS and ops.slack_rows(x.cuda()) == 0
     out = ops.jagged_weight_grad(dg, xg, offsets.cuda())
     assert out is not None and tuple(out.shape) == (E, N, Kin)
+    assert "grouped_gemm_ring_kernel" in kernels_run(lambda: ops.jagged_weight_grad(dg, xg, offsets.cuda()))[-1]
     assert ops.jagged_weight_grad(d.cuda(), xg, offsets.cuda()) is None      # no slack behind dout: refused
     ref = torch.stack([d[offsets[e]:offsets[e + 1]].float().t() @ x[offsets[e]:offsets[e + 1]].float() for e in range(E)])
     got = out.float().cpu()
@@ -495,6 +497,22 @@ def test_gradients_of_rows_off_a_16_byte_boundary(dtype, where):
         rounded = 2.0 ** -8 * (want.abs() + bound) if dtype == BF16 else 0
         for got in grads:
             assert bool(((got[1][e].double() - want).abs() <= bound + rounded).all()), e
+
+
+@pytest.mark.parametrize("R,E", [(1, 1), (60, 3), (500, 9)])
+def test_weight_gradient_of_few_rows_needs_nothing_behind_them(R, E):
+    """Operands that end with their storage: the kernel reads nothing behind the last row, so no slack is asked for."""
+    from fast_moe_amd.kernels.hip import ops
+    from helpers import kernels_run
+    g = torch.Generator(device="cuda").manual_seed(R)
+    d, x = (torch.randn(R, n, generator=g, device="cuda").to(BF16) for n in (136, 264))
+    off = (torch.arange(E + 1) * R // E).cuda()
+    got = ops.jagged_weight_grad(d, x, off)
+    assert got is not None and "grouped_wgrad_kernel" in kernels_run(lambda: ops.jagged_weight_grad(d, x, off))[-1]
+    for e in range(E):
+        a, b = d[off[e]:off[e + 1]].double(), x[off[e]:off[e + 1]].double()
+        want, bound = a.t() @ b, (R + 1) * 2.0 ** -24 * (a.abs().t() @ b.abs())
+        assert bool(((got[e].double() - want).abs() <= bound + 2.0 ** -8 * (want.abs() + bound)).all())
 
 
 def test_large_fp32_weight_gradients_take_the_transposed_copies():
