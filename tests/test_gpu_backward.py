@@ -713,7 +713,8 @@ def test_two_weight_gradients_from_one_gemm(lens, H):
     writes): one GEMM stores each matrix's gradient into its own tensor (fmoe_gemm_desc.out2),
     bit-identical to one GEMM per matrix on the halves."""
     from fast_moe_amd.kernels.hip import ops
-    E, Kin = len(lens), 392
+    from helpers import kernels_run
+    E, Kin = len(lens), 5640                    # (narrower matrices have too few of the ring's tiles)
     g = torch.Generator().manual_seed(5)
     offsets = torch.zeros(E + 1, dtype=torch.int64)
     offsets[1:] = torch.cumsum(torch.tensor(lens), 0)
@@ -728,6 +729,8 @@ def test_two_weight_gradients_from_one_gemm(lens, H):
     one, two = ops.jagged_weight_grad(left, xg, offsets.cuda()), ops.jagged_weight_grad(right, xg, offsets.cuda())
     assert one is not None and two is not None
     assert torch.equal(pair[0], one) and torch.equal(pair[1], two)
+    for t, halves in ((both, True), (left, False)):
+        assert "grouped_gemm_ring_kernel" in kernels_run(lambda: ops.jagged_weight_grad(t, xg, offsets.cuda(), halves=halves))[-1]
     # swiglu_bwd writes such a buffer: same values as the separate form
     a, b, c = (torch.randn(R, H, generator=g).to(BF16).cuda() for _ in range(3))
     dg, du = ops.swiglu_bwd(a, b, c, joint=True)

@@ -862,7 +862,7 @@ def test_silu_jagged_bmm_fp8(lens, Din, Dout):
 
 
 @pytest.mark.parametrize("swiglu", [False, True])
-@pytest.mark.parametrize("M", [96, 8192])
+@pytest.mark.parametrize("M", [96, 600, 8192])          # the few-tiles kernel, the 64-row and the tall ring
 def test_fp8_weight_scales_at_any_alignment(M, swiglu):
     """The e4m3 epilogue loads a register quad's 4 weight scales at once when the scale tensors sit
     on 16-byte boundaries and one by one otherwise: both give the same bits."""
@@ -927,31 +927,37 @@ def test_bias_at_any_alignment(M, epi):
         assert torch.equal(run(shift, pitch), aligned), (shift, pitch)
 
 
-@pytest.mark.parametrize("rows", [256, 64])
-def test_accumulation_error_stays_under_the_floors_the_stage_checks_use(rows):
+@pytest.mark.parametrize("rows,N,kernel", [(256, 16640, "ring_kernel<fmoe::RingCfg<256,"), (64, 17408, "ring_kernel<fmoe::RingCfg<64,"),
+                                           (64, 40960, "stream_kernel<"), (64, 4096, "direct_kernel<")])
+def test_accumulation_error_stays_under_the_floors_the_stage_checks_use(rows, N, kernel):
     """The absolute-error floors of tests/chain.py (BF16_FLOOR = 2^-18, FP8_FLOOR = 2^-14 of
     S = sum |a||b|) rest on a measurement: on outputs that are small by cancellation, where the final
     bf16 rounding is out of the way, the GEMMs' error against float64 is a fraction of S that
     depends on how the MFMA adds (e4m3: 64 products per instruction in a block-aligned adder that
     keeps fewer bits than an fp32 sum).  One expert, 1536-term sums, operands that are exactly
-    representable in both types; rows = 256 runs the ring kernel, 64 the short streaming tile.
+    representable in both types.
     Asserted: both stay a factor 4 under their floor, and e4m3 does accumulate less exactly than bf16."""
     from fast_moe_amd.kernels.hip import ops
     from tests.chain import BF16_FLOOR, FP8_FLOOR
     torch.manual_seed(0)
-    K, N = 1536, 4096
+    K = 1536
     a = torch.randn(rows, K, device="cuda").to(BF16)
     w = (torch.randn(1, N, K, device="cuda") * K ** -0.5).to(BF16)
     qa, sa = ops.quant_rows_fp8(a)
     qw, sw = ops.quant_rows_fp8(w)
     off = torch.tensor([0, rows], device="cuda")
-    out8 = ops.grouped_gemm(off, qa, qw.permute(0, 2, 1), total_rows=rows, a_scale=sa, b_scale=sw.reshape(1, N))
+    run8 = lambda: ops.grouped_gemm(off, qa, qw.permute(0, 2, 1), total_rows=rows, a_scale=sa, b_scale=sw.reshape(1, N))
+    out8 = run8()
     da, dw = qa.float(), qw.float()
     scale = sa.double()[:, None] * sw[0].double()[None, :]
     exact = (da.double() @ dw[0].double().T) / scale
     S = (da.double().abs() @ dw[0].double().abs().T) / scale
     # the same values through the bf16 kernel: exact products, fp32 accumulation
-    out16 = ops.grouped_gemm(off, da.to(BF16), dw.to(BF16).permute(0, 2, 1), total_rows=rows)
+    a16, w16 = da.to(BF16), dw.to(BF16).permute(0, 2, 1)
+    run16 = lambda: ops.grouped_gemm(off, a16, w16, total_rows=rows)
+    out16 = run16()
+    for run in (run8, run16):
+        assert kernel in kernels_run(run)[0]
     exact16 = da.double() @ dw[0].double().T
     S16 = da.double().abs() @ dw[0].double().abs().T
     small8, small16 = exact.abs() < 2.0 ** -12 * S, exact16.abs() < 2.0 ** -12 * S16

@@ -225,10 +225,11 @@ def test_fp8_operators_requantise_every_call_and_take_a_kept_pair():
 
 
 @pytest.mark.parametrize("E,K,N", [(1, 4, 8), (3, 60, 72), (2, 128, 64), (2, 132, 136), (1, 1000, 8), (5, 1028, 264),
-                                   (1, 8200, 128), (2, 126, 64), (1, 4100, 8), (3, 44, 72), (4, 20, 65544)])
+                                   (1, 8200, 128), (2, 126, 64), (1, 4100, 8), (3, 44, 72), (4, 20, 65544),
+                                   (3, 4156, 72), (2, 4224, 64), (2, 4228, 136), (1, 5096, 8), (5, 5124, 264)])
 def test_rows_that_are_columns_in_memory(E, K, N):
     """[E, K, N]-contiguous weights quantised per output column: tiles of 64 rows x 128 columns, their
-    remainders on both sides, whole and partial 16-byte results (K = 126, and few columns, take one launch).  Bit for bit."""
+    remainders on both sides, whole and partial 16-byte results (from K = 4100 on; below, other forms).  Bit for bit."""
     from fast_moe_amd.kernels import moe_fp8
     g = torch.Generator().manual_seed(K + N)
     w = (torch.randn(E, K, N, generator=g) * torch.exp(torch.randn(E, 1, N, generator=g) * 4)).to(torch.bfloat16)
