@@ -8,53 +8,30 @@ namespace fmoe {
 
 namespace {
 
-// The tiles of v_mfma_f32_32x32x2_f32 (their figures are from before longer K went to the other kernel).
-// It runs 64 cycles on operands of two LDS reads, so LDS and L2 bandwidth leave room for small tiles, and small
-// tiles are what fills the chip: a launch is bound by the last round of tiles over 256 CUs (4096 rows, 8 experts,
-// 4096 -> 1024 columns: 80 tiles of 256 x 256).  Several blocks share a CU and hide each other's barriers and epilogues.
-// us per GEMM, tiles of 256 x 256 / 128 x 128 / 64 x 128 / 64 x 64:
-//   4096 rows,  8 experts, 1024 -> 4096      554 /  391 /  339 /  335      (k contiguous)
-//   4096 rows,  8 experts, 4096 -> 1024     1005 /  545 /  421 /  390
-//   9189 rows, 12 experts, 2600 -> 1000      673 /  541 /  461 /  484
-//  16384 rows,  8 experts, 1024 -> 4096     1371 / 1171 / 1172 / 1235
-//     64 rows,  8 experts, 1024 -> 2048      254 /   81 /   50 /   33
+// The tiles of v_mfma_f32_32x32x2_f32, for K of up to 64: a tile is the latency of one or two slices and its stores.  us per GEMM at K = 32 (64),
+// tiles of 64 x 64 / 64 x 128 / 64 x 256, and 256 x 256 for comparison:
+//   1000 rows, 8 experts, 1024 columns    6.8 /  8.7 / 11.0   19.6    (7.7 / 10.1 / 13.4    27.3)
+//   4096 rows, 8 experts, 1024           11.9 / 11.9 / 13.1   22.4   (14.3 / 14.5 / 15.9    30.3)
+//   4096 rows, 1 expert,  4096           33.0 / 31.5 / 31.2   43.3   (42.0 / 40.1 / 39.9    52.1)
+//   600 rows, 64 experts, 4096           29.7 / 28.7 / 22.8   57.3   (38.5 / 39.0 / 32.6    87.7)
+//   65536 rows, 16 experts, 64           11.4 / 17.9 / 25.7   22.4   (13.9 / 22.1 / 34.3    31.1)
+//   SwiGLU (gate and up fragments in one wave: not 64 x 64): 4096 rows, 8 experts, 256  - / 8.8 / 11.7, 1024 - / 19.4 / 17.2; 600 rows, 64 experts,
+//   1024  - / 16.7 / 12.4; 2000 rows, 200 experts, 256  - / 20.6 / 14.4
+// So small tiles up to four 64 x 128 ones to a CU (SwiGLU: those up to two to a CU), the wide ones beyond, where they are not half empty.  With
+// SiLU on load the same.  With n-contiguous weights, whose parking costs four LDS writes a chunk, the small ones (four to seven blocks per CU).
 typedef TileCfg<64, 128, 2, 2> TileF32Wide;     // 4 waves, wave tile 32 x 64
 typedef TileCfg<64, 64, 2, 2> TileF32;          // 4 waves, wave tile 32 x 32
 
-// From four wide tiles per CU on, the remainder of the last round is a small share and the 25 % fewer operand bytes of the
-// wide tile count for more (1172 against 1235 us above); below, the finer tile fills the chip better (390 against 421).  With
-// SiLU on load, which every column of tiles repeats, from one per CU on: 375 rows, 16 experts, 860 -> 3320 columns 91 / 107 us,
-// 300 rows, 8 experts, 1024 -> 1024 80 / 61.
-// With n-contiguous weights, whose parking costs four LDS writes a chunk, the small tile was faster at every size (four to
-// seven blocks per CU instead of three): 398 / 350, 527 / 413, 1425 / 1299 us for the first, second and fourth line.
-// SwiGLU needs gate and up fragments in one wave: wide, or 64 x 256 where that is one round of tiles (two blocks per CU) and
-// wide more than one (three): 2000 rows, 200 experts, 256 -> 2 x 256 51.0 / 45.2 us.
-//
-// Whole rounds of 256 x 256 tiles, one block per CU, are faster still: a quarter of the operand reads and of the SiLU.  us,
-// 256 x 256 / 64 x 128: 4096 rows, 1 expert, 4096 -> 4096 (one round) 1037 / 1123, SiLU on load 1241 / 1479; 8192 rows, 2048 -> 4096
-// 1053 / 1123; but with 1056 tiles (65536 rows, 8 experts, 512 -> 1024: a fifth round of 32) 750 / 614.  The bound on the row
-// tiles holds however the experts share the rows; 6 % (15 % with SiLU on load) is what an unfilled remainder may cost.
 template <int EPI, int LOADS, bool A_SILU>
 int pick_tile(const GemmParams& p, hipStream_t stream) {
-    constexpr int out_cols = EPI == FMOE_EPI_SWIGLU ? 2 : 1;    // tile columns per output column
-    const int64_t cus = compute_units();
-    auto tiles = [&](int bm, int bn) { return (p.total_rows / bm + p.E) * ((p.N + bn / out_cols - 1) / (bn / out_cols)); };
+    constexpr bool swiglu = EPI == FMOE_EPI_SWIGLU;
     if constexpr (LOADS == kLoadChunks) {
-        const int64_t most = (p.total_rows + 255 * (int64_t)p.E) / 256 * ((p.N + 256 / out_cols - 1) / (256 / out_cols));
-        const double rounds = (double)((most + cus - 1) / cus * cus) * (256 * 256 / out_cols);
-        if (rounds <= (A_SILU ? 1.15 : 1.06) * (double)p.total_rows * p.N)
-            return launch_gemm<TileBig, kDtF32, EPI, LOADS, A_SILU>(p, stream);
-        if constexpr (EPI == FMOE_EPI_SWIGLU) {
-            if (tiles(TileF32Wide::BM, TileF32Wide::BN) > 3 * cus && tiles(TileSmall::BM, TileSmall::BN) <= 2 * cus)
-                return launch_gemm<TileSmall, kDtF32, EPI, LOADS, A_SILU>(p, stream);
-        }
+        constexpr int columns = swiglu ? TileF32Wide::BN / 2 : TileF32Wide::BN;
+        const int64_t tiles = (p.total_rows / TileF32Wide::BM + p.E) * ((p.N + columns - 1) / columns);
+        if (tiles > (swiglu ? 2 : 4) * (int64_t)compute_units() && p.N > 64)
+            return launch_gemm<TileSmall, kDtF32, EPI, LOADS, A_SILU>(p, stream);
     }
-    if constexpr (EPI != FMOE_EPI_SWIGLU) {
-        if (LOADS == kLoadChunksN || tiles(TileF32Wide::BM, TileF32Wide::BN) < (A_SILU ? 1 : 4) * cus)
-            return launch_gemm<TileF32, kDtF32, EPI, LOADS, A_SILU>(p, stream);
-    }
-    if constexpr (EPI == FMOE_EPI_SWIGLU || LOADS != kLoadChunksN)
-        return launch_gemm<TileF32Wide, kDtF32, EPI, LOADS, A_SILU>(p, stream);
+    return launch_gemm<std::conditional_t<swiglu, TileF32Wide, TileF32>, kDtF32, EPI, LOADS, A_SILU>(p, stream);
 }
 
 template <typename TL, int EPI, bool NCONT, bool A_SILU>
@@ -66,8 +43,8 @@ int launch_f32x3(GemmParams p, hipStream_t stream) {
     return launch_tiles<TL>(kern, p, attr_done, stream);
 }
 
-// From three slices on; up to two (K = 64) there is hardly a loop to be faster in (4096 rows, 8 experts, 512 columns, K = 72: 10.2 us on
-// v_mfma_f32_32x32x2_f32, 9.6 here; SwiGLU, K = 68: 15.2 / 13.7).
+// From three slices on.  Up to two (K = 64) it is level or ahead too (4096 rows, 8 experts, 4096 columns, K = 32 30.6 / 27.4), but a third behind
+// where many experts have a few rows each (2000 rows, 200 experts, 4096 columns, K = 64 108 / 157, SwiGLU 218 / 342).
 //
 // us per GEMM, v_mfma_f32_32x32x2_f32 on its best tile / three parts on 64 x 64 / 64 x 128 / 128 x 128:
 //   4096 rows,  8 experts, 1024 -> 4096 columns  291 / 274 / 252 / 225        16384 rows  1130 / 1051 / 960 / 865

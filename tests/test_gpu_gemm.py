@@ -1101,11 +1101,12 @@ def test_odd_numbers_of_whole_slices(E, rows, K, N, dtype, tail):
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
     (3, 190, 36, 68, "kn", 0), (3, 190, 36, 60, "nk", 0),       # below / above one 64-column tile, a rest of one chunk
     (1, 64, 32, 64, "kn", 1), (1, 65, 4, 4, "kn", 0),           # whole tiles; one row more, the least K and N
-    (5, 700, 1000, 132, "kn", 2), (5, 700, 1000, 132, "nk", 2), # gate and up halves of a 128-column tile
-    (2, 2600, 100, 3500, "nk", 1), (2, 2600, 100, 3500, "kn", 1),   # enough tiles for the wide form (nk)
-    (70, 900, 68, 256, "kn", 0),                                # more experts than lanes, some empty
-    (1, 4096, 100, 4096, "nk", 1), (1, 4000, 36, 4096, "nk", 2),    # whole rounds of 256 x 256 tiles
-    (1, 4096, 40, 4092, "nk", "silu"), (200, 2000, 256, 256, "nk", 2), (200, 2000, 40, 256, "nk", "silu"),
+    (5, 700, 60, 132, "kn", 2), (5, 700, 60, 132, "nk", 2),     # gate and up halves of a 128-column tile
+    (2, 2600, 60, 3500, "nk", 1), (2, 2600, 60, 3500, "kn", 1),     # enough tiles for the wide form (nk)
+    (70, 900, 64, 256, "kn", 0),                                # more experts than lanes, some empty
+    (1, 4000, 36, 4096, "nk", 2),
+    (1, 4096, 40, 4092, "nk", "silu"), (200, 2000, 64, 256, "nk", 2), (200, 2000, 40, 256, "nk", "silu"),
+    (5, 700, 1000, 132, "kn", 2), (2, 2600, 100, 3500, "nk", 1), (1, 4096, 100, 4096, "nk", 1), (200, 2000, 256, 256, "nk", 2),  # (gemm_f32x3.h)
     (3, 190, 36, 60, "nk", "silu"), (3, 190, 36, 68, "kn", "silu"),
 ])
 def test_fp32_kernel_tiles_and_weight_layouts(E, rows, K, N, layout, epi):
@@ -1138,21 +1139,28 @@ def test_fp32_kernel_tiles_and_weight_layouts(E, rows, K, N, layout, epi):
         assert bool(((out[int(off[e]):int(off[e + 1])].double() - want).abs() <= err).all()), f"expert {e}"
 
 
-@pytest.mark.parametrize("E,rows,N,epi,tile", [
-    (1, 4096, 4096, 0, "256, 256"), (1, 4097, 4096, 0, "64, 128"), (1, 3868, 4096, 0, "256, 256"), (1, 3860, 4096, 0, "64, 128"),
-    (2, 4096, 4096, 0, "64, 128"), (1, 4096, 4096, 2, "256, 256"), (1, 4097, 4096, 2, "64, 128"),
-    (1, 3580, 4096, "silu", "256, 256"), (1, 3560, 4096, "silu", "64, 128"),
-    (1, 4000, 512, "silu", "64, 64"), (1, 4096, 512, "silu", "64, 128"), (1, 4096, 512, 0, "64, 64"),
-    (200, 2000, 256, 2, "64, 256"), (200, 2000, 384, 2, "64, 128"), (8, 2000, 256, 2, "64, 128"),
+@pytest.mark.parametrize("E,rows,N,layout,epi,tile", [
+    (1, 4096, 1920, "nk", 0, "64, 64"), (1, 4096, 1924, "nk", 0, "64, 256"), (1, 4096, 4096, "kn", 0, "64, 64"),
+    (1, 4096, 1920, "nk", "silu", "64, 64"), (1, 4096, 1924, "nk", "silu", "64, 256"), (1, 4096, 4096, "kn", "silu", "64, 64"),
+    (1, 65536, 64, "nk", 0, "64, 64"), (1, 65536, 68, "nk", 1, "64, 256"),              # half empty otherwise
+    (1, 4096, 448, "nk", 2, "64, 128"), (1, 4096, 452, "nk", 2, "64, 256"), (1, 32768, 64, "nk", 2, "64, 128"), (200, 2000, 256, "nk", 2, "64, 256"),
+    (1, 4096, 4096, "kn", 2, "64, 128"),
 ])
-def test_fp32_tile_choice(E, rows, N, epi, tile):
-    """The tile on either side of the lines of the fp32 rule, from a trace."""
+@pytest.mark.parametrize("K", [4, 64])
+def test_fp32_tile_choice(E, rows, N, layout, epi, tile, K):
+    """The tile on either side of the lines of the fp32 rule for short K, from a trace; small integers: exact sums."""
     from fast_moe_amd.kernels.hip import ops
-    x, w = torch.zeros(rows, 32, device="cuda"), torch.zeros(E, N, 32, device="cuda").permute(0, 2, 1)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x, w = (torch.randint(-3, 4, s, generator=g, device="cuda").float() for s in ((rows, K), (E, K, N) if layout == "kn" else (E, N, K)))
+    w = w if layout == "kn" else w.permute(0, 2, 1)
     off = (torch.arange(E + 1) * rows // E).cuda()
     a_silu, epi = epi == "silu", 0 if epi == "silu" else epi
-    ran, = kernels_run(lambda: ops.grouped_gemm(off, x, w, total_rows=rows, epilogue=epi, b2=w if epi else None, a_silu=a_silu))
+    run = lambda: ops.grouped_gemm(off, x, w, total_rows=rows, epilogue=epi, b2=w if epi == 2 else None, a_silu=a_silu)
+    ran, = kernels_run(run)
     assert f"grouped_gemm_kernel<fmoe::TileCfg<{tile}," in ran, ran
+    if epi == 0 and not a_silu:
+        out = run()
+        assert all(torch.equal(out[off[e]:off[e + 1]], x[off[e]:off[e + 1]] @ w[e]) for e in range(E))
 
 
 @pytest.mark.parametrize("E,rows,K,N,layout,epi,tile", [
