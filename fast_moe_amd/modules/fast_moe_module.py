@@ -17,6 +17,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd.profiler import record_function
 from torch.nn.modules import module as _nn_module
+from torch.utils._device import DeviceContext
 
 from ..kernels.hip import _lib, ops
 from ..kernels.hip._lib import EPI_NONE, EPI_SILU
@@ -105,11 +106,11 @@ class FastMoELayer(nn.Module):
 
     def _scores(self, x: torch.Tensor) -> torch.Tensor:
         """The gate's probabilities [tokens, E]: from one launch where the batch is small, nothing needs a gradient and the gate is the
-        class's own; a caller's module, hooks and autocast are asked through the modules, and so are other shapes, which they refuse."""
+        class's own; a caller's module, hooks, modes and autocast are asked through the modules, and so are other shapes, which they refuse."""
         gate = self.gate
         if type(x) is torch.Tensor and x.ndim == 3 and x.shape[2] == self.input_dim and x.numel() <= _SMALL_BATCH * self.input_dim \
                 and type(gate) is GatingNetwork and type(gate.gate) is nn.Linear and GatingNetwork.forward is _GATE_FORWARD \
-                and not _watched(gate) and not _watched(gate.gate) and not torch.is_autocast_enabled():
+                and not _watched(gate) and not _watched(gate.gate) and not torch.is_autocast_enabled() and not _mode_active():
             weight, bias = gate.gate.weight, gate.gate.bias
             if not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)):
                 scores = ops.gate_softmax(x.reshape(-1, self.input_dim), weight, bias)
@@ -154,6 +155,13 @@ class FastMoELayer(nn.Module):
 _ROUTE = FastMoELayer.route     # what the native call stands for
 _GATE_FORWARD = GatingNetwork.forward
 _SMALL_BATCH = 128              # (the library's own rule, fmoe_gate_softmax_pays, without a call for the others)
+
+
+def _mode_active() -> bool:
+    """Whether a dispatch or function mode would see the gate's operators (torch.set_default_device is one that has no use for them)."""
+    c = torch._C
+    return bool(c._len_torch_dispatch_stack()) or any(type(c._get_function_stack_at(i)) is not DeviceContext
+                                                      for i in range(c._len_torch_function_stack()))
 
 
 def _watched(module: nn.Module) -> bool:

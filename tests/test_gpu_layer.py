@@ -360,6 +360,43 @@ def test_gate_modules_that_are_watched_are_called(monkeypatch):
     assert len(fused) == 2
 
 
+def test_modes_see_the_gate_of_a_small_batch(monkeypatch):
+    """A dispatch or function mode of the caller's sees Linear and softmax as for larger batches; the mode behind a default device does not
+    turn the one launch off."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from fast_moe_amd import FastMoELayer
+    from fast_moe_amd.kernels.hip import ops
+    layer = FastMoELayer(64, 96, 64, 4).to(BF16).cuda()
+    x = torch.randn(2, 8, 64, device="cuda").to(BF16)
+    seen, fused, real = [], [], ops.gate_softmax
+    monkeypatch.setattr(ops, "gate_softmax", lambda *a: fused.append(1) or real(*a))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.__name__)
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad():
+        want = layer(x, 2)
+        for mode in (Dispatch, Function):
+            seen.clear()
+            with mode():
+                y = layer(x, 2)
+            assert any("addmm" in n or n == "linear" for n in seen) and any("softmax" in n for n in seen), seen
+            torch.testing.assert_close(y, want, atol=2e-2, rtol=2e-2)
+        assert len(fused) == 1
+        with torch.device("cuda"):
+            layer(x, 2)
+        assert len(fused) == 2
+
+
 @pytest.mark.parametrize("T,D,H", [(64, 128, 256), (4096, 256, 4096)])
 def test_short_and_split_passes_replay_from_a_graph(T, D, H):
     """A small batch (gate and routing in one launch each) and one whose second GEMM is cut along K (its workspace comes from the graph's
