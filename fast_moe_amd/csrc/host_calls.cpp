@@ -215,9 +215,14 @@ at::Tensor allocate(fmoe_gemm_desc& d, const at::Tensor& like) {
 // (the workspace may be handed out again as soon as the call is issued: what takes it runs behind the call on the stream)
 int gemm(const fmoe_gemm_desc& d, const at::Tensor& like, void* stream) {
     const size_t bytes = gemm_workspace_bytes(&d);
-    if (!bytes) return c_grouped_gemm(&d, stream);
-    const at::Tensor workspace = empty({(int64_t)bytes}, at::kByte, like);
-    return c_grouped_gemm_ws(&d, workspace.data_ptr(), bytes, stream);
+    at::Tensor workspace;
+    if (bytes) {
+        try {
+            workspace = empty({(int64_t)bytes}, at::kByte, like);
+        } catch (const c10::OutOfMemoryError&) {    // it makes the call faster, not possible
+        }
+    }
+    return workspace.defined() ? c_grouped_gemm_ws(&d, workspace.data_ptr(), bytes, stream) : c_grouped_gemm(&d, stream);
 }
 
 struct Combine {

@@ -503,9 +503,13 @@ def grouped_gemm(offsets: torch.Tensor, a: torch.Tensor, b: torch.Tensor, *, tot
             d.a_silu = 1
     if plan_only:
         return gemm_plan(d)
-    ws_bytes = lib.fmoe_grouped_gemm_workspace_bytes(ctypes.byref(d))
+    ws_bytes, ws = lib.fmoe_grouped_gemm_workspace_bytes(ctypes.byref(d)), None
     if ws_bytes:
-        ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=a.device)
+        try:
+            ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=a.device)
+        except torch.OutOfMemoryError:      # it makes the call faster, not possible
+            pass
+    if ws is not None:
         rc = lib.fmoe_grouped_gemm_ws(ctypes.byref(d), ws.data_ptr(), ws_bytes, _stream(a))
     else:
         rc = lib.fmoe_grouped_gemm(ctypes.byref(d), _stream(a))

@@ -1382,6 +1382,33 @@ def test_streaming_kernel_choice(E, rows, K, N, dtype, direct):
     assert ("grouped_gemm_direct_kernel<" in ran) == direct, ran
 
 
+@pytest.mark.parametrize("native", [True, False])
+def test_calls_without_memory_for_a_workspace_run_uncut(native):
+    """Less memory left than the 64 MiB of the cut along K (a limit of the allocator's): the call runs as it does without a workspace."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    E, rows, K, N = 8, 2000, 4096, 512
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w = torch.randn(rows, K, generator=g, device="cuda").to(BF16), (torch.randn(E, N, K, generator=g, device="cuda") * K ** -0.5).to(BF16)
+    off, host = (torch.arange(E + 1) * rows // E).cuda(), _lib.host()
+    run = lambda: ops.grouped_gemm(off, x, w.permute(0, 2, 1), total_rows=rows)
+    cut, ran = run(), kernels_run(run)
+    assert "split_reduce" in ran[-1]
+    _lib._host = host if native else _lib._Declines()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    try:
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (40 << 20)) / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+        out = run()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        _lib._host = host
+    assert_bf16_close(out, cut.float(), rtol=1.6e-2, atol=4e-3, what="uncut")
+    assert not torch.equal(out, cut)            # (the grouping of fp32 sums)
+
+
 @pytest.mark.parametrize("E,rows,K,N,dtype,cut", [
     (6, 766, 3592, 640, "bf16", True), (6, 766, 3584, 640, "bf16", False), (6, 766, 3968, 640, "fp8", False),       # one tile per CU: by K
     (8, 2000, 3072, 448, "bf16", True), (8, 2000, 3072, 384, "bf16", False), (8, 2000, 4096, 512, "bf16", True),    # 273 and 234 tiles
