@@ -13,8 +13,9 @@ using namespace fmoe;
 //   8 experts, 512 x 256, 1024 rows each 25.7 / 19.2, one hot expert 124 / 115; 1024 x 512, 512 each 18.8 / 13.5; 4096 x 1024, 256 each (two
 //   rounds of the ring) 30.0 / 33.7
 // fp32 against the transposed copies, their index launches and the three-part GEMM, us of a layer's whole training step: 847 tokens, 5 experts,
-// top-2, 576 x 792 893 / 465; 2000 tokens, 8 experts, 512 x 1024 900 / 505; 2048, 1024 x 2048 1225 / 1185; 600 tokens, 5 experts, 2048 x 4096
-// 1374 / 1325; 1000 tokens, 8 experts, top-4, 2048 x 2048 (1.7e10 products a matrix) 1984 / 2003; 4096 tokens, 4 experts, top-3, 1024 x 4096 5188 / 5358.
+// top-2, 576 x 792 882 / 592; 2000 tokens, 8 experts, 512 x 1024 856 / 568; 2048, 1024 x 2048 1372 / 1359; 600 tokens, 5 experts, 2048 x 4096
+// 1566 / 1418; not taken: 1000 tokens, 8 experts, top-4, 2048 x 2048 (1.7e10 products a matrix) 2378 / 2274; 4096 tokens, 4 experts, top-3, 1024 x
+// 4096 (5.2e10) 5819 / 5851.
 extern "C" int fmoe_weight_grad_pays(int dtype, int num_experts, int m, int n, int64_t rows) {
     if (num_experts < 1 || m < 1 || n < 1 || rows < 1) return 0;
     if (rows <= 64 * (int64_t)num_experts) return 1;

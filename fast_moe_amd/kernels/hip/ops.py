@@ -365,7 +365,7 @@ def grouped_gemm(offsets: torch.Tensor, a: torch.Tensor, b: torch.Tensor, *, tot
     [total_rows, N] in bf16 (fp32 for fp32 operands).  ``aux`` = two tensors like the output
     that receive the SWIGLU pre-activations.  ``gate`` (bf16 [total_rows, N], with
     ``epilogue=EPI_GATED``): the result is ``silu(gate) * (A B + bias)``.  ``plan_only``: launch nothing and return the
-    _lib.PLAN_* code of the kernel this call would run (fmoe_grouped_gemm_plan).  ``scales_pow2``
+    _lib.PLAN_* code of the class of kernel this call would run (fmoe_grouped_gemm_plan).  ``scales_pow2``
     (e4m3): a promise that every scale is an exact power of two, as ``quant_rows_fp8`` writes them;
     the ring kernel then folds them into its MFMAs (fmoe_gemm_desc.scale_pow2)."""
     if not (a_silu or a_expert_stride or plan_only) and k_window is None and out is None and aux is None and gate is None:
@@ -560,7 +560,7 @@ def grouped_gemm_sum2(offsets: torch.Tensor, a: torch.Tensor, b: torch.Tensor, a
 
 
 def gemm_plan(d: GemmDesc) -> int:
-    """The kernel fmoe_grouped_gemm would run for this descriptor (one of _lib.PLAN_*)."""
+    """The class of kernel fmoe_grouped_gemm would run for this descriptor (one of _lib.PLAN_*)."""
     plan = ctypes.c_int(0)
     _lib.check(_lib.load().fmoe_grouped_gemm_plan(ctypes.byref(d), ctypes.byref(plan)), "fmoe_grouped_gemm_plan")
     return plan.value

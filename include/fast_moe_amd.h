@@ -303,15 +303,16 @@ typedef struct fmoe_gemm_desc {
 
 int fmoe_grouped_gemm(const fmoe_gemm_desc* desc /* host pointer */, fmoe_stream_t stream);
 
-/* Which kernel fmoe_grouped_gemm would run for this descriptor on the current device
- * (no launch).  The Triton reference leaves this choice to its autotuner
+/* Which class of kernel fmoe_grouped_gemm would run for this descriptor on the current device, by its
+ * operands and its rows per expert (no launch).  Within RING, STAGED and STAGED_SHORT a call of few tiles runs a
+ * kernel of 64 x 64 tiles whose waves share K, and fmoe_grouped_gemm_ws may cut a last round along K.  The Triton reference leaves this choice to its autotuner
  * (kernels/triton/triton_moe.py:146-183); here it is a pure function of the descriptor, so
  * a caller can see beforehand whether its weight layout is read in place by a streaming
  * kernel or only by the element-load kernel, and tests can name the path they cover. */
 enum fmoe_gemm_plan {
     FMOE_PLAN_NONE = -1,          /* nothing to do (no rows)                                */
     FMOE_PLAN_RING = 0,           /* persistent LDS-ring kernel, 256 x 256 tiles            */
-    FMOE_PLAN_STAGED = 1,         /* register-staged kernel, 256 x 256 tiles (fp32: 64 rows) */
+    FMOE_PLAN_STAGED = 1,         /* register-staged kernel, 256 x 256 tiles (fp32: its own tiles) */
     FMOE_PLAN_STAGED_SHORT = 2,   /* 64-row tiles (few rows per expert): the streaming kernel or the
                                      ring on short tiles, or the register-staged one where neither
                                      applies                                                */
