@@ -113,10 +113,19 @@ __global__ __launch_bounds__(kGateWaves* kWave) void gate_softmax_kernel(const u
 
 using namespace fmoe;
 
-// Batches whose pass is bound by the host or by its chain of launches; a larger one has the library GEMM's rate to lose.
+static int gate_fragments(int E) { return E <= 16 ? 1 : E <= 32 ? 2 : E <= 64 ? 4 : 6; }
+
+// Batches whose pass is bound by the host (a library GEMM and a softmax take 26 us to issue, this 7) or by its chain of launches; a larger one has
+// the library GEMM's rate to lose.  A block's eight waves walk all of K, 3 us and 0.25 for every KB of a gate row times 1 + 2 * fragments, where the
+// library's two launches take 7 to 12: us on the GPU, library / kernel, 64 tokens: bf16 128 inputs, 8 experts 7.0 / 3.8; 1024, 64 8.8 / 7.9; 2048, 96
+// 8.9 / 16.6; 4096, 64 10.4 / 20.9; 8192, 96 11.6 / 52; fp32 1024, 64 7.9 / 12.6; 2048, 64  - / 20; 8192, 96 18.6 / 101.  The line is where that is as
+// much as what issuing them costs a pass.  us of a layer's pass (top-2) among others and alone, library / kernel: bf16, 2048 inputs, 96 experts, 1 token 63 / 42 and
+// 85 / 61, 16 tokens 58 / 59 and 94 / 78, 128 tokens 128 / 130 and 164 / 147; beyond it 4096, 64, 1 token 62 / 50 and 90 / 69, 16 tokens 66 / 71 and 102 / 90;
+// fp32 4096, 64, 16 tokens 118 / 147 and 153 / 164.
 extern "C" int fmoe_gate_softmax_pays(int dtype, int64_t T, int D, int E) {
-    return (dtype == FMOE_BF16 || dtype == FMOE_F32) && T >= 1 && T <= 128 && E >= 1 && E <= kGateMostExperts && D >= 1 && D <= 8192 &&
-           D % (dtype == FMOE_F32 ? 4 : 8) == 0;
+    if ((dtype != FMOE_BF16 && dtype != FMOE_F32) || T < 1 || T > 128 || E < 1 || E > kGateMostExperts || D < 1) return 0;
+    const int chunk = dtype == FMOE_F32 ? 4 : 8;
+    return D % chunk == 0 && (int64_t)D * (16 / chunk) * (1 + 2 * gate_fragments(E)) <= 56 * 1024;
 }
 
 extern "C" int fmoe_gate_softmax(const void* x, int dtype, int64_t T, int D, int64_t x_stride_row, const void* weight, const void* bias, int E,
@@ -136,9 +145,11 @@ extern "C" int fmoe_gate_softmax(const void* x, int dtype, int64_t T, int D, int
         return check_launch("fmoe_gate_softmax");
     };
 #define FMOE_GATE(NF) (dtype == FMOE_F32 ? go(gate_softmax_kernel<true, NF>, NF) : go(gate_softmax_kernel<false, NF>, NF))
-    if (E <= 16) return FMOE_GATE(1);
-    if (E <= 32) return FMOE_GATE(2);
-    if (E <= 64) return FMOE_GATE(4);
-    return FMOE_GATE(6);
+    switch (gate_fragments(E)) {
+        case 1: return FMOE_GATE(1);
+        case 2: return FMOE_GATE(2);
+        case 4: return FMOE_GATE(4);
+        default: return FMOE_GATE(6);
+    }
 #undef FMOE_GATE
 }

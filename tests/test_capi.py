@@ -353,3 +353,14 @@ def test_column_quantiser_scratch_rule(lib, E, K, N, two_launches):
     two launches can read the operand (rows in eights, columns in fours)."""
     need = lib.fmoe_quant_rows_workspace_bytes(1, E, N, K, K * N, 1, N, 0)       # (1: FMOE_BF16)
     assert (need > 0) == two_launches
+
+
+@pytest.mark.parametrize("dtype,T,D,E,pays", [
+    (1, 128, 128, 8, True), (1, 129, 128, 8, False), (1, 0, 128, 8, False), (1, 1, 132, 8, False), (0, 1, 132, 8, True), (0, 1, 130, 8, False),
+    (1, 64, 9552, 16, True), (1, 64, 9560, 16, False), (1, 64, 5728, 32, True), (1, 64, 5736, 32, False), (1, 64, 3184, 64, True),
+    (1, 64, 3192, 64, False), (1, 64, 2200, 96, True), (1, 64, 2208, 96, False), (1, 64, 8, 97, False),
+    (0, 64, 4776, 16, True), (0, 64, 4780, 16, False), (0, 64, 2864, 32, True), (0, 64, 2864, 33, False), (2, 64, 128, 8, False),
+])
+def test_gate_of_a_small_batch_rule(lib, dtype, T, D, E, pays):
+    """Tokens, whole 16-byte chunks, and the length of a row by the experts (dtype: 0 fp32, 1 bf16)."""
+    assert bool(lib.fmoe_gate_softmax_pays(dtype, T, D, E)) == pays

@@ -265,13 +265,17 @@ def test_forward_replays_from_a_hip_graph(fp8):
 def test_gate_of_a_small_batch(T, D, E, dtype):
     """One launch for Linear + softmax: logits within the rounding of an fp32 sum (2^-24 for every product) of float64's, the softmax of the
     rounded logits as torch gives it; rows of a wider tensor; up to E = 96."""
-    from fast_moe_amd.kernels.hip import ops
+    from fast_moe_amd.kernels.hip import _lib, ops
     g = torch.Generator(device="cuda").manual_seed(T + D + E)
     x = torch.full((T, D + 8), float("nan"), dtype=dtype, device="cuda")[:, :D]
     x.copy_(torch.randn(T, D, generator=g, device="cuda"))
     w = (torch.randn(E, D, generator=g, device="cuda") * D ** -0.5).to(dtype)
     for bias in (torch.randn(E, generator=g, device="cuda").to(dtype), None):
-        got = ops.gate_softmax(x, w, bias)
+        got = _lib.host().gate_softmax(x, w, bias, ops._stream(x))
+        if _lib.load().fmoe_gate_softmax_pays(int(dtype == torch.bfloat16), T, D, E):
+            assert torch.equal(ops.gate_softmax(x, w, bias), got)
+        else:
+            assert ops.gate_softmax(x, w, bias) is None
         exact = x.double() @ w.double().t() + (0 if bias is None else bias.double())
         err = (D + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + (0 if bias is None else bias.double().abs()))
         if dtype == torch.bfloat16:
