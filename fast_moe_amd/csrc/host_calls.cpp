@@ -19,6 +19,7 @@
 #include <torch/version.h>
 
 #include <cstdint>
+#include <cstring>
 
 #include "../../include/fast_moe_amd.h"
 
@@ -753,11 +754,9 @@ PyObject* py_weight_grad(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // init(addresses of the C entry points, in the order of the pointers above)
 PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    void** const entry[] = {(void**)&route_workspace_bytes, (void**)&c_route_topk, (void**)&c_grouped_gemm, (void**)&c_combine,
-                            (void**)&c_quant_rows, (void**)&c_gate_softmax, (void**)&gemm_workspace_bytes, (void**)&c_grouped_gemm_ws,
-                            (void**)&c_gemm_plan, (void**)&c_combine_bwd, (void**)&c_segment_colsum, (void**)&c_swiglu_bwd,
-                            (void**)&c_silu_mul, (void**)&c_gather_rows, (void**)&c_invert_index, (void**)&c_gate_l1_bwd,
-                            (void**)&c_weight_grad, (void**)&weight_grad_pays, (void**)&last_error};
+    void* const entry[] = {&route_workspace_bytes, &c_route_topk, &c_grouped_gemm, &c_combine, &c_quant_rows, &c_gate_softmax, &gemm_workspace_bytes,
+                           &c_grouped_gemm_ws, &c_gemm_plan, &c_combine_bwd, &c_segment_colsum, &c_swiglu_bwd, &c_silu_mul, &c_gather_rows,
+                           &c_invert_index, &c_gate_l1_bwd, &c_weight_grad, &weight_grad_pays, &last_error};
     constexpr Py_ssize_t count = sizeof(entry) / sizeof(entry[0]);
     if (n != count) {
         PyErr_Format(PyExc_TypeError, "init: %d addresses expected", (int)count);
@@ -769,7 +768,8 @@ PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
             PyErr_SetString(PyExc_TypeError, "init: addresses are integers");
             return nullptr;
         }
-    for (int i = 0; i < count; ++i) *entry[i] = (void*)v[i];
+    static_assert(sizeof(c_combine) == sizeof(v[0]), "addresses of functions are 64 bits");
+    for (int i = 0; i < count; ++i) std::memcpy(entry[i], &v[i], sizeof(v[i]));     // (each has a type of its own)
     return none();
 }
 
