@@ -33,6 +33,7 @@ decltype(&fmoe_grouped_gemm_ws) c_grouped_gemm_ws;
 decltype(&fmoe_combine) c_combine;
 decltype(&fmoe_quant_rows_e4m3) c_quant_rows;
 decltype(&fmoe_gate_softmax) c_gate_softmax;
+decltype(&fmoe_gate_softmax_pays) gate_softmax_pays;
 decltype(&fmoe_grouped_gemm_plan) c_gemm_plan;
 decltype(&fmoe_combine_bwd) c_combine_bwd;
 decltype(&fmoe_segment_colsum) c_segment_colsum;
@@ -398,7 +399,7 @@ PyObject* py_quant_rows(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// (x [T, D], weight [E, D], bias [E] or None, stream) -> softmax(x weight^T + bias) [T, E]
+// (x [T, D], weight [E, D], bias [E] or None, stream) -> softmax(x weight^T + bias) [T, E], where fmoe_gate_softmax is the faster form
 PyObject* py_gate_softmax(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (n != 4) return none();
@@ -415,8 +416,12 @@ PyObject* py_gate_softmax(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 w.size(0) > INT32_MAX || w.size(1) > INT32_MAX)
                 return false;
             if (bias.defined() && (bias.scalar_type() != x.scalar_type() || !bias.is_contiguous() || bias.numel() != w.size(0))) return false;
+            if (!gate_softmax_pays(code, x.size(0), (int)x.size(1), (int)w.size(0)) || x.stride(0) < x.size(1) ||
+                x.stride(0) % (code == FMOE_F32 ? 4 : 8))
+                return false;
             x_data = x.data_ptr();
             w_data = w.data_ptr();
+            if ((uintptr_t)x_data % 16 || (uintptr_t)w_data % 16) return false;
             if (bias.defined()) b_data = bias.data_ptr();
             return true;
         },
@@ -756,7 +761,7 @@ PyObject* py_weight_grad(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void* const entry[] = {&route_workspace_bytes, &c_route_topk, &c_grouped_gemm, &c_combine, &c_quant_rows, &c_gate_softmax, &gemm_workspace_bytes,
                            &c_grouped_gemm_ws, &c_gemm_plan, &c_combine_bwd, &c_segment_colsum, &c_swiglu_bwd, &c_silu_mul, &c_gather_rows,
-                           &c_invert_index, &c_gate_l1_bwd, &c_weight_grad, &weight_grad_pays, &last_error};
+                           &c_invert_index, &c_gate_l1_bwd, &c_weight_grad, &weight_grad_pays, &gate_softmax_pays, &last_error};
     constexpr Py_ssize_t count = sizeof(entry) / sizeof(entry[0]);
     if (n != count) {
         PyErr_Format(PyExc_TypeError, "init: %d addresses expected", (int)count);

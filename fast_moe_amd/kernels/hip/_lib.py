@@ -146,7 +146,7 @@ HOST_ENTRY_POINTS = ("fmoe_route_workspace_bytes", "fmoe_route_topk", "fmoe_grou
                      "fmoe_quant_rows_e4m3", "fmoe_gate_softmax", "fmoe_grouped_gemm_workspace_bytes", "fmoe_grouped_gemm_ws",
                      "fmoe_grouped_gemm_plan", "fmoe_combine_bwd", "fmoe_segment_colsum", "fmoe_swiglu_bwd", "fmoe_silu_mul",
                      "fmoe_gather_rows", "fmoe_invert_index", "fmoe_gate_l1_bwd", "fmoe_weight_grad", "fmoe_weight_grad_pays",
-                     "fmoe_last_error")
+                     "fmoe_gate_softmax_pays", "fmoe_last_error")
 _host = None
 
 

@@ -130,6 +130,9 @@ def route_topk(scores: torch.Tensor, k: int, renorm=True, static_scratch: bool =
 def gate_softmax(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """``softmax(F.linear(x, weight, bias), dim=1)`` of a small batch [T, D] in one launch (fmoe_gate_softmax), or None where
     that is not the faster form or does not take the operands."""
+    scores = _lib.host().gate_softmax(x, weight, bias, _stream(x))
+    if scores is not None:
+        return scores
     T, D = x.shape
     if weight.dtype != x.dtype or x.dtype not in _DTYPE_CODE or not x.is_cuda:
         return None
@@ -141,9 +144,6 @@ def gate_softmax(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
             or not weight.is_contiguous()
             or (bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous() or bias.numel() != weight.shape[0]))):
         return None
-    scores = _lib.host().gate_softmax(x, weight, bias, _stream(x))
-    if scores is not None:
-        return scores
     _need_cuda("gate_softmax", x, weight, bias)
     scores = torch.empty((T, weight.shape[0]), dtype=x.dtype, device=x.device)
     rc = lib.fmoe_gate_softmax(x.data_ptr(), code, T, D, x.stride(0), weight.data_ptr(), _ptr(bias), weight.shape[0],

@@ -107,15 +107,17 @@ class FastMoELayer(nn.Module):
     def _scores(self, x: torch.Tensor) -> torch.Tensor:
         """The gate's probabilities [tokens, E]: from one launch where the batch is small, nothing needs a gradient and the gate is the
         class's own; a caller's module, hooks, modes and autocast are asked through the modules, and so are other shapes, which they refuse."""
-        gate = self.gate
-        if type(x) is torch.Tensor and x.ndim == 3 and x.shape[2] == self.input_dim and x.numel() <= _SMALL_BATCH * self.input_dim \
-                and type(gate) is GatingNetwork and type(gate.gate) is nn.Linear and GatingNetwork.forward is _GATE_FORWARD \
-                and not _watched(gate) and not _watched(gate.gate) and not torch.is_autocast_enabled() and not _mode_active():
-            weight, bias = gate.gate.weight, gate.gate.bias
-            if not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)):
-                scores = ops.gate_softmax(x.reshape(-1, self.input_dim), weight, bias)
-                if scores is not None:
-                    return scores
+        gate, shape = self.gate, x.shape
+        if type(x) is torch.Tensor and len(shape) == 3 and shape[2] == self.input_dim and shape[0] * shape[1] <= _SMALL_BATCH \
+                and type(gate) is GatingNetwork and GatingNetwork.forward is _GATE_FORWARD and not torch.is_autocast_enabled() \
+                and not _mode_active():
+            linear = gate.gate
+            if type(linear) is nn.Linear and not _watched(gate) and not _watched(linear):
+                weight, bias = linear.weight, linear.bias
+                if not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)):
+                    scores = ops.gate_softmax(x.reshape(-1, self.input_dim), weight, bias)
+                    if scores is not None:
+                        return scores
         return gate(x).reshape(-1, self.num_experts)
 
     def forward(self, x: torch.Tensor, num_experts_per_tok: int) -> torch.Tensor:
@@ -160,8 +162,10 @@ _SMALL_BATCH = 128              # (the library's own rule, fmoe_gate_softmax_pay
 def _mode_active() -> bool:
     """Whether a dispatch or function mode would see the gate's operators (torch.set_default_device is one that has no use for them)."""
     c = torch._C
-    return bool(c._len_torch_dispatch_stack()) or any(type(c._get_function_stack_at(i)) is not DeviceContext
-                                                      for i in range(c._len_torch_function_stack()))
+    if c._len_torch_dispatch_stack():
+        return True
+    count = c._len_torch_function_stack()
+    return count > 0 and any(type(c._get_function_stack_at(i)) is not DeviceContext for i in range(count))
 
 
 def _watched(module: nn.Module) -> bool:

@@ -271,11 +271,12 @@ def test_gate_of_a_small_batch(T, D, E, dtype):
     x.copy_(torch.randn(T, D, generator=g, device="cuda"))
     w = (torch.randn(E, D, generator=g, device="cuda") * D ** -0.5).to(dtype)
     for bias in (torch.randn(E, generator=g, device="cuda").to(dtype), None):
-        got = _lib.host().gate_softmax(x, w, bias, ops._stream(x))
-        if _lib.load().fmoe_gate_softmax_pays(int(dtype == torch.bfloat16), T, D, E):
-            assert torch.equal(ops.gate_softmax(x, w, bias), got)
-        else:
-            assert ops.gate_softmax(x, w, bias) is None
+        got, code = torch.empty(T, E, dtype=dtype, device="cuda"), int(dtype == torch.bfloat16)
+        assert _lib.load().fmoe_gate_softmax(x.data_ptr(), code, T, D, x.stride(0), w.data_ptr(), ops._ptr(bias), E, got.data_ptr(),
+                                             ops._stream(x)) == 0
+        for call in (ops.gate_softmax, lambda *a: _lib.host().gate_softmax(*a, ops._stream(x))):
+            res = call(x, w, bias)
+            assert torch.equal(res, got) if _lib.load().fmoe_gate_softmax_pays(code, T, D, E) else res is None
         exact = x.double() @ w.double().t() + (0 if bias is None else bias.double())
         err = (D + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + (0 if bias is None else bias.double().abs()))
         if dtype == torch.bfloat16:
