@@ -157,9 +157,16 @@ __device__ __forceinline__ u32x4 silu_f32x4(u32x4 v) {
     return v;
 }
 
-// LDS byte offset of a 16-byte chunk of a 64-byte row: the ds_read_b128 of an MFMA fragment is conflict free
+// LDS byte offset of a 16-byte chunk of a 64-byte row.  A ds_read_b128 is served 256 bytes at a time, to the lanes 0-3, 12-15 and
+// 20-27, to 4-11, 16-19 and 28-31, and so on for the upper half.  Fragments of 16 rows and four chunks (lane / 16) meet in different banks
+// of each only if the chunks of rows 4 q .. 4 q + 3 trade places by 0, 3, 2, 1: 570 bytes per ns and CU, 294 by 0, 1, 2, 3; fragments of
+// 32 rows and two chunks do with either.
+__device__ __forceinline__ int lds_swizzle64(int row) {
+    const int q = (row >> 2) & 3;
+    return q ^ ((q & 1) << 1);
+}
 __device__ __forceinline__ int lds_off64(int row, int chunk) {
-    return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4);
+    return row * 64 + ((chunk ^ lds_swizzle64(row)) << 4);
 }
 
 // two transposing LDS reads: this lane's 8 k values of one column of 16 rows (one MFMA's depth), a pointing at the lane's place

@@ -376,7 +376,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     // ------------------------------------------------------------ LDS-DMA geometry
     // DMA instruction i of this wave fills LDS rows (i*NW + wave)*16 .. +15 of the X (or W)
     // part of a ring slot: lane l -> row + l/4, 16-byte position l%4, which holds global
-    // chunk (l%4) ^ ((row >> 2) & 3) of that row's 64-byte K-slice (the read-side swizzle).
+    // chunk (l%4) ^ lds_swizzle64(row) of that row's 64-byte K-slice (the read-side swizzle).
     // These are needed twice per tile and cost a few VALU instructions: they are recomputed from
     // a copy of the lane number the compiler cannot see through rather than kept in registers
     // across the main loop, where the accumulators and fragments leave none to spare.
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     auto dma_swizzle = [&](int i) -> int {      // byte position inside the row's 64-byte slice
         int l = lane;
         asm volatile("" : "+v"(l));
-        return (((l & 3) ^ ((((i * NW + wave) * 16 + (l >> 2)) >> 2) & 3)) << 4);
+        return (((l & 3) ^ lds_swizzle64((i * NW + wave) * 16 + (l >> 2))) << 4);
     };
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
 
@@ -515,23 +515,36 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         }
     };
 
-    int wfrag_row[FN], xfrag_row[FM];
-#pragma unroll
-    for (int fn = 0; fn < FN; ++fn) {
-        int r;
-        if (SWIGLU) r = (fn < FN / 2 ? 0 : BN / 2) + wn * (TN / 2) + (fn % (FN / 2)) * 32;
-        else r = wn * TN + fn * 32;
-        wfrag_row[fn] = r + (lane & 31);
-    }
-#pragma unroll
-    for (int fm = 0; fm < FM; ++fm) xfrag_row[fm] = wm * TM + fm * 32 + (lane & 31);
+    // e4m3: byte offsets, in a slot's weight and activation part, of the two 16-byte chunks that this lane reads of a fragment of 32 rows
+    // (fragments lie whole 32-row blocks apart: constants)
+    const int wq_lo = lds_off64((SWIGLU ? wn * (TN / 2) : wn * TN) + (lane & 31), 2 * khalf);
+    const int wq_hi = lds_off64((SWIGLU ? wn * (TN / 2) : wn * TN) + (lane & 31), 2 * khalf + 1);
+    const int xq_lo = lds_off64(wm * TM + (lane & 31), 2 * khalf), xq_hi = lds_off64(wm * TM + (lane & 31), 2 * khalf + 1);
+    auto wq_block = [](int fn) { return SWIGLU ? fn / (FN / 2) * (BN / 2) * 64 + fn % (FN / 2) * 2048 : fn * 2048; };
+    auto load_q = [](const uint8_t* base, int lo_at, int hi_at) -> i32x8 {
+        const u32x4 lo = *reinterpret_cast<const u32x4*>(base + lo_at), hi = *reinterpret_cast<const u32x4*>(base + hi_at);
+        return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+    };
+    // bf16 with k contiguous: 16 x 16 x 32 MFMAs.  Under the chip's power cap a chain of them sustains 2050 TFLOP/s where one of 32 x 32 x 16 sustains
+    // 1805 (half the accumulator traffic for a product).  A wave's 32 x 32 block of the output is four of them, two column blocks
+    // a and two row blocks b.  Lane group g = lane / 16 of block a holds the four columns 16 a + 8 (g % 2) + 4 (g / 2) .. + 3 (the
+    // order in which the weight rows are read below), so that exchanging lane groups between the row blocks (v_permlane16_swap,
+    // behind the main loop) leaves the sums as v_mfma_f32_32x32x16_bf16 would: one layout for the epilogue.
+    constexpr bool B16 = !FP8 && !WTR && !XTR;
+    constexpr int FN16 = 2 * FN, HX = FM;
+    const int kquarter = lane >> 4;
+    const int wfrag_lane16 = 8 * ((lane >> 2) & 1) + 4 * ((lane >> 3) & 1) + (lane & 3);      // weight row of this lane in a block of 16
+    // byte offsets, in a slot, of this lane's 16-byte chunk of weight fragment f (in the weight part) and activation fragment 0 (+ 1024 each)
+    const int wfrag_lane = lds_off64((SWIGLU ? wn * (TN / 2) : wn * TN) + wfrag_lane16, kquarter);
+    auto wfrag_off = [&](int f) { return wfrag_lane + (SWIGLU ? f / FN * (BN / 2) * 64 + f % FN * 1024 : f * 1024); };
+    const int xfrag_lane = lds_off64(wm * TM + (lane & 15), kquarter);
     // WTR: byte offset, inside the weight part of a slot, of this lane's first transposing read
     // of fragment fn (rows 8*khalf + l16/4 of the slice's first 16; +1024: the next 4 rows)
     int wtr_off[FN];
 #pragma unroll
     for (int fn = 0; fn < FN; ++fn) {
         const int l16 = lane & 15;
-        const int frag0 = wfrag_row[fn] - (lane & 31);                       // first tile column of the fragment
+        const int frag0 = SWIGLU ? fn / (FN / 2) * (BN / 2) + wn * (TN / 2) + fn % (FN / 2) * 32 : wn * TN + fn * 32;   // first tile column of the fragment
         const int ncol = frag0 % (BN / 2) + 16 * ((lane >> 4) & 1) + 4 * (l16 & 3);
         const int row = 8 * khalf + (l16 >> 2);
         wtr_off[fn] = (frag0 / (BN / 2)) * 8192 + row * 256 + (((ncol >> 3) ^ (4 * (l16 >> 2))) << 4) + (ncol & 7) * 2;
@@ -697,16 +710,25 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
     int landed = -1;                        // 4-slot ring: items <= landed are complete for this wave
     int c = 0;                              // 4-slot ring: item being computed
     int cslot = 0;                          // ring slot of the item being computed
-    bf16x8 wfa[FN], xfa[FM], wfb[FN], xfb[FM];   // fragment double buffer of the pipelined loop
-    i32x8 qwa[FN], qwb[FN], qx0[FM / 2], qx1[FM / 2];   // the same for e4m3 fragments
+    bf16x8 wf[FN16], xh0[HX], xh1[HX];      // fragments of the pipelined loop: weights, the two halves of the activations
+    bf16x8 wfa[FN], xfa[FM], wfb[FN], xfb[FM];   // transposing reads: double buffer of half slices
+    i32x8 qwa[FN], qwb[FN], qx0[FM / 2], qx1[FM / 2];   // the same for e4m3 fragments, the weights twice
     for (int tile_i = 0; tile_i < my_tiles; ++tile_i) {
         f32x16 acc[FN][FM];
+        f32x4 acc16[FN16][2 * HX];              // B16: sums of 16 x 16 blocks
+        if constexpr (!B16) {
 #pragma unroll
-        for (int i = 0; i < FN; ++i)
+            for (int i = 0; i < FN; ++i)
 #pragma unroll
-            for (int j = 0; j < FM; ++j)
+                for (int j = 0; j < FM; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+                    for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+        } else {
+#pragma unroll
+            for (int i = 0; i < FN16; ++i)
+#pragma unroll
+                for (int j = 0; j < 2 * HX; ++j) acc16[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
 #ifdef FMOE_TRACE
         uint64_t tstamp[18] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         FMOE_TRACE_STAMP(0);
@@ -717,37 +739,22 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             const uint8_t* sx = smem + cslot * TL::STAGE_BYTES;
             const uint8_t* sw = sx + BM * 64;
             if (!FP8) {
+                bf16x8 w4[FN16], x4[2 * HX];
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const int chunk = 2 * s + khalf;
-                    bf16x8 wf[FN], xf[FM];
+                for (int f = 0; f < FN16; ++f) w4[f] = *reinterpret_cast<const bf16x8*>(sw + wfrag_off(f));
 #pragma unroll
-                    for (int fn = 0; fn < FN; ++fn)
-                        wf[fn] = *reinterpret_cast<const bf16x8*>(sw + lds_off64(wfrag_row[fn], chunk));
+                for (int f = 0; f < 2 * HX; ++f) x4[f] = *reinterpret_cast<const bf16x8*>(sx + xfrag_lane + f * 1024);
 #pragma unroll
-                    for (int fm = 0; fm < FM; ++fm)
-                        xf[fm] = *reinterpret_cast<const bf16x8*>(sx + lds_off64(xfrag_row[fm], chunk));
+                for (int fn = 0; fn < FN16; ++fn)
 #pragma unroll
-                    for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-                        for (int fm = 0; fm < FM; ++fm)
-                            acc[fn][fm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[fn], xf[fm], acc[fn][fm], 0, 0, 0);
-                }
+                    for (int fm = 0; fm < 2 * HX; ++fm)
+                        acc16[fn][fm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w4[fn], x4[fm], acc16[fn][fm], 0, 0, 0);
             } else {
-                const int chunk = 2 * khalf;
                 i32x8 wf[FN], xf[FM];
 #pragma unroll
-                for (int fn = 0; fn < FN; ++fn) {
-                    const u32x4 lo = *reinterpret_cast<const u32x4*>(sw + lds_off64(wfrag_row[fn], chunk));
-                    const u32x4 hi = *reinterpret_cast<const u32x4*>(sw + lds_off64(wfrag_row[fn], chunk + 1));
-                    wf[fn] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-                }
+                for (int fn = 0; fn < FN; ++fn) wf[fn] = load_q(sw + wq_block(fn), wq_lo, wq_hi);
 #pragma unroll
-                for (int fm = 0; fm < FM; ++fm) {
-                    const u32x4 lo = *reinterpret_cast<const u32x4*>(sx + lds_off64(xfrag_row[fm], chunk));
-                    const u32x4 hi = *reinterpret_cast<const u32x4*>(sx + lds_off64(xfrag_row[fm], chunk + 1));
-                    xf[fm] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-                }
+                for (int fm = 0; fm < FM; ++fm) xf[fm] = load_q(sx + fm * 2048, xq_lo, xq_hi);
 #pragma unroll
                 for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
@@ -758,7 +765,198 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             cslot = cslot + 1 == STAGES ? 0 : cslot + 1;
         };
 
-        if constexpr (PAIR && !FP8) {
+        if constexpr (PAIR && B16) {
+            // Software pipeline over "blocks" (half a K-slice's MFMAs: all weight fragments against one half of the activation
+            // fragments): the other half's fragments are read while block 0 multiplies; under block 1 the next slice's first half
+            // and, each behind its last use, its weight fragments.  Two barriers per pair of items c, c+1 (a "double step"):
+            //   B  after the last read of item c      -> its slot and the one of c-1 are refilled
+            //   A' before the first read of item c+2  -> pair (c+2, c+3) has landed everywhere
+            // Raw s_barrier (no fence): LDS reads of slots that stay valid may be in flight
+            // across a barrier; the asm statements keep the compiler from moving LDS reads
+            // over them.  The steady state is straight-line code: the issue side always has
+            // something to fetch (past the end of the block's stream it re-reads the last
+            // tile's rows into slots nobody looks at), and everything that depends on the
+            // wave's half is a template parameter.
+            // KTAIL: what the pair before the last one has multiplied already, masked where it is used: behind a load the mask would wait
+            // for it.  item: the slice's number inside the tile.  (A fragment is one 16-byte chunk: masked whole or not at all.)
+            auto masked = [&](bf16x8 f, int item) -> bf16x8 {
+                const int at = (item - (KT - 2)) * BK + 8 * kquarter;
+                const uint32_t m1 = at >= 0 && at < tail_dup ? 0u : 0xffffffffu;
+                return __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, f) & u32x4{m1, m1, m1, m1});
+            };
+            auto load_w = [&](int slot_i, int f) -> bf16x8 {
+                return *reinterpret_cast<const bf16x8*>(smem + slot_i * TL::STAGE_BYTES + BM * 64 + wfrag_off(f));
+            };
+            auto load_x = [&](bf16x8 (&xh)[HX], int half, int slot_i) {
+                const uint8_t* sx = smem + slot_i * TL::STAGE_BYTES + half * HX * 1024;
+#pragma unroll
+                for (int i = 0; i < HX; ++i) xh[i] = *reinterpret_cast<const bf16x8*>(sx + xfrag_lane + i * 1024);
+            };
+            // The MFMAs of a block, with the L parts of the pair being issued between them
+            // when DMA is set.  The two waves of a SIMD (w and w + NW/2) issue in different
+            // blocks, so that while one sits in its VMEM issue the other feeds the MFMA pipe.
+            // roll: the weight fragments of the item in slot `slot_i` take the places of this one's, each behind its last use.
+            // mask: the item is masked as number `item`.
+            // skip: the block's row blocks hold no valid row (sparse tile); its share of the DMA issue and the reads are left.
+            auto mma_block = [&](bf16x8 (&xh)[HX], auto half_c, auto dma_c, auto roll_c, auto skip_c, int slot_i, int item, auto mask_c) {
+                constexpr int M0 = decltype(half_c)::value * HX;
+                if constexpr (decltype(mask_c)::value && !decltype(skip_c)::value) {
+#pragma unroll
+                    for (int fm = 0; fm < HX; ++fm) xh[fm] = masked(xh[fm], item);
+#pragma unroll
+                    for (int fn = 0; fn < FN16; ++fn)
+                        if (M0 == 0) wf[fn] = masked(wf[fn], item);
+                }
+                constexpr bool DMA = decltype(dma_c)::value, ROLL = decltype(roll_c)::value;
+                constexpr int NM = FN16 * HX;
+                // part q of the pair goes out behind MFMA ceil((q + 1) * NM / L) - 1: evenly spread
+                // whether the parts are as many as the MFMAs, a divisor or a multiple of them, or neither
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    const int fn = m / HX, fm = m % HX;
+                    if constexpr (!decltype(skip_c)::value)
+                        acc16[fn][M0 + fm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[fn], xh[fm], acc16[fn][M0 + fm], 0, 0, 0);
+                    if constexpr (DMA) {
+                        constexpr auto slot_of = [](int q) { return ((q + 1) * NM + L - 1) / L - 1; };
+                        bool any = false;
+#pragma unroll
+                        for (int q = 0; q < L; ++q) any |= slot_of(q) == m;
+                        if (any) {
+                            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                            for (int q = 0; q < L; ++q)
+                                if (slot_of(q) == m) issue_part(q);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+                    if constexpr (ROLL) {
+                        if (fm == HX - 1) wf[fn] = load_w(slot_i, fn);
+                    }
+                }
+            };
+            // one fragment read in the shadow of every MFMA: the activation fragments first, then the rolling weights
+            auto interleave = [&](auto x_c, auto roll_c) {
+                constexpr int NX = decltype(x_c)::value ? HX : 0;
+                constexpr bool ROLL = decltype(roll_c)::value;
+#pragma unroll
+                for (int i = 0; i < FN16; ++i) {
+#pragma unroll
+                    for (int j = 0; j < HX; ++j) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        if (i * HX + j < NX) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    }
+                    if (ROLL) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+            };
+            auto barrier = [&]() {
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            };
+            // sched_barrier(0) pins the order "reads of the next block, then the MFMAs of this
+            // one"; left alone the scheduler sinks the reads to just before their first use.
+            int kitem = KSPLIT ? cur.k0 : 0;        // number, inside the tile, of the item in slot cslot
+            // skip_wait (wave-uniform): the pair this step would wait for is known to have landed.  That
+            // holds for the first step of every tile but the block's first: the pair was issued before
+            // the previous epilogue, whose stores are all issued whatever their lanes' predicates
+            // (store16_uniform_base) and followed by a wait that leaves at most that many operations
+            // in flight, i.e. nothing older than the stores.  The counted wait here would sit out the
+            // stores' own round trip instead (one counter serves loads and stores, in order).
+            auto double_step = [&](auto half_c, auto mask_c, auto sparse_c, bool skip_wait) __attribute__((always_inline)) {
+                constexpr int HALF = decltype(half_c)::value;
+                constexpr bool SP = decltype(sparse_c)::value;   // row blocks of the second half are not multiplied
+                constexpr std::true_type yes{};
+                constexpr std::false_type no{};
+                constexpr std::integral_constant<int, 0> h0{};
+                constexpr std::integral_constant<int, 1> h1{};
+                constexpr std::integral_constant<bool, !SP> dense{};
+                const int s1 = cslot + 1 == STAGES ? 0 : cslot + 1;
+                const int s2 = s1 + 1 == STAGES ? 0 : s1 + 1;
+                if (!SP) load_x(xh1, 1, cslot);
+                mma_block(xh0, h0, no, no, no, 0, kitem, mask_c);
+                interleave(dense, no);
+                __builtin_amdgcn_sched_barrier(0);
+                load_x(xh0, 0, s1);
+                mma_block(xh1, h1, no, yes, sparse_c, s1, kitem, mask_c);
+                if (!SP) interleave(yes, yes);
+                __builtin_amdgcn_sched_barrier(0);
+                barrier();                  // B
+                part_a = lds_base + islot * TL::STAGE_BYTES;    // pair (c + 2 * AHEAD, + 1)
+                islot = islot + 1 == STAGES ? 0 : islot + 1;
+                part_b = lds_base + islot * TL::STAGE_BYTES;
+                islot = islot + 1 == STAGES ? 0 : islot + 1;
+                part_koff = (int64_t)ikt * xstep;
+                if constexpr (KTAIL) part_koff = ikt == KT - 2 ? tail_x : part_koff;
+                part_wkoff = part_koff;
+                ikt += 2;
+                if (!SP) load_x(xh1, 1, s1);
+                if constexpr (HALF == 0) __builtin_amdgcn_sched_barrier(0);
+                mma_block(xh0, h0, std::integral_constant<bool, HALF == 0>{}, no, no, 0, kitem + 1, mask_c);
+                if constexpr (HALF != 0) interleave(dense, no);
+                __builtin_amdgcn_sched_barrier(0);
+                // pair (c+2, c+3) is older than the other pairs in flight, 2L instructions each, the one the
+                // first half just issued among them
+                if (!skip_wait) {
+                    if (HALF == 0) wait_vmcnt<2 * L * (TL::AHEAD - 1)>();
+                    else wait_vmcnt<2 * L * (TL::AHEAD - 2)>();
+                }
+                barrier();                  // A'
+                load_x(xh0, 0, s2);
+                if constexpr (HALF == 1) __builtin_amdgcn_sched_barrier(0);
+                mma_block(xh1, h1, std::integral_constant<bool, HALF == 1>{}, yes, sparse_c, s2, kitem + 1, mask_c);
+                if constexpr (HALF != 1 && !SP) interleave(yes, yes);
+                __builtin_amdgcn_sched_barrier(0);
+                cslot = s2;
+                kitem += 2;
+            };
+            // The issue side runs 2 * AHEAD items ahead: it enters the next tile that many items before the end; the last two double
+            // steps hold the end of a KTAIL tile's columns and mask it.  All steps of a tile are one loop, the last one reads
+            // the next tile's first fragments for nothing: sums that leave the loop between peeled steps do not stay in their
+            // registers (the compiler gives the MFMAs of straight-line code other destinations, and spills).
+            auto tile_steps = [&](auto half_c, auto sparse_c) __attribute__((always_inline)) {
+                constexpr int MASKED = KTAIL ? 4 : 0;     // slices (two steps: a loop)
+                const int tile_kt = __builtin_amdgcn_readfirstlane(KWIN || KSPLIT ? cur.kt : KT);
+                int landed = tile_i > 0;        // the first step's pair landed before the previous epilogue's stores
+                auto steps = [&](int kt, int end, auto mask_c) __attribute__((always_inline)) {
+#pragma unroll 1
+                    for (; kt < end; kt += 2) {
+                        asm volatile("" : "+v"(landed));        // (no peeled first step)
+                        const bool skip_wait = __builtin_amdgcn_readfirstlane(landed) != 0;
+                        if (kt == tile_kt - 2 * TL::AHEAD) {
+                            FMOE_TRACE_STAMP(10);
+                            enter_next();
+                            ikt = KSPLIT ? nxt.k0 : 0;
+                        }
+                        double_step(half_c, mask_c, sparse_c, skip_wait);
+                        landed = 0;
+#ifdef FMOE_TRACE
+                        if (kt < 8) FMOE_TRACE_STAMP(6 + kt / 2);
+                        if (kt == tile_kt - 4) FMOE_TRACE_STAMP(11);
+#endif
+                    }
+                };
+                steps(0, tile_kt - MASKED, std::false_type{});
+                if constexpr (MASKED > 0) steps(tile_kt - MASKED, tile_kt, std::true_type{});
+            };
+            if (tile_i == 0) {              // pair 0 has landed everywhere
+                wait_vmcnt<2 * L * (TL::AHEAD - 1)>();
+                barrier();
+            }
+            load_x(xh0, 0, cslot);
+#pragma unroll
+            for (int f = 0; f < FN16; ++f) wf[f] = load_w(cslot, f);
+            const bool sparse = SPARSE && cur.rows_valid <= p.short_tile_rows;
+            if (wave < NW / 2) {
+                if (sparse) tile_steps(std::integral_constant<int, 0>{}, std::integral_constant<bool, SPARSE>{});
+                else tile_steps(std::integral_constant<int, 0>{}, std::false_type{});
+            } else {
+                if (sparse) tile_steps(std::integral_constant<int, 1>{}, std::integral_constant<bool, SPARSE>{});
+                else tile_steps(std::integral_constant<int, 1>{}, std::false_type{});
+            }
+        } else if constexpr (PAIR && WTR) {
+            // transposing reads (WTR, XTR): 32 x 32 x 16 MFMAs.  (On 16 x 16 x 32 ones, rolling as above, the weight gradients of 131072 rows,
+            // 64 experts, 2048 x 1408 take 2.10 ms for the two where these take 2.06, the input gradients 1.95 against 1.92: the LDS, which serves
+            // transposing reads at two thirds of the rate of others, is the limit there, and the next item's weights come in one bunch.)
             // Software pipeline over "blocks" (half a K-slice: one 16-byte chunk per row and
             // lane half, 8 MFMAs): the fragments of block b+1 are read while block b
             // multiplies.  Two barriers per pair of items c, c+1 (a "double step"):
@@ -781,13 +979,12 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 const int chunk = 2 * sub + khalf;
 #pragma unroll
                 for (int fn = 0; fn < FN; ++fn) {
-                    if constexpr (WTR) wf[fn] = read_tr8<1024>(sw + wtr_off[fn] + sub * 4096);
-                    else wf[fn] = *reinterpret_cast<const bf16x8*>(sw + lds_off64(wfrag_row[fn], chunk));
+                    wf[fn] = read_tr8<1024>(sw + wtr_off[fn] + sub * 4096);
                 }
 #pragma unroll
                 for (int fm = 0; fm < ACT; ++fm) {
                     if constexpr (XTR) xf[fm] = read_tr8<1024>(sx + xtr_off[fm] + sub * 4096);
-                    else xf[fm] = *reinterpret_cast<const bf16x8*>(sx + lds_off64(xfrag_row[fm], chunk));
+                    else xf[fm] = *reinterpret_cast<const bf16x8*>(sx + lds_off64(wm * TM + (lane & 31), chunk) + fm * 2048);
                 }
                 if constexpr (MASK_TAIL) {      // (a fragment is one 16-byte chunk: masked whole or not at all)
                     const int at = (item - (KT - 2)) * BK + 16 * sub + 8 * khalf;
@@ -960,23 +1157,17 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             // fragments and activation fragments 0..FM/2-1, block 1 the other activation
             // fragments and reuses the weights.
             constexpr int HM = FM / 2;
-            auto load_frag = [&](const uint8_t* base, int row) -> i32x8 {
-                const int chunk = 2 * khalf;
-                const u32x4 lo = *reinterpret_cast<const u32x4*>(base + lds_off64(row, chunk));
-                const u32x4 hi = *reinterpret_cast<const u32x4*>(base + lds_off64(row, chunk + 1));
-                return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-            };
             auto load_w_x0 = [&](i32x8 (&wf)[FN], i32x8 (&xh)[HM], int slot_i) {
                 const uint8_t* sx = smem + slot_i * TL::STAGE_BYTES;
 #pragma unroll
-                for (int fn = 0; fn < FN; ++fn) wf[fn] = load_frag(sx + BM * 64, wfrag_row[fn]);
+                for (int fn = 0; fn < FN; ++fn) wf[fn] = load_q(sx + BM * 64 + wq_block(fn), wq_lo, wq_hi);
 #pragma unroll
-                for (int fm = 0; fm < HM; ++fm) xh[fm] = load_frag(sx, xfrag_row[fm]);
+                for (int fm = 0; fm < HM; ++fm) xh[fm] = load_q(sx + fm * 2048, xq_lo, xq_hi);
             };
             auto load_x1 = [&](i32x8 (&xh)[HM], int slot_i) {
                 const uint8_t* sx = smem + slot_i * TL::STAGE_BYTES;
 #pragma unroll
-                for (int fm = 0; fm < HM; ++fm) xh[fm] = load_frag(sx, xfrag_row[HM + fm]);
+                for (int fm = 0; fm < HM; ++fm) xh[fm] = load_q(sx + (HM + fm) * 2048, xq_lo, xq_hi);
             };
             // KTAIL: the fragment of the item in the first (HALF_ITEM 0) or second slot of the last pair, masked
             // where the pair before it reached (in groups of 8 bytes of a lane's 32)
@@ -1159,6 +1350,21 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             // behind them.
             wait_vmcnt<L>();
             landed = issued - 2;
+        }
+        if constexpr (B16) {
+            // lane groups 1 and 3 of row block 2 fm against lane groups 0 and 2 of the one behind it: quads of columns 2 q + lane / 32
+#pragma unroll
+            for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+                for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const int a = 2 * fn + i / 4, v = i % 4;
+                        const u32x2 s = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc16[a][2 * fm][v]), __float_as_uint(acc16[a][2 * fm + 1][v]),
+                                                                         false, false);
+                        acc[fn][fm][8 * (i / 4) + v] = __uint_as_float(s[0]);
+                        acc[fn][fm][8 * (i / 4) + 4 + v] = __uint_as_float(s[1]);
+                    }
         }
         if constexpr (MSC) mfma_results_guard();    // the last MFMAs' results are read by VALU code from here on
         FMOE_TRACE_STAMP(1);
