@@ -24,6 +24,7 @@ namespace fmoe {
 // counted wait behind them, where the compiler's own count of what is still in flight is exact
 // (behind the join of the epilogue's variants it is not: it has to assume the path that stored
 // nothing).  The ring kernel converts the row indices it fetched before the epilogue there.
+constexpr int kEpilogueStageBytes = 4096;      // LDS of a wave for the staged form (ALWAYS_VEC)
 struct NoAfterStores {
     __device__ __forceinline__ void operator()() const {}
     __device__ __forceinline__ void block_done(int) const {}
@@ -84,7 +85,7 @@ template <int FM, int FN, int TM, int TN, bool FP8, int EPI, bool ALWAYS_VEC = f
           bool OUT2 = false, bool ROW_IL = false, typename AfterStores = NoAfterStores, bool MSC = false>
 __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)[FN][FM], int expert,
                                               int n0, int64_t row0, int rows_valid, int wm, int wn,
-                                              int lane, AfterStores after_stores = AfterStores(),
+                                              int lane, uint8_t* stage = nullptr, AfterStores after_stores = AfterStores(),
                                               uint64_t* ets = nullptr) {
     constexpr bool SWIGLU = EPI == FMOE_EPI_SWIGLU;
     constexpr bool GATED = EPI == FMOE_EPI_GATED;   // out = silu(gate from p.aux) * (acc + bias); bf16 operands
@@ -220,7 +221,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
     auto run = [&](auto has_bias_c, auto has_aux_c) {
         constexpr bool HAS_BIAS = decltype(has_bias_c)::value;
         constexpr bool HAS_AUX = SWIGLU && decltype(has_aux_c)::value;   // keep the pre-activations (training)
-        constexpr bool QUAD = ALWAYS_VEC && !SWIGLU && FN_OUT == 2;   // plain and SiLU epilogues of the ring kernel, bf16 and e4m3
         // per-column biases of this lane, indexed like rsw
         float bv[FN_OUT][2][2][4], bv2[FN_OUT][2][2][4];
         // with a bias, at least one of the two pointers is set: both loads go through a valid
@@ -250,146 +250,169 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                     }
         __builtin_amdgcn_sched_barrier(0);
         FMOE_EPI_STAMP(0);
-        // GATED in the rearranged form: a lane's gate values are the 16 bytes at the position its
-        // store i of a row block writes; the four loads of block fm + 1 go out before block fm's
-        // arithmetic, so that one memory latency per tile is waited for, not one per block.
-        u32x4 gate_next[4] = {};
-        auto fetch_gate = [&](int fm, u32x4 (&g)[4]) {
+        // Staged form.  The store unit merges what ADJACENT lanes write: a 128 KB tile drains in 1.3 us where neighbouring lanes write
+        // neighbouring bytes and in 3.9 where a lane's neighbour in memory is 32 lanes away, as in the MFMA's layout.  So a row block
+        // (two of them where the wave has 32 output columns) goes through the wave's own 4 KB of LDS: pieces of 4 columns in, whole rows of
+        // 16-byte chunks out, which 8 (4) adjacent lanes store.  Rearranging the same rows in registers (lane swaps, transposes of
+        // quads by DPP moves and selects) was 330 of an epilogue's 640 vector instructions, and the two waves of a SIMD are bound by those.
+        // Chunk c of row r lies at position c ^ (r / 2) % 8 (c ^ (r / 4) % 4), its two halves swapped in rows 16..31 of each 32: neither
+        // the writes nor the reads meet in a bank.  A wave's LDS instructions execute in order, nothing has to be waited for in between.
+        if constexpr (ALWAYS_VEC) {
+            constexpr int CH = 4 * FN_OUT;                      // 16-byte chunks of a row
+            constexpr int RB = FN_OUT == 2 || FM < 2 ? 1 : 2;   // row blocks at a time
+            constexpr int RPI = kWave / CH;                     // rows of a store instruction
+            constexpr int NI = 32 * RB / RPI;
+            constexpr int KINDS = HAS_AUX ? 3 : 1;              // the result, the two pre-activations
+            static_assert(32 * RB * CH * 16 <= kEpilogueStageBytes, "a wave's share of the staging rows");
             int l = lane;
             asm volatile("" : "+v"(l));
-            const int quad_row = 4 * ((l & 31) >> 2);
-            const int col = col0 + 32 * (l >> 5) + 8 * (l & 3);
+            const int wr = l & 31;
+            const int put_at = wr * (16 * CH) + ((CH == 8 ? (wr >> 1) & 7 : (wr >> 2) & 3) << 4) + ((khalf ^ (wr >> 4)) << 3);
+            const int sr = l / CH, sc = l % CH;
+            const int take_at = sr * (16 * CH) + ((sc ^ (l >> 4)) << 4);
+            // rows that this lane may store, counted from its row of a store instruction
+            const int row_limit = col0 + 8 * sc + 7 < p.N ? rows_valid - sr : 0;
+            auto put = [&](int b, int piece, uint32_t lo, uint32_t hi) {
+                *reinterpret_cast<u32x2*>(stage + (b * 32 * 16 * CH) + (put_at ^ (piece << 4))) = u32x2{lo, hi};
+            };
+            u32x4 rows[NI];
+            auto take = [&]() {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const bool ok = frag_row(fm) + quad_row + i < rows_valid && col + 7 < p.N;
-                const uint16_t* src = p.aux + (row0 + (ok ? frag_row(fm) + quad_row + i : 0)) * p.aux_stride + (ok ? col : 0);
-                if (p.gate_vec16) {
-                    g[i] = *reinterpret_cast<const u32x4*>(src);
-                } else {
-                    uint32_t e[8];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) e[j] = ok ? (uint32_t)src[j] : 0u;
-                    g[i] = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
+                for (int i = 0; i < NI; ++i) {
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(stage + i * 1024 + (CH == 8 && (i & 1) ? take_at ^ 64 : take_at));
+                    const bool swapped = ((i * RPI) >> 4) & 1;
+                    rows[i] = swapped ? u32x4{v[2], v[3], v[0], v[1]} : v;
                 }
-            }
-        };
-        if constexpr (QUAD && GATED) fetch_gate(0, gate_next);
-        // rows outermost: the stores that complete a row's 128-byte line follow each other
+            };
+            // GATED: a lane's gate values are the 16 bytes at the position its store i of a row block writes; the loads of
+            // block fm + 1 go out before block fm's arithmetic, so that one memory latency per tile is waited for, not one per block.
+            u32x4 gate_next[NI] = {}, gate_cur[NI] = {};
+            auto fetch_gate = [&](int fm) {
 #pragma unroll
-        for (int fm = 0; fm < FM; ++fm) {
-            if (fm > 0) FMOE_EPI_STAMP(fm);
-            if constexpr (QUAD) {
-                u32x4 gate_cur[4];
-                if constexpr (GATED) {
+                for (int i = 0; i < NI; ++i) {
+                    const int col = col0 + 8 * sc;
+                    const bool ok = frag_row(fm) + i * RPI < row_limit;
+                    const uint16_t* src = p.aux + (row0 + (ok ? frag_row(fm) + i * RPI + sr : 0)) * p.aux_stride + (ok ? col : 0);
+                    if (p.gate_vec16) {
+                        gate_next[i] = *reinterpret_cast<const u32x4*>(src);
+                    } else {
+                        uint32_t e[8];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) gate_cur[i] = gate_next[i];
-                    if (fm + 1 < FM) fetch_gate(fm + 1, gate_next);
+                        for (int j = 0; j < 8; ++j) e[j] = ok ? (uint32_t)src[j] : 0u;
+                        gate_next[i] = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
+                    }
                 }
-                // The store unit merges what ADJACENT lanes write: a lane and its partner 32 lanes
-                // away cost two requests even for neighbouring bytes, four adjacent lanes on 64
-                // contiguous bytes cost one (a 128 KB tile drains in 1.3 us instead of 3.9).  So:
-                // the halves of the wave trade pieces until a low lane owns columns 0..31 of its row
-                // and its partner 32..63, then every quad of lanes transposes its 4 rows x 4 chunks
-                // of 16 bytes, and store i of the block writes row 4q + i from the 4 lanes of quad q.
-                uint32_t pk[8][2];          // piece g: columns 8g + 4*khalf + 0..3 of the wave's 64
+            };
+            // what the lane contributes to piece 4 fn + 2 gp + q of row block fm, rounded to bf16
+            auto emit = [&](int fm, int kind) {
 #pragma unroll
-                for (int fn = 0; fn < 2; ++fn)
+                for (int fn = 0; fn < FN_OUT; ++fn)
 #pragma unroll
                     for (int gp = 0; gp < 2; ++gp)
 #pragma unroll
-                        for (int q = 0; q < 2; ++q)
+                        for (int q = 0; q < 2; ++q) {
+                            uint32_t pk[2];
 #pragma unroll
-                            for (int j = 0; j < 4; j += 2) {
+                            for (int j = 0; j < 4; j += 2) {        // two columns at a time: one conversion instruction rounds a pair
                                 const int v = 4 * (2 * gp + q) + j;
-                                float ya = acc[fn][fm][v], yb = acc[fn][fm][v + 1];
-                                if (FP8) {
-                                    if (SCALE) {
-                                        ya *= rsa[fm] * rsw[fn][gp][q][j];
-                                        yb *= rsa[fm] * rsw[fn][gp][q][j + 1];
+                                auto branch = [&](float a, float b, const float (&sw)[4], const float (&bias)[4], const void* given) -> uint32_t {
+                                    if (FP8) {
+                                        if (SCALE) {
+                                            a *= rsa[fm] * sw[j];
+                                            b *= rsa[fm] * sw[j + 1];
+                                        }
+                                        if (HAS_BIAS && given) {
+                                            rbf2(a, b);
+                                            a += bias[j];
+                                            b += bias[j + 1];
+                                        }
+                                    } else if (HAS_BIAS) {
+                                        a += bias[j];
+                                        b += bias[j + 1];
                                     }
-                                    if (HAS_BIAS && p.bias) {
-                                        rbf2(ya, yb);
-                                        ya += bv[fn][gp][q][j];
-                                        yb += bv[fn][gp][q][j + 1];
-                                    }
-                                } else if (HAS_BIAS) {
-                                    ya += bv[fn][gp][q][j];
-                                    yb += bv[fn][gp][q][j + 1];
-                                }
-                                if (EPI == FMOE_EPI_SILU) {
-                                    rbf2(ya, yb);
-                                    ya = fast_silu_f32(ya);
-                                    yb = fast_silu_f32(yb);
-                                }
-                                pk[4 * fn + 2 * gp + q][j / 2] = pack_bf16(ya, yb);
+                                    return pack_bf16(a, b);
+                                };
+                                auto low = [](uint32_t u) { return __uint_as_float(u << 16); };
+                                auto high = [](uint32_t u) { return __uint_as_float(u & 0xffff0000u); };
+                                uint32_t y = kind == 2 ? 0u : branch(acc[fn][fm][v], acc[fn][fm][v + 1], rsw[fn][gp][q], bv[fn][gp][q], p.bias);
+                                uint32_t u = 0;
+                                if (SWIGLU && kind != 1)
+                                    u = branch(acc[fn + FN / 2][fm][v], acc[fn + FN / 2][fm][v + 1], rsw2[fn][gp][q], bv2[fn][gp][q], p.bias2);
+                                if (kind == 2) y = u;
+                                if (EPI == FMOE_EPI_SILU || (SWIGLU && kind == 0)) y = pack_bf16(fast_silu_f32(low(y)), fast_silu_f32(high(y)));
+                                if (SWIGLU && kind == 0) y = pack_bf16(low(y) * low(u), high(y) * high(u));
+                                pk[j / 2] = y;
                             }
-                uint32_t ch[4][4];          // chunk c: columns 32*khalf + 8c + 0..7, afterwards row 4q + c's
+                            put(fm % RB, 4 * fn + 2 * gp + q, pk[0], pk[1]);
+                        }
+            };
+            auto store = [&](int fm0, int kind) {       // the rows taken last
+                const int64_t stride = kind ? p.aux_stride : p.out_stride;
+                const uint32_t lane_off = ((uint32_t)sr * (uint32_t)stride + (uint32_t)(8 * sc)) * 2u;
 #pragma unroll
-                for (int c = 0; c < 4; ++c)
-#pragma unroll
-                    for (int d = 0; d < 2; ++d) {
-                        const u32x2 s = __builtin_amdgcn_permlane32_swap(pk[c][d], pk[c + 4][d], false, false);
-                        ch[c][d] = s[0];
-                        ch[c][2 + d] = s[1];
+                for (int i = 0; i < NI; ++i) {
+                    const int fm = fm0 + i * RPI / 32, in_block = i * RPI % 32;
+                    const int64_t block_row = row0 + frag_row(fm);
+                    uint16_t* obase = (kind == 0 ? p.out : kind == 1 ? p.aux : p.aux2) + block_row * stride;
+                    if constexpr (OUT2) {
+                        if (p.out2) {       // (scalar arithmetic: everything here is wave-uniform)
+                            // (offsets that are not the promised e * 2h are not followed out of
+                            // the two tensors: the block's row is forced into [0, 2h), whole blocks)
+                            int64_t m = block_row - (int64_t)expert * (2 * p.out_half);
+                            m = m < 0 ? 0 : (m > 2 * p.out_half - 32 ? 2 * p.out_half - 32 : m);
+                            m &= ~(int64_t)31;
+                            const bool upper = m >= p.out_half;
+                            obase = (upper ? p.out2 : p.out) +
+                                    ((int64_t)expert * p.out_half + (upper ? m - p.out_half : m)) * p.out_stride;
+                        }
                     }
-                int l = lane;
-                asm volatile("" : "+v"(l));
-                const bool odd = (l & 1) != 0, up = (l & 2) != 0;
-#pragma unroll
-                for (int pr = 0; pr < 4; pr += 2)       // lanes j, j ^ 1 trade across slots (pr, pr + 1)
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        const uint32_t send = odd ? ch[pr][d] : ch[pr + 1][d];
-                        const uint32_t recv = (uint32_t)__builtin_amdgcn_mov_dpp((int)send, 0xB1, 0xF, 0xF, true);
-                        ch[pr][d] = odd ? recv : ch[pr][d];
-                        ch[pr + 1][d] = odd ? ch[pr + 1][d] : recv;
-                    }
-#pragma unroll
-                for (int pr = 0; pr < 2; ++pr)          // lanes j, j ^ 2 trade across slots (pr, pr + 2)
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        const uint32_t send = up ? ch[pr][d] : ch[pr + 2][d];
-                        const uint32_t recv = (uint32_t)__builtin_amdgcn_mov_dpp((int)send, 0x4E, 0xF, 0xF, true);
-                        ch[pr][d] = up ? recv : ch[pr][d];
-                        ch[pr + 2][d] = up ? ch[pr + 2][d] : recv;
-                    }
-                const int64_t block_row = row0 + frag_row(fm);
-                uint16_t* obase = p.out + block_row * p.out_stride;
-                if constexpr (OUT2) {
-                    if (p.out2) {       // (as below: wave-uniform, forced into the two tensors)
-                        int64_t m = block_row - (int64_t)expert * (2 * p.out_half);
-                        m = m < 0 ? 0 : (m > 2 * p.out_half - 32 ? 2 * p.out_half - 32 : m);
-                        m &= ~(int64_t)31;
-                        const bool upper = m >= p.out_half;
-                        obase = (upper ? p.out2 : p.out) +
-                                ((int64_t)expert * p.out_half + (upper ? m - p.out_half : m)) * p.out_stride;
-                    }
-                }
-                const int quad_row = 4 * ((l & 31) >> 2);
-                const int col = col0 + 32 * (l >> 5) + 8 * (l & 3);
-                const uint32_t lane_off = ((uint32_t)quad_row * (uint32_t)p.out_stride + (uint32_t)(32 * (l >> 5) + 8 * (l & 3))) * 2u;
-                if constexpr (GATED) {      // ch holds round(acc + bias): times the rounded SiLU of the gate
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
+                    u32x4 v = rows[i];
+                    if constexpr (GATED) {              // round(acc + bias) times the rounded SiLU of the gate
 #pragma unroll
                         for (int d = 0; d < 4; ++d) {
                             float ga = __uint_as_float(gate_cur[i][d] << 16), gb = __uint_as_float(gate_cur[i][d] & 0xffff0000u);
                             ga = fast_silu_f32(ga);
                             gb = fast_silu_f32(gb);
                             rbf2(ga, gb);
-                            ch[i][d] = pack_bf16(ga * __uint_as_float(ch[i][d] << 16), gb * __uint_as_float(ch[i][d] & 0xffff0000u));
+                            v[d] = pack_bf16(ga * __uint_as_float(v[d] << 16), gb * __uint_as_float(v[d] & 0xffff0000u));
                         }
+                    }
+                    const bool ok = frag_row(fm) + in_block < row_limit;
+                    store16_uniform_base(obase + in_block * stride + col0, ok ? lane_off : kDropLane, v);
                 }
+            };
+            if constexpr (GATED) fetch_gate(0);
+            // a step's rows are stored behind the next step's arithmetic, by when they have arrived
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    uint16_t* base = obase + i * p.out_stride + col0;
-                    const bool ok = frag_row(fm) + quad_row + i < rows_valid && col + 7 < p.N;
-                    store16_uniform_base(base, ok ? lane_off : kDropLane, u32x4{ch[i][0], ch[i][1], ch[i][2], ch[i][3]});
+            for (int step = 0; step <= FM / RB * KINDS; ++step) {
+                const int fm = step / KINDS * RB, kind = step % KINDS;
+                if (step < FM / RB * KINDS) {
+#pragma unroll
+                    for (int b = 0; b < RB; ++b) emit(fm + b, kind);
+                }
+                if (step > 0) {
+                    const int before = step - 1;
+                    store(before / KINDS * RB, before % KINDS);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (before % KINDS == KINDS - 1) {
+                        FMOE_EPI_STAMP(before / KINDS * RB);
+                        after_stores.block_done(before / KINDS * RB);
+                    }
+                }
+                if (step < FM / RB * KINDS) {
+                    if constexpr (GATED) {
+#pragma unroll
+                        for (int i = 0; i < NI; ++i) gate_cur[i] = gate_next[i];
+                        if (fm + 1 < FM) fetch_gate(fm + 1);
+                    }
+                    take();
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                after_stores.block_done(fm);
-                continue;
             }
+        }
+        // rows outermost: the stores that complete a row's 128-byte line follow each other
+#pragma unroll
+        for (int fm = 0; !ALWAYS_VEC && fm < FM; ++fm) {
             // GATED: the row block's gate values, all loads of the block issued together (one memory
             // latency per 32-row block; loaded where they are used, every group of 8 waits out its own)
             u32x2 graw[FN_OUT][2][2];
@@ -503,16 +526,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                         }
                     // base: first element of the 32-row block's first row (wave-uniform)
                     auto store = [&](const float (&val)[2][4], uint16_t* base, int64_t stride) {
-                        if constexpr (ALWAYS_VEC) {
-                            const uint32_t lane_off = lane_offset(stride);
-                            const u32x2 s0 = __builtin_amdgcn_permlane32_swap(pack_bf16(val[0][0], val[0][1]),
-                                                                              pack_bf16(val[1][0], val[1][1]), false, false);
-                            const u32x2 s1 = __builtin_amdgcn_permlane32_swap(pack_bf16(val[0][2], val[0][3]),
-                                                                              pack_bf16(val[1][2], val[1][3]), false, false);
-                            const int nb = nq + 8 * khalf;
-                            const bool ok = row_ok[fm] && nb + 7 < p.N;
-                            store16_uniform_base(base + nq, ok ? lane_off : kDropLane, u32x4{s0[0], s1[0], s0[1], s1[1]});
-                        } else if (p.vec_store) {
+                        if (p.vec_store) {
                             const uint32_t lane_off = lane_offset(stride);
                             // pair the quads of the two lane halves: low lanes end up with columns
                             // nq..nq+7, high lanes with nq+8..nq+15 of their row
@@ -537,18 +551,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                     };
                     const int64_t block_row = row0 + frag_row(fm);
                     uint16_t* obase = p.out + block_row * p.out_stride;
-                    if constexpr (OUT2) {
-                        if (p.out2) {       // (scalar arithmetic: everything here is wave-uniform)
-                            // (offsets that are not the promised e * 2h are not followed out of
-                            // the two tensors: the block's row is forced into [0, 2h), whole blocks)
-                            int64_t m = block_row - (int64_t)expert * (2 * p.out_half);
-                            m = m < 0 ? 0 : (m > 2 * p.out_half - 32 ? 2 * p.out_half - 32 : m);
-                            m &= ~(int64_t)31;
-                            const bool upper = m >= p.out_half;
-                            obase = (upper ? p.out2 : p.out) +
-                                    ((int64_t)expert * p.out_half + (upper ? m - p.out_half : m)) * p.out_stride;
-                        }
-                    }
                     store(o, obase, p.out_stride);
                     if (HAS_AUX) {
                         store(pg, p.aux + block_row * p.aux_stride, p.aux_stride);
@@ -559,7 +561,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            after_stores.block_done(fm);
         }
         // Everything older than this epilogue's own stores has completed: a wait that costs
         // nothing (the loads it names were needed above) but tells the compiler so.  Without it
@@ -569,14 +570,13 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
         // which the compiler cannot see, on every iteration.
         FMOE_EPI_STAMP(FM);
         // The number of store instructions issued above, whatever the lanes' predicates: 4 per row
-        // block in the rearranged form, one per column group (and per output tensor) otherwise.
+        // block of 64 columns in the staged form, one per column group (and per output tensor) otherwise.
         // The ring kernel's first double step of the next tile skips its own counted wait on the
         // strength of this one (see skip_wait there), which is only sound when every one of these
         // stores was issued unconditionally, i.e. through store16_uniform_base (ALWAYS_VEC).
-        constexpr int kStoresIssued = FM * (QUAD ? 4 : FN_OUT * 2 * (HAS_AUX ? 3 : 1));
-        static_assert(!QUAD || FN_OUT * 2 == 4, "the rearranged form stores as many pieces as the column-group form");
+        constexpr int kStoresIssued = FM * FN_OUT * 2 * (HAS_AUX ? 3 : 1);
         static_assert(kStoresIssued <= 63, "vmcnt is a 6-bit field");
-        wait_vmcnt<kStoresIssued>();      // (the scalar-store path issues more)
+        wait_vmcnt<kStoresIssued>();      // (the element-store path issues more)
         after_stores();
     };
     if (SWIGLU && p.aux) {

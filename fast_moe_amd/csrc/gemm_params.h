@@ -187,6 +187,10 @@ __device__ __forceinline__ void wait_vmcnt() {   // s_waitcnt vmcnt(N) only
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
+__device__ __forceinline__ void wait_lgkmcnt0() {   // s_waitcnt lgkmcnt(0) only
+    __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));
+}
+
 // 16-byte store through a buffer descriptor over [base, base + 2 GiB): a lane whose offset is
 // kDropLane lies outside the descriptor's range and the hardware drops its part, so the
 // instruction is issued whatever the lanes' predicates are.  The compiler then knows how many

@@ -894,6 +894,8 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 mma_block(xh0, h0, std::integral_constant<bool, HALF == 0>{}, no, no, 0, kitem + 1, mask_c);
                 if constexpr (HALF != 0) interleave(dense, no);
                 __builtin_amdgcn_sched_barrier(0);
+                // (all of this wave's reads of item c+1: behind A' its slot may take a tile's output rows)
+                wait_lgkmcnt0();
                 // pair (c+2, c+3) is older than the other pairs in flight, 2L instructions each, the one the
                 // first half just issued among them
                 if (!skip_wait) {
@@ -1099,6 +1101,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 mma_block(wfa, xfa, std::integral_constant<bool, HALF == 0>{}, act_c);
                 if constexpr (HALF != 0) interleave();
                 __builtin_amdgcn_sched_barrier(0);
+                wait_lgkmcnt0();            // (as above)
                 // pair (c+2, c+3) is older than the other pairs in flight, 2L instructions each, the one the
                 // first half just issued among them
                 if (!skip_wait) {
@@ -1281,6 +1284,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 __builtin_amdgcn_sched_barrier(0);
                 mma_block(qwb, qx0, std::integral_constant<int, 0>{}, std::integral_constant<bool, HALF == 0>{}, full);
                 __builtin_amdgcn_sched_barrier(0);
+                wait_lgkmcnt0();            // (as in the bf16 loop)
                 if (!skip_wait) {
                     if (HALF == 0) wait_vmcnt<2 * L * (TL::AHEAD - 1)>();
                     else wait_vmcnt<2 * L * (TL::AHEAD - 2)>();
@@ -1350,6 +1354,8 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             // behind them.
             wait_vmcnt<L>();
             landed = issued - 2;
+            wait_lgkmcnt0();
+            __builtin_amdgcn_s_barrier();       // every wave has read the last slice: its slot takes the output rows
         }
         if constexpr (B16) {
             // lane groups 1 and 3 of row block 2 fm against lane groups 0 and 2 of the one behind it: quads of columns 2 q + lane / 32
@@ -1414,15 +1420,19 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 if (fm == 0) sc_fetch_scales(cur, sc_idx, sc_xraw, sc_wraw);
             }
         };
+        // The epilogue stages its rows in the slot of the tile's last slice: every wave has read it (A', with the reads it waits
+        // for, lies behind the last of them), and the next tile's first refill of it lies behind the next barrier B.
+        static_assert(TL::STAGE_BYTES >= NW * kEpilogueStageBytes, "the epilogue's rows fit a slot");
+        uint8_t* const stage = smem + (cslot == 0 ? STAGES - 1 : cslot - 1) * TL::STAGE_BYTES + wave * kEpilogueStageBytes;
         auto hooks = make_hooks(scales_behind_block0, convert_rows);
 #ifdef FMOE_TRACE
         gemm_epilogue<FM, FN, TM, TN, FP8, EPI, true, PAIR, XTR, ROW_IL, decltype(hooks), MSC>(
-            p, acc, done.expert, done.nt * BN_OUT, done.row0, done.rows_valid, wm, wn, lane, hooks,
+            p, acc, done.expert, done.nt * BN_OUT, done.row0, done.rows_valid, wm, wn, lane, stage, hooks,
             (p.trace && tile_i < 32 && (wave == 0 || wave == NW / 2)) ? tstamp + 12 : nullptr);
 #else
         static_assert(kEpilogueStoresUnconditional, "skip_wait needs an epilogue whose stores are all issued");
         gemm_epilogue<FM, FN, TM, TN, FP8, EPI, kEpilogueStoresUnconditional, PAIR, XTR, ROW_IL, decltype(hooks), MSC>(
-            p, acc, done.expert, done.nt * BN_OUT, done.row0, done.rows_valid, wm, wn, lane, hooks);
+            p, acc, done.expert, done.nt * BN_OUT, done.row0, done.rows_valid, wm, wn, lane, stage, hooks);
 #endif
 #ifdef FMOE_TRACE
         FMOE_TRACE_STAMP(3);

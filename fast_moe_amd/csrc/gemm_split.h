@@ -101,8 +101,9 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const GemmParams p) {
             }
     }
     const int n0 = tile.nt * (EPI == FMOE_EPI_SWIGLU ? 128 : 256);
+    __shared__ __align__(16) uint8_t stage[4 * kEpilogueStageBytes];
     gemm_epilogue<1, 2, 32, 64, FP8, EPI, true, true, false, false, NoAfterStores, MSC>(p, acc, tile.expert, n0, tile.row0, tile.rows_valid, rb, wn,
-                                                                                       lane);
+                                                                                       lane, stage + wn * kEpilogueStageBytes);
 }
 
 }  // namespace fmoe

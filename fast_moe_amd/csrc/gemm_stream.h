@@ -323,7 +323,8 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_stream_kernel(const GemmP
             fetch_scales(nxt, sraw, xs, ws);
         }
         gemm_epilogue<FM, FN, TM, TN, FP8, EPI, true, false, false, false, NoAfterStores, MSC>(
-            p, acc, cur.expert, cur.nt * BN_OUT, cur.row0, cur.rows_valid, 0, wn, lane);
+            p, acc, cur.expert, cur.nt * BN_OUT, cur.row0, cur.rows_valid, 0, wn, lane,
+            smem + STAGE_BYTES + wn * kEpilogueStageBytes);     // (stage 1: filled again behind the next tile's first barrier)
         if (has_next) pack_scales(xs, ws);
         cur = nxt;
     }

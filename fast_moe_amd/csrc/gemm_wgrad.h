@@ -156,8 +156,12 @@ __global__ __launch_bounds__(WgradTile::NT, 3) void grouped_wgrad_kernel(const G
                 }
             }
         } else {
+            // the output rows are staged in the buffer read last: behind this barrier by nobody any more, and filled again behind the next one
+            __syncthreads();
+            uint8_t* const stage = smem + (buffer ^ 1) * 2 * WgradTile::OPERAND_BYTES + (wm * 2 + wn) * kEpilogueStageBytes;
+            static_assert(2 * WgradTile::OPERAND_BYTES >= 4 * kEpilogueStageBytes, "the epilogue's rows fit a buffer");
             gemm_epilogue<2, 2, 64, 64, false, FMOE_EPI_NONE, true, true, true>(p, acc, expert, done, (int64_t)expert * t.m + m0, rows_valid, wm,
-                                                                                wn, lane);
+                                                                                wn, lane, stage);
         }
         if (!more) break;
     }
