@@ -22,7 +22,7 @@ PLAN_NONE, PLAN_RING, PLAN_STAGED, PLAN_STAGED_SHORT, PLAN_ELEMENT = -1, 0, 1, 2
 EXPORTED_SYMBOLS = (
     "fmoe_version", "fmoe_last_error", "fmoe_route_workspace_bytes", "fmoe_route_topk",
     "fmoe_route_from_topk", "fmoe_quant_rows_e4m3",
-    "fmoe_quant_rows_workspace_bytes", "fmoe_quant_rows_e4m3_ws", "fmoe_grouped_gemm", "fmoe_grouped_gemm_plan",
+    "fmoe_quant_rows_workspace_bytes", "fmoe_quant_rows_e4m3_ws", "fmoe_quant_expert_weights_e4m3", "fmoe_grouped_gemm", "fmoe_grouped_gemm_plan",
     "fmoe_grouped_gemm_workspace_bytes", "fmoe_grouped_gemm_ws",
     "fmoe_combine",
     "fmoe_silu_mul", "fmoe_transpose_last2", "fmoe_jagged_transpose", "fmoe_segment_colsum",
@@ -91,6 +91,9 @@ def load() -> ctypes.CDLL:
     lib.fmoe_quant_rows_workspace_bytes.argtypes = [c_int] + [c_int64] * 6 + [c_int]
     lib.fmoe_quant_rows_e4m3_ws.restype = c_int
     lib.fmoe_quant_rows_e4m3_ws.argtypes = (lib.fmoe_quant_rows_e4m3.argtypes[:-1] + [c_void_p, c_size_t, c_void_p])
+    lib.fmoe_quant_expert_weights_e4m3.restype = c_int
+    lib.fmoe_quant_expert_weights_e4m3.argtypes = ([c_void_p, c_int] + [c_int64] * 6 + [c_void_p] + [c_int64] * 3 +
+                                                   [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p])
     lib.fmoe_grouped_gemm.restype = c_int
     lib.fmoe_grouped_gemm.argtypes = [POINTER(GemmDesc), c_void_p]
     lib.fmoe_grouped_gemm_workspace_bytes.restype = c_size_t

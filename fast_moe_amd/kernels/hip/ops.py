@@ -188,11 +188,13 @@ def route_from_topk(topk_idx: torch.Tensor, num_experts: int) -> Dict[str, torch
 
 # ---------------------------------------------------------------- fp8 quant
 def quant_rows_fp8(a: torch.Tensor, apply_silu: bool = False, reciprocal_scale: bool = False,
-                   out_like_input: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
+                   out_like_input: bool = False, offsets: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """Row-wise (last dim) e4m3fn quantisation of ``a`` [..., rows, cols] read through its strides.
 
     Returns ``(q, scale)``: q is float8_e4m3fn, contiguous in a's logical shape (or laid out
-    with a's own strides when ``out_like_input``), scale is fp32 with a's leading shape."""
+    with a's own strides when ``out_like_input``), scale is fp32 with a's leading shape.
+    ``offsets`` (int64 [a.shape[0] + 1], weights of experts): the caller uses the result in GEMMs over these offsets only, and
+    what belongs to an expert without rows may stay unwritten (fmoe_quant_expert_weights_e4m3)."""
     if not out_like_input and a.ndim == 2:
         pair = _lib.host().quant_rows(a, int(apply_silu), int(reciprocal_scale), _stream(a))
         if pair is not None:
@@ -224,8 +226,12 @@ def quant_rows_fp8(a: torch.Tensor, apply_silu: bool = False, reciprocal_scale: 
     ws_bytes = 0
     if a3.stride(1) == 1 and a3.stride(2) != 1 and not out_like_input:      # rows are columns in memory, but not of q
         ws_bytes = lib.fmoe_quant_rows_workspace_bytes(*args[1:8], args[8])
-    if ws_bytes:
-        ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
+    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev) if ws_bytes else None
+    if (offsets is not None and a.ndim == 3 and not (apply_silu or reciprocal_scale or out_like_input) and offsets.dtype == torch.int64
+            and offsets.device == dev and offsets.ndim == 1 and offsets.is_contiguous() and offsets.numel() == B + 1):
+        rc = lib.fmoe_quant_expert_weights_e4m3(*args[:8], *args[9:14], offsets.data_ptr(), None if ws is None else ws.data_ptr(),
+                                                ws_bytes, _stream(a))
+    elif ws_bytes:
         rc = lib.fmoe_quant_rows_e4m3_ws(*args, ws.data_ptr(), ws_bytes, _stream(a))
     else:
         rc = lib.fmoe_quant_rows_e4m3(*args, _stream(a))

@@ -106,13 +106,16 @@ def cached_quantize_expert_weights(weight: torch.Tensor) -> Tuple[torch.Tensor, 
     return weight_quant_cache.get(weight, quantize_expert_weights)
 
 
-def _weight_pair(weight: torch.Tensor, fp8_weight) -> Tuple[torch.Tensor, torch.Tensor]:
+def _weight_pair(weight: torch.Tensor, fp8_weight, offsets=None) -> Tuple[torch.Tensor, torch.Tensor]:
     """The (e4m3 [E, K, N], scale [E, N]) pair of ``weight``: the caller's, checked for shape, or a
-    fresh quantisation.  (A caller's own pair may carry any positive scales: the GEMM takes the
+    fresh quantisation (``offsets``: for a GEMM over these only, experts without rows may be left out).  (A caller's own pair may carry any positive scales: the GEMM takes the
     scales for powers of two only when they are tensors this package's quantiser returned,
     ``ops.scales_are_pow2``.)"""
     if fp8_weight is None:
-        return quantize_expert_weights(weight)
+        if offsets is None:
+            return quantize_expert_weights(weight)
+        q, s = ops.quant_rows_fp8(weight.permute(0, 2, 1), offsets=offsets)
+        return q.permute(0, 2, 1), s
     q, s = fp8_weight
     if (q.dtype != ops.FP8_DTYPE or tuple(q.shape) != tuple(weight.shape) or s.dtype != torch.float32
             or tuple(s.shape) != (weight.shape[0], weight.shape[2]) or q.device != weight.device):
@@ -162,7 +165,7 @@ def silu_jagged_bmm_fp8(
     require_hip_kernel(kernel, "silu_jagged_bmm_fp8")
     ops._forward_only("silu_jagged_bmm_fp8", jagged, weight, bias)
     qa, sa = ops.quant_rows_fp8(jagged, apply_silu=True)
-    qw, sw = _weight_pair(weight.permute(0, 2, 1), fp8_weight)          # rows of [E, D_out, D_in]
+    qw, sw = _weight_pair(weight.permute(0, 2, 1), fp8_weight, seq_offsets)     # rows of [E, D_out, D_in]
     return ops.grouped_gemm(seq_offsets, qa, qw, total_rows=jagged.shape[0], bias=bias,
                             scales_pow2=ops.scales_are_pow2(sa, sw), a_scale=sa, b_scale=sw, epilogue=EPI_NONE)
 
@@ -189,8 +192,9 @@ def silu_jagged_bmm_combine_fp8(
     require_hip_kernel(kernel, "silu_jagged_bmm_combine_fp8")
     L, K = reverse_index.shape
     assert index.shape[0] == L * K == jagged.shape[0]
-    qw, sw = _weight_pair(weight, fp8_weight)
-    if _ag.needs_grad(jagged, weight, bias, gating_scores):   # forward in e4m3, backward in bf16
+    grad = _ag.needs_grad(jagged, weight, bias, gating_scores)
+    qw, sw = _weight_pair(weight, fp8_weight, None if grad else offsets)
+    if grad:                                                  # forward in e4m3, backward in bf16
         return _ag.SiluJaggedBmmCombine.apply(offsets, jagged, weight, bias, index, reverse_index, gating_scores,
                                               gates_index, has_silu, (qw, sw), activation_checkpointing)
     qa, sa = ops.quant_rows_fp8(jagged, apply_silu=has_silu)
@@ -223,8 +227,9 @@ def index_select_jagged_bmm(
         return ops.grouped_gemm(offsets, jagged, weight, total_rows=index.numel(), row_index=index,
                                 index_div=index.shape[-1], bias=bias, epilogue=EPI_NONE)
     assert jagged.dtype == weight.dtype and (bias is None or jagged.dtype == bias.dtype)
-    qw, sw = _weight_pair(weight, fp8_weight)
-    if _ag.needs_grad(jagged, weight, bias):
+    grad = _ag.needs_grad(jagged, weight, bias)
+    qw, sw = _weight_pair(weight, fp8_weight, None if grad else offsets)
+    if grad:
         return _ag.IndexSelectJaggedBmmFp8.apply(offsets, index, jagged, weight, bias, (qw, sw))
     qa, sa = ops.quant_rows_fp8(jagged)
     return ops.grouped_gemm(offsets, qa, qw, total_rows=index.numel(), row_index=index,

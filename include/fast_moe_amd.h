@@ -181,6 +181,17 @@ int fmoe_quant_rows_e4m3_ws(const void* a, int a_dtype, int64_t batch, int64_t r
                             int64_t q_stride_c, float* scale, int store_reciprocal,
                             void* workspace, size_t workspace_bytes, fmoe_stream_t stream);
 
+/*
+ * The weights of one call's experts (no SiLU, the multiplier stored): as above with batch = the number of experts,
+ * but what belongs to an expert without rows (offsets[e + 1] <= offsets[e], offsets [batch + 1] in device memory) may
+ * be left unwritten: fmoe_grouped_gemm over the same offsets reads none of it.
+ */
+int fmoe_quant_expert_weights_e4m3(const void* a, int a_dtype, int64_t batch, int64_t rows, int64_t cols,
+                                   int64_t a_stride_b, int64_t a_stride_r, int64_t a_stride_c, uint8_t* q,
+                                   int64_t q_stride_b, int64_t q_stride_r, int64_t q_stride_c, float* scale,
+                                   const int64_t* offsets, void* workspace, size_t workspace_bytes,
+                                   fmoe_stream_t stream);
+
 /* -------------------------------------------------------------- grouped GEMM */
 
 /*

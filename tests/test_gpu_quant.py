@@ -302,3 +302,28 @@ def test_the_column_form_allocates_scratch_only_where_it_runs():
     assert allocations(lambda: moe_fp8.quantize_expert_weights(w)) == 3
     w = w[:, :128].contiguous()         # columns that fit a block's registers: one launch
     assert allocations(lambda: moe_fp8.quantize_expert_weights(w)) == 2
+
+
+@pytest.mark.parametrize("layout,n,k", [("nk", 24, 40), ("nk", 40, 1032), ("kn", 40, 64), ("kn", 24, 2052), ("kn", 16, 4104)])
+@pytest.mark.parametrize("counts", [(3, 0, 5, 0), (0, 0, 0, 9), (0, 0, 0, 0), (1, 1, 1, 1)])
+def test_weights_of_experts_with_rows_are_quantised_as_all_are(layout, n, k, counts):
+    """What fmoe_quant_expert_weights_e4m3 writes for an expert with rows is what the full quantisation writes, in every form of it
+    (rows in memory, columns in one launch, columns in two); the operators on it give the same bytes as on the full pair."""
+    from fast_moe_amd.kernels import moe_fp8
+    from fast_moe_amd.kernels.hip import ops
+    E, g = len(counts), torch.Generator(device="cuda").manual_seed(3)
+    w = torch.randn(E, n, k, generator=g, device="cuda").bfloat16()
+    w = w.permute(0, 2, 1) if layout == "nk" else w.permute(0, 2, 1).contiguous()          # [E, K, N]
+    offsets = torch.tensor([0, *counts], device="cuda").cumsum(0)
+    full_q, full_s = ops.quant_rows_fp8(w.permute(0, 2, 1))
+    q, s = ops.quant_rows_fp8(w.permute(0, 2, 1), offsets=offsets)
+    for e, c in enumerate(counts):
+        if c:
+            assert torch.equal(q[e].view(torch.uint8), full_q[e].view(torch.uint8)) and torch.equal(s[e], full_s[e])
+    R = sum(counts)
+    if R and k % 8 == 0:
+        x = torch.randn(R, k, generator=g, device="cuda").bfloat16()
+        index = torch.arange(R, device="cuda").view(R, 1)
+        pair = moe_fp8.quantize_expert_weights(w)
+        y = moe_fp8.index_select_jagged_bmm(0, offsets, index, x, w, None, fp8=True)
+        assert torch.equal(y, moe_fp8.index_select_jagged_bmm(0, offsets, index, x, w, None, fp8=True, fp8_weight=pair))
