@@ -236,14 +236,16 @@ inline int direct_columns(int n, bool swiglu) { return swiglu ? (n + 31) / 32 : 
 //   * fp32 streams half as much weight for a product and the other kernel is the slower one: up to 16 rows per expert whatever the tiles, from
 //     K = 1024 on, up to two per CU or up to four rows (512 rows, 128 experts, 4096 -> 2 x 1536 1384 / 1075, hot 571 / 530; 512 rows, 64 experts, 512
 //     -> 2048, not taken, level where one expert is hot), but not K of two slices (gemm_f32.hip).  With more rows the other kernel's tiles
-//     hold more of them: K from 1024 on and one tile per CU (320 rows, 8 experts, 1024 -> 512 40.0 / 17.6).  256 rows per expert and more below
-//     that K: 1000 rows, 8 experts, 256 -> 512 hot 12.6 / 16.5; more tiles: 4000 rows, 8 experts, 4096 -> 512, four per CU, 143 / 180.
+//     hold more of them: K from 1024 on and one tile per CU (320 rows, 8 experts, 1024 -> 512 40.0 / 17.6), K from 128 on in whole lines and one for two CUs (587 rows,
+//     16 experts, 960 -> 128 29.0 / 16.0; 644 rows, 4 experts, 128 -> 448 8.7 / 7.2; 306 rows, 8 experts, 640 -> 2 x 128 31.7 / 14.3: 26
+//     such calls, 1.13 to 2.2 times as fast; of K = 72 two, 1.11 to 1.21; the tests of the other kernel's edges have it at K in part).  Between them both ways: 164 tiles, 192 -> 256 10.7 / 14.6, 147 tiles, 960 -> 448 38.2 / 19.3; more tiles:
+//     4000 rows, 8 experts, 4096 -> 512, four per CU, 143 / 180.
 inline bool direct_pays(const GemmParams& p, int esize, bool swiglu) {
     const int64_t experts = p.E < p.total_rows ? p.E : p.total_rows, cus = compute_units();
     const int64_t tiles = most_row_tiles(p.total_rows, p.E, 64) * direct_columns(p.N, swiglu);
     const bool few = p.total_rows <= 16 * experts, tall = p.total_rows / p.E >= kTallRows;
     if (esize == 4) {
-        if (!few) return p.K >= 1024 && tiles <= cus;
+        if (!few) return p.K >= 1024 ? tiles <= cus : p.K >= 128 && p.K % 32 == 0 && tiles <= cus / 2;
         return p.K > 64 && (p.K >= 1024 || tiles <= 2 * cus || p.total_rows <= 4 * experts);
     }
     const int row = p.K * esize;

@@ -1368,6 +1368,7 @@ def test_streaming_kernel_recomputes_fp32_sums_that_are_not_finite():
     (4, 80, 256, 64, "bf16", False), (4, 80, 264, 64, "bf16", True), (4, 4096, 1024, 240, "bf16", True), (4, 4096, 1016, 240, "bf16", False),
     (4, 800, 1024, 2048, "bf16", True), (4, 800, 1024, 2056, "bf16", False), (4, 800, 2048, 2048, "fp8", True), (4, 800, 2048, 2064, "fp8", False),
     (4, 380, 1024, 2048, "bf16", False), (4, 300, 1024, 512, "f32", True), (4, 300, 1020, 512, "f32", False),
+    (4, 100, 992, 512, "f32", True), (8, 700, 128, 448, "f32", True), (8, 700, 128, 449, "f32", False), (8, 700, 96, 64, "f32", False),
     (16, 100, 1020, 2049, "f32", False), (16, 64, 1020, 2049, "f32", True), (16, 100, 1024, 2049, "f32", True), (16, 16, 64, 64, "f32", False),
     (8, 1, 4096, 1024, "bf16", True), (8, 2, 4096, 1024, "fp8", True), (8, 3, 4096, 1024, "f32", True), (1, 1, 128, 256, "bf16", True),
 ])
