@@ -249,14 +249,21 @@ static bool split_takes(const fmoe_gemm_desc* d, const GemmParams& p, int sel) {
            (p.K % pair == 0 ? p.K >= 4 * pair : !fp8 && ring_tail_takes(esize, p.K, p.E, p.total_rows)) && split_pays(p, esize, d->epilogue);
 }
 
+static size_t split_bytes(const fmoe_gemm_desc* d, const GemmParams& p, int sel) {
+    if (d->a_dtype == FMOE_F32) return p.direct ? 0 : gemm_f32_split_bytes(p, d->epilogue, d->a_silu != 0, sel);
+    return split_takes(d, p, sel) ? kSplitHeaderBytes + (size_t)split_blocks() * kSplitPieceBytes : 0;
+}
+
 extern "C" size_t fmoe_grouped_gemm_workspace_bytes(const fmoe_gemm_desc* d) {
     // asked before every call: those that are no tall ring's, and K of up to 15 pairs of slices, which split_pays never takes, end here
-    if (!d || d->a_dtype == FMOE_F32 || d->total_rows < kTallRows * (int64_t)d->num_experts || d->k <= (d->a_dtype == FMOE_E4M3 ? 1920 : 960))
+    // (fp32: up to 511, where a cut gains no 8 us either)
+    if (!d || (d->a_dtype != FMOE_F32 && d->total_rows < kTallRows * (int64_t)d->num_experts) ||
+        d->k <= (d->a_dtype == FMOE_E4M3 ? 1920 : d->a_dtype == FMOE_F32 ? 511 : 960))
         return 0;
     GemmParams p;
     int sel;
-    if (prepare_gemm(d, p, sel) || sel < 0 || !split_takes(d, p, sel)) return 0;
-    return kSplitHeaderBytes + (size_t)(compute_units() / kNumXcd * kNumXcd) * kSplitPieceBytes;
+    if (prepare_gemm(d, p, sel) || sel < 0) return 0;
+    return split_bytes(d, p, sel);
 }
 
 extern "C" int fmoe_grouped_gemm_ws(const fmoe_gemm_desc* d, void* workspace, size_t workspace_bytes, fmoe_stream_t stream_) {
@@ -265,9 +272,9 @@ extern "C" int fmoe_grouped_gemm_ws(const fmoe_gemm_desc* d, void* workspace, si
     int sel;
     if (int rc = prepare_gemm(d, p, sel)) return rc;
     if (sel < 0) return FMOE_OK;
-    if (workspace && aligned16(workspace) && split_takes(d, p, sel) &&
-        workspace_bytes >= kSplitHeaderBytes + (size_t)(compute_units() / kNumXcd * kNumXcd) * kSplitPieceBytes) {
+    if (const size_t need = workspace && aligned16(workspace) ? split_bytes(d, p, sel) : 0; need && workspace_bytes >= need) {
         p.split_ws = (SplitWorkspace*)workspace;
+        if (d->a_dtype == FMOE_F32) return run_gemm_f32(p, d->epilogue, d->a_silu != 0, sel, stream);
         return d->a_dtype == FMOE_E4M3 ? run_ring_split_fp8(p, d->epilogue, stream) : run_ring_split_bf16(p, d->epilogue, stream);
     }
     if (p.direct)

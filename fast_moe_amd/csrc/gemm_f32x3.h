@@ -34,6 +34,70 @@ struct TileF32x3 {
     static_assert((BM * 4) % NT == 0 && (BN * 4) % NT == 0, "loader passes must be whole");
 };
 
+// Last round cut along K, as the tall ring's (gemm_split.h): 128 x 128 tiles.  Two of them on a CU take 1.75 times as long as one, so a launch ends
+// with the CUs that have one tile more.  The tiles beyond whole rounds of one per CU go out as pieces of K behind them; each leaves its sums in the
+// workspace, f32x3_reduce_kernel adds them in the order of K.  us, whole tiles / cut: 8000 rows, 24 experts, 2048 -> 1024 353 / 280; 16000 rows, 20
+// experts, 1536 -> 1024 403 / 347; 9189 rows, 12 experts, 2600 -> 1000 429 / 345, 1000 -> 2600 396 / 370; 4096 rows, 8 experts, 1024 -> 4096 284 / 266; 2500
+// rows, 10 experts, 768 -> 3072 137 / 115; 4096 rows, 4 experts, 3072 -> 2048, hot 542 / 377; SwiGLU, 8192 rows, 8 experts, 2048 -> 2 x 2048 935 / 879.
+// (64 x 128 tiles, two or three to a CU, gained 0 to 5 % from the same and lost up to 7: not built.)  The error against 64 bits is no larger: fewer terms
+// meet in one chain of roundings.
+//
+// Pieces of each of `rest` tiles: two pairs of slices to a piece at least, and the shortest of this model in us / 9: a pair of slices takes 4 us of a
+// lone block, 1.75 times that with more pieces than CUs, a piece's 64 KB of sums 0.025 us of everybody's bandwidth, the second launch 6.
+// Integers: host and device agree.
+typedef TileF32x3<128, 128, 2, 2> TileF32Large;         // wave tile 64 x 64
+constexpr int kF32x3CutTile = 128 * 128, kF32x3PieceBytes = 128 * 128 * 4, kF32x3PairCost = 36;
+__host__ __device__ inline int f32x3_split_pieces(int rest, int pairs, int blocks, int* cost = nullptr) {
+    int best = 1, least = kF32x3PairCost * pairs;
+    for (int s = 2; s * rest <= 2 * blocks && 2 * s <= pairs; ++s) {
+        const int loop = (kF32x3PairCost * pairs + s - 1) / s;
+        const int c = (s * rest > blocks ? loop * 7 / 4 : loop) + rest * s * 2 / 9 + 54;
+        if (c < least) {
+            least = c;
+            best = s;
+        }
+    }
+    if (cost) *cost = least;
+    return best;
+}
+// a 32 x 32 block of a piece's sums, [quad][lane]
+template <typename TL>
+__device__ __forceinline__ f32x4* f32x3_sums(SplitWorkspace* ws, int piece, int row_block, int col_block) {
+    return reinterpret_cast<f32x4*>(reinterpret_cast<uint8_t*>(ws) + kSplitHeaderBytes + (int64_t)piece * kF32x3PieceBytes) +
+           (row_block * (TL::BN / 32) + col_block) * 4 * kWave;
+}
+
+// Wave: 32 x 32 outputs of a cut tile.
+template <typename TL, int EPI>
+__global__ __launch_bounds__(256) void f32x3_reduce_kernel(const GemmParams p) {
+    constexpr bool SWIGLU = EPI == FMOE_EPI_SWIGLU;
+    constexpr int PARTS = SWIGLU ? 2 : 1, COLS = TL::BN / 32 / PARTS, BLOCKS = TL::BM / 32 * COLS;
+    const int lane = threadIdx.x & 63, w = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = w / BLOCKS, rb = w % BLOCKS / COLS, cb = w % COLS;
+    const int tiles = p.split_ws->tiles, pieces = p.split_ws->pieces;
+    if (t >= tiles) return;
+    const SplitTile tile = p.split_ws->tile[t];
+    if (rb * 32 >= tile.rows_valid) return;
+    f32x16 acc[PARTS][1];
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][0][v] = 0.0f;
+#pragma unroll 4
+    for (int s = 0; s < pieces; ++s)
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i) {
+            const f32x4* const src = f32x3_sums<TL>(p.split_ws, s * tiles + t, rb, i * COLS + cb) + lane;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 v = src[g * kWave];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][0][4 * g + j] += v[j];
+            }
+        }
+    gemm_epilogue_f32<1, PARTS, 32, 32 * PARTS, EPI>(p, acc, tile.expert, tile.nt * (TL::BN / PARTS), tile.row0, tile.rows_valid, rb, cb, lane);
+}
+
 // Written out with packed operations on two values: 11 VALU instructions, which a block does once per operand value and slice.
 __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
     h = cvt_pk_bf16(a, b);
@@ -58,7 +122,7 @@ template <typename TL, int EPI, bool NCONT, bool A_SILU>
 __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const GemmParams p) {
     constexpr int BM = TL::BM, BN = TL::BN, NT = TL::NT, BK = TL::BK;
     constexpr int FM = TL::FM, FN = TL::FN, TM = TL::TM, TN = TL::TN;
-    constexpr bool SWIGLU = EPI == FMOE_EPI_SWIGLU;
+    constexpr bool SWIGLU = EPI == FMOE_EPI_SWIGLU, CUT = BM * BN == kF32x3CutTile;
     constexpr int BN_OUT = SWIGLU ? BN / 2 : BN;
     constexpr int XP = BM * 4 / NT, WP = BN * 4 / NT;       // units of 8 values a thread brings in per slice
     static_assert(EPI != FMOE_EPI_SWIGLU || FN % 2 == 0, "gate and up fragments come in pairs");
@@ -73,7 +137,24 @@ __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const Gem
     const int khalf = lane >> 5;
 
     BlockTile tile;
-    if (!tile.locate(p, BM)) return;
+    int piece = -1, first_slice = 0, slices = 0, cut_tiles = 1;
+    const int pairs = (p.K + 2 * BK - 1) / (2 * BK);
+    const bool here = CUT && p.split_ws ? tile.locate(p, BM, [&](int64_t total_tiles) -> int64_t {
+        const SplitDeal deal((int)total_tiles, p.split_slots, blockIdx.x % kNumXcd, pairs,
+                             [](int rest, int pairs, int blocks) { return f32x3_split_pieces(rest, pairs, blocks); });
+        if (blockIdx.x == 0 && tid == 0) {
+            p.split_ws->tiles = deal.pieces > 1 ? deal.rest : 0;
+            p.split_ws->pieces = deal.pieces;
+        }
+        const int j = blockIdx.x / kNumXcd;
+        if (j >= deal.count) return -1;
+        int part;
+        const int number = deal.tile(j, piece, part);
+        if (piece >= 0) deal.slices(part, pairs, first_slice, slices);
+        cut_tiles = deal.rest;
+        return number;
+    }) : tile.locate(p, BM);
+    if (!here) return;
     const int expert = __builtin_amdgcn_readfirstlane(tile.expert), nt = __builtin_amdgcn_readfirstlane(tile.nt);
     const int rows_valid = __builtin_amdgcn_readfirstlane(tile.rows_valid);
     const int64_t row0 = tile.row0;
@@ -85,6 +166,10 @@ __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const Gem
         k_begin = p.k_window[expert];
         const int64_t span = p.k_window[expert + 1] - k_begin;
         Kdim = (int)(span < 0 ? 0 : (span < p.K ? span : p.K));
+    }
+    if (CUT && piece >= 0) {
+        k_begin = first_slice * BK;
+        Kdim = p.K - (int)k_begin < slices * BK ? p.K - (int)k_begin : slices * BK;
     }
 
     const float* a_base = reinterpret_cast<const float*>(p.a) + (int64_t)expert * p.a_stride_e + k_begin;
@@ -286,6 +371,19 @@ __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const Gem
                         acc[fn][fm] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(wv[fn][j]), __uint_as_float(xv[fm][j]),
                                                                             acc[fn][fm], 0, 0, 0);
         }
+    }
+    if (CUT && piece >= 0) {
+        if (first_slice == 0 && tid == 0) p.split_ws->tile[piece % cut_tiles] = SplitTile{expert, nt, (int)row0, rows_valid};
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+            for (int fn = 0; fn < FN; ++fn) {
+                f32x4* const out = f32x3_sums<TL>(p.split_ws, piece, wm * FM + fm, frag_col(fn) / 32) + lane;
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    out[g * kWave] = f32x4{acc[fn][fm][4 * g], acc[fn][fm][4 * g + 1], acc[fn][fm][4 * g + 2], acc[fn][fm][4 * g + 3]};
+            }
+        return;
     }
     gemm_epilogue_f32<FM, FN, TM, TN, EPI>(p, acc, expert, n0, row0, rows_valid, wm, wn, lane);
 }

@@ -357,5 +357,8 @@ int dispatch_tile(const GemmParams& p, int sel, hipStream_t stream) {
 int run_gemm_bf16(GemmParams& p, int epilogue, bool a_silu, int sel, hipStream_t stream);
 int run_gemm_fp8(GemmParams& p, int epilogue, int sel, hipStream_t stream);
 int run_gemm_f32(GemmParams& p, int epilogue, bool a_silu, int sel, hipStream_t stream);
+// workspace of a prepared fp32 call whose last round is cut along K, 0: none is
+size_t gemm_f32_split_bytes(const GemmParams& p, int epilogue, bool a_silu, int sel);
+inline int split_blocks() { return compute_units() / kNumXcd * kNumXcd; }
 
 }  // namespace fmoe

@@ -59,7 +59,8 @@ struct GemmParams {
     int64_t out_half;
     const uint8_t* a2;                  // second product a2 * b2 summed into the same output, or null
     int k_split;                        // ... whose contraction covers k in [k_split, K)
-    SplitWorkspace* split_ws;           // ring with tiles cut along K: where their sums meet, or null
+    SplitWorkspace* split_ws;           // tiles cut along K: where their sums meet, or null
+    int split_slots;                    // fp32: blocks of a round, for one XCD
 #ifdef FMOE_TRACE
     uint64_t* trace;                    // debug builds: per-tile time stamps of the ring kernel
 #endif

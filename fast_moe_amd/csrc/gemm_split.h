@@ -46,12 +46,17 @@ struct SplitDeal {
     int whole, base, first, xcd;
 
     __host__ __device__ __forceinline__ SplitDeal() : count(0), rest(0), pieces(1), whole(0), base(0), first(0), xcd(0) {}
-    __host__ __device__ __forceinline__ SplitDeal(int total, int slots, int xcd_, int pairs) : xcd(xcd_) {
+    __host__ __device__ __forceinline__ SplitDeal(int total, int slots, int xcd_, int pairs)
+        : SplitDeal(total, slots, xcd_, pairs, [](int rest, int pairs, int blocks) {
+              return split_pieces(rest, pairs, blocks < kSplitMost ? blocks : kSplitMost);
+          }) {}
+    template <typename Pieces>
+    __host__ __device__ __forceinline__ SplitDeal(int total, int slots, int xcd_, int pairs, Pieces&& pieces_of) : xcd(xcd_) {
         const int blocks = 8 * slots, rounds = total / blocks;
         whole = rounds * slots;
         base = rounds * blocks;
         rest = total - base;
-        pieces = rest ? split_pieces(rest, pairs, blocks < kSplitMost ? blocks : kSplitMost) : 1;
+        pieces = rest ? pieces_of(rest, pairs, blocks) : 1;
         const int all = rest * pieces, share = (all + 7) / 8;
         first = xcd * share;
         const int left = all - first;

@@ -1,7 +1,7 @@
 // Register-staged grouped GEMM kernel: everything the ring and streaming kernels do not take.
 #pragma once
 
-#include "gemm_epilogue.h"
+#include "gemm_split.h"
 
 namespace fmoe {
 
@@ -31,6 +31,15 @@ struct BlockTile {
 
     // false: the launch has no tile for this block (the grid is an upper bound)
     __device__ __forceinline__ bool locate(const GemmParams& p, int BM) {
+        return locate(p, BM, [&](int64_t total_tiles) -> int64_t {
+            const int64_t per_xcd = (total_tiles + kNumXcd - 1) / kNumXcd, slot = blockIdx.x / kNumXcd;
+            const int64_t logical = (int64_t)(blockIdx.x % kNumXcd) * per_xcd + slot;
+            return slot < per_xcd && logical < total_tiles ? logical : -1;
+        });
+    }
+    // number_of: the block's tile among that many, or -1
+    template <typename Number>
+    __device__ __forceinline__ bool locate(const GemmParams& p, int BM, Number&& number_of) {
         const int lane = threadIdx.x & 63;
         const int64_t R = p.total_rows;
         int64_t total_m = 0;
@@ -45,7 +54,6 @@ struct BlockTile {
             total_m += wave_bcast(inc, kWave - 1);
         }
         const int64_t total_tiles = total_m * p.n_tiles;
-        const int64_t per_xcd = (total_tiles + kNumXcd - 1) / kNumXcd;
         const int64_t slot = blockIdx.x / kNumXcd;
         const int64_t group_span = (int64_t)kGroupM * p.n_tiles;
         int64_t group;
@@ -56,9 +64,8 @@ struct BlockTile {
             group = slot / group_span * kNumXcd + blockIdx.x % kNumXcd;
             within = (int)(slot % group_span);
         } else {
-            if (slot >= per_xcd) return false;
-            const int64_t logical = (int64_t)(blockIdx.x % kNumXcd) * per_xcd + slot;
-            if (logical >= total_tiles) return false;
+            const int64_t logical = number_of(total_tiles);
+            if (logical < 0) return false;
             group = logical / group_span;
             within = (int)(logical - group * group_span);
         }

@@ -1224,6 +1224,59 @@ def test_fp32_on_bf16_matrix_cores(E, rows, K, N, layout, epi, tile, case):
             assert bool(((got - want).abs() <= err).cpu()[near].all())
 
 
+@pytest.mark.parametrize("lens,K,N,layout,epi", [
+    ([2048] * 3 + [2049], 1024, 1024, "nk", 0),             # two whole rounds and eight tiles of a row
+    ([0, 4000, 2500, 2100, 3], 996, 1020, "kn", 1), ([4000, 2500, 2100, 130], 1028, 964, "nk", "silu"),
+    ([3000, 3500, 30], 772, 700, "nk", 2), ([3000, 3500, 30], 1024, 700, "kn", 2),
+    ([2100, 0, 500, 400, 33], 4100, 1000, "kn", 1), ([2100, 500, 400, 33], 4160, 904, "nk", "silu"),       # less than a round
+    ([500] * 66, 1024, 252, "nk", 0),                       # more than 64 experts
+])
+@pytest.mark.parametrize("case", ["normal", "special"])
+def test_fp32_last_round_cut_along_k(lens, K, N, layout, epi, case):
+    """Against float64, in the bound of test_fp32_on_bf16_matrix_cores (grouping the sums adds none to it); the same bits twice.  special: an
+    infinity, a NaN and a value beyond 2^104 in single rows; the other rows do not see them."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    E, rows = len(lens), sum(lens)
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    off = torch.tensor([0, *torch.tensor(lens).cumsum(0)]).cuda()
+    a_silu, epi = epi == "silu", 0 if epi == "silu" else epi
+    x = torch.randn((rows + 1) // 2, K, generator=g, device="cuda")
+    index = torch.arange(rows, device="cuda")
+    bias = [torch.randn(E, N, generator=g, device="cuda") for _ in range(2)]
+    ws = [torch.randn(*((E, K, N) if layout == "kn" else (E, N, K)), generator=g, device="cuda") * K ** -0.5 for _ in range(2)]
+    odd = torch.zeros(rows, dtype=torch.bool, device="cuda")
+    if case == "special":
+        x[2, K - 1], x[x.shape[0] - 1, 0], x[x.shape[0] // 2, K // 2] = float("inf"), float("nan"), 3e38
+        for r in (2, x.shape[0] - 1, x.shape[0] // 2):
+            odd[2 * r:2 * r + 2] = True
+    ws = [w if layout == "kn" else w.permute(0, 2, 1) for w in ws]
+    swiglu = epi == _lib.EPI_SWIGLU
+    kw = dict(total_rows=rows, row_index=index, index_div=2, bias=bias[0], epilogue=epi, a_silu=a_silu)
+    if swiglu:
+        kw.update(b2=ws[1], bias2=bias[1])
+    ran = kernels_run(lambda: ops.grouped_gemm(off, x, ws[0], **kw))
+    out = ops.grouped_gemm(off, x, ws[0], **kw)
+    again = ops.grouped_gemm(off, x, ws[0], **kw)
+    assert torch.equal(out.nan_to_num(7.0), again.nan_to_num(7.0))
+    assert [n.split("<")[0].split("::")[-1] for n in ran] == ["grouped_gemm_f32x3_kernel", "f32x3_reduce_kernel"], ran
+    assert "TileF32x3<128, 128" in ran[0], ran
+    unit = (K + 4) * 2.0 ** -24 + (2.0 ** -21 if a_silu else 0)         # (a rounding for the bias)
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        a = x[index[lo:hi] // 2].double()
+        a = torch.nn.functional.silu(a) if a_silu else a
+        want, err = a @ ws[0][e].double() + bias[0][e].double(), unit * (a.abs() @ ws[0][e].double().abs() + bias[0][e].double().abs())
+        if epi != _lib.EPI_NONE:
+            want, err = torch.nn.functional.silu(want), 1.1 * err + 2.0 ** -21 * want.abs()
+        if swiglu:
+            up, up_err = a @ ws[1][e].double() + bias[1][e].double(), unit * (a.abs() @ ws[1][e].double().abs() + bias[1][e].double().abs())
+            want, err = want * up, err * up.abs() + (want.abs() + err) * up_err + 2.0 ** -23 * (want * up).abs()
+        plain = ~odd[lo:hi]
+        assert bool(((out[lo:hi].double() - want).abs() <= err)[plain].all()), f"expert {e}"
+        if case == "special" and epi == _lib.EPI_NONE and not a_silu:
+            assert bool((~out[lo:hi][~plain].isfinite() | (want[~plain].abs() < 3.5e38)).all())
+
+
 @pytest.mark.parametrize("E,rows,K,N,layout", [(3, 700, 256, 1156, "nk"), (3, 700, 256, 1156, "kn"), (3, 190, 200, 60, "nk"), (3, 4800, 256, 1156, "kn"),
                                                (4, 40, 1024, 264, "nk"), (8, 200, 1024, 132, "nk")])
 @pytest.mark.parametrize("nonzero", [1, 2, 5, 16])

@@ -1,25 +1,28 @@
 """The tall ring's last round cut along K (csrc/gemm_split.h), walked on the host: every tile once, whole or as parts that cover every
-pair of its K-slices once, no more pieces than blocks and none of fewer than two pairs; no block has work behind a piece."""
+pair of its K-slices once, no more pieces than blocks and none of fewer than two pairs; no block has work behind a piece.
+And the fp32 kernel's (csrc/gemm_f32x3.h), a block of which takes one tile or piece: up to two pieces to a CU."""
 import os
 import subprocess
 
 PROGRAM = r"""
 #include <cstdio>
 #include <vector>
-#include "gemm_split.h"
+#include "gemm_f32x3.h"
 
-int check(int total, int slots, int pairs) {
+int check(int total, int slots, int pairs, bool f32) {
     std::vector<std::vector<int>> seen(total, std::vector<int>(pairs, 0));
-    std::vector<int> pieces_seen(fmoe::kSplitMost, 0);
+    std::vector<int> pieces_seen(2 * fmoe::kSplitMost, 0);
     for (int xcd = 0; xcd < 8; ++xcd) {
-        const fmoe::SplitDeal d(total, slots, xcd, pairs);
+        const fmoe::SplitDeal d = f32 ? fmoe::SplitDeal(total, slots, xcd, pairs, [](int r, int p, int b) { return fmoe::f32x3_split_pieces(r, p, b); })
+                                      : fmoe::SplitDeal(total, slots, xcd, pairs);
+        if (f32 && d.count > (total / (8 * slots) + 2) * slots) return printf("%d blocks of an XCD\n", d.count), 1;   // the launch's grid
         for (int j = 0; j < d.count; ++j) {
             int piece, part, first = 0, number = 2 * pairs;
             const int t = d.tile(j, piece, part);
             if (t < 0 || t >= total) return printf("tile %d of %d\n", t, total), 1;
             if (piece >= 0) {
-                if (piece >= fmoe::kSplitMost || pieces_seen[piece]++) return printf("piece %d\n", piece), 1;
-                if (j + slots < d.count) return printf("work behind a piece\n"), 1;
+                if (piece >= (f32 ? 16 * slots : fmoe::kSplitMost) || pieces_seen[piece]++) return printf("piece %d\n", piece), 1;
+                if (!f32 && j + slots < d.count) return printf("work behind a piece\n"), 1;
                 if (piece % d.rest != t - d.base || piece / d.rest != part) return printf("piece %d is not part %d of %d\n", piece, part, t), 1;
                 d.slices(part, pairs, first, number);
                 if (number < 4) return printf("%d slices\n", number), 1;
@@ -38,7 +41,7 @@ int main() {
     for (int slots : {32, 31, 4, 1})
         for (int pairs : {4, 5, 16, 61, 64, 200})
             for (int total = 0; total <= 40 * slots; total += total < 300 ? 1 : 37)
-                if (check(total, slots, pairs)) return printf("total %d, slots %d, pairs %d\n", total, slots, pairs), 1;
+                if (check(total, slots, pairs, false) || check(total, slots, pairs, true)) return printf("total %d, slots %d, pairs %d\n", total, slots, pairs), 1;
     return 0;
 }
 """
