@@ -93,6 +93,25 @@ __device__ __forceinline__ void silu_round_bf16_pair(float& a, float& b) {
     a = ya;
     b = yb;
 }
+// The same for a 16-byte chunk of eight values, with one look for the low end: a branch behind every pair leaves its chain of v_exp_f32 and
+// v_rcp_f32 nothing to overlap with.
+__device__ __forceinline__ u32x4 silu_round_bf16_x8(u32x4 v) {
+    constexpr float kLog2e = 1.44269504088896341f, kOnePlus = 1.00000012f;
+    float x[8], y[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        x[j] = j & 1 ? __uint_as_float(v[j / 2] & 0xffff0000u) : __uint_as_float(v[j / 2] << 16);
+        y[j] = x[j] * __builtin_amdgcn_rcpf(kOnePlus + __builtin_amdgcn_exp2f(x[j] * -kLog2e));
+    }
+    if (fminf(fminf(fminf(x[0], x[1]), fminf(x[2], x[3])), fminf(fminf(x[4], x[5]), fminf(x[6], x[7]))) < -87.0f) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float scaled = x[j] * __builtin_amdgcn_exp2f(__builtin_fmaf(x[j], kLog2e, 32.0f));
+            y[j] = x[j] < -87.0f && x[j] > -88.7f ? scaled * 0x1p-32f : y[j];
+        }
+    }
+    return u32x4{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3]), cvt_pk_bf16(y[4], y[5]), cvt_pk_bf16(y[6], y[7])};
+}
 __device__ __forceinline__ float silu_round_bf16(float x) {
     float other = 0.0f;
     silu_round_bf16_pair(x, other);

@@ -33,12 +33,12 @@ __global__ __launch_bounds__(256) void silu_mul_bf16_kernel(const uint16_t* __re
         const u32x4 va = *reinterpret_cast<const u32x4*>(a + i0);
         const u32x4 vb = GATED ? *reinterpret_cast<const u32x4*>(b + i0) : u32x4{0, 0, 0, 0};
         u32x4 vo;
+        vo = silu_round_bf16_x8(va);
+        if constexpr (GATED) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float x0 = bf16_bits_to_f32(va[j] & 0xffffu), x1 = __uint_as_float(va[j] & 0xffff0000u);
-            silu_round_bf16_pair(x0, x1);
-            vo[j] = GATED ? cvt_pk_bf16(x0 * bf16_bits_to_f32(vb[j] & 0xffffu), x1 * __uint_as_float(vb[j] & 0xffff0000u))
-                          : cvt_pk_bf16(x0, x1);
+            for (int j = 0; j < 4; ++j)
+                vo[j] = cvt_pk_bf16(bf16_bits_to_f32(vo[j] & 0xffffu) * bf16_bits_to_f32(vb[j] & 0xffffu),
+                                    __uint_as_float(vo[j] & 0xffff0000u) * __uint_as_float(vb[j] & 0xffff0000u));
         }
         *reinterpret_cast<u32x4*>(out + i0) = vo;
     } else {

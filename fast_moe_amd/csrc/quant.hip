@@ -87,6 +87,8 @@ __device__ __forceinline__ u32x2 encode8(const u32x4& v, float s, bool special) 
 // 4096 x 1024 weights 21.9 -> 22.0 us; 54 experts, 576 x 3776, two of them with a row 66 -> 6.)
 __device__ __forceinline__ bool idle_expert(const int64_t* offsets, int64_t e) { return offsets && offsets[e + 1] <= offsets[e]; }
 
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
+
 // ---- fast path: bf16, contiguous columns, cols % 8 == 0, <= CH*512 columns
 // W16: a lane takes pairs of neighbouring 16-byte chunks (32 contiguous input bytes), so that its
 // eight-byte results pair up into one 16-byte store (rows of a whole number of such pairs)
@@ -96,9 +98,9 @@ __global__ __launch_bounds__(256) void quant_rows_bf16_wave(
     int64_t a_sr, uint8_t* __restrict__ q, int64_t q_sb, int64_t q_sr, float* __restrict__ scale,
     int store_reciprocal, const int64_t* __restrict__ offsets) {
     const int lane = lane_id();
-    const int64_t row = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
+    const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (row >= total_rows) return;
-    const int64_t b = row / rows, r = row - b * rows;
+    const int64_t b = rows == total_rows ? 0 : row / rows, r = row - b * rows;      // (scalar: the loads wait for it)
     if (idle_expert(offsets, b)) return;
     const uint16_t* src = a + b * a_sb + r * a_sr;
     uint8_t* dst = q + b * q_sb + r * q_sr;
@@ -113,23 +115,17 @@ __global__ __launch_bounds__(256) void quant_rows_bf16_wave(
         const int c = chunk_of(i);
         v[i] = c < chunks ? *reinterpret_cast<const u32x4*>(src + (int64_t)c * 8) : u32x4{0, 0, 0, 0};
     }
-    float m = 0.0f;
-    bool nan = false;
+    u16x2 most = {0, 0};                            // |value| bits of the low and the high halves: they compare as integers, NaN above inf
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
+        if (SILU) v[i] = silu_round_bf16_x8(v[i]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float lo = bf16_bits_to_f32(v[i][j] & 0xffffu);
-            float hi = __uint_as_float(v[i][j] & 0xffff0000u);
-            if (SILU) {
-                silu_round_bf16_pair(lo, hi);
-                v[i][j] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
-            }
-            m = amax_update(m, lo, nan);
-            m = amax_update(m, hi, nan);
-        }
+        for (int j = 0; j < 4; ++j) most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, v[i][j] & 0x7fff7fffu));
     }
-    m = finish_amax(m, nan);
+    uint32_t bits = max((uint32_t)most[0], (uint32_t)most[1]);
+#pragma unroll
+    for (int o = kWave / 2; o >= 1; o >>= 1) bits = max(bits, (uint32_t)__shfl_xor((int)bits, o, kWave));
+    const float m = bf16_bits_to_f32(bits);
     const float s = scale_from_amax<true>(m);   // every element is a bf16 value
     if (lane == 0) scale[row] = store_reciprocal ? 1.0f / s : s;
     const bool special = !(m <= 3.4028234664e38f);   // NaN or inf in the row
@@ -168,14 +164,7 @@ __global__ __launch_bounds__(256) void quant_rows_bf16_block(
     const int64_t chunks = cols >> 3;
     auto load = [&](int64_t c) {
         u32x4 v = *reinterpret_cast<const u32x4*>(src + c * 8);
-        if (SILU) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float lo = bf16_bits_to_f32(v[j] & 0xffffu), hi = __uint_as_float(v[j] & 0xffff0000u);
-                silu_round_bf16_pair(lo, hi);
-                v[j] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
-            }
-        }
+        if (SILU) v = silu_round_bf16_x8(v);
         return v;
     };
     float m = 0.0f;
