@@ -5,115 +5,35 @@
 // 61 us, bound by the host).  Logits are fp32 sums plus bias rounded to the scores' type, as torch.nn.functional.linear rounds
 // them, and the softmax is torch's, step by step (one wave per token, expert e in lane e % 64, butterfly sums from the
 // widest distance down).
-#include "common.h"
+#include "gate.h"
 
 namespace fmoe {
 namespace {
 
-constexpr int kGateWaves = 8, kGateTokens = 16, kGateMostExperts = 96;
-
-// Block: 16 tokens x all experts on 16 x 16 MFMAs, weights from the A port.  The waves share K in pieces of 64 bytes per row (a lane's
-// 16 bytes of row lane % 16 at 16 * (lane / 16); the order of k inside a piece is the same on both sides, so it is free) and
-// their sums are added in LDS in wave order.  What bounds it is the chain of loads: 2048 inputs, 64 experts 7 us.
+// Block: 16 tokens x all experts on 16 x 16 MFMAs, weights from the A port, the eight waves' sums added in LDS in wave order.  What bounds it is the
+// chain of loads: 2048 inputs, 64 experts 7 us.
 template <bool F32, int NF>
 __global__ __launch_bounds__(kGateWaves* kWave) void gate_softmax_kernel(const uint8_t* __restrict__ x, int64_t T, int D, int64_t x_stride,
                                                                        const uint8_t* __restrict__ w, const void* __restrict__ bias,
                                                                        int E, void* __restrict__ scores) {
-    constexpr int ESIZE = F32 ? 4 : 2, LD = NF * 16 + 4;
-    extern __shared__ float red[];              // [wave][token][LD]
-    const int lane = lane_id(), wave = threadIdx.x / kWave, r16 = lane & 15, quarter = lane >> 4;
+    extern __shared__ float red[];
+    const int wave = threadIdx.x / kWave;
     const int64_t t0 = (int64_t)blockIdx.x * kGateTokens;
-    const int kbytes = D * ESIZE, pieces = (kbytes + 63) / 64;
-    const int64_t token = t0 + r16 < T ? t0 + r16 : T - 1;
-    const uint8_t* const xrow = x + token * x_stride * ESIZE + 16 * quarter;
-    const uint8_t* wrow[NF];
-#pragma unroll
-    for (int f = 0; f < NF; ++f) wrow[f] = w + (int64_t)(16 * f + r16 < E ? 16 * f + r16 : E - 1) * kbytes + 16 * quarter;
-    f32x4 acc[NF];
-#pragma unroll
-    for (int f = 0; f < NF; ++f) acc[f] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    constexpr int AHEAD = NF <= 2 ? 4 : 2;      // pieces on their way
-    u32x4 xv[AHEAD], wv[AHEAD][NF];
-    auto load = [&](int c, int i) {
-        const bool in = c * 64 + 16 * quarter < kbytes;         // (rows are whole 16-byte chunks)
-        const u32x4 zero = {0, 0, 0, 0};
-        xv[i] = in ? *reinterpret_cast<const u32x4*>(xrow + c * 64) : zero;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) wv[i][f] = in ? *reinterpret_cast<const u32x4*>(wrow[f] + c * 64) : zero;
-    };
-#pragma unroll
-    for (int i = 0; i < AHEAD; ++i) load(wave + i * kGateWaves, i);
-    for (int c0 = wave; c0 < pieces; c0 += AHEAD * kGateWaves) {
-#pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
-            const int c = c0 + i * kGateWaves;
-            if (c >= pieces) break;
-#pragma unroll
-            for (int f = 0; f < NF; ++f) {
-                if constexpr (F32) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(wv[i][f][j]), __uint_as_float(xv[i][j]), acc[f], 0, 0, 0);
-                } else {
-                    acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[i][f]), __builtin_bit_cast(bf16x8, xv[i]),
-                                                                     acc[f], 0, 0, 0);
-                }
-            }
-            load(c + AHEAD * kGateWaves, i);
-        }
-    }
-    // lane l: experts 16 * f + 4 * (l / 16) .. + 3 of token l % 16
-#pragma unroll
-    for (int f = 0; f < NF; ++f)
-        *reinterpret_cast<f32x4*>(red + (wave * kGateTokens + r16) * LD + 16 * f + 4 * quarter) = acc[f];
+    gate_sums<F32, NF>(x, T, D, x_stride, w, E, t0, wave, red);
     __syncthreads();
-    constexpr int PER = (NF * 16 + kWave - 1) / kWave;          // experts of a lane
-    for (int t = wave; t < kGateTokens; t += kGateWaves) {
-        if (t0 + t >= T) break;
-        float v[PER], most = -__builtin_inff();
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int e = i * kWave + lane;
-            v[i] = -__builtin_inff();
-            if (e < E) {
-                float s = red[t * LD + e];
-#pragma unroll
-                for (int j = 1; j < kGateWaves; ++j) s += red[(j * kGateTokens + t) * LD + e];
-                if (bias) s += F32 ? reinterpret_cast<const float*>(bias)[e] : bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(bias)[e]);
-                v[i] = F32 ? s : round_bf16(s);
-            }
-            most = most > v[i] ? most : v[i];
-        }
-#pragma unroll
-        for (int o = kWave / 2; o >= 1; o >>= 1) {
-            const float other = __shfl_xor(most, o, kWave);
-            most = most < other ? other : most;
-        }
-        float sum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            v[i] = i * kWave + lane < E ? expf(v[i] - most) : 0.0f;
-            sum += v[i];
-        }
-#pragma unroll
-        for (int o = kWave / 2; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, kWave);
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int e = i * kWave + lane;
-            if (e >= E) continue;
-            const float p = v[i] / sum;
+    const int tokens = T - t0 < kGateTokens ? (int)(T - t0) : kGateTokens;
+    constexpr int STEP = gate_wave_tokens(NF);
+    for (int first = wave * STEP; first < tokens; first += kGateWaves * STEP)
+        gate_softmax_tokens<F32, NF>(red, first, tokens, bias, E, [&](int t, int e, float p) {
             if constexpr (F32) reinterpret_cast<float*>(scores)[(t0 + t) * E + e] = p;
             else reinterpret_cast<uint16_t*>(scores)[(t0 + t) * E + e] = (uint16_t)f32_to_bf16_bits(p);
-        }
-    }
+        });
 }
 
 }  // namespace
 }  // namespace fmoe
 
 using namespace fmoe;
-
-static int gate_fragments(int E) { return E <= 16 ? 1 : E <= 32 ? 2 : E <= 64 ? 4 : 6; }
 
 // Batches whose pass is bound by the host (a library GEMM and a softmax take 26 us to issue, this 7) or by its chain of launches; a larger one has
 // the library GEMM's rate to lose.  A block's eight waves walk all of K, 3 us and 0.25 for every KB of a gate row times 1 + 2 * fragments, where the
@@ -139,7 +59,7 @@ extern "C" int fmoe_gate_softmax(const void* x, int dtype, int64_t T, int D, int
                      aligned16(weight) && T < ((int64_t)1 << 31),
                  "fmoe_gate_softmax: up to %d experts, rows of whole 16-byte chunks at 16-byte boundaries", kGateMostExperts);
     auto go = [&](auto kern, int nf) {
-        const size_t lds = (size_t)kGateWaves * kGateTokens * (nf * 16 + 4) * sizeof(float);
+        const size_t lds = (size_t)gate_sums_floats(nf) * sizeof(float);
         kern<<<(unsigned)((T + kGateTokens - 1) / kGateTokens), kGateWaves * kWave, lds, (hipStream_t)stream_>>>(
             (const uint8_t*)x, T, D, x_stride_row, (const uint8_t*)weight, bias, E, scores);
         return check_launch("fmoe_gate_softmax");

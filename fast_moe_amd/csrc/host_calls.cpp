@@ -34,6 +34,8 @@ decltype(&fmoe_combine) c_combine;
 decltype(&fmoe_quant_rows_e4m3) c_quant_rows;
 decltype(&fmoe_gate_softmax) c_gate_softmax;
 decltype(&fmoe_gate_softmax_pays) gate_softmax_pays;
+decltype(&fmoe_gate_route_pays) gate_route_pays;
+decltype(&fmoe_gate_route) c_gate_route;
 decltype(&fmoe_grouped_gemm_plan) c_gemm_plan;
 decltype(&fmoe_combine_bwd) c_combine_bwd;
 decltype(&fmoe_segment_colsum) c_segment_colsum;
@@ -399,6 +401,23 @@ PyObject* py_quant_rows(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// What the launches that stand for the gate take: one type, rows of x and the weight at 16-byte boundaries.
+bool gate_ok(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, const void** x_data, const void** w_data, const void** b_data) {
+    const int code = dtype_code(x.scalar_type());
+    if ((code != FMOE_F32 && code != FMOE_BF16) || w.scalar_type() != x.scalar_type() || x.dim() != 2 || w.dim() != 2 ||
+        x.size(1) != w.size(1) || x.stride(1) != 1 || !w.is_contiguous() || !same_device(x, w) || !same_device(x, bias) ||
+        w.size(0) > INT32_MAX || w.size(1) > INT32_MAX)
+        return false;
+    if (bias.defined() && (bias.scalar_type() != x.scalar_type() || !bias.is_contiguous() || bias.numel() != w.size(0))) return false;
+    if (!gate_softmax_pays(code, x.size(0), (int)x.size(1), (int)w.size(0)) || x.stride(0) < x.size(1) ||
+        x.stride(0) % (code == FMOE_F32 ? 4 : 8))
+        return false;
+    *x_data = x.data_ptr();
+    *w_data = w.data_ptr();
+    *b_data = bias.defined() ? bias.data_ptr() : nullptr;
+    return (uintptr_t)*x_data % 16 == 0 && (uintptr_t)*w_data % 16 == 0;
+}
+
 // (x [T, D], weight [E, D], bias [E] or None, stream) -> softmax(x weight^T + bias) [T, E], where fmoe_gate_softmax is the faster form
 PyObject* py_gate_softmax(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -409,22 +428,7 @@ PyObject* py_gate_softmax(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!x.defined() || !w.defined() || !optional_tensor(args[2], &bias) || !as_int(args[3], &stream)) return none();
     const void *x_data, *w_data, *b_data = nullptr;
     const int status = run(
-        [&] {
-            const int code = dtype_code(x.scalar_type());
-            if ((code != FMOE_F32 && code != FMOE_BF16) || w.scalar_type() != x.scalar_type() || x.dim() != 2 || w.dim() != 2 ||
-                x.size(1) != w.size(1) || x.stride(1) != 1 || !w.is_contiguous() || !same_device(x, w) || !same_device(x, bias) ||
-                w.size(0) > INT32_MAX || w.size(1) > INT32_MAX)
-                return false;
-            if (bias.defined() && (bias.scalar_type() != x.scalar_type() || !bias.is_contiguous() || bias.numel() != w.size(0))) return false;
-            if (!gate_softmax_pays(code, x.size(0), (int)x.size(1), (int)w.size(0)) || x.stride(0) < x.size(1) ||
-                x.stride(0) % (code == FMOE_F32 ? 4 : 8))
-                return false;
-            x_data = x.data_ptr();
-            w_data = w.data_ptr();
-            if ((uintptr_t)x_data % 16 || (uintptr_t)w_data % 16) return false;
-            if (bias.defined()) b_data = bias.data_ptr();
-            return true;
-        },
+        [&] { return gate_ok(x, w, bias, &x_data, &w_data, &b_data); },
         [&] {
             scores = empty({x.size(0), w.size(0)}, x.scalar_type(), x);
             return c_gate_softmax(x_data, dtype_code(x.scalar_type()), x.size(0), (int)x.size(1), x.stride(0), w_data, b_data, (int)w.size(0),
@@ -436,11 +440,16 @@ PyObject* py_gate_softmax(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // (scores [T, E], x [T, D], w1 [E, D, H], bias1, w2 [E, H, O], bias2, k, mode, epilogue1, stream) -> [T, O]:
-// routing, the gather GEMM with its activation, the second GEMM, the merge
+// routing, the gather GEMM with its activation, the second GEMM, the merge.  With scores None, a gate's weight [E, D] and its bias [E] or None
+// behind the stream: where the gate and the routing are one launch (fmoe_gate_route_pays)
 PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 10) return none();
-    const at::Tensor scores = gpu_tensor(args[0]), x = gpu_tensor(args[1]), w1 = gpu_tensor(args[2]);
+    if (n != 10 && n != 12) return none();
+    const bool gate = n == 12;
+    const at::Tensor scores = gate ? gpu_tensor(args[10]) : gpu_tensor(args[0]);        // (gate: [E, D] in its place)
+    const at::Tensor x = gpu_tensor(args[1]), w1 = gpu_tensor(args[2]);
+    at::Tensor gate_bias;
+    if (gate && (args[0] != Py_None || !optional_tensor(args[11], &gate_bias))) return none();
     const at::Tensor b1 = gpu_tensor(args[3]), w2 = gpu_tensor(args[4]), b2 = gpu_tensor(args[5]);
     int64_t k, mode, epilogue, stream;
     for (const at::Tensor* t : {&scores, &x, &w1, &b1, &w2, &b2})
@@ -448,7 +457,7 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!as_int(args[6], &k) || !as_int(args[7], &mode) || !as_int(args[8], &epilogue) || !as_int(args[9], &stream))
         return none();
     at::Tensor scratch, y;
-    const void* data;
+    const void *data = nullptr, *x_data = nullptr, *gate_bias_data = nullptr;
     char* base = nullptr;
     size_t at_ws = 0, ws_bytes = 0;
     int64_t *topk_idx = nullptr, *lengths = nullptr, *offsets = nullptr, *gate_index = nullptr, *token_index = nullptr, *reverse = nullptr;
@@ -460,12 +469,20 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     // is declined has routed nothing.  One allocation holds the intermediates (twelve were 10 of the 30 us that the call took).
     const int status = run(
         [&] {
-            if (x.dim() != 2 || scores.dim() != 2 || scores.size(0) != x.size(0) || w1.dim() != 3 || w2.dim() != 3 ||
-                w1.size(0) != scores.size(1) || w2.size(0) != scores.size(1) || w2.size(1) != w1.size(2) ||
+            if (x.dim() != 2 || scores.dim() != 2 || w1.dim() != 3 || w2.dim() != 3 || w2.size(1) != w1.size(2) ||
                 w2.scalar_type() != w1.scalar_type() || scores.device() != x.device() || w1.device() != x.device() ||
-                w2.device() != x.device() || !route_ok(scores, k, &data))
+                w2.device() != x.device())
                 return false;
-            const int64_t T = x.size(0), E = scores.size(1), H = w1.size(2), O = w2.size(2), R = T * k;
+            const int64_t T = x.size(0), E = scores.size(gate ? 0 : 1);
+            if (w1.size(0) != E || w2.size(0) != E) return false;
+            if (gate) {
+                if (!gate_ok(x, scores, gate_bias, &x_data, &data, &gate_bias_data) || k < 1 || k > E ||
+                    !gate_route_pays(dtype_code(x.scalar_type()), T, (int)x.size(1), (int)E, (int)k))
+                    return false;
+            } else if (scores.size(0) != T || !route_ok(scores, k, &data)) {
+                return false;
+            }
+            const int64_t H = w1.size(2), O = w2.size(2), R = T * k;
             const int64_t row_size = w1.scalar_type() == at::kFloat ? 4 : 2;
             size_t bytes = 0;
             auto take = [&](int64_t n, int64_t size) {
@@ -473,7 +490,7 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 bytes += ((size_t)(n * size) + 255) & ~(size_t)255;
                 return at;
             };
-            ws_bytes = route_workspace_bytes(T, (int)E, (int)k);
+            ws_bytes = gate ? 0 : route_workspace_bytes(T, (int)E, (int)k);
             const size_t at_topk = take(R, 8), at_lengths = take(E, 8), at_offsets = take(E + 1, 8), at_gate = take(R, 8);
             const size_t at_token = take(R, 8), at_reverse = take(R, 8), at_gates = take(R, (int64_t)scores.element_size());
             at_ws = take((int64_t)ws_bytes, 1);
@@ -523,9 +540,17 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
             return true;
         },
         [&] {
-            if (const int rc = c_route_topk(data, dtype_code(scores.scalar_type()), merge.T, (int)scores.size(1), (int)k, (int)mode, topk_idx,
-                                            gates, lengths, offsets, gate_index, token_index, reverse, base + at_ws, ws_bytes, (void*)stream))
+            if (gate) {
+                what = "fmoe_gate_route";
+                if (const int rc = c_gate_route(x_data, dtype_code(x.scalar_type()), merge.T, (int)x.size(1), x.stride(0), data, gate_bias_data,
+                                                (int)scores.size(0), (int)k, (int)mode, topk_idx, gates, lengths, offsets, gate_index,
+                                                token_index, reverse, (void*)stream))
+                    return rc;
+            } else if (const int rc = c_route_topk(data, dtype_code(scores.scalar_type()), merge.T, (int)scores.size(1), (int)k, (int)mode,
+                                                   topk_idx, gates, lengths, offsets, gate_index, token_index, reverse, base + at_ws,
+                                                   ws_bytes, (void*)stream)) {
                 return rc;
+            }
             RECORD_USER_SCOPE("## expert_forward##");
             what = "fmoe_grouped_gemm";
             if (const int rc = gemm(up, x, (void*)stream)) return rc;
@@ -761,7 +786,8 @@ PyObject* py_weight_grad(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void* const entry[] = {&route_workspace_bytes, &c_route_topk, &c_grouped_gemm, &c_combine, &c_quant_rows, &c_gate_softmax, &gemm_workspace_bytes,
                            &c_grouped_gemm_ws, &c_gemm_plan, &c_combine_bwd, &c_segment_colsum, &c_swiglu_bwd, &c_silu_mul, &c_gather_rows,
-                           &c_invert_index, &c_gate_l1_bwd, &c_weight_grad, &weight_grad_pays, &gate_softmax_pays, &last_error};
+                           &c_invert_index, &c_gate_l1_bwd, &c_weight_grad, &weight_grad_pays, &gate_softmax_pays,
+                           &gate_route_pays, &c_gate_route, &last_error};
     constexpr Py_ssize_t count = sizeof(entry) / sizeof(entry[0]);
     if (n != count) {
         PyErr_Format(PyExc_TypeError, "init: %d addresses expected", (int)count);

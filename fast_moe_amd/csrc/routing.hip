@@ -15,7 +15,7 @@
 //      chunks: lengths; wave scan over the experts: offsets), every wave adds the counts of
 //      the waves before it in its chunk and then places its positions: a wave-level
 //      match/rank gives each position its slot inside its expert segment
-#include "common.h"
+#include "gate.h"
 
 #include <mutex>
 
@@ -500,19 +500,15 @@ __global__ __launch_bounds__(1024) void scan_scatter_kernel(const uint16_t* __re
 }
 
 // Both launches in one block of 16 waves for a batch of few tokens (route_one_block): the counts and the expert ids stay in LDS, and
-// one barrier on either side of the prefix sums takes the place of the second launch.
+// one barrier on either side of the prefix sums takes the place of the second launch.  scores: global memory or LDS.
 template <typename T, int LPT, int VPL>
-__global__ __launch_bounds__(kMaxRouteWaves* kWave) void route_block_kernel(const T* __restrict__ scores, int num_tokens, int E, int K,
-                                                                    int ebits, int renorm, int tokens_per_wave,
-                                                                    int64_t* __restrict__ topk_idx, T* __restrict__ gates,
-                                                                    int64_t* __restrict__ lengths, int64_t* __restrict__ offsets,
-                                                                    int64_t* __restrict__ gate_index,
-                                                                    int64_t* __restrict__ token_index,
-                                                                    int64_t* __restrict__ reverse_index) {
+__device__ __forceinline__ void route_in_block(const T* scores, int num_tokens, int E, int K, int ebits, int renorm, int tokens_per_wave,
+                                               int64_t* __restrict__ topk_idx, T* __restrict__ gates, int64_t* __restrict__ lengths,
+                                               int64_t* __restrict__ offsets, int64_t* __restrict__ gate_index,
+                                               int64_t* __restrict__ token_index, int64_t* __restrict__ reverse_index, int32_t* s_hist,
+                                               uint16_t* s_ids) {
     constexpr int WPB = kMaxRouteWaves, NT = WPB * kWave;
     __shared__ float s_sel[WPB][kWave / LPT][64];
-    extern __shared__ int32_t s_hist[];       // [WPB][E] counts per wave, then every wave's next free slots
-    uint16_t* s_ids = reinterpret_cast<uint16_t*>(s_hist + WPB * E);     // [T * K]
     const int lane = lane_id();
     const int wave = threadIdx.x / kWave;
     for (int i = threadIdx.x; i < WPB * E; i += NT) s_hist[i] = 0;
@@ -548,6 +544,57 @@ __global__ __launch_bounds__(kMaxRouteWaves* kWave) void route_block_kernel(cons
     }
     __syncthreads();
     place_positions(s_ids, t_begin, t_end, tokens_per_wave, K, ebits, s_hist + wave * E, gate_index, token_index, reverse_index);
+}
+
+template <typename T, int LPT, int VPL>
+__global__ __launch_bounds__(kMaxRouteWaves* kWave) void route_block_kernel(const T* __restrict__ scores, int num_tokens, int E, int K,
+                                                                    int ebits, int renorm, int tokens_per_wave,
+                                                                    int64_t* __restrict__ topk_idx, T* __restrict__ gates,
+                                                                    int64_t* __restrict__ lengths, int64_t* __restrict__ offsets,
+                                                                    int64_t* __restrict__ gate_index,
+                                                                    int64_t* __restrict__ token_index,
+                                                                    int64_t* __restrict__ reverse_index) {
+    extern __shared__ int32_t s_hist[];       // [waves][E] counts per wave, then every wave's next free slots; [T * K] expert ids
+    route_in_block<T, LPT, VPL>(scores, num_tokens, E, K, ebits, renorm, tokens_per_wave, topk_idx, gates, lengths, offsets, gate_index,
+                                token_index, reverse_index, s_hist, reinterpret_cast<uint16_t*>(s_hist + kMaxRouteWaves * E));
+}
+
+// The gate of such a batch as well: the scores never leave LDS.  Groups of eight waves take 16 tokens at a time, as gate_softmax_kernel's blocks
+// do (the same sums in the same order), then the block routes them.
+constexpr int gate_groups(int nf) { return nf <= 2 ? 2 : 1; }
+template <typename T, int NF, int LPT, int VPL>
+__global__ __launch_bounds__(kMaxRouteWaves* kWave) void gate_softmax_route_kernel(
+    const uint8_t* __restrict__ x, int D, int64_t x_stride, const uint8_t* __restrict__ w, const void* __restrict__ bias, int num_tokens, int E,
+    int K, int ebits, int renorm, int tokens_per_wave, int64_t* __restrict__ topk_idx, T* __restrict__ gates, int64_t* __restrict__ lengths,
+    int64_t* __restrict__ offsets, int64_t* __restrict__ gate_index, int64_t* __restrict__ token_index, int64_t* __restrict__ reverse_index) {
+    constexpr bool F32 = sizeof(T) == 4;
+    constexpr int GROUPS = gate_groups(NF), TOKENS = GROUPS * kGateTokens;
+    extern __shared__ __align__(16) float red[];                    // [GROUPS] sums of a group; then counts, scores and expert ids
+    int32_t* const s_hist = reinterpret_cast<int32_t*>(red + GROUPS * gate_sums_floats(NF));
+    T* const s_scores = reinterpret_cast<T*>(s_hist + kMaxRouteWaves * E);
+    uint16_t* const s_ids = reinterpret_cast<uint16_t*>(s_scores + num_tokens * E);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), group = wave / kGateWaves;
+    for (int t0 = 0; t0 < num_tokens; t0 += TOKENS) {
+        if (t0) __syncthreads();                // the sums before have been read
+        if (group < GROUPS && t0 + group * kGateTokens < num_tokens)
+            gate_sums<F32, NF>(x, num_tokens, D, x_stride, w, E, t0 + group * kGateTokens, wave % kGateWaves, red + group * gate_sums_floats(NF));
+        __syncthreads();
+        constexpr int STEP = gate_wave_tokens(NF);              // (a wave's tokens lie in one group)
+        for (int first = wave * STEP; first < TOKENS && t0 + first < num_tokens; first += kMaxRouteWaves * STEP) {
+            const int g0 = first / kGateTokens * kGateTokens, tokens = num_tokens - t0 - g0 < kGateTokens ? num_tokens - t0 - g0 : kGateTokens;
+            gate_softmax_tokens<F32, NF>(red + first / kGateTokens * gate_sums_floats(NF), first - g0, tokens, bias, E, [&](int t, int e, float p) {
+                if constexpr (F32) s_scores[(t0 + g0 + t) * E + e] = p;
+                else s_scores[(t0 + g0 + t) * E + e] = (uint16_t)f32_to_bf16_bits(p);
+            });
+        }
+    }
+    // (the barrier behind the clearing of the counts publishes the scores)
+    route_in_block<T, LPT, VPL>(s_scores, num_tokens, E, K, ebits, renorm, tokens_per_wave, topk_idx, gates, lengths, offsets, gate_index,
+                                token_index, reverse_index, s_hist, s_ids);
+}
+inline size_t gate_route_lds(int esize, int64_t T, int E, int K) {
+    const int nf = gate_fragments(E);
+    return (size_t)gate_groups(nf) * gate_sums_floats(nf) * 4 + (size_t)kMaxRouteWaves * E * 4 + (size_t)T * E * esize + (size_t)T * K * 2;
 }
 
 int ceil_log2(int v) {
@@ -700,6 +747,46 @@ extern "C" int fmoe_route_topk(const void* scores, int score_dtype, int64_t T, i
     return route_topk_impl("fmoe_route_topk", scores, score_dtype, T, E, K, renorm, topk_idx, gates, lengths,
                            offsets, gate_index, token_index, reverse_index, workspace, workspace_bytes,
                            (hipStream_t)stream_);
+}
+
+// Where the gate and the routing of a batch are one launch: the one block can hold the scores, and walks the gate's rows in a time that the saved
+// launch covers.  Bytes of a gate row times 1 + fragments, for every 16 tokens: us of a layer's pass (256 hidden columns) among others and alone,
+// two launches / one: bf16 64 tokens, 128 inputs, 8 experts (2048) 28.8 / 23.9 and 45.1 / 42.7; 1, 128, 8 (512) 27.1 / 22.9 and 41.5 / 37.9; 16, 1024, 8
+// (4096) 26.3 / 24.7 and 47.6 / 45.4; 1, 2048, 8 (8192) 27.6 / 26.4 and 49.0 / 47.2; fp32 16, 1024, 8 (8192) 34.1 / 32.9 and 54.1 / 53.8.  Beyond: bf16 1,
+// 2048, 32 (12288) 31.1 / 30.0 and 50.2 / 50.6; several groups of tokens: fp32 64, 128, 8 (4096) 27.7 / 28.3 and 50.4 / 48.7; bf16 64, 512, 32 (12288)
+// 26.7 / 29.0 and 46.6 / 49.3; 64, 1024, 8 (16384) 28.0 / 31.8.
+extern "C" int fmoe_gate_route_pays(int dtype, int64_t T, int D, int E, int K) {
+    if (!fmoe_gate_softmax_pays(dtype, T, D, E) || K < 1 || K > E || E > 64 || !route_one_block(T, E, K)) return 0;
+    const int esize = dtype == FMOE_F32 ? 4 : 2, nf = gate_fragments(E);
+    const size_t selected = (size_t)kMaxRouteWaves * (kWave / (E <= 8 ? 8 : 16)) * 64 * 4;
+    if (gate_route_lds(esize, T, E, K) + selected > 65536) return 0;
+    const int64_t groups = (T + kGateTokens - 1) / kGateTokens;
+    return groups * D * esize * (1 + nf) <= (groups == 1 ? 8192 : 3072);
+}
+
+extern "C" int fmoe_gate_route(const void* x, int dtype, int64_t T, int D, int64_t x_stride_row, const void* weight, const void* bias, int E, int K,
+                               int renorm, int64_t* topk_idx, void* gates, int64_t* lengths, int64_t* offsets, int64_t* gate_index,
+                               int64_t* token_index, int64_t* reverse_index, fmoe_stream_t stream_) {
+    FMOE_REQUIRE(fmoe_gate_route_pays(dtype, T, D, E, K), "fmoe_gate_route: not a call that fmoe_gate_route_pays takes");
+    FMOE_REQUIRE(renorm >= 0 && renorm <= 3, "fmoe_gate_route: gate mode %d is not one of 0..3", renorm);
+    const int esize = dtype == FMOE_F32 ? 4 : 2;
+    FMOE_REQUIRE(x && weight && topk_idx && gates && lengths && offsets && gate_index && token_index && reverse_index,
+                 "fmoe_gate_route: NULL tensor pointer");
+    FMOE_REQUIRE(D <= (1 << 24) && x_stride_row >= D && x_stride_row % (16 / esize) == 0 && aligned16(x) && aligned16(weight),
+                 "fmoe_gate_route: rows of whole 16-byte chunks at 16-byte boundaries");
+    const size_t lds = gate_route_lds(esize, T, E, K);
+#define FMOE_GATE_ROUTE(TYPE, NF, LPT, VPL)                                                                                                     \
+    gate_softmax_route_kernel<TYPE, NF, LPT, VPL><<<1, kMaxRouteWaves * kWave, lds, (hipStream_t)stream_>>>(                                     \
+        (const uint8_t*)x, D, x_stride_row, (const uint8_t*)weight, bias, (int)T, E, K, ceil_log2(E), renorm,                                    \
+        (int)((T + kMaxRouteWaves - 1) / kMaxRouteWaves), topk_idx, (TYPE*)gates, lengths, offsets, gate_index, token_index, reverse_index)
+#define FMOE_GATE_ROUTE_E(TYPE)                                                                                                                  \
+    (E <= 8 ? (void)(FMOE_GATE_ROUTE(TYPE, 1, 8, 1)) : E <= 16 ? (void)(FMOE_GATE_ROUTE(TYPE, 1, 16, 1))                                         \
+     : E <= 32 ? (void)(FMOE_GATE_ROUTE(TYPE, 2, 16, 2)) : (void)(FMOE_GATE_ROUTE(TYPE, 4, 16, 4)))
+    if (dtype == FMOE_F32) FMOE_GATE_ROUTE_E(float);
+    else FMOE_GATE_ROUTE_E(uint16_t);
+#undef FMOE_GATE_ROUTE_E
+#undef FMOE_GATE_ROUTE
+    return check_launch("fmoe_gate_route");
 }
 
 // ------------------------------------------------------------ allocation-free variant

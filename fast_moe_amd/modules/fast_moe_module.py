@@ -10,7 +10,7 @@ syncs once for ``max_seq_len``, fast_moe_module.py:135).
 """
 from __future__ import annotations
 
-from typing import Dict
+from typing import Dict, Optional
 
 import torch
 import torch.nn as nn
@@ -107,18 +107,24 @@ class FastMoELayer(nn.Module):
     def _scores(self, x: torch.Tensor) -> torch.Tensor:
         """The gate's probabilities [tokens, E]: from one launch where the batch is small, nothing needs a gradient and the gate is the
         class's own; a caller's module, hooks, modes and autocast are asked through the modules, and so are other shapes, which they refuse."""
+        linear = self._small_gate(x)
+        if linear is not None:
+            scores = ops.gate_softmax(x.reshape(-1, self.input_dim), linear.weight, linear.bias)
+            if scores is not None:
+                return scores
+        return self.gate(x).reshape(-1, self.num_experts)
+
+    def _small_gate(self, x: torch.Tensor) -> Optional[nn.Linear]:
+        """The gate's Linear where a launch may stand for the gate of ``x``."""
         gate, shape = self.gate, x.shape
         if type(x) is torch.Tensor and len(shape) == 3 and shape[2] == self.input_dim and shape[0] * shape[1] <= _SMALL_BATCH \
                 and type(gate) is GatingNetwork and GatingNetwork.forward is _GATE_FORWARD and not torch.is_autocast_enabled() \
                 and not _mode_active():
             linear = gate.gate
             if type(linear) is nn.Linear and not _watched(gate) and not _watched(linear):
-                weight, bias = linear.weight, linear.bias
-                if not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)):
-                    scores = ops.gate_softmax(x.reshape(-1, self.input_dim), weight, bias)
-                    if scores is not None:
-                        return scores
-        return gate(x).reshape(-1, self.num_experts)
+                if not (torch.is_grad_enabled() and (x.requires_grad or linear.weight.requires_grad)):
+                    return linear
+        return None
 
     def forward(self, x: torch.Tensor, num_experts_per_tok: int) -> torch.Tensor:
         require_hip_kernel(self.kernel, "FastMoELayer.forward")
@@ -130,10 +136,18 @@ class FastMoELayer(nn.Module):
         k = num_experts_per_tok
         if getattr(self.route, "__func__", None) is _ROUTE and x.ndim == 3:
             # the same steps as below, issued by one native call (a route() of a subclass's or a caller's own is asked)
-            scores = self._scores(x)
-            y = _lib.host().mlp_forward(
-                scores, x.reshape(-1, self.input_dim), self._experts_hidden_w.permute(0, 2, 1), self._experts_hidden_bias,
-                self._experts_w.permute(0, 2, 1), self._experts_bias, k, ops.GATE_L1, EPI_SILU, ops._stream(x))
+            forward = _lib.host().mlp_forward
+            linear = self._small_gate(x) if ops.gate_softmax is _GATE_SOFTMAX else None
+            scores = None if linear is not None else self._scores(x)
+            args = (x.reshape(-1, self.input_dim), self._experts_hidden_w.permute(0, 2, 1), self._experts_hidden_bias,
+                    self._experts_w.permute(0, 2, 1), self._experts_bias, k, ops.GATE_L1, EPI_SILU, ops._stream(x))
+            y = None
+            if linear is not None:
+                y = forward(None, *args, linear.weight, linear.bias)
+                if y is None:
+                    scores = self._scores(x)
+            if y is None:
+                y = forward(scores, *args)
             if y is not None:
                 return y.view(original_shape[0], original_shape[1], self.output_dim)
             r = ops.route_topk(scores, k, renorm=True)
@@ -156,6 +170,7 @@ class FastMoELayer(nn.Module):
 
 _ROUTE = FastMoELayer.route     # what the native call stands for
 _GATE_FORWARD = GatingNetwork.forward
+_GATE_SOFTMAX = ops.gate_softmax
 _SMALL_BATCH = 128              # (the library's own rule, fmoe_gate_softmax_pays, without a call for the others)
 
 

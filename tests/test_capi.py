@@ -355,6 +355,17 @@ def test_column_quantiser_scratch_rule(lib, E, K, N, two_launches):
     assert (need > 0) == two_launches
 
 
+@pytest.mark.parametrize("dtype,T,D,E,K,pays", [
+    (1, 64, 128, 8, 2, True), (1, 64, 192, 16, 2, True), (1, 64, 200, 8, 2, False), (1, 16, 2048, 16, 4, True), (1, 16, 2056, 16, 4, False),
+    (1, 17, 2048, 16, 4, False), (1, 16, 1360, 32, 4, True), (1, 16, 1368, 32, 4, False), (1, 16, 816, 64, 8, True), (1, 16, 816, 65, 8, False),
+    (0, 16, 1024, 16, 4, True), (0, 16, 1028, 16, 4, False), (1, 16, 128, 8, 9, False), (1, 0, 128, 8, 2, False), (1, 64, 132, 8, 2, False),
+    (1, 96, 128, 16, 2, True), (1, 97, 128, 16, 2, False),
+])
+def test_gate_and_routing_in_one_launch_rule(lib, dtype, T, D, E, K, pays):
+    """Bytes of a gate row times one more than the fragments of 16 experts, for every 16 tokens (dtype: 0 fp32, 1 bf16)."""
+    assert bool(lib.fmoe_gate_route_pays(dtype, T, D, E, K)) == pays
+
+
 @pytest.mark.parametrize("dtype,T,D,E,pays", [
     (1, 128, 128, 8, True), (1, 129, 128, 8, False), (1, 0, 128, 8, False), (1, 1, 132, 8, False), (0, 1, 132, 8, True), (0, 1, 130, 8, False),
     (1, 64, 9552, 16, True), (1, 64, 9560, 16, False), (1, 64, 5728, 32, True), (1, 64, 5736, 32, False), (1, 64, 3184, 64, True),

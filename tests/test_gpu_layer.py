@@ -303,6 +303,38 @@ def test_gate_of_a_small_batch_declines_a_bias_of_another_length(entries):
     assert ops.gate_softmax(x, w, torch.zeros(8, device="cuda")) is not None
 
 
+@pytest.mark.parametrize("T,D,E,K", [(1, 8, 4, 2), (16, 1024, 8, 2), (17, 128, 7, 3), (33, 64, 16, 2), (64, 128, 8, 8), (64, 48, 17, 1), (96, 128, 16, 4),
+                                     (13, 1360, 32, 5), (47, 48, 33, 8), (16, 408, 64, 16), (40, 16, 64, 9)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bias", [True, False])
+def test_gate_and_routing_in_one_launch(T, D, E, K, dtype, bias, monkeypatch):
+    """Against the two launches, which a caller's own ops.gate_softmax asks for: the same bits; and from its trace that it is one.  NaN and
+    infinite scores among them."""
+    from fast_moe_amd import FastMoELayer
+    from fast_moe_amd.kernels.hip import _lib, ops
+    from tests.helpers import kernels_run
+    g = torch.Generator(device="cuda").manual_seed(T + D)
+    layer = FastMoELayer(D, 64, D, E, dtype=dtype).to(dtype).cuda()
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.copy_(torch.randn(p.shape, generator=g, device="cuda") * p.shape[-1] ** -0.5)
+        if not bias:
+            layer.gate.gate.bias = None
+        x = torch.randn(1, T, D, generator=g, device="cuda").to(dtype)
+        if T > 16:
+            x[0, 3, 1], x[0, T - 1, 0], x[0, 16] = float("nan"), float("inf"), 0
+        one = bool(_lib.load().fmoe_gate_route_pays(ops._DTYPE_CODE[dtype], T, D, E, K))
+        assert one or dtype == torch.float32
+        ran = kernels_run(lambda: layer(x, K))
+        assert any("gate_softmax_route_kernel" in n for n in ran) == one, ran
+        got, real = layer(x, K), ops.gate_softmax
+        monkeypatch.setattr(ops, "gate_softmax", lambda *a: real(*a))
+        ran = kernels_run(lambda: layer(x, K))
+        assert any("gate_softmax_kernel" in n for n in ran) and not any("gate_softmax_route" in n for n in ran), ran
+        want = layer(x, K)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
 @pytest.mark.parametrize("shape", [(1, 4, 128), (2, 4, 32), (8, 64), (512,), (2, 2, 2, 64)])
 def test_small_batches_of_another_shape_go_through_the_gate_module(shape):
     """What Linear and the softmax over the third dimension refuse is refused whatever the batch, before anything is routed, and what they
