@@ -35,7 +35,6 @@ decltype(&fmoe_quant_rows_e4m3) c_quant_rows;
 decltype(&fmoe_gate_softmax) c_gate_softmax;
 decltype(&fmoe_gate_softmax_pays) gate_softmax_pays;
 decltype(&fmoe_gate_route_pays) gate_route_pays;
-decltype(&fmoe_gate_route) c_gate_route;
 decltype(&fmoe_grouped_gemm_plan) c_gemm_plan;
 decltype(&fmoe_combine_bwd) c_combine_bwd;
 decltype(&fmoe_segment_colsum) c_segment_colsum;
@@ -540,17 +539,11 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
             return true;
         },
         [&] {
-            if (gate) {
-                what = "fmoe_gate_route";
-                if (const int rc = c_gate_route(x_data, dtype_code(x.scalar_type()), merge.T, (int)x.size(1), x.stride(0), data, gate_bias_data,
-                                                (int)scores.size(0), (int)k, (int)mode, topk_idx, gates, lengths, offsets, gate_index,
-                                                token_index, reverse, (void*)stream))
-                    return rc;
-            } else if (const int rc = c_route_topk(data, dtype_code(scores.scalar_type()), merge.T, (int)scores.size(1), (int)k, (int)mode,
-                                                   topk_idx, gates, lengths, offsets, gate_index, token_index, reverse, base + at_ws,
-                                                   ws_bytes, (void*)stream)) {
+            const fmoe_gate g = {x_data, data, gate_bias_data, x.stride(0), dtype_code(x.scalar_type()), (int)x.size(1)};
+            if (const int rc = c_route_topk(gate ? &g : data, gate ? FMOE_SCORES_OF_GATE : dtype_code(scores.scalar_type()), merge.T,
+                                            (int)w1.size(0), (int)k, (int)mode, topk_idx, gates, lengths, offsets, gate_index, token_index,
+                                            reverse, base + at_ws, ws_bytes, (void*)stream))
                 return rc;
-            }
             RECORD_USER_SCOPE("## expert_forward##");
             what = "fmoe_grouped_gemm";
             if (const int rc = gemm(up, x, (void*)stream)) return rc;
@@ -787,7 +780,7 @@ PyObject* py_init(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void* const entry[] = {&route_workspace_bytes, &c_route_topk, &c_grouped_gemm, &c_combine, &c_quant_rows, &c_gate_softmax, &gemm_workspace_bytes,
                            &c_grouped_gemm_ws, &c_gemm_plan, &c_combine_bwd, &c_segment_colsum, &c_swiglu_bwd, &c_silu_mul, &c_gather_rows,
                            &c_invert_index, &c_gate_l1_bwd, &c_weight_grad, &weight_grad_pays, &gate_softmax_pays,
-                           &gate_route_pays, &c_gate_route, &last_error};
+                           &gate_route_pays, &last_error};
     constexpr Py_ssize_t count = sizeof(entry) / sizeof(entry[0]);
     if (n != count) {
         PyErr_Format(PyExc_TypeError, "init: %d addresses expected", (int)count);

@@ -740,15 +740,6 @@ static int route_topk_impl(const char* who, const void* scores, int score_dtype,
                        stream);
 }
 
-extern "C" int fmoe_route_topk(const void* scores, int score_dtype, int64_t T, int E, int K, int renorm,
-                               int64_t* topk_idx, void* gates, int64_t* lengths, int64_t* offsets,
-                               int64_t* gate_index, int64_t* token_index, int64_t* reverse_index,
-                               void* workspace, size_t workspace_bytes, fmoe_stream_t stream_) {
-    return route_topk_impl("fmoe_route_topk", scores, score_dtype, T, E, K, renorm, topk_idx, gates, lengths,
-                           offsets, gate_index, token_index, reverse_index, workspace, workspace_bytes,
-                           (hipStream_t)stream_);
-}
-
 // Where the gate and the routing of a batch are one launch: the one block can hold the scores, and walks the gate's rows in a time that the saved
 // launch covers.  Bytes of a gate row times 1 + fragments, for every 16 tokens: us of a layer's pass (256 hidden columns) among others and alone,
 // two launches / one: bf16 64 tokens, 128 inputs, 8 experts (2048) 28.8 / 23.9 and 45.1 / 42.7; 1, 128, 8 (512) 27.1 / 22.9 and 41.5 / 37.9; 16, 1024, 8
@@ -764,29 +755,40 @@ extern "C" int fmoe_gate_route_pays(int dtype, int64_t T, int D, int E, int K) {
     return groups * D * esize * (1 + nf) <= (groups == 1 ? 8192 : 3072);
 }
 
-extern "C" int fmoe_gate_route(const void* x, int dtype, int64_t T, int D, int64_t x_stride_row, const void* weight, const void* bias, int E, int K,
-                               int renorm, int64_t* topk_idx, void* gates, int64_t* lengths, int64_t* offsets, int64_t* gate_index,
-                               int64_t* token_index, int64_t* reverse_index, fmoe_stream_t stream_) {
-    FMOE_REQUIRE(fmoe_gate_route_pays(dtype, T, D, E, K), "fmoe_gate_route: not a call that fmoe_gate_route_pays takes");
-    FMOE_REQUIRE(renorm >= 0 && renorm <= 3, "fmoe_gate_route: gate mode %d is not one of 0..3", renorm);
-    const int esize = dtype == FMOE_F32 ? 4 : 2;
-    FMOE_REQUIRE(x && weight && topk_idx && gates && lengths && offsets && gate_index && token_index && reverse_index,
-                 "fmoe_gate_route: NULL tensor pointer");
-    FMOE_REQUIRE(D <= (1 << 24) && x_stride_row >= D && x_stride_row % (16 / esize) == 0 && aligned16(x) && aligned16(weight),
-                 "fmoe_gate_route: rows of whole 16-byte chunks at 16-byte boundaries");
+static int gate_route(const fmoe_gate* g, int64_t T, int E, int K, int renorm, int64_t* topk_idx, void* gates, int64_t* lengths, int64_t* offsets,
+                      int64_t* gate_index, int64_t* token_index, int64_t* reverse_index, hipStream_t stream) {
+    FMOE_REQUIRE(g && fmoe_gate_route_pays(g->dtype, T, g->d, E, K), "fmoe_route_topk: not a gate that fmoe_gate_route_pays takes");
+    FMOE_REQUIRE(renorm >= 0 && renorm <= 3, "fmoe_route_topk: gate mode %d is not one of 0..3", renorm);
+    const int esize = g->dtype == FMOE_F32 ? 4 : 2;
+    FMOE_REQUIRE(g->x && g->weight && topk_idx && gates && lengths && offsets && gate_index && token_index && reverse_index,
+                 "fmoe_route_topk: NULL tensor pointer");
+    FMOE_REQUIRE(g->x_stride_row >= g->d && g->x_stride_row % (16 / esize) == 0 && aligned16(g->x) && aligned16(g->weight),
+                 "fmoe_route_topk: gate rows of whole 16-byte chunks at 16-byte boundaries");
     const size_t lds = gate_route_lds(esize, T, E, K);
 #define FMOE_GATE_ROUTE(TYPE, NF, LPT, VPL)                                                                                                     \
-    gate_softmax_route_kernel<TYPE, NF, LPT, VPL><<<1, kMaxRouteWaves * kWave, lds, (hipStream_t)stream_>>>(                                     \
-        (const uint8_t*)x, D, x_stride_row, (const uint8_t*)weight, bias, (int)T, E, K, ceil_log2(E), renorm,                                    \
+    gate_softmax_route_kernel<TYPE, NF, LPT, VPL><<<1, kMaxRouteWaves * kWave, lds, stream>>>(                                                    \
+        (const uint8_t*)g->x, g->d, g->x_stride_row, (const uint8_t*)g->weight, g->bias, (int)T, E, K, ceil_log2(E), renorm,                                    \
         (int)((T + kMaxRouteWaves - 1) / kMaxRouteWaves), topk_idx, (TYPE*)gates, lengths, offsets, gate_index, token_index, reverse_index)
 #define FMOE_GATE_ROUTE_E(TYPE)                                                                                                                  \
     (E <= 8 ? (void)(FMOE_GATE_ROUTE(TYPE, 1, 8, 1)) : E <= 16 ? (void)(FMOE_GATE_ROUTE(TYPE, 1, 16, 1))                                         \
      : E <= 32 ? (void)(FMOE_GATE_ROUTE(TYPE, 2, 16, 2)) : (void)(FMOE_GATE_ROUTE(TYPE, 4, 16, 4)))
-    if (dtype == FMOE_F32) FMOE_GATE_ROUTE_E(float);
+    if (g->dtype == FMOE_F32) FMOE_GATE_ROUTE_E(float);
     else FMOE_GATE_ROUTE_E(uint16_t);
 #undef FMOE_GATE_ROUTE_E
 #undef FMOE_GATE_ROUTE
-    return check_launch("fmoe_gate_route");
+    return check_launch("fmoe_route_topk");
+}
+
+extern "C" int fmoe_route_topk(const void* scores, int score_dtype, int64_t T, int E, int K, int renorm,
+                               int64_t* topk_idx, void* gates, int64_t* lengths, int64_t* offsets,
+                               int64_t* gate_index, int64_t* token_index, int64_t* reverse_index,
+                               void* workspace, size_t workspace_bytes, fmoe_stream_t stream_) {
+    if (score_dtype == FMOE_SCORES_OF_GATE)
+        return gate_route((const fmoe_gate*)scores, T, E, K, renorm, topk_idx, gates, lengths, offsets, gate_index, token_index, reverse_index,
+                          (hipStream_t)stream_);
+    return route_topk_impl("fmoe_route_topk", scores, score_dtype, T, E, K, renorm, topk_idx, gates, lengths,
+                           offsets, gate_index, token_index, reverse_index, workspace, workspace_bytes,
+                           (hipStream_t)stream_);
 }
 
 // ------------------------------------------------------------ allocation-free variant

@@ -27,7 +27,7 @@ EXPORTED_SYMBOLS = (
     "fmoe_combine",
     "fmoe_silu_mul", "fmoe_transpose_last2", "fmoe_jagged_transpose", "fmoe_segment_colsum",
     "fmoe_swiglu_bwd", "fmoe_combine_bwd", "fmoe_gather_rows", "fmoe_invert_index",
-    "fmoe_gate_l1_bwd", "fmoe_gate_softmax_pays", "fmoe_gate_softmax", "fmoe_gate_route_pays", "fmoe_gate_route", "fmoe_weight_grad_pays", "fmoe_weight_grad", "fmoe_route_topk_static", "fmoe_hbm_probe",
+    "fmoe_gate_l1_bwd", "fmoe_gate_softmax_pays", "fmoe_gate_softmax", "fmoe_gate_route_pays", "fmoe_weight_grad_pays", "fmoe_weight_grad", "fmoe_route_topk_static", "fmoe_hbm_probe",
 )
 ROUTE_STATIC_MAX_POSITIONS, ROUTE_STATIC_MAX_EXPERTS = 1 << 20, 512
 
@@ -106,8 +106,6 @@ def load() -> ctypes.CDLL:
     lib.fmoe_gate_softmax_pays.argtypes = [c_int, c_int64, c_int, c_int]
     lib.fmoe_gate_route_pays.restype = c_int
     lib.fmoe_gate_route_pays.argtypes = [c_int, c_int64, c_int, c_int, c_int]
-    lib.fmoe_gate_route.restype = c_int
-    lib.fmoe_gate_route.argtypes = [c_void_p, c_int, c_int64, c_int, c_int64, c_void_p, c_void_p, c_int, c_int, c_int] + [c_void_p] * 8
     lib.fmoe_gate_softmax.restype = c_int
     lib.fmoe_gate_softmax.argtypes = [c_void_p, c_int, c_int64, c_int, c_int64, c_void_p, c_void_p, c_int, c_void_p, c_void_p]
     lib.fmoe_weight_grad_pays.restype = c_int
@@ -153,7 +151,7 @@ HOST_ENTRY_POINTS = ("fmoe_route_workspace_bytes", "fmoe_route_topk", "fmoe_grou
                      "fmoe_quant_rows_e4m3", "fmoe_gate_softmax", "fmoe_grouped_gemm_workspace_bytes", "fmoe_grouped_gemm_ws",
                      "fmoe_grouped_gemm_plan", "fmoe_combine_bwd", "fmoe_segment_colsum", "fmoe_swiglu_bwd", "fmoe_silu_mul",
                      "fmoe_gather_rows", "fmoe_invert_index", "fmoe_gate_l1_bwd", "fmoe_weight_grad", "fmoe_weight_grad_pays",
-                     "fmoe_gate_softmax_pays", "fmoe_gate_route_pays", "fmoe_gate_route", "fmoe_last_error")
+                     "fmoe_gate_softmax_pays", "fmoe_gate_route_pays", "fmoe_last_error")
 _host = None
 
 

@@ -142,13 +142,19 @@ int fmoe_gate_softmax_pays(int dtype, int64_t T, int D, int E);
 int fmoe_gate_softmax(const void* x, int dtype, int64_t T, int D, int64_t x_stride_row, const void* weight, const void* bias,
                       int E, void* scores, fmoe_stream_t stream);
 /*
- * fmoe_gate_softmax and fmoe_route_topk of its scores (which are not written) in one launch, the same outputs bit for bit, for the calls that
+ * fmoe_gate_softmax and fmoe_route_topk of its scores (which are not written) in one launch, the same outputs bit for bit: fmoe_route_topk with
+ * score_dtype FMOE_SCORES_OF_GATE and a host fmoe_gate in the place of the scores (no workspace; gates in its dtype), for the calls that
  * fmoe_gate_route_pays names (a few tokens, up to 64 experts).
  */
+enum { FMOE_SCORES_OF_GATE = 0x100 };
+typedef struct fmoe_gate {
+    const void* x;              /* [T, d] rows at x_stride_row, 16-byte aligned, whole 16-byte chunks */
+    const void* weight;         /* [E, d], 16-byte aligned */
+    const void* bias;           /* [E] or NULL */
+    int64_t x_stride_row;
+    int32_t dtype, d;
+} fmoe_gate;
 int fmoe_gate_route_pays(int dtype, int64_t T, int D, int E, int K);
-int fmoe_gate_route(const void* x, int dtype, int64_t T, int D, int64_t x_stride_row, const void* weight, const void* bias, int E, int K,
-                    int renorm, int64_t* topk_idx, void* gates, int64_t* lengths, int64_t* offsets, int64_t* gate_index, int64_t* token_index,
-                    int64_t* reverse_index, fmoe_stream_t stream);
 
 /* ---------------------------------------------------------- FP8 quantisation */
 
