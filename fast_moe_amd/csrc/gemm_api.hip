@@ -45,7 +45,7 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
     FMOE_REQUIRE(d->epilogue >= FMOE_EPI_NONE && d->epilogue <= FMOE_EPI_GATED,
                  "fmoe_grouped_gemm: unknown epilogue %d", d->epilogue);
     if (d->total_rows == 0) return FMOE_OK;     // sel stays -1
-    FMOE_REQUIRE(d->offsets && d->a && d->b && d->out, "fmoe_grouped_gemm: NULL tensor pointer");
+    FMOE_REQUIRE((d->offsets || d->a_stride_k > 1) && d->a && d->b && d->out, "fmoe_grouped_gemm: NULL tensor pointer");
     FMOE_REQUIRE(d->a_rows >= 1, "fmoe_grouped_gemm: a_rows < 1");
     FMOE_REQUIRE(d->index_div >= 1, "fmoe_grouped_gemm: index_div < 1");
     const bool row_indexed = d->a_stride_k > 1;      // A (and B) given with k as the row index
@@ -85,6 +85,13 @@ static int prepare_gemm(const fmoe_gemm_desc* d, GemmParams& p, int& sel) {
     }
 
     p.offsets = d->offsets;
+    p.rows_each = 0;
+    if (!d->offsets) {
+        FMOE_REQUIRE(d->total_rows % d->num_experts == 0 && d->total_rows < ((int64_t)1 << 31),
+                     "fmoe_grouped_gemm: without offsets every expert has as many output rows (total_rows=%lld E=%d)", (long long)d->total_rows,
+                     d->num_experts);
+        p.rows_each = (int)(d->total_rows / d->num_experts);
+    }
     p.row_index = d->row_index;
     p.E = d->num_experts;
     p.N = d->n;

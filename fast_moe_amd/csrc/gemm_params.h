@@ -60,6 +60,7 @@ struct GemmParams {
     const uint8_t* a2;                  // second product a2 * b2 summed into the same output, or null
     int k_split;                        // ... whose contraction covers k in [k_split, K)
     SplitWorkspace* split_ws;           // tiles cut along K: where their sums meet, or null
+    int rows_each;                      // row-indexed operands without offsets: output rows of every expert
     int split_slots;                    // fp32: blocks of a round, for one XCD
 #ifdef FMOE_TRACE
     uint64_t* trace;                    // debug builds: per-tile time stamps of the ring kernel

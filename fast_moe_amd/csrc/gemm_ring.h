@@ -158,9 +158,14 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             const int e = i * kWave + lane;
             int64_t lo = 0, len = 0;
             if (e < p.E) {
-                lo = clamp_i64(p.offsets[e], 0, R);
-                const int64_t hi = clamp_i64(p.offsets[e + 1], 0, R);
-                len = hi > lo ? hi - lo : 0;
+                if (XTR && !p.offsets) {
+                    lo = (int64_t)e * p.rows_each;
+                    len = p.rows_each;
+                } else {
+                    lo = clamp_i64(p.offsets[e], 0, R);
+                    const int64_t hi = clamp_i64(p.offsets[e + 1], 0, R);
+                    len = hi > lo ? hi - lo : 0;
+                }
             }
             e_lo[i] = (int)lo;
             e_len[i] = (int)len;
@@ -320,7 +325,12 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
             }
             const int expert = KWIN ? ex : cnt;
             int64_t o_lo, o_hi;
-            scalar_load_i64x2(p.offsets + expert, o_lo, o_hi);
+            if (XTR && !p.offsets) {
+                o_lo = (int64_t)expert * p.rows_each;
+                o_hi = o_lo + p.rows_each;
+            } else {
+                scalar_load_i64x2(p.offsets + expert, o_lo, o_hi);
+            }
             o_lo = clamp_i64(o_lo, 0, R);
             o_hi = clamp_i64(o_hi, 0, R);
             const int lo = (int)o_lo, len = (int)(o_hi > o_lo ? o_hi - o_lo : 0);

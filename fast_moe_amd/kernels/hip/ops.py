@@ -330,7 +330,6 @@ def jagged_weight_grad(dout: torch.Tensor, a_rows: torch.Tensor, offsets: torch.
         return None
     dev = dout.device
     offsets = _i64("offsets", offsets)
-    seg = torch.arange(0, E * N + 1, N, device=dev, dtype=torch.int64)
     if halves:
         out = torch.empty((E * (N // 2), Kin), dtype=torch.bfloat16, device=dev)
         out2 = torch.empty_like(out)
@@ -341,7 +340,6 @@ def jagged_weight_grad(dout: torch.Tensor, a_rows: torch.Tensor, offsets: torch.
     if halves:
         d.out2 = out2.data_ptr()
     d.total_rows, d.a_rows = E * N, N
-    d.offsets = seg.data_ptr()
     d.a, d.a_dtype, d.a_stride_row, d.a_stride_k = dout.data_ptr(), _DTYPE_CODE[dout.dtype], 1, dout.stride(0)
     d.b, d.b_stride_e, d.b_stride_k, d.b_stride_n = a_rows.data_ptr(), 0, a_rows.stride(0), 1
     d.epilogue, d.out_dtype = EPI_NONE, _DTYPE_CODE[torch.bfloat16]

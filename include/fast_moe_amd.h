@@ -248,7 +248,7 @@ typedef struct fmoe_gemm_desc {
     int32_t index_div;      /* divisor applied to row_index values (>= 1)         */
     int64_t total_rows;     /* rows of `out` (= offsets[E]; host-known upper bound) */
     int64_t a_rows;         /* rows of A (bound for gathered sources)             */
-    const int64_t* offsets; /* [E+1]                                              */
+    const int64_t* offsets; /* [E+1]; may be NULL with a_stride_k > 1: total_rows / E for every expert */
     const int64_t* row_index; /* [total_rows] or NULL                             */
 
     const void* a;          /* [a_rows, k] (or [a_rows, E, k] with a_stride_e)    */

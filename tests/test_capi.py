@@ -344,6 +344,20 @@ def test_the_built_host_module_loads(lib):
         assert _lib.host().torch_version
 
 
+def test_offsets_may_be_left_out_with_row_indexed_operands_only(lib):
+    from fast_moe_amd.kernels.hip._lib import GemmDesc
+    d = GemmDesc()
+    d.num_experts, d.n, d.k, d.index_div, d.total_rows, d.a_rows = 3, 256, 256, 1, 512, 512
+    d.a, d.b, d.out, d.a_dtype, d.out_dtype = 64, 64, 64, 1, 1
+    d.a_stride_row, d.b_stride_k, d.b_stride_n, d.out_stride_row = 256, 256, 1, 256
+    plan = ctypes.c_int(7)
+    assert lib.fmoe_grouped_gemm_plan(ctypes.byref(d), ctypes.byref(plan)) == 1
+    assert b"NULL tensor pointer" in lib.fmoe_last_error()
+    d.a_stride_row, d.a_stride_k = 1, 512
+    assert lib.fmoe_grouped_gemm_plan(ctypes.byref(d), ctypes.byref(plan)) == 1
+    assert b"as many output rows" in lib.fmoe_last_error()
+
+
 @pytest.mark.parametrize("E,K,N,two_launches", [
     (1, 4096, 8, False), (1, 4100, 8, True), (1, 4096, 64, False), (2, 4100, 64, True), (128, 44, 1024, False),
     (1, 4104, 12, False), (1, 4102, 16, False),

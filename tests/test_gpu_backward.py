@@ -515,6 +515,30 @@ def test_weight_gradient_of_few_rows_needs_nothing_behind_them(R, E):
         assert bool(((got[e].double() - want).abs() <= bound + 2.0 ** -8 * (want.abs() + bound)).all())
 
 
+@pytest.mark.parametrize("E,N,Kin,halves", [(1, 1152, 2048, False), (5, 1032, 1160, False), (64, 320, 264, True), (70, 264, 328, False), (200, 128, 264, True)])
+def test_weight_gradient_without_offsets(E, N, Kin, halves):
+    """The ring's weight gradients find every expert's output rows by its number (offsets NULL): fp64 with the roundings of an fp32 sum over the
+    expert's rows and of the bf16 result.  Experts without rows and one with most of them."""
+    from fast_moe_amd.kernels.hip import ops
+    from helpers import kernels_run
+    R = 40 * E + 6000
+    g = torch.Generator(device="cuda").manual_seed(E)
+    lens = [0 if e % 3 == 1 else 40 for e in range(E)]
+    lens[E // 2] += R - sum(lens)
+    off = torch.tensor([0, *torch.tensor(lens).cumsum(0)]).cuda()
+    d, x = (ops.empty_rows(R, n, BF16, "cuda") for n in (N, Kin))
+    for t in (d, x):
+        t.copy_(torch.randn(t.shape, generator=g, device="cuda"))
+    ran = kernels_run(lambda: ops.jagged_weight_grad(d, x, off, halves=halves))
+    assert len(ran) == 1, ran
+    got = ops.jagged_weight_grad(d, x, off, halves=halves)
+    got = torch.cat(got, dim=1) if halves else got
+    for e in range(E):
+        a, b = d[off[e]:off[e + 1]].double(), x[off[e]:off[e + 1]].double()
+        want, bound = a.t() @ b, (R + 1) * 2.0 ** -24 * (a.abs().t() @ b.abs())
+        assert bool(((got[e].double() - want).abs() <= bound + 2.0 ** -8 * (want.abs() + bound)).all()), e
+
+
 def test_large_fp32_weight_gradients_take_the_transposed_copies():
     from fast_moe_amd.kernels.hip import ops
     assert ops.weight_grad_pays(torch.float32, 8, 1000, 1000, 12000) and not ops.weight_grad_pays(torch.float32, 8, 1000, 1000, 12001)
