@@ -61,7 +61,9 @@ bool f32x3_split_pays(const GemmParams& p, bool swiglu) {
     const int bn_out = swiglu ? 64 : 128, pairs = (p.K + 63) / 64;
     const int64_t blocks = split_blocks(), n_tiles = (p.N + bn_out - 1) / bn_out;
     const int64_t least = (p.total_rows + 127) / 128 * n_tiles, most = most_row_tiles(p.total_rows, p.E, 128) * n_tiles;
-    if (blocks < kNumXcd || blocks > kSplitMost || pairs < 4 || least < kNumXcd || most >= ((int64_t)1 << 30)) return false;
+    if (blocks < kNumXcd || blocks > kSplitMost || pairs < 4 || least < kNumXcd || most >= ((int64_t)1 << 30) ||
+        p.total_rows >= ((int64_t)1 << 31))
+        return false;
     const int64_t middle = (least + most) / 2, rounds = middle / blocks;
     if (most / blocks > least / blocks + 1 || rounds == 1 || (rounds == 0 && (most > blocks || 8 * least < 5 * blocks))) return false;
     const int rest = (int)(middle % blocks);

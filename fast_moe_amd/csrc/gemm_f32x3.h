@@ -142,8 +142,8 @@ __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const Gem
     const bool here = CUT && p.split_ws ? tile.locate(p, BM, [&](int64_t total_tiles) -> int64_t {
         const SplitDeal deal((int)total_tiles, p.split_slots, blockIdx.x % kNumXcd, pairs,
                              [](int rest, int pairs, int blocks) { return f32x3_split_pieces(rest, pairs, blocks); });
-        if (blockIdx.x == 0 && tid == 0) {
-            p.split_ws->tiles = deal.pieces > 1 ? deal.rest : 0;
+        if (blockIdx.x == 0 && tid == 0) {      // (offsets that overlap name more tiles than the grid has blocks: nothing is added up then)
+            p.split_ws->tiles = deal.pieces > 1 && deal.count * kNumXcd <= (int)gridDim.x ? deal.rest : 0;
             p.split_ws->pieces = deal.pieces;
         }
         const int j = blockIdx.x / kNumXcd;
