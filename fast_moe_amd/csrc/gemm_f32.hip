@@ -40,8 +40,7 @@ int launch_f32x3(GemmParams p, hipStream_t stream) {
     p.n_tiles = (p.N + bn_out - 1) / bn_out;
     auto kern = grouped_gemm_f32x3_kernel<TL, EPI, NCONT, A_SILU>;
     static bool attr_done = false;
-    if constexpr (TL::BM * TL::BN != kF32x3CutTile) return launch_tiles<TL>(kern, p, attr_done, stream);
-    if (!p.split_ws) return launch_tiles<TL>(kern, p, attr_done, stream);
+    if (!TL::template kCut<EPI == FMOE_EPI_SWIGLU> || !p.split_ws) return launch_tiles<TL>(kern, p, attr_done, stream);
     if (int rc = reserve_lds(kern, TL::LDS_BYTES, attr_done)) return rc;
     const int64_t blocks = split_blocks(), rounds = most_row_tiles(p.total_rows, p.E, TL::BM) * p.n_tiles / blocks;
     p.split_slots = (int)blocks / kNumXcd;
@@ -51,24 +50,28 @@ int launch_f32x3(GemmParams p, hipStream_t stream) {
     return check_launch("fmoe_grouped_gemm");
 }
 
-// Whether a call's last round is cut along K: the 128 x 128 tiles it leaves, halfway between the fewest and the most that the row count allows (which
+// Whether a call's last round is cut along K: the tiles of BM x 128 it leaves, halfway between the fewest and the most that the row count allows (which
 // lie in one round of one per CU or the next), cost less as pieces by 8 us at least.
 //   * not behind a single round: its tiles run one to a CU, at seven eighths of the rate of two, until the pieces join them.  4096 rows, 8 experts,
 //     4096 -> 1024 (64 x 128 tiles instead) 320 / 341, 3000 rows, 5 experts, 2048 -> 2048 184 / 189; a few gain (4 experts, 1000 rows, 2048 -> 4096 162 / 155)
 //   * less than a round, from 5/8 of one on, all of it as pieces, two or three to a CU: 3000 rows, 4 experts, 4096 -> 1024, hot 256 / 201; 1000 rows,
 //     4 experts, 4096 -> 2560 206 / 196, 4096 -> 2 x 1280 207 / 193
+//   * 64 x 128 tiles behind two whole rounds, the pieces as third blocks (three rounds: 3000 rows, 5 experts, 2048 -> 2048 188 / 198).  An even load
+//     that leaves no tile pays for the second launch: 4096 rows, 8 experts, 4096 -> 1024 245 / 254
+template <int BM>
 bool f32x3_split_pays(const GemmParams& p, bool swiglu) {
     const int bn_out = swiglu ? 64 : 128, pairs = (p.K + 63) / 64;
     const int64_t blocks = split_blocks(), n_tiles = (p.N + bn_out - 1) / bn_out;
-    const int64_t least = (p.total_rows + 127) / 128 * n_tiles, most = most_row_tiles(p.total_rows, p.E, 128) * n_tiles;
+    const int64_t least = (p.total_rows + BM - 1) / BM * n_tiles, most = most_row_tiles(p.total_rows, p.E, BM) * n_tiles;
     if (blocks < kNumXcd || blocks > kSplitMost || pairs < 4 || least < kNumXcd || most >= ((int64_t)1 << 30) ||
         p.total_rows >= ((int64_t)1 << 31))
         return false;
     const int64_t middle = (least + most) / 2, rounds = middle / blocks;
-    if (most / blocks > least / blocks + 1 || rounds == 1 || (rounds == 0 && (most > blocks || 8 * least < 5 * blocks))) return false;
+    if (most / blocks > least / blocks + 1) return false;
+    if (BM == 64 ? rounds != 2 || least < 2 * blocks : rounds == 1 || (rounds == 0 && (most > blocks || 8 * least < 5 * blocks))) return false;
     const int rest = (int)(middle % blocks);
     int cost;
-    return rest && f32x3_split_pieces(rest, pairs, (int)blocks, &cost) > 1 && kF32x3PairCost * pairs - cost >= 72;
+    return rest && f32x3_split_pieces<BM>(rest, pairs, (int)blocks, &cost) > 1 && (BM == 128 ? 36 : 18) * pairs - cost >= 72;
 }
 
 // From three slices on.  Up to two (K = 64) it is level or ahead too (4096 rows, 8 experts, 4096 columns, K = 32 30.6 / 27.4), but a third behind
@@ -83,16 +86,20 @@ bool f32x3_split_pays(const GemmParams& p, bool swiglu) {
 // 16384 rows are 159 TFLOP/s, 1270 of bf16 products: what the chip's power allows.
 //   * 128 x 128 reads the least from LDS for a product: where the rows fill five such tiles for every four CUs.
 //   * 64 x 64: up to four per CU however the rows fall (two with SiLU on load, which every column of tiles repeats).
+bool f32x3_takes_large(const GemmParams& p, bool swiglu) {
+    return p.total_rows / 128 * ((p.N * (swiglu ? 2 : 1) + 127) / 128) * 4 >= 5 * compute_units();
+}
+bool f32x3_takes_small(const GemmParams& p, bool a_silu) { return (p.total_rows / 64 + p.E) * ((p.N + 63) / 64) <= (a_silu ? 2 : 4) * compute_units(); }
+bool f32x3_takes_mid(const GemmParams& p, bool a_silu) { return !f32x3_takes_large(p, false) && !f32x3_takes_small(p, a_silu); }
+
 template <int EPI, bool NCONT, bool A_SILU>
 int pick_f32x3(const GemmParams& p, hipStream_t stream) {
     constexpr bool swiglu = EPI == FMOE_EPI_SWIGLU;
     typedef TileF32x3<64, 128, swiglu ? 2 : 1, swiglu ? 2 : 4> Mid;
     typedef TileF32x3<64, 64, 2, 2> Small;
-    const int64_t cus = compute_units();
-    auto columns = [&](int bn) { return (p.N * (swiglu ? 2 : 1) + bn - 1) / bn; };
-    if (p.split_ws || p.total_rows / 128 * columns(128) * 4 >= 5 * cus) return launch_f32x3<TileF32Large, EPI, NCONT, A_SILU>(p, stream);
+    if (p.split_ws ? f32x3_split_pays<128>(p, swiglu) : f32x3_takes_large(p, swiglu)) return launch_f32x3<TileF32Large, EPI, NCONT, A_SILU>(p, stream);
     if constexpr (!swiglu) {
-        if ((p.total_rows / 64 + p.E) * columns(64) <= (A_SILU ? 2 : 4) * cus) return launch_f32x3<Small, EPI, NCONT, A_SILU>(p, stream);
+        if (!p.split_ws && f32x3_takes_small(p, A_SILU)) return launch_f32x3<Small, EPI, NCONT, A_SILU>(p, stream);
     }
     return launch_f32x3<Mid, EPI, NCONT, A_SILU>(p, stream);
 }
@@ -109,8 +116,9 @@ int dispatch(const GemmParams& p, int sel, hipStream_t stream) {
 
 size_t gemm_f32_split_bytes(const GemmParams& p, int epilogue, bool a_silu, int sel) {
     if (sel == kSelGeneric || p.K <= 2 * 32 || p.k_window || epilogue == FMOE_EPI_GATED) return 0;
-    if (!f32x3_split_pays(p, epilogue == FMOE_EPI_SWIGLU)) return 0;
-    return kSplitHeaderBytes + (size_t)(2 * split_blocks()) * kF32x3PieceBytes;
+    const bool swiglu = epilogue == FMOE_EPI_SWIGLU;
+    const int bm = f32x3_split_pays<128>(p, swiglu) ? 128 : !swiglu && f32x3_takes_mid(p, a_silu) && f32x3_split_pays<64>(p, false) ? 64 : 0;
+    return bm ? kSplitHeaderBytes + (size_t)(2 * split_blocks()) * f32x3_piece_bytes(bm) : 0;
 }
 
 int run_gemm_f32(GemmParams& p, int epilogue, bool a_silu, int sel, hipStream_t stream) {

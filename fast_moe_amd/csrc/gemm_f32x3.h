@@ -32,26 +32,32 @@ struct TileF32x3 {
     static constexpr int LDS_BYTES = 3 * (A_PLANE + B_PLANE);
     static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile must hold whole 32x32 fragments");
     static_assert((BM * 4) % NT == 0 && (BN * 4) % NT == 0, "loader passes must be whole");
+    // the tiles whose last round is cut along K
+    template <bool SWIGLU>
+    static constexpr bool kCut = BN == 128 && (BM == 128 || !SWIGLU);
 };
 
-// Last round cut along K, as the tall ring's (gemm_split.h): 128 x 128 tiles.  Two of them on a CU take 1.75 times as long as one, so a launch ends
+// Last round cut along K, as the tall ring's (gemm_split.h).  Two 128 x 128 tiles on a CU take 1.75 times as long as one, so a launch ends
 // with the CUs that have one tile more.  The tiles beyond whole rounds of one per CU go out as pieces of K behind them; each leaves its sums in the
 // workspace, f32x3_reduce_kernel adds them in the order of K.  us, whole tiles / cut: 8000 rows, 24 experts, 2048 -> 1024 353 / 280; 16000 rows, 20
 // experts, 1536 -> 1024 403 / 347; 9189 rows, 12 experts, 2600 -> 1000 429 / 345, 1000 -> 2600 396 / 370; 4096 rows, 8 experts, 1024 -> 4096 284 / 266; 2500
 // rows, 10 experts, 768 -> 3072 137 / 115; 4096 rows, 4 experts, 3072 -> 2048, hot 542 / 377; SwiGLU, 8192 rows, 8 experts, 2048 -> 2 x 2048 935 / 879.
-// (64 x 128 tiles, two or three to a CU, gained 0 to 5 % from the same and lost up to 7: not built.)  The error against 64 bits is no larger: fewer terms
-// meet in one chain of roundings.
+// 64 x 128 tiles: 1, 2 and 3 on a CU take 154, 255 and 342 us (K = 4096); 4096 rows, 8 experts, 4096 -> 1024 329 / 274, 2048 -> 1024 167 / 142, 1536 ->
+// 1024 with SiLU 131 / 114; 2100 rows, 5 experts, 2048 -> 2048 170 / 148.  The error against 64 bits is no larger: fewer terms meet in one chain of
+// roundings.
 //
-// Pieces of each of `rest` tiles: two pairs of slices to a piece at least, and the shortest of this model in us / 9: a pair of slices takes 4 us of a
-// lone block, 1.75 times that with more pieces than CUs, a piece's 64 KB of sums 0.025 us of everybody's bandwidth, the second launch 6.
+// Pieces of each of `rest` tiles of BM rows: two pairs of slices to a piece at least, and the shortest of this model in us / 9: a pair of slices takes
+// 4 us (BM = 64: 2) of a lone block, 1.75 times that (2) with more pieces than CUs, 64 KB of sums 0.025 us of everybody's bandwidth, the second
+// launch 6.
 // Integers: host and device agree.
 typedef TileF32x3<128, 128, 2, 2> TileF32Large;         // wave tile 64 x 64
-constexpr int kF32x3CutTile = 128 * 128, kF32x3PieceBytes = 128 * 128 * 4, kF32x3PairCost = 36;
+template <int BM>
 __host__ __device__ inline int f32x3_split_pieces(int rest, int pairs, int blocks, int* cost = nullptr) {
-    int best = 1, least = kF32x3PairCost * pairs;
+    constexpr int pair = BM == 128 ? 36 : 18, two = BM == 128 ? 7 : 8;
+    int best = 1, least = pair * pairs;
     for (int s = 2; s * rest <= 2 * blocks && 2 * s <= pairs; ++s) {
-        const int loop = (kF32x3PairCost * pairs + s - 1) / s;
-        const int c = (s * rest > blocks ? loop * 7 / 4 : loop) + rest * s * 2 / 9 + 54;
+        const int loop = (pair * pairs + s - 1) / s;
+        const int c = (s * rest > blocks ? loop * two / 4 : loop) + rest * s * (BM / 64) / 9 + 54;
         if (c < least) {
             least = c;
             best = s;
@@ -60,10 +66,11 @@ __host__ __device__ inline int f32x3_split_pieces(int rest, int pairs, int block
     if (cost) *cost = least;
     return best;
 }
+constexpr int f32x3_piece_bytes(int bm) { return bm * 128 * 4; }
 // a 32 x 32 block of a piece's sums, [quad][lane]
 template <typename TL>
 __device__ __forceinline__ f32x4* f32x3_sums(SplitWorkspace* ws, int piece, int row_block, int col_block) {
-    return reinterpret_cast<f32x4*>(reinterpret_cast<uint8_t*>(ws) + kSplitHeaderBytes + (int64_t)piece * kF32x3PieceBytes) +
+    return reinterpret_cast<f32x4*>(reinterpret_cast<uint8_t*>(ws) + kSplitHeaderBytes + (int64_t)piece * f32x3_piece_bytes(TL::BM)) +
            (row_block * (TL::BN / 32) + col_block) * 4 * kWave;
 }
 
@@ -122,7 +129,7 @@ template <typename TL, int EPI, bool NCONT, bool A_SILU>
 __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const GemmParams p) {
     constexpr int BM = TL::BM, BN = TL::BN, NT = TL::NT, BK = TL::BK;
     constexpr int FM = TL::FM, FN = TL::FN, TM = TL::TM, TN = TL::TN;
-    constexpr bool SWIGLU = EPI == FMOE_EPI_SWIGLU, CUT = BM * BN == kF32x3CutTile;
+    constexpr bool SWIGLU = EPI == FMOE_EPI_SWIGLU, CUT = TL::template kCut<SWIGLU>;
     constexpr int BN_OUT = SWIGLU ? BN / 2 : BN;
     constexpr int XP = BM * 4 / NT, WP = BN * 4 / NT;       // units of 8 values a thread brings in per slice
     static_assert(EPI != FMOE_EPI_SWIGLU || FN % 2 == 0, "gate and up fragments come in pairs");
@@ -141,7 +148,7 @@ __global__ __launch_bounds__(TL::NT, 2) void grouped_gemm_f32x3_kernel(const Gem
     const int pairs = (p.K + 2 * BK - 1) / (2 * BK);
     const bool here = CUT && p.split_ws ? tile.locate(p, BM, [&](int64_t total_tiles) -> int64_t {
         const SplitDeal deal((int)total_tiles, p.split_slots, blockIdx.x % kNumXcd, pairs,
-                             [](int rest, int pairs, int blocks) { return f32x3_split_pieces(rest, pairs, blocks); });
+                             [](int rest, int pairs, int blocks) { return f32x3_split_pieces<BM>(rest, pairs, blocks); });
         if (blockIdx.x == 0 && tid == 0) {      // (offsets that overlap name more tiles than the grid has blocks: nothing is added up then)
             p.split_ws->tiles = deal.pieces > 1 && deal.count * kNumXcd <= (int)gridDim.x ? deal.rest : 0;
             p.split_ws->pieces = deal.pieces;

@@ -1224,15 +1224,18 @@ def test_fp32_on_bf16_matrix_cores(E, rows, K, N, layout, epi, tile, case):
             assert bool(((got - want).abs() <= err).cpu()[near].all())
 
 
-@pytest.mark.parametrize("lens,K,N,layout,epi", [
-    ([2048] * 3 + [2049], 1024, 1024, "nk", 0),             # two whole rounds and eight tiles of a row
-    ([0, 4000, 2500, 2100, 3], 996, 1020, "kn", 1), ([4000, 2500, 2100, 130], 1028, 964, "nk", "silu"),
-    ([3000, 3500, 30], 772, 700, "nk", 2), ([3000, 3500, 30], 1024, 700, "kn", 2),
-    ([2100, 0, 500, 400, 33], 4100, 1000, "kn", 1), ([2100, 500, 400, 33], 4160, 904, "nk", "silu"),       # less than a round
-    ([500] * 66, 1024, 252, "nk", 0),                       # more than 64 experts
+@pytest.mark.parametrize("lens,K,N,layout,epi,tile", [
+    ([2048] * 3 + [2049], 1024, 1024, "nk", 0, 128),        # two whole rounds and eight tiles of a row
+    ([0, 4000, 2500, 2100, 3], 996, 1020, "kn", 1, 128), ([4000, 2500, 2100, 130], 1028, 964, "nk", "silu", 128),
+    ([3000, 3500, 30], 772, 700, "nk", 2, 128), ([3000, 3500, 30], 1024, 700, "kn", 2, 128),
+    ([2100, 0, 500, 400, 33], 4100, 1000, "kn", 1, 128), ([2100, 500, 400, 33], 4160, 904, "nk", "silu", 128),       # less than a round
+    ([500] * 66, 1024, 252, "nk", 0, 128),                  # more than 64 experts
+    ([512] * 7 + [513], 4096, 1024, "nk", 0, 64), ([520, 0, 500, 600, 1400, 1033], 1028, 1000, "kn", 1, 64),
+    ([520, 0, 500, 600, 1400, 1033], 996, 964, "nk", "silu", 64), ([520, 3, 500, 600, 1400, 1033], 2052, 900, "kn", "silu", 64),
+    ([512] * 8, 1024, 1024, "nk", 0, 64),                   # no tile left: nothing is cut
 ])
 @pytest.mark.parametrize("case", ["normal", "special"])
-def test_fp32_last_round_cut_along_k(lens, K, N, layout, epi, case):
+def test_fp32_last_round_cut_along_k(lens, K, N, layout, epi, tile, case):
     """Against float64, in the bound of test_fp32_on_bf16_matrix_cores (grouping the sums adds none to it); the same bits twice.  special: an
     infinity, a NaN and a value beyond 2^104 in single rows; the other rows do not see them."""
     from fast_moe_amd.kernels.hip import _lib, ops
@@ -1259,7 +1262,7 @@ def test_fp32_last_round_cut_along_k(lens, K, N, layout, epi, case):
     again = ops.grouped_gemm(off, x, ws[0], **kw)
     assert torch.equal(out.nan_to_num(7.0), again.nan_to_num(7.0))
     assert [n.split("<")[0].split("::")[-1] for n in ran] == ["grouped_gemm_f32x3_kernel", "f32x3_reduce_kernel"], ran
-    assert "TileF32x3<128, 128" in ran[0], ran
+    assert f"TileF32x3<{tile}, 128" in ran[0], ran
     unit = (K + 4) * 2.0 ** -24 + (2.0 ** -21 if a_silu else 0)         # (a rounding for the bias)
     for e in range(E):
         lo, hi = int(off[e]), int(off[e + 1])

@@ -9,11 +9,11 @@ PROGRAM = r"""
 #include <vector>
 #include "gemm_f32x3.h"
 
-int check(int total, int slots, int pairs, bool f32) {
+int check(int total, int slots, int pairs, int f32) {
     std::vector<std::vector<int>> seen(total, std::vector<int>(pairs, 0));
     std::vector<int> pieces_seen(2 * fmoe::kSplitMost, 0);
     for (int xcd = 0; xcd < 8; ++xcd) {
-        const fmoe::SplitDeal d = f32 ? fmoe::SplitDeal(total, slots, xcd, pairs, [](int r, int p, int b) { return fmoe::f32x3_split_pieces(r, p, b); })
+        const fmoe::SplitDeal d = f32 ? fmoe::SplitDeal(total, slots, xcd, pairs, [&](int r, int p, int b) { return f32 == 128 ? fmoe::f32x3_split_pieces<128>(r, p, b) : fmoe::f32x3_split_pieces<64>(r, p, b); })
                                       : fmoe::SplitDeal(total, slots, xcd, pairs);
         if (f32 && d.count > (total / (8 * slots) + 2) * slots) return printf("%d blocks of an XCD\n", d.count), 1;   // the launch's grid
         for (int j = 0; j < d.count; ++j) {
@@ -41,7 +41,7 @@ int main() {
     for (int slots : {32, 31, 4, 1})
         for (int pairs : {4, 5, 16, 61, 64, 200})
             for (int total = 0; total <= 40 * slots; total += total < 300 ? 1 : 37)
-                if (check(total, slots, pairs, false) || check(total, slots, pairs, true)) return printf("total %d, slots %d, pairs %d\n", total, slots, pairs), 1;
+                if (check(total, slots, pairs, 0) || check(total, slots, pairs, 64) || check(total, slots, pairs, 128)) return printf("total %d, slots %d, pairs %d\n", total, slots, pairs), 1;
     return 0;
 }
 """
