@@ -535,12 +535,13 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         const u32x4 lo = *reinterpret_cast<const u32x4*>(base + lo_at), hi = *reinterpret_cast<const u32x4*>(base + hi_at);
         return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
     };
-    // bf16 with k contiguous: 16 x 16 x 32 MFMAs.  Under the chip's power cap a chain of them sustains 2050 TFLOP/s where one of 32 x 32 x 16 sustains
+    // bf16 with k contiguous on tall tiles: 16 x 16 x 32 MFMAs.  (The four waves of a 64-row tile wait for loads and LDS, not for power: 600 rows, 12
+    // experts, 2368 -> 2 x 704 22.3 us with 32 x 32 x 16 ones, 27.0 with these; 700 rows, 8 experts, 4096 -> 2048 37.3 / 41.0.)  Under the chip's power cap a chain of them sustains 2050 TFLOP/s where one of 32 x 32 x 16 sustains
     // 1805 (half the accumulator traffic for a product).  A wave's 32 x 32 block of the output is four of them, two column blocks
     // a and two row blocks b.  Lane group g = lane / 16 of block a holds the four columns 16 a + 8 (g % 2) + 4 (g / 2) .. + 3 (the
     // order in which the weight rows are read below), so that exchanging lane groups between the row blocks (v_permlane16_swap,
     // behind the main loop) leaves the sums as v_mfma_f32_32x32x16_bf16 would: one layout for the epilogue.
-    constexpr bool B16 = !FP8 && !WTR && !XTR;
+    constexpr bool B16 = !FP8 && !WTR && !XTR && BM >= 256;
     constexpr int FN16 = 2 * FN, HX = FM;
     const int kquarter = lane >> 4;
     const int wfrag_lane16 = 8 * ((lane >> 2) & 1) + 4 * ((lane >> 3) & 1) + (lane & 3);      // weight row of this lane in a block of 16
@@ -965,8 +966,8 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 if (sparse) tile_steps(std::integral_constant<int, 1>{}, std::integral_constant<bool, SPARSE>{});
                 else tile_steps(std::integral_constant<int, 1>{}, std::false_type{});
             }
-        } else if constexpr (PAIR && WTR) {
-            // transposing reads (WTR, XTR): 32 x 32 x 16 MFMAs.  (On 16 x 16 x 32 ones, rolling as above, the weight gradients of 131072 rows,
+        } else if constexpr (PAIR && !FP8) {
+            // transposing reads (WTR, XTR) and 64-row tiles: 32 x 32 x 16 MFMAs.  (On 16 x 16 x 32 ones, rolling as above, the weight gradients of 131072 rows,
             // 64 experts, 2048 x 1408 take 2.10 ms for the two where these take 2.06, the input gradients 1.95 against 1.92: the LDS, which serves
             // transposing reads at two thirds of the rate of others, is the limit there, and the next item's weights come in one bunch.)
             // Software pipeline over "blocks" (half a K-slice: one 16-byte chunk per row and
@@ -991,7 +992,8 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 const int chunk = 2 * sub + khalf;
 #pragma unroll
                 for (int fn = 0; fn < FN; ++fn) {
-                    wf[fn] = read_tr8<1024>(sw + wtr_off[fn] + sub * 4096);
+                    if constexpr (WTR) wf[fn] = read_tr8<1024>(sw + wtr_off[fn] + sub * 4096);
+                    else wf[fn] = *reinterpret_cast<const bf16x8*>(sw + lds_off64((SWIGLU ? wn * (TN / 2) : wn * TN) + (lane & 31), chunk) + wq_block(fn));
                 }
 #pragma unroll
                 for (int fm = 0; fm < ACT; ++fm) {
