@@ -440,7 +440,7 @@ PyObject* py_gate_softmax(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // (scores [T, E], x [T, D], w1 [E, D, H], bias1, w2 [E, H, O], bias2, k, mode, epilogue1, stream) -> [T, O]:
 // routing, the gather GEMM with its activation, the second GEMM, the merge.  With scores None, a gate's weight [E, D] and its bias [E] or None
-// behind the stream: where the gate and the routing are one launch (fmoe_gate_route_pays)
+// behind the stream: the gate as fmoe_gate_softmax (where that pays), in the routing's launch where fmoe_gate_route_pays
 PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (n != 10 && n != 12) return none();
@@ -460,7 +460,8 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     char* base = nullptr;
     size_t at_ws = 0, ws_bytes = 0;
     int64_t *topk_idx = nullptr, *lengths = nullptr, *offsets = nullptr, *gate_index = nullptr, *token_index = nullptr, *reverse = nullptr;
-    void* gates = nullptr;
+    void *gates = nullptr, *gate_scores = nullptr;
+    bool one_launch = false;
     fmoe_gemm_desc up, down;
     Combine merge;
     const char* what = "fmoe_route_topk";
@@ -475,9 +476,8 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
             const int64_t T = x.size(0), E = scores.size(gate ? 0 : 1);
             if (w1.size(0) != E || w2.size(0) != E) return false;
             if (gate) {
-                if (!gate_ok(x, scores, gate_bias, &x_data, &data, &gate_bias_data) || k < 1 || k > E ||
-                    !gate_route_pays(dtype_code(x.scalar_type()), T, (int)x.size(1), (int)E, (int)k))
-                    return false;
+                if (!gate_ok(x, scores, gate_bias, &x_data, &data, &gate_bias_data) || k < 1 || k > E) return false;
+                one_launch = gate_route_pays(dtype_code(x.scalar_type()), T, (int)x.size(1), (int)E, (int)k) != 0;
             } else if (scores.size(0) != T || !route_ok(scores, k, &data)) {
                 return false;
             }
@@ -489,10 +489,11 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 bytes += ((size_t)(n * size) + 255) & ~(size_t)255;
                 return at;
             };
-            ws_bytes = gate ? 0 : route_workspace_bytes(T, (int)E, (int)k);
+            ws_bytes = one_launch ? 0 : route_workspace_bytes(T, (int)E, (int)k);
             const size_t at_topk = take(R, 8), at_lengths = take(E, 8), at_offsets = take(E + 1, 8), at_gate = take(R, 8);
             const size_t at_token = take(R, 8), at_reverse = take(R, 8), at_gates = take(R, (int64_t)scores.element_size());
             at_ws = take((int64_t)ws_bytes, 1);
+            const size_t at_scores = take(gate && !one_launch ? T * E : 0, (int64_t)scores.element_size());
             const size_t at_hidden = take((R + kSlackRows) * H, row_size), at_rows = take((R + kSlackRows) * O, row_size);
             scratch = empty({(int64_t)bytes}, at::kByte, x);
             base = (char*)scratch.data_ptr();
@@ -503,6 +504,7 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
             token_index = (int64_t*)(base + at_token);
             reverse = (int64_t*)(base + at_reverse);
             gates = base + at_gates;
+            gate_scores = base + at_scores;
             GemmArgs g;
             g.offsets_data = offsets;
             g.a = x;
@@ -539,8 +541,16 @@ PyObject* py_mlp_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
             return true;
         },
         [&] {
-            const fmoe_gate g = {x_data, data, gate_bias_data, x.stride(0), dtype_code(x.scalar_type()), (int)x.size(1)};
-            if (const int rc = c_route_topk(gate ? &g : data, gate ? FMOE_SCORES_OF_GATE : dtype_code(scores.scalar_type()), merge.T,
+            const int code = dtype_code(scores.scalar_type());
+            const fmoe_gate g = {x_data, data, gate_bias_data, x.stride(0), code, (int)x.size(1)};
+            if (gate && !one_launch) {
+                what = "fmoe_gate_softmax";
+                if (const int rc = c_gate_softmax(x_data, code, merge.T, g.d, g.x_stride_row, data, gate_bias_data, (int)w1.size(0), gate_scores,
+                                                  (void*)stream))
+                    return rc;
+                what = "fmoe_route_topk";
+            }
+            if (const int rc = c_route_topk(one_launch ? (const void*)&g : gate ? gate_scores : data, one_launch ? FMOE_SCORES_OF_GATE : code, merge.T,
                                             (int)w1.size(0), (int)k, (int)mode, topk_idx, gates, lengths, offsets, gate_index, token_index,
                                             reverse, base + at_ws, ws_bytes, (void*)stream))
                 return rc;
