@@ -79,6 +79,146 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
+// The reciprocal scales of e4m3 operands that a lane's sums meet: of its rows, and of its columns, [fn][gp][q][j] <-> column nq + 8*q +
+// 4*khalf + j with nq = first column of register-quad pair gp of fragment fn.
+template <int FM, int FN, int TM, int TN, int EPI, bool ROWS32, bool ROW_IL>
+__device__ __forceinline__ void fetch_reciprocal_scales(const GemmParams& p, float (&rsa)[FM], float (&rsw)[EPI == FMOE_EPI_SWIGLU ? FN / 2 : FN][2][2][4],
+                                                        float (&rsw2)[EPI == FMOE_EPI_SWIGLU ? FN / 2 : FN][2][2][4], int expert, int n0, int64_t row0,
+                                                        int rows_valid, int wm, int wn, int lane) {
+    constexpr bool SWIGLU = EPI == FMOE_EPI_SWIGLU;
+    constexpr int FN_OUT = SWIGLU ? FN / 2 : FN;
+    asm volatile("" : "+v"(lane));      // (see gemm_epilogue)
+    wm = __builtin_amdgcn_readfirstlane(wm);
+    wn = __builtin_amdgcn_readfirstlane(wn);
+    const int khalf = lane >> 5;
+    auto frag_row = [&](int fm) -> int { return ROW_IL ? (fm * 2 + wm) * 32 : wm * TM + fm * 32; };
+    const int col0 = n0 + (SWIGLU ? wn * (TN / 2) : wn * TN);
+    bool row_ok[FM];
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) row_ok[fm] = frag_row(fm) + (lane & 31) < rows_valid;
+    // the activation scales of this lane's rows: all index loads, then all scale loads (two
+    // memory latencies, not two per row block)
+    typedef typename std::conditional<ROWS32, int32_t, int64_t>::type row_t;
+    row_t src[FM];
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm)
+        src[fm] = (row_t)(row0 + (row_ok[fm] ? frag_row(fm) + (lane & 31) : 0));
+    if (p.row_index) {
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm) {
+            if (ROWS32) src[fm] = reinterpret_cast<const int32_t*>(p.row_index)[2 * (int64_t)src[fm]];   // low half
+            else src[fm] = (row_t)p.row_index[src[fm]];
+        }
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm)
+            if (ROWS32) src[fm] = (row_t)div_index32(p, (int32_t)src[fm]);
+            else src[fm] = p.index_shift >= 0 ? (src[fm] >> p.index_shift) : src[fm] / (row_t)p.index_div;
+    }
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) {
+        const row_t last = (row_t)(p.a_rows - 1);
+        src[fm] = src[fm] < 0 ? 0 : (src[fm] > last ? last : src[fm]);
+    }
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) rsa[fm] = p.a_scale[src[fm]];
+    // The weight-scale loads go out right behind the activation-scale loads, before anything
+    // waits for either, so that the two round trips overlap (one memory latency per tile less;
+    // the raw values wait in the registers their reciprocals end up in).
+    constexpr int WCOLS = FN_OUT * 32;          // output columns of this wave
+    if (p.scale_vec && col0 + WCOLS <= p.N) {
+        // the wave's columns lie inside N: the 4 scales of a register quad in one 16-byte load
+        // from a wave-uniform base plus the lane half's 16 bytes plus a constant
+        const float* sb = p.b_scale + ((int64_t)expert * p.N + col0);
+        const float* sb2 = SWIGLU ? p.b2_scale + ((int64_t)expert * p.N + col0) : sb;
+        const int half4 = 4 * khalf;
+        typedef __attribute__((ext_vector_type(4))) float f32x4;
+#pragma unroll
+        for (int fn = 0; fn < FN_OUT; ++fn)
+#pragma unroll
+            for (int gp = 0; gp < 2; ++gp)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int c = fn * 32 + 16 * gp + 8 * q;
+                    const f32x4 s1 = *reinterpret_cast<const f32x4*>(sb + half4 + c);
+                    f32x4 s2 = s1;
+                    if (SWIGLU) s2 = *reinterpret_cast<const f32x4*>(sb2 + half4 + c);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        rsw[fn][gp][q][j] = s1[j];
+                        if (SWIGLU) rsw2[fn][gp][q][j] = s2[j];
+                    }
+                }
+    } else {
+        // the last column tile, or scale tensors off a 16-byte boundary: one clamped load a column
+#pragma unroll
+        for (int fn = 0; fn < FN_OUT; ++fn)
+#pragma unroll
+            for (int gp = 0; gp < 2; ++gp)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int n = col0 + fn * 32 + 16 * gp + 8 * q + 4 * khalf + j;
+                        const int nc = n < p.N ? n : p.N - 1;
+                        rsw[fn][gp][q][j] = p.b_scale[(int64_t)expert * p.N + nc];
+                        if (SWIGLU) rsw2[fn][gp][q][j] = p.b2_scale[(int64_t)expert * p.N + nc];
+                    }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // (v_rcp_f32 is exact on the powers of two the reference's scales are)
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) rsa[fm] = __builtin_amdgcn_rcpf(rsa[fm]);
+#pragma unroll
+    for (int fn = 0; fn < FN_OUT; ++fn)
+#pragma unroll
+        for (int gp = 0; gp < 2; ++gp)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    rsw[fn][gp][q][j] = __builtin_amdgcn_rcpf(rsw[fn][gp][q][j]);
+                    if (SWIGLU) rsw2[fn][gp][q][j] = __builtin_amdgcn_rcpf(rsw2[fn][gp][q][j]);
+                }
+}
+
+// Plain and SwiGLU: the sums divided by the scales in place, ahead of everything else an epilogue does.  The reciprocals of a SwiGLU wave's columns are
+// 32 registers, and beside rows on their way through LDS the kernels spill 70 to 90, whose reloads lie in the tile loop.  us, scales multiplied at
+// the sums' use / in place: 512 rows, 64 experts, 2048 -> 2 x 1408 90.2 / 73.5, plain 32.6 / 30.5; 8192 rows, 8 experts, 1024 -> 2 x 4096 89.2 /
+// 86.4; 30000 rows, 200 experts, 1024 -> 2 x 512 79.1 / 76.0.  SiLU keeps them: with a bias 64.2 / 66.7, 8192 rows, 8 experts, 1024 -> 4096.
+// whole: else the sums stay as they are (times one: a piece of a tile cut along K goes through here as well, as sums that two branches read
+// are not scaled in their own registers).
+constexpr bool divides_in_place(int epi) { return epi != FMOE_EPI_SILU; }
+template <int FM, int FN, int TM, int TN, int EPI, bool ROWS32, bool ROW_IL>
+__device__ __forceinline__ void divide_scales_out(const GemmParams& p, f32x16 (&acc)[FN][FM], int expert, int n0, int64_t row0, int rows_valid, int wm,
+                                                  int wn, int lane, bool whole = true) {
+    constexpr bool SWIGLU = EPI == FMOE_EPI_SWIGLU;
+    constexpr int FN_OUT = SWIGLU ? FN / 2 : FN;
+    float rsa[FM], rsw[FN_OUT][2][2][4], rsw2[FN_OUT][2][2][4];
+    fetch_reciprocal_scales<FM, FN, TM, TN, EPI, ROWS32, ROW_IL>(p, rsa, rsw, rsw2, expert, n0, row0, rows_valid, wm, wn, lane);
+    if (!whole) {
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm) rsa[fm] = 1.0f;
+#pragma unroll
+        for (int i = 0; i < FN_OUT * 16; ++i) {
+            rsw[i / 16][i / 8 % 2][i / 4 % 2][i % 4] = 1.0f;
+            if (SWIGLU) rsw2[i / 16][i / 8 % 2][i / 4 % 2][i % 4] = 1.0f;
+        }
+    }
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+        for (int fn = 0; fn < FN_OUT; ++fn)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    acc[fn][fm][4 * g + j] *= rsa[fm] * rsw[fn][g / 2][g % 2][j];
+                    if (SWIGLU) acc[fn + FN / 2][fm][4 * g + j] *= rsa[fm] * rsw2[fn][g / 2][g % 2][j];
+                }
+                __builtin_amdgcn_sched_barrier(0);      // (all products first is a register for each)
+            }
+}
+
 // MSC (e4m3): the scales were applied by the MFMAs themselves (power-of-two scales as block scales of
 // the instruction): acc already holds sum / (s_a * s_w) and the epilogue loads and multiplies nothing.
 template <int FM, int FN, int TM, int TN, bool FP8, int EPI, bool ALWAYS_VEC = false, bool ROWS32 = false,
@@ -120,103 +260,16 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
     };
     // first tile row of the wave's row block fm
     auto frag_row = [&](int fm) -> int { return ROW_IL ? (fm * 2 + wm) * 32 : wm * TM + fm * 32; };
-    float rsa[FM];
     bool row_ok[FM];
 #pragma unroll
-    for (int fm = 0; fm < FM; ++fm) {
-        row_ok[fm] = frag_row(fm) + (lane & 31) < rows_valid;
-        rsa[fm] = 1.0f;
-    }
-    // per-column reciprocal weight scales of this lane (e4m3): [fn][gp][q][j] <-> column
-    // nq + 8*q + 4*khalf + j with nq = first column of register-quad pair gp of fragment fn
-    float rsw[FN_OUT][2][2][4], rsw2[FN_OUT][2][2][4];
+    for (int fm = 0; fm < FM; ++fm) row_ok[fm] = frag_row(fm) + (lane & 31) < rows_valid;
     const int col0 = n0 + (SWIGLU ? wn * (TN / 2) : wn * TN);
-    constexpr bool SCALE = FP8 && !MSC;         // divide the scales out here
-    if (SCALE) {
-        // the activation scales of this lane's rows: all index loads, then all scale loads (two
-        // memory latencies, not two per row block)
-        typedef typename std::conditional<ROWS32, int32_t, int64_t>::type row_t;
-        row_t src[FM];
-#pragma unroll
-        for (int fm = 0; fm < FM; ++fm)
-            src[fm] = (row_t)(row0 + (row_ok[fm] ? frag_row(fm) + (lane & 31) : 0));
-        if (p.row_index) {
-#pragma unroll
-            for (int fm = 0; fm < FM; ++fm) {
-                if (ROWS32) src[fm] = reinterpret_cast<const int32_t*>(p.row_index)[2 * (int64_t)src[fm]];   // low half
-                else src[fm] = (row_t)p.row_index[src[fm]];
-            }
-#pragma unroll
-            for (int fm = 0; fm < FM; ++fm)
-                if (ROWS32) src[fm] = (row_t)div_index32(p, (int32_t)src[fm]);
-                else src[fm] = p.index_shift >= 0 ? (src[fm] >> p.index_shift) : src[fm] / (row_t)p.index_div;
-        }
-#pragma unroll
-        for (int fm = 0; fm < FM; ++fm) {
-            const row_t last = (row_t)(p.a_rows - 1);
-            src[fm] = src[fm] < 0 ? 0 : (src[fm] > last ? last : src[fm]);
-        }
-#pragma unroll
-        for (int fm = 0; fm < FM; ++fm) rsa[fm] = p.a_scale[src[fm]];
-        // The weight-scale loads go out right behind the activation-scale loads, before anything
-        // waits for either, so that the two round trips overlap (one memory latency per tile less;
-        // the raw values wait in the registers their reciprocals end up in).
-        constexpr int WCOLS = FN_OUT * 32;          // output columns of this wave
-        if (p.scale_vec && col0 + WCOLS <= p.N) {
-            // the wave's columns lie inside N: the 4 scales of a register quad in one 16-byte load
-            // from a wave-uniform base plus the lane half's 16 bytes plus a constant
-            const float* sb = p.b_scale + ((int64_t)expert * p.N + col0);
-            const float* sb2 = SWIGLU ? p.b2_scale + ((int64_t)expert * p.N + col0) : sb;
-            const int half4 = 4 * khalf;
-            typedef __attribute__((ext_vector_type(4))) float f32x4;
-#pragma unroll
-            for (int fn = 0; fn < FN_OUT; ++fn)
-#pragma unroll
-                for (int gp = 0; gp < 2; ++gp)
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        const int c = fn * 32 + 16 * gp + 8 * q;
-                        const f32x4 s1 = *reinterpret_cast<const f32x4*>(sb + half4 + c);
-                        f32x4 s2 = s1;
-                        if (SWIGLU) s2 = *reinterpret_cast<const f32x4*>(sb2 + half4 + c);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            rsw[fn][gp][q][j] = s1[j];
-                            rsw2[fn][gp][q][j] = s2[j];
-                        }
-                    }
-        } else {
-            // the last column tile, or scale tensors off a 16-byte boundary: one clamped load a column
-#pragma unroll
-            for (int fn = 0; fn < FN_OUT; ++fn)
-#pragma unroll
-                for (int gp = 0; gp < 2; ++gp)
-#pragma unroll
-                    for (int q = 0; q < 2; ++q)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const int n = col0 + fn * 32 + 16 * gp + 8 * q + 4 * khalf + j;
-                            const int nc = n < p.N ? n : p.N - 1;
-                            rsw[fn][gp][q][j] = rsw2[fn][gp][q][j] = p.b_scale[(int64_t)expert * p.N + nc];
-                            if (SWIGLU) rsw2[fn][gp][q][j] = p.b2_scale[(int64_t)expert * p.N + nc];
-                        }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        // (v_rcp_f32 is exact on the powers of two the reference's scales are)
-#pragma unroll
-        for (int fm = 0; fm < FM; ++fm) rsa[fm] = __builtin_amdgcn_rcpf(rsa[fm]);
-#pragma unroll
-        for (int fn = 0; fn < FN_OUT; ++fn)
-#pragma unroll
-            for (int gp = 0; gp < 2; ++gp)
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        rsw[fn][gp][q][j] = __builtin_amdgcn_rcpf(rsw[fn][gp][q][j]);
-                        if (SWIGLU) rsw2[fn][gp][q][j] = __builtin_amdgcn_rcpf(rsw2[fn][gp][q][j]);
-                    }
-    }
+    constexpr bool SCALE = FP8 && !MSC && !divides_in_place(EPI);       // times the reciprocal scales at their use
+    float rsa[FM], rsw[FN_OUT][2][2][4], rsw2[FN_OUT][2][2][4];
+    if constexpr (SCALE)
+        fetch_reciprocal_scales<FM, FN, TM, TN, EPI, ROWS32, ROW_IL>(p, rsa, rsw, rsw2, expert, n0, row0, rows_valid, wm, wn, lane);
+    else if constexpr (FP8 && !MSC)
+        divide_scales_out<FM, FN, TM, TN, EPI, ROWS32, ROW_IL>(p, acc, expert, n0, row0, rows_valid, wm, wn, lane);
     // the bias-free form (FastMoE's SwiGLU experts, every fp8 call without bias) skips the adds
     auto run = [&](auto has_bias_c, auto has_aux_c) {
         constexpr bool HAS_BIAS = decltype(has_bias_c)::value;
@@ -225,7 +278,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
         float bv[FN_OUT][2][2][4], bv2[FN_OUT][2][2][4];
         // with a bias, at least one of the two pointers is set: both loads go through a valid
         // pointer and a select drops the value of a missing one (a branch per load would make
-        // every load wait for the one before)
+        // every load wait for the one before).  Sums that were divided in place take a missing one as
+        // -0, which changes no sum, instead of a branch at every pair of columns.
+        constexpr bool SELECT = FP8 && !MSC && !SCALE;
+        constexpr float NO_BIAS = SELECT ? -0.0f : 0.0f;
         const uint16_t* bias_a = p.bias ? p.bias : p.bias2;
         const uint16_t* bias_b = p.bias2 ? p.bias2 : p.bias;
 #pragma unroll
@@ -241,11 +297,11 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                         bv[fn][gp][q][j] = bv2[fn][gp][q][j] = 0.0f;
                         if (HAS_BIAS) {
                             const float a = bf16_bits_to_f32(bias_a[bias_row + nc]);
-                            bv[fn][gp][q][j] = p.bias ? a : 0.0f;
+                            bv[fn][gp][q][j] = p.bias ? a : NO_BIAS;
                         }
                         if (HAS_BIAS && SWIGLU) {
                             const float b = bf16_bits_to_f32(bias_b[bias_row + nc]);
-                            bv2[fn][gp][q][j] = p.bias2 ? b : 0.0f;
+                            bv2[fn][gp][q][j] = p.bias2 ? b : NO_BIAS;
                         }
                     }
         __builtin_amdgcn_sched_barrier(0);
@@ -315,18 +371,13 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
 #pragma unroll
                             for (int j = 0; j < 4; j += 2) {        // two columns at a time: one conversion instruction rounds a pair
                                 const int v = 4 * (2 * gp + q) + j;
-                                auto branch = [&](float a, float b, const float (&sw)[4], const float (&bias)[4], const void* given) -> uint32_t {
-                                    if (FP8) {
-                                        if (SCALE) {
-                                            a *= rsa[fm] * sw[j];
-                                            b *= rsa[fm] * sw[j + 1];
-                                        }
-                                        if (HAS_BIAS && given) {
-                                            rbf2(a, b);
-                                            a += bias[j];
-                                            b += bias[j + 1];
-                                        }
-                                    } else if (HAS_BIAS) {
+                                auto branch = [&](float a, float b, const float (&bias)[4], const void* given) -> uint32_t {
+                                    if (SCALE) {        // (no SwiGLU: the first half's columns)
+                                        a *= rsa[fm] * rsw[fn][gp][q][j];
+                                        b *= rsa[fm] * rsw[fn][gp][q][j + 1];
+                                    }
+                                    if (HAS_BIAS && (!FP8 || SELECT || given)) {
+                                        if (FP8) rbf2(a, b);
                                         a += bias[j];
                                         b += bias[j + 1];
                                     }
@@ -334,10 +385,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                                 };
                                 auto low = [](uint32_t u) { return __uint_as_float(u << 16); };
                                 auto high = [](uint32_t u) { return __uint_as_float(u & 0xffff0000u); };
-                                uint32_t y = kind == 2 ? 0u : branch(acc[fn][fm][v], acc[fn][fm][v + 1], rsw[fn][gp][q], bv[fn][gp][q], p.bias);
+                                uint32_t y = kind == 2 ? 0u : branch(acc[fn][fm][v], acc[fn][fm][v + 1], bv[fn][gp][q], p.bias);
                                 uint32_t u = 0;
                                 if (SWIGLU && kind != 1)
-                                    u = branch(acc[fn + FN / 2][fm][v], acc[fn + FN / 2][fm][v + 1], rsw2[fn][gp][q], bv2[fn][gp][q], p.bias2);
+                                    u = branch(acc[fn + FN / 2][fm][v], acc[fn + FN / 2][fm][v + 1], bv2[fn][gp][q], p.bias2);
                                 if (kind == 2) y = u;
                                 if (EPI == FMOE_EPI_SILU || (SWIGLU && kind == 0)) y = pack_bf16(fast_silu_f32(low(y)), fast_silu_f32(high(y)));
                                 if (SWIGLU && kind == 0) y = pack_bf16(low(y) * low(u), high(y) * high(u));
@@ -475,10 +526,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                                     rbf2(ya, yb);
                                 }
                                 if (SWIGLU) {
-                                    if (SCALE) {
-                                        ua *= rsa[fm] * rsw2[fn][gp][q][j];
-                                        ub *= rsa[fm] * rsw2[fn][gp][q][j + 1];
-                                    }
                                     rbf2(ua, ub);
                                     if (HAS_BIAS && p.bias2) {
                                         ua += bv2[fn][gp][q][j];

@@ -1386,7 +1386,11 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         }
         if constexpr (MSC) mfma_results_guard();    // the last MFMAs' results are read by VALU code from here on
         FMOE_TRACE_STAMP(1);
+        constexpr bool DIVIDED = KSPLIT && FP8 && !MSC && divides_in_place(EPI);     // here instead of in the epilogue
         if constexpr (KSPLIT) {
+            if constexpr (DIVIDED)
+                divide_scales_out<FM, FN, TM, TN, EPI, PAIR, ROW_IL>(p, acc, cur.expert, cur.nt * BN_OUT, cur.row0, cur.rows_valid, wm, wn, lane,
+                                                                     cur.piece < 0);
             if (cur.piece >= 0) {       // the block's last
                 SplitTile* const info = p.split_ws->tile + cur.piece % split.rest;
                 if (cur.k0 == 0 && tid == 0) *info = SplitTile{__builtin_amdgcn_readfirstlane(cur.expert), cur.nt, (int)cur.row0, cur.rows_valid};
@@ -1438,12 +1442,12 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         uint8_t* const stage = smem + (cslot == 0 ? STAGES - 1 : cslot - 1) * TL::STAGE_BYTES + wave * kEpilogueStageBytes;
         auto hooks = make_hooks(scales_behind_block0, convert_rows);
 #ifdef FMOE_TRACE
-        gemm_epilogue<FM, FN, TM, TN, FP8, EPI, true, PAIR, XTR, ROW_IL, decltype(hooks), MSC>(
+        gemm_epilogue<FM, FN, TM, TN, FP8, EPI, true, PAIR, XTR, ROW_IL, decltype(hooks), MSC || DIVIDED>(
             p, acc, done.expert, done.nt * BN_OUT, done.row0, done.rows_valid, wm, wn, lane, stage, hooks,
             (p.trace && tile_i < 32 && (wave == 0 || wave == NW / 2)) ? tstamp + 12 : nullptr);
 #else
         static_assert(kEpilogueStoresUnconditional, "skip_wait needs an epilogue whose stores are all issued");
-        gemm_epilogue<FM, FN, TM, TN, FP8, EPI, kEpilogueStoresUnconditional, PAIR, XTR, ROW_IL, decltype(hooks), MSC>(
+        gemm_epilogue<FM, FN, TM, TN, FP8, EPI, kEpilogueStoresUnconditional, PAIR, XTR, ROW_IL, decltype(hooks), MSC || DIVIDED>(
             p, acc, done.expert, done.nt * BN_OUT, done.row0, done.rows_valid, wm, wn, lane, stage, hooks);
 #endif
 #ifdef FMOE_TRACE

@@ -1019,6 +1019,34 @@ def test_scales_applied_by_the_mfma_equal_scales_divided_out_in_the_epilogue(E, 
     assert torch.equal(again.view(torch.int16), folded.view(torch.int16))
 
 
+@pytest.mark.parametrize("E,rows,K,N,epi", [
+    (8, 4096, 1024, 712, 2), (8, 4096, 1024, 712, 0), (8, 4096, 832, 520, 2), (8, 4000, 1040, 264, 2),     # the ring, with four slots, with a tail of K
+    (130, 40000, 256, 264, 2), (6, 2000, 8192, 712, 2), (6, 2000, 8192, 712, 0),                         # many experts; cut along K
+    (64, 512, 2048, 712, 2), (64, 512, 2048, 712, 0), (5, 300, 528, 136, 2),                             # streamed; 64-row tiles
+])
+@pytest.mark.parametrize("given", ["none", "first", "second", "both"])
+def test_scales_divided_out_with_either_bias(E, rows, K, N, epi, given):
+    """Scales divided out in the epilogue against scales in the MFMAs, bit for bit (see above), zeros' signs included: with one bias of two, which
+    the columns without one do not see."""
+    from fast_moe_amd.kernels.hip import ops
+    if epi != 2 and given in ("second", "both"):
+        pytest.skip("one bias")
+    g = torch.Generator(device="cuda").manual_seed(E + K)
+    x = torch.randn(rows, K, generator=g, device="cuda")
+    x[::9] = 0.0
+    x[1::9] = -2.0 ** -60            # products that round to -0 and 0
+    qx, sx = ops.quant_rows_fp8(x.to(BF16))
+    qw = [ops.quant_rows_fp8((torch.randn(E, N, K, generator=g, device="cuda") * K ** -0.5).to(BF16)) for _ in range(2)]
+    cuts = torch.randint(0, rows, (E - 1,), generator=g, device="cuda").sort().values
+    off = torch.cat([cuts.new_zeros(1), cuts, cuts.new_full((1,), rows)])
+    bias = [torch.randn(E, N, generator=g, device="cuda").to(BF16) if given in (side, "both") else None for side in ("first", "second")]
+    kw = dict(total_rows=rows, a_scale=sx, b_scale=qw[0][1], epilogue=epi, bias=bias[0])
+    if epi == 2:
+        kw.update(b2=qw[1][0].permute(0, 2, 1), b2_scale=qw[1][1], bias2=bias[1])
+    divided, folded = (ops.grouped_gemm(off, qx, qw[0][0].permute(0, 2, 1), scales_pow2=pow2, **kw) for pow2 in (False, True))
+    assert torch.equal(divided.view(torch.int16), folded.view(torch.int16))
+
+
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
     (3, 700, 72, 264, "nk", 0), (3, 700, 120, 136, "kn", 0),        # one pair of K-slices and the shortest / longest rest
     (2, 1000, 1000, 520, "nk", 2), (2, 1000, 1000, 520, "kn", 2),
