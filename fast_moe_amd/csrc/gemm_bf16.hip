@@ -1,4 +1,4 @@
-// bf16 instantiations of the jagged GEMM (v_mfma_f32_32x32x16_bf16).
+// bf16 instantiations of the jagged GEMM.
 #include "gemm_kernel.h"
 
 namespace fmoe {

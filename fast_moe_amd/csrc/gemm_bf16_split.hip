@@ -5,8 +5,12 @@ namespace fmoe {
 
 template <int EPI, bool WTR>
 static int launch(const GemmParams& p, hipStream_t stream) {
-    if (p.K % 64 || p.E > TileRing5::kMaxExperts) return launch_ring_cfg<RingSplitCfg<4>, false, EPI, WTR, false, false, false, true>(p, stream);
-    return launch_ring_cfg<RingSplitCfg<1>, false, EPI, WTR>(p, stream);
+    const bool tail = p.K % 64 || p.E > TileRing5::kMaxExperts;
+    if constexpr (WTR) {
+        if (tail) return launch_ring_cfg<RingSplitCfg<4>, false, EPI, true, false, false, false, true>(p, stream);
+        return launch_ring_cfg<RingSplitCfg<1>, false, EPI, true>(p, stream);
+    }
+    return tail ? launch_ring_bf16<RingSplitCfg<4>, EPI, true>(p, stream) : launch_ring_bf16<RingSplitCfg<1>, EPI>(p, stream);
 }
 
 template <int EPI>

@@ -7,7 +7,7 @@ template <int EPI>
 static int launch(const GemmParams& p, hipStream_t stream) {
     if (p.b_sn == 1 && p.b_sk != 1)
         return launch_ring_cfg<TileRing5W, false, EPI, true, false, false, false, true>(p, stream);
-    return launch_ring_cfg<TileRing5W, false, EPI, false, false, false, false, true>(p, stream);
+    return launch_ring_bf16<TileRing5W, EPI, true>(p, stream);
 }
 
 int run_ring_tail_bf16(const GemmParams& p, int epilogue, hipStream_t stream) {

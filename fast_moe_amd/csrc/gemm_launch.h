@@ -283,6 +283,29 @@ inline bool split_before_direct(const GemmParams& p, int esize, int epilogue) {
            (p.K > 3584 || most_row_tiles(p.total_rows, p.E, 64) * direct_columns(p.N, epilogue == FMOE_EPI_SWIGLU) > compute_units());
 }
 
+// bf16 tall ring with k contiguous: whether a launch, row tiles halfway between the fewest and the most that the row count allows, draws the chip's power
+// cap in its main loops.  There the lower draw of 16 x 16 x 32 MFMAs is worth 1 to 4 %; below it their finer issue between the LDS reads costs up to
+// 12 %, and a tile's end costs more (the exchange of lane groups).  us, 32 x 32 x 16 / 16 x 16 x 32 on two cards, 8 experts unless stated:
+//   plain   4096 rows, 1024 -> 1024 24.3 / 26.5, 2048 -> 1024 39.5 / 43.7    16384, 1024 -> 3072 100.6 / 100.7, 106.2 / 109.1, -> 4096 126.6 / 125.3,
+//           132.7 / 136.1    32768, 1024 -> 3072 184.5 / 181.7, 192.6 / 193.9, -> 5120 313 / 311, 323 / 318, 512 -> 3072 105.4 / 104.8, 113.6 / 113.9
+//           8192, 2048 -> 3072 93.1 / 92.9, 98.3 / 96.2, 4096 -> 1024 74.9 / 80.3    12288, 4096 -> 1024 90.9 / 89.5, 95.3 / 92.3, 2048 -> 1024 51.1 / 51.7
+//           16384, 2048 -> 1024 86.1 / 88.4, -> 2048 136.7 / 136.5, 143.3 / 140.6, 4096 -> 1024 125.8 / 122.8, 128.9 / 124.2
+//           24 experts, Zipf, 8192, 2048 -> 2048 88.0 / 89.1    12 experts, 9189, 1000 -> 1024 32.5 / 33.3, 2600 -> 2600 135.7 / 131.1, 142.2 / 134.4
+//   SwiGLU  16384, 1024 -> 2 x 2048 131.7 / 132.5, 140.6 / 146.5    32768, 1024 -> 2 x 1536 188.8 / 187.4, 200.8 / 206.6, -> 2 x 2560 309 / 305, 321 / 325
+//           16384, 2048 -> 2 x 1536 190.3 / 190.1, 197.5 / 204.1, -> 2 x 2048 241 / 239, 250 / 252    32768, 2048 -> 2 x 2560 577 / 564, 589 / 579
+//           16384, 4096 -> 2 x 512 127.2 / 124.5, 130.4 / 125.5    8192, 4096 -> 2 x 512 75.9 / 81.8    65536, 512 -> 2 x 2048 288.9 / 294.9
+// So by CUs' worths of K: 3072 from K of 2048 on (SwiGLU 4096), 6000 (8192) below.
+inline bool mfma16_pays(const GemmParams& p, bool swiglu) {
+    const int bn = swiglu ? 128 : 256, need = p.K >= (swiglu ? 4096 : 2048) ? 3072 : swiglu ? 8192 : 6000;
+    const int64_t n_tiles = (p.N + bn - 1) / bn, least = (p.total_rows + 255) / 256, most = most_row_tiles(p.total_rows, p.E, 256);
+    return (least + most) * n_tiles >= 2 * (int64_t)need * compute_units() / p.K && (!swiglu || p.K >= 1024);
+}
+template <typename TL, int EPI, bool KTAIL = false>
+int launch_ring_bf16(const GemmParams& p, hipStream_t stream) {
+    if (mfma16_pays(p, EPI == FMOE_EPI_SWIGLU)) return launch_ring_cfg<Mfma16<TL>, false, EPI, false, false, false, false, KTAIL>(p, stream);
+    return launch_ring_cfg<TL, false, EPI, false, false, false, false, KTAIL>(p, stream);
+}
+
 // The 5-slot ring needs every byte of a 160 KB LDS, an even number of K-slices per tile,
 // row numbers that fit 32 bits and few enough experts for the register tables.
 template <bool FP8, int EPI>
@@ -312,9 +335,9 @@ int launch_ring(const GemmParams& p, hipStream_t stream) {
     if (p.k_window) {                      // built for the weight gradient: bf16, no epilogue
         if constexpr (!FP8 && EPI == FMOE_EPI_NONE) {
             if (pair_ok && window_ok && p.E <= TileRing5::kMaxExperts)
-                return launch_ring_cfg<TileRing5, FP8, EPI, false, true>(p, stream);
+                return launch_ring_cfg<Mfma16<TileRing5>, FP8, EPI, false, true>(p, stream);
             if (pair_ok && window_ok && p.E <= TileRing5W::kMaxExperts)
-                return launch_ring_cfg<TileRing5W, FP8, EPI, false, true>(p, stream);
+                return launch_ring_cfg<Mfma16<TileRing5W>, FP8, EPI, false, true>(p, stream);
         }
         return launch_gemm<TileBig, FP8 ? kDtE4m3 : kDtBf16, EPI, kLoadChunks, false>(p, stream);
     }
@@ -326,9 +349,14 @@ int launch_ring(const GemmParams& p, hipStream_t stream) {
         if (p.scale_pow2 && pair_ok && p.E <= TileRing5W::kMaxExperts)
             return launch_ring_cfg<TileRing5W, FP8, EPI, false, false, false, true>(p, stream);
     }
-    if (pair_ok && p.E <= TileRing5::kMaxExperts) return launch_ring_cfg<TileRing5F, FP8, EPI>(p, stream);
-    if (pair_ok && p.E <= TileRing5M::kMaxExperts) return launch_ring_cfg<TileRing5M, FP8, EPI>(p, stream);
-    if (pair_ok && p.E <= TileRing5W::kMaxExperts) return launch_ring_cfg<TileRing5W, FP8, EPI>(p, stream);
+    auto go = [&](auto tile) {
+        typedef decltype(tile) TL;
+        if constexpr (FP8) return launch_ring_cfg<TL, true, EPI>(p, stream);
+        else return launch_ring_bf16<TL, EPI>(p, stream);
+    };
+    if (pair_ok && p.E <= TileRing5::kMaxExperts) return go(TileRing5F{});
+    if (pair_ok && p.E <= TileRing5M::kMaxExperts) return go(TileRing5M{});
+    if (pair_ok && p.E <= TileRing5W::kMaxExperts) return go(TileRing5W{});
     return launch_ring_cfg<TileRing4, FP8, EPI>(p, stream);
 }
 

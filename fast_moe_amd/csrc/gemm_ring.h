@@ -19,6 +19,7 @@ struct RingCfg {
     static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NREG = NREG_;
     static constexpr bool PAIR = NREG_ > 0;
     static constexpr bool KSPLIT = false;
+    static constexpr bool MFMA16 = !PAIR;           // bf16, k contiguous: 16 x 16 x 32 MFMAs
     static constexpr int AHEAD = AHEAD_;
     static constexpr int STAGES = PAIR ? 2 * AHEAD + 1 : 4;
     static constexpr int NW = WGM * WGN;
@@ -40,6 +41,12 @@ struct RingCfg {
 template <int NREG_>
 struct RingSplitCfg : RingCfg<256, 256, 2, 4, NREG_> {
     static constexpr bool KSPLIT = true;
+};
+
+// ... with 16 x 16 x 32 MFMAs on bf16 operands whose k is contiguous (mfma16_pays)
+template <typename TL>
+struct Mfma16 : TL {
+    static constexpr bool MFMA16 = true;
 };
 
 // One 16-byte-per-lane global -> LDS transfer from base + voff: a wave-uniform base in
@@ -535,13 +542,15 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
         const u32x4 lo = *reinterpret_cast<const u32x4*>(base + lo_at), hi = *reinterpret_cast<const u32x4*>(base + hi_at);
         return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
     };
-    // bf16 with k contiguous on tall tiles: 16 x 16 x 32 MFMAs.  (The four waves of a 64-row tile wait for loads and LDS, not for power: 600 rows, 12
-    // experts, 2368 -> 2 x 704 22.3 us with 32 x 32 x 16 ones, 27.0 with these; 700 rows, 8 experts, 4096 -> 2048 37.3 / 41.0.)  Under the chip's power cap a chain of them sustains 2050 TFLOP/s where one of 32 x 32 x 16 sustains
-    // 1805 (half the accumulator traffic for a product).  A wave's 32 x 32 block of the output is four of them, two column blocks
+    // bf16 with k contiguous, launches of tall tiles that reach the chip's power cap (mfma16_pays): 16 x 16 x 32 MFMAs.  There a chain of them
+    // sustains 2050 TFLOP/s where one of 32 x 32 x 16 sustains 1805 (half the accumulator traffic for a product).  (The four waves of a 64-row tile
+    // wait for loads and LDS, not for power: 600 rows, 12 experts, 2368 -> 2 x 704 22.3 us with 32 x 32 x 16 ones, 27.0 with these; 700 rows, 8
+    // experts, 4096 -> 2048 37.3 / 41.0.)  A wave's 32 x 32 block of the output is four of them, two column blocks
     // a and two row blocks b.  Lane group g = lane / 16 of block a holds the four columns 16 a + 8 (g % 2) + 4 (g / 2) .. + 3 (the
     // order in which the weight rows are read below), so that exchanging lane groups between the row blocks (v_permlane16_swap,
     // behind the main loop) leaves the sums as v_mfma_f32_32x32x16_bf16 would: one layout for the epilogue.
-    constexpr bool B16 = !FP8 && !WTR && !XTR && BM >= 256;
+    constexpr bool B16 = !FP8 && !WTR && !XTR && TL::MFMA16;
+    static_assert(PAIR || FP8 || B16, "single slices of bf16 operands are multiplied into the sums of 16 x 16 blocks");
     constexpr int FN16 = 2 * FN, HX = FM;
     const int kquarter = lane >> 4;
     const int wfrag_lane16 = 8 * ((lane >> 2) & 1) + 4 * ((lane >> 3) & 1) + (lane & 3);      // weight row of this lane in a block of 16
@@ -967,7 +976,7 @@ __global__ __launch_bounds__(TL::NT) void grouped_gemm_ring_kernel(const GemmPar
                 else tile_steps(std::integral_constant<int, 1>{}, std::false_type{});
             }
         } else if constexpr (PAIR && !FP8) {
-            // transposing reads (WTR, XTR) and 64-row tiles: 32 x 32 x 16 MFMAs.  (On 16 x 16 x 32 ones, rolling as above, the weight gradients of 131072 rows,
+            // transposing reads (WTR, XTR), 64-row tiles and launches below the power cap: 32 x 32 x 16 MFMAs.  (On 16 x 16 x 32 ones, rolling as above, the weight gradients of 131072 rows,
             // 64 experts, 2048 x 1408 take 2.10 ms for the two where these take 2.06, the input gradients 1.95 against 1.92: the LDS, which serves
             // transposing reads at two thirds of the rate of others, is the limit there, and the next item's weights come in one bunch.)
             // Software pipeline over "blocks" (half a K-slice: one 16-byte chunk per row and

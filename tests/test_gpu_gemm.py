@@ -1047,6 +1047,34 @@ def test_scales_divided_out_with_either_bias(E, rows, K, N, epi, given):
     assert torch.equal(divided.view(torch.int16), folded.view(torch.int16))
 
 
+@pytest.mark.parametrize("E,rows,K,N,epi,sixteen", [
+    (8, 4096, 1024, 1024, 0, False), (8, 8192, 2048, 3064, 0, True), (8, 8192, 2048, 2304, 1, False), (100, 20000, 2048, 1016, 0, True),
+    (200, 30000, 1024, 2056, 3, True), (200, 30000, 512, 776, 1, False), (5, 9001, 2600, 2600, 0, True), (5, 9001, 1000, 2600, 0, False),
+    (8, 8192, 2048, 3840, 2, True), (8, 8192, 2048, 1280, 2, False), (8, 16384, 4096, 512, 2, True), (4, 33000, 960, 2176, 2, False), (70, 9001, 2632, 2600, 2, True),
+    (8, 16384, 4096, 1024, 0, True), (8, 4096, 4096, 1024, 0, False), (6, 16400, 4168, 1024, 1, True), (6, 4001, 4168, 1024, 1, False),      # cut along K
+])
+def test_tall_ring_by_the_launch_takes_one_of_two_mfma_shapes(E, rows, K, N, epi, sixteen):
+    """Launches that reach the power cap run 16 x 16 x 32 MFMAs (mfma16_pays), others 32 x 32 x 16 ones, as all do whose weights have n contiguous:
+    the same bits as those."""
+    from fast_moe_amd.kernels.hip import _lib, ops
+    g = torch.Generator(device="cuda").manual_seed(E + K + N)
+    x = torch.randn(rows, K, generator=g, device="cuda").to(BF16)
+    ws = [(torch.randn(E, N, K, generator=g, device="cuda") * K ** -0.5).to(BF16) for _ in range(2 if epi == 2 else 1)]
+    cuts = torch.randint(0, rows, (E - 1,), generator=g, device="cuda").sort().values
+    off = torch.cat([cuts.new_zeros(1), cuts, cuts.new_full((1,), rows)])
+    kw = dict(total_rows=rows, epilogue=epi, bias=torch.randn(E, N, generator=g, device="cuda").to(BF16))
+    if epi == _lib.EPI_GATED:
+        kw["gate"] = torch.randn(rows, N, generator=g, device="cuda").to(BF16)
+    def run(views):
+        return ops.grouped_gemm(off, x, views[0], **kw, **({"b2": views[1]} if epi == 2 else {}))
+    nk = [w.permute(0, 2, 1) for w in ws]
+    ran = kernels_run(lambda: run(nk))[0]
+    assert "ring_kernel" in ran and ("Mfma16" in ran) == sixteen, ran
+    kn = [w.contiguous() for w in nk]
+    assert "Mfma16" not in kernels_run(lambda: run(kn))[0]
+    assert torch.equal(run(nk).view(torch.int16), run(kn).view(torch.int16))
+
+
 @pytest.mark.parametrize("E,rows,K,N,layout,epi", [
     (3, 700, 72, 264, "nk", 0), (3, 700, 120, 136, "kn", 0),        # one pair of K-slices and the shortest / longest rest
     (2, 1000, 1000, 520, "nk", 2), (2, 1000, 1000, 520, "kn", 2),

@@ -41,7 +41,8 @@ def scratch(tmp_path_factory):
 # ring kernels: <configuration, e4m3, epilogue, wtr, kwin, xtr, msc, ktail>; streaming ones: <e4m3, epilogue, msc>
 @pytest.mark.parametrize("pattern,most", [
     (r"ring_kernel<RingCfg<256, 256, 2, 4, [124], 2>, true, \d, false, false, false, (true|false), false>", 0),     # scales in the MFMAs or divided out
-    (r"ring_kernel<RingCfg<256, 256, 2, 4, [12], 2>, false, \d, false, false, false, false, false>", 0),
+    (r"ring_kernel<(Mfma16<)?RingCfg<256, 256, 2, 4, [124], 2>( >)?, false, \d, false, false, false, false, (true|false)>", 0),
+    (r"ring_kernel<(Mfma16<)?RingSplitCfg<[14]>( >)?, false, ", 20),
     (r"ring_kernel<RingCfg<256, 256, 2, 4, 0, 2>, true, [02], ", 0),
     (r"ring_kernel<RingCfg<256, 256, 2, 4, 0, 2>, true, 1, ", 24),
     (r"ring_kernel<RingCfg<256, 256, 2, 4, 4, 2>, true, \d, false, false, false, (true|false), true>", 32),         # K tails
