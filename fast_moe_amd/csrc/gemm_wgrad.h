@@ -46,7 +46,7 @@ __global__ __launch_bounds__(WgradTile::NT, 3) void grouped_wgrad_kernel(const G
     int expert, mt, st;
     if (!t.locate(expert, mt, st)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave & 1, wn = wave >> 1, khalf = lane >> 5, l16 = lane & 15;
+    const int wm = wave & 1, wn = wave >> 1, khalf = lane >> 5;
     const int m0 = mt * BM, rows_valid = t.m - m0 < BM ? t.m - m0 : BM;
     int n0 = st * t.strip * BN;
     const int n_end = n0 + t.strip * BN < p.N ? n0 + t.strip * BN : p.N;
@@ -70,21 +70,24 @@ __global__ __launch_bounds__(WgradTile::NT, 3) void grouped_wgrad_kernel(const G
     // (bf16: rows 16 apart have the same place in their group of 4)
     const int put = r * (BN * ESIZE) + ((F32 ? c : c ^ (4 * (r & 3))) << 4);
     // where this lane reads the fragment of columns 32 * f .. 32 * f + 31: its first transposing read; fp32: its column of row khalf
-    auto place = [&](int f) -> int {
+    auto place = [&](int f, int lane) -> int {
+        const int khalf = lane >> 5, l16 = lane & 15;
         if constexpr (F32) return khalf * (BN * ESIZE) + (32 * f + (lane & 31)) * ESIZE;
         const int col = 32 * f + 16 * ((lane >> 4) & 1) + 4 * (l16 & 3), row = 8 * khalf + (l16 >> 2);
         return row * 256 + (((col >> 3) ^ (4 * (l16 >> 2))) << 4) + (col & 7) * 2;
     };
-    int at_a[2], at_b[2];
-#pragma unroll
-    for (int f = 0; f < 2; ++f) {
-        at_a[f] = place(2 * wm + f);
-        at_b[f] = place(2 * wn + f) + WgradTile::OPERAND_BYTES;
-    }
-
     fetch(0);
     int buffer = 0;
     for (;;) {
+        // (found again for every tile: kept over the epilogue they are spilled, and the reload waits for the next tile's rows and this one's stores: 128
+        // experts of 32 rows, 1536 x 4096 379 us, 303 so; 12 experts, 200 rows, 1000 x 2600 16.3 / 15.8)
+        int at_a[2], at_b[2], l = lane;
+        asm volatile("" : "+v"(l));
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            at_a[f] = place(2 * wm + f, l);
+            at_b[f] = place(2 * wn + f, l) + WgradTile::OPERAND_BYTES;
+        }
         f32x16 acc[2][2];       // [column block][row block]
 #pragma unroll
         for (int i = 0; i < 2; ++i)

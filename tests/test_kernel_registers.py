@@ -48,6 +48,7 @@ def scratch(tmp_path_factory):
     (r"ring_kernel<RingCfg<256, 256, 2, 4, 4, 2>, true, \d, false, false, false, (true|false), true>", 32),         # K tails
     (r"ring_kernel<RingSplitCfg<1>, true, ", 40),
     (r"stream_kernel<1, [02], ", 0),
+    (r"grouped_wgrad_kernel<", 0),
     (r"stream_kernel<1, 1, ", 44),
 ])
 def test_scratch_of_the_kernels_that_fill_the_register_file(scratch, pattern, most):
