@@ -1,5 +1,5 @@
 // The epilogue all grouped GEMM kernels share: scales, bias, SiLU / SwiGLU / gating, bf16 rounding,
-// and the stores (rearranged in registers so that adjacent lanes write contiguous bytes).
+// and the stores (through LDS, or between the lanes of a row, so that adjacent lanes write contiguous bytes).
 #pragma once
 
 #include "gemm_params.h"
@@ -359,15 +359,28 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                     }
                 }
             };
+            // SwiGLU on 64-row tiles: the two lanes of a row trade the halves of 16 columns and store 32 bytes, in the midst of the arithmetic.  Such a
+            // launch has a tile or two for a CU, and ends with them: rows through LDS leave only behind all of it.  us, LDS / this: 600 rows, 12
+            // experts, 2368 -> 2 x 704 23.5 / 23.2, e4m3 16.2 / 15.6; 800 rows, 16 experts, 2048 -> 2 x 512 20.5 / 20.0, e4m3 14.6 / 14.1; many tiles are
+            // level (4000 rows, 64 experts, 2048 -> 2 x 1408 189.5 / 189.1, with the pre-activations 197.6 / 198.7).
+            constexpr bool DIRECT = SWIGLU && FM == 2;
+            auto store_pair = [&](int fm, int kind, int nq, const uint32_t (&pk)[2][2]) {
+                const int64_t stride = kind ? p.aux_stride : p.out_stride;
+                const u32x2 s0 = __builtin_amdgcn_permlane32_swap(pk[0][0], pk[1][0], false, false);
+                const u32x2 s1 = __builtin_amdgcn_permlane32_swap(pk[0][1], pk[1][1], false, false);
+                uint16_t* const base = (kind == 0 ? p.out : kind == 1 ? p.aux : p.aux2) + (row0 + frag_row(fm)) * stride + nq;
+                const bool ok = row_ok[fm] && nq + 8 * khalf + 7 < p.N;
+                store16_uniform_base(base, ok ? lane_offset(stride) : kDropLane, u32x4{s0[0], s1[0], s0[1], s1[1]});
+            };
             // what the lane contributes to piece 4 fn + 2 gp + q of row block fm, rounded to bf16
             auto emit = [&](int fm, int kind) {
 #pragma unroll
                 for (int fn = 0; fn < FN_OUT; ++fn)
 #pragma unroll
-                    for (int gp = 0; gp < 2; ++gp)
+                    for (int gp = 0; gp < 2; ++gp) {
+                        uint32_t pk[2][2];
 #pragma unroll
                         for (int q = 0; q < 2; ++q) {
-                            uint32_t pk[2];
 #pragma unroll
                             for (int j = 0; j < 4; j += 2) {        // two columns at a time: one conversion instruction rounds a pair
                                 const int v = 4 * (2 * gp + q) + j;
@@ -392,10 +405,12 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                                 if (kind == 2) y = u;
                                 if (EPI == FMOE_EPI_SILU || (SWIGLU && kind == 0)) y = pack_bf16(fast_silu_f32(low(y)), fast_silu_f32(high(y)));
                                 if (SWIGLU && kind == 0) y = pack_bf16(low(y) * low(u), high(y) * high(u));
-                                pk[j / 2] = y;
+                                pk[q][j / 2] = y;
                             }
-                            put(fm % RB, 4 * fn + 2 * gp + q, pk[0], pk[1]);
+                            if (!DIRECT) put(fm % RB, 4 * fn + 2 * gp + q, pk[q][0], pk[q][1]);
                         }
+                        if (DIRECT) store_pair(fm, kind, col0 + 32 * fn + 16 * gp, pk);
+                    }
             };
             auto store = [&](int fm0, int kind) {       // the rows taken last
                 const int64_t stride = kind ? p.aux_stride : p.out_stride;
@@ -433,9 +448,18 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
                 }
             };
             if constexpr (GATED) fetch_gate(0);
+#pragma unroll
+            for (int fm = 0; DIRECT && fm < FM; ++fm) {
+#pragma unroll
+                for (int kind = 0; kind < KINDS; ++kind) {
+                    emit(fm, kind);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                after_stores.block_done(fm);
+            }
             // a step's rows are stored behind the next step's arithmetic, by when they have arrived
 #pragma unroll
-            for (int step = 0; step <= FM / RB * KINDS; ++step) {
+            for (int step = 0; !DIRECT && step <= FM / RB * KINDS; ++step) {
                 const int fm = step / KINDS * RB, kind = step % KINDS;
                 if (step < FM / RB * KINDS) {
 #pragma unroll
@@ -617,7 +641,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
         // which the compiler cannot see, on every iteration.
         FMOE_EPI_STAMP(FM);
         // The number of store instructions issued above, whatever the lanes' predicates: 4 per row
-        // block of 64 columns in the staged form, one per column group (and per output tensor) otherwise.
+        // block of 64 columns in the staged form, one per column group (and per output tensor) otherwise (as many).
         // The ring kernel's first double step of the next tile skips its own counted wait on the
         // strength of this one (see skip_wait there), which is only sound when every one of these
         // stores was issued unconditionally, i.e. through store16_uniform_base (ALWAYS_VEC).
