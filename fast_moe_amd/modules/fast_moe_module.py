@@ -137,7 +137,9 @@ class FastMoELayer(nn.Module):
         if getattr(self.route, "__func__", None) is _ROUTE and x.ndim == 3:
             # the same steps as below, issued by one native call (a route() of a subclass's or a caller's own is asked)
             forward = _lib.host().mlp_forward
-            linear = self._small_gate(x) if ops.gate_softmax is _GATE_SOFTMAX else None
+            # (and so is a _scores(), or a replaced ops.gate_softmax)
+            own = ops.gate_softmax is _GATE_SOFTMAX and getattr(self._scores, "__func__", None) is _SCORES
+            linear = self._small_gate(x) if own else None
             scores = None if linear is not None else self._scores(x)
             args = (x.reshape(-1, self.input_dim), self._experts_hidden_w.permute(0, 2, 1), self._experts_hidden_bias,
                     self._experts_w.permute(0, 2, 1), self._experts_bias, k, ops.GATE_L1, EPI_SILU, ops._stream(x))
@@ -169,6 +171,7 @@ class FastMoELayer(nn.Module):
 
 
 _ROUTE = FastMoELayer.route     # what the native call stands for
+_SCORES = FastMoELayer._scores
 _GATE_FORWARD = GatingNetwork.forward
 _GATE_SOFTMAX = ops.gate_softmax
 _SMALL_BATCH = 128              # (the library's own rule, fmoe_gate_softmax_pays, without a call for the others)

@@ -335,6 +335,31 @@ def test_gate_and_routing_in_one_launch(T, D, E, K, dtype, bias, monkeypatch):
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
 
 
+@pytest.mark.parametrize("tokens", [16, 200])
+def test_scores_of_a_subclass_are_asked_whatever_the_batch(tokens):
+    """A _scores() of a subclass's or an instance's own gives the probabilities, for a batch whose gate the native call would issue as for others."""
+    from fast_moe_amd import FastMoELayer
+
+    class Last(FastMoELayer):
+        def _scores(self, x):
+            scores = torch.zeros(x.shape[0] * x.shape[1], self.num_experts, dtype=x.dtype, device=x.device)
+            scores[:, -2:] = 0.5
+            return scores
+
+    layer = FastMoELayer(64, 96, 64, 4).to(BF16).cuda()
+    own = Last(64, 96, 64, 4).to(BF16).cuda()
+    own.load_state_dict(layer.state_dict())
+    x = torch.randn(1, tokens, 64, device="cuda").to(BF16)
+    with torch.no_grad():
+        plain, want = layer(x, 2), own(x, 2)
+        layer._scores = lambda t: own._scores(t)
+        got = layer(x, 2)
+        hidden = [torch.nn.functional.silu(x[0] @ own._experts_hidden_w[e].t() + own._experts_hidden_bias[e]) for e in (2, 3)]
+        last = sum(0.5 * (h @ own._experts_w[e].t() + own._experts_bias[e]).float() for h, e in zip(hidden, (2, 3)))
+    assert torch.equal(got, want) and not torch.equal(got, plain)
+    torch.testing.assert_close(want[0].float(), last, atol=2e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("shape", [(1, 4, 128), (2, 4, 32), (8, 64), (512,), (2, 2, 2, 64)])
 def test_small_batches_of_another_shape_go_through_the_gate_module(shape):
     """What Linear and the softmax over the third dimension refuse is refused whatever the batch, before anything is routed, and what they
