@@ -263,9 +263,9 @@ static size_t split_bytes(const fmoe_gemm_desc* d, const GemmParams& p, int sel)
 
 extern "C" size_t fmoe_grouped_gemm_workspace_bytes(const fmoe_gemm_desc* d) {
     // asked before every call: those that are no tall ring's, and K of up to 15 pairs of slices, which split_pays never takes, end here
-    // (fp32: up to 511, where a cut gains no 8 us either)
+    // (fp32: up to five pairs, which no number of tiles lets f32x3_split_pays take)
     if (!d || (d->a_dtype != FMOE_F32 && d->total_rows < kTallRows * (int64_t)d->num_experts) ||
-        d->k <= (d->a_dtype == FMOE_E4M3 ? 1920 : d->a_dtype == FMOE_F32 ? 511 : 960))
+        d->k <= (d->a_dtype == FMOE_E4M3 ? 1920 : d->a_dtype == FMOE_F32 ? 320 : 960))
         return 0;
     GemmParams p;
     int sel;

@@ -58,6 +58,8 @@ int launch_f32x3(GemmParams p, hipStream_t stream) {
 //     4 experts, 4096 -> 2560 206 / 196, 4096 -> 2 x 1280 207 / 193
 //   * 64 x 128 tiles behind two whole rounds, the pieces as third blocks (three rounds: 3000 rows, 5 experts, 2048 -> 2048 188 / 198).  An even load
 //     that leaves no tile pays for the second launch: 4096 rows, 8 experts, 4096 -> 1024 245 / 254
+// From six pairs of slices on (K of 321): 8192 rows, 8 experts, 324 -> 1024 72.9 / 62.6, 384 76.1 / 64.9, 504 98.2 / 79.3; 16384 rows, 384 -> 1024 121 / 110;
+// 24 experts, 8000 rows, 480 -> 1024 89.8 / 82.1; SwiGLU, 8192 rows, 416 -> 2 x 1024 129 / 120.
 template <int BM>
 bool f32x3_split_pays(const GemmParams& p, bool swiglu) {
     const int bn_out = swiglu ? 64 : 128, pairs = (p.K + 63) / 64;

@@ -369,6 +369,20 @@ def test_column_quantiser_scratch_rule(lib, E, K, N, two_launches):
     assert (need > 0) == two_launches
 
 
+@pytest.mark.parametrize("rows,E,K,N,cut", [
+    (8192, 8, 512, 1024, True), (8192, 8, 504, 1024, True), (8192, 8, 384, 1024, True), (8192, 8, 324, 1024, True), (8192, 8, 320, 1024, False),
+    (8000, 24, 480, 1024, True), (8000, 24, 448, 1024, False), (4096, 8, 416, 2048, True), (4096, 8, 384, 2048, False), (4096, 8, 504, 4096, False),
+])
+def test_fp32_calls_of_short_contractions_that_are_cut_along_k(lib, rows, E, K, N, cut):
+    """The look at K ahead of the rule turns nothing away that the rule takes."""
+    from fast_moe_amd.kernels.hip._lib import GemmDesc
+    d = GemmDesc()
+    d.num_experts, d.n, d.k, d.index_div, d.total_rows, d.a_rows = E, N, K, 1, rows, rows
+    d.offsets, d.a, d.b, d.out, d.a_dtype, d.out_dtype = 64, 64, 64, 64, 0, 0
+    d.a_stride_row, d.b_stride_e, d.b_stride_k, d.b_stride_n, d.out_stride_row = K, K * N, 1, K, N
+    assert (lib.fmoe_grouped_gemm_workspace_bytes(ctypes.byref(d)) > 0) == cut
+
+
 @pytest.mark.parametrize("dtype,T,D,E,K,pays", [
     (1, 64, 128, 8, 2, True), (1, 64, 192, 16, 2, True), (1, 64, 200, 8, 2, False), (1, 16, 2048, 16, 4, True), (1, 16, 2056, 16, 4, False),
     (1, 17, 2048, 16, 4, False), (1, 16, 1360, 32, 4, True), (1, 16, 1368, 32, 4, False), (1, 16, 816, 64, 8, True), (1, 16, 816, 65, 8, False),

@@ -1286,6 +1286,7 @@ def test_fp32_on_bf16_matrix_cores(E, rows, K, N, layout, epi, tile, case):
     ([3000, 3500, 30], 772, 700, "nk", 2, 128), ([3000, 3500, 30], 1024, 700, "kn", 2, 128),
     ([2100, 0, 500, 400, 33], 4100, 1000, "kn", 1, 128), ([2100, 500, 400, 33], 4160, 904, "nk", "silu", 128),       # less than a round
     ([500] * 66, 1024, 252, "nk", 0, 128),                  # more than 64 experts
+    ([2048] * 3 + [2049], 324, 1024, "nk", 0, 128), ([1000, 1100, 900, 1024, 1100, 1000, 1068, 1000], 420, 1020, "kn", 2, 128),      # six and seven pairs of slices
     ([512] * 7 + [513], 4096, 1024, "nk", 0, 64), ([520, 0, 500, 600, 1400, 1033], 1028, 1000, "kn", 1, 64),
     ([520, 0, 500, 600, 1400, 1033], 996, 964, "nk", "silu", 64), ([520, 3, 500, 600, 1400, 1033], 2052, 900, "kn", "silu", 64),
     ([512] * 8, 1024, 1024, "nk", 0, 64),                   # no tile left: nothing is cut
