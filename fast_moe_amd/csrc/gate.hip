@@ -3,8 +3,8 @@
 // What it is for: 64 tokens, 8 experts, 128 inputs: the library GEMM with its bias epilogue takes 25 us of host time to issue and 5 us to run, the
 // softmax 6 and 3; this kernel 4 us to issue and as long to run.  A batch of few tokens is a chain of such launches (the layer's pass
 // 61 us, bound by the host).  Logits are fp32 sums plus bias rounded to the scores' type, as torch.nn.functional.linear rounds
-// them, and the softmax is torch's, step by step (one wave per token, expert e in lane e % 64, butterfly sums from the
-// widest distance down).
+// them, and the softmax is torch's, step by step (expert e in lane e % 64 of a token's, butterfly sums from the widest
+// distance down; up to 32 experts a wave has two tokens, up to 16 four, whose wider steps would only add zeros).
 #include "gate.h"
 
 namespace fmoe {

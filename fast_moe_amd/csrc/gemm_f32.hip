@@ -56,8 +56,9 @@ int launch_f32x3(GemmParams p, hipStream_t stream) {
 //     4096 -> 1024 (64 x 128 tiles instead) 320 / 341, 3000 rows, 5 experts, 2048 -> 2048 184 / 189; a few gain (4 experts, 1000 rows, 2048 -> 4096 162 / 155)
 //   * less than a round, from 5/8 of one on, all of it as pieces, two or three to a CU: 3000 rows, 4 experts, 4096 -> 1024, hot 256 / 201; 1000 rows,
 //     4 experts, 4096 -> 2560 206 / 196, 4096 -> 2 x 1280 207 / 193
-//   * 64 x 128 tiles behind two whole rounds, the pieces as third blocks (three rounds: 3000 rows, 5 experts, 2048 -> 2048 188 / 198).  An even load
-//     that leaves no tile pays for the second launch: 4096 rows, 8 experts, 4096 -> 1024 245 / 254
+//   * 64 x 128 tiles behind two whole rounds, the pieces as third blocks (behind one, three and four 12 calls, gate and Zipf loads, are level, 0.99 to
+//     1.013: 5000 rows, 8 experts, 4096 -> 1280 379 / 384, 2300 rows, 10 experts, 1024 -> 2560 106 / 105).  An even load that leaves no tile pays for
+//     the second launch, which takes 4 us to find that: 4096 rows, 8 experts, 4096 -> 1024 238 / 246, 1024 -> 4096 230 / 233
 // From six pairs of slices on (K of 321): 8192 rows, 8 experts, 324 -> 1024 72.9 / 62.6, 384 76.1 / 64.9, 504 98.2 / 79.3; 16384 rows, 384 -> 1024 121 / 110;
 // 24 experts, 8000 rows, 480 -> 1024 89.8 / 82.1; SwiGLU, 8192 rows, 416 -> 2 x 1024 129 / 120.
 template <int BM>

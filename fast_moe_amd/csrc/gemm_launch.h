@@ -238,7 +238,8 @@ inline int direct_columns(int n, bool swiglu) { return swiglu ? (n + 31) / 32 : 
 //     -> 2048, not taken, level where one expert is hot), but not K of two slices (gemm_f32.hip).  With more rows the other kernel's tiles
 //     hold more of them: K from 1024 on and one tile per CU (320 rows, 8 experts, 1024 -> 512 40.0 / 17.6), K from 128 on in whole lines and one for two CUs (587 rows,
 //     16 experts, 960 -> 128 29.0 / 16.0; 644 rows, 4 experts, 128 -> 448 8.7 / 7.2; 306 rows, 8 experts, 640 -> 2 x 128 31.7 / 14.3: 26
-//     such calls, 1.13 to 2.2 times as fast; of K = 72 two, 1.11 to 1.21; the tests of the other kernel's edges have it at K in part).  Between them both ways: 164 tiles, 192 -> 256 10.7 / 14.6, 147 tiles, 960 -> 448 38.2 / 19.3; more tiles:
+//     such calls, 1.13 to 2.2 times as fast).  K in part and below 128 would gain as well (300 rows, 8 experts, 100 -> 128 8.3 / 6.2, 260 -> 128 11.9 / 7.7, 600
+//     -> 128 19.7 / 10.2): not taken, the tests of the other kernel's edges and of this line are at such K.  Between them both ways: 164 tiles, 192 -> 256 10.7 / 14.6, 147 tiles, 960 -> 448 38.2 / 19.3; more tiles:
 //     4000 rows, 8 experts, 4096 -> 512, four per CU, 143 / 180.
 inline bool direct_pays(const GemmParams& p, int esize, bool swiglu) {
     const int64_t experts = p.E < p.total_rows ? p.E : p.total_rows, cus = compute_units();
