@@ -295,15 +295,19 @@ inline bool split_before_direct(const GemmParams& p, int esize, int epilogue) {
 //   SwiGLU  16384, 1024 -> 2 x 2048 131.7 / 132.5, 140.6 / 146.5    32768, 1024 -> 2 x 1536 188.8 / 187.4, 200.8 / 206.6, -> 2 x 2560 309 / 305, 321 / 325
 //           16384, 2048 -> 2 x 1536 190.3 / 190.1, 197.5 / 204.1, -> 2 x 2048 241 / 239, 250 / 252    32768, 2048 -> 2 x 2560 577 / 564, 589 / 579
 //           16384, 4096 -> 2 x 512 127.2 / 124.5, 130.4 / 125.5    8192, 4096 -> 2 x 512 75.9 / 81.8    65536, 512 -> 2 x 2048 288.9 / 294.9
-// So by CUs' worths of K: 3072 from K of 2048 on (SwiGLU 4096), 6000 (8192) below.
-inline bool mfma16_pays(const GemmParams& p, bool swiglu) {
-    const int bn = swiglu ? 128 : 256, need = p.K >= (swiglu ? 4096 : 2048) ? 3072 : swiglu ? 8192 : 6000;
+//   K in part (the loop of 32 x 32 x 16 masks behind its loads)    9189 rows, 12 experts, 2600 -> 1000 68.8 / 67.9, 1000 -> 2600 66.5 / 66.0, 1000 -> 1024
+//           33.0 / 34.2, 4104 -> 1024 97.0 / 95.9    16384, 8 experts, 2600 -> 1000 101.5 / 98.6, 1000 -> 2600 102.7 / 101.3, 1000 -> 1024 57.8 / 59.0, 520 ->
+//           3000 84.0 / 84.7    SwiGLU 2600 -> 2 x 1296 229 / 219, 1000 -> 2 x 1296 102.7 / 102.6, -> 2 x 2496 187 / 189, 520 -> 2 x 1496 82.5 / 87.1
+// So by CUs' worths of K: 3072 from K of 2048 on (SwiGLU 4096), 6000 (8192) below; K in part 1600 from 2048 (plain 768) on.
+inline bool mfma16_pays(const GemmParams& p, bool swiglu, bool in_part) {
+    const int bn = swiglu ? 128 : 256;
+    const int need = in_part && p.K >= (swiglu ? 2048 : 768) ? 1600 : p.K >= (swiglu ? 4096 : 2048) ? 3072 : swiglu ? 8192 : 6000;
     const int64_t n_tiles = (p.N + bn - 1) / bn, least = (p.total_rows + 255) / 256, most = most_row_tiles(p.total_rows, p.E, 256);
     return (least + most) * n_tiles >= 2 * (int64_t)need * compute_units() / p.K && (!swiglu || p.K >= 1024);
 }
 template <typename TL, int EPI, bool KTAIL = false>
 int launch_ring_bf16(const GemmParams& p, hipStream_t stream) {
-    if (mfma16_pays(p, EPI == FMOE_EPI_SWIGLU)) return launch_ring_cfg<Mfma16<TL>, false, EPI, false, false, false, false, KTAIL>(p, stream);
+    if (mfma16_pays(p, EPI == FMOE_EPI_SWIGLU, p.K % 64 != 0)) return launch_ring_cfg<Mfma16<TL>, false, EPI, false, false, false, false, KTAIL>(p, stream);
     return launch_ring_cfg<TL, false, EPI, false, false, false, false, KTAIL>(p, stream);
 }
 

@@ -1049,7 +1049,8 @@ def test_scales_divided_out_with_either_bias(E, rows, K, N, epi, given):
 
 @pytest.mark.parametrize("E,rows,K,N,epi,sixteen", [
     (8, 4096, 1024, 1024, 0, False), (8, 8192, 2048, 3064, 0, True), (8, 8192, 2048, 2304, 1, False), (100, 20000, 2048, 1016, 0, True),
-    (200, 30000, 1024, 2056, 3, True), (200, 30000, 512, 776, 1, False), (5, 9001, 2600, 2600, 0, True), (5, 9001, 1000, 2600, 0, False),
+    (200, 30000, 1024, 2056, 3, True), (200, 30000, 512, 776, 1, False), (5, 9001, 2600, 2600, 0, True), (5, 9001, 1000, 2600, 0, True), (5, 9001, 1000, 2296, 0, False), (12, 9189, 2600, 1000, 0, True),
+    (5, 9001, 2600, 1400, 2, True), (5, 9001, 1000, 2600, 2, False),
     (8, 8192, 2048, 3840, 2, True), (8, 8192, 2048, 1280, 2, False), (8, 16384, 4096, 512, 2, True), (4, 33000, 960, 2176, 2, False), (70, 9001, 2632, 2600, 2, True),
     (8, 16384, 4096, 1024, 0, True), (8, 4096, 4096, 1024, 0, False), (6, 16400, 4168, 1024, 1, True), (6, 4001, 4168, 1024, 1, False),      # cut along K
 ])
