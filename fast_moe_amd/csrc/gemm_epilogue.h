@@ -311,8 +311,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)
         // (two of them where the wave has 32 output columns) goes through the wave's own 4 KB of LDS: pieces of 4 columns in, whole rows of
         // 16-byte chunks out, which 8 (4) adjacent lanes store.  Rearranging the same rows in registers (lane swaps, transposes of
         // quads by DPP moves and selects) was 330 of an epilogue's 640 vector instructions, and the two waves of a SIMD are bound by those.
-        // Chunk c of row r lies at position c ^ (r / 2) % 8 (c ^ (r / 4) % 4), its two halves swapped in rows 16..31 of each 32: neither
-        // the writes nor the reads meet in a bank.  A wave's LDS instructions execute in order, nothing has to be waited for in between.
+        // Chunk c of row r lies at position c ^ (r / 2) % 8 (c ^ (r / 4) % 4), its two halves swapped in rows 16..31 of each 32: the reads do not
+        // meet in a bank, the writes, served 16 lanes and 128 bytes at a time, two by two (SQ_LDS_BANK_CONFLICT: 4 cycles a write, 2 to 9 % of a launch's
+        // LDS cycles; c ^ r % 8, c ^ (r / 2) % 4 and halves swapped by r / 8 have none, and whole passes take the same time with them).  A
+        // wave's LDS instructions execute in order, nothing has to be waited for in between.
         if constexpr (ALWAYS_VEC) {
             constexpr int CH = 4 * FN_OUT;                      // 16-byte chunks of a row
             constexpr int RB = FN_OUT == 2 || FM < 2 ? 1 : 2;   // row blocks at a time
